@@ -32,9 +32,9 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
 KERNEL_SOURCES = ["fo_gemm.hip", "fo_aux.hip", "fo_algo.cpp", "fo_overlap.cpp"]
-# fo_gemm256_inst.hip holds one instantiation of the 256x256 GEMM kernel per compilation
-# (dtype fp16 / bf16 x plain / signal / scatter epilogue); each takes minutes, so they are separate jobs.
-GEMM256_INSTANCES = [(d, m) for d in (0, 1) for m in (0, 1, 2)]
+# fo_gemm256_inst.hip and fo_gemm_tile_inst.hip hold the instantiations of the GEMM kernels for one dtype (fp16 / bf16)
+# and one epilogue (plain / signal / scatter) per compilation; they take up to minutes, so they are separate jobs.
+GEMM_INSTANCES = [(src, d, m) for src in ("fo_gemm256_inst.hip", "fo_gemm_tile_inst.hip") for d in (0, 1) for m in (0, 1, 2)]
 
 # -packed-fp32-ops off: hipcc must not form v_pk_*_f32 from the float code here.
 HIP_FLAGS = [
@@ -65,8 +65,7 @@ def build_kernels(extra_flags=()):
         return obj
 
     # the long jobs first
-    jobs = [("fo_gemm256_inst.hip", [f"-DFO_INST_DTYPE={d}", f"-DFO_INST_MODE={m}"], f"_{d}_{m}")
-            for d, m in GEMM256_INSTANCES]
+    jobs = [(src, [f"-DFO_INST_DTYPE={d}", f"-DFO_INST_MODE={m}"], f"_{d}_{m}") for src, d, m in GEMM_INSTANCES]
     jobs += [(src, [], "") for src in KERNEL_SOURCES]
     with ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 4)) as pool:
         objs = list(pool.map(compile_one, jobs))

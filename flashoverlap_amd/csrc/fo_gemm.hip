@@ -1,17 +1,10 @@
-// Host side of the gfx950 MFMA GEMM: picks the kernel shape for a problem and
+// Host side of the gfx950 MFMA GEMM: picks the workgroup tile for a problem and
 // launches it (plain, signal and scatter epilogues).  The device code is in
-// fo_gemm_kernel.h and fo_gemm256_kernel.h; the latter's six instantiations are
-// compiled in translation units of their own (fo_gemm256_inst.hip).
+// fo_gemm256_kernel.h and fo_gemm_tile_kernel.h, whose instantiations are
+// compiled in translation units of their own (fo_gemm256_inst.hip, fo_gemm_tile_inst.hip).
 #include <atomic>
 
-#include "fo_gemm_kernel.h"
 #include "fo_gemm_launch.h"
-
-namespace {
-
-using namespace fo_gemm_dev;
-
-}  // namespace
 
 int fo_gemm_dev::fo_gemm256_launch(int dtype, int mode, const GemmArgs &a, hipStream_t stream, int *resident_out,
                                    int expect_resident) {
@@ -28,38 +21,129 @@ int fo_gemm_dev::fo_gemm256_launch(int dtype, int mode, const GemmArgs &a, hipSt
     return FO_ERR_ARG;
 }
 
+int fo_gemm_dev::fo_gemm_tile_launch(int dtype, int mode, const GemmArgs &a, int tm, int tn, hipStream_t stream,
+                                     int *resident_out, int expect_resident) {
+    const int key = (dtype == FO_BF16 ? 3 : 0) + mode;
+    switch (key) {
+        case 0: return fo_gemm_tile_launch_0_0(a, tm, tn, stream, resident_out, expect_resident);
+        case 1: return fo_gemm_tile_launch_0_1(a, tm, tn, stream, resident_out, expect_resident);
+        case 2: return fo_gemm_tile_launch_0_2(a, tm, tn, stream, resident_out, expect_resident);
+        case 3: return fo_gemm_tile_launch_1_0(a, tm, tn, stream, resident_out, expect_resident);
+        case 4: return fo_gemm_tile_launch_1_1(a, tm, tn, stream, resident_out, expect_resident);
+        case 5: return fo_gemm_tile_launch_1_2(a, tm, tn, stream, resident_out, expect_resident);
+    }
+    return FO_ERR_ARG;
+}
+
 namespace {
 
-template <typename Tag, int MTM, int MTN, int BK, int SA, int SB, int WM, int WN, int MODE>
-int launch_variant(const GemmArgs &a, hipStream_t stream, int *resident_out, int expect_resident) {
-    return launch_kernel<fo_gemm_kernel<Tag, MTM, MTN, BK, SA, SB, WM, WN, MODE>, smem_bytes<MTM, MTN, BK, SA, SB>(),
-                         WM * WN * 64>(a, stream, resident_out, expect_resident);
+using namespace fo_gemm_dev;
+
+int launch_tile(int dtype, int mode, const GemmArgs &a, int tm, int tn, hipStream_t stream, int *resident_out = nullptr,
+                int expect_resident = 0) {
+    if (dtype != FO_F16 && dtype != FO_BF16) return FO_ERR_DTYPE;
+    if (tm == 256 && tn == 256) return fo_gemm256_launch(dtype, mode, a, stream, resident_out, expect_resident);
+    return fo_gemm_tile_launch(dtype, mode, a, tm, tn, stream, resident_out, expect_resident);
 }
 
-// Macro tile -> kernel.  256x256 (fo_gemm256_kernel.h: four wavefronts of 128x128, two 64 KiB slots) is
-// the workhorse; the smaller shapes (fo_gemm_kernel.h: three slots for 128x256 and 256x128, two for
-// 128x128) serve problems whose M or N is not a multiple of 256 or that have too few 256x256 tiles to
-// fill the chip.
-template <typename Tag, int MODE>
-int launch_tile(const GemmArgs &a, int mtm, int mtn, hipStream_t stream, int *resident_out, int expect_resident) {
-    if (mtm == 256 && mtn == 256)
-        return fo_gemm256_launch(std::is_same<Tag, fo_bf16_tag>::value ? FO_BF16 : FO_F16, MODE, a, stream, resident_out,
-                                 expect_resident);
-    if (mtm == 128 && mtn == 128)
-        return launch_variant<Tag, 128, 128, 64, 2, 2, 2, 2, MODE>(a, stream, resident_out, expect_resident);
-    if (mtm == 128 && mtn == 256)
-        return launch_variant<Tag, 128, 256, 64, 3, 3, 2, 4, MODE>(a, stream, resident_out, expect_resident);
-    if (mtm == 256 && mtn == 128)
-        return launch_variant<Tag, 256, 128, 64, 3, 3, 2, 2, MODE>(a, stream, resident_out, expect_resident);
-    return FO_ERR_ALGO;
+// How a problem is launched: workgroup tile and raster, and what a second launch computes in a smaller tile.
+struct launch_plan {
+    int tm, tn;                            // workgroup tile
+    int grid_m, grid_n, panel, xcd_remap;  // its raster
+    int count;                             // tiles the launch computes
+    bool whole;                            // a tile is one or more whole reorder tiles, so the kernel can count them
+    int tail, tail_tm, tail_tn;            // raster positions left to the second launch, and its tile
+};
+
+// A launch of parts of reorder tiles cannot count them; fo_signal_all_kernel behind it does (about 3 us).  Shorter
+// products than this many columns of K are computed in whole reorder tiles instead when counters are wanted.
+constexpr int kSignalAfterFromK = 1536;
+
+// 256x256 where fo_pick_raster says so.  Otherwise the smallest tile whose count still fits the chip in one round,
+// one per CU: a smaller tile moves more operand bytes per flop (64x64 twice those of 128x128), but it puts the
+// operand paths of CUs to work that a larger tile leaves idle, and up to that point the time of these sizes is the
+// per-CU operand stream.  Measured over M = 128..4224, N = 1024..8192, K = 512, 2048, 8192: the rule picks the
+// fastest tile or one within a few percent of it (K = 2048, us: 128x4096 64x32 7.3, 64x64 8.1, 128x128 12.8;
+// 512x4096 64x128 11.7, 128x128 13.7, 64x64 16.2; 1024x4096 128x128 16.8, 128x256 21.8, 64x128 21.7; 2048x4096
+// 128x256 29.2, 128x128 31.7).  What needs more than one round of those goes to the 256x256 tile as well if it gives
+// 60 % of the CUs something to do; M and N need not be multiples of 256 for that, only of 128 (the last tile of a
+// dimension then repeats half of its neighbour).
+launch_plan plan_launch(const fo_raster &r, int M, int N, int BM, int BN, bool whole_only) {
+    launch_plan p;
+    p.tail = p.tail_tm = p.tail_tn = 0;
+    auto set = [&](int tm, int tn) {
+        p.tm = tm;
+        p.tn = tn;
+        p.grid_m = (M + tm - 1) / tm;
+        p.grid_n = (N + tn - 1) / tn;
+        p.whole = tm % BM == 0 && tn % BN == 0;
+        p.count = p.grid_m * p.grid_n;
+        p.xcd_remap = p.count >= 16 ? 1 : 0;
+    };
+    // The tile of the second launch: 128x128 while one round of them does it, else 128x256 or 256x128.
+    auto set_tail = [&](int positions, long cus) {
+        p.tail = positions;
+        p.count -= positions;
+        p.tail_tm = BM;
+        p.tail_tn = BN;
+        if (BM == 128 && BN == 128 && positions * 4 > cus && N % 256 == 0) p.tail_tn = 256;
+    };
+    if (r.mtm == 256 && r.mtn == 256) {
+        set(256, 256);
+        p.panel = r.panel;
+        p.xcd_remap = r.xcd_remap;
+        if (r.tail_tiles) set_tail(r.tail_tiles, r.resident);
+        return p;
+    }
+    const long cus = fo_main_tile_resident();
+    static const int shapes[][2] = {{32, 32},  {64, 32},   {64, 64},   {64, 96},   {64, 128},
+                                    {96, 128}, {128, 128}, {128, 192}, {128, 256}, {256, 128}};
+    for (const auto &s : shapes) {
+        if (M < s[0] || N < s[1] || (long)((M + s[0] - 1) / s[0]) * ((N + s[1] - 1) / s[1]) > cus) continue;
+        if (whole_only && (s[0] % BM || s[1] % BN)) continue;
+        set(s[0], s[1]);
+        // of the two largest, the one that holds whole reorder tiles
+        if (!p.whole && s[0] == 128 && s[1] == 256 && M >= 256 && (long)((M + 255) / 256) * (N / 128) <= cus) set(256, 128);
+        // An XCD's workgroups (every eighth of the launch) take one stretch of panels of eight tile rows: they share
+        // operand rows in its L2 both ways.
+        p.panel = p.grid_m < 8 ? p.grid_m : 8;
+        return p;
+    }
+    // Several rounds walk the tiles in strips of the order that fo_schedule_order reports (panels of r.panel rows of
+    // reorder tiles).
+    const int nt = ((M + 255) / 256) * ((N + 255) / 256);
+    if (M >= 256 && N >= 256 && (long)M * N > 512L * 128 * 128 && nt * 5 > cus * 3) {
+        set(256, 256);
+        p.panel = r.panel * BM >= 512 ? r.panel * BM / 256 : 1;
+        const int rem = nt % cus;
+        if (nt > cus && rem && rem * 2 <= cus) set_tail(rem, cus);
+        return p;
+    }
+    p.panel = r.panel;
+    if (N % 256 == 0 && BM == 128) {
+        set(128, 256);
+    } else if (M % 256 == 0 && BN == 128) {
+        set(256, 128);
+        if (BM == 128 && p.panel > 1) p.panel /= 2;
+    } else {
+        set(BM, BN);
+    }
+    return p;
 }
 
-template <int MODE>
-int launch_dtype(int dtype, const GemmArgs &a, int mtm, int mtn, hipStream_t stream, int *resident_out = nullptr,
-                 int expect_resident = 0) {
-    if (dtype == FO_F16) return launch_tile<fo_f16_tag, MODE>(a, mtm, mtn, stream, resident_out, expect_resident);
-    if (dtype == FO_BF16) return launch_tile<fo_bf16_tag, MODE>(a, mtm, mtn, stream, resident_out, expect_resident);
-    return FO_ERR_DTYPE;
+// Signals of a launch whose workgroup tiles are parts of reorder tiles: behind it on the stream, everything at once
+// (such a launch is a single round of short tiles; its reorder tiles complete together anyway).  MM[g] += cseg[g]
+// and, with the monitor on, stamps in tile order (src/overlap/gemm_with_signal.h:343-351).
+__global__ __launch_bounds__(256) void fo_signal_all_kernel(const int32_t *cseg, int G, int32_t *MM, const int32_t *RA, int T,
+                                                            int TN, int monitor) {
+    for (int g = threadIdx.x; g < G; g += 256)
+        __hip_atomic_fetch_add(MM + g, cseg[g], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!monitor) return;
+    __shared__ int first;
+    if (threadIdx.x == 0) first = __hip_atomic_fetch_add(MM + (TN - 1), T, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    for (int t = threadIdx.x; t < T; t += 256)
+        __hip_atomic_store(MM + TN + RA[t], first + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *cseg, int G,
@@ -74,7 +158,7 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     if (rc) return rc;
     if (K % 8) return FO_ERR_SHAPE;  // operand rows are fetched in 16-byte chunks
     if (K > (1 << 21)) return FO_ERR_SHAPE;  // 256 operand rows are addressed through one 31-bit buffer range
-    // the epilogue assumes a wavefront's 128 x 64 (or 64 x 64) block lies inside one reorder tile
+    // the epilogues assume reorder tiles made of 128 x 128 blocks
     if (e->f[0] % 128 || e->f[1] % 128) return FO_ERR_ALGO;
     GemmArgs a;
     a.A = static_cast<const uint16_t *>(A);
@@ -86,10 +170,14 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     a.TN = N / a.BN;
     a.rLDN = rLDN;
     a.RA = RA; a.RE = RE; a.cseg = cseg; a.G = G; a.MM = MM; a.monitor = monitor;
-    a.grid_m = r.grid_m; a.grid_n = r.grid_n; a.panel = r.panel; a.xcd_remap = r.xcd_remap;
+    const launch_plan plan = plan_launch(r, M, N, a.BM, a.BN, mode != MODE_PLAIN && !quiet && K < kSignalAfterFromK);
+    a.grid_m = plan.grid_m; a.grid_n = plan.grid_n; a.panel = plan.panel; a.xcd_remap = plan.xcd_remap;
     a.first = 0; a.sub_m = a.sub_n = 1;
-    a.count = r.grid_m * r.grid_n - r.tail_tiles;
-    a.quiet = quiet ? 1 : 0;
+    a.count = plan.count;
+    a.half = (M % 256 ? 1 : 0) | (N % 256 ? 2 : 0);
+    // counters the launch cannot move itself are moved behind it
+    const bool signal_after = mode != MODE_PLAIN && !quiet && !plan.whole;
+    a.quiet = quiet || signal_after ? 1 : 0;
     a.stream_out = (int64_t)M * N * 2 > kStreamOutAboveBytes ? 1 : 0;
     if (mode != MODE_PLAIN) {
         const long T = (long)(M / a.BM) * a.TN;
@@ -100,22 +188,20 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
         if (monitor && G > a.TN - 1) return FO_ERR_SEGMENTS;
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    auto launch = [&](const GemmArgs &g, int mtm, int mtn, int expect) {
-        switch (mode) {
-            case MODE_PLAIN: return launch_dtype<MODE_PLAIN>(dtype, g, mtm, mtn, s, nullptr, expect);
-            case MODE_SIGNAL: return launch_dtype<MODE_SIGNAL>(dtype, g, mtm, mtn, s, nullptr, expect);
-            default: return launch_dtype<MODE_SCATTER>(dtype, g, mtm, mtn, s, nullptr, expect);
-        }
-    };
-    // the tail split was computed for r.resident workgroups of the main launch
-    rc = launch(a, r.mtm, r.mtn, r.tail_tiles ? r.resident : 0);
-    if (rc || !r.tail_tiles) return rc;
-    // the last, partial wave of 256x256 tiles: the same raster positions in the Algo's own tile
+    // the tail split was computed for that many workgroups of the main launch
+    rc = launch_tile(dtype, mode, a, plan.tm, plan.tn, s, nullptr, plan.tail ? fo_main_tile_resident() : 0);
+    if (rc) return rc;
+    if (signal_after) {
+        hipLaunchKernelGGL(fo_signal_all_kernel, dim3(1), dim3(256), 0, s, cseg, G, MM, RA, (M / a.BM) * a.TN, a.TN, monitor);
+        FO_LAUNCH_CHECK();
+    }
+    if (!plan.tail) return FO_OK;
+    // the last, partial wave of 256x256 tiles: the same raster positions in a smaller tile
     GemmArgs t = a;
     t.first = a.count;
-    t.sub_m = r.tail_sub_m; t.sub_n = r.tail_sub_n;
-    t.count = r.tail_tiles * r.tail_sub_m * r.tail_sub_n;
-    return launch(t, a.BM, a.BN, 0);
+    t.sub_m = 256 / plan.tail_tm; t.sub_n = 256 / plan.tail_tn;
+    t.count = plan.tail * t.sub_m * t.sub_n;
+    return launch_tile(dtype, mode, t, plan.tail_tm, plan.tail_tn, s);
 }
 
 }  // namespace
@@ -143,7 +229,7 @@ int fo_main_tile_resident() {
     GemmArgs a = {};
     a.count = 1 << 30;
     int info[5] = {0, 0, 0, 0, 0};
-    if (launch_dtype<MODE_SIGNAL>(FO_F16, a, 256, 256, nullptr, info) != FO_OK || info[4] <= 0 || info[4] > 0xFFFF) {
+    if (launch_tile(FO_F16, MODE_SIGNAL, a, 256, 256, nullptr, info) != FO_OK || info[4] <= 0 || info[4] > 0xFFFF) {
         (void)hipGetLastError();
         return no_device;
     }
@@ -176,14 +262,15 @@ extern "C" int fo_gemm_wave_tiles(int dtype, int algo, int M, int N, int32_t *ti
     fo_raster r;
     int rc = fo_pick_raster(algo, M, N, &r);
     if (rc) return rc;
+    const launch_plan plan = plan_launch(r, M, N, e->f[0], e->f[1], false);
     GemmArgs a = {};
-    a.grid_m = r.grid_m;
-    a.grid_n = r.grid_n;
-    a.count = r.grid_m * r.grid_n - r.tail_tiles;
+    a.count = plan.count;
     int info[5] = {0, 0, 0, 0, 0};
-    rc = launch_dtype<MODE_SIGNAL>(dtype, a, r.mtm, r.mtn, nullptr, info);
+    rc = launch_tile(dtype, MODE_SIGNAL, a, plan.tm, plan.tn, nullptr, info);
     if (rc) return rc;
-    *tiles = info[0] * (r.mtm / e->f[0]) * (r.mtn / e->f[1]);
+    const long all = (long)(M / e->f[0]) * (N / e->f[1]);
+    const long wave = (long)info[0] * plan.tm * plan.tn / ((long)e->f[0] * e->f[1]);
+    *tiles = (int32_t)(!plan.whole || wave > all ? all : wave);
     return FO_OK;
 }
 
@@ -192,17 +279,13 @@ extern "C" int fo_gemm_kernel_info(int dtype, int algo, int M, int N, int epilog
     fo_raster r;
     int rc = fo_pick_raster(algo, M, N, &r);
     if (rc) return rc;
+    const fo_algo_entry *e = fo_algo_lookup(algo);
+    const launch_plan plan = plan_launch(r, M, N, e->f[0], e->f[1], false);
     GemmArgs a = {};
-    a.grid_m = r.grid_m;
-    a.grid_n = r.grid_n;
-    a.count = r.grid_m * r.grid_n - r.tail_tiles;
+    a.count = plan.count;
     int out[5] = {0, 0, 0, 0, 0};
-    switch (epilogue) {
-        case MODE_PLAIN: rc = launch_dtype<MODE_PLAIN>(dtype, a, r.mtm, r.mtn, nullptr, out); break;
-        case MODE_SIGNAL: rc = launch_dtype<MODE_SIGNAL>(dtype, a, r.mtm, r.mtn, nullptr, out); break;
-        case MODE_SCATTER: rc = launch_dtype<MODE_SCATTER>(dtype, a, r.mtm, r.mtn, nullptr, out); break;
-        default: return FO_ERR_ARG;
-    }
+    if (epilogue < MODE_PLAIN || epilogue > MODE_SCATTER) return FO_ERR_ARG;
+    rc = launch_tile(dtype, epilogue, a, plan.tm, plan.tn, nullptr, out);
     if (rc) return rc;
     for (int i = 0; i < 4; i++) info[i] = out[i];
     return FO_OK;

@@ -1,5 +1,5 @@
 // The 256x256 workgroup tile of the gfx950 MFMA GEMM (plain, signal and scatter
-// epilogues; same arguments, raster and epilogue semantics as fo_gemm_kernel.h,
+// epilogues; same arguments, raster and epilogue semantics as fo_gemm_tile_kernel.h,
 // whose reference citations hold here too:
 // src/overlap/gemm_with_signal.h:236-256, :291-361, src/overlap/gemm_scatter.cu:15-98).
 //
@@ -15,7 +15,7 @@
 // Operands travel HBM/L2 -> LDS directly (buffer_load_dwordx4 ... lds, 1 KiB per
 // wavefront instruction) into two slots of 64 KiB (BK = 64: 256 rows of A and
 // 256 of B, 128 bytes each, the 16-byte chunks XOR-swizzled by the choice of the
-// global chunk each lane fetches, exactly as in fo_gemm_kernel.h).  The buffer
+// global chunk each lane fetches, as in fo_gemm_tile_kernel.h).  The buffer
 // descriptor covers the tile's rows only, and the chunks of a last, partial K
 // step that lie beyond K are requested out of its range: the hardware writes
 // zeros for them, nothing outside A or B is ever addressed.
@@ -46,20 +46,9 @@
 // that wait and the counter update.
 #pragma once
 
-#include "fo_gemm_kernel.h"
+#include "fo_gemm_common.h"
 
 namespace fo_gemm_dev {
-
-typedef unsigned int fo_srd_t __attribute__((ext_vector_type(4)));  // buffer descriptor
-
-// 16 bytes per lane, global -> LDS: address = descriptor base + soff + voff (out of range: zeros),
-// LDS address = lds_addr + lane * 16 (through M0; the s_nop is the wait state between an M0 write and its use).
-__device__ __forceinline__ void dma_buf16(fo_srd_t srd, unsigned voff, unsigned soff, unsigned lds_addr) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :
-                 : "s"(lds_addr), "v"(voff), "s"(srd), "s"(soff)
-                 : "memory");
-}
 
 // The MFMAs of this kernel: accumulator in the accumulation registers, tied to the destination
 // (see fo_elem::mfma for why they are assembly); `go_load` carries a direct-to-LDS load in the
@@ -136,7 +125,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     const int KT = (p.K + BK - 1) / BK;
     const bool ktail = (p.K % BK) != 0;
 
-    // Fragment addressing as in fo_gemm_kernel.h: lane l supplies row l & 15, k-chunk l >> 4 of a 16x32 block.
+    // Fragment addressing as in fo_gemm_tile_kernel.h: lane l supplies row l & 15, k-chunk l >> 4 of a 16x32 block.
     const int frow = lane & 15, fk = lane >> 4;
     const int fkey = (frow >> 1) & 7;
     const unsigned la0 = smem_lds + (unsigned)((wm * 128 + frow) * 8 + (fk ^ fkey)) * 16;
@@ -162,30 +151,40 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
         soff_a[c] = __builtin_amdgcn_readfirstlane((unsigned)(c * 32 * p.lda * 2));
     }
 
+    // M and N are multiples of 128, not of 256: where half a tile is left at the end of a dimension, the tile is moved
+    // back by half its size, so that all of its operand rows exist; its first half there repeats the neighbour's
+    // product and is neither stored nor counted (p.half: bit 0 along M, bit 1 along N).
+    int half = p.half;
+    asm volatile("" : "+s"(half));  // in a register from here on: loaded again inside the K loop, it would turn every wait for LDS data into a wait for everything
+    // Coordinates of raster position t in halves of tiles, bits 0 and 1 of *repeated: which halves another tile
+    // computes (the upper rows, the left columns).
+    auto locate = [&](int t, int *pm_, int *pn_, int *repeated_) {
+        int qm, qn;
+        fo_wg_to_tile(t, p.grid_m, p.grid_n, p.panel, p.xcd_remap, &qm, &qn);
+        const int rep = __builtin_amdgcn_readfirstlane(half & ((qm == p.grid_m - 1 ? 1 : 0) | (qn == p.grid_n - 1 ? 2 : 0)));
+        *pm_ = __builtin_amdgcn_readfirstlane(2 * qm - (rep & 1));
+        *pn_ = __builtin_amdgcn_readfirstlane(2 * qn - (rep >> 1));
+        *repeated_ = rep;
+    };
+    int pm, pn, repeated;  // the first tile's are found once, for the loader, the slots and the tile itself
+    locate(blockIdx.x, &pm, &pn, &repeated);
+
     // Loader state: the stage being requested (it runs two K steps ahead of the MFMAs, across tiles).
     int ld_tile = blockIdx.x, ld_kt = 0;
     unsigned a_cur = (ktail && KT == 1) ? a_off_t : a_off;  // this stage's lane offsets, A and B alike
     fo_srd_t ra, rb;
-    auto make_srd = [&](const void *base, unsigned records) {
-        const uint64_t b = (uint64_t)(uintptr_t)base;
-        fo_srd_t r;
-        r.x = __builtin_amdgcn_readfirstlane((unsigned)b);
-        r.y = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32) & 0xFFFF);  // stride 0: raw buffer
-        r.z = __builtin_amdgcn_readfirstlane(records);
-        r.w = 0x00020000u;  // 32-bit data format, no swizzle
-        return r;
+    auto point_loader = [&](int pm_, int pn_) {
+        ra = fo_make_srd(p.A + (size_t)pm_ * 128 * p.lda, a_span);
+        rb = fo_make_srd(p.B + (size_t)pn_ * 128 * p.lda, a_span);
     };
     auto set_loader_tile = [&]() {
         if (ld_tile < ntiles) {
-            int pm_, pn_;
-            fo_unit_to_tile(ld_tile, p.first, p.sub_m, p.sub_n, p.grid_m, p.grid_n, p.panel, p.xcd_remap, &pm_, &pn_);
-            pm_ = __builtin_amdgcn_readfirstlane(pm_);
-            pn_ = __builtin_amdgcn_readfirstlane(pn_);
-            ra = make_srd(p.A + (size_t)pm_ * MT * p.lda, a_span);
-            rb = make_srd(p.B + (size_t)pn_ * MT * p.lda, a_span);
+            int pm_, pn_, rep_;
+            locate(ld_tile, &pm_, &pn_, &rep_);
+            point_loader(pm_, pn_);
         } else {
-            ra = make_srd(p.A, 0);  // behind the last tile: every load is out of range, nothing is fetched
-            rb = make_srd(p.B, 0);
+            ra = fo_make_srd(p.A, 0);  // behind the last tile: every load is out of range, nothing is fetched
+            rb = fo_make_srd(p.B, 0);
         }
     };
     auto advance_loader = [&]() {
@@ -229,7 +228,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
         }
     };
 
-    // ---- signalling state (signal and scatter epilogues), as in fo_gemm_kernel.h
+    // ---- signalling state (signal and scatter epilogues)
     const int sub_n = MT / p.BN, nsub = (MT / p.BM) * sub_n;  // reorder tiles per macro tile
     typedef const __attribute__((address_space(4))) int32_t *cptr_t;
     const cptr_t RAc = (cptr_t)(uintptr_t)p.RA;
@@ -300,7 +299,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                 if (q >= lane) count++;
             }
         }
-        if (lane < nsub) {
+        if (lane < nsub && g >= 0) {
             if (first) __hip_atomic_fetch_add(p.MM + g, count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (p.monitor) {
                 int o = __hip_atomic_fetch_add(p.MM + (p.TN - 1), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -313,15 +312,12 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     // tile's start: the round trip to memory then costs nothing, and no scalar load is pending at the K loop's head,
     // where it would turn every wait for LDS data into a wait for everything (scalar loads return out of order).
     int rs_next[kMaxSub] = {0, 0, 0, 0};
-    auto request_slots = [&](int t) {
+    auto request_slots = [&](int pm_, int pn_) {
         if (MODE != MODE_PLAIN) {
-            int tm_, tn_;
-            fo_unit_to_tile(t, p.first, p.sub_m, p.sub_n, p.grid_m, p.grid_n, p.panel, p.xcd_remap, &tm_, &tn_);
-            tm_ = __builtin_amdgcn_readfirstlane(tm_);
-            tn_ = __builtin_amdgcn_readfirstlane(tn_);
+            const int tm_ = pm_ >> (p.BM >> 8), tn_ = pn_ >> (p.BN >> 8);  // in reorder tiles (BM, BN: 128 or 256)
 #pragma unroll
             for (int s = 0; s < kMaxSub; s++)
-                if (s < nsub) rs_next[s] = RAc[(tm_ * (MT / p.BM) + s / sub_n) * p.TN + tn_ * sub_n + s % sub_n];
+                if (s < nsub) rs_next[s] = RAc[(tm_ + s / sub_n) * p.TN + tn_ + s % sub_n];
         }
     };
     // The slots that request_slots brought, as the rest of the kernel uses them: this wavefront's own reorder tile as a
@@ -352,8 +348,8 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     };
 
     // ---- pipeline fill: stage 0 -> slot 0, stage 1 -> slot 1; the loader then stands at stage 1
-    request_slots(blockIdx.x);
-    set_loader_tile();
+    request_slots(pm, pn);
+    point_loader(pm, pn);
 #pragma unroll
     for (int c = 0; c < 16; c++) load_chunk(c, 0);
     advance_loader();
@@ -371,10 +367,6 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     int tile = blockIdx.x;
     unsigned slot_b = 0;  // byte offset of the slot the next K step reads
     for (;;) {
-        int pm, pn;
-        fo_unit_to_tile(tile, p.first, p.sub_m, p.sub_n, p.grid_m, p.grid_n, p.panel, p.xcd_remap, &pm, &pn);
-        pm = __builtin_amdgcn_readfirstlane(pm);
-        pn = __builtin_amdgcn_readfirstlane(pn);
         if (tile == (int)blockIdx.x) take_slots();  // later tiles: taken inside the previous tile's epilogue
         // Scatter: the row map entries of the wavefront's 128 rows, two per lane (lane l: rows l and 64 + l), are
         // requested here and rest in two registers through the K loop; the epilogue hands them to the lanes that
@@ -494,7 +486,11 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
         fo_mfma_fence();
         const int next = tile + gridDim.x;
         const bool has_next = next < ntiles;
-        if (has_next) request_slots(next);
+        int next_pm = 0, next_pn = 0, next_repeated = 0;
+        if (has_next) {
+            locate(next, &next_pm, &next_pn, &next_repeated);
+            request_slots(next_pm, next_pn);
+        }
 
         int v_done = 0;  // the slots of the tile that this epilogue stores (per lane)
         // ---- epilogue.  A wavefront's 128x128 block lies inside one reorder tile (BM and BN are multiples of
@@ -510,11 +506,12 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             const int row0 = (wm * 128) % p.BM, col0 = (wn * 128) % p.BN;
             const int r = r_mine;
             const int v_cur = v_rs;  // this tile's slots: the next tile's replace them inside the loop below
-            const long trow = MODE == MODE_PLAIN ? (long)pm * MT + wm * 128 : (long)(r / p.rLDN) * p.BM + row0;
-            const long tcol = MODE == MODE_PLAIN ? (long)pn * MT + wn * 128 : (long)(r % p.rLDN) * p.BN + col0;
+            const long trow = MODE == MODE_PLAIN ? (long)(pm + wm) * 128 : (long)(r / p.rLDN) * p.BM + row0;
+            const long tcol = MODE == MODE_PLAIN ? (long)(pn + wn) * 128 : (long)(r % p.rLDN) * p.BN + col0;
             char *cbase = reinterpret_cast<char *>(p.C) + (trow * ldp + tcol) * 2;  // wave-uniform
             const unsigned lane_off = (unsigned)(srow * ldp + scol * 8) * 2;
             const bool stream_out = p.stream_out != 0;  // wave-uniform
+            const bool keep = !((repeated & 1) && wm == 0) && !((repeated & 2) && wn == 0);  // wave-uniform
 #pragma unroll
             for (int i = 0; i < F; i++) {  // 16 output rows = one row of accumulator blocks
                 __builtin_amdgcn_sched_barrier(0);
@@ -535,6 +532,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_s_waitcnt(0xC07F);
                 __builtin_amdgcn_wave_barrier();
+                if (keep)
 #pragma unroll
                 for (int ps = 0; ps < 16 / RPP; ps++) {
                     const int row = ps * RPP + srow;
@@ -572,11 +570,11 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
         }
 
         if (signalling) {
-            int v_g = 0;  // lane s: group of reorder tile s
+            int v_g = -1;  // lane s: group of reorder tile s, -1 where another workgroup tile counts it
             if (wave == 0) {
 #pragma unroll
                 for (int s = 0; s < kMaxSub; s++) {
-                    if (s < nsub) {
+                    if (s < nsub && !((repeated & 1) && s < sub_n) && !((repeated & 2) && s % sub_n == 0)) {
                         const int g = group_of(__builtin_amdgcn_readlane(v_done, s));
                         v_g = lane == s ? g : v_g;
                     }
@@ -601,6 +599,9 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
         }
         if (!has_next) break;
         tile = next;
+        pm = next_pm;
+        pn = next_pn;
+        repeated = next_repeated;
     }
     __builtin_amdgcn_s_waitcnt(0);  // nothing of this wavefront is in flight when it ends
 }

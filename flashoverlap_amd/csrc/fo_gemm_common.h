@@ -1,0 +1,147 @@
+// What the kernels of the gfx950 MFMA GEMM share: launch arguments, the group search, counted waits, stores and
+// the direct-to-LDS load.
+//
+//   C[M,N] = A[M,K] . B[N,K]^T   (both operands K-contiguous), fp32 accumulate.
+//
+// Replaces the CUTLASS kernels behind gemm_func_table / signal_func_table /
+// scatter_func_table of the reference (src/gemm/gemm.cu:23-110,
+// src/overlap/gemm_signal.cu:15-97, src/overlap/gemm_scatter.cu:15-98; epilogue
+// semantics src/overlap/gemm_with_signal.h:236-256, :291-361).
+//
+// Two kernels: fo_gemm256_kernel.h (256x256 workgroup tiles, four wavefronts, persistent) and
+// fo_gemm_tile_kernel.h (everything smaller).  Both use v_mfma_f32_16x16x32_{f16,bf16} over ascending K: in an
+// MFMA-only loop under this part's power limit that form sustains 14 % more than 32x32x16 (a quarter of the
+// accumulator registers per instruction, half of their traffic per flop), and large products are power-limited.
+#pragma once
+
+#include "fo_common.h"
+
+namespace fo_gemm_dev {
+
+enum { MODE_PLAIN = 0, MODE_SIGNAL = 1, MODE_SCATTER = 2 };
+
+struct GemmArgs {
+    const uint16_t *A;
+    const uint16_t *B;
+    uint16_t *C;
+    int M, N, K;
+    int lda, ldb;          // row strides of A and B in elements (multiples of 8)
+    int BM, BN, TN, rLDN;  // reorder/signal tile, tiles along N, reshaped width in tiles
+    const int32_t *RA;
+    const int32_t *RE;
+    const int32_t *cseg;
+    int G;
+    int32_t *MM;
+    int monitor;
+    int grid_m, grid_n, panel, xcd_remap;  // the raster of this launch's parent tiles
+    int first, sub_m, sub_n, count;        // this launch: positions from `first`, each cut into sub_m x sub_n macro tiles, `count` of them
+    int quiet;                             // signalling epilogues: store the tiles reordered, touch no counter
+    int half;                              // 256x256 kernel: half a tile is left at the end of M (bit 0), N (bit 1)
+    int stream_out;                        // 256x256 kernel: store the output with the non-temporal hint
+};
+
+constexpr int kMaxSub = 4;        // reorder tiles per macro tile (256x256 over 128x128)
+constexpr int kPrefixRegs = 256;  // group search on prefix sums held in registers (one per 64 groups) up to this many groups
+
+// Group of storage slot r: smallest g with cseg[0]+..+cseg[g] > r
+// (src/overlap/gemm_with_signal.h:343-349), found by one wavefront with a
+// 64-wide prefix sum per step instead of a serial scan.  All 64 lanes call it.
+__device__ __forceinline__ int find_group(const int32_t *cseg, int G, int r, int lane) {
+    int base = 0;
+    for (int it = 0; it < G; it += 64) {
+        int idx = it + lane;
+        int s = idx < G ? cseg[idx] : 0;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            int o = __shfl_up(s, d, 64);
+            if (lane >= d) s += o;
+        }
+        s += base;
+        unsigned long long hit = __ballot(idx < G && s > r);
+        if (hit) return it + (int)__builtin_ctzll(hit);
+        base = __shfl(s, 63, 64);
+    }
+    return G - 1;  // unreachable when sum(cseg) covers every slot (validated on the host)
+}
+
+// s_waitcnt vmcnt(n) only (expcnt/lgkmcnt left at their maxima); gfx9 encoding:
+// vmcnt = imm[15:14]:imm[3:0], expcnt = imm[6:4], lgkmcnt = imm[11:8].
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+    static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
+
+// 16-byte global stores written as assembly so that the number of vector memory
+// instructions in flight is known exactly (the main loop waits on vmcnt with
+// non-zero counts; the compiler does not see these instructions in its own
+// count, which can only make its waits longer, never shorter).  The
+// write-through form (system-scope cache policy) is used for the signalled
+// epilogues: the tile must be visible to other XCDs before its counter is
+// bumped, and a tile that never becomes dirty in L2 needs no releasing
+// write-back before the signal.  The trailing s_nop covers
+// the wait states gfx9 requires between a VMEM store of more than 8 bytes and a
+// VALU write of its data registers.
+__device__ __forceinline__ void store16_write_through(void *ptr, fo_u32x4 v) {
+    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" : : "v"(ptr), "v"(v) : "memory");
+}
+// saddr forms: wave-uniform base (SGPR pair) + 32-bit per-lane byte offset
+__device__ __forceinline__ void store16_write_through(char *base, unsigned lane_off, fo_u32x4 v) {
+    asm volatile("global_store_dwordx4 %0, %1, %2 sc0 sc1\n\ts_nop 1"
+                 :
+                 : "v"(lane_off), "v"(v), "s"((__attribute__((address_space(1))) char *)base)
+                 : "memory");
+}
+__device__ __forceinline__ void store16(char *base, unsigned lane_off, fo_u32x4 v) {
+    asm volatile("global_store_dwordx4 %0, %1, %2\n\ts_nop 1"
+                 :
+                 : "v"(lane_off), "v"(v), "s"((__attribute__((address_space(1))) char *)base)
+                 : "memory");
+}
+// The same with the non-temporal hint, for outputs too large to be found in a cache by whoever reads them
+// next (GemmArgs::stream_out): the resident workgroups finish their tiles together and store 128 KB each
+// at once, and output lines that took room in the L2 would push out the operand panels the next tile's
+// first K steps are about to share.  8192^3: GEMM alone 1.7 % faster, the overlapped step unchanged; on
+// the 8192x4096 output (67 MB), which the consumer finds in the memory-side cache, the hint made the
+// overlapped step 2 % and the serial step 8 % slower, so smaller outputs stay cacheable.
+__device__ __forceinline__ void store16_write_through_nt(void *ptr, fo_u32x4 v) {
+    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt\n\ts_nop 1" : : "v"(ptr), "v"(v) : "memory");
+}
+__device__ __forceinline__ void store16_write_through_nt(char *base, unsigned lane_off, fo_u32x4 v) {
+    asm volatile("global_store_dwordx4 %0, %1, %2 sc0 sc1 nt\n\ts_nop 1"
+                 :
+                 : "v"(lane_off), "v"(v), "s"((__attribute__((address_space(1))) char *)base)
+                 : "memory");
+}
+__device__ __forceinline__ void store16_nt(char *base, unsigned lane_off, fo_u32x4 v) {
+    asm volatile("global_store_dwordx4 %0, %1, %2 nt\n\ts_nop 1"
+                 :
+                 : "v"(lane_off), "v"(v), "s"((__attribute__((address_space(1))) char *)base)
+                 : "memory");
+}
+
+#define FO_LDS_PTR(p) ((__attribute__((address_space(3))) void *)(p))
+
+typedef unsigned int fo_srd_t __attribute__((ext_vector_type(4)));  // buffer descriptor
+
+// Raw buffer of `bytes` bytes at a wave-uniform address.
+__device__ __forceinline__ fo_srd_t fo_make_srd(const void *base, unsigned bytes) {
+    const uint64_t b = (uint64_t)(uintptr_t)base;
+    fo_srd_t r;
+    r.x = __builtin_amdgcn_readfirstlane((unsigned)b);
+    r.y = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32) & 0xFFFF);  // stride 0: raw buffer
+    r.z = __builtin_amdgcn_readfirstlane(bytes);
+    r.w = 0x00020000u;  // 32-bit data format, no swizzle
+    return r;
+}
+
+// 16 bytes per lane, global -> LDS: address = descriptor base + soff + voff (out of range: zeros),
+// LDS address = lds_addr + lane * 16 (through M0; the s_nop is the wait state between an M0 write and its use).
+__device__ __forceinline__ void dma_buf16(fo_srd_t srd, unsigned voff, unsigned soff, unsigned lds_addr) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds_addr), "v"(voff), "s"(srd), "s"(soff)
+                 : "memory");
+}
+
+}  // namespace fo_gemm_dev

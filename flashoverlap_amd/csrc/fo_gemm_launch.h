@@ -1,11 +1,11 @@
 // Launch of one compiled GEMM kernel, shared by the translation units that hold
-// kernel instantiations (fo_gemm.hip, fo_gemm256_inst.hip).
+// kernel instantiations (fo_gemm256_inst.hip, fo_gemm_tile_inst.hip).
 #pragma once
 
 #include <atomic>
 #include <mutex>
 
-#include "fo_gemm_kernel.h"
+#include "fo_gemm_common.h"
 
 namespace fo_gemm_dev {
 
@@ -87,5 +87,15 @@ int fo_gemm256_launch(int dtype, int mode, const GemmArgs &a, hipStream_t stream
 FO_GEMM256_INST_DECL(0, 0) FO_GEMM256_INST_DECL(0, 1) FO_GEMM256_INST_DECL(0, 2)
 FO_GEMM256_INST_DECL(1, 0) FO_GEMM256_INST_DECL(1, 1) FO_GEMM256_INST_DECL(1, 2)
 #undef FO_GEMM256_INST_DECL
+
+// The smaller tiles (fo_gemm_tile_kernel.h), the same way (fo_gemm_tile_inst.hip); FO_ERR_ALGO for a tile that is not built.
+int fo_gemm_tile_launch(int dtype, int mode, const GemmArgs &a, int tm, int tn, hipStream_t stream, int *resident_out,
+                        int expect_resident);
+#define FO_GEMM_TILE_INST_DECL(D_, M_)                                                                              \
+    int fo_gemm_tile_launch_##D_##_##M_(const GemmArgs &a, int tm, int tn, hipStream_t stream, int *resident_out, \
+                                        int expect_resident);
+FO_GEMM_TILE_INST_DECL(0, 0) FO_GEMM_TILE_INST_DECL(0, 1) FO_GEMM_TILE_INST_DECL(0, 2)
+FO_GEMM_TILE_INST_DECL(1, 0) FO_GEMM_TILE_INST_DECL(1, 1) FO_GEMM_TILE_INST_DECL(1, 2)
+#undef FO_GEMM_TILE_INST_DECL
 
 }  // namespace fo_gemm_dev

@@ -1,0 +1,43 @@
+// The instantiations of the smaller-tile GEMM kernel for one type and one epilogue per translation unit: built
+// six times with -DFO_INST_DTYPE={0,1} (fp16, bf16) and -DFO_INST_MODE={0,1,2} (plain, signal, scatter epilogue).
+#include "fo_gemm_launch.h"
+#include "fo_gemm_tile_kernel.h"
+
+#if !defined(FO_INST_DTYPE) || !defined(FO_INST_MODE)
+#error "compile with -DFO_INST_DTYPE=0|1 -DFO_INST_MODE=0|1|2"
+#endif
+
+namespace fo_gemm_dev {
+
+#define FO_CAT3_(a, b, c, d) a##b##c##d
+#define FO_CAT3(a, b, c, d) FO_CAT3_(a, b, c, d)
+
+#if FO_INST_DTYPE == 0
+typedef fo_f16_tag inst_tag;
+#else
+typedef fo_bf16_tag inst_tag;
+#endif
+
+// Columns per stage and slots of each tile: as many operand bytes in flight as 160 KB of LDS hold (96 to 128 KB),
+// in steps of 128 columns where a tile's step of 64 is too short to hide a barrier in.
+int FO_CAT3(fo_gemm_tile_launch_, FO_INST_DTYPE, _, FO_INST_MODE)(const GemmArgs &a, int tm, int tn, hipStream_t stream,
+                                                              int *resident_out, int expect_resident) {
+#define FO_TILE(TM_, TN_, BK_, S_)                                                                                       \
+    if (tm == TM_ && tn == TN_)                                                                                          \
+        return launch_kernel<fo_gemm_tile_kernel<inst_tag, TM_, TN_, BK_, S_, FO_INST_MODE>,                             \
+                             tile_smem_bytes<TM_, TN_, BK_, S_>(), kTileThreads>(a, stream, resident_out, expect_resident);
+    FO_TILE(32, 32, 128, 8)
+    FO_TILE(64, 32, 128, 6)
+    FO_TILE(64, 64, 128, 4)
+    FO_TILE(64, 96, 128, 3)
+    FO_TILE(64, 128, 128, 3)
+    FO_TILE(96, 128, 64, 5)
+    FO_TILE(128, 128, 64, 4)
+    FO_TILE(128, 192, 64, 3)
+    FO_TILE(128, 256, 64, 3)
+    FO_TILE(256, 128, 64, 3)
+#undef FO_TILE
+    return FO_ERR_ALGO;
+}
+
+}  // namespace fo_gemm_dev

@@ -1,0 +1,331 @@
+// The workgroup tiles from 32x32 to 128x256 / 256x128 of the gfx950 MFMA GEMM (plain, signal and scatter
+// epilogues): problems that do not fill the chip with 256x256 tiles, the remainder of a last wave of those,
+// and sizes that 256 does not divide.  Arguments, raster and epilogue semantics are those of fo_gemm_common.h
+// (its reference citations hold here too), and every product is summed in the same order (ascending K,
+// 32 columns per MFMA) whatever the tile, so all shapes give the same bits.
+//
+// What bounds these sizes is not the matrix pipe but getting operands to it: a CU takes 64 bytes per clock
+// from its L2 (152 GB/s measured on one CU, 130 with all of them loading), returned in order, so that a load
+// that misses the L2 holds up the hits behind it, and a wavefront that presents loads faster than they drain
+// stands still with its MFMAs behind them.  The workgroup is therefore split in two roles, four wavefronts
+// each: loaders, which do nothing but move operand stages HBM/L2 -> LDS (buffer_load_dwordx4 ... lds) up to
+// S - 1 stages ahead and may stand still as long as they like, and computing wavefronts, which touch nothing
+// but LDS and the matrix pipe.  One barrier per K step (BK columns), placed near the start of the step's last MFMA
+// group: it says that the step's slot has been read by everyone (the loaders refill it next) and that the
+// next stage has landed, so its first fragments are fetched behind that last group's MFMAs.  Fragment
+// fetches are spread between MFMAs (k_step below): issued as one burst in front of them, all
+// wavefronts burst together behind the barrier and the matrix pipe waits for the LDS.
+//
+// Measured against the kernel this one replaced (loads issued by the computing wavefronts; fp16, GEMM alone,
+// operands of three buffer sets in turn): 512x4096x4096 39.1 -> 21 us, 256x8192x3584 35.5 -> 19.5,
+// 128x4096x1024 10.4 -> 4.5, 128x1024x8192 71 -> 12.5, 2048x4096x4096 62 -> 55.  512x4096x4096 with the MFMAs taken
+// out takes 18.7 us: the rest of its time is the operand stream.
+#pragma once
+
+#include "fo_gemm_common.h"
+
+namespace fo_gemm_dev {
+
+template <typename Tag> struct fo_mfma16;
+template <> struct fo_mfma16<fo_f16_tag> {
+    typedef fo_half8 frag;
+    static __device__ __forceinline__ fo_float4v go(frag a, frag b, fo_float4v c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+    }
+};
+template <> struct fo_mfma16<fo_bf16_tag> {
+    typedef fo_bf8 frag;
+    static __device__ __forceinline__ fo_float4v go(frag a, frag b, fo_float4v c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+    }
+};
+
+constexpr int kTileLoaders = 4, kTileComputers = 4, kTileThreads = (kTileLoaders + kTileComputers) * 64;
+
+// S operand slots; the output tile is staged in the same space once the K loop is done.
+template <int TM, int TN, int BK, int S>
+constexpr int tile_smem_bytes() {
+    return S * (TM + TN) * BK * 2 > TM * (TN + 8) * 2 ? S * (TM + TN) * BK * 2 : TM * (TN + 8) * 2;
+}
+
+template <typename Tag, int TM, int TN, int BK, int S, int MODE>
+__global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs p) {
+    typedef fo_elem<Tag> E;
+    typedef fo_mfma16<Tag> X;
+    typedef typename X::frag frag;
+    constexpr int NL = kTileLoaders, KB = BK / 64, KK = BK / 32;  // 64-column blocks and MFMA k-steps per stage
+    constexpr int WTM = TM / 2, WTN = TN / 2, FM = WTM / 16, FN = WTN / 16;  // computing wavefronts: 2 x 2
+    constexpr int PA = TM / 8 / NL, PB = TN / 8 / NL, P = KB * (PA + PB);    // 1 KiB loads per loader and stage
+    constexpr unsigned A_BLK = TM * 128, B_BLK = TN * 128, STAGE = KB * (A_BLK + B_BLK);
+    constexpr int PITCH = TN + 8, CPR = TN / 8, NCH = (TM * CPR + kTileThreads - 1) / kTileThreads;  // output staging
+    static_assert(BK % 64 == 0 && TM % 32 == 0 && TN % 32 == 0, "whole 1 KiB loads for every loader");
+    static_assert(S >= 2 && (S - 1) * P < 64, "vmcnt range");
+
+    extern __shared__ fo_u32x4 smem[];
+    __shared__ int32_t row_map[MODE == MODE_SCATTER ? 256 : 1];  // scatter: where the tile's rows go
+    const unsigned lds0 = (unsigned)(uintptr_t)FO_LDS_PTR(smem);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool loader = wave_id < NL;
+    const int wave = loader ? wave_id : wave_id - NL;
+    const int wm = wave >> 1, wn = wave & 1;
+    const int KT = (p.K + BK - 1) / BK;
+
+    const int bm_shift = p.BM == 256 ? 8 : 7, bn_shift = p.BN == 256 ? 8 : 7;  // reorder tiles: 128 or 256 each way
+    const int ldp = MODE == MODE_PLAIN ? p.N : p.rLDN * p.BN;  // leading dimension of the output view
+    const bool signalling = MODE != MODE_PLAIN && !p.quiet;
+    typedef const __attribute__((address_space(4))) int32_t *cptr_t;  // read-only for the whole launch: scalar loads
+    const cptr_t RAc = (cptr_t)(uintptr_t)p.RA;
+
+    for (int tile = blockIdx.x; tile < p.count; tile += gridDim.x) {
+        int pm, pn;
+        fo_unit_to_tile(tile, p.first, p.sub_m, p.sub_n, p.grid_m, p.grid_n, p.panel, p.xcd_remap, &pm, &pn);
+        pm = __builtin_amdgcn_readfirstlane(pm);
+        pn = __builtin_amdgcn_readfirstlane(pn);
+        if (pm * TM >= p.M || pn * TN >= p.N) continue;  // cut from a 256x256 position that reaches beyond the matrix
+        // Where the dimension ends inside the tile, the tile is moved back so that all of its operand rows exist; the
+        // rows or columns it then shares with its neighbour are neither stored nor counted.
+        const int m0 = pm * TM + TM > p.M ? p.M - TM : pm * TM, n0 = pn * TN + TN > p.N ? p.N - TN : pn * TN;
+        const int skip_m = pm * TM - m0, skip_n = pn * TN - n0;
+        // The tile lies in one reorder tile or in two, one above or beside the other; the second begins at row split_m
+        // or column split_n.  r0, r1: their storage slots.
+        int r0 = 0, r1 = 0;
+        bool two_m = false, two_n = false;
+        int split_m = TM, split_n = TN;
+        if (MODE != MODE_PLAIN) {
+            const int tm0 = m0 >> bm_shift, tn0 = n0 >> bn_shift;
+            two_m = (m0 + TM - 1) >> bm_shift != tm0;
+            two_n = (n0 + TN - 1) >> bn_shift != tn0;
+            if (two_m) split_m = ((tm0 + 1) << bm_shift) - m0;
+            if (two_n) split_n = ((tn0 + 1) << bn_shift) - n0;
+            r0 = RAc[tm0 * p.TN + tn0];
+            r1 = two_m || two_n ? RAc[(tm0 + two_m) * p.TN + tn0 + two_n] : r0;
+        }
+        // Row of the output view that the tile's row 0 has (or would have) in storage slot r, and the same for columns.
+        auto row_base = [&](int r, int rldn, bool second) __attribute__((always_inline)) {
+            return (r / rldn << bm_shift) + (second && two_m ? -split_m : m0 & (p.BM - 1));
+        };
+        auto col_base = [&](int r, int rldn, bool second) __attribute__((always_inline)) {
+            return (r % rldn << bn_shift) + (second && two_n ? -split_n : n0 & (p.BN - 1));
+        };
+
+        fo_float4v acc[FM][FN];
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++) acc[i][j] = fo_float4v{0.f, 0.f, 0.f, 0.f};
+        int g0 = 0, g1 = 0;  // groups of r0 and r1 (the wavefront that signals)
+
+        if (loader) {
+            // Load u of a 64-column block brings rows (u * NL + wave) * 8 + lane / 8 of an operand, 128 bytes each; LDS
+            // slot `lane` of the 1 KiB block is (row lane / 8, chunk lane % 8) and receives chunk phys ^ key(row).
+            const int lrow = lane >> 3, lchunk = (lane & 7) ^ (((wave * 8 + lrow) >> 1) & 7);
+            const unsigned lane_off = (unsigned)((wave * 8 + lrow) * p.lda * 2 + lchunk * 16);
+            const unsigned row_step = (unsigned)(NL * 8 * p.lda * 2);
+            const fo_srd_t ra = fo_make_srd(p.A + (size_t)m0 * p.lda, (unsigned)TM * p.lda * 2);
+            const fo_srd_t rb = fo_make_srd(p.B + (size_t)n0 * p.ldb, (unsigned)TN * p.ldb * 2);
+            const unsigned wave_lds = lds0 + wave * 1024;
+            auto request = [&](int kt, unsigned slot_v) __attribute__((always_inline)) {
+                const unsigned slot = __builtin_amdgcn_readfirstlane(slot_v);  // uniform by construction; said so for the assembly's operands
+#pragma unroll
+                for (int kb = 0; kb < KB; kb++) {
+                    const int col = __builtin_amdgcn_readfirstlane(kt * BK + kb * 64);
+                    // chunks beyond K (a partial last step, stages behind the last) are requested out of range: zeros
+                    const unsigned voff = lchunk * 8 < p.K - col ? lane_off : 0x80000000u;
+#pragma unroll
+                    for (int u = 0; u < PB; u++)
+                        dma_buf16(rb, voff, __builtin_amdgcn_readfirstlane(u * row_step + col * 2), wave_lds + slot + KB * A_BLK + kb * B_BLK + u * NL * 1024);
+#pragma unroll
+                    for (int u = 0; u < PA; u++)
+                        dma_buf16(ra, voff, __builtin_amdgcn_readfirstlane(u * row_step + col * 2), wave_lds + slot + kb * A_BLK + u * NL * 1024);
+                }
+            };
+            __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+            for (int s = 0; s < S - 1; s++) request(s, s * STAGE);
+            wait_vmcnt<(S - 2) * P>();  // stage 0 has landed (vmcnt retires in issue order)
+            __builtin_amdgcn_s_barrier();
+            unsigned slot = (S - 1) * STAGE;
+            for (int kt = 0; kt < KT; kt++) {
+                request(kt + S - 1, slot);  // the slot of stage kt - 1, given up at the last barrier
+                slot = slot + STAGE == S * STAGE ? 0 : slot + STAGE;
+                wait_vmcnt<(S - 2) * P>();  // stage kt + 1
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+            }
+            wait_vmcnt<0>();  // nothing lands in the space the output is staged in
+        } else {
+            // Fragment addressing: lane l supplies row l & 15, k-chunk l >> 4 of a 16x32 block.  The operand of which a
+            // wavefront holds more fragments is the long one: a k-step goes through it fragment by fragment (a "row"),
+            // each with all fragments of the short one.
+            constexpr bool LONG_B = FN > FM;
+            constexpr int FL = LONG_B ? FN : FM, FS = LONG_B ? FM : FN;
+            constexpr unsigned L_BLK = LONG_B ? B_BLK : A_BLK, S_BLK = LONG_B ? A_BLK : B_BLK;
+            const int frow = lane & 15, fk = lane >> 4, key = (frow >> 1) & 7;
+            const unsigned la = lds0 + (unsigned)((wm * WTM + frow) * 8 + (fk ^ key)) * 16;
+            const unsigned lb = lds0 + KB * A_BLK + (unsigned)((wn * WTN + frow) * 8 + (fk ^ key)) * 16;
+            const unsigned l_lds = LONG_B ? lb : la, s_lds = LONG_B ? la : lb;
+            typedef const __attribute__((address_space(3))) frag *lds_frag_t;
+            // Two sets of short fragments take turns.  Long ones: two sets as well, or, from four on, one set whose
+            // members are replaced right behind the row that used them (two full sets beside 128 accumulators would
+            // leave no room for a consumer's wavefront on the SIMD).
+            constexpr bool RING = FL >= 4;
+            constexpr int MEET = RING ? 1 : 0;  // the barrier stands in front of this row of the step's last k-step
+            frag lf[RING ? 1 : 2][FL], sf[2][FS];
+            auto fetch_l = [&](int kk, unsigned slot, int i) __attribute__((always_inline)) {
+                const unsigned at = (l_lds + slot + (kk >> 1) * L_BLK) ^ ((kk & 1) * 64);
+                lf[RING ? 0 : kk & 1][i] = *(lds_frag_t)(uintptr_t)(at + i * 2048);
+            };
+            auto fetch_s = [&](int kk, unsigned slot, int j) __attribute__((always_inline)) {
+                const unsigned at = (s_lds + slot + (kk >> 1) * S_BLK) ^ ((kk & 1) * 64);
+                sf[kk & 1][j] = *(lds_frag_t)(uintptr_t)(at + j * 2048);
+            };
+            // k-step kk with the fetches of the next one (the first of the next slot behind the last) spread over its
+            // rows from `from` on, the earlier ones a little denser: what is fetched last is needed soon.
+            auto k_step = [&](int kk, unsigned slot, unsigned next) __attribute__((always_inline)) {
+                const bool last = kk == KK - 1;
+                const int from = last ? MEET : 0;
+                const int nkk = last ? 0 : kk + 1;
+                int l_done = 0, s_done = 0;
+#pragma unroll
+                for (int i = 0; i < FL; i++) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (last && i == MEET) {
+                        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wavefront's fetches from the slot have returned
+                        __builtin_amdgcn_s_barrier();
+                        asm volatile("" ::: "memory");
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+#pragma unroll
+                    for (int j = 0; j < FS; j++) {
+                        if constexpr (LONG_B)
+                            acc[j][i] = X::go(lf[RING ? 0 : kk & 1][i], sf[kk & 1][j], acc[j][i]);
+                        else
+                            acc[i][j] = X::go(sf[kk & 1][j], lf[RING ? 0 : kk & 1][i], acc[i][j]);
+                    }
+                    if (i >= from) {
+                        const int by_now = (i - from + 1) * (FL + FS) * 4 / (3 * (FL - from)) - (i + 1);
+                        const int s_to = by_now < 0 ? 0 : i == FL - 1 || by_now > FS ? FS : by_now;
+                        const int n = i + 1 - l_done + s_to - s_done;
+#pragma unroll
+                        for (int q = 0; q < FS; q++)
+                            if (q >= s_done && q < s_to) fetch_s(nkk, last ? next : slot, q);
+#pragma unroll
+                        for (int q = 0; q < FL; q++)
+                            if (q >= l_done && q <= i) fetch_l(nkk, last ? next : slot, q);
+                        l_done = i + 1;
+                        s_done = s_to;
+#pragma unroll
+                        for (int t = 0; t < FL + FS; t++) {
+                            if (t < n) {
+                                const int m = (t + 1) * FS / n - t * FS / n;  // MFMAs in front of this fetch
+                                if (m == 1) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                                if (m == 2) __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                                if (m == 3) __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+                                if (m >= 4) __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+                                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                            }
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            __builtin_amdgcn_s_setprio(2);
+            // While the first stage is on its way: row map entries, and the groups to signal.
+            if (MODE == MODE_SCATTER) {
+                const int e = wave * 64 + lane;  // row e, or (two reorder tiles side by side) row e % TM of one of them
+                if (e < (two_n ? 2 * TM : TM)) {
+                    const int row = two_n && e >= TM ? e - TM : e;
+                    const bool second = two_n ? e >= TM : row >= split_m;
+                    row_map[e] = p.RE[row_base(second ? r1 : r0, p.rLDN, second) + row];
+                }
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): written when the first barrier is passed
+            }
+            if (signalling && wave == 0) {
+                g0 = find_group(p.cseg, p.G, r0, lane);
+                g1 = r1 != r0 ? find_group(p.cseg, p.G, r1, lane) : g0;
+            }
+            unsigned slot = 0;
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int j = 0; j < FS; j++) fetch_s(0, 0, j);
+#pragma unroll
+            for (int i = 0; i < FL; i++) fetch_l(0, 0, i);
+            for (int kt = 0; kt < KT; kt++) {
+                const unsigned next = slot + STAGE == S * STAGE ? 0 : slot + STAGE;
+#pragma unroll
+                for (int kk = 0; kk < KK; kk++) k_step(kk, slot, next);  // the last one fetches from the next slot: behind the last stage, zeros never used
+                slot = next;
+            }
+            __builtin_amdgcn_s_waitcnt(0xC07F);
+        }
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+
+        // ---- epilogue: accumulators -> 16 bit -> LDS -> 16-byte pieces of output rows, by all eight wavefronts
+        // (the thread id is laundered so that this addressing is computed here instead of resting in registers across
+        // the K loop)
+        int et = tid;
+        asm volatile("" : "+v"(et));
+        uint16_t *stage = reinterpret_cast<uint16_t *>(smem);
+        if (!loader) {
+            const int erow = et & 15, ek = (et & 63) >> 4;  // accumulator block: row erow, columns 4*ek .. 4*ek+3
+#pragma unroll
+            for (int i = 0; i < FM; i++)
+#pragma unroll
+                for (int j = 0; j < FN; j++) {
+                    fo_u32x2 v;
+                    v.x = (uint32_t)E::from_f32(acc[i][j][0]) | ((uint32_t)E::from_f32(acc[i][j][1]) << 16);
+                    v.y = (uint32_t)E::from_f32(acc[i][j][2]) | ((uint32_t)E::from_f32(acc[i][j][3]) << 16);
+                    *reinterpret_cast<fo_u32x2 *>(stage + (wm * WTM + i * 16 + erow) * PITCH + wn * WTN + j * 16 + ek * 4) = v;
+                }
+        }
+        int rldn = p.rLDN;
+        asm volatile("" : "+s"(rldn));  // the divisions by it too
+        int row0 = 0, row1 = 0, col0 = 0, col1 = 0;
+        if (MODE != MODE_PLAIN) {
+            row0 = row_base(r0, rldn, false);
+            col0 = col_base(r0, rldn, false);
+            row1 = row_base(r1, rldn, true);
+            col1 = col_base(r1, rldn, true);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < NCH; u++) {
+            const int idx = u * kTileThreads + et, row = idx / CPR, col = idx % CPR * 8;
+            // piece u of a thread: columns 8 * (idx % CPR) of row idx / CPR
+            if ((TM * CPR % kTileThreads == 0 || row < TM) && row >= skip_m && col >= skip_n) {
+                const fo_u32x4 v = *reinterpret_cast<const fo_u32x4 *>(stage + row * PITCH + col);
+                if constexpr (MODE == MODE_PLAIN) {
+                    *reinterpret_cast<fo_u32x4 *>(p.C + (size_t)(m0 + row) * ldp + n0 + col) = v;
+                } else {
+                    const bool second = row >= split_m || col >= split_n;
+                    const int to_row = MODE == MODE_SCATTER ? row_map[two_n && second ? TM + row : row] : (second ? row1 : row0) + row;
+                    store16_write_through(p.C + (size_t)to_row * ldp + (second ? col1 : col0) + col, v);
+                }
+            }
+        }
+        if (signalling) {
+            // Whole reorder tiles only (the launcher sees to it): every wavefront's write-through stores are
+            // acknowledged, the barrier collects the workgroup, then the counters move (the reference has no fence
+            // here, src/overlap/gemm_with_signal.h:337-351).
+            __builtin_amdgcn_s_waitcnt(0);
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            const bool first_counts = skip_m < split_m && skip_n < split_n;
+            if (wave_id == NL && ((lane == 0 && first_counts) || (lane == 1 && (two_m || two_n)))) {
+                const int g = lane ? g1 : g0, r = lane ? r1 : r0;
+                __hip_atomic_fetch_add(p.MM + g, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (p.monitor) {
+                    int o = __hip_atomic_fetch_add(p.MM + (p.TN - 1), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(p.MM + p.TN + r, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+        }
+        if (tile + (int)gridDim.x < p.count) __syncthreads();  // the staged tile has been read by everyone
+    }
+}
+
+}  // namespace fo_gemm_dev

@@ -1,0 +1,84 @@
+"""GPU parity of every workgroup tile of the GEMM at the sizes where it can go wrong: tiles moved back at the end of
+a dimension, tiles that lie across two reorder tiles, partial last K steps, one K step, the second launch over the
+last wave's positions.  The plain product against torch in fp32; the reordered store (row-mapped as well) bit for
+bit against the plain product through the inverse permutation; counters and stamps exact."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import BF16, F16, TORCH_DTYPE, max_rel_err, seeded
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # dtype, reorder tile, M, N, K                workgroup tile
+    (F16, 128, 128, 128, 256, 8),                      # 32x32, one chunk of K
+    (BF16, 128, 256, 256, 1024, 1544),                 # 32x32, parts of a 128x256 reorder tile, counted behind the launch
+    (F16, 128, 128, 128, 3072, 136),                   # 64x32
+    (BF16, 256, 128, 256, 2944, 1672),                 # 64x64
+    (F16, 128, 128, 384, 3200, 200),                   # 64x96, across reorder tiles and moved back along N
+    (BF16, 128, 256, 256, 5632, 1608),                 # 64x96 over 256-wide reorder tiles
+    (F16, 128, 128, 512, 3456, 1600),                  # 64x128
+    (BF16, 128, 128, 1408, 1536, 328),                 # 96x128, moved back along M
+    (F16, 256, 128, 1536, 1408, 1544),                 # 96x128 over 256-high reorder tiles
+    (F16, 128, 128, 2560, 1280, 64),                   # 128x128, one K step
+    (BF16, 128, 128, 1920, 2560, 136),                 # 128x192, moved back along N
+    (F16, 256, 128, 2048, 2432, 1600),                 # 128x192, half of each 256-high reorder tile
+    (F16, 128, 128, 3968, 1920, 72),                   # 128x256, moved back along N
+    (BF16, 256, 128, 3840, 1920, 192),                 # 256x128
+    (F16, 128, 128, 4224, 3200, 136),                  # 256x256, half a tile left along both
+    (BF16, 128, 256, 4224, 3328, 72),                  # 256x256, half a tile left along M
+    (BF16, 128, 128, 4224, 4352, 264),                 # 256x256 and a second launch for the last wave
+]
+
+
+@pytest.mark.parametrize("dtype,bm,bn,M,N,K", CASES)
+def test_workgroup_tiles(fo, dtype, bm, bn, M, N, K):
+    ops, layout, td = fo.ops, fo.layout, TORCH_DTYPE[dtype]
+    algo = fo._capi.find_algo(bm, bn, swizzle=4)
+    TM, TN = M // bm, N // bn
+    T = TM * TN
+    A, _ = seeded((M, K), dtype, M + K)
+    B, _ = seeded((N, K), dtype, N + K, scale=K ** -0.5)
+    plain = torch.full((M, N), float("nan"), device="cuda", dtype=td)
+    ops.gemm(A, B, plain, algo)
+    assert max_rel_err(plain.float(), A.float() @ B.float().T) <= 1e-2
+    rng = np.random.default_rng(M + N)
+    RA = torch.from_numpy(rng.permutation(T).astype(np.int32)).reshape(TM, TN).cuda()
+    cseg = [T] if T < 3 else [1, T // 2, T - 1 - T // 2]
+    cs_cpu = torch.tensor(cseg, dtype=torch.int32)
+    cs_gpu = cs_cpu.cuda()
+    RE = layout.generate_row_mapping(M, N, bm, bn, cseg, 2)
+    Cp = torch.empty(M * N, device="cuda", dtype=td)
+
+    def check(what, RE=None, rLDN=1):
+        torch.cuda.synchronize()
+        assert torch.equal(layout.unpermute(Cp, M, N, bm, bn, RA, rLDN=rLDN, RE=RE), plain), what
+        Cp.fill_(float("nan"))
+
+    Cp.fill_(float("nan"))
+    # with counters
+    MM = torch.zeros(layout.counter_size(len(cseg), TM, TN), dtype=torch.int32, device="cuda")
+    for re, rldn in ((None, 1), (RE, 1), (None, 2 if T % 2 == 0 else 1)):
+        ops.gemm_signal(A, B, Cp, MM, RA, cs_gpu, algo, rLDN=rldn, RE=re)
+        check("signalled", re, rldn)
+        assert MM[:len(cseg)].tolist() == cseg and (MM[len(cseg):] == 0).all()
+        MM.zero_()
+    if len(cseg) <= TN - 1:  # monitor: its order counter lives at MM[TN - 1]
+        MMm = torch.zeros(layout.counter_size(len(cseg), TM, TN, True), dtype=torch.int32, device="cuda")
+        ops.gemm_signal(A, B, Cp, MMm, RA, cs_gpu, algo, monitor=True)
+        check("monitored")
+        mm = MMm.cpu()
+        assert mm[:len(cseg)].tolist() == cseg and mm[TN - 1] == T
+        assert sorted(mm[TN:TN + T].tolist()) == list(range(T))
+    # without (a call that stays on one stream)
+    ov = ops.Overlap(world=2)
+    ov.set_schedule(in_stream_below_flop=1e15)
+    ov.gemm_allreduce_overlap(A, B, Cp, MM, RA, 1, cs_cpu, cs_gpu, algo)
+    check("on one stream")
+    D = torch.empty(M // 2, N, device="cuda", dtype=td)
+    ov.gemm_reducescatter_overlap(A, B, Cp, D, MM, RA, RE, 1, cs_cpu, cs_gpu, algo)
+    torch.cuda.synchronize()
+    assert torch.equal(layout.unpermute(D.reshape(-1), M // 2, N, bm // 2, bn, RA), plain[0::2])
+    check("on one stream, row-mapped", RE)
+    assert (MM == 0).all()
+    ov.close()
