@@ -68,19 +68,6 @@ __global__ __launch_bounds__(WAIT_GROUPS_THREADS) void fo_wait_groups_kernel(int
 }
 
 // ------------------------------------------------------------------ consumer
-template <typename Tag>
-__device__ __forceinline__ fo_u32x4 add8(fo_u32x4 a, fo_u32x4 b) {
-    typedef fo_elem<Tag> E;
-    uint32_t x[4] = {a.x, a.y, a.z, a.w}, y[4] = {b.x, b.y, b.z, b.w}, o[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        float lo = E::to_f32((uint16_t)(x[i] & 0xffff)) + E::to_f32((uint16_t)(y[i] & 0xffff));
-        float hi = E::to_f32((uint16_t)(x[i] >> 16)) + E::to_f32((uint16_t)(y[i] >> 16));
-        o[i] = (uint32_t)E::from_f32(lo) | ((uint32_t)E::from_f32(hi) << 16);
-    }
-    return fo_u32x4{o[0], o[1], o[2], o[3]};
-}
-
 // The consumer runs beside the GEMM, whose workgroups each need most of a CU's
 // LDS and registers.  It therefore uses few, thin workgroups (256 lanes, no LDS,
 // a register budget that fits next to two GEMM wavefronts per SIMD) and gets
@@ -148,7 +135,7 @@ __device__ __forceinline__ void reduce_range(const fo_u32x4 *src, fo_u32x4 *dst,
 #pragma unroll
         for (int u = 0; u < U; u++) {
             fo_u32x4 *d = where(i + (long)u * nthreads);
-            const fo_u32x4 v = add8<Tag>(b[u], a[u]);
+            const fo_u32x4 v = fo_add8<Tag>(b[u], a[u]);
             if (STREAM)
                 __builtin_nontemporal_store(v, d);
             else
@@ -161,7 +148,7 @@ __device__ __forceinline__ void reduce_range(const fo_u32x4 *src, fo_u32x4 *dst,
         if (first + tid < hi) {
             fo_u32x4 *d = where(first + tid);
             const fo_u32x4 a = fetch(first, 0);
-            const fo_u32x4 v = add8<Tag>(STREAM ? __builtin_nontemporal_load(d) : *d, a);
+            const fo_u32x4 v = fo_add8<Tag>(STREAM ? __builtin_nontemporal_load(d) : *d, a);
             if (STREAM)
                 __builtin_nontemporal_store(v, d);
             else

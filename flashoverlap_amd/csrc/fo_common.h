@@ -68,6 +68,21 @@ template <> struct fo_elem<fo_bf16_tag> {
     }
 };
 
+// 16-bit sums of eight elements, each in fp32 and rounded once: what the consumer does to the accumulator.
+template <typename Tag>
+static __device__ __forceinline__ fo_u32x4 fo_add8(fo_u32x4 a, fo_u32x4 b) {
+    typedef fo_elem<Tag> E;
+    fo_u32x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t x = a[i], y = b[i];
+        const float lo = E::to_f32((uint16_t)(x & 0xffff)) + E::to_f32((uint16_t)(y & 0xffff));
+        const float hi = E::to_f32((uint16_t)(x >> 16)) + E::to_f32((uint16_t)(y >> 16));
+        o[i] = (uint32_t)E::from_f32(lo) | ((uint32_t)E::from_f32(hi) << 16);
+    }
+    return o;
+}
+
 // Wait states between the assembly MFMAs and ordinary VALU code touching their
 // accumulators (longest case: an 8-pass MFMA result read by a VALU instruction).
 static __device__ __forceinline__ void fo_mfma_fence() {
@@ -102,6 +117,9 @@ int fo_main_tile_resident();
 
 // fo_gemm_signal / fo_gemm_scatter (RE != nullptr) without the counters: tiles are
 // stored reordered, MM is never touched (fo_gemm.hip; used by fo_overlap.cpp).
+// fo_gemm_accumulate: the same (RA null: as fo_gemm stores), and the accumulator updated by the GEMM itself.
+int fo_gemm_accumulate(int dtype, int M, int N, int K, int rLDN, const int32_t *cseg_dev, int G, const void *A, const void *B,
+                       void *C, void *acc, const int32_t *RA, int algo, fo_stream_t stream);
 int fo_gemm_reordered_quiet(int dtype, int M, int N, int K, int rLDN, const int32_t *cseg_dev, int G,
                             const void *A, const void *B, void *C, const int32_t *RA, const int32_t *RE,
                             int algo, fo_stream_t stream);

@@ -9,28 +9,32 @@
 int fo_gemm_dev::fo_gemm256_launch(int dtype, int mode, const GemmArgs &a, hipStream_t stream, int *resident_out,
                                    int expect_resident) {
     if (a.lda != a.ldb) return FO_ERR_ARG;  // the kernel addresses both operands with one leading dimension
-    const int key = (dtype == FO_BF16 ? 3 : 0) + mode;
+    const int key = (dtype == FO_BF16 ? 4 : 0) + mode;
     switch (key) {
         case 0: return fo_gemm256_launch_0_0(a, stream, resident_out, expect_resident);
         case 1: return fo_gemm256_launch_0_1(a, stream, resident_out, expect_resident);
         case 2: return fo_gemm256_launch_0_2(a, stream, resident_out, expect_resident);
-        case 3: return fo_gemm256_launch_1_0(a, stream, resident_out, expect_resident);
-        case 4: return fo_gemm256_launch_1_1(a, stream, resident_out, expect_resident);
-        case 5: return fo_gemm256_launch_1_2(a, stream, resident_out, expect_resident);
+        case 3: return fo_gemm256_launch_0_3(a, stream, resident_out, expect_resident);
+        case 4: return fo_gemm256_launch_1_0(a, stream, resident_out, expect_resident);
+        case 5: return fo_gemm256_launch_1_1(a, stream, resident_out, expect_resident);
+        case 6: return fo_gemm256_launch_1_2(a, stream, resident_out, expect_resident);
+        case 7: return fo_gemm256_launch_1_3(a, stream, resident_out, expect_resident);
     }
     return FO_ERR_ARG;
 }
 
 int fo_gemm_dev::fo_gemm_tile_launch(int dtype, int mode, const GemmArgs &a, int tm, int tn, hipStream_t stream,
                                      int *resident_out, int expect_resident) {
-    const int key = (dtype == FO_BF16 ? 3 : 0) + mode;
+    const int key = (dtype == FO_BF16 ? 4 : 0) + mode;
     switch (key) {
         case 0: return fo_gemm_tile_launch_0_0(a, tm, tn, stream, resident_out, expect_resident);
         case 1: return fo_gemm_tile_launch_0_1(a, tm, tn, stream, resident_out, expect_resident);
         case 2: return fo_gemm_tile_launch_0_2(a, tm, tn, stream, resident_out, expect_resident);
-        case 3: return fo_gemm_tile_launch_1_0(a, tm, tn, stream, resident_out, expect_resident);
-        case 4: return fo_gemm_tile_launch_1_1(a, tm, tn, stream, resident_out, expect_resident);
-        case 5: return fo_gemm_tile_launch_1_2(a, tm, tn, stream, resident_out, expect_resident);
+        case 3: return fo_gemm_tile_launch_0_3(a, tm, tn, stream, resident_out, expect_resident);
+        case 4: return fo_gemm_tile_launch_1_0(a, tm, tn, stream, resident_out, expect_resident);
+        case 5: return fo_gemm_tile_launch_1_1(a, tm, tn, stream, resident_out, expect_resident);
+        case 6: return fo_gemm_tile_launch_1_2(a, tm, tn, stream, resident_out, expect_resident);
+        case 7: return fo_gemm_tile_launch_1_3(a, tm, tn, stream, resident_out, expect_resident);
     }
     return FO_ERR_ARG;
 }
@@ -148,7 +152,7 @@ __global__ __launch_bounds__(256) void fo_signal_all_kernel(const int32_t *cseg,
 
 int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *cseg, int G,
              const void *A, const void *B, void *C, int32_t *MM, const int32_t *RA,
-             const int32_t *RE, int monitor, int algo, fo_stream_t stream, bool quiet = false) {
+             const int32_t *RE, int monitor, int algo, fo_stream_t stream, bool quiet = false, void *acc = nullptr) {
     if (dtype != FO_F16 && dtype != FO_BF16) return FO_ERR_DTYPE;
     const fo_algo_entry *e = fo_algo_lookup(algo);
     if (!e) return FO_ERR_ALGO;
@@ -164,22 +168,25 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     a.A = static_cast<const uint16_t *>(A);
     a.B = static_cast<const uint16_t *>(B);
     a.C = static_cast<uint16_t *>(C);
+    a.ACC = static_cast<uint16_t *>(acc);
     a.M = M; a.N = N; a.K = K;
     a.lda = K; a.ldb = K;
     a.BM = e->f[0]; a.BN = e->f[1];
     a.TN = N / a.BN;
     a.rLDN = rLDN;
     a.RA = RA; a.RE = RE; a.cseg = cseg; a.G = G; a.MM = MM; a.monitor = monitor;
-    const launch_plan plan = plan_launch(r, M, N, a.BM, a.BN, mode != MODE_PLAIN && !quiet && K < kSignalAfterFromK);
+    const bool counts = (mode == MODE_SIGNAL || mode == MODE_SCATTER) && !quiet;
+    const launch_plan plan = plan_launch(r, M, N, a.BM, a.BN, counts && K < kSignalAfterFromK);
     a.grid_m = plan.grid_m; a.grid_n = plan.grid_n; a.panel = plan.panel; a.xcd_remap = plan.xcd_remap;
     a.first = 0; a.sub_m = a.sub_n = 1;
     a.count = plan.count;
     a.half = (M % 256 ? 1 : 0) | (N % 256 ? 2 : 0);
     // counters the launch cannot move itself are moved behind it
-    const bool signal_after = mode != MODE_PLAIN && !quiet && !plan.whole;
+    const bool signal_after = counts && !plan.whole;
     a.quiet = quiet || signal_after ? 1 : 0;
     a.stream_out = (int64_t)M * N * 2 > kStreamOutAboveBytes ? 1 : 0;
-    if (mode != MODE_PLAIN) {
+    if (mode == MODE_ACC && (((uintptr_t)C | (uintptr_t)acc) & 15)) return FO_ERR_SHAPE;  // as the consumer launch would
+    if (mode != MODE_PLAIN && !(mode == MODE_ACC && !RA)) {
         const long T = (long)(M / a.BM) * a.TN;
         if ((!MM && !quiet) || !RA || !cseg) return FO_ERR_ARG;
         if (mode == MODE_SCATTER && !RE) return FO_ERR_ARG;
@@ -253,6 +260,12 @@ int fo_gemm_reordered_quiet(int dtype, int M, int N, int K, int rLDN, const int3
                             int algo, fo_stream_t stream) {
     return run_gemm(RE ? MODE_SCATTER : MODE_SIGNAL, dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, nullptr, RA, RE,
                     0, algo, stream, true);
+}
+
+int fo_gemm_accumulate(int dtype, int M, int N, int K, int rLDN, const int32_t *cseg_dev, int G, const void *A, const void *B,
+                       void *C, void *acc, const int32_t *RA, int algo, fo_stream_t stream) {
+    if (!acc) return FO_ERR_ARG;
+    return run_gemm(MODE_ACC, dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, nullptr, RA, nullptr, 0, algo, stream, true, acc);
 }
 
 extern "C" int fo_gemm_wave_tiles(int dtype, int algo, int M, int N, int32_t *tiles) {

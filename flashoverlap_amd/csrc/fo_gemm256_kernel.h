@@ -90,6 +90,7 @@ template <typename Tag, int MODE>
 __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     typedef fo_elem<Tag> E;
     typedef fo_mfma256<Tag> X;
+    constexpr bool ACC = MODE == MODE_ACC, COUNTS = MODE == MODE_SIGNAL || MODE == MODE_SCATTER;
     constexpr int MT = 256, BK = 64, F = 8, ROWS = 16, AHEAD = 7, ARING = AHEAD + 1;
     constexpr int FREE = ROWS - AHEAD;  // row behind whose MFMAs the step's slot is given up
     constexpr int PUB = 12;             // row behind whose MFMAs the next step's slot is published
@@ -237,7 +238,8 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
 #pragma unroll
     for (int q = 0; q < NPRE; q++) pre[q] = 0;
     const bool reg_search = p.G <= kPrefixRegs;
-    const bool signalling = MODE != MODE_PLAIN && !p.quiet;
+    const bool signalling = COUNTS && !p.quiet;
+    const bool reorder = ACC ? p.RA != nullptr : COUNTS;
     // The group sizes are requested in front of the pipeline fill and summed behind it (a round trip to memory and
     // some two dozen dependent cross-lane steps otherwise stand between the kernel's start and its first operand
     // load).  The requests are assembly: their registers are read only behind the fill's wait for loads that were
@@ -313,7 +315,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     // where it would turn every wait for LDS data into a wait for everything (scalar loads return out of order).
     int rs_next[kMaxSub] = {0, 0, 0, 0};
     auto request_slots = [&](int pm_, int pn_) {
-        if (MODE != MODE_PLAIN) {
+        if (reorder) {
             const int tm_ = pm_ >> (p.BM >> 8), tn_ = pn_ >> (p.BN >> 8);  // in reorder tiles (BM, BN: 128 or 256)
 #pragma unroll
             for (int s = 0; s < kMaxSub; s++)
@@ -325,7 +327,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     const int my_sub = __builtin_amdgcn_readfirstlane(((wm * 128) / p.BM) * sub_n + (wn * 128) / p.BN);
     int r_mine = 0, v_rs = 0;
     auto take_slots = [&]() {
-        if (MODE != MODE_PLAIN) {
+        if (reorder) {
 #pragma unroll
             for (int s = 0; s < kMaxSub; s++) {
                 int rr = rs_next[s];
@@ -391,7 +393,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
         // barrier behind the wait.  The test inside the step (one scalar compare and branch per K step, after the PUB
         // meeting) cost the large square 4 us.
         int kt = 0;
-        int kt_stop = (MODE != MODE_PLAIN && owed > 0) ? 1 : KT;
+        int kt_stop = (COUNTS && owed > 0) ? 1 : KT;
         for (;;) {
         do {
             unsigned la_ = la0 ^ slot_b, lb_ = lb0 ^ slot_b;
@@ -473,7 +475,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             }
             slot_b ^= SLOT_B;
         } while (++kt < kt_stop);
-            if (MODE == MODE_PLAIN || owed == 0) break;
+            if (!COUNTS || owed == 0) break;
             owed = 0;
             if (wave == 0) announce(v_prev_r, v_prev_g);
             // Nothing scalar stays in flight behind this rare path: with a scalar load possibly pending, the K
@@ -502,16 +504,27 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             const int erow = el & 15, ek = el >> 4;  // accumulator block: row erow, columns 4*ek .. 4*ek+3
             uint16_t *strip = reinterpret_cast<uint16_t *>(reinterpret_cast<char *>(smem) + STRIP_B) + wave * (16 * PITCH);
             const int srow = el / CPR, scol = el % CPR;
-            const int ldp = MODE == MODE_PLAIN ? p.N : p.rLDN * p.BN;  // leading dimension of the output view
+            const int ldp = reorder ? p.rLDN * p.BN : p.N;  // leading dimension of the output view
             const int row0 = (wm * 128) % p.BM, col0 = (wn * 128) % p.BN;
             const int r = r_mine;
             const int v_cur = v_rs;  // this tile's slots: the next tile's replace them inside the loop below
-            const long trow = MODE == MODE_PLAIN ? (long)(pm + wm) * 128 : (long)(r / p.rLDN) * p.BM + row0;
-            const long tcol = MODE == MODE_PLAIN ? (long)(pn + wn) * 128 : (long)(r % p.rLDN) * p.BN + col0;
+            const long trow = !reorder ? (long)(pm + wm) * 128 : (long)(r / p.rLDN) * p.BM + row0;
+            const long tcol = !reorder ? (long)(pn + wn) * 128 : (long)(r % p.rLDN) * p.BN + col0;
             char *cbase = reinterpret_cast<char *>(p.C) + (trow * ldp + tcol) * 2;  // wave-uniform
             const unsigned lane_off = (unsigned)(srow * ldp + scol * 8) * 2;
             const bool stream_out = p.stream_out != 0;  // wave-uniform
             const bool keep = !((repeated & 1) && wm == 0) && !((repeated & 2) && wn == 0);  // wave-uniform
+            // MODE_ACC: the accumulator's values of the whole block, 32 pieces a lane: this wavefront owns the SIMD and
+            // has the registers.  They are awaited together, in front of the first store: a later wait would count the
+            // stores between them as well.  4096x4096x512: 30 us, where the reordering GEMM took 21 and a consumer
+            // launch behind it 16 (whole pass 52 -> 46).
+            fo_u32x4 old[ACC ? NST : 1];
+            char *abase = ACC ? reinterpret_cast<char *>(p.ACC) + (trow * ldp + tcol) * 2 : nullptr;
+            if (ACC && keep) {
+#pragma unroll
+                for (int k = 0; k < NST; k++)
+                    old[k] = *reinterpret_cast<const fo_u32x4 *>(abase + (size_t)(k * RPP) * ldp * 2 + lane_off);
+            }
 #pragma unroll
             for (int i = 0; i < F; i++) {  // 16 output rows = one row of accumulator blocks
                 __builtin_amdgcn_sched_barrier(0);
@@ -532,6 +545,10 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_s_waitcnt(0xC07F);
                 __builtin_amdgcn_wave_barrier();
+                if (ACC && i == 0) {
+#pragma unroll
+                    for (int k = 0; k < NST; k++) asm volatile("" : "+v"(old[ACC ? k : 0]));
+                }
                 if (keep)
 #pragma unroll
                 for (int ps = 0; ps < 16 / RPP; ps++) {
@@ -547,7 +564,15 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                             store16_write_through(p.C + (size_t)prow * ldp + tcol + scol * 8, v);
                     } else {
                         char *sb = cbase + (size_t)(i * 16 + ps * RPP) * ldp * 2;
-                        if (MODE == MODE_PLAIN) {
+                        if constexpr (ACC) {
+                            char *ab = abase + (size_t)(i * 16 + ps * RPP) * ldp * 2;
+                            const fo_u32x4 sum = fo_add8<Tag>(old[i * (16 / RPP) + ps], v);
+                            if (stream_out)
+                                store16_nt(ab, lane_off, sum);
+                            else
+                                store16(ab, lane_off, sum);
+                        }
+                        if (!COUNTS) {
                             if (stream_out)
                                 store16_nt(sb, lane_off, v);
                             else

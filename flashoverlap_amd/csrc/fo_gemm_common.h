@@ -18,12 +18,15 @@
 
 namespace fo_gemm_dev {
 
-enum { MODE_PLAIN = 0, MODE_SIGNAL = 1, MODE_SCATTER = 2 };
+// MODE_ACC: for a call that stays on one stream.  The tile is stored as the plain epilogue does (RA null) or reordered,
+// without counters, and ACC[o] = round16(ACC[o] + C[o]) is done for every element stored.
+enum { MODE_PLAIN = 0, MODE_SIGNAL = 1, MODE_SCATTER = 2, MODE_ACC = 3 };
 
 struct GemmArgs {
     const uint16_t *A;
     const uint16_t *B;
     uint16_t *C;
+    uint16_t *ACC;         // MODE_ACC: the accumulator, addressed as C is
     int M, N, K;
     int lda, ldb;          // row strides of A and B in elements (multiples of 8)
     int BM, BN, TN, rLDN;  // reorder/signal tile, tiles along N, reshaped width in tiles

@@ -20,7 +20,15 @@
 // operands of three buffer sets in turn): 512x4096x4096 39.1 -> 21 us, 256x8192x3584 35.5 -> 19.5,
 // 128x4096x1024 10.4 -> 4.5, 128x1024x8192 71 -> 12.5, 2048x4096x4096 62 -> 55.  512x4096x4096 with the MFMAs taken
 // out takes 18.7 us: the rest of its time is the operand stream.
+//
+// MODE_ACC, the epilogue of calls that stay on one stream: what the consumer kernel would do behind the GEMM (read C and
+// the accumulator, write the accumulator) is done on the tile in LDS.  The loaders, idle by then, request the
+// accumulator's values while the last S - 1 stages are multiplied and write the sums; the computing wavefronts store
+// C.  Saves the second read of C and a launch.  Whole passes: 512x4096x4096 29.5 -> 28.7 us, 1152x5120x1720
+// 42.7 -> 40.7, 1024x8192x2048 49 -> 46.2.
 #pragma once
+
+#include <type_traits>
 
 #include "fo_gemm_common.h"
 
@@ -57,13 +65,17 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
     constexpr int WTM = TM / 2, WTN = TN / 2, FM = WTM / 16, FN = WTN / 16;  // computing wavefronts: 2 x 2
     constexpr int PA = TM / 8 / NL, PB = TN / 8 / NL, P = KB * (PA + PB);    // 1 KiB loads per loader and stage
     constexpr unsigned A_BLK = TM * 128, B_BLK = TN * 128, STAGE = KB * (A_BLK + B_BLK);
-    constexpr int PITCH = TN + 8, CPR = TN / 8, NCH = (TM * CPR + kTileThreads - 1) / kTileThreads;  // output staging
+    constexpr bool ACC = MODE == MODE_ACC, COUNTS = MODE == MODE_SIGNAL || MODE == MODE_SCATTER;
+    // output staging; with an accumulator the computing wavefronts store the tile and the loaders update the accumulator
+    constexpr int STORERS = ACC ? kTileComputers * 64 : kTileThreads;
+    constexpr int PITCH = TN + 8, CPR = TN / 8, NCH = (TM * CPR + STORERS - 1) / STORERS;
     static_assert(BK % 64 == 0 && TM % 32 == 0 && TN % 32 == 0, "whole 1 KiB loads for every loader");
-    static_assert(S >= 2 && (S - 1) * P < 64, "vmcnt range");
+    static_assert(S >= 2 && (S - 1) * P < 64 && (!ACC || (S - 3) * P + NCH < 64), "vmcnt range");
 
     extern __shared__ fo_u32x4 smem[];
     __shared__ int32_t row_map[MODE == MODE_SCATTER ? 256 : 1];  // scatter: where the tile's rows go
     const unsigned lds0 = (unsigned)(uintptr_t)FO_LDS_PTR(smem);
+    uint16_t *stage = reinterpret_cast<uint16_t *>(smem);  // the output tile, once the K loop is done
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool loader = wave_id < NL;
@@ -72,8 +84,9 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
     const int KT = (p.K + BK - 1) / BK;
 
     const int bm_shift = p.BM == 256 ? 8 : 7, bn_shift = p.BN == 256 ? 8 : 7;  // reorder tiles: 128 or 256 each way
-    const int ldp = MODE == MODE_PLAIN ? p.N : p.rLDN * p.BN;  // leading dimension of the output view
-    const bool signalling = MODE != MODE_PLAIN && !p.quiet;
+    const bool reorder = MODE == MODE_ACC ? p.RA != nullptr : MODE != MODE_PLAIN;
+    const int ldp = reorder ? p.rLDN * p.BN : p.N;  // leading dimension of the output view
+    const bool signalling = COUNTS && !p.quiet;
     typedef const __attribute__((address_space(4))) int32_t *cptr_t;  // read-only for the whole launch: scalar loads
     const cptr_t RAc = (cptr_t)(uintptr_t)p.RA;
 
@@ -92,7 +105,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
         int r0 = 0, r1 = 0;
         bool two_m = false, two_n = false;
         int split_m = TM, split_n = TN;
-        if (MODE != MODE_PLAIN) {
+        if (reorder) {
             const int tm0 = m0 >> bm_shift, tn0 = n0 >> bn_shift;
             two_m = (m0 + TM - 1) >> bm_shift != tm0;
             two_n = (n0 + TN - 1) >> bn_shift != tn0;
@@ -109,12 +122,56 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             return (r % rldn << bn_shift) + (second && two_n ? -split_n : n0 & (p.BN - 1));
         };
 
-        fo_float4v acc[FM][FN];
-#pragma unroll
-        for (int i = 0; i < FM; i++)
-#pragma unroll
-            for (int j = 0; j < FN; j++) acc[i][j] = fo_float4v{0.f, 0.f, 0.f, 0.f};
         int g0 = 0, g1 = 0;  // groups of r0 and r1 (the wavefront that signals)
+        // Row and column of the output view at which the tile's row and column 0 are, or would be, in r0 and in r1.
+        int row0 = m0, row1 = m0, col0 = n0, col1 = n0;
+        auto find_bases = [&]() __attribute__((always_inline)) {
+            if (!reorder) return;
+            int rldn = p.rLDN;
+            asm volatile("" : "+s"(rldn));  // the divisions by it are done here, not in front of the K loop
+            int q0 = r0, q1 = r1;
+            if (rldn != 1) {
+                q0 /= rldn;
+                q1 /= rldn;
+            }
+            row0 = (q0 << bm_shift) + (m0 & (p.BM - 1));
+            row1 = (q1 << bm_shift) + (two_m ? -split_m : m0 & (p.BM - 1));
+            col0 = (r0 - q0 * rldn << bn_shift) + (n0 & (p.BN - 1));
+            col1 = (r1 - q1 * rldn << bn_shift) + (two_n ? -split_n : n0 & (p.BN - 1));
+        };
+        // The tile in pieces of 16 bytes: act(u, row, column, address in the view `out`) for thread t's piece u, those
+        // to be stored or (EVERY) all of them.  A tile that lies in one reorder tile and is stored whole needs one address
+        // per thread, the pieces following at a uniform distance (the general address costs some forty instructions, and
+        // a thread has up to sixteen pieces).  (The thread id is laundered so that this is computed here instead of
+        // resting in registers across the K loop.)
+        const bool simple = !two_m && !two_n && !skip_m && !skip_n && ldp < 1 << 22;
+        auto each_piece = [&](int t, uint16_t *out, auto every, auto act) __attribute__((always_inline)) {
+            constexpr bool EVERY = decltype(every)::value;
+            asm volatile("" : "+v"(t));
+            if (simple) {
+                uint16_t *base = out + (size_t)row0 * ldp + col0;
+#pragma unroll
+                for (int u = 0; u < NCH; u++) {
+                    const bool steps = STORERS % CPR == 0;
+                    const int idx = (u * STORERS + t) % (EVERY ? TM * CPR : 1 << 30);
+                    const int row = steps ? u * (STORERS / CPR) + t / CPR : idx / CPR, col = (steps ? t : idx) % CPR * 8;
+                    const unsigned off = (unsigned)((steps ? t / CPR : row) * ldp + col);
+                    if (EVERY || TM * CPR % STORERS == 0 || row < TM)
+                        act(u, row, col, base + (steps ? (size_t)(u * (STORERS / CPR)) * ldp : 0) + off);
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < NCH; u++) {
+                    const int idx = (u * STORERS + t) % (EVERY ? TM * CPR : 1 << 30), row = idx / CPR, col = idx % CPR * 8;
+                    const bool second = row >= split_m || col >= split_n;
+                    if (EVERY || ((TM * CPR % STORERS == 0 || row < TM) && row >= skip_m && col >= skip_n))
+                        act(u, row, col, out + (size_t)((second ? row1 : row0) + row) * ldp + (second ? col1 : col0) + col);
+                }
+            }
+        };
+        auto piece = [&](int row, int col) __attribute__((always_inline)) {
+            return *reinterpret_cast<const fo_u32x4 *>(stage + row * PITCH + col);
+        };
 
         if (loader) {
             // Load u of a 64-column block brings rows (u * NL + wave) * 8 + lane / 8 of an operand, 128 bytes each; LDS
@@ -146,15 +203,55 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             wait_vmcnt<(S - 2) * P>();  // stage 0 has landed (vmcnt retires in issue order)
             __builtin_amdgcn_s_barrier();
             unsigned slot = (S - 1) * STAGE;
-            for (int kt = 0; kt < KT; kt++) {
+            // With an accumulator the steps behind the last request ask for its values instead of further stages: they
+            // arrive while the last S - 1 stages are multiplied.
+            const int fetching = ACC ? (KT > S - 1 ? KT - (S - 1) : 0) : KT;
+            for (int kt = 0; kt < fetching; kt++) {
                 request(kt + S - 1, slot);  // the slot of stage kt - 1, given up at the last barrier
                 slot = slot + STAGE == S * STAGE ? 0 : slot + STAGE;
                 wait_vmcnt<(S - 2) * P>();  // stage kt + 1
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
             }
-            wait_vmcnt<0>();  // nothing lands in the space the output is staged in
+            fo_u32x4 old[ACC ? NCH : 1];  // the accumulator's values
+            if constexpr (ACC) {
+                find_bases();
+                // every wavefront loads every piece, needed or not: the waits below count
+                each_piece(wave * 64 + lane, p.ACC, std::true_type{}, [&](int u, int, int, uint16_t *at) __attribute__((always_inline)) {
+                    old[u] = *reinterpret_cast<const fo_u32x4 *>(at);
+                });
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int j = 0; j < S - 1; j++) {
+                    if (fetching + j < KT) {
+                        if (j < S - 2) asm volatile("s_waitcnt vmcnt(%0)" : : "i"((S - 3 - j) * P + NCH) : "memory");  // stage fetching + j + 1
+                        __builtin_amdgcn_s_barrier();
+                        asm volatile("" ::: "memory");
+                    }
+                }
+                wait_vmcnt<NCH>();
+            } else {
+                wait_vmcnt<0>();  // nothing lands in the space the output is staged in
+            }
+            __builtin_amdgcn_s_barrier();  // every fragment has been fetched
+            asm volatile("" ::: "memory");
+            if constexpr (ACC) {
+                __builtin_amdgcn_s_barrier();  // the tile has been staged
+                asm volatile("" ::: "memory");
+                // All of them are awaited, those of pieces that are not stored too: one left pending would be waited for
+                // in the next tile's K loop, with everything else in flight.
+#pragma unroll
+                for (int u = 0; u < NCH; u++) asm volatile("" : "+v"(old[u]));
+                each_piece(wave * 64 + lane, p.ACC, std::false_type{}, [&](int u, int row, int col, uint16_t *at) __attribute__((always_inline)) {
+                    *reinterpret_cast<fo_u32x4 *>(at) = fo_add8<Tag>(old[u], piece(row, col));
+                });
+            }
         } else {
+            fo_float4v acc[FM][FN];
+#pragma unroll
+            for (int i = 0; i < FM; i++)
+#pragma unroll
+                for (int j = 0; j < FN; j++) acc[i][j] = fo_float4v{0.f, 0.f, 0.f, 0.f};
             // Fragment addressing: lane l supplies row l & 15, k-chunk l >> 4 of a 16x32 block.  The operand of which a
             // wavefront holds more fragments is the long one: a k-step goes through it fragment by fragment (a "row"),
             // each with all fragments of the short one.
@@ -260,18 +357,13 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                 slot = next;
             }
             __builtin_amdgcn_s_waitcnt(0xC07F);
-        }
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-
-        // ---- epilogue: accumulators -> 16 bit -> LDS -> 16-byte pieces of output rows, by all eight wavefronts
-        // (the thread id is laundered so that this addressing is computed here instead of resting in registers across
-        // the K loop)
-        int et = tid;
-        asm volatile("" : "+v"(et));
-        uint16_t *stage = reinterpret_cast<uint16_t *>(smem);
-        if (!loader) {
-            const int erow = et & 15, ek = (et & 63) >> 4;  // accumulator block: row erow, columns 4*ek .. 4*ek+3
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            // ---- epilogue: accumulators -> 16 bit -> LDS -> 16-byte pieces of output rows.  (The thread id is laundered
+            // so that this addressing is computed here instead of resting in registers across the K loop.)
+            int el = lane;
+            asm volatile("" : "+v"(el));
+            const int erow = el & 15, ek = el >> 4;  // accumulator block: row erow, columns 4*ek .. 4*ek+3
 #pragma unroll
             for (int i = 0; i < FM; i++)
 #pragma unroll
@@ -281,31 +373,31 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                     v.y = (uint32_t)E::from_f32(acc[i][j][2]) | ((uint32_t)E::from_f32(acc[i][j][3]) << 16);
                     *reinterpret_cast<fo_u32x2 *>(stage + (wm * WTM + i * 16 + erow) * PITCH + wn * WTN + j * 16 + ek * 4) = v;
                 }
+            if constexpr (ACC) {
+                find_bases();
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_waitcnt(0xC07F);
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                each_piece(wave * 64 + lane, p.C, std::false_type{}, [&](int, int row, int col, uint16_t *at) __attribute__((always_inline)) {
+                    *reinterpret_cast<fo_u32x4 *>(at) = piece(row, col);
+                });
+            }
         }
-        int rldn = p.rLDN;
-        asm volatile("" : "+s"(rldn));  // the divisions by it too
-        int row0 = 0, row1 = 0, col0 = 0, col1 = 0;
-        if (MODE != MODE_PLAIN) {
-            row0 = row_base(r0, rldn, false);
-            col0 = col_base(r0, rldn, false);
-            row1 = row_base(r1, rldn, true);
-            col1 = col_base(r1, rldn, true);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < NCH; u++) {
-            const int idx = u * kTileThreads + et, row = idx / CPR, col = idx % CPR * 8;
-            // piece u of a thread: columns 8 * (idx % CPR) of row idx / CPR
-            if ((TM * CPR % kTileThreads == 0 || row < TM) && row >= skip_m && col >= skip_n) {
-                const fo_u32x4 v = *reinterpret_cast<const fo_u32x4 *>(stage + row * PITCH + col);
+        if constexpr (!ACC) {
+            find_bases();
+            __syncthreads();
+            each_piece(tid, p.C, std::false_type{}, [&](int, int row, int col, uint16_t *at) __attribute__((always_inline)) {
                 if constexpr (MODE == MODE_PLAIN) {
-                    *reinterpret_cast<fo_u32x4 *>(p.C + (size_t)(m0 + row) * ldp + n0 + col) = v;
+                    *reinterpret_cast<fo_u32x4 *>(at) = piece(row, col);
+                } else if constexpr (MODE == MODE_SIGNAL) {
+                    store16_write_through(at, piece(row, col));
                 } else {
                     const bool second = row >= split_m || col >= split_n;
-                    const int to_row = MODE == MODE_SCATTER ? row_map[two_n && second ? TM + row : row] : (second ? row1 : row0) + row;
-                    store16_write_through(p.C + (size_t)to_row * ldp + (second ? col1 : col0) + col, v);
+                    const int to_row = row_map[two_n && second ? TM + row : row];
+                    store16_write_through(p.C + (size_t)to_row * ldp + (second ? col1 : col0) + col, piece(row, col));
                 }
-            }
+            });
         }
         if (signalling) {
             // Whole reorder tiles only (the launcher sees to it): every wavefront's write-through stores are

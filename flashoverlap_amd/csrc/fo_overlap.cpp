@@ -28,8 +28,8 @@ enum {
 //
 // In automatic mode a GEMM shorter than kInStreamBelowFlop (about 50 us of this
 // GPU) keeps the whole call on the GEMM stream: the GEMM with its reordered
-// store and one consumer launch (with the monitor on: the signalling GEMM and
-// one wait that resets every counter between them).  Fork, join and pollers beside the
+// store, whose epilogue does the all-reduce consumer's work too (with the monitor on: the signalling
+// GEMM, one wait that resets every counter and one consumer launch).  Fork, join and pollers beside the
 // GEMM cost more than such a GEMM can hide (4096x4096x512 with 256 groups:
 // 71 us overlapped, 48 us in stream).
 //
@@ -420,9 +420,12 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
     // to do: unless the caller wants the monitor's stamps, the GEMM then leaves
     // the counters alone (they stay zero, as the waits would have left them).
     const bool quiet = same_stream && !monitor;
-    rc = quiet ? fo_gemm_reordered_quiet(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, RA, nullptr, algo,
-                                         h->gemm_stream)
-               : fo_gemm_signal(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, MM, RA, monitor, algo,
+    // With nothing to wait for, the GEMM's epilogue does the consumer's work on the tile it holds in LDS.
+    const bool consumed = quiet && h->acc;
+    rc = consumed ? fo_gemm_accumulate(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, h->acc, RA, algo, h->gemm_stream)
+         : quiet  ? fo_gemm_reordered_quiet(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, RA, nullptr, algo,
+                                            h->gemm_stream)
+                  : fo_gemm_signal(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, MM, RA, monitor, algo,
                                 h->gemm_stream);
     if (rc) return rc;  // the GEMM was refused: nothing of this call follows on either stream
 
@@ -455,7 +458,7 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
                                 : fo_wait_groups_with(j - i, cseg_dev + i, MM + i, h->max_polls, gave_up, cstream);
                 if (rc) return rc;
             }
-            if (acc) {  // the groups of a batch are one contiguous range
+            if (acc && !consumed) {  // the groups of a batch are one contiguous range
                 rc = fo_consumer_reduce_with(dtype, c + off, acc + off, n, 1, 0, nullptr, 0, stream_acc, cstream,
                                              j < G && !same_stream);  // every batch but the last runs beside the GEMM
                 if (rc) return rc;
@@ -643,12 +646,9 @@ extern "C" int fo_overlap_gemm_allreduce_serial(fo_overlap_t *h, int dtype, int 
     if (!h) return FO_ERR_ARG;
     if (!h->gemm_ready) return FO_ERR_STATE;
     if (h->acc && h->acc_nelem < (int64_t)M * N) return FO_ERR_ARG;
-    int rc = fo_gemm(dtype, M, N, K, A, B, C, algo, h->gemm_stream);
+    int rc = h->acc ? fo_gemm_accumulate(dtype, M, N, K, 1, nullptr, 0, A, B, C, h->acc, nullptr, algo, h->gemm_stream)
+                    : fo_gemm(dtype, M, N, K, A, B, C, algo, h->gemm_stream);
     if (rc) return rc;
-    if (h->acc) {
-        rc = fo_consumer_reduce(dtype, C, h->acc, (int64_t)M * N, h->gemm_stream);
-        if (rc) return rc;
-    }
     return link_time(h, (int64_t)M * N * 2, h->gemm_stream);
 }
 

@@ -82,3 +82,37 @@ def test_workgroup_tiles(fo, dtype, bm, bn, M, N, K):
     check("on one stream, row-mapped", RE)
     assert (MM == 0).all()
     ov.close()
+
+
+@pytest.mark.parametrize("dtype,bm,bn,M,N,K", CASES)
+def test_accumulating_epilogue(fo, dtype, bm, bn, M, N, K):
+    """A call on one stream with an accumulator attached: same product, and the accumulator the once-rounded sum."""
+    ops, layout, td = fo.ops, fo.layout, TORCH_DTYPE[dtype]
+    algo = fo._capi.find_algo(bm, bn, swizzle=4)
+    TM, TN = M // bm, N // bn
+    T = TM * TN
+    A, _ = seeded((M, K), dtype, M + K)
+    B, _ = seeded((N, K), dtype, N + K, scale=K ** -0.5)
+    before, _ = seeded((M, N), dtype, 7)
+    acc = before.clone()
+    plain, C = (torch.full((M, N), float("nan"), device="cuda", dtype=td) for _ in range(2))
+    ops.gemm(A, B, plain, algo)
+    ov = ops.Overlap()
+    ov.set_schedule(in_stream_below_flop=1e15)
+    ov.set_accumulator(acc)
+    ov.gemm_allreduce(A, B, C, algo)
+    torch.cuda.synchronize()
+    assert torch.equal(C, plain)
+    assert torch.equal(acc, (before.float() + plain.float()).to(td))
+    RA = torch.from_numpy(np.random.default_rng(M + N).permutation(T).astype(np.int32)).reshape(TM, TN).cuda()
+    cs_cpu = torch.tensor([T], dtype=torch.int32)
+    MM = torch.zeros(layout.counter_size(1, TM, TN), dtype=torch.int32, device="cuda")
+    for rldn in (1, 2 if T % 2 == 0 else 1):
+        C.fill_(float("nan"))
+        acc.copy_(before)
+        ov.gemm_allreduce_overlap(A, B, C, MM, RA, rldn, cs_cpu, cs_cpu.cuda(), algo)
+        torch.cuda.synchronize()
+        assert torch.equal(layout.unpermute(C, M, N, bm, bn, RA, rLDN=rldn), plain)
+        assert torch.equal(acc.reshape(-1), (before.float() + C.float()).to(td).reshape(-1))
+    assert (MM == 0).all()
+    ov.close()
