@@ -33,8 +33,8 @@ ARCH = "gfx950"
 
 KERNEL_SOURCES = ["fo_gemm.hip", "fo_aux.hip", "fo_algo.cpp", "fo_overlap.cpp"]
 # fo_gemm256_inst.hip and fo_gemm_tile_inst.hip hold the instantiations of the GEMM kernels for one dtype (fp16 / bf16)
-# and one epilogue (plain / signal / scatter / accumulating) per compilation; they take up to minutes, so they are separate jobs.
-GEMM_INSTANCES = [(src, d, m) for src in ("fo_gemm256_inst.hip", "fo_gemm_tile_inst.hip") for d in (0, 1) for m in (0, 1, 2, 3)]
+# and one epilogue (plain / signal / scatter / accumulating / reduce-scatter) per compilation; they take up to minutes, so they are separate jobs.
+GEMM_INSTANCES = [(src, d, m) for src in ("fo_gemm256_inst.hip", "fo_gemm_tile_inst.hip") for d in (0, 1) for m in (0, 1, 2, 3, 4)]
 
 # -packed-fp32-ops off: hipcc must not form v_pk_*_f32 from the float code here.
 HIP_FLAGS = [

@@ -120,6 +120,11 @@ int fo_main_tile_resident();
 // fo_gemm_accumulate: the same (RA null: as fo_gemm stores), and the accumulator updated by the GEMM itself.
 int fo_gemm_accumulate(int dtype, int M, int N, int K, int rLDN, const int32_t *cseg_dev, int G, const void *A, const void *B,
                        void *C, void *acc, const int32_t *RA, int algo, fo_stream_t stream);
+// The row-mapped store with rLDN == 1, the accumulator (may be null) updated in its reduce-scatter layout and this rank's
+// chunk of every group copied to `own` (may be null).  W divides the Algo's tile height; C, acc and own are 16-byte aligned.
+int fo_gemm_reduce_scatter(int dtype, int M, int N, int K, const int32_t *cseg_dev, int G, const void *A, const void *B, void *C,
+                           void *acc, void *own, const int32_t *RA, const int32_t *RE, int W, int rank, int algo,
+                           fo_stream_t stream);
 int fo_gemm_reordered_quiet(int dtype, int M, int N, int K, int rLDN, const int32_t *cseg_dev, int G,
                             const void *A, const void *B, void *C, const int32_t *RA, const int32_t *RE,
                             int algo, fo_stream_t stream);

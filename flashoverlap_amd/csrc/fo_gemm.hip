@@ -9,32 +9,36 @@
 int fo_gemm_dev::fo_gemm256_launch(int dtype, int mode, const GemmArgs &a, hipStream_t stream, int *resident_out,
                                    int expect_resident) {
     if (a.lda != a.ldb) return FO_ERR_ARG;  // the kernel addresses both operands with one leading dimension
-    const int key = (dtype == FO_BF16 ? 4 : 0) + mode;
+    const int key = (dtype == FO_BF16 ? 5 : 0) + mode;
     switch (key) {
         case 0: return fo_gemm256_launch_0_0(a, stream, resident_out, expect_resident);
         case 1: return fo_gemm256_launch_0_1(a, stream, resident_out, expect_resident);
         case 2: return fo_gemm256_launch_0_2(a, stream, resident_out, expect_resident);
         case 3: return fo_gemm256_launch_0_3(a, stream, resident_out, expect_resident);
-        case 4: return fo_gemm256_launch_1_0(a, stream, resident_out, expect_resident);
-        case 5: return fo_gemm256_launch_1_1(a, stream, resident_out, expect_resident);
-        case 6: return fo_gemm256_launch_1_2(a, stream, resident_out, expect_resident);
-        case 7: return fo_gemm256_launch_1_3(a, stream, resident_out, expect_resident);
+        case 4: return fo_gemm256_launch_0_4(a, stream, resident_out, expect_resident);
+        case 5: return fo_gemm256_launch_1_0(a, stream, resident_out, expect_resident);
+        case 6: return fo_gemm256_launch_1_1(a, stream, resident_out, expect_resident);
+        case 7: return fo_gemm256_launch_1_2(a, stream, resident_out, expect_resident);
+        case 8: return fo_gemm256_launch_1_3(a, stream, resident_out, expect_resident);
+        case 9: return fo_gemm256_launch_1_4(a, stream, resident_out, expect_resident);
     }
     return FO_ERR_ARG;
 }
 
 int fo_gemm_dev::fo_gemm_tile_launch(int dtype, int mode, const GemmArgs &a, int tm, int tn, hipStream_t stream,
                                      int *resident_out, int expect_resident) {
-    const int key = (dtype == FO_BF16 ? 4 : 0) + mode;
+    const int key = (dtype == FO_BF16 ? 5 : 0) + mode;
     switch (key) {
         case 0: return fo_gemm_tile_launch_0_0(a, tm, tn, stream, resident_out, expect_resident);
         case 1: return fo_gemm_tile_launch_0_1(a, tm, tn, stream, resident_out, expect_resident);
         case 2: return fo_gemm_tile_launch_0_2(a, tm, tn, stream, resident_out, expect_resident);
         case 3: return fo_gemm_tile_launch_0_3(a, tm, tn, stream, resident_out, expect_resident);
-        case 4: return fo_gemm_tile_launch_1_0(a, tm, tn, stream, resident_out, expect_resident);
-        case 5: return fo_gemm_tile_launch_1_1(a, tm, tn, stream, resident_out, expect_resident);
-        case 6: return fo_gemm_tile_launch_1_2(a, tm, tn, stream, resident_out, expect_resident);
-        case 7: return fo_gemm_tile_launch_1_3(a, tm, tn, stream, resident_out, expect_resident);
+        case 4: return fo_gemm_tile_launch_0_4(a, tm, tn, stream, resident_out, expect_resident);
+        case 5: return fo_gemm_tile_launch_1_0(a, tm, tn, stream, resident_out, expect_resident);
+        case 6: return fo_gemm_tile_launch_1_1(a, tm, tn, stream, resident_out, expect_resident);
+        case 7: return fo_gemm_tile_launch_1_2(a, tm, tn, stream, resident_out, expect_resident);
+        case 8: return fo_gemm_tile_launch_1_3(a, tm, tn, stream, resident_out, expect_resident);
+        case 9: return fo_gemm_tile_launch_1_4(a, tm, tn, stream, resident_out, expect_resident);
     }
     return FO_ERR_ARG;
 }
@@ -150,9 +154,16 @@ __global__ __launch_bounds__(256) void fo_signal_all_kernel(const int32_t *cseg,
         __hip_atomic_store(MM + TN + RA[t], first + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// What the epilogue of a reduce-scatter on one stream does besides storing C (MODE_RS in fo_gemm_common.h).
+struct rs_args {
+    void *own;
+    int W, rank;
+};
+
 int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *cseg, int G,
              const void *A, const void *B, void *C, int32_t *MM, const int32_t *RA,
-             const int32_t *RE, int monitor, int algo, fo_stream_t stream, bool quiet = false, void *acc = nullptr) {
+             const int32_t *RE, int monitor, int algo, fo_stream_t stream, bool quiet = false, void *acc = nullptr,
+             const rs_args *rs = nullptr) {
     if (dtype != FO_F16 && dtype != FO_BF16) return FO_ERR_DTYPE;
     const fo_algo_entry *e = fo_algo_lookup(algo);
     if (!e) return FO_ERR_ALGO;
@@ -175,6 +186,10 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     a.TN = N / a.BN;
     a.rLDN = rLDN;
     a.RA = RA; a.RE = RE; a.cseg = cseg; a.G = G; a.MM = MM; a.monitor = monitor;
+    a.OWN = static_cast<uint16_t *>(rs ? rs->own : nullptr);
+    a.W = rs ? rs->W : 1;
+    a.rank = rs ? rs->rank : 0;
+    a.seg_rows = (int)((int64_t)M * N / a.BN / a.W);
     const bool counts = (mode == MODE_SIGNAL || mode == MODE_SCATTER) && !quiet;
     const launch_plan plan = plan_launch(r, M, N, a.BM, a.BN, counts && K < kSignalAfterFromK);
     a.grid_m = plan.grid_m; a.grid_n = plan.grid_n; a.panel = plan.panel; a.xcd_remap = plan.xcd_remap;
@@ -189,7 +204,7 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     if (mode != MODE_PLAIN && !(mode == MODE_ACC && !RA)) {
         const long T = (long)(M / a.BM) * a.TN;
         if ((!MM && !quiet) || !RA || !cseg) return FO_ERR_ARG;
-        if (mode == MODE_SCATTER && !RE) return FO_ERR_ARG;
+        if ((mode == MODE_SCATTER || mode == MODE_RS) && !RE) return FO_ERR_ARG;
         if (rLDN <= 0 || T % rLDN) return FO_ERR_SHAPE;
         if (G <= 0 || G > T) return FO_ERR_SEGMENTS;
         if (monitor && G > a.TN - 1) return FO_ERR_SEGMENTS;
@@ -266,6 +281,16 @@ int fo_gemm_accumulate(int dtype, int M, int N, int K, int rLDN, const int32_t *
                        void *C, void *acc, const int32_t *RA, int algo, fo_stream_t stream) {
     if (!acc) return FO_ERR_ARG;
     return run_gemm(MODE_ACC, dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, nullptr, RA, nullptr, 0, algo, stream, true, acc);
+}
+
+int fo_gemm_reduce_scatter(int dtype, int M, int N, int K, const int32_t *cseg_dev, int G, const void *A, const void *B, void *C,
+                           void *acc, void *own, const int32_t *RA, const int32_t *RE, int W, int rank, int algo,
+                           fo_stream_t stream) {
+    const fo_algo_entry *e = fo_algo_lookup(algo);
+    if (!e) return FO_ERR_ALGO;
+    if (W <= 0 || rank < 0 || rank >= W || e->f[0] % W || (((uintptr_t)C | (uintptr_t)acc | (uintptr_t)own) & 15)) return FO_ERR_ARG;
+    const rs_args rs = {own, W, rank};
+    return run_gemm(MODE_RS, dtype, M, N, K, 1, cseg_dev, G, A, B, C, nullptr, RA, RE, 0, algo, stream, true, acc, &rs);
 }
 
 extern "C" int fo_gemm_wave_tiles(int dtype, int algo, int M, int N, int32_t *tiles) {

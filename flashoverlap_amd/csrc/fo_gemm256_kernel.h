@@ -90,7 +90,8 @@ template <typename Tag, int MODE>
 __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     typedef fo_elem<Tag> E;
     typedef fo_mfma256<Tag> X;
-    constexpr bool ACC = MODE == MODE_ACC, COUNTS = MODE == MODE_SIGNAL || MODE == MODE_SCATTER;
+    constexpr bool ACC = MODE == MODE_ACC || MODE == MODE_RS, COUNTS = MODE == MODE_SIGNAL || MODE == MODE_SCATTER;
+    constexpr bool MAPPED = MODE == MODE_SCATTER || MODE == MODE_RS;
     constexpr int MT = 256, BK = 64, F = 8, ROWS = 16, AHEAD = 7, ARING = AHEAD + 1;
     constexpr int FREE = ROWS - AHEAD;  // row behind whose MFMAs the step's slot is given up
     constexpr int PUB = 12;             // row behind whose MFMAs the next step's slot is published
@@ -239,14 +240,15 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     for (int q = 0; q < NPRE; q++) pre[q] = 0;
     const bool reg_search = p.G <= kPrefixRegs;
     const bool signalling = COUNTS && !p.quiet;
-    const bool reorder = ACC ? p.RA != nullptr : COUNTS;
+    const bool reorder = MODE == MODE_ACC ? p.RA != nullptr : COUNTS || MODE == MODE_RS;
+    const bool groups = signalling || MODE == MODE_RS;  // group sizes are needed
     // The group sizes are requested in front of the pipeline fill and summed behind it (a round trip to memory and
     // some two dozen dependent cross-lane steps otherwise stand between the kernel's start and its first operand
     // load).  The requests are assembly: their registers are read only behind the fill's wait for loads that were
     // requested after them, and the compiler, which knows nothing of the fill's loads, would otherwise wait for
     // every one of those as well.  Lanes beyond G ask for element 0.
     int cs_raw[NPRE];
-    if (signalling && reg_search) {
+    if (groups && reg_search) {
 #pragma unroll
         for (int q = 0; q < NPRE; q++) {
             const int32_t *src = p.cseg + (q * 64 + lane < p.G ? q * 64 + lane : 0);
@@ -254,7 +256,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
         }
     }
     auto sum_groups = [&]() {
-        if (signalling && reg_search) {
+        if (groups && reg_search) {
             int base = 0;
 #pragma unroll
             for (int q = 0; q < NPRE; q++) {
@@ -281,6 +283,22 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             return p.G - 1;
         }
         return find_group(p.cseg, p.G, r, lane);
+    };
+    // Slots of the group that holds slot r (MODE_RS).
+    auto group_range = [&](int r, int *first, int *count) __attribute__((always_inline)) {
+        if (reg_search) {
+            const int g = group_of(r);
+            int end = 0, begin = 0;
+#pragma unroll
+            for (int q = 0; q < NPRE; q++) {
+                if (g >> 6 == q) end = __builtin_amdgcn_readlane(pre[q], g & 63);
+                if (g > 0 && (g - 1) >> 6 == q) begin = __builtin_amdgcn_readlane(pre[q], (g - 1) & 63);
+            }
+            *first = begin;
+            *count = end - begin;
+        } else {
+            find_group_range(p.cseg, p.G, r, lane, first, count);
+        }
     };
     // Wavefront 0 announces a macro tile's reorder tiles: lane s < nsub holds the storage slot r and the group g of
     // reorder tile s (one register each; as scalars, slots and groups of this tile and of the one whose signal is
@@ -374,7 +392,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
         // requested here and rest in two registers through the K loop; the epilogue hands them to the lanes that
         // store each row.  Requested in the epilogue they cost every tile a round trip to memory with nothing to hide it.
         int32_t re_lo = 0, re_hi = 0;
-        if (MODE == MODE_SCATTER) {
+        if (MAPPED) {
             const long trow = (long)(r_mine / p.rLDN) * p.BM + (wm * 128) % p.BM;
             re_lo = p.RE[trow + lane];
             re_hi = p.RE[trow + 64 + lane];
@@ -520,10 +538,32 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             // launch behind it 16 (whole pass 52 -> 46).
             fo_u32x4 old[ACC ? NST : 1];
             char *abase = ACC ? reinterpret_cast<char *>(p.ACC) + (trow * ldp + tcol) * 2 : nullptr;
-            if (ACC && keep) {
+            // MODE_RS: the accumulator rows of the wavefront's rows, held as re_lo and re_hi are.
+            int ac_lo = 0, ac_hi = 0;
+            const bool sums = MODE == MODE_ACC || (MODE == MODE_RS && p.ACC);
+            const int own_first = MODE == MODE_RS ? p.rank * p.seg_rows : 0, own_rows = MODE == MODE_RS && p.OWN ? p.seg_rows : 0;
+            auto row_of = [&](int k, int lo, int hi) __attribute__((always_inline)) {  // row k * RPP + srow of the block: its entry sits in that lane
+                return __builtin_amdgcn_ds_bpermute((k * RPP % 64 + srow) * 4, k * RPP < 64 ? lo : hi);
+            };
+            if (MODE == MODE_RS) {
+                int first, count;
+                group_range(r, &first, &count);
+                ac_lo = rs_row(p.cseg, p.G, p.BM, p.W, p.seg_rows, re_lo, first * p.BM, count * p.BM);
+                ac_hi = rs_row(p.cseg, p.G, p.BM, p.W, p.seg_rows, re_hi, first * p.BM, count * p.BM);
+            }
+            if (sums && keep) {
 #pragma unroll
-                for (int k = 0; k < NST; k++)
-                    old[k] = *reinterpret_cast<const fo_u32x4 *>(abase + (size_t)(k * RPP) * ldp * 2 + lane_off);
+                for (int k = 0; k < NST; k++) {
+                    if (MODE == MODE_RS) {
+                        const int to = row_of(k, ac_lo, ac_hi);
+                        old[k] = *reinterpret_cast<const fo_u32x4 *>(p.ACC + (size_t)(to < 0 ? 0 : to) * ldp + tcol + scol * 8);
+                    } else {
+                        old[ACC ? k : 0] = *reinterpret_cast<const fo_u32x4 *>(abase + (size_t)(k * RPP) * ldp * 2 + lane_off);
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < (ACC ? NST : 1); k++) old[k] = fo_u32x4{0, 0, 0, 0};
             }
 #pragma unroll
             for (int i = 0; i < F; i++) {  // 16 output rows = one row of accumulator blocks
@@ -545,7 +585,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_s_waitcnt(0xC07F);
                 __builtin_amdgcn_wave_barrier();
-                if (ACC && i == 0) {
+                if (sums && i == 0) {
 #pragma unroll
                     for (int k = 0; k < NST; k++) asm volatile("" : "+v"(old[ACC ? k : 0]));
                 }
@@ -554,17 +594,25 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                 for (int ps = 0; ps < 16 / RPP; ps++) {
                     const int row = ps * RPP + srow;
                     fo_u32x4 v = *reinterpret_cast<const fo_u32x4 *>(strip + row * PITCH + scol * 8);
-                    if (MODE == MODE_SCATTER) {
-                        // row i * 16 + ps * RPP + srow of the block: its entry sits in that lane of re_lo / re_hi
-                        const long prow = __builtin_amdgcn_ds_bpermute(((i * 16 + ps * RPP) % 64 + srow) * 4,
-                                                                       i * 16 + ps * RPP < 64 ? re_lo : re_hi);
-                        if (stream_out)
-                            store16_write_through_nt(p.C + (size_t)prow * ldp + tcol + scol * 8, v);
-                        else
-                            store16_write_through(p.C + (size_t)prow * ldp + tcol + scol * 8, v);
+                    if (MAPPED) {
+                        const int k = i * (16 / RPP) + ps;
+                        const long prow = row_of(k, re_lo, re_hi);
+                        uint16_t *to = p.C + (size_t)prow * ldp + tcol + scol * 8;
+                        if (MODE == MODE_RS) {
+                            const int ac = row_of(k, ac_lo, ac_hi);
+                            if (sums && ac >= 0)
+                                store16(p.ACC + (size_t)ac * ldp + tcol + scol * 8, fo_add8<Tag>(old[ACC ? k : 0], v));
+                            if ((unsigned)(ac - own_first) < (unsigned)own_rows)
+                                store16(p.OWN + (size_t)(ac - own_first) * ldp + tcol + scol * 8, v);
+                            store16(to, v);
+                        } else if (stream_out) {
+                            store16_write_through_nt(to, v);
+                        } else {
+                            store16_write_through(to, v);
+                        }
                     } else {
                         char *sb = cbase + (size_t)(i * 16 + ps * RPP) * ldp * 2;
-                        if constexpr (ACC) {
+                        if constexpr (MODE == MODE_ACC) {
                             char *ab = abase + (size_t)(i * 16 + ps * RPP) * ldp * 2;
                             const fo_u32x4 sum = fo_add8<Tag>(old[i * (16 / RPP) + ps], v);
                             if (stream_out)

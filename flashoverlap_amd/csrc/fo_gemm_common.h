@@ -20,13 +20,16 @@ namespace fo_gemm_dev {
 
 // MODE_ACC: for a call that stays on one stream.  The tile is stored as the plain epilogue does (RA null) or reordered,
 // without counters, and ACC[o] = round16(ACC[o] + C[o]) is done for every element stored.
-enum { MODE_PLAIN = 0, MODE_SIGNAL = 1, MODE_SCATTER = 2, MODE_ACC = 3 };
+// MODE_RS: the same for a reduce-scatter (the scatter epilogue's row map, rLDN == 1): C is cut into ranges of rows, one
+// per group, and each range into W chunks of consecutive rows; row i of chunk q of a range that starts at row f is added
+// to row q * seg_rows + f / W + i of the accumulator (if any) and, for q == rank, stored to row f / W + i of OWN (if any).
+enum { MODE_PLAIN = 0, MODE_SIGNAL = 1, MODE_SCATTER = 2, MODE_ACC = 3, MODE_RS = 4 };
 
 struct GemmArgs {
     const uint16_t *A;
     const uint16_t *B;
     uint16_t *C;
-    uint16_t *ACC;         // MODE_ACC: the accumulator, addressed as C is
+    uint16_t *ACC;         // MODE_ACC, MODE_RS: the accumulator
     int M, N, K;
     int lda, ldb;          // row strides of A and B in elements (multiples of 8)
     int BM, BN, TN, rLDN;  // reorder/signal tile, tiles along N, reshaped width in tiles
@@ -40,6 +43,8 @@ struct GemmArgs {
     int first, sub_m, sub_n, count;        // this launch: positions from `first`, each cut into sub_m x sub_n macro tiles, `count` of them
     int quiet;                             // signalling epilogues: store the tiles reordered, touch no counter
     int half;                              // 256x256 kernel: half a tile is left at the end of M (bit 0), N (bit 1)
+    uint16_t *OWN;                         // MODE_RS: this rank's rows
+    int W, rank, seg_rows;                 // MODE_RS: ranks, this rank, rows of the view per rank
     int stream_out;                        // 256x256 kernel: store the output with the non-temporal hint
 };
 
@@ -67,6 +72,47 @@ __device__ __forceinline__ int find_group(const int32_t *cseg, int G, int r, int
     return G - 1;  // unreachable when sum(cseg) covers every slot (validated on the host)
 }
 
+// The same, with the group's first storage slot and its slot count.
+__device__ __forceinline__ void find_group_range(const int32_t *cseg, int G, int r, int lane, int *first, int *count) {
+    int base = 0;
+    *first = *count = 0;
+    for (int it = 0; it < G; it += 64) {
+        const int idx = it + lane, n = idx < G ? cseg[idx] : 0;
+        int s = n;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            int o = __shfl_up(s, d, 64);
+            if (lane >= d) s += o;
+        }
+        s += base;
+        unsigned long long hit = __ballot(idx < G && s > r);
+        if (hit) {
+            const int at = (int)__builtin_ctzll(hit);
+            *count = __shfl(n, at, 64);
+            *first = __shfl(s, at, 64) - *count;
+            return;
+        }
+        base = __shfl(s, 63, 64);
+    }
+}
+
+// MODE_RS: accumulator row of view row `row`, whose group holds the rows [first, first + count); -1 for a row that the
+// map sent out of its group's range and that belongs to nobody's (the host's row maps do not).
+__device__ __forceinline__ int rs_row(const int32_t *cseg, int G, int BM, int W, int seg_rows, int row, int first, int count) {
+    if (row < first || row >= first + count) {
+        first = 0;
+        int g = 0;
+        for (; g < G; g++) {
+            count = cseg[g] * BM;
+            if (row < first + count) break;
+            first += count;
+        }
+        if (g == G || row < 0) return -1;
+    }
+    const int chunk = count / W, in = row - first, q = in / chunk;
+    return q * seg_rows + first / W + (in - q * chunk);
+}
+
 // s_waitcnt vmcnt(n) only (expcnt/lgkmcnt left at their maxima); gfx9 encoding:
 // vmcnt = imm[15:14]:imm[3:0], expcnt = imm[6:4], lgkmcnt = imm[11:8].
 template <int N>
@@ -87,6 +133,9 @@ __device__ __forceinline__ void wait_vmcnt() {
 // VALU write of its data registers.
 __device__ __forceinline__ void store16_write_through(void *ptr, fo_u32x4 v) {
     asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" : : "v"(ptr), "v"(v) : "memory");
+}
+__device__ __forceinline__ void store16(void *ptr, fo_u32x4 v) {
+    asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" : : "v"(ptr), "v"(v) : "memory");
 }
 // saddr forms: wave-uniform base (SGPR pair) + 32-bit per-lane byte offset
 __device__ __forceinline__ void store16_write_through(char *base, unsigned lane_off, fo_u32x4 v) {

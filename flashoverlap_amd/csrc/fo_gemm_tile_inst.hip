@@ -1,10 +1,10 @@
 // The instantiations of the smaller-tile GEMM kernel for one type and one epilogue per translation unit: built
-// eight times with -DFO_INST_DTYPE={0,1} (fp16, bf16) and -DFO_INST_MODE={0,1,2,3} (plain, signal, scatter, accumulating epilogue).
+// ten times with -DFO_INST_DTYPE={0,1} (fp16, bf16) and -DFO_INST_MODE={0,1,2,3,4} (plain, signal, scatter, accumulating, reduce-scatter epilogue).
 #include "fo_gemm_launch.h"
 #include "fo_gemm_tile_kernel.h"
 
 #if !defined(FO_INST_DTYPE) || !defined(FO_INST_MODE)
-#error "compile with -DFO_INST_DTYPE=0|1 -DFO_INST_MODE=0|1|2|3"
+#error "compile with -DFO_INST_DTYPE=0|1 -DFO_INST_MODE=0|1|2|3|4"
 #endif
 
 namespace fo_gemm_dev {

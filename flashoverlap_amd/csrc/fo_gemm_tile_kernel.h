@@ -65,7 +65,8 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
     constexpr int WTM = TM / 2, WTN = TN / 2, FM = WTM / 16, FN = WTN / 16;  // computing wavefronts: 2 x 2
     constexpr int PA = TM / 8 / NL, PB = TN / 8 / NL, P = KB * (PA + PB);    // 1 KiB loads per loader and stage
     constexpr unsigned A_BLK = TM * 128, B_BLK = TN * 128, STAGE = KB * (A_BLK + B_BLK);
-    constexpr bool ACC = MODE == MODE_ACC, COUNTS = MODE == MODE_SIGNAL || MODE == MODE_SCATTER;
+    constexpr bool ACC = MODE == MODE_ACC || MODE == MODE_RS, COUNTS = MODE == MODE_SIGNAL || MODE == MODE_SCATTER;
+    constexpr bool MAPPED = MODE == MODE_SCATTER || MODE == MODE_RS;
     // output staging; with an accumulator the computing wavefronts store the tile and the loaders update the accumulator
     constexpr int STORERS = ACC ? kTileComputers * 64 : kTileThreads;
     constexpr int PITCH = TN + 8, CPR = TN / 8, NCH = (TM * CPR + STORERS - 1) / STORERS;
@@ -73,7 +74,8 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
     static_assert(S >= 2 && (S - 1) * P < 64 && (!ACC || (S - 3) * P + NCH < 64), "vmcnt range");
 
     extern __shared__ fo_u32x4 smem[];
-    __shared__ int32_t row_map[MODE == MODE_SCATTER ? 256 : 1];  // scatter: where the tile's rows go
+    __shared__ int32_t row_map[MAPPED ? 256 : 1];          // where the tile's rows go
+    __shared__ int32_t rs_map[MODE == MODE_RS ? 256 : 1];  // and their rows in the accumulator
     const unsigned lds0 = (unsigned)(uintptr_t)FO_LDS_PTR(smem);
     uint16_t *stage = reinterpret_cast<uint16_t *>(smem);  // the output tile, once the K loop is done
     const int tid = threadIdx.x, lane = tid & 63;
@@ -114,14 +116,6 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             r0 = RAc[tm0 * p.TN + tn0];
             r1 = two_m || two_n ? RAc[(tm0 + two_m) * p.TN + tn0 + two_n] : r0;
         }
-        // Row of the output view that the tile's row 0 has (or would have) in storage slot r, and the same for columns.
-        auto row_base = [&](int r, int rldn, bool second) __attribute__((always_inline)) {
-            return (r / rldn << bm_shift) + (second && two_m ? -split_m : m0 & (p.BM - 1));
-        };
-        auto col_base = [&](int r, int rldn, bool second) __attribute__((always_inline)) {
-            return (r % rldn << bn_shift) + (second && two_n ? -split_n : n0 & (p.BN - 1));
-        };
-
         int g0 = 0, g1 = 0;  // groups of r0 and r1 (the wavefront that signals)
         // Row and column of the output view at which the tile's row and column 0 are, or would be, in r0 and in r1.
         int row0 = m0, row1 = m0, col0 = n0, col1 = n0;
@@ -169,6 +163,24 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                 }
             }
         };
+        // The same where a map in LDS says which row of the view a row goes to.  Only rows [from, from + rows) of the view
+        // exist, and `out` is where the first of them begins; the others' pieces are left out (EVERY: read at row 0).
+        auto each_mapped_piece = [&](int t, const int32_t *map, uint16_t *out, auto every, auto act, int from = 0,
+                                     int rows = 0x7fffffff) __attribute__((always_inline)) {
+            constexpr bool EVERY = decltype(every)::value;
+            asm volatile("" : "+v"(t));
+#pragma unroll
+            for (int u = 0; u < NCH; u++) {
+                const int idx = (u * STORERS + t) % (EVERY ? TM * CPR : 1 << 30), row = idx / CPR, col = idx % CPR * 8;
+                const bool second = row >= split_m || col >= split_n;
+                if (EVERY || ((TM * CPR % STORERS == 0 || row < TM) && row >= skip_m && col >= skip_n)) {
+                    const int to = map[two_n && second ? TM + row : row] - from;
+                    if (EVERY || (unsigned)to < (unsigned)rows)
+                        act(u, row, col, out + (size_t)(to < 0 ? 0 : to) * ldp + (second ? col1 : col0) + col);
+                }
+                if (u % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // sixteen addresses at once would be too many registers
+            }
+        };
         auto piece = [&](int row, int col) __attribute__((always_inline)) {
             return *reinterpret_cast<const fo_u32x4 *>(stage + row * PITCH + col);
         };
@@ -205,7 +217,8 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             unsigned slot = (S - 1) * STAGE;
             // With an accumulator the steps behind the last request ask for its values instead of further stages: they
             // arrive while the last S - 1 stages are multiplied.
-            const int fetching = ACC ? (KT > S - 1 ? KT - (S - 1) : 0) : KT;
+            const bool sums = ACC && (MODE != MODE_RS || p.ACC);
+            const int fetching = sums ? (KT > S - 1 ? KT - (S - 1) : 0) : KT;
             for (int kt = 0; kt < fetching; kt++) {
                 request(kt + S - 1, slot);  // the slot of stage kt - 1, given up at the last barrier
                 slot = slot + STAGE == S * STAGE ? 0 : slot + STAGE;
@@ -214,37 +227,56 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                 asm volatile("" ::: "memory");
             }
             fo_u32x4 old[ACC ? NCH : 1];  // the accumulator's values
-            if constexpr (ACC) {
-                find_bases();
+            if (ACC && sums) {
                 // every wavefront loads every piece, needed or not: the waits below count
-                each_piece(wave * 64 + lane, p.ACC, std::true_type{}, [&](int u, int, int, uint16_t *at) __attribute__((always_inline)) {
-                    old[u] = *reinterpret_cast<const fo_u32x4 *>(at);
-                });
+                auto take = [&](int u, int, int, uint16_t *at) __attribute__((always_inline)) {
+                    old[ACC ? u : 0] = *reinterpret_cast<const fo_u32x4 *>(at);
+                };
+                find_bases();
+                if constexpr (MODE == MODE_RS)
+                    each_mapped_piece(wave * 64 + lane, rs_map, p.ACC, std::true_type{}, take);
+                else
+                    each_piece(wave * 64 + lane, p.ACC, std::true_type{}, take);
                 asm volatile("" ::: "memory");
 #pragma unroll
                 for (int j = 0; j < S - 1; j++) {
                     if (fetching + j < KT) {
-                        if (j < S - 2) asm volatile("s_waitcnt vmcnt(%0)" : : "i"((S - 3 - j) * P + NCH) : "memory");  // stage fetching + j + 1
+                        if (j < S - 2) asm volatile("s_waitcnt vmcnt(%0)" : : "i"(ACC ? (S - 3 - j) * P + NCH : 0) : "memory");  // stage fetching + j + 1
                         __builtin_amdgcn_s_barrier();
                         asm volatile("" ::: "memory");
                     }
                 }
-                wait_vmcnt<NCH>();
+                wait_vmcnt<ACC ? NCH : 0>();
             } else {
                 wait_vmcnt<0>();  // nothing lands in the space the output is staged in
+#pragma unroll
+                for (int u = 0; u < (ACC ? NCH : 1); u++) old[u] = fo_u32x4{0, 0, 0, 0};  // defined here, or the compiler keeps its registers across the computing wavefronts' K loop
             }
             __builtin_amdgcn_s_barrier();  // every fragment has been fetched
             asm volatile("" ::: "memory");
             if constexpr (ACC) {
                 __builtin_amdgcn_s_barrier();  // the tile has been staged
                 asm volatile("" ::: "memory");
-                // All of them are awaited, those of pieces that are not stored too: one left pending would be waited for
-                // in the next tile's K loop, with everything else in flight.
+                if (sums) {
+                    // All of them are awaited, those of pieces that are not stored too: one left pending would be waited
+                    // for in the next tile's K loop, with everything else in flight.
 #pragma unroll
-                for (int u = 0; u < NCH; u++) asm volatile("" : "+v"(old[u]));
-                each_piece(wave * 64 + lane, p.ACC, std::false_type{}, [&](int u, int row, int col, uint16_t *at) __attribute__((always_inline)) {
-                    *reinterpret_cast<fo_u32x4 *>(at) = fo_add8<Tag>(old[u], piece(row, col));
-                });
+                    for (int u = 0; u < NCH; u++) asm volatile("" : "+v"(old[u]));
+                    auto add = [&](int u, int row, int col, uint16_t *at) __attribute__((always_inline)) {
+                        *reinterpret_cast<fo_u32x4 *>(at) = fo_add8<Tag>(old[u], piece(row, col));
+                    };
+                    if constexpr (MODE == MODE_RS)
+                        each_mapped_piece(wave * 64 + lane, rs_map, p.ACC, std::false_type{}, add);
+                    else
+                        each_piece(wave * 64 + lane, p.ACC, std::false_type{}, add);
+                }
+                if (MODE == MODE_RS && p.OWN) {
+                    find_bases();
+                    each_mapped_piece(wave * 64 + lane, rs_map, p.OWN, std::false_type{},
+                                      [&](int, int row, int col, uint16_t *at) __attribute__((always_inline)) {
+                        *reinterpret_cast<fo_u32x4 *>(at) = piece(row, col);
+                    }, p.rank * p.seg_rows, p.seg_rows);
+                }
             }
         } else {
             fo_float4v acc[FM][FN];
@@ -329,12 +361,24 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             };
             __builtin_amdgcn_s_setprio(2);
             // While the first stage is on its way: row map entries, and the groups to signal.
-            if (MODE == MODE_SCATTER) {
+            if (MAPPED) {
+                int first0 = 0, count0 = 0, first1 = 0, count1 = 0;  // MODE_RS: the groups' slots
+                if (MODE == MODE_RS) {
+                    find_group_range(p.cseg, p.G, r0, lane, &first0, &count0);
+                    first1 = first0;
+                    count1 = count0;
+                    if (r1 != r0) find_group_range(p.cseg, p.G, r1, lane, &first1, &count1);
+                }
                 const int e = wave * 64 + lane;  // row e, or (two reorder tiles side by side) row e % TM of one of them
                 if (e < (two_n ? 2 * TM : TM)) {
                     const int row = two_n && e >= TM ? e - TM : e;
                     const bool second = two_n ? e >= TM : row >= split_m;
-                    row_map[e] = p.RE[row_base(second ? r1 : r0, p.rLDN, second) + row];
+                    const int r = second ? r1 : r0;
+                    const int to = p.RE[(r / p.rLDN << bm_shift) + (second && two_m ? -split_m : m0 & (p.BM - 1)) + row];
+                    row_map[e] = to;
+                    if (MODE == MODE_RS)
+                        rs_map[e] = rs_row(p.cseg, p.G, p.BM, p.W, p.seg_rows, to, (second ? first1 : first0) << bm_shift,
+                                           (second ? count1 : count0) << bm_shift);
                 }
                 asm volatile("" ::: "memory");
                 __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): written when the first barrier is passed
@@ -379,25 +423,28 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                 __builtin_amdgcn_s_waitcnt(0xC07F);
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
-                each_piece(wave * 64 + lane, p.C, std::false_type{}, [&](int, int row, int col, uint16_t *at) __attribute__((always_inline)) {
+                auto put = [&](int, int row, int col, uint16_t *at) __attribute__((always_inline)) {
                     *reinterpret_cast<fo_u32x4 *>(at) = piece(row, col);
-                });
+                };
+                if constexpr (MODE == MODE_RS)
+                    each_mapped_piece(wave * 64 + lane, row_map, p.C, std::false_type{}, put);
+                else
+                    each_piece(wave * 64 + lane, p.C, std::false_type{}, put);
             }
         }
         if constexpr (!ACC) {
             find_bases();
             __syncthreads();
-            each_piece(tid, p.C, std::false_type{}, [&](int, int row, int col, uint16_t *at) __attribute__((always_inline)) {
-                if constexpr (MODE == MODE_PLAIN) {
+            auto put = [&](int, int row, int col, uint16_t *at) __attribute__((always_inline)) {
+                if constexpr (MODE == MODE_PLAIN)
                     *reinterpret_cast<fo_u32x4 *>(at) = piece(row, col);
-                } else if constexpr (MODE == MODE_SIGNAL) {
+                else
                     store16_write_through(at, piece(row, col));
-                } else {
-                    const bool second = row >= split_m || col >= split_n;
-                    const int to_row = row_map[two_n && second ? TM + row : row];
-                    store16_write_through(p.C + (size_t)to_row * ldp + (second ? col1 : col0) + col, piece(row, col));
-                }
-            });
+            };
+            if constexpr (MODE == MODE_SCATTER)
+                each_mapped_piece(tid, row_map, p.C, std::false_type{}, put);
+            else
+                each_piece(tid, p.C, std::false_type{}, put);
         }
         if (signalling) {
             // Whole reorder tiles only (the launcher sees to it): every wavefront's write-through stores are

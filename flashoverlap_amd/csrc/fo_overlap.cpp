@@ -574,6 +574,14 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
         if (rc) return rc;
     }
     const bool quiet = same_stream && !monitor;  // as in fo_overlap_gemm_allreduce
+    // Where whole rows of the output view are this rank's, the GEMM's epilogue also does what follows it: a copy per
+    // group (4-5 us each on this GPU) and the consumer.  2048x4096x2048, four groups, eight ranks, no accumulator, whole pass
+    // with the normalisation: 42.0 us with copies, 37.5 so.
+    if (quiet && rLDN == 1 && info[0] % W == 0 && !(((uintptr_t)C | (uintptr_t)D | (uintptr_t)h->acc) & 15)) {
+        rc = fo_gemm_reduce_scatter(dtype, M, N, K, cseg_dev, G, A, B, C, h->acc, D, RA, RE, W, h->rank, algo, h->gemm_stream);
+        if (rc) return rc;
+        return link_time(h, (int64_t)M * N * 2, h->gemm_stream);
+    }
     rc = quiet ? fo_gemm_reordered_quiet(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, RA, RE, algo,
                                          h->gemm_stream)
                : fo_gemm_scatter(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, MM, RA, RE, monitor, algo,

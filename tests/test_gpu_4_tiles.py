@@ -116,3 +116,51 @@ def test_accumulating_epilogue(fo, dtype, bm, bn, M, N, K):
         assert torch.equal(acc.reshape(-1), (before.float() + C.float()).to(td).reshape(-1))
     assert (MM == 0).all()
     ov.close()
+
+
+@pytest.mark.parametrize("dtype,bm,bn,M,N,K", CASES)
+@pytest.mark.parametrize("W", [1, 8])
+def test_reduce_scatter_epilogue(fo, dtype, bm, bn, M, N, K, W):
+    """A reduce-scatter on one stream, with and without an accumulator: product, this rank's rows and the
+    accumulator's W segments against the definition, group by group."""
+    ops, layout, td = fo.ops, fo.layout, TORCH_DTYPE[dtype]
+    algo = fo._capi.find_algo(bm, bn, swizzle=4)
+    TM, TN = M // bm, N // bn
+    T = TM * TN
+    A, _ = seeded((M, K), dtype, M + K)
+    B, _ = seeded((N, K), dtype, N + K, scale=K ** -0.5)
+    before, _ = seeded((M * N,), dtype, 7)
+    acc = before.clone()
+    plain = torch.empty(M, N, device="cuda", dtype=td)
+    ops.gemm(A, B, plain, algo)
+    cseg = [T] if T < 3 else [1, T // 2, T - 1 - T // 2]
+    if T > 600:
+        cseg = [1] * 300 + [T - 300]  # more groups than the 256x256 kernel holds in registers
+    RA = torch.from_numpy(np.random.default_rng(M + N).permutation(T).astype(np.int32)).reshape(TM, TN).cuda()
+    RE = layout.generate_row_mapping(M, N, bm, bn, cseg, W)
+    cs_cpu = torch.tensor(cseg, dtype=torch.int32)
+    MM = torch.zeros(layout.counter_size(len(cseg), TM, TN), dtype=torch.int32, device="cuda")
+    rank = W - 1
+    ov = ops.Overlap(rank=rank, world=W)
+    ov.set_schedule(in_stream_below_flop=1e15)
+    for with_acc in (True, False):
+        ov.set_accumulator(acc if with_acc else None)
+        C = torch.full((M * N,), float("nan"), device="cuda", dtype=td)
+        D = torch.full((M // W, N), float("nan"), device="cuda", dtype=td)
+        ov.gemm_reducescatter_overlap(A, B, C, D, MM, RA, RE, 1, cs_cpu, cs_cpu.cuda(), algo)
+        torch.cuda.synchronize()
+        assert torch.equal(layout.unpermute(C, M, N, bm, bn, RA, RE=RE), plain)
+        rows, seg = C.view(-1, bn), M * N // bn // W
+        want, own = torch.empty_like(rows), []
+        first = 0
+        for n in cseg:
+            chunk = rows[first:first + n * bm].view(W, n * bm // W, bn)
+            for q in range(W):
+                want[q * seg + first // W:q * seg + (first + n * bm) // W] = chunk[q]
+            own.append(chunk[rank])
+            first += n * bm
+        assert torch.equal(D.view(-1, bn), torch.cat(own))
+        if with_acc:
+            assert torch.equal(acc, (before.float() + want.reshape(-1).float()).to(td))
+    assert (MM == 0).all()
+    ov.close()
