@@ -3,11 +3,13 @@
 There is no CPU fallback: if the library has not been built, loading raises.
 """
 import ctypes
+import importlib.util
 import os
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 KERNEL_LIB = os.path.join(_PKG, "lib", "libfo_kernels.so")
 SHIM_LIB = os.path.join(_PKG, "lib", "libst_pybinding.so")
+NATIVE_LIB = os.path.join(_PKG, "lib", "_fo_native.so")
 
 F16, BF16 = 0, 1
 
@@ -100,6 +102,24 @@ def lib():
             fn.argtypes = args
         _lib = L
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The extension module with the per-call host path (csrc/fo_native.cpp).  Its functions return None, with nothing
+    enqueued, for arguments that the Python path has to look at."""
+    global _native
+    if _native is None:
+        if not os.path.exists(NATIVE_LIB):
+            raise ImportError(f"{NATIVE_LIB} is missing: build it with `python -m flashoverlap_amd.build`")
+        import torch  # noqa: F401  the module links against torch's libraries
+        spec = importlib.util.spec_from_file_location("flashoverlap_amd._fo_native", NATIVE_LIB)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _native = module
+    return _native
 
 
 def check(code, what):

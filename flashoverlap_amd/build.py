@@ -8,7 +8,10 @@
                       file name is the one the reference scripts load
                       (example/RMSNorm.py:5, README.md:69)
 
-Both land in flashoverlap_amd/lib/; the shim is also copied to build/lib/ so that
+  _fo_native.so       Python extension module: the per-call host path of ops.py and
+                      layers.py (argument checks, output allocation, one call of the C ABI)
+
+All land in flashoverlap_amd/lib/; the shim is also copied to build/lib/ so that
 `torch.ops.load_library("../build/lib/libst_pybinding.so")` keeps working from a
 sub-directory of the repository root.
 
@@ -18,6 +21,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 PKG = os.path.dirname(os.path.abspath(__file__))
@@ -27,6 +31,7 @@ LIBDIR = os.path.join(PKG, "lib")
 OBJDIR = os.path.join(LIBDIR, "obj")
 KERNEL_LIB = os.path.join(LIBDIR, "libfo_kernels.so")
 SHIM_LIB = os.path.join(LIBDIR, "libst_pybinding.so")
+NATIVE_LIB = os.path.join(LIBDIR, "_fo_native.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
@@ -73,26 +78,36 @@ def build_kernels(extra_flags=()):
     return KERNEL_LIB
 
 
-def build_shim():
+def _build_torch_lib(src, out, includes=(), libs=()):
+    """One g++ source against torch's headers and libraries and libfo_kernels.so."""
     import torch
     from torch.utils import cpp_extension
 
     os.makedirs(OBJDIR, exist_ok=True)
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
     incs = []
-    for p in cpp_extension.include_paths():
+    for p in list(cpp_extension.include_paths()) + list(includes):
         incs += ["-isystem", p]
     abi = int(getattr(torch._C, "_GLIBCXX_USE_CXX11_ABI", True))
-    obj = os.path.join(OBJDIR, "fo_torch_shim.o")
-    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-c", os.path.join(CSRC, "fo_torch_shim.cpp"),
+    obj = os.path.join(OBJDIR, os.path.splitext(src)[0] + ".o")
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-c", os.path.join(CSRC, src),
           "-o", obj, "-I" + os.path.join(ROOT, "include"), "-isystem", "/opt/rocm/include",
           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
           "-Wno-deprecated-declarations"] + incs)
-    _run(["g++", "-shared", "-fPIC", "-o", SHIM_LIB, obj,
+    _run(["g++", "-shared", "-fPIC", "-o", out, obj,
           "-L" + LIBDIR, "-lfo_kernels", "-Wl,-rpath,$ORIGIN",
-          "-L" + torch_lib, "-ltorch", "-ltorch_cpu", "-lc10", "-ltorch_hip", "-lc10_hip",
+          "-L" + torch_lib, *libs, "-ltorch", "-ltorch_cpu", "-lc10", "-ltorch_hip", "-lc10_hip",
           "-Wl,-rpath," + torch_lib,
           "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib"])
+    return out
+
+
+def build_native():
+    return _build_torch_lib("fo_native.cpp", NATIVE_LIB, [sysconfig.get_paths()["include"]], ["-ltorch_python"])
+
+
+def build_shim():
+    _build_torch_lib("fo_torch_shim.cpp", SHIM_LIB)
     dst_dir = os.path.join(ROOT, "build", "lib")
     os.makedirs(dst_dir, exist_ok=True)
     # Same directory layout as the reference build output; both libraries are
@@ -105,7 +120,7 @@ def build_shim():
 def build_all(shim=True):
     out = [build_kernels()]
     if shim:
-        out.append(build_shim())
+        out += [build_shim(), build_native()]
     return out
 
 

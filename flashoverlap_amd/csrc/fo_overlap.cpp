@@ -365,6 +365,12 @@ int last_slots(const int32_t *RA_host, int TM, int TN, std::vector<long> &last_s
     return FO_OK;
 }
 
+int check_slots(const int32_t *RA_host, int T) {  // FO_ERR_ARG for an entry outside [0, T)
+    uint32_t most = 0;
+    for (int t = 0; t < T; t++) most = (uint32_t)RA_host[t] > most ? (uint32_t)RA_host[t] : most;
+    return most < (uint32_t)T ? FO_OK : FO_ERR_ARG;
+}
+
 int norm_ready_rows(const norm_plan &np, long *last_slot, int TM, long done, bool final_batch, int dtype, const void *C,
                     int M, int N, int BM, int BN, int rLDN, const int32_t *RA, bool beside_gemm, fo_stream_t stream) {
     std::vector<int> runs;
@@ -397,11 +403,14 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
     if (np) {
         if (!np->Y || !np->Wt || !np->RA_host) return FO_ERR_ARG;
         if (N % 8 || N > 16384 || (int64_t)M * N * 2 > 0xFFFFFFFFLL) return FO_ERR_SHAPE;
-        rc = last_slots(np->RA_host, TM, TN, last_slot);
-        if (rc) return rc;
     }
 
     const bool same_stream = in_stream(h, M, N, K);
+    if (np) {
+        // on one stream all rows follow in one launch, whatever their slots
+        rc = same_stream ? check_slots(np->RA_host, TM * TN) : last_slots(np->RA_host, TM, TN, last_slot);
+        if (rc) return rc;
+    }
     const int fused = same_stream ? 0 : fused_grid(h, G);
     fo_stream_t cstream = same_stream ? h->gemm_stream : h->comm_stream;
     int32_t wave = 0;
@@ -411,7 +420,7 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
         rc = fo_gemm_wave_tiles(dtype, algo, M, N, &wave);
         if (rc) return rc;
     }
-    const bool captured = capturing(h);
+    const bool captured = !same_stream && capturing(h);
     if (!same_stream) {
         rc = fork(h, captured, fused != 0);
         if (rc) return rc;
@@ -467,9 +476,12 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
             if (rc) return rc;
             off += n;
             done += tiles;
-            if (np) {
+            if (np && same_stream) {
+                rc = norm_tile_rows(*np, dtype, C, M, N, info[0], info[1], rLDN, RA, 0, TM, false, cstream);
+                if (rc) return rc;
+            } else if (np) {
                 rc = norm_ready_rows(*np, last_slot.data(), TM, done, j == G, dtype, C, M, N, info[0], info[1], rLDN, RA,
-                                     j < G && !same_stream, cstream);
+                                     j < G, cstream);
                 if (rc) return rc;
             }
             i = j;
@@ -568,7 +580,7 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
         rc = fo_gemm_wave_tiles(dtype, algo, M, N, &wave);
         if (rc) return rc;
     }
-    const bool captured = capturing(h);
+    const bool captured = !same_stream && capturing(h);
     if (!same_stream) {
         rc = fork(h, captured, fused != 0);
         if (rc) return rc;

@@ -222,6 +222,8 @@ struct OverlapImpl : torch::CustomClassHolder {
     void set_link_rate(double gigabytes_per_second) {
         check(fo_overlap_set_link_rate(h, gigabytes_per_second), "set_link_rate");
     }
+    // addition: the C handle, for the layers' native call path; valid as long as this object.
+    int64_t handle() { return reinterpret_cast<int64_t>(h); }
     // addition: whether a bounded device-side wait gave up since the last query (synchronises).
     int64_t status() {
         int32_t gave_up = 0;
@@ -360,6 +362,7 @@ TORCH_LIBRARY(flashoverlap_class, m) {
         .def("clear_accumulator", &OverlapImpl::clear_accumulator)
         .def("set_fused_consumer", &OverlapImpl::set_fused_consumer)
         .def("set_link_rate", &OverlapImpl::set_link_rate)
+        .def("handle", &OverlapImpl::handle)
         .def("status", &OverlapImpl::status);
 }
 

@@ -55,7 +55,11 @@ class ReorderRMSNorm(nn.Module):
         self.reorder_array = reorder_indices(tm * tn, hint, device=device).reshape((tm, tn))
 
     def forward(self, x):
-        out = torch.empty_like(x)
+        out = _capi.native().reorder_rmsnorm_layer(x, self._parameters.get("weight"), self.bm, self.bn, self.reorder_array,
+                                                   self.eps)
+        if out is not None:
+            return out
+        out = torch.empty_like(x)  # an argument the native path leaves to this one, or refused
         torch.ops.flashoverlap_op.reorder_rmsnorm_eps(x, out, self.weight, self.bm, self.bn, 1,
                                                       self.reorder_array, self.eps)
         return out
@@ -115,8 +119,22 @@ class OverlapRowParallelLayer(nn.Module):
             self.row_array = generate_row_mapping(M, out_features, BM, BN, cseg, world_size, device=device)
         else:
             self.row_array = None
+        self._handle = (None, 0)  # an OverlapImpl and its C handle
 
     def forward(self, x):
+        impl = self.overlap_class
+        if self._handle[0] is not impl:
+            self._handle = (impl, impl.handle())
+        if self.comm_op == "all_reduce":
+            out = _capi.native().allreduce_layer(self._handle[1], x, self._parameters.get("weight"), self.counter,
+                                                 self.reorder_array, self.cseg_cpu, self.cseg_gpu, self.algo)
+        else:
+            out = _capi.native().reducescatter_layer(self._handle[1], x, self._parameters.get("weight"), self.counter,
+                                                     self.reorder_array, self.row_array, self.cseg_cpu, self.cseg_gpu,
+                                                     self.algo, self.world_size)
+        if out is not None:
+            return out
+        # an argument the native path leaves to this one, or refused
         n = self.weight.size(0)
         if self.comm_op == "all_reduce":
             out = torch.empty((x.size(0), n), dtype=x.dtype, device=x.device)

@@ -6,7 +6,7 @@ import ctypes
 import torch
 
 from . import _capi
-from ._capi import F16, BF16, check, lib
+from ._capi import F16, BF16, check, lib, native
 from .layout import counter_size
 
 
@@ -185,6 +185,11 @@ def _check_norm(X, Y, Wt):
 
 
 def reorder_rmsnorm(X, Y, Wt, BM, BN, rldn, RA, eps=1e-5, stream=None):
+    if stream is None:
+        rc = native().reorder_rmsnorm(X, Y, Wt, BM, BN, rldn, RA, eps)
+        if rc is not None:
+            check(rc, "fo_reorder_rmsnorm")
+            return
     _check_norm(X, Y, Wt)
     bs, dim = X.shape
     if BM <= 0 or BN <= 0 or bs % BM or dim % BN:
@@ -297,6 +302,10 @@ class Overlap:
 
     def gemm_allreduce_overlap(self, A, B, C, MM, RA, rLDN, cseg_cpu, cseg_gpu, algo,
                                monitor=False):
+        rc = native().allreduce(self._h.value, A, B, C, MM, RA, rLDN, cseg_cpu, cseg_gpu, algo, monitor, self._acc)
+        if rc is not None:
+            check(rc, "fo_overlap_gemm_allreduce")
+            return
         M, N, K = self._check_call(A, B, C, MM, RA, rLDN, cseg_cpu, cseg_gpu, algo, monitor)
         TM, TN = RA.shape
         check(lib().fo_overlap_gemm_allreduce(
@@ -310,6 +319,11 @@ class Overlap:
         """gemm_allreduce_overlap + reorder_rmsnorm(C -> Y) in one call: the rows are normalised on the consumer
         stream as the groups that complete them have been consumed.  RA_cpu: host copy of RA (None: copied here,
         which synchronises)."""
+        rc = native().allreduce_norm(self._h.value, A, B, C, MM, RA, RA_cpu, rLDN, cseg_cpu, cseg_gpu, algo, monitor,
+                                     self._acc, Y, Wt, eps)
+        if rc is not None:
+            check(rc, "fo_overlap_gemm_allreduce_norm")
+            return
         M, N, K = self._check_call(A, B, C, MM, RA, rLDN, cseg_cpu, cseg_gpu, algo, monitor)
         TM, TN = RA.shape
         if RA_cpu is None:
@@ -327,6 +341,11 @@ class Overlap:
 
     def gemm_reducescatter_overlap(self, A, B, C, D, MM, RA, RE, rLDN, cseg_cpu, cseg_gpu, algo,
                                    monitor=False):
+        rc = native().reducescatter(self._h.value, A, B, C, D, MM, RA, RE, rLDN, cseg_cpu, cseg_gpu, algo, monitor,
+                                    self._acc, self.world)
+        if rc is not None:
+            check(rc, "fo_overlap_gemm_reducescatter")
+            return
         M, N, K = self._check_call(A, B, C, MM, RA, rLDN, cseg_cpu, cseg_gpu, algo, monitor, RE=RE, D=D)
         TM, TN = RA.shape
         check(lib().fo_overlap_gemm_reducescatter(
