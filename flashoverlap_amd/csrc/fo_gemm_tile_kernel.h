@@ -70,6 +70,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
     // output staging; with an accumulator the computing wavefronts store the tile and the loaders update the accumulator
     constexpr int STORERS = ACC ? kTileComputers * 64 : kTileThreads;
     constexpr int PITCH = TN + 8, CPR = TN / 8, NCH = (TM * CPR + STORERS - 1) / STORERS;
+    static_assert(STORERS % CPR || TM * CPR < STORERS || TM * CPR % STORERS == 0, "a piece per thread and step, none behind the tile");
     static_assert(BK % 64 == 0 && TM % 32 == 0 && TN % 32 == 0, "whole 1 KiB loads for every loader");
     static_assert(S >= 2 && (S - 1) * P < 64 && (!ACC || (S - 3) * P + NCH < 64), "vmcnt range");
 
@@ -142,6 +143,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
         auto each_piece = [&](int t, uint16_t *out, auto every, auto act) __attribute__((always_inline)) {
             constexpr bool EVERY = decltype(every)::value;
             asm volatile("" : "+v"(t));
+            if (EVERY && TM * CPR < STORERS) t %= TM * CPR;  // threads beyond the tile's pieces read some of them again, nothing behind the tile
             if (simple) {
                 uint16_t *base = out + (size_t)row0 * ldp + col0;
 #pragma unroll

@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
 CASES = [  # dtype, reorder tile, M, N, K                workgroup tile
     (F16, 128, 128, 128, 256, 8),                      # 32x32, one chunk of K
     (BF16, 128, 256, 256, 1024, 1544),                 # 32x32, parts of a 128x256 reorder tile, counted behind the launch
+    (BF16, 128, 128, 128, 1024, 1000),                 # 32x32, accumulator no larger than an allocation's granule
     (F16, 128, 128, 128, 3072, 136),                   # 64x32
     (BF16, 256, 128, 256, 2944, 1672),                 # 64x64
     (F16, 128, 128, 384, 3200, 200),                   # 64x96, across reorder tiles and moved back along N
