@@ -1,6 +1,7 @@
 // Host orchestration of the overlap path: the counterpart of class OverlapImpl
 // (src/overlap_impl.h:12-43, src/overlap_impl.cu) behind a C handle.  Two HIP
 // streams; every call only enqueues work and returns.  May be captured into a HIP graph.
+#include <initializer_list>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -135,6 +136,21 @@ int check_segments(const int32_t *cseg_host, int G, long tiles) {
         sum += cseg_host[i];
     }
     return sum == tiles ? FO_OK : FO_ERR_SEGMENTS;
+}
+
+// Whether `out` (elements of 16 bits) shares no memory with any of the others.  A GEMM whose epilogue also writes `out`
+// writes it while other workgroups still read operands; one that is followed by a consumer does not.
+struct span {
+    const void *p;
+    int64_t n;
+};
+bool apart(span out, std::initializer_list<span> others) {
+    const uintptr_t a = (uintptr_t)out.p, a_end = a + out.n * 2;
+    for (const span &o : others) {
+        const uintptr_t b = (uintptr_t)o.p;
+        if (out.p && o.p && a < b + o.n * 2 && b < a_end) return false;
+    }
+    return true;
 }
 
 // While the GEMM stream is being captured into a HIP graph the two streams are tied
@@ -430,7 +446,8 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
     // the counters alone (they stay zero, as the waits would have left them).
     const bool quiet = same_stream && !monitor;
     // With nothing to wait for, the GEMM's epilogue does the consumer's work on the tile it holds in LDS.
-    const bool consumed = quiet && h->acc;
+    const int64_t mn = (int64_t)M * N;
+    const bool consumed = quiet && h->acc && apart({h->acc, mn}, {{A, (int64_t)M * K}, {B, (int64_t)N * K}, {C, mn}});
     rc = consumed ? fo_gemm_accumulate(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, h->acc, RA, algo, h->gemm_stream)
          : quiet  ? fo_gemm_reordered_quiet(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, RA, nullptr, algo,
                                             h->gemm_stream)
@@ -589,7 +606,9 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     // Where whole rows of the output view are this rank's, the GEMM's epilogue also does what follows it: a copy per
     // group (4-5 us each on this GPU) and the consumer.  2048x4096x2048, four groups, eight ranks, no accumulator, whole pass
     // with the normalisation: 42.0 us with copies, 37.5 so.
-    if (quiet && rLDN == 1 && info[0] % W == 0 && !(((uintptr_t)C | (uintptr_t)D | (uintptr_t)h->acc) & 15)) {
+    const span a = {A, (int64_t)M * K}, b = {B, (int64_t)N * K}, prod = {C, (int64_t)M * N}, sum = {h->acc, (int64_t)M * N};
+    if (quiet && rLDN == 1 && info[0] % W == 0 && !(((uintptr_t)C | (uintptr_t)D | (uintptr_t)h->acc) & 15) &&
+        apart(sum, {a, b, prod}) && apart({D, seg_stride}, {a, b, prod, sum})) {
         rc = fo_gemm_reduce_scatter(dtype, M, N, K, cseg_dev, G, A, B, C, h->acc, D, RA, RE, W, h->rank, algo, h->gemm_stream);
         if (rc) return rc;
         return link_time(h, (int64_t)M * N * 2, h->gemm_stream);
@@ -666,8 +685,11 @@ extern "C" int fo_overlap_gemm_allreduce_serial(fo_overlap_t *h, int dtype, int 
     if (!h) return FO_ERR_ARG;
     if (!h->gemm_ready) return FO_ERR_STATE;
     if (h->acc && h->acc_nelem < (int64_t)M * N) return FO_ERR_ARG;
-    int rc = h->acc ? fo_gemm_accumulate(dtype, M, N, K, 1, nullptr, 0, A, B, C, h->acc, nullptr, algo, h->gemm_stream)
-                    : fo_gemm(dtype, M, N, K, A, B, C, algo, h->gemm_stream);
+    const int64_t mn = (int64_t)M * N;
+    const bool consumed = h->acc && apart({h->acc, mn}, {{A, (int64_t)M * K}, {B, (int64_t)N * K}, {C, mn}});
+    int rc = consumed ? fo_gemm_accumulate(dtype, M, N, K, 1, nullptr, 0, A, B, C, h->acc, nullptr, algo, h->gemm_stream)
+                      : fo_gemm(dtype, M, N, K, A, B, C, algo, h->gemm_stream);
+    if (!rc && h->acc && !consumed) rc = fo_consumer_reduce(dtype, C, h->acc, mn, h->gemm_stream);
     if (rc) return rc;
     return link_time(h, (int64_t)M * N * 2, h->gemm_stream);
 }

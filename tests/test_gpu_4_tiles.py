@@ -165,3 +165,43 @@ def test_reduce_scatter_epilogue(fo, dtype, bm, bn, M, N, K, W):
             assert torch.equal(acc, (before.float() + want.reshape(-1).float()).to(td))
     assert (MM == 0).all()
     ov.close()
+
+
+@pytest.mark.parametrize("alias", ["C", "A"])
+def test_accumulator_in_an_operand_or_the_product(fo, alias):
+    """An accumulator that shares memory with an operand or with the product is updated behind the GEMM, not by it."""
+    ops, M, N = fo.ops, 256, 512
+    algo = fo._capi.find_algo(128, 128, swizzle=4)
+    A, _ = seeded((M, N), F16, 1)
+    B, _ = seeded((N, N), F16, 2, scale=N ** -0.5)
+    plain = torch.empty(M, N, device="cuda", dtype=torch.float16)
+    ops.gemm(A, B, plain, algo)
+    cs = torch.tensor([M // 128 * (N // 128)], dtype=torch.int32)
+    RA = torch.arange(int(cs[0]), dtype=torch.int32, device="cuda").reshape(M // 128, N // 128)
+    MM = torch.zeros(fo.layout.counter_size(1, M // 128, N // 128), dtype=torch.int32, device="cuda")
+    RE = fo.layout.generate_row_mapping(M, N, 128, 128, [int(cs[0])], 1)
+    for call in ("serial", "overlap", "scatter"):
+        C = torch.empty_like(plain)
+        a = A.clone()
+        acc = C if alias == "C" else a
+        D = torch.empty_like(plain)
+        ov = ops.Overlap()
+        ov.set_accumulator(acc)
+        if call == "serial":
+            ov.gemm_allreduce(a, B, C, algo)
+        elif call == "overlap":
+            ov.gemm_allreduce_overlap(a, B, C, MM, RA, 1, cs, cs.cuda(), algo)
+        else:
+            ov.gemm_reducescatter_overlap(a, B, C, D, MM, RA, RE, 1, cs, cs.cuda(), algo)
+        torch.cuda.synchronize()
+        if alias == "A":
+            product = C
+            want = (A.float().reshape(-1) + C.float().reshape(-1)).half()
+        else:
+            product = C / 2  # exact: the product added to itself
+            want = C.reshape(-1)
+        product = product.reshape(-1) if call == "serial" else fo.layout.unpermute(
+            product.reshape(-1), M, N, 128, 128, RA, RE=RE if call == "scatter" else None)
+        assert torch.equal(product.reshape(-1), plain.reshape(-1)), call
+        assert torch.equal(acc.reshape(-1), want), call
+        ov.close()
