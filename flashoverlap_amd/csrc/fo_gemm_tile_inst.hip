@@ -22,10 +22,22 @@ typedef fo_bf16_tag inst_tag;
 // in steps of 128 columns where a tile's step of 64 is too short to hide a barrier in.
 int FO_CAT3(fo_gemm_tile_launch_, FO_INST_DTYPE, _, FO_INST_MODE)(const GemmArgs &a, int tm, int tn, hipStream_t stream,
                                                               int *resident_out, int expect_resident) {
-#define FO_TILE(TM_, TN_, BK_, S_)                                                                                       \
+#define FO_TILE(TM_, TN_, BK_, S_) FO_TILE_(TM_, TN_, BK_, S_, false)
+#define FO_TILE_(TM_, TN_, BK_, S_, SHIFT_)                                                                                       \
     if (tm == TM_ && tn == TN_)                                                                                          \
-        return launch_kernel<fo_gemm_tile_kernel<inst_tag, TM_, TN_, BK_, S_, FO_INST_MODE>,                             \
+        return launch_kernel<fo_gemm_tile_kernel<inst_tag, TM_, TN_, BK_, S_, FO_INST_MODE, SHIFT_>,                     \
                              tile_smem_bytes<TM_, TN_, BK_, S_>(), kTileThreads>(a, stream, resident_out, expect_resident);
+    // Operand rows that do not begin on 128-byte lines: the form that loads whole lines, for the tiles whose stages leave
+    // LDS for one more in flight beside the two a step then reads.
+    if (((uintptr_t)a.A | (uintptr_t)a.B | (unsigned)a.lda * 2) & 127) {
+        FO_TILE_(32, 32, 128, 8, true)
+        FO_TILE_(64, 32, 128, 6, true)
+        FO_TILE_(64, 64, 128, 4, true)
+        FO_TILE_(64, 96, 64, 7, true)
+        FO_TILE_(64, 128, 64, 6, true)
+        FO_TILE_(96, 128, 64, 5, true)
+        FO_TILE_(128, 128, 64, 4, true)
+    }
     FO_TILE(32, 32, 128, 8)
     FO_TILE(64, 32, 128, 6)
     FO_TILE(64, 64, 128, 4)
@@ -37,6 +49,7 @@ int FO_CAT3(fo_gemm_tile_launch_, FO_INST_DTYPE, _, FO_INST_MODE)(const GemmArgs
     FO_TILE(128, 256, 64, 3)
     FO_TILE(256, 128, 64, 3)
 #undef FO_TILE
+#undef FO_TILE_
     return FO_ERR_ALGO;
 }
 

@@ -21,6 +21,16 @@
 // 128x4096x1024 10.4 -> 4.5, 128x1024x8192 71 -> 12.5, 2048x4096x4096 62 -> 55.  512x4096x4096 with the MFMAs taken
 // out takes 18.7 us: the rest of its time is the operand stream.
 //
+// SHIFT: operand rows that do not begin on 128-byte lines (K no multiple of 64, or an operand's own address).  A load of
+// eight rows x 128 bytes then touches sixteen lines instead of eight, and the operand stream, which is what bounds these
+// sizes, slows down by 30 to 40 %.  Shifted, the loaders fetch whole lines: row r's stage begins at the line that holds
+// the stage's first column, up to seven chunks early, and a computing lane whose chunk lies behind that line's end
+// takes it from the following block (all its fragments belong to rows 16 apart, so that is a constant of the lane).
+// A step thus reads its own stage and the next, which costs one stage of the ones in flight; the products and their
+// order are the same.  K = 4088 against 4096 (us): 512x4096 30.4 -> 22.6 against 22.2, 1024x4096 41.4 -> 34.5 against 32.5,
+// 128x4096 15.4 -> 13.2 against 12.3.  Tiles with room for three stages only (128x192 and larger) keep the plain
+// form: with both stages of a step awaited, nothing would be in flight.
+//
 // MODE_ACC, the epilogue of calls that stay on one stream: what the consumer kernel would do behind the GEMM (read C and
 // the accumulator, write the accumulator) is done on the tile in LDS.  The loaders, idle by then, request the
 // accumulator's values while the last S - 1 stages are multiplied and write the sums; the computing wavefronts store
@@ -50,13 +60,19 @@ template <> struct fo_mfma16<fo_bf16_tag> {
 
 constexpr int kTileLoaders = 4, kTileComputers = 4, kTileThreads = (kTileLoaders + kTileComputers) * 64;
 
+// Columns, in chunks of 8, by which row `row` (0..15) of an operand that begins at `base` lies behind the start of its
+// 128-byte line.  The same for rows 8 apart, whatever the leading dimension (a multiple of 8).
+__device__ __forceinline__ int row_shift(const uint16_t *base, int ld, int row) {
+    return (int)(((uintptr_t)base >> 4) + (unsigned)(row * (ld >> 3))) & 7;
+}
+
 // S operand slots; the output tile is staged in the same space once the K loop is done.
 template <int TM, int TN, int BK, int S>
 constexpr int tile_smem_bytes() {
     return S * (TM + TN) * BK * 2 > TM * (TN + 8) * 2 ? S * (TM + TN) * BK * 2 : TM * (TN + 8) * 2;
 }
 
-template <typename Tag, int TM, int TN, int BK, int S, int MODE>
+template <typename Tag, int TM, int TN, int BK, int S, int MODE, bool SHIFT>
 __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs p) {
     typedef fo_elem<Tag> E;
     typedef fo_mfma16<Tag> X;
@@ -72,6 +88,10 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
     constexpr int PITCH = TN + 8, CPR = TN / 8, NCH = (TM * CPR + STORERS - 1) / STORERS;
     static_assert(STORERS % CPR || TM * CPR < STORERS || TM * CPR % STORERS == 0, "a piece per thread and step, none behind the tile");
     static_assert(BK % 64 == 0 && TM % 32 == 0 && TN % 32 == 0, "whole 1 KiB loads for every loader");
+    // Loads that may be in flight while a K step is multiplied whose successor is to be ready: all stages behind that one
+    // or, shifted, behind the first 64 columns of the stage that follows it.
+    constexpr int FLIGHT = SHIFT ? (S - 3) * P + (KB - 1) * (P / KB) : (S - 2) * P;
+    static_assert(!SHIFT || (S >= 4 && KB <= 2), "a shifted step reads two stages, one more has to be in flight");
     static_assert(S >= 2 && (S - 1) * P < 64 && (!ACC || (S - 3) * P + NCH < 64), "vmcnt range");
 
     extern __shared__ fo_u32x4 smem[];
@@ -190,11 +210,18 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
         if (loader) {
             // Load u of a 64-column block brings rows (u * NL + wave) * 8 + lane / 8 of an operand, 128 bytes each; LDS
             // slot `lane` of the 1 KiB block is (row lane / 8, chunk lane % 8) and receives chunk phys ^ key(row).
-            const int lrow = lane >> 3, lchunk = (lane & 7) ^ (((wave * 8 + lrow) >> 1) & 7);
-            const unsigned lane_off = (unsigned)((wave * 8 + lrow) * p.lda * 2 + lchunk * 16);
+            // Shifted, slot `lane` receives chunk (phys - key(row) + shift(row)) % 8 of the row's aligned line: what lies
+            // before the row's first column or behind its last is requested out of range (zeros).
+            const int lrow = lane >> 3, lkey = ((wave * 8 + lrow) >> 1) & 7;
+            const uint16_t *a0 = p.A + (size_t)m0 * p.lda, *b0 = p.B + (size_t)n0 * p.ldb;
+            const int a_shift = SHIFT ? row_shift(a0, p.lda, lrow) : 0, b_shift = SHIFT ? row_shift(b0, p.ldb, lrow) : 0;
+            const int a_chunk = SHIFT ? ((lane - lkey + a_shift) & 7) - a_shift : (lane & 7) ^ lkey;
+            const int b_chunk = SHIFT ? ((lane - lkey + b_shift) & 7) - b_shift : (lane & 7) ^ lkey;
+            constexpr int LEAD = SHIFT ? 128 : 0;  // the range starts a line early: no lane's offset is negative
+            const unsigned lane_row = (unsigned)((wave * 8 + lrow) * p.lda * 2 + LEAD);
             const unsigned row_step = (unsigned)(NL * 8 * p.lda * 2);
-            const fo_srd_t ra = fo_make_srd(p.A + (size_t)m0 * p.lda, (unsigned)TM * p.lda * 2);
-            const fo_srd_t rb = fo_make_srd(p.B + (size_t)n0 * p.ldb, (unsigned)TN * p.ldb * 2);
+            const fo_srd_t ra = fo_make_srd(a0 - LEAD / 2, (unsigned)TM * p.lda * 2 + LEAD);
+            const fo_srd_t rb = fo_make_srd(b0 - LEAD / 2, (unsigned)TN * p.ldb * 2 + LEAD);
             const unsigned wave_lds = lds0 + wave * 1024;
             auto request = [&](int kt, unsigned slot_v) __attribute__((always_inline)) {
                 const unsigned slot = __builtin_amdgcn_readfirstlane(slot_v);  // uniform by construction; said so for the assembly's operands
@@ -202,29 +229,31 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                 for (int kb = 0; kb < KB; kb++) {
                     const int col = __builtin_amdgcn_readfirstlane(kt * BK + kb * 64);
                     // chunks beyond K (a partial last step, stages behind the last) are requested out of range: zeros
-                    const unsigned voff = lchunk * 8 < p.K - col ? lane_off : 0x80000000u;
+                    const unsigned a_off = (SHIFT ? (unsigned)(col + a_chunk * 8) < (unsigned)p.K : a_chunk * 8 < p.K - col) ? lane_row + a_chunk * 16 : 0x80000000u;
+                    const unsigned b_off = !SHIFT ? a_off : (unsigned)(col + b_chunk * 8) < (unsigned)p.K ? lane_row + b_chunk * 16 : 0x80000000u;
 #pragma unroll
                     for (int u = 0; u < PB; u++)
-                        dma_buf16(rb, voff, __builtin_amdgcn_readfirstlane(u * row_step + col * 2), wave_lds + slot + KB * A_BLK + kb * B_BLK + u * NL * 1024);
+                        dma_buf16(rb, b_off, __builtin_amdgcn_readfirstlane(u * row_step + col * 2), wave_lds + slot + KB * A_BLK + kb * B_BLK + u * NL * 1024);
 #pragma unroll
                     for (int u = 0; u < PA; u++)
-                        dma_buf16(ra, voff, __builtin_amdgcn_readfirstlane(u * row_step + col * 2), wave_lds + slot + kb * A_BLK + u * NL * 1024);
+                        dma_buf16(ra, a_off, __builtin_amdgcn_readfirstlane(u * row_step + col * 2), wave_lds + slot + kb * A_BLK + u * NL * 1024);
                 }
             };
             __builtin_amdgcn_s_setprio(3);
 #pragma unroll
             for (int s = 0; s < S - 1; s++) request(s, s * STAGE);
-            wait_vmcnt<(S - 2) * P>();  // stage 0 has landed (vmcnt retires in issue order)
+            wait_vmcnt<FLIGHT>();  // what the first step reads has landed (vmcnt retires in issue order)
             __builtin_amdgcn_s_barrier();
             unsigned slot = (S - 1) * STAGE;
             // With an accumulator the steps behind the last request ask for its values instead of further stages: they
             // arrive while the last S - 1 stages are multiplied.
             const bool sums = ACC && (MODE != MODE_RS || p.ACC);
-            const int fetching = sums ? (KT > S - 1 ? KT - (S - 1) : 0) : KT;
+            const int stages = SHIFT ? KT + 1 : KT;
+            const int fetching = sums ? (stages > S - 1 ? stages - (S - 1) : 0) : KT;
             for (int kt = 0; kt < fetching; kt++) {
                 request(kt + S - 1, slot);  // the slot of stage kt - 1, given up at the last barrier
                 slot = slot + STAGE == S * STAGE ? 0 : slot + STAGE;
-                wait_vmcnt<(S - 2) * P>();  // stage kt + 1
+                wait_vmcnt<FLIGHT>();  // what step kt + 1 reads
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
             }
@@ -243,7 +272,8 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
 #pragma unroll
                 for (int j = 0; j < S - 1; j++) {
                     if (fetching + j < KT) {
-                        if (j < S - 2) asm volatile("s_waitcnt vmcnt(%0)" : : "i"(ACC ? (S - 3 - j) * P + NCH : 0) : "memory");  // stage fetching + j + 1
+                        const int left = FLIGHT - (j + 1) * P;  // the same, with one stage fewer requested each time
+                        if (j < S - 2) asm volatile("s_waitcnt vmcnt(%0)" : : "i"(ACC ? (left > 0 ? left : 0) + NCH : 0) : "memory");
                         __builtin_amdgcn_s_barrier();
                         asm volatile("" ::: "memory");
                     }
@@ -293,8 +323,9 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             constexpr int FL = LONG_B ? FN : FM, FS = LONG_B ? FM : FN;
             constexpr unsigned L_BLK = LONG_B ? B_BLK : A_BLK, S_BLK = LONG_B ? A_BLK : B_BLK;
             const int frow = lane & 15, fk = lane >> 4, key = (frow >> 1) & 7;
-            const unsigned la = lds0 + (unsigned)((wm * WTM + frow) * 8 + (fk ^ key)) * 16;
-            const unsigned lb = lds0 + KB * A_BLK + (unsigned)((wn * WTN + frow) * 8 + (fk ^ key)) * 16;
+            const int phys = SHIFT ? (fk + key) & 7 : fk ^ key;  // chunk fk; four further on is ^ 4 in both
+            const unsigned la = lds0 + (unsigned)((wm * WTM + frow) * 8 + phys) * 16;
+            const unsigned lb = lds0 + KB * A_BLK + (unsigned)((wn * WTN + frow) * 8 + phys) * 16;
             const unsigned l_lds = LONG_B ? lb : la, s_lds = LONG_B ? la : lb;
             typedef const __attribute__((address_space(3))) frag *lds_frag_t;
             // Two sets of short fragments take turns.  Long ones: two sets as well, or, from four on, one set whose
@@ -303,17 +334,30 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             constexpr bool RING = FL >= 4;
             constexpr int MEET = RING ? 1 : 0;  // the barrier stands in front of this row of the step's last k-step
             frag lf[RING ? 1 : 2][FL], sf[2][FS];
-            auto fetch_l = [&](int kk, unsigned slot, int i) __attribute__((always_inline)) {
-                const unsigned at = (l_lds + slot + (kk >> 1) * L_BLK) ^ ((kk & 1) * 64);
+            // Shifted: column chunk c of a 64-column block lies c + shift chunks behind the start of the row's line, that is
+            // in the following block from 8 on (all rows of a lane have the same shift: they are 16 apart).
+            int l_shift = 0, s_shift = 0;
+            if (SHIFT) {
+                const int a_shift = row_shift(p.A + (size_t)m0 * p.lda, p.lda, frow), b_shift = row_shift(p.B + (size_t)n0 * p.ldb, p.ldb, frow);
+                l_shift = fk + (LONG_B ? b_shift : a_shift);
+                s_shift = fk + (LONG_B ? a_shift : b_shift);
+            }
+            auto block_of = [&](int kk, unsigned slot, unsigned next, unsigned blk, int shift) __attribute__((always_inline)) {
+                const unsigned here = slot + (kk >> 1) * blk, behind = (kk >> 1) + 1 < KB ? here + blk : next;
+                return SHIFT && shift + (kk & 1) * 4 >= 8 ? behind : here;
+            };
+            auto fetch_l = [&](int kk, unsigned slot, unsigned next, int i) __attribute__((always_inline)) {
+                const unsigned at = (l_lds + block_of(kk, slot, next, L_BLK, l_shift)) ^ ((kk & 1) * 64);
                 lf[RING ? 0 : kk & 1][i] = *(lds_frag_t)(uintptr_t)(at + i * 2048);
             };
-            auto fetch_s = [&](int kk, unsigned slot, int j) __attribute__((always_inline)) {
-                const unsigned at = (s_lds + slot + (kk >> 1) * S_BLK) ^ ((kk & 1) * 64);
+            auto fetch_s = [&](int kk, unsigned slot, unsigned next, int j) __attribute__((always_inline)) {
+                const unsigned at = (s_lds + block_of(kk, slot, next, S_BLK, s_shift)) ^ ((kk & 1) * 64);
                 sf[kk & 1][j] = *(lds_frag_t)(uintptr_t)(at + j * 2048);
             };
+            auto behind_slot = [&](unsigned slot) __attribute__((always_inline)) { return slot + STAGE == S * STAGE ? 0 : slot + STAGE; };
             // k-step kk with the fetches of the next one (the first of the next slot behind the last) spread over its
             // rows from `from` on, the earlier ones a little denser: what is fetched last is needed soon.
-            auto k_step = [&](int kk, unsigned slot, unsigned next) __attribute__((always_inline)) {
+            auto k_step = [&](int kk, unsigned slot, unsigned next, unsigned after) __attribute__((always_inline)) {
                 const bool last = kk == KK - 1;
                 const int from = last ? MEET : 0;
                 const int nkk = last ? 0 : kk + 1;
@@ -340,10 +384,10 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                         const int n = i + 1 - l_done + s_to - s_done;
 #pragma unroll
                         for (int q = 0; q < FS; q++)
-                            if (q >= s_done && q < s_to) fetch_s(nkk, last ? next : slot, q);
+                            if (q >= s_done && q < s_to) fetch_s(nkk, last ? next : slot, last ? after : next, q);
 #pragma unroll
                         for (int q = 0; q < FL; q++)
-                            if (q >= l_done && q <= i) fetch_l(nkk, last ? next : slot, q);
+                            if (q >= l_done && q <= i) fetch_l(nkk, last ? next : slot, last ? after : next, q);
                         l_done = i + 1;
                         s_done = s_to;
 #pragma unroll
@@ -393,13 +437,13 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
 #pragma unroll
-            for (int j = 0; j < FS; j++) fetch_s(0, 0, j);
+            for (int j = 0; j < FS; j++) fetch_s(0, 0, STAGE, j);
 #pragma unroll
-            for (int i = 0; i < FL; i++) fetch_l(0, 0, i);
+            for (int i = 0; i < FL; i++) fetch_l(0, 0, STAGE, i);
             for (int kt = 0; kt < KT; kt++) {
-                const unsigned next = slot + STAGE == S * STAGE ? 0 : slot + STAGE;
+                const unsigned next = behind_slot(slot), after = SHIFT ? behind_slot(next) : next;
 #pragma unroll
-                for (int kk = 0; kk < KK; kk++) k_step(kk, slot, next);  // the last one fetches from the next slot: behind the last stage, zeros never used
+                for (int kk = 0; kk < KK; kk++) k_step(kk, slot, next, after);  // the last one fetches from the next slot: behind the last stage, zeros never used
                 slot = next;
             }
             __builtin_amdgcn_s_waitcnt(0xC07F);

@@ -167,6 +167,60 @@ def test_reduce_scatter_epilogue(fo, dtype, bm, bn, M, N, K, W):
     ov.close()
 
 
+LINES = [  # dtype, reorder tile, M, N, K       workgroup tile; K / 8 odd, even, a multiple of four; one to many K steps
+    (F16, 128, 128, 128, 1024, 8),           # 32x32
+    (BF16, 128, 128, 128, 1024, 1000),
+    (F16, 128, 128, 128, 3072, 1112),        # 64x32
+    (BF16, 128, 128, 256, 3072, 144),        # 64x64, one step and a part
+    (F16, 128, 256, 256, 3072, 1064),
+    (BF16, 128, 128, 384, 3200, 72),         # 64x96
+    (F16, 128, 128, 384, 3200, 1120),
+    (F16, 128, 128, 512, 3456, 456),         # 64x128
+    (BF16, 256, 128, 512, 3456, 1656),
+    (BF16, 128, 128, 1408, 1536, 184),       # 96x128
+    (F16, 128, 128, 2560, 1280, 40),         # 128x128
+    (F16, 128, 128, 2560, 1280, 1096),
+]
+
+
+@pytest.mark.parametrize("dtype,bm,bn,M,N,K", LINES)
+def test_operand_rows_off_the_line(fo, dtype, bm, bn, M, N, K):
+    """Operand rows that begin anywhere in a 128-byte line, by the leading dimension and by the operand's own address: every
+    product is summed in the same order, so each result is that of the operands padded with zero columns to whole lines,
+    bit for bit, whatever stands in memory around them."""
+    ops, td = fo.ops, TORCH_DTYPE[dtype]
+    algo = fo._capi.find_algo(bm, bn, swizzle=4)
+    A, _ = seeded((M, K), dtype, M + K)
+    B, _ = seeded((N, K), dtype, N + K, scale=K ** -0.5)
+    before, _ = seeded((M, N), dtype, 7)
+    Kp = -(-K // 64) * 64
+    Ap, Bp = (torch.nn.functional.pad(t, (0, Kp - K)) for t in (A, B))
+    want = torch.empty(M, N, device="cuda", dtype=td)
+    ops.gemm(Ap, Bp, want, algo)
+    assert max_rel_err(want.float(), A.float() @ B.float().T) <= 1e-2
+
+    def placed(t, columns):  # t, that many columns behind a line's start, with NaN on both sides
+        room = torch.full((t.numel() + 128,), float("nan"), device="cuda", dtype=td)
+        view = room[columns:columns + t.numel()].view_as(t)
+        view.copy_(t)
+        return view
+
+    ov = ops.Overlap()
+    for a_columns, b_columns in ((64, 64), (72, 64), (88, 120)):
+        a, b = placed(A, a_columns), placed(B, b_columns)
+        C = torch.full((M, N), float("nan"), device="cuda", dtype=td)
+        ops.gemm(a, b, C, algo)
+        torch.cuda.synchronize()
+        assert torch.equal(C, want), (a_columns, b_columns)
+        acc = before.clone()
+        C.fill_(float("nan"))
+        ov.set_accumulator(acc)
+        ov.gemm_allreduce(a, b, C, algo)
+        torch.cuda.synchronize()
+        assert torch.equal(C, want) and torch.equal(acc, (before.float() + want.float()).to(td))
+    ov.close()
+
+
 @pytest.mark.parametrize("alias", ["C", "A"])
 def test_accumulator_in_an_operand_or_the_product(fo, alias):
     """An accumulator that shares memory with an operand or with the product is updated behind the GEMM, not by it."""
