@@ -67,16 +67,38 @@ struct launch_plan {
 // products than this many columns of K are computed in whole reorder tiles instead when counters are wanted.
 constexpr int kSignalAfterFromK = 1536;
 
-// 256x256 where fo_pick_raster says so.  Otherwise the smallest tile whose count still fits the chip in one round,
-// one per CU: a smaller tile moves more operand bytes per flop (64x64 twice those of 128x128), but it puts the
-// operand paths of CUs to work that a larger tile leaves idle, and up to that point the time of these sizes is the
-// per-CU operand stream.  Measured over M = 128..4224, N = 1024..8192, K = 512, 2048, 8192: the rule picks the
-// fastest tile or one within a few percent of it (K = 2048, us: 128x4096 64x32 7.3, 64x64 8.1, 128x128 12.8;
-// 512x4096 64x128 11.7, 128x128 13.7, 64x64 16.2; 1024x4096 128x128 16.8, 128x256 21.8, 64x128 21.7; 2048x4096
-// 128x256 29.2, 128x128 31.7).  What needs more than one round of those goes to the 256x256 tile as well if it gives
-// 60 % of the CUs something to do; M and N need not be multiples of 256 for that, only of 128 (the last tile of a
-// dimension then repeats half of its neighbour).
-launch_plan plan_launch(const fo_raster &r, int M, int N, int BM, int BN, bool whole_only) {
+// What one round of a tile takes, all CUs busy: microseconds at K = 4096, with operand rows on 128-byte lines and off them
+// (the tiles up to 128x160 then load whole lines, the larger ones cannot).  Ratios at K = 1024 are the same.
+struct tile_cost {
+    int tm, tn, on_lines, off_lines;
+};
+constexpr tile_cost kTileCosts[] = {{96, 128, 26, 27},  {128, 128, 31, 33}, {128, 160, 36, 38}, {128, 192, 42, 54},
+                                    {128, 256, 57, 71}, {256, 128, 57, 71}, {256, 256, 97, 110}};
+
+// Estimate for `count` tiles: whole rounds, and a last one that costs 60 % of a round plus its share of the CUs (fewer
+// active CUs share the L2s, HBM and the power limit).
+double rounds_cost(long count, long cus, int round) {
+    const long full = count / cus, rest = count % cus;
+    return round * (full + (rest ? 0.6 + 0.4 * rest / cus : 0.0));
+}
+
+// What fits the chip in one round, one tile per CU, takes the smallest tile that does: a smaller tile moves
+// more operand bytes per flop (64x64 twice those of 128x128), but it puts the operand paths of CUs to work that a larger
+// tile leaves idle, and up to that point the time of these sizes is the per-CU operand stream.  Measured over
+// M = 128..4224, N = 1024..8192, K = 512, 2048, 8192: the rule picks the fastest tile or one within a few percent of it
+// (K = 2048, us: 128x4096 64x32 7.3, 64x64 8.1, 128x128 12.8; 512x4096 64x128 11.7, 128x128 13.7, 64x64 16.2; 1024x4096
+// 128x128 16.8, 128x256 21.8, 64x128 21.7).
+// Up to 128x160 that is so whatever the estimate above says; beyond, it decides, for launches whose order and counters
+// nobody waits for.  K = 4096 and 4088, us, against the rule before it (the largest tile that fits, else 256x256 from 60 %
+// of the CUs on, else rounds of 128x256): 2048x4224 87.6 -> 64.1 and 117.9 -> 67.9 (two rounds of 128x160), 2048x5120
+// 80.5 -> 75.5 and 93.9 -> 77.2, 2304x4096 77.1 -> 68.1 and 80.8 -> 71.8, 3456x4864 124.1 -> 119.7 (three rounds of
+// 128x192); one round: 1536x3328 39.4 -> 36.2 and 50.7 -> 38.4 (128x160).
+// Launches that move counters (`counted`) want whole reorder tiles, and rounds in the order that fo_schedule_order
+// reports: more than a round goes to the 256x256 tile if it gives 60 % of the CUs something to do, else to rounds of the
+// Algo's own tile or the larger one beside it.
+// M and N need only be multiples of 128: the last tile of a dimension is moved back or, 256x256, repeats half of its
+// neighbour.
+launch_plan plan_launch(const fo_raster &r, int M, int N, int BM, int BN, bool whole_only, bool counted, bool on_lines) {
     launch_plan p;
     p.tail = p.tail_tm = p.tail_tn = 0;
     auto set = [&](int tm, int tn) {
@@ -96,7 +118,8 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int BM, int BN, bool w
         p.tail_tn = BN;
         if (BM == 128 && BN == 128 && positions * 4 > cus && N % 256 == 0) p.tail_tn = 256;
     };
-    if (r.mtm == 256 && r.mtn == 256) {
+    const bool square = r.mtm == 256 && r.mtn == 256;  // what fo_schedule_order assumes
+    if (square && counted) {
         set(256, 256);
         p.panel = r.panel;
         p.xcd_remap = r.xcd_remap;
@@ -104,27 +127,55 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int BM, int BN, bool w
         return p;
     }
     const long cus = fo_main_tile_resident();
-    static const int shapes[][2] = {{32, 32},  {64, 32},   {64, 64},   {64, 96},   {64, 128},
-                                    {96, 128}, {128, 128}, {128, 192}, {128, 256}, {256, 128}};
-    for (const auto &s : shapes) {
-        if (M < s[0] || N < s[1] || (long)((M + s[0] - 1) / s[0]) * ((N + s[1] - 1) / s[1]) > cus) continue;
-        if (whole_only && (s[0] % BM || s[1] % BN)) continue;
-        set(s[0], s[1]);
-        // of the two largest, the one that holds whole reorder tiles
-        if (!p.whole && s[0] == 128 && s[1] == 256 && M >= 256 && (long)((M + 255) / 256) * (N / 128) <= cus) set(256, 128);
-        // An XCD's workgroups (every eighth of the launch) take one stretch of panels of eight tile rows: they share
-        // operand rows in its L2 both ways.
+    auto tiles = [&](int tm, int tn) { return (long)((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
+    // An XCD's workgroups (every eighth of the launch) take one stretch of panels of eight tile rows: they share operand
+    // rows in its L2 both ways.
+    auto set_shared = [&](int tm, int tn) {
+        set(tm, tn);
         p.panel = p.grid_m < 8 ? p.grid_m : 8;
+    };
+    static const int shapes[][2] = {{32, 32},  {64, 32},   {64, 64},   {64, 96},   {64, 128}, {96, 128},
+                                    {128, 128}, {128, 160}, {128, 192}, {128, 256}, {256, 128}};
+    for (const auto &s : shapes) {
+        if (!counted && s[0] * s[1] > 128 * 160) break;
+        if (square || M < s[0] || N < s[1] || tiles(s[0], s[1]) > cus) continue;
+        if (whole_only && (s[0] % BM || s[1] % BN)) continue;
+        set_shared(s[0], s[1]);
+        // of the two largest, the one that holds whole reorder tiles
+        if (!p.whole && s[0] == 128 && s[1] == 256 && M >= 256 && tiles(256, 128) <= cus) set_shared(256, 128);
+        return p;
+    }
+    const long nt = tiles(256, 256);
+    const int rem = square ? r.tail_tiles : nt > cus && nt % cus * 2 <= cus ? (int)(nt % cus) : 0;
+    if (!counted) {
+        const tile_cost *best = nullptr;
+        double least = 0;
+        for (const tile_cost &t : kTileCosts) {
+            if (M < t.tm || N < t.tn) continue;
+            const int round = on_lines ? t.on_lines : t.off_lines;
+            const bool split = t.tm == 256 && t.tn == 256 && rem;  // the last positions go to a second launch
+            const double cost = split ? rounds_cost(nt - rem, cus, round) + (rem * 4 <= cus ? 33 : 60)
+                                      : rounds_cost(tiles(t.tm, t.tn), cus, round);
+            if (best && cost >= least) continue;
+            best = &t;
+            least = cost;
+        }
+        set_shared(best->tm, best->tn);  // the 96x128 tile at least: M and N are multiples of 128
+        if (p.tm == 256 && p.tn == 256) {
+            if (rem) set_tail(rem, cus);
+            if (square) {
+                p.panel = r.panel;
+                p.xcd_remap = r.xcd_remap;
+            }
+        }
         return p;
     }
     // Several rounds walk the tiles in strips of the order that fo_schedule_order reports (panels of r.panel rows of
     // reorder tiles).
-    const int nt = ((M + 255) / 256) * ((N + 255) / 256);
     if (M >= 256 && N >= 256 && (long)M * N > 512L * 128 * 128 && nt * 5 > cus * 3) {
         set(256, 256);
         p.panel = r.panel * BM >= 512 ? r.panel * BM / 256 : 1;
-        const int rem = nt % cus;
-        if (nt > cus && rem && rem * 2 <= cus) set_tail(rem, cus);
+        if (rem) set_tail(rem, cus);
         return p;
     }
     p.panel = r.panel;
@@ -191,7 +242,7 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     a.rank = rs ? rs->rank : 0;
     a.seg_rows = (int)((int64_t)M * N / a.BN / a.W);
     const bool counts = (mode == MODE_SIGNAL || mode == MODE_SCATTER) && !quiet;
-    const launch_plan plan = plan_launch(r, M, N, a.BM, a.BN, counts && K < kSignalAfterFromK);
+    const launch_plan plan = plan_launch(r, M, N, a.BM, a.BN, counts && K < kSignalAfterFromK, counts, on_lines(a));
     a.grid_m = plan.grid_m; a.grid_n = plan.grid_n; a.panel = plan.panel; a.xcd_remap = plan.xcd_remap;
     a.first = 0; a.sub_m = a.sub_n = 1;
     a.count = plan.count;
@@ -300,7 +351,7 @@ extern "C" int fo_gemm_wave_tiles(int dtype, int algo, int M, int N, int32_t *ti
     fo_raster r;
     int rc = fo_pick_raster(algo, M, N, &r);
     if (rc) return rc;
-    const launch_plan plan = plan_launch(r, M, N, e->f[0], e->f[1], false);
+    const launch_plan plan = plan_launch(r, M, N, e->f[0], e->f[1], false, true, true);
     GemmArgs a = {};
     a.count = plan.count;
     int info[5] = {0, 0, 0, 0, 0};
@@ -318,7 +369,7 @@ extern "C" int fo_gemm_kernel_info(int dtype, int algo, int M, int N, int epilog
     int rc = fo_pick_raster(algo, M, N, &r);
     if (rc) return rc;
     const fo_algo_entry *e = fo_algo_lookup(algo);
-    const launch_plan plan = plan_launch(r, M, N, e->f[0], e->f[1], false);
+    const launch_plan plan = plan_launch(r, M, N, e->f[0], e->f[1], false, epilogue != MODE_PLAIN, true);
     GemmArgs a = {};
     a.count = plan.count;
     int out[5] = {0, 0, 0, 0, 0};

@@ -48,6 +48,9 @@ struct GemmArgs {
     int stream_out;                        // 256x256 kernel: store the output with the non-temporal hint
 };
 
+// Every operand row begins on a 128-byte line.
+inline bool on_lines(const GemmArgs &a) { return (((uintptr_t)a.A | (uintptr_t)a.B | (uintptr_t)a.lda * 2) & 127) == 0; }
+
 constexpr int kMaxSub = 4;        // reorder tiles per macro tile (256x256 over 128x128)
 constexpr int kPrefixRegs = 256;  // group search on prefix sums held in registers (one per 64 groups) up to this many groups
 

@@ -29,7 +29,7 @@ int FO_CAT3(fo_gemm_tile_launch_, FO_INST_DTYPE, _, FO_INST_MODE)(const GemmArgs
                              tile_smem_bytes<TM_, TN_, BK_, S_>(), kTileThreads>(a, stream, resident_out, expect_resident);
     // Operand rows that do not begin on 128-byte lines: the form that loads whole lines, for the tiles whose stages leave
     // LDS for one more in flight beside the two a step then reads.
-    if (((uintptr_t)a.A | (uintptr_t)a.B | (unsigned)a.lda * 2) & 127) {
+    if (!on_lines(a)) {
         FO_TILE_(32, 32, 128, 8, true)
         FO_TILE_(64, 32, 128, 6, true)
         FO_TILE_(64, 64, 128, 4, true)
@@ -37,6 +37,7 @@ int FO_CAT3(fo_gemm_tile_launch_, FO_INST_DTYPE, _, FO_INST_MODE)(const GemmArgs
         FO_TILE_(64, 128, 64, 6, true)
         FO_TILE_(96, 128, 64, 5, true)
         FO_TILE_(128, 128, 64, 4, true)
+        FO_TILE_(128, 160, 64, 4, true)
     }
     FO_TILE(32, 32, 128, 8)
     FO_TILE(64, 32, 128, 6)
@@ -45,6 +46,7 @@ int FO_CAT3(fo_gemm_tile_launch_, FO_INST_DTYPE, _, FO_INST_MODE)(const GemmArgs
     FO_TILE(64, 128, 128, 3)
     FO_TILE(96, 128, 64, 5)
     FO_TILE(128, 128, 64, 4)
+    FO_TILE(128, 160, 64, 4)
     FO_TILE(128, 192, 64, 3)
     FO_TILE(128, 256, 64, 3)
     FO_TILE(256, 128, 64, 3)

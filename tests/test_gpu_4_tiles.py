@@ -22,13 +22,21 @@ CASES = [  # dtype, reorder tile, M, N, K                workgroup tile
     (BF16, 128, 128, 1408, 1536, 328),                 # 96x128, moved back along M
     (F16, 256, 128, 1536, 1408, 1544),                 # 96x128 over 256-high reorder tiles
     (F16, 128, 128, 2560, 1280, 64),                   # 128x128, one K step
-    (BF16, 128, 128, 1920, 2560, 136),                 # 128x192, moved back along N
-    (F16, 256, 128, 2048, 2432, 1600),                 # 128x192, half of each 256-high reorder tile
-    (F16, 128, 128, 3968, 1920, 72),                   # 128x256, moved back along N
+    (BF16, 128, 128, 1920, 2560, 136),                 # 128x160
+    (F16, 256, 128, 2048, 2432, 1600),                 # 128x160, half of each 256-high reorder tile, moved back along N
+    (F16, 128, 128, 3968, 1920, 72),                   # two rounds of 128x128
     (BF16, 256, 128, 3840, 1920, 192),                 # 256x128
     (F16, 128, 128, 4224, 3200, 136),                  # 256x256, half a tile left along both
     (BF16, 128, 256, 4224, 3328, 72),                  # 256x256, half a tile left along M
     (BF16, 128, 128, 4224, 4352, 264),                 # 256x256 and a second launch for the last wave
+    (F16, 128, 128, 1280, 4096, 192),                  # 128x192, operand rows on 128-byte lines
+    (BF16, 256, 128, 2048, 2816, 64),                  # 128x192 over 256-high reorder tiles
+    (F16, 128, 128, 3968, 1920, 128),                  # 128x256, the same
+    (F16, 128, 128, 2048, 4224, 136),                  # two rounds of 128x160; 256x256 with counters
+    (BF16, 128, 256, 2048, 4608, 1600),                # the same over 256-wide reorder tiles, on lines
+    (BF16, 256, 128, 2304, 4096, 72),                  # the same over 256-high ones
+    (BF16, 128, 128, 1792, 4608, 72),                  # two rounds of 128x128
+    (F16, 128, 128, 3456, 4864, 64),                   # three rounds of 128x192
 ]
 
 
