@@ -69,9 +69,19 @@ namespace {
 
 // With a link rate the automatic choices go to per-wave launches on the second stream: the link time
 // follows each consumer launch, and it is what the second stream is there to hide.
-bool in_stream(const fo_overlap *h, int M, int N, int K) {
+//
+// Longer GEMMs stay on one stream too where there is nothing to overlap: `idle`, a call without a consumer and without a
+// normalisation (4224x7168x3584 221 -> 215 us, 3712x8192x3456 216 -> 207), and a product of less than about one round of
+// 256x256 tiles, whose groups all complete at its end, so that the second stream adds its launches and polls and hides
+// nothing (us, two streams -> one: 2304x4096x3560 96 -> 83, 1792x4608x4520 125 -> 108, 2048x4224x6968 256 -> 167,
+// 2176x5888x3312 133 -> 127, 207 of 256 tiles; with 231 tiles, 5376x2688x3544, 141 -> 147).  in_stream_below_flop = 0
+// still asks for two streams always.
+bool in_stream(const fo_overlap *h, int M, int N, int K, bool idle, bool monitor) {
     if (!h->comm_stream) return true;
-    return h->fused < 0 && h->link_bytes_per_s <= 0 && 2.0 * M * N * K < h->in_stream_below_flop;
+    if (h->fused >= 0 || h->link_bytes_per_s > 0 || h->in_stream_below_flop <= 0) return false;
+    if (2.0 * M * N * K < h->in_stream_below_flop) return true;
+    if (monitor) return false;  // its GEMM counts and is waited for in any case
+    return idle || (long)((M + 255) / 256) * ((N + 255) / 256) * 6 <= (long)fo_main_tile_resident() * 5;
 }
 
 int fused_grid(const fo_overlap *h, int G) {  // 0: per-group launches, otherwise workgroups of the one launch
@@ -421,7 +431,7 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
         if (N % 8 || N > 16384 || (int64_t)M * N * 2 > 0xFFFFFFFFLL) return FO_ERR_SHAPE;
     }
 
-    const bool same_stream = in_stream(h, M, N, K);
+    const bool same_stream = in_stream(h, M, N, K, !h->acc && !np, monitor != 0);
     if (np) {
         // on one stream all rows follow in one launch, whatever their slots
         rc = same_stream ? check_slots(np->RA_host, TM * TN) : last_slots(np->RA_host, TM, TN, last_slot);
@@ -587,7 +597,7 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     rc = link_fits(h, (int64_t)M * N * 2);
     if (rc) return rc;
 
-    const bool same_stream = in_stream(h, M, N, K);
+    const bool same_stream = in_stream(h, M, N, K, false, monitor != 0);
     const int fused = same_stream ? 0 : fused_grid(h, G);
     fo_stream_t cstream = same_stream ? h->gemm_stream : h->comm_stream;
     int32_t wave = 0;

@@ -292,7 +292,9 @@ int fo_overlap_plan_norm_rows(const int32_t *RA_host, int TM, int TN, const int3
  * keeps the whole call on the GEMM stream (the GEMM with its reordered store,
  * then one consumer launch: nothing that short can hide a fork and a join, and
  * the stream orders the two, so MM is not touched and stays zero; with the
- * monitor on, the signalling GEMM and one wait over all groups as elsewhere);
+ * monitor on, the signalling GEMM and one wait over all groups as elsewhere),
+ * and so does, without the monitor, a product of less than about one round of
+ * 256x256 tiles or an all-reduce with neither accumulator nor normalisation;
  * otherwise one launch when there are more than 16 groups, else per-wave
  * launches.  0: always the second stream with wait + consumer launches per
  * group (per GEMM wave) as the reference's host loop
@@ -300,7 +302,8 @@ int fo_overlap_plan_norm_rows(const int32_t *RA_host, int TM, int TN, const int3
  * with the default grid; n > 1: the same with n workgroups. */
 int fo_overlap_set_fused_consumer(fo_overlap_t *h, int fused);
 /* The two thresholds of the automatic choice above (no counterpart in the
- * reference): GEMMs below in_stream_below_flop stay on the GEMM stream, more
+ * reference): GEMMs below in_stream_below_flop stay on the GEMM stream (0: none
+ * does, whatever its size), more
  * than fused_from_groups groups get the one-launch consumer.  The defaults
  * (6.4e10, 16) were measured on one MI355X; a negative value restores one. */
 int fo_overlap_set_schedule(fo_overlap_t *h, double in_stream_below_flop, int fused_from_groups);
