@@ -518,6 +518,9 @@ int launch_rmsnorm_as(const void *X, void *Y, const void *Wt, int bs, int dim, i
     return launch_rmsnorm_on<Tag, STREAM, NORM_GENERAL>(X, Y, Wt, bs, dim, BM, BN, rldn, RA, eps, stream);
 }
 
+// Up to this many rows a normalisation gets a workgroup per row.
+inline int few_norm_rows(int dim) { return dim > 2048 ? 2048 : 512; }
+
 template <typename Tag>
 int launch_rmsnorm(const void *X, void *Y, const void *Wt, int bs, int dim, int BM, int BN,
                    int rldn, const int32_t *RA, float eps, hipStream_t stream) {
@@ -525,7 +528,14 @@ int launch_rmsnorm(const void *X, void *Y, const void *Wt, int bs, int dim, int 
     // lane), and there it is the faster of the two: 8192 x 8192, nothing cached, 45.5-46.7 us against 47-50
     // (fp16 and bf16, reorder or not).  Narrower rows leave its lanes idle (16384 x 1024: 15.5 against 11.8 us)
     // and longer ones cost it its look-ahead.
-    if (dim == 8192 && (int64_t)bs * dim * 2 <= 0xFFFFFFFFLL)
+    // Few rows: one wavefront per row leaves most of the chip idle (128 rows: 32 workgroups) and is a chain of up to
+    // sixteen loads, sums and stores; a workgroup per row is four times as many wavefronts and a quarter of the chain.
+    // Reordered input, us, before -> after (fp16 / bf16): 128 x 4096 3.43 -> 2.71 / 3.90 -> 2.84, 512 x 7168 5.71 -> 4.35
+    // / 6.69 -> 4.76, 1152 x 5120 8.00 -> 6.50 / 9.27 -> 7.34, 2048 x 4096 8.09 -> 7.42 / 9.12 -> 8.37.  Beyond, the row's
+    // wavefront wins again: 4096 x 4096 11.4 against 12.1, and with rows of up to 2048 elements, which leave half of
+    // the workgroup's lanes idle, from 1152 rows on (1024 elements 3.0 against 3.6).
+    const bool few = dim <= 8192 && bs <= few_norm_rows(dim);
+    if (few || (dim == 8192 && (int64_t)bs * dim * 2 <= 0xFFFFFFFFLL))
         return fo_norm_rows_with(std::is_same<Tag, fo_bf16_tag>::value ? FO_BF16 : FO_F16, X, Y, Wt, 0, bs, bs, dim, BM,
                                  BN, rldn, RA, eps, fo_streams((int64_t)bs * dim * 4), false, 0, stream);
     // input and output together against the cache that would have to hold them
@@ -682,7 +692,8 @@ __global__ __launch_bounds__(256, (CH <= 4 && !(CH == 4 && std::is_same<Tag, fo_
     }
 }
 
-// grid <= 0: one workgroup per 2 rows, at most 4096 (8192 x 8192 fp16 alone: 45.5 us from 4096 workgroups, 47.3 from 2048).  beside_gemm: at most 256 workgroups, each asking for
+// grid <= 0: one workgroup per row while they are few (1152 x 4096 5.3 us against 5.6 with two, 512 x 5120 3.6 against 4.1), else per
+// 2 rows, at most 4096 (8192 x 8192 fp16 alone: 45.5 us from 4096 workgroups, 47.3 from 2048).  beside_gemm: at most 256 workgroups, each asking for
 // kBesideGemmLds bytes of LDS it never touches (one workgroup per CU beside the GEMM's, as for the consumer).
 template <typename Tag, bool STREAM, int PATH>
 int launch_norm_rows_on(const void *X, void *Y, const void *Wt, int row0, int nrows, int dim, int BM, int BN, int rldn,
@@ -690,7 +701,7 @@ int launch_norm_rows_on(const void *X, void *Y, const void *Wt, int row0, int nr
                         int32_t *info) {
     const int nch = dim / 8;
     if (nrows < 1) nrows = 1;  // the query for the kernel's resources comes with no rows
-    if (grid <= 0) grid = (nrows + 1) / 2;
+    if (grid <= 0) grid = nrows <= few_norm_rows(dim) ? nrows : (nrows + 1) / 2;
     const int most = beside_gemm ? 256 : 4096;
     if (grid > most) grid = most;
     const int rows_per_wg = (nrows + grid - 1) / grid;
@@ -714,6 +725,8 @@ int launch_norm_rows_on(const void *X, void *Y, const void *Wt, int row0, int nr
         FO_NORM_ROWS(1);
     } else if (nch <= 512) {
         FO_NORM_ROWS(2);
+    } else if (nch <= 768) {
+        FO_NORM_ROWS(3);
     } else if (nch <= 1024) {
         FO_NORM_ROWS(4);
     } else if (nch <= 2048) {

@@ -494,3 +494,33 @@ def test_reorder_table_changed_in_place_between_launches(fo):
         assert MM[:4].tolist() == groups
         assert torch.equal(fo.layout.unpermute(Cp, M, N, bm, bn, RA), plain)
         MM.zero_()
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("bm,bn,bs,dim", [
+    (8, 8, 16, 1024), (128, 128, 512, 2048), (1, 8, 513, 2048),          # a workgroup per row up to 512 rows of 2048
+    (16, 8, 32, 2056), (8, 8, 8, 4096), (8, 8, 16, 4104),                # the edges of two, three and four chunks a lane
+    (64, 128, 64, 5120), (8, 8, 24, 6144), (4, 8, 12, 6152), (128, 256, 2048, 2304), (1, 8, 2049, 2064),
+])
+def test_rmsnorm_of_few_rows(fo, dtype, bm, bn, bs, dim):
+    """Both sides of the limits of the kernel that takes a workgroup per row, against 64 bits: the result is rounded to 16
+    bits twice (x * rsqrt, times the weight), half a unit in the last place each; a tenth is left for the 32-bit sum."""
+    td = TORCH_DTYPE[dtype]
+    g = torch.Generator(device="cuda").manual_seed(bs + dim)
+    x = torch.randn(bs, dim, generator=g, device="cuda").to(td)
+    w = (1 + 0.1 * torch.randn(dim, generator=g, device="cuda")).to(td)
+    T = bs // bm * (dim // bn)
+    RA = torch.randperm(T, generator=g, device="cuda").to(torch.int32).reshape(bs // bm, dim // bn)
+    want = x.double() * torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True) + 1e-6) * w.double()
+    tol = 1.1 * torch.finfo(td).eps
+    buf = torch.empty(T, bm, bn, device="cuda", dtype=td)
+    buf[RA.reshape(-1).long()] = x.view(bs // bm, bm, dim // bn, bn).permute(0, 2, 1, 3).reshape(T, bm, bn)
+    for reordered in (False, True):
+        y = torch.full((bs, dim), float("nan"), device="cuda", dtype=td)
+        if reordered:
+            fo.ops.reorder_rmsnorm(buf.view(bs, dim), y, w, bm, bn, 1, RA, eps=1e-6)
+        else:
+            fo.ops.rmsnorm(x, y, w, eps=1e-6)
+        torch.cuda.synchronize()
+        # below the smallest normal number the unit is absolute
+        assert ((y.double() - want).abs() <= tol * want.abs() + torch.finfo(td).tiny * tol).all(), reordered
