@@ -597,7 +597,17 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     rc = link_fits(h, (int64_t)M * N * 2);
     if (rc) return rc;
 
-    const bool same_stream = in_stream(h, M, N, K, false, monitor != 0);
+    // Where whole rows of the output view are this rank's, the GEMM's epilogue can do what follows it on one stream: a copy
+    // per group (4-5 us each on this GPU) and the consumer.  2048x4096x2048, four groups, eight ranks, no accumulator, whole
+    // pass with the normalisation: 42.0 us with copies, 37.5 so.
+    const span a = {A, (int64_t)M * K}, b = {B, (int64_t)N * K}, prod = {C, (int64_t)M * N}, sum = {h->acc, (int64_t)M * N};
+    const bool by_epilogue = rLDN == 1 && info[0] % W == 0 && !(((uintptr_t)C | (uintptr_t)D | (uintptr_t)h->acc) & 15) &&
+                             apart(sum, {a, b, prod}) && apart({D, seg_stride}, {a, b, prod, sum});
+    // Without an accumulator all there is to overlap are those copies, and with many groups they take longer than the GEMM:
+    // 5504x3840x3640 with four ranks, two streams against one, us: 4 groups 192 and 186, 16 214 and 187, 64 320 and 187, 1290
+    // 3404 and 218; 8192x4096x4096 with two: 4 groups 228 and 249, 16 236 and 247, 24 284 and 252, 64 369 and 253.
+    const bool only_copies = !h->acc && by_epilogue && G > h->fused_from_groups;
+    const bool same_stream = in_stream(h, M, N, K, only_copies, monitor != 0);
     const int fused = same_stream ? 0 : fused_grid(h, G);
     fo_stream_t cstream = same_stream ? h->gemm_stream : h->comm_stream;
     int32_t wave = 0;
@@ -613,12 +623,7 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
         if (rc) return rc;
     }
     const bool quiet = same_stream && !monitor;  // as in fo_overlap_gemm_allreduce
-    // Where whole rows of the output view are this rank's, the GEMM's epilogue also does what follows it: a copy per
-    // group (4-5 us each on this GPU) and the consumer.  2048x4096x2048, four groups, eight ranks, no accumulator, whole pass
-    // with the normalisation: 42.0 us with copies, 37.5 so.
-    const span a = {A, (int64_t)M * K}, b = {B, (int64_t)N * K}, prod = {C, (int64_t)M * N}, sum = {h->acc, (int64_t)M * N};
-    if (quiet && rLDN == 1 && info[0] % W == 0 && !(((uintptr_t)C | (uintptr_t)D | (uintptr_t)h->acc) & 15) &&
-        apart(sum, {a, b, prod}) && apart({D, seg_stride}, {a, b, prod, sum})) {
+    if (quiet && by_epilogue) {
         rc = fo_gemm_reduce_scatter(dtype, M, N, K, cseg_dev, G, A, B, C, h->acc, D, RA, RE, W, h->rank, algo, h->gemm_stream);
         if (rc) return rc;
         return link_time(h, (int64_t)M * N * 2, h->gemm_stream);

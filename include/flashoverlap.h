@@ -294,7 +294,8 @@ int fo_overlap_plan_norm_rows(const int32_t *RA_host, int TM, int TN, const int3
  * the stream orders the two, so MM is not touched and stays zero; with the
  * monitor on, the signalling GEMM and one wait over all groups as elsewhere),
  * and so does, without the monitor, a product of less than about one round of
- * 256x256 tiles or an all-reduce with neither accumulator nor normalisation;
+ * 256x256 tiles, an all-reduce with neither accumulator nor normalisation, or a
+ * reduce-scatter of more than 16 groups without accumulator;
  * otherwise one launch when there are more than 16 groups, else per-wave
  * launches.  0: always the second stream with wait + consumer launches per
  * group (per GEMM wave) as the reference's host loop

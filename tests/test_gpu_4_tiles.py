@@ -267,3 +267,34 @@ def test_accumulator_in_an_operand_or_the_product(fo, alias):
         assert torch.equal(product.reshape(-1), plain.reshape(-1)), call
         assert torch.equal(acc.reshape(-1), want), call
         ov.close()
+
+
+@pytest.mark.parametrize("groups", [16, 17, 300])
+def test_reduce_scatter_without_accumulator_by_groups(fo, groups):
+    """Both sides of the group count from which a long reduce-scatter without an accumulator stays on one stream."""
+    ops, M, N, K, W, bm = fo.ops, 4352, 4352, 2048, 4, 128   # more than 6.4e10 flop, 289 tiles of 256x256
+    algo = fo._capi.find_algo(bm, 128, swizzle=4)
+    TM, TN = M // bm, N // 128
+    T = TM * TN
+    A, _ = seeded((M, K), F16, 1)
+    B, _ = seeded((N, K), F16, 2, scale=K ** -0.5)
+    plain = torch.empty(M, N, device="cuda", dtype=torch.float16)
+    ops.gemm(A, B, plain, algo)
+    cseg = [1] * (groups - 1) + [T - groups + 1]
+    RA = torch.from_numpy(np.random.default_rng(3).permutation(T).astype(np.int32)).reshape(TM, TN).cuda()
+    RE = fo.layout.generate_row_mapping(M, N, bm, 128, cseg, W)
+    cs_cpu = torch.tensor(cseg, dtype=torch.int32)
+    MM = torch.zeros(fo.layout.counter_size(groups, TM, TN), dtype=torch.int32, device="cuda")
+    ov = ops.Overlap(rank=1, world=W)
+    C = torch.full((M * N,), float("nan"), device="cuda", dtype=torch.float16)
+    D = torch.full((M // W, N), float("nan"), device="cuda", dtype=torch.float16)
+    ov.gemm_reducescatter_overlap(A, B, C, D, MM, RA, RE, 1, cs_cpu, cs_cpu.cuda(), algo)
+    torch.cuda.synchronize()
+    assert torch.equal(fo.layout.unpermute(C, M, N, bm, 128, RA, RE=RE), plain)
+    rows, own, first = C.view(-1, 128), [], 0
+    for n in cseg:
+        own.append(rows[first:first + n * bm].view(W, n * bm // W, 128)[1])
+        first += n * bm
+    assert torch.equal(D.view(-1, 128), torch.cat(own))
+    assert (MM == 0).all() and ov.status() == 0
+    ov.close()
