@@ -32,7 +32,7 @@ enum {
 // store, whose epilogue does the all-reduce consumer's work too (with the monitor on: the signalling
 // GEMM, one wait that resets every counter and one consumer launch).  Fork, join and pollers beside the
 // GEMM cost more than such a GEMM can hide (4096x4096x512 with 256 groups:
-// 71 us overlapped, 48 us in stream).
+// 71 us overlapped, 44 us in stream).
 //
 // kGemmFlopPerNs: what a GEMM is expected to sustain, for sizing the pause
 // between polls only.
