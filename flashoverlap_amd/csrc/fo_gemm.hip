@@ -93,9 +93,11 @@ double rounds_cost(long count, long cus, int round) {
 // of the CUs on, else rounds of 128x256): 2048x4224 87.6 -> 64.1 and 117.9 -> 67.9 (two rounds of 128x160), 2048x5120
 // 80.5 -> 75.5 and 93.9 -> 77.2, 2304x4096 77.1 -> 68.1 and 80.8 -> 71.8, 3456x4864 124.1 -> 119.7 (three rounds of
 // 128x192); one round: 1536x3328 39.4 -> 36.2 and 50.7 -> 38.4 (128x160).
-// Launches that move counters (`counted`) want whole reorder tiles, and rounds in the order that fo_schedule_order
-// reports: more than a round goes to the 256x256 tile if it gives 60 % of the CUs something to do, else to rounds of the
-// Algo's own tile or the larger one beside it.
+// Launches that move counters (`counted`) want whole reorder tiles, and what takes more than one round is walked in the
+// raster that fo_schedule_order reports, tile by tile: a consumer waits for the groups in that order.  A larger tile
+// beside the Algo's own would be faster (256x256 with half tiles where 256 does not divide M or N: 97 us a round of four
+// times the output against 31), but its workgroups cross the order's XCD ranges, and the first group of such a launch
+// was complete in its last round (8064x8192 in four groups: rounds 3, 1, 2, 3 of 0..3).
 // M and N need only be multiples of 128: the last tile of a dimension is moved back or, 256x256, repeats half of its
 // neighbour.
 launch_plan plan_launch(const fo_raster &r, int M, int N, int BM, int BN, bool whole_only, bool counted, bool on_lines) {
@@ -119,13 +121,6 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int BM, int BN, bool w
         if (BM == 128 && BN == 128 && positions * 4 > cus && N % 256 == 0) p.tail_tn = 256;
     };
     const bool square = r.mtm == 256 && r.mtn == 256;  // what fo_schedule_order assumes
-    if (square && counted) {
-        set(256, 256);
-        p.panel = r.panel;
-        p.xcd_remap = r.xcd_remap;
-        if (r.tail_tiles) set_tail(r.tail_tiles, r.resident);
-        return p;
-    }
     const long cus = fo_main_tile_resident();
     auto tiles = [&](int tm, int tn) { return (long)((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
     // An XCD's workgroups (every eighth of the launch) take one stretch of panels of eight tile rows: they share operand
@@ -170,23 +165,10 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int BM, int BN, bool w
         }
         return p;
     }
-    // Several rounds walk the tiles in strips of the order that fo_schedule_order reports (panels of r.panel rows of
-    // reorder tiles).
-    if (M >= 256 && N >= 256 && (long)M * N > 512L * 128 * 128 && nt * 5 > cus * 3) {
-        set(256, 256);
-        p.panel = r.panel * BM >= 512 ? r.panel * BM / 256 : 1;
-        if (rem) set_tail(rem, cus);
-        return p;
-    }
+    set(r.mtm, r.mtn);
     p.panel = r.panel;
-    if (N % 256 == 0 && BM == 128) {
-        set(128, 256);
-    } else if (M % 256 == 0 && BN == 128) {
-        set(256, 128);
-        if (BM == 128 && p.panel > 1) p.panel /= 2;
-    } else {
-        set(BM, BN);
-    }
+    p.xcd_remap = r.xcd_remap;
+    if (r.tail_tiles) set_tail(r.tail_tiles, r.resident);
     return p;
 }
 

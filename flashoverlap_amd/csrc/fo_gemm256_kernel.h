@@ -155,7 +155,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
 
     // M and N are multiples of 128, not of 256: where half a tile is left at the end of a dimension, the tile is moved
     // back by half its size, so that all of its operand rows exist; its first half there repeats the neighbour's
-    // product and is neither stored nor counted (p.half: bit 0 along M, bit 1 along N).
+    // product and is not stored (p.half: bit 0 along M, bit 1 along N; never in a launch that counts, see plan_launch).
     int half = p.half;
     asm volatile("" : "+s"(half));  // in a register from here on: loaded again inside the K loop, it would turn every wait for LDS data into a wait for everything
     // Coordinates of raster position t in halves of tiles, bits 0 and 1 of *repeated: which halves another tile
@@ -319,7 +319,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                 if (q >= lane) count++;
             }
         }
-        if (lane < nsub && g >= 0) {
+        if (lane < nsub) {
             if (first) __hip_atomic_fetch_add(p.MM + g, count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (p.monitor) {
                 int o = __hip_atomic_fetch_add(p.MM + (p.TN - 1), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -643,11 +643,11 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
         }
 
         if (signalling) {
-            int v_g = -1;  // lane s: group of reorder tile s, -1 where another workgroup tile counts it
+            int v_g = 0;  // lane s: group of reorder tile s
             if (wave == 0) {
 #pragma unroll
                 for (int s = 0; s < kMaxSub; s++) {
-                    if (s < nsub && !((repeated & 1) && s < sub_n) && !((repeated & 2) && s % sub_n == 0)) {
+                    if (s < nsub) {
                         const int g = group_of(__builtin_amdgcn_readlane(v_done, s));
                         v_g = lane == s ? g : v_g;
                     }

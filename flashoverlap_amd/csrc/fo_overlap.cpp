@@ -34,10 +34,14 @@ enum {
 // GEMM cost more than such a GEMM can hide (4096x4096x512 with 256 groups:
 // 71 us overlapped, 44 us in stream).
 //
+// kRsEpilogueBelowFlop, kFewCopies: see fo_overlap_gemm_reducescatter.
+//
 // kGemmFlopPerNs: what a GEMM is expected to sustain, for sizing the pause
 // between polls only.
 constexpr int kFusedFromGroups = 16;
 constexpr double kInStreamBelowFlop = 6.4e10;
+constexpr double kRsEpilogueBelowFlop = 5e11;
+constexpr int kFewCopies = 16;
 constexpr double kGemmFlopPerNs = 1.2e6;
 
 }  // namespace
@@ -76,12 +80,18 @@ namespace {
 // nothing (us, two streams -> one: 2304x4096x3560 96 -> 83, 1792x4608x4520 125 -> 108, 2048x4224x6968 256 -> 167,
 // 2176x5888x3312 133 -> 127, 207 of 256 tiles; with 231 tiles, 5376x2688x3544, 141 -> 147).  in_stream_below_flop = 0
 // still asks for two streams always.
-bool in_stream(const fo_overlap *h, int M, int N, int K, bool idle, bool monitor) {
+//
+// `ragged`, a call that could do either and whose M or N is an odd multiple of 128: a launch that counts keeps the order of
+// the groups in the Algo's own tile (plan_launch), one that does not takes 256x256 tiles with half tiles at the end, and
+// what that saves is more than the second stream hides (us, two streams -> one, with an accumulator and the normalisation:
+// 3456x4352x3072 127 -> 93, 2432x7040x7056 271 -> 245, 8064x8064x4096 586 -> 465, 6272x8192x7168 661 -> 636; reduce-scatter,
+// eight ranks: 3456x4352x3072 123 -> 95, 4224x7168x3584 205 -> 194, 6272x8192x7168 651 -> 630, 8192x8064x7168 801 -> 751).
+bool in_stream(const fo_overlap *h, int M, int N, int K, bool idle, bool monitor, bool ragged) {
     if (!h->comm_stream) return true;
     if (h->fused >= 0 || h->link_bytes_per_s > 0 || h->in_stream_below_flop <= 0) return false;
     if (2.0 * M * N * K < h->in_stream_below_flop) return true;
     if (monitor) return false;  // its GEMM counts and is waited for in any case
-    return idle || (long)((M + 255) / 256) * ((N + 255) / 256) * 6 <= (long)fo_main_tile_resident() * 5;
+    return idle || ragged || (long)((M + 255) / 256) * ((N + 255) / 256) * 6 <= (long)fo_main_tile_resident() * 5;
 }
 
 int fused_grid(const fo_overlap *h, int G) {  // 0: per-group launches, otherwise workgroups of the one launch
@@ -431,7 +441,7 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
         if (N % 8 || N > 16384 || (int64_t)M * N * 2 > 0xFFFFFFFFLL) return FO_ERR_SHAPE;
     }
 
-    const bool same_stream = in_stream(h, M, N, K, !h->acc && !np, monitor != 0);
+    const bool same_stream = in_stream(h, M, N, K, !h->acc && !np, monitor != 0, M % 256 || N % 256);
     if (np) {
         // on one stream all rows follow in one launch, whatever their slots
         rc = same_stream ? check_slots(np->RA_host, TM * TN) : last_slots(np->RA_host, TM, TN, last_slot);
@@ -607,7 +617,15 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     // 5504x3840x3640 with four ranks, two streams against one, us: 4 groups 192 and 186, 16 214 and 187, 64 320 and 187, 1290
     // 3404 and 218; 8192x4096x4096 with two: 4 groups 228 and 249, 16 236 and 247, 24 284 and 252, 64 369 and 253.
     const bool only_copies = !h->acc && by_epilogue && G > h->fused_from_groups;
-    const bool same_stream = in_stream(h, M, N, K, only_copies, monitor != 0);
+    const bool in_any_case = in_stream(h, M, N, K, only_copies, monitor != 0, false);
+    // A large ragged call leaves the rest to launches behind the GEMM (one consumer launch for all groups, or a few copies):
+    // the epilogue holds up the next tile's loads.  By the epilogue and by launches, us, eight ranks and an accumulator:
+    // 8192x8064x7168 803 and 751, 8064x8064x4096 494 and 470 (two ranks 508 and 509), 4224x7168x3584 194 and 193,
+    // 8064x8192x1024 183 and 200; sixteen copies: 8192x8064x7168 737 and 693, 4224x7168x3584 182 and 192.
+    const bool few_launches = h->acc ? W > 1 : G <= kFewCopies;
+    const bool ragged = (M % 256 || N % 256) && (by_epilogue || few_launches);
+    const bool same_stream = in_any_case || in_stream(h, M, N, K, only_copies, monitor != 0, ragged);
+    const bool in_epilogue = by_epilogue && (in_any_case || !few_launches || 2.0 * M * N * K < kRsEpilogueBelowFlop);
     const int fused = same_stream ? 0 : fused_grid(h, G);
     fo_stream_t cstream = same_stream ? h->gemm_stream : h->comm_stream;
     int32_t wave = 0;
@@ -623,7 +641,7 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
         if (rc) return rc;
     }
     const bool quiet = same_stream && !monitor;  // as in fo_overlap_gemm_allreduce
-    if (quiet && by_epilogue) {
+    if (quiet && in_epilogue) {
         rc = fo_gemm_reduce_scatter(dtype, M, N, K, cseg_dev, G, A, B, C, h->acc, D, RA, RE, W, h->rank, algo, h->gemm_stream);
         if (rc) return rc;
         return link_time(h, (int64_t)M * N * 2, h->gemm_stream);

@@ -55,14 +55,19 @@ int fo_algo_info(int algo, int32_t info[12]);
  * counterpart of the hint that tune/search.py:83-157 measures in monitor
  * mode; order must hold (M/BM)*(N/BN) ints (host memory).  Where the last
  * wave of 256x256 workgroup tiles is at most half full, those tiles are
- * computed by a second launch in BM x BN tiles; the order lists them last. */
+ * computed by a second launch in BM x BN tiles; the order lists them last.
+ * It is the order of the launches that move counters (fo_gemm_signal,
+ * fo_gemm_scatter and the overlapped calls where a consumer waits).  What fits
+ * the chip in one round of workgroups, and every launch without counters, may
+ * use other tiles: those complete together, or are waited for by nobody. */
 int fo_schedule_order(int algo, int M, int N, int32_t *order);
 
 /* How the GEMM kernels cover the problem: reorder tiles per workgroup (the
  * workgroup tile may span several BM x BN tiles) and the number of workgroups.
  * One wave of the 256-CU chip completes 256 * tiles_per_workgroup tiles; the
  * reference's tuner uses sm_count - 2 tiles per wave (tune/search.py:404).
- * Both numbers describe the main launch's tiling of the whole problem. */
+ * Both numbers describe the main launch's tiling of the whole problem, for the
+ * launches whose order fo_schedule_order reports. */
 int fo_workgroup_tiles(int algo, int M, int N, int32_t *tiles_per_workgroup, int32_t *workgroups);
 /* Reorder tiles that complete together: the workgroups the persistent GEMM
  * keeps resident on the current device times the reorder tiles per workgroup
@@ -294,8 +299,9 @@ int fo_overlap_plan_norm_rows(const int32_t *RA_host, int TM, int TN, const int3
  * the stream orders the two, so MM is not touched and stays zero; with the
  * monitor on, the signalling GEMM and one wait over all groups as elsewhere),
  * and so does, without the monitor, a product of less than about one round of
- * 256x256 tiles, an all-reduce with neither accumulator nor normalisation, or a
- * reduce-scatter of more than 16 groups without accumulator;
+ * 256x256 tiles, one that 256 does not divide in M or N, an all-reduce with
+ * neither accumulator nor normalisation, or a reduce-scatter of more than 16
+ * groups without accumulator;
  * otherwise one launch when there are more than 16 groups, else per-wave
  * launches.  0: always the second stream with wait + consumer launches per
  * group (per GEMM wave) as the reference's host loop

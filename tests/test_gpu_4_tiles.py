@@ -298,3 +298,76 @@ def test_reduce_scatter_without_accumulator_by_groups(fo, groups):
     assert torch.equal(D.view(-1, 128), torch.cat(own))
     assert (MM == 0).all() and ov.status() == 0
     ov.close()
+
+
+@pytest.mark.parametrize("bm,bn,M,N", [
+    (128, 128, 4224, 4352),  # 256 divides N only
+    (128, 256, 4224, 4352),
+    (256, 128, 4352, 4224),  # 256 divides M only
+    (128, 128, 2432, 7040),  # neither
+    (128, 128, 8064, 4096),  # a last round that is nearly full
+    (128, 128, 4096, 6144),  # 256x256 tiles: a round and a half
+    (128, 256, 8192, 4096),  # 256x256 tiles: two rounds of whole rows
+])
+def test_counted_launch_walks_the_reported_order(fo, bm, bn, M, N):
+    """What a consumer waits for group by group completes in the order that it was told: with the slots in the order of
+    fo_schedule_order, workgroup w stamps the tiles of positions w, w + 256, ... one after the other."""
+    ops, K = fo.ops, 128
+    algo = fo._capi.find_algo(bm, bn, swizzle=4)
+    TM, TN = M // bm, N // bn
+    T = TM * TN
+    per = (256 // bm) * (256 // bn) if M % 256 == 0 and N % 256 == 0 else 1
+    A, _ = seeded((M, K), F16, 1)
+    B, _ = seeded((N, K), F16, 2, scale=K ** -0.5)
+    C = torch.empty(M * N, device="cuda", dtype=torch.float16)
+    RA = fo.layout.reorder_indices(T, fo._capi.schedule_order(algo, M, N)).reshape(TM, TN)
+    for RE in (None, fo.layout.generate_row_mapping(M, N, bm, bn, [T], 2)):
+        MM = torch.zeros(fo.layout.counter_size(1, TM, TN, True), dtype=torch.int32, device="cuda")
+        ops.gemm_signal(A, B, C, MM, RA, torch.tensor([T], dtype=torch.int32, device="cuda"), algo, monitor=True, RE=RE)
+        stamps = MM[TN:TN + T].cpu()
+        assert sorted(stamps.tolist()) == list(range(T))
+        rounds = stamps.reshape(-1, per)
+        assert (rounds[:-256].amax(dim=1) < rounds[256:].amin(dim=1)).all()
+    assert fo._capi.wave_tiles(algo, M, N) == 256 * per
+
+
+@pytest.mark.parametrize("M,N,K", [(4224, 4352, 2048), (8064, 8064, 4096)])  # 7.5e10 and 5.3e11 flop
+@pytest.mark.parametrize("with_acc", [True, False])
+@pytest.mark.parametrize("W", [1, 4])
+def test_reduce_scatter_that_256_does_not_divide(fo, M, N, K, with_acc, W):
+    """Both sides of the size from which such a call leaves sums and copies to launches behind the GEMM."""
+    ops, bm, groups = fo.ops, 128, 5
+    algo = fo._capi.find_algo(bm, 128, swizzle=4)
+    TM, TN = M // bm, N // 128
+    T = TM * TN
+    A, _ = seeded((M, K), F16, 1)
+    B, _ = seeded((N, K), F16, 2, scale=K ** -0.5)
+    plain = torch.empty(M, N, device="cuda", dtype=torch.float16)
+    ops.gemm(A, B, plain, algo)
+    cseg = [T // groups] * (groups - 1) + [T - T // groups * (groups - 1)]
+    RA = fo.layout.reorder_indices(T, fo._capi.schedule_order(algo, M, N)).reshape(TM, TN)
+    RE = fo.layout.generate_row_mapping(M, N, bm, 128, cseg, W)
+    cs_cpu = torch.tensor(cseg, dtype=torch.int32)
+    MM = torch.zeros(fo.layout.counter_size(groups, TM, TN), dtype=torch.int32, device="cuda")
+    before, _ = seeded((M * N,), F16, 7)
+    acc = before.clone()
+    ov = ops.Overlap(rank=W - 1, world=W)
+    ov.set_accumulator(acc if with_acc else None)
+    C = torch.full((M * N,), float("nan"), device="cuda", dtype=torch.float16)
+    D = torch.full((M // W, N), float("nan"), device="cuda", dtype=torch.float16)
+    ov.gemm_reducescatter_overlap(A, B, C, D, MM, RA, RE, 1, cs_cpu, cs_cpu.cuda(), algo)
+    torch.cuda.synchronize()
+    assert torch.equal(fo.layout.unpermute(C, M, N, bm, 128, RA, RE=RE), plain)
+    rows, seg, own, first = C.view(-1, 128), M * N // 128 // W, [], 0
+    want = torch.empty_like(rows)
+    for n in cseg:
+        chunk = rows[first:first + n * bm].view(W, n * bm // W, 128)
+        for q in range(W):
+            want[q * seg + first // W:q * seg + (first + n * bm) // W] = chunk[q]
+        own.append(chunk[W - 1])
+        first += n * bm
+    assert torch.equal(D.view(-1, 128), torch.cat(own))
+    if with_acc:
+        assert torch.equal(acc, (before.float() + want.reshape(-1).float()).half())
+    assert (MM == 0).all() and ov.status() == 0
+    ov.close()
