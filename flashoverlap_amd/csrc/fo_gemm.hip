@@ -64,7 +64,8 @@ struct launch_plan {
 };
 
 // A launch of parts of reorder tiles cannot count them; fo_signal_all_kernel behind it does (about 3 us).  Shorter
-// products than this many columns of K are computed in whole reorder tiles instead when counters are wanted.
+// products than this many columns of K are computed in whole reorder tiles instead when counters are wanted, and so is
+// whatever the monitor watches: its stamps say in which order the launch completed its tiles.
 constexpr int kSignalAfterFromK = 1536;
 
 // What one round of a tile takes, all CUs busy: microseconds at K = 4096, with operand rows on 128-byte lines and off them
@@ -173,18 +174,10 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int BM, int BN, bool w
 }
 
 // Signals of a launch whose workgroup tiles are parts of reorder tiles: behind it on the stream, everything at once
-// (such a launch is a single round of short tiles; its reorder tiles complete together anyway).  MM[g] += cseg[g]
-// and, with the monitor on, stamps in tile order (src/overlap/gemm_with_signal.h:343-351).
-__global__ __launch_bounds__(256) void fo_signal_all_kernel(const int32_t *cseg, int G, int32_t *MM, const int32_t *RA, int T,
-                                                            int TN, int monitor) {
+// (such a launch is a single round of short tiles; its reorder tiles complete together anyway).  MM[g] += cseg[g].
+__global__ __launch_bounds__(256) void fo_signal_all_kernel(const int32_t *cseg, int G, int32_t *MM) {
     for (int g = threadIdx.x; g < G; g += 256)
         __hip_atomic_fetch_add(MM + g, cseg[g], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (!monitor) return;
-    __shared__ int first;
-    if (threadIdx.x == 0) first = __hip_atomic_fetch_add(MM + (TN - 1), T, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    for (int t = threadIdx.x; t < T; t += 256)
-        __hip_atomic_store(MM + TN + RA[t], first + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // What the epilogue of a reduce-scatter on one stream does besides storing C (MODE_RS in fo_gemm_common.h).
@@ -224,7 +217,7 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     a.rank = rs ? rs->rank : 0;
     a.seg_rows = (int)((int64_t)M * N / a.BN / a.W);
     const bool counts = (mode == MODE_SIGNAL || mode == MODE_SCATTER) && !quiet;
-    const launch_plan plan = plan_launch(r, M, N, a.BM, a.BN, counts && K < kSignalAfterFromK, counts, on_lines(a));
+    const launch_plan plan = plan_launch(r, M, N, a.BM, a.BN, counts && (monitor || K < kSignalAfterFromK), counts, on_lines(a));
     a.grid_m = plan.grid_m; a.grid_n = plan.grid_n; a.panel = plan.panel; a.xcd_remap = plan.xcd_remap;
     a.first = 0; a.sub_m = a.sub_n = 1;
     a.count = plan.count;
@@ -247,7 +240,7 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     rc = launch_tile(dtype, mode, a, plan.tm, plan.tn, s, nullptr, plan.tail ? fo_main_tile_resident() : 0);
     if (rc) return rc;
     if (signal_after) {
-        hipLaunchKernelGGL(fo_signal_all_kernel, dim3(1), dim3(256), 0, s, cseg, G, MM, RA, (M / a.BM) * a.TN, a.TN, monitor);
+        hipLaunchKernelGGL(fo_signal_all_kernel, dim3(1), dim3(256), 0, s, cseg, G, MM);
         FO_LAUNCH_CHECK();
     }
     if (!plan.tail) return FO_OK;

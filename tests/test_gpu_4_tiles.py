@@ -371,3 +371,21 @@ def test_reduce_scatter_that_256_does_not_divide(fo, M, N, K, with_acc, W):
         assert torch.equal(acc, (before.float() + want.reshape(-1).float()).half())
     assert (MM == 0).all() and ov.status() == 0
     ov.close()
+
+
+@pytest.mark.parametrize("bm,bn,M,N,K", [(128, 128, 512, 4096, 2048), (128, 256, 256, 8192, 1544), (256, 128, 512, 4096, 1536)])
+def test_monitor_stamps_of_one_round_are_measured(fo, bm, bn, M, N, K):
+    """Products that a launch without the monitor computes in parts of reorder tiles: the stamps are the order in which
+    the launch completed the tiles (the eight XCDs interleave them), not the tiles' own order."""
+    ops, T = fo.ops, (M // bm) * (N // bn)
+    algo = fo._capi.find_algo(bm, bn, swizzle=4)
+    TN = N // bn
+    A, _ = seeded((M, K), F16, 1)
+    B, _ = seeded((N, K), F16, 2, scale=K ** -0.5)
+    C = torch.empty(M * N, device="cuda", dtype=torch.float16)
+    RA = torch.arange(T, dtype=torch.int32, device="cuda").reshape(M // bm, TN)
+    MM = torch.zeros(fo.layout.counter_size(1, M // bm, TN, True), dtype=torch.int32, device="cuda")
+    ops.gemm_signal(A, B, C, MM, RA, torch.tensor([T], dtype=torch.int32, device="cuda"), algo, monitor=True)
+    stamps = MM[TN:TN + T].tolist()
+    assert MM[0] == T and MM[TN - 1] == T and sorted(stamps) == list(range(T))
+    assert stamps != list(range(T))
