@@ -5,10 +5,11 @@
 // the two layers of a decode step (128x4096x1024, whose kernels run 8.5 us) 17.3 -> 11.1 us, the all-reduce call
 // 9.6 -> 4.0, the same with the normalisation 13.9 -> 6.8, the normalisation alone 9.3 -> 3.6.  Each function here does what its Python counterpart does
 // for the arguments of an ordinary call: the same checks, then one call of the C ABI.  Whatever it does not
-// recognise or would refuse it leaves alone: it returns None with nothing enqueued, and the caller takes its
-// Python path, which raises the proper error or handles the unusual argument.
+// recognise or its checks would refuse it leaves alone: it returns None without having called the C ABI, and the
+// caller takes its Python path, which raises the proper error or handles the unusual argument.
 //
-// Functions that enqueue return the C ABI's error code; the layer functions return the output tensor.
+// Functions that enqueue return the C ABI's error code; the layer functions return the output tensor, and raise what
+// the C ABI refuses: a second call by another path could enqueue twice.
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -247,9 +248,9 @@ PyObject *reorder_rmsnorm(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
     END_HANDLE_TH_ERRORS
 }
 
-// A layer's call that the C ABI refused: None as well, so that the layer's other path reports the error.
-PyObject *tensor_or_none(int rc, const at::Tensor &t) {
-    if (rc) Py_RETURN_NONE;
+// The output of a layer's call, or the error that the registered classes and operators raise for that code.
+PyObject *output_of(int rc, const char *what, const at::Tensor &t) {
+    TORCH_CHECK(rc == 0, "flashoverlap: ", what, " failed: ", fo_error_string(rc), " (code ", rc, ")");
     return THPVariable_Wrap(t);
 }
 
@@ -264,10 +265,11 @@ PyObject *allreduce_layer(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
     Product p;
     if (!in.done() || !p.fits(*A, *B) || !s.fits(p, nullptr, nullptr, 1)) Py_RETURN_NONE;
     const at::Tensor out = at::empty({p.M, p.N}, A->options());
-    return tensor_or_none(enqueue([&] {
+    const int rc = enqueue([&] {
         return fo_overlap_gemm_allreduce(h, dtype_of(*A), p.M, p.N, p.K, A->data_ptr(), B->data_ptr(), out.data_ptr(), ints(*s.MM),
                                          ints(*s.RA), s.TM(), s.TN(), 1, ints(*s.cseg_cpu), ints(*s.cseg_gpu), s.G(), s.algo, 0);
-    }), out);
+    });
+    return output_of(rc, "gemm_allreduce_overlap", out);
     END_HANDLE_TH_ERRORS
 }
 
@@ -285,11 +287,12 @@ PyObject *reducescatter_layer(PyObject *, PyObject *const *argv, Py_ssize_t argc
     Product p;
     if (!in.done() || !p.fits(*A, *B) || W <= 0 || p.M % W || !s.fits(p, RE, nullptr, W)) Py_RETURN_NONE;
     const at::Tensor all = at::empty({p.M, p.N}, A->options()), out = at::empty({p.M / W, p.N}, A->options());
-    return tensor_or_none(enqueue([&] {
+    const int rc = enqueue([&] {
         return fo_overlap_gemm_reducescatter(h, dtype_of(*A), p.M, p.N, p.K, A->data_ptr(), B->data_ptr(), all.data_ptr(),
                                              out.data_ptr(), ints(*s.MM), ints(*s.RA), ints(*RE), s.TM(), s.TN(), 1,
                                              ints(*s.cseg_cpu), ints(*s.cseg_gpu), s.G(), s.algo, 0);
-    }), out);
+    });
+    return output_of(rc, "gemm_reducescatter_overlap", out);
     END_HANDLE_TH_ERRORS
 }
 
@@ -303,7 +306,7 @@ PyObject *reorder_rmsnorm_layer(PyObject *, PyObject *const *argv, Py_ssize_t ar
     const double eps = in.real();
     if (!in.done() || !norm_fits(*X, *Wt, BM, BN, *RA)) Py_RETURN_NONE;
     const at::Tensor out = at::empty(X->sizes(), X->options());
-    return tensor_or_none(norm_on_current(*X, out, *Wt, BM, BN, 1, *RA, eps), out);
+    return output_of(norm_on_current(*X, out, *Wt, BM, BN, 1, *RA, eps), "reorder_rmsnorm", out);
     END_HANDLE_TH_ERRORS
 }
 

@@ -59,7 +59,7 @@ class ReorderRMSNorm(nn.Module):
                                                    self.eps)
         if out is not None:
             return out
-        out = torch.empty_like(x)  # an argument the native path leaves to this one, or refused
+        out = torch.empty_like(x)  # an argument the native path leaves to this one
         torch.ops.flashoverlap_op.reorder_rmsnorm_eps(x, out, self.weight, self.bm, self.bn, 1,
                                                       self.reorder_array, self.eps)
         return out
@@ -134,7 +134,7 @@ class OverlapRowParallelLayer(nn.Module):
                                                      self.algo, self.world_size)
         if out is not None:
             return out
-        # an argument the native path leaves to this one, or refused
+        # an argument the native path leaves to this one
         n = self.weight.size(0)
         if self.comm_op == "all_reduce":
             out = torch.empty((x.size(0), n), dtype=x.dtype, device=x.device)
