@@ -125,6 +125,9 @@ int fo_gemm_accumulate(int dtype, int M, int N, int K, int rLDN, const int32_t *
 int fo_gemm_reduce_scatter(int dtype, int M, int N, int K, const int32_t *cseg_dev, int G, const void *A, const void *B, void *C,
                            void *acc, void *own, const int32_t *RA, const int32_t *RE, int W, int rank, int algo,
                            fo_stream_t stream);
+// What fo_gemm_signal / fo_gemm_scatter (RE != nullptr) would refuse; nothing is enqueued.
+int fo_gemm_signal_check(int dtype, int M, int N, int K, int rLDN, const int32_t *cseg_dev, int G, const void *A, const void *B,
+                         const void *C, const int32_t *MM, const int32_t *RA, const int32_t *RE, int monitor, int algo);
 int fo_gemm_reordered_quiet(int dtype, int M, int N, int K, int rLDN, const int32_t *cseg_dev, int G,
                             const void *A, const void *B, void *C, const int32_t *RA, const int32_t *RE,
                             int algo, fo_stream_t stream);

@@ -186,21 +186,41 @@ struct rs_args {
     int W, rank;
 };
 
-int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *cseg, int G,
-             const void *A, const void *B, void *C, int32_t *MM, const int32_t *RA,
-             const int32_t *RE, int monitor, int algo, fo_stream_t stream, bool quiet = false, void *acc = nullptr,
-             const rs_args *rs = nullptr) {
+// What a launch refuses, asked before anything is enqueued.
+int check_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *cseg, int G, const void *A, const void *B,
+               const void *C, const int32_t *MM, const int32_t *RA, const int32_t *RE, int monitor, int algo, bool quiet,
+               const void *acc) {
     if (dtype != FO_F16 && dtype != FO_BF16) return FO_ERR_DTYPE;
     const fo_algo_entry *e = fo_algo_lookup(algo);
     if (!e) return FO_ERR_ALGO;
     if (!A || !B || !C || M <= 0 || N <= 0 || K <= 0) return FO_ERR_ARG;
-    fo_raster r;
-    int rc = fo_pick_raster(algo, M, N, &r);
-    if (rc) return rc;
+    if (M % e->f[0] || N % e->f[1]) return FO_ERR_SHAPE;
     if (K % 8) return FO_ERR_SHAPE;  // operand rows are fetched in 16-byte chunks
     if (K > (1 << 21)) return FO_ERR_SHAPE;  // 256 operand rows are addressed through one 31-bit buffer range
     // the epilogues assume reorder tiles made of 128 x 128 blocks
     if (e->f[0] % 128 || e->f[1] % 128) return FO_ERR_ALGO;
+    if (mode == MODE_ACC && (((uintptr_t)C | (uintptr_t)acc) & 15)) return FO_ERR_SHAPE;  // as the consumer launch would
+    if (mode == MODE_PLAIN || (mode == MODE_ACC && !RA)) return FO_OK;
+    const int TN = N / e->f[1];
+    const long T = (long)(M / e->f[0]) * TN;
+    if ((!MM && !quiet) || !RA || !cseg) return FO_ERR_ARG;
+    if ((mode == MODE_SCATTER || mode == MODE_RS) && !RE) return FO_ERR_ARG;
+    if (rLDN <= 0 || T % rLDN) return FO_ERR_SHAPE;
+    if (G <= 0 || G > T) return FO_ERR_SEGMENTS;
+    if (monitor && G > TN - 1) return FO_ERR_SEGMENTS;
+    return FO_OK;
+}
+
+int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *cseg, int G,
+             const void *A, const void *B, void *C, int32_t *MM, const int32_t *RA,
+             const int32_t *RE, int monitor, int algo, fo_stream_t stream, bool quiet = false, void *acc = nullptr,
+             const rs_args *rs = nullptr) {
+    int rc = check_gemm(mode, dtype, M, N, K, rLDN, cseg, G, A, B, C, MM, RA, RE, monitor, algo, quiet, acc);
+    if (rc) return rc;
+    const fo_algo_entry *e = fo_algo_lookup(algo);
+    fo_raster r;
+    rc = fo_pick_raster(algo, M, N, &r);
+    if (rc) return rc;
     GemmArgs a;
     a.A = static_cast<const uint16_t *>(A);
     a.B = static_cast<const uint16_t *>(B);
@@ -226,15 +246,6 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     const bool signal_after = counts && !plan.whole;
     a.quiet = quiet || signal_after ? 1 : 0;
     a.stream_out = (int64_t)M * N * 2 > kStreamOutAboveBytes ? 1 : 0;
-    if (mode == MODE_ACC && (((uintptr_t)C | (uintptr_t)acc) & 15)) return FO_ERR_SHAPE;  // as the consumer launch would
-    if (mode != MODE_PLAIN && !(mode == MODE_ACC && !RA)) {
-        const long T = (long)(M / a.BM) * a.TN;
-        if ((!MM && !quiet) || !RA || !cseg) return FO_ERR_ARG;
-        if ((mode == MODE_SCATTER || mode == MODE_RS) && !RE) return FO_ERR_ARG;
-        if (rLDN <= 0 || T % rLDN) return FO_ERR_SHAPE;
-        if (G <= 0 || G > T) return FO_ERR_SEGMENTS;
-        if (monitor && G > a.TN - 1) return FO_ERR_SEGMENTS;
-    }
     hipStream_t s = static_cast<hipStream_t>(stream);
     // the tail split was computed for that many workgroups of the main launch
     rc = launch_tile(dtype, mode, a, plan.tm, plan.tn, s, nullptr, plan.tail ? fo_main_tile_resident() : 0);
@@ -301,6 +312,12 @@ int fo_gemm_reordered_quiet(int dtype, int M, int N, int K, int rLDN, const int3
                             int algo, fo_stream_t stream) {
     return run_gemm(RE ? MODE_SCATTER : MODE_SIGNAL, dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, nullptr, RA, RE,
                     0, algo, stream, true);
+}
+
+int fo_gemm_signal_check(int dtype, int M, int N, int K, int rLDN, const int32_t *cseg_dev, int G, const void *A, const void *B,
+                         const void *C, const int32_t *MM, const int32_t *RA, const int32_t *RE, int monitor, int algo) {
+    return check_gemm(RE ? MODE_SCATTER : MODE_SIGNAL, dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, MM, RA, RE, monitor, algo,
+                      false, nullptr);
 }
 
 int fo_gemm_accumulate(int dtype, int M, int N, int K, int rLDN, const int32_t *cseg_dev, int G, const void *A, const void *B,

@@ -61,7 +61,9 @@ struct fo_overlap {
     int fused_from_groups = kFusedFromGroups;
     double in_stream_below_flop = kInStreamBelowFlop;
     int token = 1;         // value the fork and join words carry from one stream to the other
-    bool always_fork = false;  // the consumer stream must not start before this call's first kernel on the GEMM stream
+    // A handle-free call: its words may hold what another call left.  They are cleared first, and the consumer stream
+    // must not start before that.
+    bool static_words = false;
     // Link-rate model (fo_overlap_set_link_rate): bytes per second a collective over the group's bytes would
     // sustain; 0: none.  With a rate every consumer launch is followed on its stream by a kernel that holds the
     // stream for the bytes' link time, so that the schedule can be timed against a link-bound collective on
@@ -86,11 +88,12 @@ namespace {
 // what that saves is more than the second stream hides (us, two streams -> one, with an accumulator and the normalisation:
 // 3456x4352x3072 127 -> 93, 2432x7040x7056 271 -> 245, 8064x8064x4096 586 -> 465, 6272x8192x7168 661 -> 636; reduce-scatter,
 // eight ranks: 3456x4352x3072 123 -> 95, 4224x7168x3584 205 -> 194, 6272x8192x7168 651 -> 630, 8192x8064x7168 801 -> 751).
-bool in_stream(const fo_overlap *h, int M, int N, int K, bool idle, bool monitor, bool ragged) {
+// `fits`: the accumulator is one that every path takes; one that is not aligned is left to the one-launch consumer.
+bool in_stream(const fo_overlap *h, int M, int N, int K, bool idle, bool monitor, bool ragged, bool fits) {
     if (!h->comm_stream) return true;
     if (h->fused >= 0 || h->link_bytes_per_s > 0 || h->in_stream_below_flop <= 0) return false;
     if (2.0 * M * N * K < h->in_stream_below_flop) return true;
-    if (monitor) return false;  // its GEMM counts and is waited for in any case
+    if (monitor || !fits) return false;  // the monitor's GEMM counts and is waited for in any case
     return idle || ragged || (long)((M + 255) / 256) * ((N + 255) / 256) * 6 <= (long)fo_main_tile_resident() * 5;
 }
 
@@ -173,6 +176,11 @@ bool apart(span out, std::initializer_list<span> others) {
     return true;
 }
 
+// Whether the consumer launches take these buffers (16-byte accesses; null: none).
+bool aligned(const void *C, const void *acc, const void *own = nullptr) {
+    return !(((uintptr_t)C | (uintptr_t)acc | (uintptr_t)own) & 15);
+}
+
 // While the GEMM stream is being captured into a HIP graph the two streams are tied
 // together with events, as in the reference (src/overlap_impl.cu:246, :260-263): the
 // event wait pulls the consumer stream into the capture, and in the graph the dependency
@@ -196,7 +204,7 @@ int fork(fo_overlap *h, bool captured, bool polling_consumer) {
         FO_HIP_CHECK(hipStreamWaitEvent(h->comm_stream, h->forked, 0));
         return FO_OK;
     }
-    if (!polling_consumer && !h->always_fork) return FO_OK;
+    if (!polling_consumer && !h->static_words) return FO_OK;
     int rc = fo_set(h->workspace + kWsFork, h->token, h->gemm_stream);
     if (rc) return rc;
     return fo_wait_with(h->token, h->workspace + kWsFork, h->max_polls, h->workspace + kWsGaveUp, h->comm_stream);
@@ -441,7 +449,8 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
         if (N % 8 || N > 16384 || (int64_t)M * N * 2 > 0xFFFFFFFFLL) return FO_ERR_SHAPE;
     }
 
-    const bool same_stream = in_stream(h, M, N, K, !h->acc && !np, monitor != 0, M % 256 || N % 256);
+    const bool fits = !h->acc || aligned(C, h->acc);
+    const bool same_stream = in_stream(h, M, N, K, !h->acc && !np, monitor != 0, M % 256 || N % 256, fits);
     if (np) {
         // on one stream all rows follow in one launch, whatever their slots
         rc = same_stream ? check_slots(np->RA_host, TM * TN) : last_slots(np->RA_host, TM, TN, last_slot);
@@ -456,7 +465,18 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
         rc = fo_gemm_wave_tiles(dtype, algo, M, N, &wave);
         if (rc) return rc;
     }
+    // Whatever can be refused is refused here: a refusal between the launches would leave counters standing and the
+    // streams apart.
+    rc = fo_gemm_signal_check(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, MM, RA, nullptr, monitor, algo);
+    if (rc) return rc;
+    if (!fused && !fits) return FO_ERR_SHAPE;
     const bool captured = !same_stream && capturing(h);
+    if (h->static_words) {
+        // By a kernel, not a memset node, in case the GEMM stream is being captured.  The give-up word is left standing:
+        // fo_static_status reads and clears it.
+        rc = fo_fill_words(h->workspace, kWorkspaceWords + G, 0, h->gemm_stream, kWsGaveUp);
+        if (rc) return rc;
+    }
     if (!same_stream) {
         rc = fork(h, captured, fused != 0);
         if (rc) return rc;
@@ -617,14 +637,19 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     // 5504x3840x3640 with four ranks, two streams against one, us: 4 groups 192 and 186, 16 214 and 187, 64 320 and 187, 1290
     // 3404 and 218; 8192x4096x4096 with two: 4 groups 228 and 249, 16 236 and 247, 24 284 and 252, 64 369 and 253.
     const bool only_copies = !h->acc && by_epilogue && G > h->fused_from_groups;
-    const bool in_any_case = in_stream(h, M, N, K, only_copies, monitor != 0, false);
+    // With an accumulator and W > 1 the consumer also writes this rank's chunk of
+    // every group to D (ncclReduceScatter(C+acc -> D+acc/W, n/W) with one rank
+    // present, src/overlap_impl.cu:312-313); otherwise a copy per group does.
+    const bool own_in_consumer = D && h->acc && W > 1;
+    const bool fits = !h->acc || aligned(C, h->acc, own_in_consumer ? D : nullptr);
+    const bool in_any_case = in_stream(h, M, N, K, only_copies, monitor != 0, false, fits);
     // A large ragged call leaves the rest to launches behind the GEMM (one consumer launch for all groups, or a few copies):
     // the epilogue holds up the next tile's loads.  By the epilogue and by launches, us, eight ranks and an accumulator:
     // 8192x8064x7168 803 and 751, 8064x8064x4096 494 and 470 (two ranks 508 and 509), 4224x7168x3584 194 and 193,
     // 8064x8192x1024 183 and 200; sixteen copies: 8192x8064x7168 737 and 693, 4224x7168x3584 182 and 192.
     const bool few_launches = h->acc ? W > 1 : G <= kFewCopies;
     const bool ragged = (M % 256 || N % 256) && (by_epilogue || few_launches);
-    const bool same_stream = in_any_case || in_stream(h, M, N, K, only_copies, monitor != 0, ragged);
+    const bool same_stream = in_any_case || in_stream(h, M, N, K, only_copies, monitor != 0, ragged, fits);
     const bool in_epilogue = by_epilogue && (in_any_case || !few_launches || 2.0 * M * N * K < kRsEpilogueBelowFlop);
     const int fused = same_stream ? 0 : fused_grid(h, G);
     fo_stream_t cstream = same_stream ? h->gemm_stream : h->comm_stream;
@@ -635,6 +660,9 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
         rc = fo_gemm_wave_tiles(dtype, algo, M, N, &wave);
         if (rc) return rc;
     }
+    rc = fo_gemm_signal_check(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, MM, RA, RE, monitor, algo);
+    if (rc) return rc;
+    if (!fused && !fits) return FO_ERR_SHAPE;
     const bool captured = !same_stream && capturing(h);
     if (!same_stream) {
         rc = fork(h, captured, fused != 0);
@@ -655,10 +683,6 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     uint16_t *c = static_cast<uint16_t *>(C);
     uint16_t *d = static_cast<uint16_t *>(D);
     uint16_t *acc = static_cast<uint16_t *>(h->acc);
-    // With an accumulator and W > 1 the consumer also writes this rank's chunk of
-    // every group to D (ncclReduceScatter(C+acc -> D+acc/W, n/W) with one rank
-    // present, src/overlap_impl.cu:312-313); otherwise a copy per group does.
-    const bool own_in_consumer = d && acc && W > 1;
     const bool stream_acc = fo_streams((int64_t)M * N * 4);
     if (fused) {
         rc = fo_wait_reduce_groups_with(dtype, C, h->acc, MM, cseg_dev, G, tile_elems, W, seg_stride,
@@ -719,9 +743,12 @@ extern "C" int fo_overlap_gemm_allreduce_serial(fo_overlap_t *h, int dtype, int 
     if (!h->gemm_ready) return FO_ERR_STATE;
     if (h->acc && h->acc_nelem < (int64_t)M * N) return FO_ERR_ARG;
     const int64_t mn = (int64_t)M * N;
+    int rc = link_fits(h, mn * 2);
+    if (rc) return rc;
+    if (h->acc && !aligned(C, h->acc)) return FO_ERR_SHAPE;
     const bool consumed = h->acc && apart({h->acc, mn}, {{A, (int64_t)M * K}, {B, (int64_t)N * K}, {C, mn}});
-    int rc = consumed ? fo_gemm_accumulate(dtype, M, N, K, 1, nullptr, 0, A, B, C, h->acc, nullptr, algo, h->gemm_stream)
-                      : fo_gemm(dtype, M, N, K, A, B, C, algo, h->gemm_stream);
+    rc = consumed ? fo_gemm_accumulate(dtype, M, N, K, 1, nullptr, 0, A, B, C, h->acc, nullptr, algo, h->gemm_stream)
+                  : fo_gemm(dtype, M, N, K, A, B, C, algo, h->gemm_stream);
     if (!rc && h->acc && !consumed) rc = fo_consumer_reduce(dtype, C, h->acc, mn, h->gemm_stream);
     if (rc) return rc;
     return link_time(h, (int64_t)M * N * 2, h->gemm_stream);
@@ -735,11 +762,21 @@ extern "C" int fo_overlap_seg_allreduce(fo_overlap_t *h, int dtype, void *C, int
     if (h->acc && h->acc_nelem < MN) return FO_ERR_ARG;
     const int64_t unit = MN / seg_num;
     int64_t off = 0;
+    if (h->acc && !aligned(C, h->acc)) return FO_ERR_SHAPE;
+    for (int s = 0; s < seg_num; s++) {  // all of them before the first is enqueued
+        const int64_t n = unit * cseg_host[s];
+        if (off + n > MN) return FO_ERR_SEGMENTS;
+        if (h->acc && n < 0) return FO_ERR_ARG;
+        if (h->acc && n % 8) return FO_ERR_SHAPE;
+        const int rc = link_fits(h, n * 2);
+        if (rc) return rc;
+        off += n;
+    }
+    off = 0;
     uint16_t *c = static_cast<uint16_t *>(C);
     uint16_t *acc = static_cast<uint16_t *>(h->acc);
     for (int s = 0; s < seg_num; s++) {  // the reference iterates SegNum times over cSEG_CPU
         const int64_t n = unit * cseg_host[s];
-        if (off + n > MN) return FO_ERR_SEGMENTS;
         if (acc) {
             int rc = fo_consumer_reduce(dtype, c + off, acc + off, n, h->gemm_stream);
             if (rc) return rc;
@@ -808,22 +845,8 @@ extern "C" int fo_gemm_allreduce_overlap_static(int dtype, int M, int N, int K, 
     ctx.acc_nelem = acc ? (int64_t)M * N : 0;
     ctx.fused = fused < 0 ? -1 : fused;
     ctx.token = token;
-    ctx.always_fork = true;
-    // Validate before the first launch, so that a refused call leaves nothing enqueued.
-    int32_t info[12];
-    rc = fo_algo_info(algo, info);
-    if (rc) return rc;
-    if (M <= 0 || N <= 0 || M % info[0] || N % info[1] || TM != M / info[0] || TN != N / info[1]) return FO_ERR_SHAPE;
-    rc = check_segments(cseg_host, G, (long)TM * TN);
-    if (rc) return rc;
-    if (!A || !B || !C || !RA || K <= 0 || K % 8) return !A || !B || !C || !RA || K <= 0 ? FO_ERR_ARG : FO_ERR_SHAPE;
+    ctx.static_words = true;
     if (ctx.comm_stream && capturing(&ctx)) return FO_ERR_STATE;  // two streams under capture need the handle's events
-    // The array keeps what the last call on this device left: counters of a call whose
-    // bounded wait gave up would still be standing.  Cleared by a kernel, not a memset
-    // node, in case the GEMM stream is being captured.
-    // The give-up word is left standing: fo_static_status reads and clears it.
-    rc = fo_fill_words(ws, kWorkspaceWords + G, 0, ctx.gemm_stream, kWsGaveUp);
-    if (rc) return rc;
     return allreduce_overlap(&ctx, dtype, M, N, K, A, B, C, ws + kWorkspaceWords, RA, TM, TN, rLDN, cseg_host,
                              cseg_dev, G, algo, 0);
 }

@@ -775,3 +775,54 @@ def test_overlapped_step_captured_in_a_hip_graph(fo, fused, one_call):
         assert torch.equal(ACC.float(), expect), f"replay {it}"
         assert (MM == 0).all()
     ov.close()
+
+
+@pytest.mark.parametrize("call", ["allreduce", "norm", "reducescatter", "serial", "link", "segments"])
+def test_a_refused_call_enqueues_nothing(fo, call):
+    """A refusal leaves every buffer as it was, the counters zero and the handle usable, on two streams as well (6.9e10 flop,
+    256 workgroup tiles)."""
+    ops, M, N, K, bm, W = fo.ops, 4096, 4096, 2048, 128, 2
+    algo = fo._capi.find_algo(bm, bm, swizzle=4)
+    TM, TN = M // bm, N // bm
+    T = TM * TN
+    cs = torch.tensor([T // 4] * 4, dtype=torch.int32)
+    A, B = (torch.ones(r, K, device="cuda", dtype=torch.float16) for r in (M, N))
+    C = torch.full((M, N), -1.0, device="cuda", dtype=torch.float16)
+    Y, D, w = C.clone(), C[:M // W].clone(), torch.ones(N, device="cuda", dtype=torch.float16)
+    acc = torch.full((M * N + 8,), -1.0, device="cuda", dtype=torch.float16)
+    RA = torch.arange(T, dtype=torch.int32, device="cuda").reshape(TM, TN)
+    RE = fo.layout.generate_row_mapping(M, N, bm, bm, cs.tolist(), W)
+    MM = torch.zeros(fo.layout.counter_size(4, TM, TN), dtype=torch.int32, device="cuda")
+    ov = ops.Overlap(world=W)
+    ov.set_accumulator(acc[1:M * N + 1])   # off the consumer's 16-byte pieces
+    code = -2
+    with pytest.raises(fo.FlashOverlapError) as e:
+        if call == "allreduce":
+            ov.gemm_allreduce_overlap(A, B, C, MM, RA, 1, cs, cs.cuda(), algo)
+        elif call == "norm":
+            ov.gemm_allreduce_rmsnorm_overlap(A, B, C, MM, RA, RA.cpu(), 1, cs, cs.cuda(), algo, Y, w)
+        elif call == "reducescatter":
+            ov.gemm_reducescatter_overlap(A, B, C, D, MM, RA, RE, 1, cs, cs.cuda(), algo)
+        elif call == "serial":
+            ov.set_accumulator(C.view(-1)[:M * N])
+            ov.set_link_rate(1e-3)         # half a minute of link time
+            code = -7
+            ov.gemm_allreduce(A, B, C, algo)
+        elif call == "link":
+            ov.set_accumulator(acc[:M * N])
+            ov.set_link_rate(1e-3)
+            code = -7
+            ov.gemm_allreduce_overlap(A, B, C, MM, RA, 1, cs, cs.cuda(), algo)
+        else:                              # the second of two segments reaches beyond C
+            ov.set_accumulator(acc[:M * N])
+            code = -5
+            ov.seg_allreduce(C, torch.tensor([1, 2], dtype=torch.int32), 2)
+    assert e.value.code == code
+    torch.cuda.synchronize()
+    assert all((t == -1).all() for t in (C, Y, D, acc)) and (MM == 0).all()
+    ov.set_link_rate(0)
+    ov.set_accumulator(None)
+    ov.gemm_allreduce_overlap(A, B, C, MM, RA, 1, cs, cs.cuda(), algo)
+    torch.cuda.synchronize()
+    assert (C == K).all() and (MM == 0).all() and ov.status() == 0
+    ov.close()
