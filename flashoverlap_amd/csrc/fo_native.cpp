@@ -11,6 +11,10 @@
 // Functions that enqueue return the C ABI's error code; the layer functions return the output tensor, and raise what
 // the C ABI refuses: a second call by another path could enqueue twice.
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/record_function.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/Exceptions.h>
@@ -44,6 +48,11 @@ struct Args {
         // tensors that Python code dispatches on (fake tensors, wrapper subclasses) have no memory to point at
         if (!t.defined() || t.key_set().has(c10::DispatchKey::Python) || !t.has_storage()) ok = false;
         return &t;
+    }
+    // A tensor of no class but torch's own: what the other path makes of a subclass (its results' class, its hooks) stays with it.
+    const at::Tensor *plain_tensor() {
+        if (i < n && !THPVariable_CheckExact(a[i])) ok = false;
+        return tensor();
     }
     const at::Tensor *tensor_or_none() {
         if (i < n && a[i] == Py_None) {
@@ -220,6 +229,13 @@ PyObject *reducescatter(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
     END_HANDLE_TH_ERRORS
 }
 
+// Whether somebody follows the operators that run (a profiler or tracer, a function or dispatch mode, a transform): the
+// layers then go through the registered ones.
+bool followed() {
+    return at::hasCallbacks() || at::impl::torch_function_mode_enabled() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+           !(c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty();
+}
+
 bool norm_fits(const at::Tensor &X, const at::Tensor &Wt, int BM, int BN, const at::Tensor &RA) {
     if (X.dim() != 2 || !value_type(X) || !on_gpu(X) || !values(Wt, X) || Wt.numel() < X.size(1) || !gpu_ints(RA)) return false;
     const int64_t bs = X.size(0), dim = X.size(1);
@@ -259,11 +275,11 @@ PyObject *allreduce_layer(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
     HANDLE_TH_ERRORS
     Args in{argv, argc};
     fo_overlap_t *h = static_cast<fo_overlap_t *>(in.pointer());
-    const at::Tensor *A = in.tensor(), *B = in.tensor();
+    const at::Tensor *A = in.plain_tensor(), *B = in.plain_tensor();
     Schedule s;
     s.MM = in.tensor(), s.RA = in.tensor(), s.cseg_cpu = in.tensor(), s.cseg_gpu = in.tensor(), s.algo = in.int32();
     Product p;
-    if (!in.done() || !p.fits(*A, *B) || !s.fits(p, nullptr, nullptr, 1)) Py_RETURN_NONE;
+    if (followed() || !in.done() || !p.fits(*A, *B) || !s.fits(p, nullptr, nullptr, 1)) Py_RETURN_NONE;
     const at::Tensor out = at::empty({p.M, p.N}, A->options());
     const int rc = enqueue([&] {
         return fo_overlap_gemm_allreduce(h, dtype_of(*A), p.M, p.N, p.K, A->data_ptr(), B->data_ptr(), out.data_ptr(), ints(*s.MM),
@@ -278,14 +294,14 @@ PyObject *reducescatter_layer(PyObject *, PyObject *const *argv, Py_ssize_t argc
     HANDLE_TH_ERRORS
     Args in{argv, argc};
     fo_overlap_t *h = static_cast<fo_overlap_t *>(in.pointer());
-    const at::Tensor *A = in.tensor(), *B = in.tensor();
+    const at::Tensor *A = in.plain_tensor(), *B = in.plain_tensor();
     Schedule s;
     s.MM = in.tensor(), s.RA = in.tensor();
     const at::Tensor *RE = in.tensor();
     s.cseg_cpu = in.tensor(), s.cseg_gpu = in.tensor(), s.algo = in.int32();
     const int64_t W = in.integer();
     Product p;
-    if (!in.done() || !p.fits(*A, *B) || W <= 0 || p.M % W || !s.fits(p, RE, nullptr, W)) Py_RETURN_NONE;
+    if (followed() || !in.done() || !p.fits(*A, *B) || W <= 0 || p.M % W || !s.fits(p, RE, nullptr, W)) Py_RETURN_NONE;
     const at::Tensor all = at::empty({p.M, p.N}, A->options()), out = at::empty({p.M / W, p.N}, A->options());
     const int rc = enqueue([&] {
         return fo_overlap_gemm_reducescatter(h, dtype_of(*A), p.M, p.N, p.K, A->data_ptr(), B->data_ptr(), all.data_ptr(),
@@ -300,11 +316,11 @@ PyObject *reducescatter_layer(PyObject *, PyObject *const *argv, Py_ssize_t argc
 PyObject *reorder_rmsnorm_layer(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
     HANDLE_TH_ERRORS
     Args in{argv, argc};
-    const at::Tensor *X = in.tensor(), *Wt = in.tensor();
+    const at::Tensor *X = in.plain_tensor(), *Wt = in.plain_tensor();
     const int BM = in.int32(), BN = in.int32();
     const at::Tensor *RA = in.tensor();
     const double eps = in.real();
-    if (!in.done() || !norm_fits(*X, *Wt, BM, BN, *RA)) Py_RETURN_NONE;
+    if (followed() || !in.done() || !norm_fits(*X, *Wt, BM, BN, *RA)) Py_RETURN_NONE;
     const at::Tensor out = at::empty(X->sizes(), X->options());
     return output_of(norm_on_current(*X, out, *Wt, BM, BN, 1, *RA, eps), "reorder_rmsnorm", out);
     END_HANDLE_TH_ERRORS

@@ -49,3 +49,52 @@ def test_a_refused_layer_call_is_not_made_again(fo, comm_op):
         assert proj(x).shape == (M // 2 if comm_op == "reduce_scatter" else M, N)
     torch.cuda.synchronize()
     assert (proj.counter == 0).all()
+
+
+class Tagged(torch.Tensor):
+    """A subclass without a dispatch of its own."""
+
+
+class Seen(torch.overrides.TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.names.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+def test_the_norm_layer_keeps_classes_and_is_seen(fo):
+    """A subclass goes through torch.empty_like and the registered operator, and so does every call that a mode or the
+    profiler follows; the values are those of the native call."""
+    from flashoverlap_amd import layers
+    M, N = 256, 1024
+    hint = fo._capi.schedule_order(fo._capi.find_algo(128, 128), M, N)
+    norm = layers.ReorderRMSNorm(N, M, 128, 128, hint)
+    x = torch.randn(M, N, device="cuda").half()
+    with torch.no_grad():
+        want = norm(x)
+        tagged = norm(x.as_subclass(Tagged))
+        assert type(want) is torch.Tensor and type(tagged) is Tagged
+        with Seen() as seen:
+            followed = norm(x)
+        assert any("reorder_rmsnorm_eps" in name for name in seen.names), seen.names
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+            profiled = norm(x)
+        assert any("reorder_rmsnorm_eps" in event.key for event in prof.key_averages())
+    for y in (tagged.as_subclass(torch.Tensor), followed, profiled):
+        assert torch.equal(y, want)
+
+
+def test_the_projection_layer_takes_a_subclass(fo):
+    M, N, K = 256, 512, 64
+    proj, hint = _projection(fo, M, N, K)
+    proj.overlap_class = Watched(proj.overlap_class)
+    x = torch.randn(M, K, device="cuda").half()
+    with torch.no_grad():
+        want = proj(x)
+        assert proj.overlap_class.calls == []
+        got = proj(x.as_subclass(Tagged))
+        assert proj.overlap_class.calls == ["gemm_allreduce_overlap"]
+    assert torch.equal(got.as_subclass(torch.Tensor), want)
