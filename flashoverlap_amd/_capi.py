@@ -104,6 +104,14 @@ def lib():
     return _lib
 
 
+class _NoNative:
+    """Stands in for the extension module where only the kernel library was built (build_all(shim=False)): every call
+    is left to the Python path."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 _native = None
 
 
@@ -113,7 +121,8 @@ def native():
     global _native
     if _native is None:
         if not os.path.exists(NATIVE_LIB):
-            raise ImportError(f"{NATIVE_LIB} is missing: build it with `python -m flashoverlap_amd.build`")
+            _native = _NoNative()
+            return _native
         import torch  # noqa: F401  the module links against torch's libraries
         spec = importlib.util.spec_from_file_location("flashoverlap_amd._fo_native", NATIVE_LIB)
         module = importlib.util.module_from_spec(spec)

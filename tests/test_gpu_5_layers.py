@@ -98,3 +98,33 @@ def test_the_projection_layer_takes_a_subclass(fo):
         got = proj(x.as_subclass(Tagged))
         assert proj.overlap_class.calls == ["gemm_allreduce_overlap"]
     assert torch.equal(got.as_subclass(torch.Tensor), want)
+
+
+def test_calls_without_the_extension_module(fo, monkeypatch, tmp_path):
+    """The kernel library alone serves the overlapped calls and the normalisation, with the same results."""
+    ops, M, N, K = fo.ops, 256, 512, 64
+    algo = fo._capi.find_algo(128, 128)
+    T, TN = M // 128 * (N // 128), N // 128
+    A, B = torch.randn(M, K, device="cuda").half(), torch.randn(N, K, device="cuda").half()
+    w = torch.rand(N, device="cuda").half()
+    RA = torch.arange(T, dtype=torch.int32, device="cuda").flip(0).contiguous().reshape(M // 128, TN)
+    RE = fo.layout.generate_row_mapping(M, N, 128, 128, [T // 2, T // 2], 2)
+    cs = torch.tensor([T // 2, T // 2], dtype=torch.int32)
+
+    def results():
+        MM = torch.zeros(fo.layout.counter_size(2, M // 128, TN), dtype=torch.int32, device="cuda")
+        C, Y, Z = (torch.empty(M, N, device="cuda", dtype=torch.float16) for _ in range(3))
+        D = torch.empty(M // 2, N, device="cuda", dtype=torch.float16)
+        ov = ops.Overlap(world=2)
+        ov.gemm_reducescatter_overlap(A, B, C, D, MM, RA, RE, 1, cs, cs.cuda(), algo)
+        ov.gemm_allreduce_overlap(A, B, C, MM, RA, 1, cs, cs.cuda(), algo)
+        ov.gemm_allreduce_rmsnorm_overlap(A, B, C, MM, RA, RA.cpu(), 1, cs, cs.cuda(), algo, Y, w)
+        ops.reorder_rmsnorm(C, Z, w, 128, 128, 1, RA)
+        torch.cuda.synchronize()
+        ov.close()
+        return C, D, Y, Z, MM
+
+    want = results()
+    monkeypatch.setattr(fo._capi, "NATIVE_LIB", str(tmp_path / "_fo_native.so"))
+    monkeypatch.setattr(fo._capi, "_native", None)
+    assert all(torch.equal(a, b) for a, b in zip(results(), want))

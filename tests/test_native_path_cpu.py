@@ -35,3 +35,15 @@ def test_norm_and_layers_decline():
     one, algo = torch.ones(1, **I32), fo._capi.find_algo(128, 128)
     assert native.allreduce_layer(1, X, X, one, RA, one, one, algo) is None
     assert native.reducescatter_layer(1, X, X, one, RA, one, one, one, algo, 0) is None
+
+
+def test_the_kernel_library_alone_is_enough(monkeypatch, tmp_path):
+    """Without the extension module (a build without the torch parts) the Python path serves the calls: here it refuses
+    tensors in host memory itself."""
+    monkeypatch.setattr(fo._capi, "NATIVE_LIB", str(tmp_path / "_fo_native.so"))
+    monkeypatch.setattr(fo._capi, "_native", None)
+    ops = fo.ops
+    X, w, RA = torch.zeros(128, 128, dtype=H), torch.zeros(128, dtype=H), torch.zeros(1, 1, **I32)
+    with pytest.raises(ValueError, match="must live on the GPU"):
+        ops.reorder_rmsnorm(X, X.clone(), w, 128, 128, 1, RA, stream=None)
+    assert fo._capi.native().allreduce(*_overlap_args()) is None
