@@ -34,7 +34,7 @@ enum {
 // GEMM cost more than such a GEMM can hide (4096x4096x512 with 256 groups:
 // 71 us overlapped, 44 us in stream).
 //
-// kRsEpilogueBelowFlop, kFewCopies: see fo_overlap_gemm_reducescatter.
+// kRsEpilogueBelowFlop, kFewCopies: see fo_overlap_gemm_reducescatter.  Neither is a threshold of a handle.
 //
 // kGemmFlopPerNs: what a GEMM is expected to sustain, for sizing the pause
 // between polls only.
@@ -636,7 +636,7 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     // Without an accumulator all there is to overlap are those copies, and with many groups they take longer than the GEMM:
     // 5504x3840x3640 with four ranks, two streams against one, us: 4 groups 192 and 186, 16 214 and 187, 64 320 and 187, 1290
     // 3404 and 218; 8192x4096x4096 with two: 4 groups 228 and 249, 16 236 and 247, 24 284 and 252, 64 369 and 253.
-    const bool only_copies = !h->acc && by_epilogue && G > h->fused_from_groups;
+    const bool only_copies = !h->acc && by_epilogue && G > kFewCopies;
     // With an accumulator and W > 1 the consumer also writes this rank's chunk of
     // every group to D (ncclReduceScatter(C+acc -> D+acc/W, n/W) with one rank
     // present, src/overlap_impl.cu:312-313); otherwise a copy per group does.

@@ -826,3 +826,27 @@ def test_a_refused_call_enqueues_nothing(fo, call):
     torch.cuda.synchronize()
     assert (C == K).all() and (MM == 0).all() and ov.status() == 0
     ov.close()
+
+
+@pytest.mark.parametrize("groups,fused_from,two_streams", [(4, -1, True), (4, 2, True), (16, 2, True), (17, -1, False), (17, 64, False)])
+def test_stream_choice_of_a_reduce_scatter_without_accumulator(fo, groups, fused_from, two_streams):
+    """A long reduce-scatter without an accumulator stays on one stream beyond 16 groups, whatever the group count from
+    which the handle uses the one-launch consumer.  A counter that can never reach its group size tells: only on two
+    streams is there a bounded wait that gives up on it."""
+    ops, M, N, K, bm, W = fo.ops, 4096, 4096, 2048, 128, 2
+    algo = fo._capi.find_algo(bm, bm, swizzle=4)
+    TM, TN = M // bm, N // bm
+    T = TM * TN
+    cs = torch.tensor([T // groups] * (groups - 1) + [T - T // groups * (groups - 1)], dtype=torch.int32)
+    A, B = (torch.ones(r, K, device="cuda", dtype=torch.float16) for r in (M, N))
+    C, D = torch.empty(M, N, device="cuda", dtype=torch.float16), torch.empty(M // W, N, device="cuda", dtype=torch.float16)
+    RA = torch.arange(T, dtype=torch.int32, device="cuda").reshape(TM, TN)
+    RE = fo.layout.generate_row_mapping(M, N, bm, bm, cs.tolist(), W)
+    MM = torch.zeros(fo.layout.counter_size(groups, TM, TN), dtype=torch.int32, device="cuda")
+    ov = ops.Overlap(world=W)
+    ov.set_schedule(fused_from_groups=fused_from)
+    ov.set_wait_limit(20000)
+    MM[0] = -1000
+    ov.gemm_reducescatter_overlap(A, B, C, D, MM, RA, RE, 1, cs, cs.cuda(), algo)
+    assert ov.status() == int(two_streams)
+    ov.close()
