@@ -53,7 +53,8 @@ namespace fo_gemm_dev {
 // The MFMAs of this kernel: accumulator in the accumulation registers, tied to the destination
 // (see fo_elem::mfma for why they are assembly); `go_load` carries a direct-to-LDS load in the
 // MFMA's shadow: the M0 update in front of the MFMA, which also separates it from its use, the
-// load behind it.
+// load behind it.  (Two wait states, where a scalar out of a vector lane needs five: see dma_buf16.  None of
+// the K loop's comes from there, which a test checks in the built code.)
 template <typename Tag> struct fo_mfma256;
 #define FO_MFMA256(TAG_, OPC_)                                                                                        \
     template <> struct fo_mfma256<TAG_> {                                                                             \
@@ -213,9 +214,9 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     // load c of the loader's stage into the slot at byte offset `slot` (pipeline fill)
     auto load_chunk = [&](int c, unsigned slot) {
         if (c < 8)
-            dma_buf16(ra, a_cur, soff_a[c & 7], (wa0 ^ slot) + c * CHUNK_B);
+            dma_buf16(ra, a_cur, soff_a[c & 7], 0, (wa0 ^ slot) + c * CHUNK_B);
         else
-            dma_buf16(rb, a_cur, soff_a[c & 7], (wa0 ^ slot) + c * CHUNK_B);
+            dma_buf16(rb, a_cur, soff_a[c & 7], 0, (wa0 ^ slot) + c * CHUNK_B);
     };
     // the same riding on an MFMA (K loop)
     auto mfma_load_chunk = [&](fo_u32x4 x, fo_u32x4 y, fo_float4v &cc, int c, unsigned lds_base) {

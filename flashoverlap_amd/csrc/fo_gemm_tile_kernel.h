@@ -233,10 +233,10 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                     const unsigned b_off = !SHIFT ? a_off : (unsigned)(col + b_chunk * 8) < (unsigned)p.K ? lane_row + b_chunk * 16 : 0x80000000u;
 #pragma unroll
                     for (int u = 0; u < PB; u++)
-                        dma_buf16(rb, b_off, __builtin_amdgcn_readfirstlane(u * row_step + col * 2), wave_lds + slot + KB * A_BLK + kb * B_BLK + u * NL * 1024);
+                        dma_buf16(rb, b_off, __builtin_amdgcn_readfirstlane(u * row_step), col * 2, wave_lds + slot + KB * A_BLK + kb * B_BLK + u * NL * 1024);
 #pragma unroll
                     for (int u = 0; u < PA; u++)
-                        dma_buf16(ra, a_off, __builtin_amdgcn_readfirstlane(u * row_step + col * 2), wave_lds + slot + kb * A_BLK + u * NL * 1024);
+                        dma_buf16(ra, a_off, __builtin_amdgcn_readfirstlane(u * row_step), col * 2, wave_lds + slot + kb * A_BLK + u * NL * 1024);
                 }
             };
             __builtin_amdgcn_s_setprio(3);
