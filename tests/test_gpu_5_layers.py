@@ -128,3 +128,45 @@ def test_calls_without_the_extension_module(fo, monkeypatch, tmp_path):
     monkeypatch.setattr(fo._capi, "NATIVE_LIB", str(tmp_path / "_fo_native.so"))
     monkeypatch.setattr(fo._capi, "_native", None)
     assert all(torch.equal(a, b) for a, b in zip(results(), want))
+
+
+def test_native_calls_decline_one_wrong_argument(fo):
+    """The native calls take the right arguments (error code 0) and leave alone (None) every call with one wrong one."""
+    ops, native, M, N, K = fo.ops, fo._capi.native(), 256, 512, 64
+    algo = fo._capi.find_algo(128, 128)
+    T, TN = M // 128 * (N // 128), N // 128
+    half = lambda *s: torch.zeros(*s, device="cuda", dtype=torch.float16)
+    ints = lambda *s: torch.zeros(*s, device="cuda", dtype=torch.int32)
+    A, B, C, D, Y, w, acc = half(M, K), half(N, K), half(M, N), half(M // 2, N), half(M, N), half(N), half(M * N)
+    MM, RA, cs = ints(TN), torch.arange(T, dtype=torch.int32, device="cuda").reshape(M // 128, TN), torch.tensor([T // 2] * 2, dtype=torch.int32)
+    RE = fo.layout.generate_row_mapping(M, N, 128, 128, [T // 2] * 2, 2)
+    ov = ops.Overlap(world=2)
+    ov.set_accumulator(acc)
+    h = ov._h.value
+    off = lambda t: torch.zeros(2 * t.numel(), device=t.device, dtype=t.dtype)[::2].view(t.shape)  # every other element
+    tensor = [lambda t: None, lambda t: t.cpu() if t.is_cuda else t.cuda(), lambda t: t.float(), off]
+    small = lambda t: t.reshape(-1)[:-1]
+    number = [lambda v: None, lambda v: float(v), lambda v: 1 << 40]
+    calls = {
+        "allreduce": ([h, A, B, C, MM, RA, 1, cs, cs.cuda(), algo, False, acc],
+                      {0: number[:2], 1: tensor, 2: tensor, 3: tensor + [small], 4: tensor + [small], 5: tensor + [small],
+                       6: number + [lambda v: 3], 7: tensor, 8: tensor, 9: number + [lambda v: -1], 11: [tensor[2], small]}),
+        "allreduce_norm": ([h, A, B, C, MM, RA, RA.cpu(), 1, cs, cs.cuda(), algo, False, acc, Y, w, 1e-5],
+                           {6: tensor + [small], 13: tensor + [small], 14: tensor + [small], 15: [lambda v: 1]}),
+        "reducescatter": ([h, A, B, C, D, MM, RA, RE, 1, cs, cs.cuda(), algo, False, acc, 2],
+                          {4: tensor + [small], 7: tensor + [small], 14: number[:2] + [lambda v: 0]}),
+        "reorder_rmsnorm": ([C, Y, w, 128, 128, 1, RA, 1e-5],
+                            {0: tensor, 1: tensor + [small], 2: tensor + [small], 3: number + [lambda v: 96], 4: number, 5: number,
+                             6: tensor + [small], 7: [lambda v: 1]}),
+    }
+    for name, (right, wrong) in calls.items():
+        assert getattr(native, name)(*right) == 0, name
+        assert getattr(native, name)(*right, 0) is None and getattr(native, name)(*right[:-1]) is None
+        for i, changes in wrong.items():
+            for k, change in enumerate(changes):
+                args = list(right)
+                args[i] = change(args[i])
+                assert getattr(native, name)(*args) is None, (name, i, k)
+    torch.cuda.synchronize()
+    assert (MM == 0).all() and ov.status() == 0
+    ov.close()
