@@ -85,7 +85,7 @@ double rounds_cost(long count, long cus, int round) {
 
 // What fits the chip in one round, one tile per CU, takes the smallest tile that does: a smaller tile moves
 // more operand bytes per flop (64x64 twice those of 128x128), but it puts the operand paths of CUs to work that a larger
-// tile leaves idle, and up to that point the time of these sizes is the per-CU operand stream.  Measured over
+// tile leaves idle, and up to that point a CU's time goes into waiting for its operands.  Measured over
 // M = 128..4224, N = 1024..8192, K = 512, 2048, 8192: the rule picks the fastest tile or one within a few percent of it
 // (K = 2048, us: 128x4096 64x32 7.3, 64x64 8.1, 128x128 12.8; 512x4096 64x128 11.7, 128x128 13.7, 64x64 16.2; 1024x4096
 // 128x128 16.8, 128x256 21.8, 64x128 21.7).

@@ -4,7 +4,7 @@
 // (its reference citations hold here too), and every product is summed in the same order (ascending K,
 // 32 columns per MFMA) whatever the tile, so all shapes give the same bits.
 //
-// What bounds these sizes is not the matrix pipe but getting operands to it: a CU takes 64 bytes per clock
+// What bounds these sizes is not the matrix pipe but getting operands to it: a CU takes at most 64 bytes per clock
 // from its L2 (152 GB/s measured on one CU, 130 with all of them loading), returned in order, so that a load
 // that misses the L2 holds up the hits behind it, and a wavefront that presents loads faster than they drain
 // stands still with its MFMAs behind them.  The workgroup is therefore split in two roles, four wavefronts
@@ -17,19 +17,22 @@
 // wavefronts burst together behind the barrier and the matrix pipe waits for the LDS.
 //
 // Measured against the kernel this one replaced (loads issued by the computing wavefronts; fp16, GEMM alone,
-// operands of three buffer sets in turn): 512x4096x4096 39.1 -> 21 us, 256x8192x3584 35.5 -> 19.5,
-// 128x4096x1024 10.4 -> 4.5, 128x1024x8192 71 -> 12.5, 2048x4096x4096 62 -> 55.  512x4096x4096 with the MFMAs taken
-// out takes 18.7 us: the rest of its time is the operand stream.
+// operands of three buffer sets in turn, which the memory-side cache holds): 512x4096x4096 39.1 -> 21 us, 256x8192x3584
+// 35.5 -> 19.5, 128x4096x1024 10.4 -> 4.5, 128x1024x8192 71 -> 12.5, 2048x4096x4096 62 -> 55.
+// None of it is at a unit's limit.  512x4096x4096 on 64x128 tiles: 39 bytes a clock and CU of the 64, matrix pipe busy
+// 40 % of the clocks, LDS reads 32 %; with the MFMAs taken out 18.7 us, so what is left is round trips to the operands.
+// With operands that no cache holds (eight sets in turn) the same misses take longer: 29.6 us, 256x8192x3584 20.1 -> 30.0.
+// One round of 128x256 tiles (1024x8192x2048, 31.3 us) has the matrix pipe busy for 64 % and LDS reads for 27 %.
 //
 // SHIFT: operand rows that do not begin on 128-byte lines (K no multiple of 64, or an operand's own address).  A load of
-// eight rows x 128 bytes then touches sixteen lines instead of eight, and the operand stream, which is what bounds these
-// sizes, slows down by 30 to 40 %.  Shifted, the loaders fetch whole lines: row r's stage begins at the line that holds
-// the stage's first column, up to seven chunks early, and a computing lane whose chunk lies behind that line's end
-// takes it from the following block (all its fragments belong to rows 16 apart, so that is a constant of the lane).
-// A step thus reads its own stage and the next, which costs one stage of the ones in flight; the products and their
-// order are the same.  K = 4088 against 4096 (us): 512x4096 30.4 -> 22.6 against 22.2, 1024x4096 41.4 -> 34.5 against 32.5,
-// 128x4096 15.4 -> 13.2 against 12.3.  Tiles with room for three stages only (128x192 and larger) keep the plain
-// form: with both stages of a step awaited, nothing would be in flight.
+// eight rows x 128 bytes then touches sixteen lines instead of eight, and these sizes slow down by 30 to 40 %.  Shifted,
+// the loaders fetch whole lines: row r's stage begins at the line that holds the stage's first column, up to seven chunks
+// early, and a computing lane whose chunk lies behind that line's end takes it from the following block (all its
+// fragments belong to rows 16 apart, so that is a constant of the lane).  A step thus reads its own stage and the next,
+// which costs one stage of the ones in flight; the products and their order are the same.  K = 4088 against 4096 (us):
+// 512x4096 30.4 -> 22.6 against 22.2, 1024x4096 41.4 -> 34.5 against 32.5, 128x4096 15.4 -> 13.2 against 12.3.  (Half of
+// this form's LDS time is bank conflicts, 1152x5120x1720; the plain form has 2 to 4 %.)  Tiles with room for three
+// stages only (128x192 and larger) keep the plain form: with both stages of a step awaited, nothing would be in flight.
 //
 // MODE_ACC, the epilogue of calls that stay on one stream: what the consumer kernel would do behind the GEMM (read C and
 // the accumulator, write the accumulator) is done on the tile in LDS.  The loaders, idle by then, request the
