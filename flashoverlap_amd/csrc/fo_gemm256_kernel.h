@@ -214,9 +214,9 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     // load c of the loader's stage into the slot at byte offset `slot` (pipeline fill)
     auto load_chunk = [&](int c, unsigned slot) {
         if (c < 8)
-            dma_buf16(ra, a_cur, soff_a[c & 7], 0, (wa0 ^ slot) + c * CHUNK_B);
+            dma_buf16(ra, a_cur, soff_a[c & 7], (wa0 ^ slot) + c * CHUNK_B);
         else
-            dma_buf16(rb, a_cur, soff_a[c & 7], 0, (wa0 ^ slot) + c * CHUNK_B);
+            dma_buf16(rb, a_cur, soff_a[c & 7], (wa0 ^ slot) + c * CHUNK_B);
     };
     // the same riding on an MFMA (K loop)
     auto mfma_load_chunk = [&](fo_u32x4 x, fo_u32x4 y, fo_float4v &cc, int c, unsigned lds_base) {

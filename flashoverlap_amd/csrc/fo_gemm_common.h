@@ -190,13 +190,21 @@ __device__ __forceinline__ fo_srd_t fo_make_srd(const void *base, unsigned bytes
     return r;
 }
 
-// 16 bytes per lane, global -> LDS: address = descriptor base + row_off + col_off + voff (out of range: zeros),
-// LDS address = lds_addr + lane * 16 (through M0, which wants a wait state between its write and its use: the addition).
+// 16 bytes per lane, global -> LDS: address = descriptor base + soff + voff (out of range: zeros),
+// LDS address = lds_addr + lane * 16 (through M0; the s_nop is the wait state between an M0 write and its use).
 // A vector-memory instruction that reads a scalar register has to stay five wait states behind a vector instruction that
-// wrote it.  The compiler does not look into this statement and returns spilled scalars (v_readlane) right in front of it;
-// the offsets therefore pass through the scalar addition, which needs no distance (five wait states instead: 128x256 tiles
-// 1 % slower).  The descriptor is not protected: no build so far has it in a vector lane, and a test looks for that.
-__device__ __forceinline__ void dma_buf16(fo_srd_t srd, unsigned voff, unsigned row_off, unsigned col_off, unsigned lds_addr) {
+// wrote it, and the compiler, which does not look into this statement, may return a spilled scalar (v_readlane) right in
+// front of it.  Where it does, dma_buf16_sum takes its place; a test looks for such pairs in the built code.
+__device__ __forceinline__ void dma_buf16(fo_srd_t srd, unsigned voff, unsigned soff, unsigned lds_addr) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds_addr), "v"(voff), "s"(srd), "s"(soff)
+                 : "memory");
+}
+// The same with soff = row_off + col_off, added here: the load reads a scalar that a scalar instruction wrote, which needs
+// no distance.  (As fast on the tiles that use it; five wait states instead cost 128x256 tiles 1 %.  On smaller tiles,
+// which keep their offsets in scalar registers, this form is up to 4 % slower: 384x2304x4760 in 64x64 tiles, 22.3 -> 23.1.)
+__device__ __forceinline__ void dma_buf16_sum(fo_srd_t srd, unsigned voff, unsigned row_off, unsigned col_off, unsigned lds_addr) {
     unsigned soff;
     asm volatile("s_mov_b32 m0, %1\n\ts_add_u32 %0, %4, %5\n\tbuffer_load_dwordx4 %2, %3, %0 offen lds"
                  : "=&s"(soff)

@@ -226,6 +226,13 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             const fo_srd_t ra = fo_make_srd(a0 - LEAD / 2, (unsigned)TM * p.lda * 2 + LEAD);
             const fo_srd_t rb = fo_make_srd(b0 - LEAD / 2, (unsigned)TN * p.ldb * 2 + LEAD);
             const unsigned wave_lds = lds0 + wave * 1024;
+            // With twelve loads a stage the row offsets no longer fit the scalar registers.
+            auto load = [&](fo_srd_t srd, unsigned voff, unsigned row_off, unsigned col_off, unsigned lds_addr) __attribute__((always_inline)) {
+                if constexpr (P >= 12)
+                    dma_buf16_sum(srd, voff, __builtin_amdgcn_readfirstlane(row_off), col_off, lds_addr);
+                else
+                    dma_buf16(srd, voff, __builtin_amdgcn_readfirstlane(row_off + col_off), lds_addr);
+            };
             auto request = [&](int kt, unsigned slot_v) __attribute__((always_inline)) {
                 const unsigned slot = __builtin_amdgcn_readfirstlane(slot_v);  // uniform by construction; said so for the assembly's operands
 #pragma unroll
@@ -236,10 +243,10 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                     const unsigned b_off = !SHIFT ? a_off : (unsigned)(col + b_chunk * 8) < (unsigned)p.K ? lane_row + b_chunk * 16 : 0x80000000u;
 #pragma unroll
                     for (int u = 0; u < PB; u++)
-                        dma_buf16(rb, b_off, __builtin_amdgcn_readfirstlane(u * row_step), col * 2, wave_lds + slot + KB * A_BLK + kb * B_BLK + u * NL * 1024);
+                        load(rb, b_off, u * row_step, col * 2, wave_lds + slot + KB * A_BLK + kb * B_BLK + u * NL * 1024);
 #pragma unroll
                     for (int u = 0; u < PA; u++)
-                        dma_buf16(ra, a_off, __builtin_amdgcn_readfirstlane(u * row_step), col * 2, wave_lds + slot + kb * A_BLK + u * NL * 1024);
+                        load(ra, a_off, u * row_step, col * 2, wave_lds + slot + kb * A_BLK + u * NL * 1024);
                 }
             };
             __builtin_amdgcn_s_setprio(3);
