@@ -34,14 +34,14 @@ enum {
 // GEMM cost more than such a GEMM can hide (4096x4096x512 with 256 groups:
 // 71 us overlapped, 44 us in stream).
 //
-// kRsEpilogueBelowFlop, kFewCopies: see fo_overlap_gemm_reducescatter.  Neither is a threshold of a handle.
+// kRsEpilogueBelowFlop, kFewCopies: see fo_overlap_gemm_reducescatter.  They are no thresholds of a handle.
 //
 // kGemmFlopPerNs: what a GEMM is expected to sustain, for sizing the pause
 // between polls only.
 constexpr int kFusedFromGroups = 16;
 constexpr double kInStreamBelowFlop = 6.4e10;
 constexpr double kRsEpilogueBelowFlop = 5e11;
-constexpr int kFewCopies = 16;
+constexpr int kFewCopies = 16, kFewCopiesOfShort = 6;
 constexpr double kGemmFlopPerNs = 1.2e6;
 
 }  // namespace
@@ -643,14 +643,16 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     const bool own_in_consumer = D && h->acc && W > 1;
     const bool fits = !h->acc || aligned(C, h->acc, own_in_consumer ? D : nullptr);
     const bool in_any_case = in_stream(h, M, N, K, only_copies, monitor != 0, false, fits);
-    // A large ragged call leaves the rest to launches behind the GEMM (one consumer launch for all groups, or a few copies):
-    // the epilogue holds up the next tile's loads.  By the epilogue and by launches, us, eight ranks and an accumulator:
+    // A ragged call may leave the rest to launches behind the GEMM, one consumer launch for all groups or a copy for each:
+    // the epilogue holds up the next tile's loads.  By the epilogue and by launches, us, eight ranks: with an accumulator
     // 8192x8064x7168 803 and 751, 8064x8064x4096 494 and 470 (two ranks 508 and 509), 4224x7168x3584 194 and 193,
-    // 8064x8192x1024 183 and 200; sixteen copies: 8192x8064x7168 737 and 693, 4224x7168x3584 182 and 192.
-    const bool few_launches = h->acc ? W > 1 : G <= kFewCopies;
-    const bool ragged = (M % 256 || N % 256) && (by_epilogue || few_launches);
+    // 8064x8192x1024 183 and 200; copies, 6400x2176x4648: four 136 and 126, ten 132 and 130, sixteen 133 and 142;
+    // 3456x7424x3328: six 170 and 165, ten 170 and 174; 8192x8064x7168: sixteen 737 and 693.
+    const bool large = 2.0 * M * N * K >= kRsEpilogueBelowFlop;
+    const bool by_launches = h->acc ? W > 1 && large : G <= (large ? kFewCopies : kFewCopiesOfShort);
+    const bool ragged = (M % 256 || N % 256) && (by_epilogue || by_launches || (h->acc && W > 1));
     const bool same_stream = in_any_case || in_stream(h, M, N, K, only_copies, monitor != 0, ragged, fits);
-    const bool in_epilogue = by_epilogue && (in_any_case || !few_launches || 2.0 * M * N * K < kRsEpilogueBelowFlop);
+    const bool in_epilogue = by_epilogue && (in_any_case || !by_launches);
     const int fused = same_stream ? 0 : fused_grid(h, G);
     fo_stream_t cstream = same_stream ? h->gemm_stream : h->comm_stream;
     int32_t wave = 0;

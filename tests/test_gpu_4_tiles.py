@@ -334,9 +334,10 @@ def test_counted_launch_walks_the_reported_order(fo, bm, bn, M, N):
 @pytest.mark.parametrize("M,N,K", [(4224, 4352, 2048), (8064, 8064, 4096)])  # 7.5e10 and 5.3e11 flop
 @pytest.mark.parametrize("with_acc", [True, False])
 @pytest.mark.parametrize("W", [1, 4])
-def test_reduce_scatter_that_256_does_not_divide(fo, M, N, K, with_acc, W):
-    """Both sides of the size from which such a call leaves sums and copies to launches behind the GEMM."""
-    ops, bm, groups = fo.ops, 128, 5
+@pytest.mark.parametrize("groups", [5, 9])
+def test_reduce_scatter_that_256_does_not_divide(fo, M, N, K, with_acc, W, groups):
+    """Both sides of the size and the group count from which such a call leaves sums and copies to launches behind the GEMM."""
+    ops, bm = fo.ops, 128
     algo = fo._capi.find_algo(bm, 128, swizzle=4)
     TM, TN = M // bm, N // 128
     T = TM * TN
