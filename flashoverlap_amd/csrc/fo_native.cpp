@@ -14,7 +14,6 @@
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/record_function.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
-#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/Exceptions.h>
@@ -230,10 +229,11 @@ PyObject *reducescatter(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
 }
 
 // Whether somebody follows the operators that run (a profiler or tracer, a function or dispatch mode, a transform): the
-// layers then go through the registered ones.
+// layers then go through the registered ones.  Dispatch modes, tracers and transforms put keys of theirs among the ones
+// that every dispatch includes.
 bool followed() {
-    return at::hasCallbacks() || at::impl::torch_function_mode_enabled() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
-           !(c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty();
+    return !(c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty() || at::hasCallbacks() ||
+           at::impl::torch_function_mode_enabled();
 }
 
 bool norm_fits(const at::Tensor &X, const at::Tensor &Wt, int BM, int BN, const at::Tensor &RA) {

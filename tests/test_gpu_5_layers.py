@@ -1,6 +1,7 @@
 """GPU tests of the layers' native call path: what it enqueues, refuses and leaves to the registered operators."""
 import pytest
 import torch
+import torch.utils._python_dispatch  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
@@ -65,6 +66,16 @@ class Seen(torch.overrides.TorchFunctionMode):
         return func(*args, **(kwargs or {}))
 
 
+class Dispatched(torch.utils._python_dispatch.TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.names.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
 def test_the_norm_layer_keeps_classes_and_is_seen(fo):
     """A subclass goes through torch.empty_like and the registered operator, and so does every call that a mode or the
     profiler follows; the values are those of the native call."""
@@ -80,10 +91,13 @@ def test_the_norm_layer_keeps_classes_and_is_seen(fo):
         with Seen() as seen:
             followed = norm(x)
         assert any("reorder_rmsnorm_eps" in name for name in seen.names), seen.names
+        with Dispatched() as dispatched:
+            seen_below = norm(x)
+        assert any("empty_like" in name for name in dispatched.names)  # the composite operator itself is above such modes
         with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
             profiled = norm(x)
         assert any("reorder_rmsnorm_eps" in event.key for event in prof.key_averages())
-    for y in (tagged.as_subclass(torch.Tensor), followed, profiled):
+    for y in (tagged.as_subclass(torch.Tensor), followed, seen_below, profiled):
         assert torch.equal(y, want)
 
 
