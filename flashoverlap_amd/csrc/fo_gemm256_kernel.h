@@ -20,16 +20,32 @@
 // step that lie beyond K are requested out of its range: the hardware writes
 // zeros for them, nothing outside A or B is ever addressed.
 //
-// A K step has sixteen rows (one A fragment x eight B fragments) and two
-// meetings of the workgroup:
+// A K step is four strips, each two A blocks x eight B blocks x two k-steps, and
+// each strip four rows of eight MFMAs.  The order inside a strip is chosen for
+// energy, because large products run at this part's power limit: both k-steps of
+// an accumulator block follow one another (the sum then stays in the matrix
+// pipe's own path instead of going through the register file), and from one
+// block to the next only one of the two operands changes.  MFMAs alone, random
+// operands, at the power limit: 8.60 ns per MFMA with the k-steps 64 MFMAs apart
+// and one A fragment x eight B fragments in a row, 8.14 in this order (bf16 8.05
+// -> 7.74); 7.94 with four k-steps in a chain and 7.66 with eight, for which LDS
+// and registers do not hold the operands.  This kernel: 8192^3 766 -> 749 us,
+// 8192x4096x4096 205.5 -> 199.2, 4096x4096x512 20.7 -> 20.0, the same bits.  (With
+// the two A blocks in the same order for every B block, so that A changes each
+// time, 761.)
+//
+// Two meetings of the workgroup per K step:
 //   FREE (behind row 9): every wavefront has fetched its last fragment of the
-//     step's slot (the A ring runs seven rows ahead; the second k-step's B
-//     fragments are fetched in rows 0-3), so the slot may be refilled.  The
-//     sixteen loads of the stage two steps ahead follow, two per row in rows
-//     10-13, then one per row until row 5 of the next step.
+//     step's slot (B is complete by row 1, a strip's A fragments are fetched in
+//     the strip before it, the last ones in row 8), so the slot may be refilled.
+//     The sixteen loads of the stage two steps ahead follow, two per row in rows
+//     10-12, then one per row until row 6 of the next step (two in row 13 as well:
+//     8192x4096x4096 200.4 us; that row has six fragment fetches).
 //   PUB (behind row 12): the other slot's loads, requested one step earlier,
 //     have landed (vmcnt) in every wavefront; rows 13-15 fetch the next step's
-//     first fragments from it.
+//     first A fragments from it and the B fragments, each into the registers of the
+//     block that the last strip has just finished with; the last of them follow in
+//     rows 0 and 1.
 // With one meeting for both, a stage's loads would have to leave within a few
 // rows (the load path of a CU delivers a stage in about half a K step, and a
 // wavefront that presents loads faster than they drain stalls with its MFMAs
@@ -76,7 +92,7 @@ FO_MFMA256(fo_bf16_tag, "bf16")
 #undef FO_MFMA256
 
 // Direct-to-LDS loads per wavefront in the rows behind FREE (rows 10, 11, ... wrapping into the next step).
-constexpr int kLoadRows256[] = {2, 2, 2, 2, 1, 1, 1, 1, 1, 1, 1, 1};
+constexpr int kLoadRows256[] = {2, 2, 2, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1};
 constexpr int kLoadSpan256 = sizeof(kLoadRows256) / sizeof(int);
 constexpr int loads_in_row256(int d) { return d >= 0 && d < kLoadSpan256 ? kLoadRows256[d] : 0; }
 constexpr int loads_before_row256(int d) {
@@ -93,9 +109,9 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     typedef fo_mfma256<Tag> X;
     constexpr bool ACC = MODE == MODE_ACC || MODE == MODE_RS, COUNTS = MODE == MODE_SIGNAL || MODE == MODE_SCATTER;
     constexpr bool MAPPED = MODE == MODE_SCATTER || MODE == MODE_RS;
-    constexpr int MT = 256, BK = 64, F = 8, ROWS = 16, AHEAD = 7, ARING = AHEAD + 1;
-    constexpr int FREE = ROWS - AHEAD;  // row behind whose MFMAs the step's slot is given up
-    constexpr int PUB = 12;             // row behind whose MFMAs the next step's slot is published
+    constexpr int MT = 256, BK = 64, F = 8, ROWS = 16;
+    constexpr int FREE = 9;   // row behind whose MFMAs the step's slot is given up
+    constexpr int PUB = 12;   // row behind whose MFMAs the next step's slot is published
     constexpr unsigned SLOT_B = 65536, BPART_B = 32768, BLOCK_B = 2048, KSTEP_X = 64, CHUNK_B = 4096;
     constexpr int PITCH = 128 + 8, CPR = 16, RPP = 4;
     constexpr unsigned STRIP_B = 2 * SLOT_B;
@@ -104,7 +120,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     static_assert(loads_before_row256(kLoadSpan256) == 16, "a stage is sixteen loads per wavefront");
     static_assert(FREE + kLoadSpan256 - ROWS < FREE && PUB > FREE && PUB <= 13, "load rows lie between two FREE meetings");
     // YOUNG is exact: between a FREE meeting (row 9) and the PUB meeting of the same step (row 12) rows 10-12 issue
-    // loads_in_row256(0..2) loads and nothing else that counts in vmcnt; a tile's stores and the loads of rows 0-5 of
+    // loads_in_row256(0..2) loads and nothing else that counts in vmcnt; a tile's stores and the loads of rows 0-6 of
     // its successor's first step are older than those.  Further vector-memory instructions in that stretch would
     // only make the PUB wait stricter.  The wait relies on vmcnt retiring loads and stores in issue order (one
     // counter for both on this part); a part with a counter of its own for stores needs a wait on that one as well.
@@ -360,12 +376,12 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     int owed = 0;                    // PUB meetings until that signal may be sent
 
     fo_float4v acc[F][F];
-    fo_u32x4 af[ARING], bf[2][F];
-    auto load_a = [&](int slot, unsigned base, int kk, int i) {
-        af[slot] = *reinterpret_cast<lds16_t>((base ^ (kk * KSTEP_X)) + i * BLOCK_B);
+    fo_u32x4 af[2][2][2], bf[2][F];
+    auto load_a = [&](int buf, unsigned base, int i, int kk) {
+        af[buf][i % 2][kk] = *reinterpret_cast<lds16_t>((base ^ (kk * KSTEP_X)) + i * BLOCK_B);
     };
-    auto load_b = [&](int buf, unsigned base, int kk, int j) {
-        bf[buf][j] = *reinterpret_cast<lds16_t>((base ^ (kk * KSTEP_X)) + j * BLOCK_B);
+    auto load_b = [&](unsigned base, int j, int kk) {
+        bf[kk][j] = *reinterpret_cast<lds16_t>((base ^ (kk * KSTEP_X)) + j * BLOCK_B);
     };
 
     // ---- pipeline fill: stage 0 -> slot 0, stage 1 -> slot 1; the loader then stands at stage 1
@@ -380,9 +396,9 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int j = 0; j < F; j++) load_b(0, lb0, 0, j);
+    for (int q = 0; q < 4; q++) load_a(0, la0, q / 2, q % 2);
 #pragma unroll
-    for (int i = 0; i < AHEAD; i++) load_a(i, la0, 0, i);
+    for (int q = 0; q < 10; q++) load_b(lb0, q / 2, q % 2);
     sum_groups();  // the group sizes arrived before stage 0 did (requested earlier, vmcnt retires in issue order)
 
     int tile = blockIdx.x;
@@ -408,7 +424,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
 
         // A tile whose predecessor's signal is still owed leaves the K loop after its first step, sends the signal and
         // re-enters: that step's PUB meeting has waited for the predecessor's stores in every wavefront (part of the
-        // stage's loads was requested behind them, rows 0-5, and vmcnt retires in issue order), with the meeting's
+        // stage's loads was requested behind them, rows 0-6, and vmcnt retires in issue order), with the meeting's
         // barrier behind the wait.  The test inside the step (one scalar compare and branch per K step, after the PUB
         // meeting) cost the large square 4 us.
         int kt = 0;
@@ -422,38 +438,30 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             const unsigned lds_cur = __builtin_amdgcn_readfirstlane(wa0 ^ slot_b), lds_prev = lds_cur ^ SLOT_B;
 #pragma unroll
             for (int r = 0; r < ROWS; r++) {
-                const int kk = r / F, i = r % F;
+                const int strip = r / 4, next_a = (strip + 1) % 2;
                 // The row's LDS fetches in issue order; executes number t (none for t < 0), returns how many there are.
-                //   up to FREE: the A fragment of row r + AHEAD and, in rows 0-3, the second k-step's B fragments;
-                //   behind PUB: the next step's first fragments (the A rows whose ring entry has fallen free: all
-                //   of them so far in row PUB + 1, then one per row; its first k-step's B fragments, four per row).
                 auto fetches = [&](int t) {
                     int n = 0;
-                    const int q = r + AHEAD;  // A row the ring takes in behind row r, counted from this step's row 0
-                    if (q < ROWS) {
-                        if (t == n) load_a(q % ARING, la_, q / F, q % F);
+                    auto fetch_a = [&](unsigned base, int i, int kk) {
+                        if (t == n) load_a(next_a, base, i, kk);
                         n++;
-                    } else if (r > PUB) {
+                    };
+                    auto fetch_b = [&](unsigned base, int j) {
 #pragma unroll
-                        for (int qq = ROWS; qq < ROWS + ARING; qq++) {
-                            if (qq <= q && (r == PUB + 1 || qq == q)) {
-                                if (t == n) load_a(qq % ARING, lan, 0, qq - ROWS);
-                                n++;
-                            }
-                        }
-                    }
-                    if (r < 4) {
-                        if (t == n) load_b(1, lb_, 1, 2 * r);
-                        if (t == n + 1) load_b(1, lb_, 1, 2 * r + 1);
-                        n += 2;
-                    }
-                    if (r > PUB && r - PUB <= 2) {
-#pragma unroll
-                        for (int j = 0; j < 4; j++) {
-                            if (t == n) load_b(0, lbn, 0, (r - PUB - 1) * 4 + j);
+                        for (int kk = 0; kk < 2; kk++) {
+                            if (t == n) load_b(base, j, kk);
                             n++;
                         }
-                    }
+                    };
+                    if (r == 0) { fetch_b(lb_, 5); fetch_b(lb_, 6); }
+                    if (r == 1) { fetch_b(lb_, 7); fetch_a(la_, 2, 0); fetch_a(la_, 2, 1); }
+                    if (r == 2) { fetch_a(la_, 3, 0); fetch_a(la_, 3, 1); }
+                    if (r == 4) { fetch_a(la_, 4, 0); fetch_a(la_, 4, 1); }
+                    if (r == 5) { fetch_a(la_, 5, 0); fetch_a(la_, 5, 1); }
+                    if (r == 8) { fetch_a(la_, 6, 0); fetch_a(la_, 6, 1); fetch_a(la_, 7, 0); fetch_a(la_, 7, 1); }
+                    if (r == 13) { fetch_a(lan, 0, 0); fetch_a(lan, 0, 1); fetch_b(lbn, 0); fetch_a(lan, 1, 0); fetch_a(lan, 1, 1); }
+                    if (r == 14) { fetch_b(lbn, 1); fetch_b(lbn, 2); }
+                    if (r == 15) { fetch_b(lbn, 3); fetch_b(lbn, 4); }
                     return n;
                 };
                 const int nops = fetches(-1);
@@ -461,19 +469,20 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                 const int d = r > FREE ? r - FREE - 1 : r + ROWS - FREE - 1;  // rows since the one behind FREE
                 const int dfirst = loads_before_row256(d);
 #pragma unroll
-                for (int j = 0; j < F; j++) {
+                for (int m = 0; m < F; m++) {
+                    const int j = r % 4 * 2 + m / 4, h = (m / 2 % 2) ^ (j % 2), i = strip * 2 + h, kk = m % 2;
                     int dc = -1;
 #pragma unroll
                     for (int c = 0; c < 2; c++)
-                        if (c < loads_in_row256(d) && j == 1 + 4 * c) dc = c;
+                        if (c < loads_in_row256(d) && m == 1 + 4 * c) dc = c;
                     if (dc >= 0)
-                        mfma_load_chunk(bf[kk][j], af[r % ARING], acc[i][j], dfirst + dc, r > FREE ? lds_cur : lds_prev);
+                        mfma_load_chunk(bf[kk][j], af[strip % 2][h][kk], acc[i][j], dfirst + dc, r > FREE ? lds_cur : lds_prev);
                     else
-                        X::go(bf[kk][j], af[r % ARING], acc[i][j]);
+                        X::go(bf[kk][j], af[strip % 2][h][kk], acc[i][j]);
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int t = 0; t < 16; t++)
-                        if (t >= j * nops / F && t < (j + 1) * nops / F) fetches(t);
+                        if (t >= m * nops / F && t < (m + 1) * nops / F) fetches(t);
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 if (r == FREE) {
@@ -485,7 +494,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                 if (r == PUB) {
                     // The stage the next step reads has landed; younger and allowed in flight: this step's YOUNG loads.
                     // In a tile's first step the wait also covers the previous tile's stores: part of the stage's
-                    // loads was requested behind them (rows 0-5), and vmcnt retires in issue order.
+                    // loads was requested behind them (rows 0-6), and vmcnt retires in issue order.
                     wait_vmcnt<YOUNG>();
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" ::: "memory");
