@@ -30,8 +30,10 @@
 // early, and a computing lane whose chunk lies behind that line's end takes it from the following block (all its
 // fragments belong to rows 16 apart, so that is a constant of the lane).  A step thus reads its own stage and the next,
 // which costs one stage of the ones in flight; the products and their order are the same.  K = 4088 against 4096 (us):
-// 512x4096 30.4 -> 22.6 against 22.2, 1024x4096 41.4 -> 34.5 against 32.5, 128x4096 15.4 -> 13.2 against 12.3.  (Half of
-// this form's LDS time is bank conflicts, 1152x5120x1720; the plain form has 2 to 4 %.)  Tiles with room for three
+// 512x4096 30.4 -> 22.6 against 22.2, 1024x4096 41.4 -> 34.5 against 32.5, 128x4096 15.4 -> 13.2 against 12.3.  Both forms
+// permute a row's chunks by exclusive or: a fetch takes lanes of two chunk columns in one pass, and with the chunks rotated
+// instead half of this form's LDS time was bank conflicts (exclusive or against rotated: 1152x5120x1720 27.8 -> 26.8 us,
+// 512x4096x4088 23.3 -> 22.6, 384x4096x4088 39.0 -> 36.9, 128x4096x4088 12.7 -> 12.3).  Tiles with room for three
 // stages only (128x192 and larger) keep the plain form: with both stages of a step awaited, nothing would be in flight.
 //
 // MODE_ACC, the epilogue of calls that stay on one stream: what the consumer kernel would do behind the GEMM (read C and
@@ -213,13 +215,14 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
         if (loader) {
             // Load u of a 64-column block brings rows (u * NL + wave) * 8 + lane / 8 of an operand, 128 bytes each; LDS
             // slot `lane` of the 1 KiB block is (row lane / 8, chunk lane % 8) and receives chunk phys ^ key(row).
-            // Shifted, slot `lane` receives chunk (phys - key(row) + shift(row)) % 8 of the row's aligned line: what lies
-            // before the row's first column or behind its last is requested out of range (zeros).
+            // Shifted, slot `lane` receives chunk ((phys ^ key(row)) + shift(row)) % 8 of the row's aligned line, so that a
+            // column's chunk lies where it would unshifted; what lies before the row's first column or behind its last is
+            // requested out of range (zeros).
             const int lrow = lane >> 3, lkey = ((wave * 8 + lrow) >> 1) & 7;
             const uint16_t *a0 = p.A + (size_t)m0 * p.lda, *b0 = p.B + (size_t)n0 * p.ldb;
             const int a_shift = SHIFT ? row_shift(a0, p.lda, lrow) : 0, b_shift = SHIFT ? row_shift(b0, p.ldb, lrow) : 0;
-            const int a_chunk = SHIFT ? ((lane - lkey + a_shift) & 7) - a_shift : (lane & 7) ^ lkey;
-            const int b_chunk = SHIFT ? ((lane - lkey + b_shift) & 7) - b_shift : (lane & 7) ^ lkey;
+            const int a_chunk = SHIFT ? ((((lane & 7) ^ lkey) + a_shift) & 7) - a_shift : (lane & 7) ^ lkey;
+            const int b_chunk = SHIFT ? ((((lane & 7) ^ lkey) + b_shift) & 7) - b_shift : (lane & 7) ^ lkey;
             constexpr int LEAD = SHIFT ? 128 : 0;  // the range starts a line early: no lane's offset is negative
             const unsigned lane_row = (unsigned)((wave * 8 + lrow) * p.lda * 2 + LEAD);
             const unsigned row_step = (unsigned)(NL * 8 * p.lda * 2);
@@ -333,9 +336,8 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             constexpr int FL = LONG_B ? FN : FM, FS = LONG_B ? FM : FN;
             constexpr unsigned L_BLK = LONG_B ? B_BLK : A_BLK, S_BLK = LONG_B ? A_BLK : B_BLK;
             const int frow = lane & 15, fk = lane >> 4, key = (frow >> 1) & 7;
-            const int phys = SHIFT ? (fk + key) & 7 : fk ^ key;  // chunk fk; four further on is ^ 4 in both
-            const unsigned la = lds0 + (unsigned)((wm * WTM + frow) * 8 + phys) * 16;
-            const unsigned lb = lds0 + KB * A_BLK + (unsigned)((wn * WTN + frow) * 8 + phys) * 16;
+            const unsigned la = lds0 + (unsigned)((wm * WTM + frow) * 8 + (fk ^ key)) * 16;
+            const unsigned lb = lds0 + KB * A_BLK + (unsigned)((wn * WTN + frow) * 8 + (fk ^ key)) * 16;
             const unsigned l_lds = LONG_B ? lb : la, s_lds = LONG_B ? la : lb;
             typedef const __attribute__((address_space(3))) frag *lds_frag_t;
             // Two sets of short fragments take turns.  Long ones: two sets as well, or, from four on, one set whose
