@@ -10,11 +10,21 @@
 // stands still with its MFMAs behind them.  The workgroup is therefore split in two roles, four wavefronts
 // each: loaders, which do nothing but move operand stages HBM/L2 -> LDS (buffer_load_dwordx4 ... lds) up to
 // S - 1 stages ahead and may stand still as long as they like, and computing wavefronts, which touch nothing
-// but LDS and the matrix pipe.  One barrier per K step (BK columns), placed near the start of the step's last MFMA
-// group: it says that the step's slot has been read by everyone (the loaders refill it next) and that the
-// next stage has landed, so its first fragments are fetched behind that last group's MFMAs.  Fragment
-// fetches are spread between MFMAs (k_step below): issued as one burst in front of them, all
-// wavefronts burst together behind the barrier and the matrix pipe waits for the LDS.
+// but LDS and the matrix pipe.  One barrier per K step (BK columns) says that the step's slot has been read by everyone
+// (the loaders refill it next) and that the next stage has landed.
+//
+// The MFMAs of a step run in strips of two long fragments (those of the operand of which a wavefront holds more) by all
+// short ones, all k-steps of an accumulator block in a row and one operand changing from block to block: the order that
+// costs least energy (fo_gemm256_kernel.h; these sizes run at 1.65 to 1.9 GHz of 2.4 with random operands and at 2.37 with
+// zeros).  Fragment fetches are spread between the MFMAs: issued as one burst, all wavefronts burst together behind the
+// barrier and the matrix pipe waits for the LDS.  Two ways to hold fragments:
+//   AHEAD: the whole next stage in a second set of registers, fetched from the middle of the step on.  Small wavefront
+//     tiles, whose step is too short to hide a fetch in, and the shifted form, whose fetches take longer.
+//   otherwise long fragments a strip ahead; a short one is replaced once the last strip is done with it.
+// In us against one set of fragments per k-step, fetched a k-step ahead (fp16, GEMM alone): AHEAD 128x1024x8192 15.8 ->
+// 12.8, 128x4096x1024 5.4 -> 5.2, 128x4096x4088 12.7 -> 11.7, 384x4096x4088 37.7 -> 30.6, 1152x5120x1720 26.4 -> 25.1;
+// strips 1024x4096x2048 18.3 -> 17.8, 1536x3328x4096 37.1 -> 36.6, 1536x4096x4096 69.7 -> 68.0, 1024x8192x2048 30.7 -> 29.9,
+// 512x4096x4096 the same.  The other way round: 1024x4096x4088 in strips 34.2 against 33.4, 128x160 tiles hold no second set.
 //
 // Measured against the kernel this one replaced (loads issued by the computing wavefronts; fp16, GEMM alone,
 // operands of three buffer sets in turn, which the memory-side cache holds): 512x4096x4096 39.1 -> 21 us, 256x8192x3584
@@ -104,7 +114,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
     __shared__ int32_t rs_map[MODE == MODE_RS ? 256 : 1];  // and their rows in the accumulator
     const unsigned lds0 = (unsigned)(uintptr_t)FO_LDS_PTR(smem);
     uint16_t *stage = reinterpret_cast<uint16_t *>(smem);  // the output tile, once the K loop is done
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int tid = threadIdx.x;
     const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool loader = wave_id < NL;
     const int wave = loader ? wave_id : wave_id - NL;
@@ -119,6 +129,10 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
     const cptr_t RAc = (cptr_t)(uintptr_t)p.RA;
 
     for (int tile = blockIdx.x; tile < p.count; tile += gridDim.x) {
+        // What is computed from the lane is computed for each tile: kept from one to the next, the group search's and the
+        // loaders' part of it alone took twenty registers through the K loop.
+        int lane = tid & 63;
+        asm volatile("" : "+v"(lane));
         int pm, pn;
         fo_unit_to_tile(tile, p.first, p.sub_m, p.sub_n, p.grid_m, p.grid_n, p.panel, p.xcd_remap, &pm, &pn);
         pm = __builtin_amdgcn_readfirstlane(pm);
@@ -340,12 +354,12 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             const unsigned lb = lds0 + KB * A_BLK + (unsigned)((wn * WTN + frow) * 8 + (fk ^ key)) * 16;
             const unsigned l_lds = LONG_B ? lb : la, s_lds = LONG_B ? la : lb;
             typedef const __attribute__((address_space(3))) frag *lds_frag_t;
-            // Two sets of short fragments take turns.  Long ones: two sets as well, or, from four on, one set whose
-            // members are replaced right behind the row that used them (two full sets beside 128 accumulators would
-            // leave no room for a consumer's wavefront on the SIMD).
-            constexpr bool RING = FL >= 4;
-            constexpr int MEET = RING ? 1 : 0;  // the barrier stands in front of this row of the step's last k-step
-            frag lf[RING ? 1 : 2][FL], sf[2][FS];
+            constexpr int NS = (FL + 1) / 2;  // strips; an odd one out is a strip of its own, the first
+            // (Up to 224 registers in all, and a consumer's wavefront still fits on the SIMD beside this kernel's two.)
+            constexpr bool AHEAD = (SHIFT || FL < 4) && (2 * KK * (FL + FS) + FL * FS) * 4 <= 192;
+            static_assert(AHEAD || (FL >= 4 && FS >= 2), "a strip in front of the last one fetches the last short fragment");
+            constexpr int LSETS = AHEAD ? 2 : NS % 2 ? NS : 2;  // AHEAD: one per stage, else one per strip
+            frag lf[LSETS][AHEAD ? FL : 2][KK], sf[AHEAD ? 2 : 1][FS][KK];
             // Shifted: column chunk c of a 64-column block lies c + shift chunks behind the start of the row's line, that is
             // in the following block from 8 on (all rows of a lane have the same shift: they are 16 apart).
             int l_shift = 0, s_shift = 0;
@@ -358,60 +372,108 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                 const unsigned here = slot + (kk >> 1) * blk, behind = (kk >> 1) + 1 < KB ? here + blk : next;
                 return SHIFT && shift + (kk & 1) * 4 >= 8 ? behind : here;
             };
-            auto fetch_l = [&](int kk, unsigned slot, unsigned next, int i) __attribute__((always_inline)) {
+            // Fragment i, k-step kk of the stage in `slot` (and, shifted, of the one in `next`).
+            auto fetch_l = [&](frag &to, int i, int kk, unsigned slot, unsigned next) __attribute__((always_inline)) {
                 const unsigned at = (l_lds + block_of(kk, slot, next, L_BLK, l_shift)) ^ ((kk & 1) * 64);
-                lf[RING ? 0 : kk & 1][i] = *(lds_frag_t)(uintptr_t)(at + i * 2048);
+                to = *(lds_frag_t)(uintptr_t)(at + i * 2048);
             };
-            auto fetch_s = [&](int kk, unsigned slot, unsigned next, int j) __attribute__((always_inline)) {
+            auto fetch_s = [&](frag &to, int j, int kk, unsigned slot, unsigned next) __attribute__((always_inline)) {
                 const unsigned at = (s_lds + block_of(kk, slot, next, S_BLK, s_shift)) ^ ((kk & 1) * 64);
-                sf[kk & 1][j] = *(lds_frag_t)(uintptr_t)(at + j * 2048);
+                to = *(lds_frag_t)(uintptr_t)(at + j * 2048);
             };
             auto behind_slot = [&](unsigned slot) __attribute__((always_inline)) { return slot + STAGE == S * STAGE ? 0 : slot + STAGE; };
-            // k-step kk with the fetches of the next one (the first of the next slot behind the last) spread over its
-            // rows from `from` on, the earlier ones a little denser: what is fetched last is needed soon.
-            auto k_step = [&](int kk, unsigned slot, unsigned next, unsigned after) __attribute__((always_inline)) {
-                const bool last = kk == KK - 1;
-                const int from = last ? MEET : 0;
-                const int nkk = last ? 0 : kk + 1;
-                int l_done = 0, s_done = 0;
+            auto meet = [&]() __attribute__((always_inline)) {
+                __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wavefront's fetches from the slot have returned
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            // A step's accumulator blocks in their order.
+            constexpr int NB = FL * FS, LEAD_B = FL % 2 * FS;  // blocks, of those in a first strip of one
+            struct block { int i, j; };
+            auto block_at = [](int c) constexpr {
+                if (c < LEAD_B) return block{0, c};
+                const int e = c - LEAD_B, j = e % (2 * FS) / 2;
+                return block{FL % 2 + e / (2 * FS) * 2 + ((e & 1) ^ (j & 1)), j};
+            };
+            auto mul = [&](frag l, frag q, block b) __attribute__((always_inline)) {
+                if constexpr (LONG_B)
+                    acc[b.j][b.i] = X::go(l, q, acc[b.j][b.i]);
+                else
+                    acc[b.i][b.j] = X::go(q, l, acc[b.i][b.j]);
+            };
+            constexpr int NF = (FL + FS) * KK, NM = NB * KK;  // fetches and MFMAs of a step
+            // AHEAD: fetch number t of a stage, in the order in which its blocks want them.
+            auto fetch_nth = [&](int t, int set, unsigned slot, unsigned next) __attribute__((always_inline)) {
+                int n = 0;
 #pragma unroll
-                for (int i = 0; i < FL; i++) {
+                for (int c = 0; c < NB; c++) {
+                    const block x = block_at(c);
+                    bool new_l = true, new_s = true;
+#pragma unroll
+                    for (int d = 0; d < c; d++) {
+                        const block y = block_at(d);
+                        if (y.i == x.i) new_l = false;
+                        if (y.j == x.j) new_s = false;
+                    }
+#pragma unroll
+                    for (int kk = 0; kk < KK; kk++) {
+                        if (new_s && n++ == t) fetch_s(sf[AHEAD ? set : 0][x.j][kk], x.j, kk, slot, next);
+                        if (new_l && n++ == t) fetch_l(lf[set][AHEAD ? x.i : 0][kk], x.i, kk, slot, next);
+                    }
+                }
+            };
+            // The step on set SET: the first half of its MFMAs, the meeting, the rest with the next stage's fetches.
+            // (Met at the start, a stage that arrives late holds up the MFMAs of two stages.)
+            auto step_ahead = [&](auto set_c, unsigned next, unsigned after) __attribute__((always_inline)) {
+                constexpr int SET = decltype(set_c)::value, MEET = NB / 2 * KK, SPAN = NB == 1 ? NM : (NM - MEET) * 3 / 4;
+#pragma unroll
+                for (int m = 0; m < NM; m++) {
+                    const block b = block_at(m / KK);
+                    if (m == MEET) meet();
+                    mul(lf[SET][AHEAD ? b.i : 0][m % KK], sf[AHEAD ? SET : 0][b.j][m % KK], b);
                     __builtin_amdgcn_sched_barrier(0);
-                    if (last && i == MEET) {
-                        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wavefront's fetches from the slot have returned
-                        __builtin_amdgcn_s_barrier();
-                        asm volatile("" ::: "memory");
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
 #pragma unroll
-                    for (int j = 0; j < FS; j++) {
-                        if constexpr (LONG_B)
-                            acc[j][i] = X::go(lf[RING ? 0 : kk & 1][i], sf[kk & 1][j], acc[j][i]);
-                        else
-                            acc[i][j] = X::go(sf[kk & 1][j], lf[RING ? 0 : kk & 1][i], acc[i][j]);
-                    }
-                    if (i >= from) {
-                        const int by_now = (i - from + 1) * (FL + FS) * 4 / (3 * (FL - from)) - (i + 1);
-                        const int s_to = by_now < 0 ? 0 : i == FL - 1 || by_now > FS ? FS : by_now;
-                        const int n = i + 1 - l_done + s_to - s_done;
+                    for (int t = 0; t < NF; t++)
+                        if (m >= MEET && t * SPAN >= (m - MEET) * NF && t * SPAN < (m - MEET + 1) * NF) fetch_nth(t, 1 - SET, next, after);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            // The step in strips.  The last strip's long fragments are the last ones fetched from the slot; with four k-steps
+            // half of that strip is enough to fetch behind, and the later a stage is asked for, the less often it is late.
+            auto step_strips = [&](unsigned slot, unsigned next, unsigned after) __attribute__((always_inline)) {
+                constexpr int LEAD = LEAD_B * KK, PER = 2 * FS * KK, MEET = KK > 2 ? PER / 2 : 0, SPAN = KK > 2 ? PER * 3 / 8 : 2 * KK;
 #pragma unroll
-                        for (int q = 0; q < FS; q++)
-                            if (q >= s_done && q < s_to) fetch_s(nkk, last ? next : slot, last ? after : next, q);
+                for (int m = 0; m < NM; m++) {
+                    const block b = block_at(m / KK);
+                    const int strip = m < LEAD ? 0 : (m - LEAD) / PER + FL % 2, w = m < LEAD ? m : (m - LEAD) % PER;
+                    const int len = m < LEAD ? LEAD : PER;
+                    if (strip == NS - 1 && w == MEET) meet();
+                    mul(lf[strip % LSETS][AHEAD ? 0 : FL % 2 ? (b.i + 1) % 2 * (b.i > 0) : b.i % 2][m % KK], sf[0][b.j][m % KK], b);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (strip < NS - 1) {
+                        // the next strip's long fragments; in front of them, in the first strip, the last short one
+                        const int ns = strip == 0 ? KK : 0, n = ns + 2 * KK, span = strip == NS - 2 ? len / 2 : len * 3 / 4;
 #pragma unroll
-                        for (int q = 0; q < FL; q++)
-                            if (q >= l_done && q <= i) fetch_l(nkk, last ? next : slot, last ? after : next, q);
-                        l_done = i + 1;
-                        s_done = s_to;
-#pragma unroll
-                        for (int t = 0; t < FL + FS; t++) {
-                            if (t < n) {
-                                const int m = (t + 1) * FS / n - t * FS / n;  // MFMAs in front of this fetch
-                                if (m == 1) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                                if (m == 2) __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-                                if (m == 3) __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
-                                if (m >= 4) __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-                                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                        for (int t = 0; t < 3 * KK; t++) {
+                            if (t < n && t * span >= w * n && t * span < (w + 1) * n) {
+                                const int h = (t - ns) / KK, kk = t % KK;
+                                if (t < ns)
+                                    fetch_s(sf[0][FS - 1][kk], FS - 1, kk, slot, next);
+                                else
+                                    fetch_l(lf[(strip + 1) % LSETS][h][kk], 2 * (strip + 1) - FL % 2 + h, kk, slot, next);
                             }
+                        }
+                    } else {
+                        // the next stage's: long fragments at once, a short one behind its last MFMA
+#pragma unroll
+                        for (int t = 0; t < (2 - FL % 2) * KK; t++)
+                            if (w == MEET + t * SPAN / (2 * KK)) fetch_l(lf[0][t / KK][t % KK], t / KK, t % KK, next, after);
+#pragma unroll
+                        for (int t = 0; t < (FS - 1) * KK; t++) {
+                            const int freed = (t / KK + 1) * 2 * KK - 1;
+                            if (w == (freed > MEET ? freed : MEET) + t % KK * SPAN / (2 * KK)) fetch_s(sf[0][t / KK][t % KK], t / KK, t % KK, next, after);
                         }
                     }
                     __builtin_amdgcn_sched_barrier(0);
@@ -448,15 +510,28 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             unsigned slot = 0;
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
+            // Behind the last stage, zeros never used are fetched.
+            if constexpr (AHEAD) {
 #pragma unroll
-            for (int j = 0; j < FS; j++) fetch_s(0, 0, STAGE, j);
+                for (int t = 0; t < NF; t++) fetch_nth(t, 0, 0, STAGE);
+                for (int kt = 0;;) {
+                    unsigned next = behind_slot(slot);
+                    step_ahead(std::integral_constant<int, 0>{}, next, behind_slot(next));
+                    if (++kt == KT) break;
+                    slot = behind_slot(next);
+                    step_ahead(std::integral_constant<int, 1>{}, slot, behind_slot(slot));
+                    if (++kt == KT) break;
+                }
+            } else {
 #pragma unroll
-            for (int i = 0; i < FL; i++) fetch_l(0, 0, STAGE, i);
-            for (int kt = 0; kt < KT; kt++) {
-                const unsigned next = behind_slot(slot), after = SHIFT ? behind_slot(next) : next;
+                for (int t = 0; t < (2 - FL % 2) * KK; t++) fetch_l(lf[0][t / KK][t % KK], t / KK, t % KK, 0, STAGE);
 #pragma unroll
-                for (int kk = 0; kk < KK; kk++) k_step(kk, slot, next, after);  // the last one fetches from the next slot: behind the last stage, zeros never used
-                slot = next;
+                for (int t = 0; t < (FS - 1) * KK; t++) fetch_s(sf[0][t / KK][t % KK], t / KK, t % KK, 0, STAGE);
+                for (int kt = 0; kt < KT; kt++) {
+                    const unsigned next = behind_slot(slot), after = behind_slot(next);
+                    step_strips(slot, next, after);
+                    slot = next;
+                }
             }
             __builtin_amdgcn_s_waitcnt(0xC07F);
             __builtin_amdgcn_s_barrier();
