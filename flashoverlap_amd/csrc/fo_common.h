@@ -194,7 +194,7 @@ int fo_pace_with(double seconds, fo_stream_t stream);  // a one-lane kernel that
 __host__ __device__ inline int fo_pack_row_waves(int log_bh, int log_bw, int log_xc, int resident) {
     return log_bh | log_bw << 4 | log_xc << 8 | resident << 12;
 }
-__host__ __device__ inline void fo_row_wave_tile(int t, int packed, int *pm, int *pn) {
+__host__ __device__ inline __attribute__((always_inline)) void fo_row_wave_tile(int t, int packed, int *pm, int *pn) {
     const int log_bh = packed & 15, log_bw = (packed >> 4) & 15, log_xc = (packed >> 8) & 15, R = packed >> 12;
     const int k = t / R, w = t - k * R;
     const int x = w & 7, j = w >> 3;
@@ -204,7 +204,7 @@ __host__ __device__ inline void fo_row_wave_tile(int t, int packed, int *pm, int
 }
 
 // Workgroup id -> macro tile coordinates; identical code on host and device.
-__host__ __device__ inline void fo_wg_to_tile(int wg, int grid_m, int grid_n, int panel,
+__host__ __device__ inline __attribute__((always_inline)) void fo_wg_to_tile(int wg, int grid_m, int grid_n, int panel,
                                               int xcd_remap, int *pm, int *pn) {
     if (xcd_remap == 2) {
         fo_row_wave_tile(wg, panel, pm, pn);
@@ -231,7 +231,7 @@ __host__ __device__ inline void fo_wg_to_tile(int wg, int grid_m, int grid_n, in
 
 // Unit u of a launch that covers raster positions first, first + 1, ... with each
 // position cut into sub_m x sub_n tiles of its own -> coordinates in those tiles.
-__host__ __device__ inline void fo_unit_to_tile(int u, int first, int sub_m, int sub_n, int grid_m,
+__host__ __device__ inline __attribute__((always_inline)) void fo_unit_to_tile(int u, int first, int sub_m, int sub_n, int grid_m,
                                                 int grid_n, int panel, int xcd_remap, int *pm, int *pn) {
     const int per = sub_m * sub_n;
     if (per == 1) {

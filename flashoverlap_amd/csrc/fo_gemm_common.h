@@ -25,13 +25,29 @@ namespace fo_gemm_dev {
 // to row q * seg_rows + f / W + i of the accumulator (if any) and, for q == rank, stored to row f / W + i of OWN (if any).
 enum { MODE_PLAIN = 0, MODE_SIGNAL = 1, MODE_SCATTER = 2, MODE_ACC = 3, MODE_RS = 4 };
 
+// Division by a number that the host knows: n / d for n and d below 32768, exactly (the product exceeds n / d * 2^31 by
+// less than n * d).
+struct fo_div {
+    uint32_t mul;  // 2^31 / d rounded up
+};
+__host__ __device__ inline __attribute__((always_inline)) int fo_divide(int n, fo_div d) {
+    return (int)((uint64_t)(uint32_t)(2 * n) * d.mul >> 32);
+}
+constexpr long kMaxDivide = 32767;
+inline fo_div fo_divisor(long d) { return {d > 0 ? (uint32_t)(((1ULL << 31) + d - 1) / d) : 0}; }
+
+// The fields that a kernel's first operand load needs stand in front: they come with one load.
 struct GemmArgs {
     const uint16_t *A;
     const uint16_t *B;
-    uint16_t *C;
-    uint16_t *ACC;         // MODE_ACC, MODE_RS: the accumulator
     int M, N, K;
     int lda, ldb;          // row strides of A and B in elements (multiples of 8)
+    int grid_m, grid_n, panel, xcd_remap;  // the raster of this launch's parent tiles
+    int first, sub_m, sub_n, count;        // this launch: positions from `first`, each cut into sub_m x sub_n macro tiles, `count` of them
+    fo_div by_panel, by_rows, by_last_rows;  // divisors of the raster walk (fo_set_divisors): tiles of a panel, its rows, the last panel's
+    int general;                           // another walk, or numbers too large for those
+    uint16_t *C;
+    uint16_t *ACC;         // MODE_ACC, MODE_RS: the accumulator
     int BM, BN, TN, rLDN;  // reorder/signal tile, tiles along N, reshaped width in tiles
     const int32_t *RA;
     const int32_t *RE;
@@ -39,14 +55,42 @@ struct GemmArgs {
     int G;
     int32_t *MM;
     int monitor;
-    int grid_m, grid_n, panel, xcd_remap;  // the raster of this launch's parent tiles
-    int first, sub_m, sub_n, count;        // this launch: positions from `first`, each cut into sub_m x sub_n macro tiles, `count` of them
     int quiet;                             // signalling epilogues: store the tiles reordered, touch no counter
     int half;                              // 256x256 kernel: half a tile is left at the end of M (bit 0), N (bit 1)
     uint16_t *OWN;                         // MODE_RS: this rank's rows
     int W, rank, seg_rows;                 // MODE_RS: ranks, this rank, rows of the view per rank
     int stream_out;                        // 256x256 kernel: store the output with the non-temporal hint
 };
+
+inline void fo_set_divisors(GemmArgs &a) {
+    const long positions = (long)a.grid_m * a.grid_n;
+    a.by_panel = fo_divisor((long)a.panel * a.grid_n);
+    a.by_rows = fo_divisor(a.panel);
+    a.by_last_rows = fo_divisor(a.panel > 0 ? a.grid_m % a.panel : 1);
+    a.general = a.xcd_remap == 2 || a.sub_m * a.sub_n > 1 || positions > kMaxDivide;
+}
+
+// Tile of unit u of a launch: what fo_unit_to_tile gives, without its divisions where the host could prepare them.  (A
+// division is some thirty instructions, and in front of a kernel's first load those are fetched from memory as well.)
+__host__ __device__ inline __attribute__((always_inline)) void fo_tile_of(const GemmArgs &p, int u, int *pm, int *pn) {
+    if (__builtin_expect(p.general, 0)) {
+        int sub_m = p.sub_m, sub_n = p.sub_n, grid_m = p.grid_m, grid_n = p.grid_n, panel = p.panel;
+#ifdef __HIP_DEVICE_COMPILE__
+        asm volatile("" : "+s"(sub_m), "+s"(sub_n), "+s"(grid_m), "+s"(grid_n), "+s"(panel));  // its divisions stay in here
+#endif
+        fo_unit_to_tile(u, p.first, sub_m, sub_n, grid_m, grid_n, panel, p.xcd_remap, pm, pn);
+        return;
+    }
+    const int t = p.first + u, nt = p.grid_m * p.grid_n, x = t & 7, rem = nt & 7;
+    const int v = p.xcd_remap ? x * (nt >> 3) + (x < rem ? x : rem) + (t >> 3) : t;
+    const int q = fo_divide(v, p.by_panel), first_m = q * p.panel, in = v - first_m * p.grid_n;
+    const bool last = p.grid_m - first_m < p.panel;
+    fo_div by;
+    by.mul = last ? p.by_last_rows.mul : p.by_rows.mul;
+    const int rows = last ? p.grid_m - first_m : p.panel, col = fo_divide(in, by);
+    *pm = first_m + in - col * rows;
+    *pn = col;
+}
 
 // Every operand row begins on a 128-byte line.
 inline bool on_lines(const GemmArgs &a) { return (((uintptr_t)a.A | (uintptr_t)a.B | (uintptr_t)a.lda * 2) & 127) == 0; }

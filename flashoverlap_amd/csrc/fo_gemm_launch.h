@@ -73,7 +73,9 @@ inline int launch_kernel(const GemmArgs &a, hipStream_t stream, int *resident_ou
         return FO_OK;
     }
     dim3 grid(ntiles < resident ? ntiles : resident), block(threads);
-    hipLaunchKernelGGL(kern, grid, block, smem, stream, a);
+    GemmArgs args = a;
+    fo_set_divisors(args);
+    hipLaunchKernelGGL(kern, grid, block, smem, stream, args);
     FO_LAUNCH_CHECK();
     return FO_OK;
 }

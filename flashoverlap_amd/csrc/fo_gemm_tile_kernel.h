@@ -88,7 +88,7 @@ constexpr int tile_smem_bytes() {
 }
 
 template <typename Tag, int TM, int TN, int BK, int S, int MODE, bool SHIFT>
-__global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs p) {
+__global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs args) {
     typedef fo_elem<Tag> E;
     typedef fo_mfma16<Tag> X;
     typedef typename X::frag frag;
@@ -119,7 +119,84 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
     const bool loader = wave_id < NL;
     const int wave = loader ? wave_id : wave_id - NL;
     const int wm = wave >> 1, wn = wave & 1;
-    const int KT = (p.K + BK - 1) / BK;
+    const int KT = (args.K + BK - 1) / BK;
+
+    // The first tile from position `tile` on.  (One cut from a 256x256 position may lie beyond the matrix.)
+    int tile = blockIdx.x, pm = 0, pn = 0;
+    auto settle = [&]() __attribute__((always_inline)) {
+        while (tile < args.count) {
+            fo_tile_of(args, tile, &pm, &pn);
+            pm = __builtin_amdgcn_readfirstlane(pm);
+            pn = __builtin_amdgcn_readfirstlane(pn);
+            if (__builtin_expect(!args.general, 1) || (pm * TM < args.M && pn * TN < args.N)) break;
+            tile += gridDim.x;
+        }
+    };
+    // A loader's part of the tile: load u of a 64-column block brings rows (u * NL + wave) * 8 + lane / 8 of an operand, 128
+    // bytes each; LDS slot `lane` of the 1 KiB block is (row lane / 8, chunk lane % 8) and receives chunk phys ^ key(row).
+    // Shifted, slot `lane` receives chunk ((phys ^ key(row)) + shift(row)) % 8 of the row's aligned line, so that a
+    // column's chunk lies where it would unshifted; what lies before the row's first column or behind its last is
+    // requested out of range (zeros).
+    fo_srd_t ra = {}, rb = {};
+    int a_chunk = 0, b_chunk = 0;
+    unsigned lane_row = 0, wave_lds = 0;
+    const unsigned row_step = (unsigned)(NL * 8 * args.lda * 2);
+    // With twelve loads a stage the row offsets no longer fit the scalar registers.
+    auto load = [&](fo_srd_t srd, unsigned voff, unsigned row_off, unsigned col_off, unsigned lds_addr) __attribute__((always_inline)) {
+        if constexpr (P >= 12)
+            dma_buf16_sum(srd, voff, __builtin_amdgcn_readfirstlane(row_off), col_off, lds_addr);
+        else
+            dma_buf16(srd, voff, __builtin_amdgcn_readfirstlane(row_off + col_off), lds_addr);
+    };
+    auto request = [&](int kt, unsigned slot_v) __attribute__((always_inline)) {
+        const unsigned slot = __builtin_amdgcn_readfirstlane(slot_v);  // uniform by construction; said so for the assembly's operands
+#pragma unroll
+        for (int kb = 0; kb < KB; kb++) {
+            const int col = __builtin_amdgcn_readfirstlane(kt * BK + kb * 64);
+            // chunks beyond K (a partial last step, stages behind the last) are requested out of range: zeros
+            const unsigned a_off = (SHIFT ? (unsigned)(col + a_chunk * 8) < (unsigned)args.K : a_chunk * 8 < args.K - col) ? lane_row + a_chunk * 16 : 0x80000000u;
+            const unsigned b_off = !SHIFT ? a_off : (unsigned)(col + b_chunk * 8) < (unsigned)args.K ? lane_row + b_chunk * 16 : 0x80000000u;
+#pragma unroll
+            for (int u = 0; u < PB; u++)
+                load(rb, b_off, u * row_step, col * 2, wave_lds + slot + KB * A_BLK + kb * B_BLK + u * NL * 1024);
+#pragma unroll
+            for (int u = 0; u < PA; u++)
+                load(ra, a_off, u * row_step, col * 2, wave_lds + slot + kb * A_BLK + u * NL * 1024);
+        }
+    };
+    // Requests the tile's first S - 1 stages.  A launch's first tile is begun in front of everything else in the kernel:
+    // every instruction and argument in front of the first load is itself fetched from memory.  With the raster's divisions,
+    // the reorder table's entries and what the compiler moves out of the tile loop there, the first load left 2800 to 3900
+    // clocks after the kernel's start, now 1200 (us, GEMM alone, plain / reordered: 128x4096x1024 5.1 -> 4.5 / 5.6 -> 4.7,
+    // 512x4096x4096 21.6 -> 21.3 / 22.1 -> 21.3, 1024x4096x2048 18.6 -> 18.0 / 19.1 -> 17.8).
+    auto begin = [&]() __attribute__((always_inline)) {
+        int lane = threadIdx.x & 63;
+        asm volatile("" : "+v"(lane));
+        const int m0 = pm * TM + TM > args.M ? args.M - TM : pm * TM, n0 = pn * TN + TN > args.N ? args.N - TN : pn * TN;  // as below
+        const int lrow = lane >> 3, lkey = ((wave * 8 + lrow) >> 1) & 7;
+        const uint16_t *a0 = args.A + (size_t)m0 * args.lda, *b0 = args.B + (size_t)n0 * args.ldb;
+        const int a_shift = SHIFT ? row_shift(a0, args.lda, lrow) : 0, b_shift = SHIFT ? row_shift(b0, args.ldb, lrow) : 0;
+        a_chunk = SHIFT ? ((((lane & 7) ^ lkey) + a_shift) & 7) - a_shift : (lane & 7) ^ lkey;
+        b_chunk = SHIFT ? ((((lane & 7) ^ lkey) + b_shift) & 7) - b_shift : (lane & 7) ^ lkey;
+        constexpr int LEAD = SHIFT ? 128 : 0;  // the range starts a line early: no lane's offset is negative
+        lane_row = (unsigned)((wave * 8 + lrow) * args.lda * 2 + LEAD);
+        ra = fo_make_srd(a0 - LEAD / 2, (unsigned)TM * args.lda * 2 + LEAD);
+        rb = fo_make_srd(b0 - LEAD / 2, (unsigned)TN * args.ldb * 2 + LEAD);
+        wave_lds = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024);
+        asm volatile("" : "+s"(wave_lds));  // the loads' LDS addresses are sums made where they are used
+        __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+        for (int s = 0; s < S - 1; s++) request(s, s * STAGE);
+    };
+    asm volatile("" : : "s"(args.A), "s"(args.B), "s"(args.count), "s"(args.general));  // all of them with the first round trip
+    settle();
+    if (loader && tile < args.count) begin();
+
+    // The arguments that are not needed before this point are read from here on, not at the kernel's entry.
+    typedef const __attribute__((address_space(4))) GemmArgs *args_t;
+    args_t rest = (args_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(rest));
+    const __attribute__((address_space(4))) GemmArgs &p = *rest;
 
     const int bm_shift = p.BM == 256 ? 8 : 7, bn_shift = p.BN == 256 ? 8 : 7;  // reorder tiles: 128 or 256 each way
     const bool reorder = MODE == MODE_ACC ? p.RA != nullptr : MODE != MODE_PLAIN;
@@ -128,16 +205,11 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
     typedef const __attribute__((address_space(4))) int32_t *cptr_t;  // read-only for the whole launch: scalar loads
     const cptr_t RAc = (cptr_t)(uintptr_t)p.RA;
 
-    for (int tile = blockIdx.x; tile < p.count; tile += gridDim.x) {
+    while (tile < args.count) {
         // What is computed from the lane is computed for each tile: kept from one to the next, the group search's and the
         // loaders' part of it alone took twenty registers through the K loop.
         int lane = tid & 63;
         asm volatile("" : "+v"(lane));
-        int pm, pn;
-        fo_unit_to_tile(tile, p.first, p.sub_m, p.sub_n, p.grid_m, p.grid_n, p.panel, p.xcd_remap, &pm, &pn);
-        pm = __builtin_amdgcn_readfirstlane(pm);
-        pn = __builtin_amdgcn_readfirstlane(pn);
-        if (pm * TM >= p.M || pn * TN >= p.N) continue;  // cut from a 256x256 position that reaches beyond the matrix
         // Where the dimension ends inside the tile, the tile is moved back so that all of its operand rows exist; the
         // rows or columns it then shares with its neighbour are neither stored nor counted.
         const int m0 = pm * TM + TM > p.M ? p.M - TM : pm * TM, n0 = pn * TN + TN > p.N ? p.N - TN : pn * TN;
@@ -227,48 +299,6 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
         };
 
         if (loader) {
-            // Load u of a 64-column block brings rows (u * NL + wave) * 8 + lane / 8 of an operand, 128 bytes each; LDS
-            // slot `lane` of the 1 KiB block is (row lane / 8, chunk lane % 8) and receives chunk phys ^ key(row).
-            // Shifted, slot `lane` receives chunk ((phys ^ key(row)) + shift(row)) % 8 of the row's aligned line, so that a
-            // column's chunk lies where it would unshifted; what lies before the row's first column or behind its last is
-            // requested out of range (zeros).
-            const int lrow = lane >> 3, lkey = ((wave * 8 + lrow) >> 1) & 7;
-            const uint16_t *a0 = p.A + (size_t)m0 * p.lda, *b0 = p.B + (size_t)n0 * p.ldb;
-            const int a_shift = SHIFT ? row_shift(a0, p.lda, lrow) : 0, b_shift = SHIFT ? row_shift(b0, p.ldb, lrow) : 0;
-            const int a_chunk = SHIFT ? ((((lane & 7) ^ lkey) + a_shift) & 7) - a_shift : (lane & 7) ^ lkey;
-            const int b_chunk = SHIFT ? ((((lane & 7) ^ lkey) + b_shift) & 7) - b_shift : (lane & 7) ^ lkey;
-            constexpr int LEAD = SHIFT ? 128 : 0;  // the range starts a line early: no lane's offset is negative
-            const unsigned lane_row = (unsigned)((wave * 8 + lrow) * p.lda * 2 + LEAD);
-            const unsigned row_step = (unsigned)(NL * 8 * p.lda * 2);
-            const fo_srd_t ra = fo_make_srd(a0 - LEAD / 2, (unsigned)TM * p.lda * 2 + LEAD);
-            const fo_srd_t rb = fo_make_srd(b0 - LEAD / 2, (unsigned)TN * p.ldb * 2 + LEAD);
-            const unsigned wave_lds = lds0 + wave * 1024;
-            // With twelve loads a stage the row offsets no longer fit the scalar registers.
-            auto load = [&](fo_srd_t srd, unsigned voff, unsigned row_off, unsigned col_off, unsigned lds_addr) __attribute__((always_inline)) {
-                if constexpr (P >= 12)
-                    dma_buf16_sum(srd, voff, __builtin_amdgcn_readfirstlane(row_off), col_off, lds_addr);
-                else
-                    dma_buf16(srd, voff, __builtin_amdgcn_readfirstlane(row_off + col_off), lds_addr);
-            };
-            auto request = [&](int kt, unsigned slot_v) __attribute__((always_inline)) {
-                const unsigned slot = __builtin_amdgcn_readfirstlane(slot_v);  // uniform by construction; said so for the assembly's operands
-#pragma unroll
-                for (int kb = 0; kb < KB; kb++) {
-                    const int col = __builtin_amdgcn_readfirstlane(kt * BK + kb * 64);
-                    // chunks beyond K (a partial last step, stages behind the last) are requested out of range: zeros
-                    const unsigned a_off = (SHIFT ? (unsigned)(col + a_chunk * 8) < (unsigned)p.K : a_chunk * 8 < p.K - col) ? lane_row + a_chunk * 16 : 0x80000000u;
-                    const unsigned b_off = !SHIFT ? a_off : (unsigned)(col + b_chunk * 8) < (unsigned)p.K ? lane_row + b_chunk * 16 : 0x80000000u;
-#pragma unroll
-                    for (int u = 0; u < PB; u++)
-                        load(rb, b_off, u * row_step, col * 2, wave_lds + slot + KB * A_BLK + kb * B_BLK + u * NL * 1024);
-#pragma unroll
-                    for (int u = 0; u < PA; u++)
-                        load(ra, a_off, u * row_step, col * 2, wave_lds + slot + kb * A_BLK + u * NL * 1024);
-                }
-            };
-            __builtin_amdgcn_s_setprio(3);
-#pragma unroll
-            for (int s = 0; s < S - 1; s++) request(s, s * STAGE);
             wait_vmcnt<FLIGHT>();  // what the first step reads has landed (vmcnt retires in issue order)
             __builtin_amdgcn_s_barrier();
             unsigned slot = (S - 1) * STAGE;
@@ -596,7 +626,12 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                 }
             }
         }
-        if (tile + (int)gridDim.x < p.count) __syncthreads();  // the staged tile has been read by everyone
+        tile += gridDim.x;
+        settle();
+        if (tile < args.count) {
+            __syncthreads();  // the staged tile has been read by everyone
+            if (loader) begin();
+        }
     }
 }
 
