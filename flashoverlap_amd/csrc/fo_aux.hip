@@ -639,7 +639,9 @@ __global__ __launch_bounds__(256, (CH <= 4 && !(CH == 4 && std::is_same<Tag, fo_
         // way during this one.  And a 16-byte store's data registers are read for some cycles after it issues, so
         // a vector instruction that writes one of them right behind it must keep two wait states; the compiler
         // leaves them out for the buffer form with a scalar offset register, and lanes 12-63 of a stored chunk
-        // then carried the next chunk's intermediate values whenever the CU was busy.
+        // then carried the next chunk's intermediate values whenever the CU was busy.  Written through, like the small
+        // GEMMs' outputs (store16_write_through in fo_gemm_common.h): whole passes 32.6 -> 31.4 us (1152x5120), 43.4 -> 42.8
+        // (1024x8192), 23.7 -> 23.3 (256x8192); the row kernel above, which is left the long matrices, gains nothing.
         const uint64_t yb = (uint64_t)(uintptr_t)(Y + (long)b * nch);
         fo_u32x4 yr;
         yr.x = __builtin_amdgcn_readfirstlane((unsigned)yb);
@@ -655,7 +657,7 @@ __global__ __launch_bounds__(256, (CH <= 4 && !(CH == 4 && std::is_same<Tag, fo_
                              : "v"(y), "v"((unsigned)tid * 16u), "s"(yr), "s"(i * 4096)
                              : "memory");
             else
-                asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen\n\ts_nop 1"
+                asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen sc0 sc1\n\ts_nop 1"
                              :
                              : "v"(y), "v"((unsigned)tid * 16u), "s"(yr), "s"(i * 4096)
                              : "memory");

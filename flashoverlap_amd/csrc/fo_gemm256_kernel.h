@@ -611,10 +611,10 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                         if (MODE == MODE_RS) {
                             const int ac = row_of(k, ac_lo, ac_hi);
                             if (sums && ac >= 0)
-                                store16(p.ACC + (size_t)ac * ldp + tcol + scol * 8, fo_add8<Tag>(old[ACC ? k : 0], v));
+                                store16_write_through(p.ACC + (size_t)ac * ldp + tcol + scol * 8, fo_add8<Tag>(old[ACC ? k : 0], v));
                             if ((unsigned)(ac - own_first) < (unsigned)own_rows)
-                                store16(p.OWN + (size_t)(ac - own_first) * ldp + tcol + scol * 8, v);
-                            store16(to, v);
+                                store16_write_through(p.OWN + (size_t)(ac - own_first) * ldp + tcol + scol * 8, v);
+                            store16_write_through(to, v);
                         } else if (stream_out) {
                             store16_write_through_nt(to, v);
                         } else {
@@ -626,21 +626,14 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                             char *ab = abase + (size_t)(i * 16 + ps * RPP) * ldp * 2;
                             const fo_u32x4 sum = fo_add8<Tag>(old[i * (16 / RPP) + ps], v);
                             if (stream_out)
-                                store16_nt(ab, lane_off, sum);
+                                store16_write_through_nt(ab, lane_off, sum);
                             else
-                                store16(ab, lane_off, sum);
+                                store16_write_through(ab, lane_off, sum);
                         }
-                        if (!COUNTS) {
-                            if (stream_out)
-                                store16_nt(sb, lane_off, v);
-                            else
-                                store16(sb, lane_off, v);
-                        } else {
-                            if (stream_out)
-                                store16_write_through_nt(sb, lane_off, v);
-                            else
-                                store16_write_through(sb, lane_off, v);
-                        }
+                        if (stream_out)
+                            store16_write_through_nt(sb, lane_off, v);
+                        else
+                            store16_write_through(sb, lane_off, v);
                     }
                 }
                 __builtin_amdgcn_s_waitcnt(0xC07F);  // strip reads done before the next pass overwrites it

@@ -171,28 +171,22 @@ __device__ __forceinline__ void wait_vmcnt() {
 // 16-byte global stores written as assembly so that the number of vector memory
 // instructions in flight is known exactly (the main loop waits on vmcnt with
 // non-zero counts; the compiler does not see these instructions in its own
-// count, which can only make its waits longer, never shorter).  The
-// write-through form (system-scope cache policy) is used for the signalled
-// epilogues: the tile must be visible to other XCDs before its counter is
-// bumped, and a tile that never becomes dirty in L2 needs no releasing
-// write-back before the signal.  The trailing s_nop covers
+// count, which can only make its waits longer, never shorter).  All of them write
+// through (system-scope cache policy).  In the signalled epilogues the tile must be
+// visible to other XCDs before its counter is bumped, and a tile that never becomes
+// dirty in L2 needs no releasing write-back before the signal.  Elsewhere the lines
+// left dirty in the L2s would be written back between this kernel and the next,
+// when nothing else runs (GEMM with an accumulator, us: 1152x5120x1720 28.4 -> 26.7,
+// 1024x4096x2048 20.0 -> 18.8, 512x4096x4096 21.8 -> 21.2, 1024x8192x2048 34.0 ->
+// 33.4; whole passes: sequence 38.0 -> 36.1, ragged 35.1 -> 33.9).  The trailing s_nop covers
 // the wait states gfx9 requires between a VMEM store of more than 8 bytes and a
 // VALU write of its data registers.
 __device__ __forceinline__ void store16_write_through(void *ptr, fo_u32x4 v) {
     asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" : : "v"(ptr), "v"(v) : "memory");
 }
-__device__ __forceinline__ void store16(void *ptr, fo_u32x4 v) {
-    asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" : : "v"(ptr), "v"(v) : "memory");
-}
 // saddr forms: wave-uniform base (SGPR pair) + 32-bit per-lane byte offset
 __device__ __forceinline__ void store16_write_through(char *base, unsigned lane_off, fo_u32x4 v) {
     asm volatile("global_store_dwordx4 %0, %1, %2 sc0 sc1\n\ts_nop 1"
-                 :
-                 : "v"(lane_off), "v"(v), "s"((__attribute__((address_space(1))) char *)base)
-                 : "memory");
-}
-__device__ __forceinline__ void store16(char *base, unsigned lane_off, fo_u32x4 v) {
-    asm volatile("global_store_dwordx4 %0, %1, %2\n\ts_nop 1"
                  :
                  : "v"(lane_off), "v"(v), "s"((__attribute__((address_space(1))) char *)base)
                  : "memory");
@@ -202,7 +196,7 @@ __device__ __forceinline__ void store16(char *base, unsigned lane_off, fo_u32x4 
 // at once, and output lines that took room in the L2 would push out the operand panels the next tile's
 // first K steps are about to share.  8192^3: GEMM alone 1.7 % faster, the overlapped step unchanged; on
 // the 8192x4096 output (67 MB), which the consumer finds in the memory-side cache, the hint made the
-// overlapped step 2 % and the serial step 8 % slower, so smaller outputs stay cacheable.
+// overlapped step 2 % and the serial step 8 % slower, so smaller outputs go without it.
 __device__ __forceinline__ void store16_write_through_nt(void *ptr, fo_u32x4 v) {
     asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt\n\ts_nop 1" : : "v"(ptr), "v"(v) : "memory");
 }
@@ -212,13 +206,6 @@ __device__ __forceinline__ void store16_write_through_nt(char *base, unsigned la
                  : "v"(lane_off), "v"(v), "s"((__attribute__((address_space(1))) char *)base)
                  : "memory");
 }
-__device__ __forceinline__ void store16_nt(char *base, unsigned lane_off, fo_u32x4 v) {
-    asm volatile("global_store_dwordx4 %0, %1, %2 nt\n\ts_nop 1"
-                 :
-                 : "v"(lane_off), "v"(v), "s"((__attribute__((address_space(1))) char *)base)
-                 : "memory");
-}
-
 #define FO_LDS_PTR(p) ((__attribute__((address_space(3))) void *)(p))
 
 typedef unsigned int fo_srd_t __attribute__((ext_vector_type(4)));  // buffer descriptor

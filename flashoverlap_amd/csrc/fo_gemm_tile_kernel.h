@@ -352,7 +352,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
 #pragma unroll
                     for (int u = 0; u < NCH; u++) asm volatile("" : "+v"(old[u]));
                     auto add = [&](int u, int row, int col, uint16_t *at) __attribute__((always_inline)) {
-                        *reinterpret_cast<fo_u32x4 *>(at) = fo_add8<Tag>(old[u], piece(row, col));
+                        store16_write_through(at, fo_add8<Tag>(old[u], piece(row, col)));
                     };
                     if constexpr (MODE == MODE_RS)
                         each_mapped_piece(wave * 64 + lane, rs_map, p.ACC, std::false_type{}, add);
@@ -363,7 +363,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                     find_bases();
                     each_mapped_piece(wave * 64 + lane, rs_map, p.OWN, std::false_type{},
                                       [&](int, int row, int col, uint16_t *at) __attribute__((always_inline)) {
-                        *reinterpret_cast<fo_u32x4 *>(at) = piece(row, col);
+                        store16_write_through(at, piece(row, col));
                     }, p.rank * p.seg_rows, p.seg_rows);
                 }
             }
@@ -587,7 +587,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
                 auto put = [&](int, int row, int col, uint16_t *at) __attribute__((always_inline)) {
-                    *reinterpret_cast<fo_u32x4 *>(at) = piece(row, col);
+                    store16_write_through(at, piece(row, col));
                 };
                 if constexpr (MODE == MODE_RS)
                     each_mapped_piece(wave * 64 + lane, row_map, p.C, std::false_type{}, put);
@@ -599,10 +599,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             find_bases();
             __syncthreads();
             auto put = [&](int, int row, int col, uint16_t *at) __attribute__((always_inline)) {
-                if constexpr (MODE == MODE_PLAIN)
-                    *reinterpret_cast<fo_u32x4 *>(at) = piece(row, col);
-                else
-                    store16_write_through(at, piece(row, col));
+                store16_write_through(at, piece(row, col));
             };
             if constexpr (MODE == MODE_SCATTER)
                 each_mapped_piece(tid, row_map, p.C, std::false_type{}, put);
