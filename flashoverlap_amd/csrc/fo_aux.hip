@@ -559,11 +559,15 @@ int launch_rmsnorm(const void *X, void *Y, const void *Wt, int bs, int dim, int 
 // Registers: up to 96 per lane, which is what the signalling GEMM's wavefront leaves of its SIMD's
 // 512 (at most 408 with the accumulators); rows above 8192 elements (CH = 8) do without the look-ahead
 // and may take 128, which fits beside the plain GEMM's wavefront only.
-template <typename Tag, int CH, bool STREAM, int PATH>
-__global__ __launch_bounds__(256, (CH <= 4 && !(CH == 4 && std::is_same<Tag, fo_bf16_tag>::value)) ? 5 : 4) void fo_norm_rows_kernel(const fo_u32x4 *X, fo_u32x4 *Y, const fo_u32x4 *Wt,
+//
+// ADD: the consumer's work on the same rows, ACC[o] = round16(ACC[o] + X[o]) at every element of theirs, so that the matrix
+// is read once for both (ACC is laid out as X).  The accumulator's chunks are requested when the row before is done with and
+// used last; up to 128 registers, which fit beside the signalling GEMM's wavefront (384).
+template <typename Tag, int CH, bool STREAM, int PATH, bool ADD>
+__global__ __launch_bounds__(256, (!ADD && CH <= 4 && !(CH == 4 && std::is_same<Tag, fo_bf16_tag>::value)) ? 5 : 4) void fo_norm_rows_kernel(const fo_u32x4 *X, fo_u32x4 *Y, const fo_u32x4 *Wt,
                                                               int row0, int nrows, int rows_per_wg, int dim, int BM,
                                                               int BN, int rldn, const int32_t *RA, float eps,
-                                                              unsigned x_bytes) {
+                                                              unsigned x_bytes, fo_u32x4 *ACC) {
     typedef norm_math<Tag> MATH;
     __shared__ float part[2][4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -581,6 +585,7 @@ __global__ __launch_bounds__(256, (CH <= 4 && !(CH == 4 && std::is_same<Tag, fo_
 #pragma unroll
     for (int i = 0; i < CH; i++) w[i] = Wt[chunk_of(i)];
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)X, 0, x_bytes, 0x00027000);
+    const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc((void *)ACC, 0, ADD ? x_bytes : 0, 0x00027000);
     const int ldn = PATH == NORM_PLAIN ? 0 : dim / BN;
     const int bn_shift = PATH == NORM_SLOTS ? __builtin_ctz(BN) : 0;
     const unsigned ldp_bytes = (unsigned)rldn * BN * 2;  // row pitch of the reordered view
@@ -588,7 +593,8 @@ __global__ __launch_bounds__(256, (CH <= 4 && !(CH == 4 && std::is_same<Tag, fo_
 #pragma unroll
     for (int i = 0; i < CH; i++) off[i] = (unsigned)chunk_of(i) * 16u;
     int slot_row = -1;
-    auto request = [&](int b, fo_u32x4(&x)[CH]) {
+    unsigned at[2][ADD ? CH : 1], at_row[2];  // where the chunks in each register set came from
+    auto request = [&](int b, fo_u32x4(&x)[CH], int set) __attribute__((always_inline)) {
         unsigned row_off;  // wave-uniform
         if (PATH == NORM_PLAIN) {
             row_off = (unsigned)b * (unsigned)dim * 2u;
@@ -612,11 +618,22 @@ __global__ __launch_bounds__(256, (CH <= 4 && !(CH == 4 && std::is_same<Tag, fo_
 #pragma unroll
         for (int i = 0; i < CH; i++)
             x[i] = __builtin_bit_cast(fo_u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, off[i], row_off, NT));
+        if (ADD) {
+            at_row[set] = row_off;
+#pragma unroll
+            for (int i = 0; i < CH; i++) at[set][ADD ? i : 0] = off[i];
+        }
     };
 
     // One row: reduce, meet, scale, store.
     int buf = 0;
-    auto finish = [&](int b, fo_u32x4(&x)[CH]) {
+    auto finish = [&](int b, fo_u32x4(&x)[CH], int set) __attribute__((always_inline)) {
+        fo_u32x4 a[ADD ? CH : 1];
+        if (ADD) {
+#pragma unroll
+            for (int i = 0; i < CH; i++)
+                a[ADD ? i : 0] = __builtin_bit_cast(fo_u32x4, __builtin_amdgcn_raw_buffer_load_b128(ar, at[set][ADD ? i : 0], at_row[set], NT));
+        }
         float ss = 0.f;
 #pragma unroll
         for (int i = 0; i < CH; i++) {
@@ -650,6 +667,7 @@ __global__ __launch_bounds__(256, (CH <= 4 && !(CH == 4 && std::is_same<Tag, fo_
         yr.w = 0x00027000u;
 #pragma unroll
         for (int i = 0; i < CH; i++) {
+            if (ADD) asm volatile("" : "+v"(w[i]));  // bf16: its conversions to 32 bits are made for each row, not kept in twice the registers
             const fo_u32x4 y = MATH::scale(x[i], s, w[i]);
             if (STREAM)
                 asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen nt\n\ts_nop 1"
@@ -661,6 +679,27 @@ __global__ __launch_bounds__(256, (CH <= 4 && !(CH == 4 && std::is_same<Tag, fo_
                              :
                              : "v"(y), "v"((unsigned)tid * 16u), "s"(yr), "s"(i * 4096)
                              : "memory");
+            if (ADD) __builtin_amdgcn_sched_barrier(0);  // one chunk's conversions at a time, or they take thirty registers more
+        }
+        if (ADD) {
+            const uint64_t ab = (uint64_t)(uintptr_t)ACC;
+            fo_u32x4 as;
+            as.x = __builtin_amdgcn_readfirstlane((unsigned)ab);
+            as.y = __builtin_amdgcn_readfirstlane((unsigned)(ab >> 32) & 0xFFFF);
+            as.z = __builtin_amdgcn_readfirstlane(x_bytes);
+            as.w = 0x00027000u;
+            const unsigned row_off = __builtin_amdgcn_readfirstlane(at_row[set]);
+#pragma unroll
+            for (int i = 0; i < CH; i++) {
+                const fo_u32x4 v = fo_add8<Tag>(a[ADD ? i : 0], x[i]);
+                // a lane beyond the row's end holds its last chunk again: out of range
+                const unsigned to = full || tid + i * 256 < nch ? at[set][ADD ? i : 0] : 0x80000000u;
+                if (STREAM)
+                    asm volatile("s_nop 4\n\tbuffer_store_dwordx4 %0, %1, %2, %3 offen nt\n\ts_nop 1" : : "v"(v), "v"(to), "s"(as), "s"(row_off) : "memory");
+                else
+                    asm volatile("s_nop 4\n\tbuffer_store_dwordx4 %0, %1, %2, %3 offen\n\ts_nop 1" : : "v"(v), "v"(to), "s"(as), "s"(row_off) : "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
     };
 
@@ -669,38 +708,38 @@ __global__ __launch_bounds__(256, (CH <= 4 && !(CH == 4 && std::is_same<Tag, fo_
     fo_u32x4 xa[CH], xb[AHEAD ? CH : 1];
     if (!AHEAD) {
         for (int b = first; b < last; b++) {
-            request(b, xa);
-            finish(b, xa);
+            request(b, xa, 0);
+            finish(b, xa, 0);
         }
         return;
     }
     // The loop body holds no branch around a request: where paths with and without a request in flight
     // meet, the compiler waits as if there were none, i.e. for everything.  The last one or two rows follow it.
     fo_u32x4(&xb_)[CH] = reinterpret_cast<fo_u32x4(&)[CH]>(xb);
-    request(first, xa);
+    request(first, xa, 0);
     int b = first;
     for (; b + 2 < last; b += 2) {
-        request(b + 1, xb_);
-        finish(b, xa);
-        request(b + 2, xa);
-        finish(b + 1, xb_);
+        request(b + 1, xb_, 1);
+        finish(b, xa, 0);
+        request(b + 2, xa, 0);
+        finish(b + 1, xb_, 1);
     }
     if (b + 1 < last) {
-        request(b + 1, xb_);
-        finish(b, xa);
-        finish(b + 1, xb_);
+        request(b + 1, xb_, 1);
+        finish(b, xa, 0);
+        finish(b + 1, xb_, 1);
     } else {
-        finish(b, xa);
+        finish(b, xa, 0);
     }
 }
 
 // grid <= 0: one workgroup per row while they are few (1152 x 4096 5.3 us against 5.6 with two, 512 x 5120 3.6 against 4.1), else per
 // 2 rows, at most 4096 (8192 x 8192 fp16 alone: 45.5 us from 4096 workgroups, 47.3 from 2048).  beside_gemm: at most 256 workgroups, each asking for
 // kBesideGemmLds bytes of LDS it never touches (one workgroup per CU beside the GEMM's, as for the consumer).
-template <typename Tag, bool STREAM, int PATH>
+template <typename Tag, bool STREAM, int PATH, bool ADD = false>
 int launch_norm_rows_on(const void *X, void *Y, const void *Wt, int row0, int nrows, int dim, int BM, int BN, int rldn,
                         const int32_t *RA, float eps, bool beside_gemm, int grid, unsigned x_bytes, hipStream_t stream,
-                        int32_t *info) {
+                        int32_t *info, void *acc = nullptr) {
     const int nch = dim / 8;
     if (nrows < 1) nrows = 1;  // the query for the kernel's resources comes with no rows
     if (grid <= 0) grid = nrows <= few_norm_rows(dim) ? nrows : (nrows + 1) / 2;
@@ -716,13 +755,13 @@ int launch_norm_rows_on(const void *X, void *Y, const void *Wt, int row0, int nr
 #define FO_NORM_ROWS(CH_)                                                                                               \
     if (info) {                                                                                                         \
         hipFuncAttributes attr;                                                                                         \
-        FO_HIP_CHECK(hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(&fo_norm_rows_kernel<Tag, CH_, STREAM, PATH>))); \
+        FO_HIP_CHECK(hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(&fo_norm_rows_kernel<Tag, CH_, STREAM, PATH, ADD>))); \
         info[0] = attr.numRegs;                                                                                         \
         info[1] = (int)attr.sharedSizeBytes + lds;                                                                      \
         return FO_OK;                                                                                                   \
     }                                                                                                                   \
-    hipLaunchKernelGGL((fo_norm_rows_kernel<Tag, CH_, STREAM, PATH>), dim3(grid), dim3(256), lds, stream, x, y, w, row0, \
-                       nrows, rows_per_wg, dim, BM, BN, rldn, RA, eps, x_bytes)
+    hipLaunchKernelGGL((fo_norm_rows_kernel<Tag, CH_, STREAM, PATH, ADD>), dim3(grid), dim3(256), lds, stream, x, y, w, row0, \
+                       nrows, rows_per_wg, dim, BM, BN, rldn, RA, eps, x_bytes, static_cast<fo_u32x4 *>(acc))
     if (nch <= 256) {
         FO_NORM_ROWS(1);
     } else if (nch <= 512) {
@@ -731,8 +770,10 @@ int launch_norm_rows_on(const void *X, void *Y, const void *Wt, int row0, int nr
         FO_NORM_ROWS(3);
     } else if (nch <= 1024) {
         FO_NORM_ROWS(4);
-    } else if (nch <= 2048) {
-        FO_NORM_ROWS(8);
+    } else if (nch <= 2048 && !ADD) {
+        if constexpr (!ADD) {
+            FO_NORM_ROWS(8);
+        }
     } else {
         return FO_ERR_SHAPE;
     }
@@ -1040,6 +1081,24 @@ int fo_norm_rows_with(int dtype, const void *X, void *Y, const void *Wt, int row
     if (dtype == FO_BF16)
         return stream_rows ? launch_norm_rows_as<fo_bf16_tag, true>(X, Y, Wt, row0, nrows, dim, BM, BN, rldn, RA, eps, beside_gemm, grid, x_bytes, s, info)
                            : launch_norm_rows_as<fo_bf16_tag, false>(X, Y, Wt, row0, nrows, dim, BM, BN, rldn, RA, eps, beside_gemm, grid, x_bytes, s, info);
+    return FO_ERR_DTYPE;
+}
+
+int fo_consume_norm_rows_with(int dtype, const void *X, void *acc, void *Y, const void *Wt, int row0, int nrows, int bs, int dim,
+                              int BM, int BN, const int32_t *RA, float eps, bool stream_rows, bool beside_gemm,
+                              fo_stream_t stream, int32_t *info) {
+    if (((!X || !acc || !Y || !Wt || !RA) && !info) || bs <= 0 || dim <= 0 || BM <= 0 || BN <= 0) return FO_ERR_ARG;
+    if (row0 < 0 || nrows < 0 || row0 + nrows > bs) return FO_ERR_ARG;
+    if (!fo_consumes_norm_rows(bs, dim, BN, 1) || dim % BN || bs % BM || ((uintptr_t)acc & 15)) return FO_ERR_SHAPE;
+    if (nrows == 0 && !info) return FO_OK;
+    const unsigned x_bytes = (unsigned)((int64_t)bs * dim * 2);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+#define FO_CONSUME(TAG_, STREAM_)                                                                                        \
+    launch_norm_rows_on<TAG_, STREAM_, NORM_SLOTS, true>(X, Y, Wt, row0, nrows, dim, BM, BN, 1, RA, eps, beside_gemm, 0, \
+                                                         x_bytes, s, info, acc)
+    if (dtype == FO_F16) return stream_rows ? FO_CONSUME(fo_f16_tag, true) : FO_CONSUME(fo_f16_tag, false);
+    if (dtype == FO_BF16) return stream_rows ? FO_CONSUME(fo_bf16_tag, true) : FO_CONSUME(fo_bf16_tag, false);
+#undef FO_CONSUME
     return FO_ERR_DTYPE;
 }
 

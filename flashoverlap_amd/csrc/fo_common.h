@@ -172,6 +172,14 @@ int fo_wait_reduce_groups_with(int dtype, const void *C, void *ACC, int32_t *MM,
 int fo_norm_rows_with(int dtype, const void *X, void *Y, const void *Wt, int row0, int nrows, int bs, int dim, int BM,
                       int BN, int rldn, const int32_t *RA, float eps, bool stream_rows, bool beside_gemm, int grid,
                       fo_stream_t stream, int32_t *info = nullptr);
+// The same with the consumer's work on these rows: acc[o] = round16(acc[o] + X[o]) wherever they lie (rldn == 1, BN a power
+// of two, rows of at most 8192 elements; acc 16-byte aligned and apart from X, Y and Wt).
+inline bool fo_consumes_norm_rows(int64_t bs, int dim, int BN, int rldn) {
+    return rldn == 1 && BN % 8 == 0 && (BN & (BN - 1)) == 0 && dim % 8 == 0 && dim <= 8192 && bs * dim * 2 <= 0x7FFFFFFFLL;
+}
+int fo_consume_norm_rows_with(int dtype, const void *X, void *acc, void *Y, const void *Wt, int row0, int nrows, int bs, int dim,
+                              int BM, int BN, const int32_t *RA, float eps, bool stream_rows, bool beside_gemm,
+                              fo_stream_t stream, int32_t *info = nullptr);
 
 // The waits with their bound and status word chosen by the caller (fo_aux.hip).
 // max_polls < 0: the bound of the environment variable FO_WAIT_MAX_POLLS (none

@@ -409,16 +409,29 @@ int last_slots(const int32_t *RA_host, int TM, int TN, std::vector<long> &last_s
     return FO_OK;
 }
 
+// Whether a batch that fills the storage slots [done, done + tiles) is exactly the tile rows `runs` it completes: then one
+// kernel consumes and normalises them, and reads C once for both.  Its registers fit beside the GEMM as the row kernel's do.
+// 8192x8192, bf16, K = 3584: a quarter's consumer and rows took 61 + 30 to 55 us beside the GEMM, more than the 95 us of a
+// wave of it, so that the consumer stream fell behind; together 71, and 28 instead of 17 + 12 and a launch behind the last
+// wave (whole call 409.9 -> 396.8 us; K = 8192, fp16, whose waves are long enough for both, the same within its noise).
+bool whole_rows(const int32_t *RA_host, int TN, const std::vector<int> &runs, long done, long tiles) {
+    long rows = 0;
+    for (size_t k = 0; k + 1 < runs.size(); k += 2) {
+        rows += runs[k + 1] - runs[k];
+        for (long t = (long)runs[k] * TN; t < (long)runs[k + 1] * TN; t++)
+            if (RA_host[t] < done) return false;  // the rows' largest slot lies in the batch: asked before
+    }
+    return rows * TN == tiles;
+}
+
 int check_slots(const int32_t *RA_host, int T) {  // FO_ERR_ARG for an entry outside [0, T)
     uint32_t most = 0;
     for (int t = 0; t < T; t++) most = (uint32_t)RA_host[t] > most ? (uint32_t)RA_host[t] : most;
     return most < (uint32_t)T ? FO_OK : FO_ERR_ARG;
 }
 
-int norm_ready_rows(const norm_plan &np, long *last_slot, int TM, long done, bool final_batch, int dtype, const void *C,
-                    int M, int N, int BM, int BN, int rLDN, const int32_t *RA, bool beside_gemm, fo_stream_t stream) {
-    std::vector<int> runs;
-    ready_tile_rows(last_slot, TM, done, final_batch, runs);
+int norm_runs(const norm_plan &np, const std::vector<int> &runs, int dtype, const void *C, int M, int N, int BM, int BN, int rLDN,
+              const int32_t *RA, bool beside_gemm, fo_stream_t stream) {
     for (size_t k = 0; k + 1 < runs.size(); k += 2) {
         int rc = norm_tile_rows(np, dtype, C, M, N, BM, BN, rLDN, RA, runs[k], runs[k + 1], beside_gemm, stream);
         if (rc) return rc;
@@ -513,6 +526,8 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
         long done = 0;
         uint16_t *c = static_cast<uint16_t *>(C);
         uint16_t *acc = static_cast<uint16_t *>(h->acc);
+        const bool consumes_rows = np && acc && !same_stream && h->link_bytes_per_s <= 0 && fo_consumes_norm_rows(M, N, info[1], rLDN) &&
+                                   apart({acc, mn}, {{C, mn}, {np->Y, mn}, {np->Wt, N}});
         for (int i = 0; i < G;) {
             const int j = batch_end(cseg_host, G, i, done, wave);
             long tiles = 0;
@@ -524,7 +539,10 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
                                 : fo_wait_groups_with(j - i, cseg_dev + i, MM + i, h->max_polls, gave_up, cstream);
                 if (rc) return rc;
             }
-            if (acc && !consumed) {  // the groups of a batch are one contiguous range
+            std::vector<int> runs;
+            if (np && !same_stream) ready_tile_rows(last_slot.data(), TM, done + tiles, j == G, runs);
+            const bool with_rows = consumes_rows && whole_rows(np->RA_host, TN, runs, done, tiles);
+            if (acc && !consumed && !with_rows) {  // the groups of a batch are one contiguous range
                 rc = fo_consumer_reduce_with(dtype, c + off, acc + off, n, 1, 0, nullptr, 0, stream_acc, cstream,
                                              j < G && !same_stream);  // every batch but the last runs beside the GEMM
                 if (rc) return rc;
@@ -536,9 +554,14 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
             if (np && same_stream) {
                 rc = norm_tile_rows(*np, dtype, C, M, N, info[0], info[1], rLDN, RA, 0, TM, false, cstream);
                 if (rc) return rc;
+            } else if (with_rows) {
+                for (size_t k = 0; k + 1 < runs.size(); k += 2) {
+                    rc = fo_consume_norm_rows_with(dtype, C, acc, np->Y, np->Wt, runs[k] * info[0], (runs[k + 1] - runs[k]) * info[0], M, N,
+                                                   info[0], info[1], RA, np->eps, fo_streams(mn * 4), j < G, cstream);
+                    if (rc) return rc;
+                }
             } else if (np) {
-                rc = norm_ready_rows(*np, last_slot.data(), TM, done, j == G, dtype, C, M, N, info[0], info[1], rLDN, RA,
-                                     j < G, cstream);
+                rc = norm_runs(*np, runs, dtype, C, M, N, info[0], info[1], rLDN, RA, j < G, cstream);
                 if (rc) return rc;
             }
             i = j;

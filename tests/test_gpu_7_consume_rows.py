@@ -1,0 +1,37 @@
+"""GPU parity of the kernel that updates the accumulator and normalises the same rows: batches that are whole tile rows and
+batches that are not, rows that fill the workgroup's lanes and rows that do not, one batch and several.  Everything the
+call leaves is compared bit for bit with the separate calls (see _run_both)."""
+import numpy as np
+import pytest
+
+from gpu_util import BF16, F16
+from test_gpu_3_norm_overlap import _run_both
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("bm,bn,M,N,cseg", [
+    (128, 128, 8192, 4096, [512] * 4),               # two waves of whole rows
+    (128, 128, 8192, 4096, [100, 412, 512, 1024]),   # groups that end inside rows
+    (128, 256, 8192, 8192, [256] * 8),               # four waves, two groups each
+    (256, 128, 4096, 8192, [1024]),                  # one group
+    (128, 256, 256, 6144, [48]),                     # three chunks a lane
+    (128, 128, 256, 1920, [10, 20]),                 # one chunk, lanes left over
+    (128, 128, 384, 4224, [33, 66]),                 # three chunks, most of the third beyond the row
+    (128, 256, 128, 256, [1]),                       # one tile
+])
+def test_rows_are_consumed_and_normalised(fo, dtype, bm, bn, M, N, cseg):
+    _run_both(fo, dtype, bm, bn, M, N, 72, cseg, 0, seed=700)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+def test_rows_in_another_order(fo, dtype):
+    """Whole rows in an order of their own, and rows spread over two batches."""
+    bm, bn, M, N = 128, 128, 8192, 4096
+    TM, TN = M // bm, N // bn
+    rng = np.random.default_rng(3)
+    rows = [t for half in (0, 1) for tm in rng.permutation(TM // 2) + half * (TM // 2) for t in rng.permutation(TN) + tm * TN]
+    _run_both(fo, dtype, bm, bn, M, N, 64, [TM * TN // 2] * 2, 0, seed=710, hint=[int(t) for t in rows])
+    spread = rng.permutation(TM * TN)
+    _run_both(fo, dtype, bm, bn, M, N, 64, [TM * TN // 2] * 2, 0, seed=711, hint=[int(t) for t in spread])

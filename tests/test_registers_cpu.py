@@ -36,3 +36,24 @@ def test_a_consumer_fits_beside_the_kernels_that_count(tmp_path):
             assert int(re.search(r"\.vgpr_spill_count: +(\d+)", rest).group(1)) == 0, name
             seen += 1
     assert seen == 2 * 2 * (11 + 8 + 1)  # types, epilogues; tiles, their shifted forms, the 256x256 kernel
+
+
+def test_the_kernel_that_consumes_and_normalises_fits_beside_the_signalling_gemm(tmp_path):
+    if not os.path.exists(os.path.join(LLVM, "llvm-readelf")):
+        pytest.skip("no llvm-readelf beside hipcc")
+    shutil.copy2(_capi.KERNEL_LIB, tmp_path / "lib.so")
+    subprocess.run([os.path.join(LLVM, "llvm-objdump"), "--offloading", "lib.so"], cwd=tmp_path, check=True,
+                   stdout=subprocess.DEVNULL)
+    gemm, rows = [], []
+    for part in sorted(p for p in os.listdir(tmp_path) if p.endswith(build.ARCH)):
+        notes = subprocess.run([os.path.join(LLVM, "llvm-readelf"), "--notes", part], cwd=tmp_path, check=True,
+                               capture_output=True, text=True).stdout
+        for name, rest in re.findall(r"\.name: +(\S+)\n(.*?\.vgpr_spill_count: +\d+)", notes, re.S):
+            registers = -(-int(re.search(r"\.vgpr_count: +(\d+)", rest).group(1)) // 8) * 8
+            if re.search(r"fo_gemm256_kernelI\w+_tagLi1E", name):
+                gemm.append(registers)
+            if re.search(r"fo_norm_rows_kernelI\w+_tagLi\dELb\dELi\dELb1E", name):
+                rows.append(registers)
+                assert int(re.search(r"\.vgpr_spill_count: +(\d+)", rest).group(1)) == 0, name
+    assert len(gemm) == 2 and len(rows) == 2 * 2 * 4  # types, cache policies, chunks a lane
+    assert max(gemm) + max(rows) <= SIMD
