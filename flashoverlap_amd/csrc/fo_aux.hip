@@ -140,6 +140,7 @@ __device__ __forceinline__ void reduce_range(const fo_u32x4 *src, fo_u32x4 *dst,
                 __builtin_nontemporal_store(v, d);
             else
                 *d = v;
+            __builtin_amdgcn_sched_barrier(0);  // one piece's sums at a time: all of them in bf16 are more than 64 registers
         }
 #pragma unroll
         for (int u = 0; u < U; u++) keep(i + (long)u * nthreads, a[u]);
@@ -317,9 +318,7 @@ template <> struct norm_math<fo_f16_tag> {
         for (int k = 0; k < 4; k++) {
             const uint32_t u = v[k], uw = w[k];
             const h2 p = __builtin_bit_cast(h2, u);
-            h2 q;
-            q.x = (_Float16)((float)p.x * s);
-            q.y = (_Float16)((float)p.y * s);
+            const h2 q = __builtin_bit_cast(h2, fo_elem<fo_f16_tag>::pack((float)p.x * s, (float)p.y * s));
             const h2 y = q * __builtin_bit_cast(h2, uw);
             o[k] = __builtin_bit_cast(uint32_t, y);
         }
@@ -329,6 +328,8 @@ template <> struct norm_math<fo_f16_tag> {
 template <> struct norm_math<fo_bf16_tag> {
     typedef __bf16 b2 __attribute__((ext_vector_type(2)));
     typedef fo_elem<fo_bf16_tag> E;
+    static __device__ __forceinline__ float lo(uint32_t u) { return __builtin_bit_cast(float, u << 16); }
+    static __device__ __forceinline__ float hi(uint32_t u) { return __builtin_bit_cast(float, u & 0xffff0000u); }
     static __device__ __forceinline__ float sumsq(fo_u32x4 v, float acc) {
 #pragma unroll
         for (int k = 0; k < 4; k++) {
@@ -343,11 +344,8 @@ template <> struct norm_math<fo_bf16_tag> {
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             const uint32_t u = v[k], uw = w[k];
-            const float lo = E::to_f32(E::from_f32(E::to_f32((uint16_t)(u & 0xffff)) * s));
-            const float hi = E::to_f32(E::from_f32(E::to_f32((uint16_t)(u >> 16)) * s));
-            const uint16_t ylo = E::from_f32(lo * E::to_f32((uint16_t)(uw & 0xffff)));
-            const uint16_t yhi = E::from_f32(hi * E::to_f32((uint16_t)(uw >> 16)));
-            o[k] = (uint32_t)ylo | ((uint32_t)yhi << 16);
+            const uint32_t q = E::pack(lo(u) * s, hi(u) * s);
+            o[k] = E::pack(lo(q) * lo(uw), hi(q) * hi(uw));
         }
         return o;
     }
@@ -564,7 +562,7 @@ int launch_rmsnorm(const void *X, void *Y, const void *Wt, int bs, int dim, int 
 // is read once for both (ACC is laid out as X).  The accumulator's chunks are requested when the row before is done with and
 // used last; up to 128 registers, which fit beside the signalling GEMM's wavefront (384).
 template <typename Tag, int CH, bool STREAM, int PATH, bool ADD>
-__global__ __launch_bounds__(256, (!ADD && CH <= 4 && !(CH == 4 && std::is_same<Tag, fo_bf16_tag>::value)) ? 5 : 4) void fo_norm_rows_kernel(const fo_u32x4 *X, fo_u32x4 *Y, const fo_u32x4 *Wt,
+__global__ __launch_bounds__(256, !ADD && CH <= 4 ? 5 : 4) void fo_norm_rows_kernel(const fo_u32x4 *X, fo_u32x4 *Y, const fo_u32x4 *Wt,
                                                               int row0, int nrows, int rows_per_wg, int dim, int BM,
                                                               int BN, int rldn, const int32_t *RA, float eps,
                                                               unsigned x_bytes, fo_u32x4 *ACC) {
@@ -667,7 +665,7 @@ __global__ __launch_bounds__(256, (!ADD && CH <= 4 && !(CH == 4 && std::is_same<
         yr.w = 0x00027000u;
 #pragma unroll
         for (int i = 0; i < CH; i++) {
-            if (ADD) asm volatile("" : "+v"(w[i]));  // bf16: its conversions to 32 bits are made for each row, not kept in twice the registers
+            if (ADD || std::is_same<Tag, fo_bf16_tag>::value) asm volatile("" : "+v"(w[i]));  // bf16: its conversions to 32 bits are made for each row, not kept in twice the registers
             const fo_u32x4 y = MATH::scale(x[i], s, w[i]);
             if (STREAM)
                 asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen nt\n\ts_nop 1"

@@ -582,13 +582,9 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                 for (int j = 0; j < F; j++) {
                     fo_float4v a4 = acc[i][j];
                     asm volatile("" : "+a"(a4));  // leaves the accumulation registers here, not in one sweep in front of the epilogue
-                    uint16_t h0 = E::from_f32(a4[0]);
-                    uint16_t h1 = E::from_f32(a4[1]);
-                    uint16_t h2 = E::from_f32(a4[2]);
-                    uint16_t h3 = E::from_f32(a4[3]);
                     fo_u32x2 v;
-                    v.x = (uint32_t)h0 | ((uint32_t)h1 << 16);
-                    v.y = (uint32_t)h2 | ((uint32_t)h3 << 16);
+                    v.x = E::pack(a4[0], a4[1]);
+                    v.y = E::pack(a4[2], a4[3]);
                     *reinterpret_cast<fo_u32x2 *>(strip + erow * PITCH + j * 16 + ek * 4) = v;
                 }
                 // the strip is private to this wavefront: order its LDS writes before its reads

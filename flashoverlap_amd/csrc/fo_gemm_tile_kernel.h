@@ -576,8 +576,8 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
 #pragma unroll
                 for (int j = 0; j < FN; j++) {
                     fo_u32x2 v;
-                    v.x = (uint32_t)E::from_f32(acc[i][j][0]) | ((uint32_t)E::from_f32(acc[i][j][1]) << 16);
-                    v.y = (uint32_t)E::from_f32(acc[i][j][2]) | ((uint32_t)E::from_f32(acc[i][j][3]) << 16);
+                    v.x = E::pack(acc[i][j][0], acc[i][j][1]);
+                    v.y = E::pack(acc[i][j][2], acc[i][j][3]);
                     *reinterpret_cast<fo_u32x2 *>(stage + (wm * WTM + i * 16 + erow) * PITCH + wn * WTN + j * 16 + ek * 4) = v;
                 }
             if constexpr (ACC) {
