@@ -36,12 +36,20 @@ enum {
 //
 // kRsEpilogueBelowFlop, kFewCopies: see fo_overlap_gemm_reducescatter.  They are no thresholds of a handle.
 //
+// kTogetherUpToK: up to this K the batches beside the GEMM are consumed and normalised by one kernel (whole_rows below).  A
+// wave of a longer GEMM lasts long enough for the consumer and the rows one after the other, and a consumer of one
+// wavefront per CU takes less from the GEMM (8192x8192, four waves, whole call, us, one after the other and together:
+// fp16 K = 2048 281 and 271, 4096 450 and 447, 6656 684 and 682, 8192 818 and 823; bf16 273 and 261, 433 and 429, 657 and 653,
+// 781 and 784).  Behind the GEMM the one kernel is the faster in any case (K = 8192 780.9 -> 776.5; 4096x8192x4096 238.2 ->
+// 233.4).
+//
 // kGemmFlopPerNs: what a GEMM is expected to sustain, for sizing the pause
 // between polls only.
 constexpr int kFusedFromGroups = 16;
 constexpr double kInStreamBelowFlop = 6.4e10;
 constexpr double kRsEpilogueBelowFlop = 5e11;
 constexpr int kFewCopies = 16, kFewCopiesOfShort = 6;
+constexpr int kTogetherUpToK = 6144;
 constexpr double kGemmFlopPerNs = 1.2e6;
 
 }  // namespace
@@ -413,7 +421,7 @@ int last_slots(const int32_t *RA_host, int TM, int TN, std::vector<long> &last_s
 // kernel consumes and normalises them, and reads C once for both.  Its registers fit beside the GEMM as the row kernel's do.
 // 8192x8192, bf16, K = 3584: a quarter's consumer and rows took 61 + 30 to 55 us beside the GEMM, more than the 95 us of a
 // wave of it, so that the consumer stream fell behind; together 71, and 28 instead of 17 + 12 and a launch behind the last
-// wave (whole call 409.9 -> 396.8 us; K = 8192, fp16, whose waves are long enough for both, the same within its noise).
+// wave (whole call 409.9 -> 396.8 us).
 bool whole_rows(const int32_t *RA_host, int TN, const std::vector<int> &runs, long done, long tiles) {
     long rows = 0;
     for (size_t k = 0; k + 1 < runs.size(); k += 2) {
@@ -541,7 +549,7 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
             }
             std::vector<int> runs;
             if (np && !same_stream) ready_tile_rows(last_slot.data(), TM, done + tiles, j == G, runs);
-            const bool with_rows = consumes_rows && whole_rows(np->RA_host, TN, runs, done, tiles);
+            const bool with_rows = consumes_rows && (j == G || K <= kTogetherUpToK) && whole_rows(np->RA_host, TN, runs, done, tiles);
             if (acc && !consumed && !with_rows) {  // the groups of a batch are one contiguous range
                 rc = fo_consumer_reduce_with(dtype, c + off, acc + off, n, 1, 0, nullptr, 0, stream_acc, cstream,
                                              j < G && !same_stream);  // every batch but the last runs beside the GEMM
