@@ -11,6 +11,7 @@
 // Functions that enqueue return the C ABI's error code; the layer functions return the output tensor, and raise what
 // the C ABI refuses: a second call by another path could enqueue twice.
 #include <ATen/ATen.h>
+#include <ATen/ops/empty_native.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/record_function.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -264,6 +265,12 @@ PyObject *reorder_rmsnorm(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
     END_HANDLE_TH_ERRORS
 }
 
+// An output of a layer's call: what at::empty comes to once nobody follows the operators (asked before), without its way
+// through the dispatcher (host time of the two layers of a decode step 10.1 -> 9.6 us).
+at::Tensor output(at::IntArrayRef sizes, const at::Tensor &like) {
+    return at::native::empty_cuda(sizes, like.scalar_type(), at::kStrided, like.device(), false, std::nullopt);
+}
+
 // The output of a layer's call, or the error that the registered classes and operators raise for that code.
 PyObject *output_of(int rc, const char *what, const at::Tensor &t) {
     TORCH_CHECK(rc == 0, "flashoverlap: ", what, " failed: ", fo_error_string(rc), " (code ", rc, ")");
@@ -280,7 +287,7 @@ PyObject *allreduce_layer(PyObject *, PyObject *const *argv, Py_ssize_t argc) {
     s.MM = in.tensor(), s.RA = in.tensor(), s.cseg_cpu = in.tensor(), s.cseg_gpu = in.tensor(), s.algo = in.int32();
     Product p;
     if (followed() || !in.done() || !p.fits(*A, *B) || !s.fits(p, nullptr, nullptr, 1)) Py_RETURN_NONE;
-    const at::Tensor out = at::empty({p.M, p.N}, A->options());
+    const at::Tensor out = output({p.M, p.N}, *A);
     const int rc = enqueue([&] {
         return fo_overlap_gemm_allreduce(h, dtype_of(*A), p.M, p.N, p.K, A->data_ptr(), B->data_ptr(), out.data_ptr(), ints(*s.MM),
                                          ints(*s.RA), s.TM(), s.TN(), 1, ints(*s.cseg_cpu), ints(*s.cseg_gpu), s.G(), s.algo, 0);
@@ -302,7 +309,7 @@ PyObject *reducescatter_layer(PyObject *, PyObject *const *argv, Py_ssize_t argc
     const int64_t W = in.integer();
     Product p;
     if (followed() || !in.done() || !p.fits(*A, *B) || W <= 0 || p.M % W || !s.fits(p, RE, nullptr, W)) Py_RETURN_NONE;
-    const at::Tensor all = at::empty({p.M, p.N}, A->options()), out = at::empty({p.M / W, p.N}, A->options());
+    const at::Tensor all = output({p.M, p.N}, *A), out = output({p.M / W, p.N}, *A);
     const int rc = enqueue([&] {
         return fo_overlap_gemm_reducescatter(h, dtype_of(*A), p.M, p.N, p.K, A->data_ptr(), B->data_ptr(), all.data_ptr(),
                                              out.data_ptr(), ints(*s.MM), ints(*s.RA), ints(*RE), s.TM(), s.TN(), 1,
@@ -321,7 +328,7 @@ PyObject *reorder_rmsnorm_layer(PyObject *, PyObject *const *argv, Py_ssize_t ar
     const at::Tensor *RA = in.tensor();
     const double eps = in.real();
     if (followed() || !in.done() || !norm_fits(*X, *Wt, BM, BN, *RA)) Py_RETURN_NONE;
-    const at::Tensor out = at::empty(X->sizes(), X->options());
+    const at::Tensor out = output(X->sizes(), *X);
     return output_of(norm_on_current(*X, out, *Wt, BM, BN, 1, *RA, eps), "reorder_rmsnorm", out);
     END_HANDLE_TH_ERRORS
 }
