@@ -535,7 +535,8 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
         uint16_t *c = static_cast<uint16_t *>(C);
         uint16_t *acc = static_cast<uint16_t *>(h->acc);
         const bool consumes_rows = np && acc && !same_stream && h->link_bytes_per_s <= 0 && fo_consumes_norm_rows(M, N, info[1], rLDN) &&
-                                   apart({acc, mn}, {{C, mn}, {np->Y, mn}, {np->Wt, N}});
+                                   apart({acc, mn}, {{C, mn}, {np->Y, mn}, {np->Wt, N}}) &&
+                                   apart({np->Y, mn}, {{C, mn}});  // the accumulator takes the product, not rows written over it
         for (int i = 0; i < G;) {
             const int j = batch_end(cseg_host, G, i, done, wave);
             long tiles = 0;
