@@ -3,8 +3,9 @@ batches that are not, rows that fill the workgroup's lanes and rows that do not,
 call leaves is compared bit for bit with the separate calls (see _run_both)."""
 import numpy as np
 import pytest
+import torch
 
-from gpu_util import BF16, F16
+from gpu_util import BF16, F16, TORCH_DTYPE
 from test_gpu_3_norm_overlap import _run_both
 
 pytestmark = pytest.mark.gpu
@@ -35,3 +36,22 @@ def test_rows_in_another_order(fo, dtype):
     _run_both(fo, dtype, bm, bn, M, N, 64, [TM * TN // 2] * 2, 0, seed=710, hint=[int(t) for t in rows])
     spread = rng.permutation(TM * TN)
     _run_both(fo, dtype, bm, bn, M, N, 64, [TM * TN // 2] * 2, 0, seed=711, hint=[int(t) for t in spread])
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("bm,bn,M,N", [(96, 128, 192, 1024), (1, 64, 5, 320), (16, 256, 48, 2048), (24, 32, 72, 96)])
+def test_tile_heights(fo, dtype, bm, bn, M, N):
+    """Tile heights that are powers of two (shifts) and that are not (divisions), against the plain rows: the same bits."""
+    td = TORCH_DTYPE[dtype]
+    T = (M // bm) * (N // bn)
+    hint = [int(t) for t in np.random.default_rng(5).permutation(T)]
+    RA = fo.layout.reorder_indices(T, hint, device="cuda").reshape(M // bm, N // bn)
+    g = torch.Generator(device="cuda").manual_seed(6)
+    C = torch.randn(M, N, device="cuda", generator=g).to(td)
+    W = torch.randn(N, device="cuda", generator=g).to(td)
+    Y, Z = torch.empty_like(C), torch.empty_like(C)
+    fo.ops.reorder_rmsnorm_rows(C, Y, W, 0, M, bm, bn, 1, RA, eps=1e-6)
+    plain = fo.layout.unpermute(C, M, N, bm, bn, RA).contiguous()
+    fo.ops.reorder_rmsnorm_rows(plain, Z, W, 0, M, 1, 8, 1, None, eps=1e-6)
+    torch.cuda.synchronize()
+    assert torch.equal(Y, Z)
