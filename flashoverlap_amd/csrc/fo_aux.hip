@@ -545,7 +545,10 @@ int launch_rmsnorm(const void *X, void *Y, const void *Wt, int bs, int dim, int 
     // Rows of exactly 8192 elements fill the row kernel's workgroup (four wavefronts per row, four chunks per
     // lane), and there it is the faster of the two: 8192 x 8192, nothing cached, 45.5-46.7 us against 47-50
     // (fp16 and bf16, reorder or not).  Narrower rows leave its lanes idle (16384 x 1024: 15.5 against 11.8 us)
-    // and longer ones cost it its look-ahead.
+    // and longer ones cost it its look-ahead.  More than 4096 elements fill the three or four chunks a lane well enough as long as
+    // the caches hold the matrix (us, a wavefront a row / a workgroup a row, bf16 reordered: 4096 x 4608 17.7 / 16.4, 3072 x 6144
+    // 17.9 / 15.8, 4224 x 7168 29.2 / 27.2, fp16 28.2 / 26.5; the whole pass around the last 185.9 -> 184.9, 6272 x 5888 223.1 ->
+    // 222.3); streamed they do not (8192 x 7168 44.9 / 45.4, 16384 x 6144 74.0 / 76.0), nor do 4096 (8192 rows 27.2 / 28.1).
     // Few rows: one wavefront per row leaves most of the chip idle (128 rows: 32 workgroups) and is a chain of up to
     // sixteen loads, sums and stores; a workgroup per row is four times as many wavefronts and a quarter of the chain.
     // Reordered input, us, before -> after (fp16 / bf16): 128 x 4096 3.43 -> 2.71 / 3.90 -> 2.84, 512 x 7168 5.71 -> 4.35
@@ -553,7 +556,8 @@ int launch_rmsnorm(const void *X, void *Y, const void *Wt, int bs, int dim, int 
     // wavefront wins again: 4096 x 4096 11.4 against 12.1, and with rows of up to 2048 elements, which leave half of
     // the workgroup's lanes idle, from 1152 rows on (1024 elements 3.0 against 3.6).
     const bool few = dim <= 8192 && bs <= few_norm_rows(dim);
-    if (few || (dim == 8192 && (int64_t)bs * dim * 2 <= 0xFFFFFFFFLL))
+    const bool wide = dim > 4096 && dim <= 8192 && !fo_streams((int64_t)bs * dim * 4);
+    if (few || wide || (dim == 8192 && (int64_t)bs * dim * 2 <= 0xFFFFFFFFLL))
         return fo_norm_rows_with(std::is_same<Tag, fo_bf16_tag>::value ? FO_BF16 : FO_F16, X, Y, Wt, 0, bs, bs, dim, BM,
                                  BN, rldn, RA, eps, fo_streams((int64_t)bs * dim * 4), false, 0, stream);
     // input and output together against the cache that would have to hold them

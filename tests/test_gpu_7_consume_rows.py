@@ -55,3 +55,23 @@ def test_tile_heights(fo, dtype, bm, bn, M, N):
     fo.ops.reorder_rmsnorm_rows(plain, Z, W, 0, M, 1, 8, 1, None, eps=1e-6)
     torch.cuda.synchronize()
     assert torch.equal(Y, Z)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("M,N", [(2176, 4224), (2304, 7168), (2176, 4096)])
+def test_many_wide_rows(fo, dtype, M, N):
+    """More rows than get a workgroup each, on both sides of the width from which they are a workgroup's anyhow: at most two
+    units in the last place from a sum in 64 bits (one for each of the two roundings, neither of which can be off by more)."""
+    td, bn = TORCH_DTYPE[dtype], 128
+    g = torch.Generator(device="cuda").manual_seed(8)
+    C = torch.randn(M, N, device="cuda", generator=g).to(td)
+    W = torch.randn(N, device="cuda", generator=g).to(td)
+    T = (M // 128) * (N // bn)
+    RA = fo.layout.reorder_indices(T, [int(t) for t in np.random.default_rng(9).permutation(T)], device="cuda").reshape(M // 128, N // bn)
+    Y = torch.empty_like(C)
+    fo.ops.reorder_rmsnorm(C, Y, W, 128, bn, 1, RA, eps=1e-6)
+    x = fo.layout.unpermute(C, M, N, 128, bn, RA).double()
+    want = x * torch.rsqrt(x.pow(2).mean(1, keepdim=True) + 1e-6) * W.double()
+    ulp = 2.0 ** -10 if dtype == F16 else 2.0 ** -7
+    torch.cuda.synchronize()
+    assert ((Y.double() - want).abs() <= 2 * ulp * want.abs() + 2.0 ** -23).all()
