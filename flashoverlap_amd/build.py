@@ -38,7 +38,7 @@ ARCH = "gfx950"
 
 KERNEL_SOURCES = ["fo_gemm.hip", "fo_aux.hip", "fo_algo.cpp", "fo_overlap.cpp"]
 # fo_gemm256_inst.hip and fo_gemm_tile_inst.hip hold the instantiations of the GEMM kernels for one dtype (fp16 / bf16)
-# and one epilogue (plain / signal / scatter / accumulating / reduce-scatter) per compilation; they take up to minutes, so they are separate jobs.
+# and one epilogue (plain / signal / scatter / accumulating / reduce-scatter) per compilation; separate jobs, for a build on many cores.
 GEMM_INSTANCES = [(src, d, m) for src in ("fo_gemm256_inst.hip", "fo_gemm_tile_inst.hip") for d in (0, 1) for m in (0, 1, 2, 3, 4)]
 
 # -packed-fp32-ops off: hipcc must not form v_pk_*_f32 from the float code here.
@@ -46,8 +46,6 @@ HIP_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-x", "hip",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
-    # the K step of the 256x256 kernel is one fully unrolled body of 128 MFMAs built from nested constant loops
-    "-mllvm", "-pragma-unroll-threshold=1000000",
     "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
 ]
 

@@ -101,6 +101,35 @@ constexpr int loads_before_row256(int d) {
     return s;
 }
 
+// The LDS fetches of each row of a K step in issue order: A or B block `block`, k-step kk, from the step's slot or the next one's.
+struct fetch256 {
+    bool b;
+    int block, kk;
+    bool next;
+};
+struct row_fetches256 {
+    int n;
+    fetch256 at[6];
+};
+constexpr row_fetches256 fetches_of_row256(int r) {
+    row_fetches256 f{};
+    auto a = [&](int block, int kk, bool next = false) { f.at[f.n++] = {false, block, kk, next}; };
+    auto b = [&](int block, bool next = false) {
+        f.at[f.n++] = {true, block, 0, next};
+        f.at[f.n++] = {true, block, 1, next};
+    };
+    if (r == 0) { b(5); b(6); }
+    if (r == 1) { b(7); a(2, 0); a(2, 1); }
+    if (r == 2) { a(3, 0); a(3, 1); }
+    if (r == 4) { a(4, 0); a(4, 1); }
+    if (r == 5) { a(5, 0); a(5, 1); }
+    if (r == 8) { a(6, 0); a(6, 1); a(7, 0); a(7, 1); }
+    if (r == 13) { a(0, 0, true); a(0, 1, true); b(0, true); a(1, 0, true); a(1, 1, true); }
+    if (r == 14) { b(1, true); b(2, true); }
+    if (r == 15) { b(3, true); b(4, true); }
+    return f;
+}
+
 constexpr int kSmem256 = 2 * 65536 + 4 * 16 * (128 + 8) * 2;  // two slots + four strips of 16 padded rows
 
 template <typename Tag, int MODE>
@@ -235,16 +264,9 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             dma_buf16(rb, a_cur, soff_a[c & 7], (wa0 ^ slot) + c * CHUNK_B);
     };
     // the same riding on an MFMA (K loop)
-    auto mfma_load_chunk = [&](fo_u32x4 x, fo_u32x4 y, fo_float4v &cc, int c, unsigned lds_base) {
-        switch (c) {
-#define FO_CASE(C_)                                                                                           \
-    case C_:                                                                                                  \
-        X::template go_load<C_ * CHUNK_B>(x, y, cc, lds_base, C_ < 8 ? ra : rb, a_cur, soff_a[C_ & 7]);       \
-        break;
-            FO_CASE(0) FO_CASE(1) FO_CASE(2) FO_CASE(3) FO_CASE(4) FO_CASE(5) FO_CASE(6) FO_CASE(7)
-            FO_CASE(8) FO_CASE(9) FO_CASE(10) FO_CASE(11) FO_CASE(12) FO_CASE(13) FO_CASE(14) FO_CASE(15)
-#undef FO_CASE
-        }
+    auto mfma_load_chunk = [&](auto chunk, fo_u32x4 x, fo_u32x4 y, fo_float4v &cc, unsigned lds_base) __attribute__((always_inline)) {
+        constexpr int c = decltype(chunk)::value;
+        X::template go_load<c * CHUNK_B>(x, y, cc, lds_base, c < 8 ? ra : rb, a_cur, soff_a[c & 7]);
     };
 
     // ---- signalling state (signal and scatter epilogues)
@@ -378,10 +400,10 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     fo_float4v acc[F][F];
     fo_u32x4 af[2][2][2], bf[2][F];
     auto load_a = [&](int buf, unsigned base, int i, int kk) {
-        af[buf][i % 2][kk] = *reinterpret_cast<lds16_t>((base ^ (kk * KSTEP_X)) + i * BLOCK_B);
+        af[buf][i % 2][kk] = *reinterpret_cast<lds16_t>(base + i * BLOCK_B);
     };
     auto load_b = [&](unsigned base, int j, int kk) {
-        bf[kk][j] = *reinterpret_cast<lds16_t>((base ^ (kk * KSTEP_X)) + j * BLOCK_B);
+        bf[kk][j] = *reinterpret_cast<lds16_t>(base + j * BLOCK_B);
     };
 
     // ---- pipeline fill: stage 0 -> slot 0, stage 1 -> slot 1; the loader then stands at stage 1
@@ -396,9 +418,9 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int q = 0; q < 4; q++) load_a(0, la0, q / 2, q % 2);
+    for (int q = 0; q < 4; q++) load_a(0, la0 ^ (q % 2 * KSTEP_X), q / 2, q % 2);
 #pragma unroll
-    for (int q = 0; q < 10; q++) load_b(lb0, q / 2, q % 2);
+    for (int q = 0; q < 10; q++) load_b(lb0 ^ (q % 2 * KSTEP_X), q / 2, q % 2);
     sum_groups();  // the group sizes arrived before stage 0 did (requested earlier, vmcnt retires in issue order)
 
     int tile = blockIdx.x;
@@ -433,65 +455,43 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
         do {
             unsigned la_ = la0 ^ slot_b, lb_ = lb0 ^ slot_b;
             asm volatile("" : "+v"(la_), "+v"(lb_));
-            const unsigned lan = la_ ^ SLOT_B, lbn = lb_ ^ SLOT_B;
+            // by slot (the step's, the next step's) and k-step, found here: computed at each fetch, they stand between the MFMAs
+            const unsigned a_at[2][2] = {{la_, la_ ^ KSTEP_X}, {la_ ^ SLOT_B, la_ ^ SLOT_B ^ KSTEP_X}};
+            const unsigned b_at[2][2] = {{lb_, lb_ ^ KSTEP_X}, {lb_ ^ SLOT_B, lb_ ^ SLOT_B ^ KSTEP_X}};
             // load targets: this step's slot, the previous step's (wave-uniform by construction; said so for the assembly's scalar operands)
             const unsigned lds_cur = __builtin_amdgcn_readfirstlane(wa0 ^ slot_b), lds_prev = lds_cur ^ SLOT_B;
-#pragma unroll
-            for (int r = 0; r < ROWS; r++) {
-                const int strip = r / 4, next_a = (strip + 1) % 2;
-                // The row's LDS fetches in issue order; executes number t (none for t < 0), returns how many there are.
-                auto fetches = [&](int t) {
-                    int n = 0;
-                    auto fetch_a = [&](unsigned base, int i, int kk) {
-                        if (t == n) load_a(next_a, base, i, kk);
-                        n++;
-                    };
-                    auto fetch_b = [&](unsigned base, int j) {
-#pragma unroll
-                        for (int kk = 0; kk < 2; kk++) {
-                            if (t == n) load_b(base, j, kk);
-                            n++;
-                        }
-                    };
-                    if (r == 0) { fetch_b(lb_, 5); fetch_b(lb_, 6); }
-                    if (r == 1) { fetch_b(lb_, 7); fetch_a(la_, 2, 0); fetch_a(la_, 2, 1); }
-                    if (r == 2) { fetch_a(la_, 3, 0); fetch_a(la_, 3, 1); }
-                    if (r == 4) { fetch_a(la_, 4, 0); fetch_a(la_, 4, 1); }
-                    if (r == 5) { fetch_a(la_, 5, 0); fetch_a(la_, 5, 1); }
-                    if (r == 8) { fetch_a(la_, 6, 0); fetch_a(la_, 6, 1); fetch_a(la_, 7, 0); fetch_a(la_, 7, 1); }
-                    if (r == 13) { fetch_a(lan, 0, 0); fetch_a(lan, 0, 1); fetch_b(lbn, 0); fetch_a(lan, 1, 0); fetch_a(lan, 1, 1); }
-                    if (r == 14) { fetch_b(lbn, 1); fetch_b(lbn, 2); }
-                    if (r == 15) { fetch_b(lbn, 3); fetch_b(lbn, 4); }
-                    return n;
-                };
-                const int nops = fetches(-1);
+            static_for<ROWS>([&](auto row) __attribute__((always_inline)) {
+                constexpr int r = decltype(row)::value, strip = r / 4, next_a = (strip + 1) % 2;
+                constexpr row_fetches256 fetches = fetches_of_row256(r);
                 // The row's direct-to-LDS loads ride on MFMA 1 and, if there are two, MFMA 5.
-                const int d = r > FREE ? r - FREE - 1 : r + ROWS - FREE - 1;  // rows since the one behind FREE
-                const int dfirst = loads_before_row256(d);
-#pragma unroll
-                for (int m = 0; m < F; m++) {
-                    const int j = r % 4 * 2 + m / 4, h = (m / 2 % 2) ^ (j % 2), i = strip * 2 + h, kk = m % 2;
-                    int dc = -1;
-#pragma unroll
-                    for (int c = 0; c < 2; c++)
-                        if (c < loads_in_row256(d) && m == 1 + 4 * c) dc = c;
-                    if (dc >= 0)
-                        mfma_load_chunk(bf[kk][j], af[strip % 2][h][kk], acc[i][j], dfirst + dc, r > FREE ? lds_cur : lds_prev);
+                constexpr int d = r > FREE ? r - FREE - 1 : r + ROWS - FREE - 1;  // rows since the one behind FREE
+                static_for<F>([&](auto mfma) __attribute__((always_inline)) {
+                    constexpr int m = decltype(mfma)::value;
+                    constexpr int j = r % 4 * 2 + m / 4, h = (m / 2 % 2) ^ (j % 2), i = strip * 2 + h, kk = m % 2;
+                    constexpr int c = m / 4;
+                    if constexpr (m % 4 == 1 && c < loads_in_row256(d))
+                        mfma_load_chunk(std::integral_constant<int, loads_before_row256(d) + c>{}, bf[kk][j], af[strip % 2][h][kk], acc[i][j],
+                                        r > FREE ? lds_cur : lds_prev);
                     else
                         X::go(bf[kk][j], af[strip % 2][h][kk], acc[i][j]);
                     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int t = 0; t < 16; t++)
-                        if (t >= m * nops / F && t < (m + 1) * nops / F) fetches(t);
+                    constexpr int first = m * fetches.n / F, last = (m + 1) * fetches.n / F;
+                    static_for<last - first>([&](auto nth) __attribute__((always_inline)) {
+                        constexpr fetch256 f = fetches.at[first + decltype(nth)::value];
+                        if constexpr (f.b)
+                            load_b(b_at[f.next][f.kk], f.block, f.kk);
+                        else
+                            load_a(next_a, a_at[f.next][f.kk], f.block, f.kk);
+                    });
                     __builtin_amdgcn_sched_barrier(0);
-                }
-                if (r == FREE) {
+                });
+                if constexpr (r == FREE) {
                     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wavefront's fetches from the step's slot have returned
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" ::: "memory");
                     advance_loader();
                 }
-                if (r == PUB) {
+                if constexpr (r == PUB) {
                     // The stage the next step reads has landed; younger and allowed in flight: this step's YOUNG loads.
                     // In a tile's first step the wait also covers the previous tile's stores: part of the stage's
                     // loads was requested behind them (rows 0-6), and vmcnt retires in issue order.
@@ -500,7 +500,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                     asm volatile("" ::: "memory");
                 }
                 __builtin_amdgcn_sched_barrier(0);
-            }
+            });
             slot_b ^= SLOT_B;
         } while (++kt < kt_stop);
             if (!COUNTS || owed == 0) break;

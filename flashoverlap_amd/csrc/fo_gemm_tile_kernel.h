@@ -87,6 +87,43 @@ constexpr int tile_smem_bytes() {
     return S * (TM + TN) * BK * 2 > TM * (TN + 8) * 2 ? S * (TM + TN) * BK * 2 : TM * (TN + 8) * 2;
 }
 
+// What a computing wavefront's K step is made of: FL x FS accumulator blocks, KK k-steps.
+template <int FL, int FS, int KK>
+struct tile_step {
+    static constexpr int NB = FL * FS, LEAD_B = FL % 2 * FS;  // blocks, of those in a first strip of one
+    static constexpr int NS = (FL + 1) / 2;                   // strips; an odd one out is a strip of its own, the first
+    static constexpr int NF = (FL + FS) * KK, NM = NB * KK;   // fetches of a stage and MFMAs of a step
+    // The blocks in their order: strips of two long fragments by all short ones, one operand changing from block to block.
+    struct block { int i, j; };
+    static constexpr block block_at(int c) {
+        if (c < LEAD_B) return block{0, c};
+        const int e = c - LEAD_B, j = e % (2 * FS) / 2;
+        return block{FL % 2 + e / (2 * FS) * 2 + ((e & 1) ^ (j & 1)), j};
+    }
+    // The fragments of a stage in the order in which its blocks want them.
+    struct fetch { bool is_long; int at, kk; };
+    struct fetch_order { fetch nth[NF]; };
+    static constexpr fetch_order fetches() {
+        fetch_order f{};
+        bool have_l[FL] = {}, have_s[FS] = {};
+        int n = 0;
+        for (int c = 0; c < NB; c++) {
+            const block x = block_at(c);
+            for (int kk = 0; kk < KK; kk++) {
+                if (!have_s[x.j]) f.nth[n++] = fetch{false, x.j, kk};
+                if (!have_l[x.i]) f.nth[n++] = fetch{true, x.i, kk};
+            }
+            have_s[x.j] = have_l[x.i] = true;
+        }
+        return f;
+    }
+    // `n` things spread evenly over `span` places: the first one at place w or behind it.
+    static constexpr int first_at(int w, int n, int span) {
+        const int t = w <= 0 ? 0 : (w * n + span - 1) / span;
+        return t < n ? t : n;
+    }
+};
+
 template <typename Tag, int TM, int TN, int BK, int S, int MODE, bool SHIFT>
 __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs args) {
     typedef fo_elem<Tag> E;
@@ -384,7 +421,8 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             const unsigned lb = lds0 + KB * A_BLK + (unsigned)((wn * WTN + frow) * 8 + (fk ^ key)) * 16;
             const unsigned l_lds = LONG_B ? lb : la, s_lds = LONG_B ? la : lb;
             typedef const __attribute__((address_space(3))) frag *lds_frag_t;
-            constexpr int NS = (FL + 1) / 2;  // strips; an odd one out is a strip of its own, the first
+            typedef tile_step<FL, FS, KK> T;
+            constexpr int NS = T::NS, NB = T::NB, NF = T::NF, NM = T::NM;
             // (Up to 224 registers in all, and a consumer's wavefront still fits on the SIMD beside this kernel's two.)
             constexpr bool AHEAD = (SHIFT || FL < 4) && (2 * KK * (FL + FS) + FL * FS) * 4 <= 192;
             static_assert(AHEAD || (FL >= 4 && FS >= 2), "a strip in front of the last one fetches the last short fragment");
@@ -405,11 +443,11 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             // Fragment i, k-step kk of the stage in `slot` (and, shifted, of the one in `next`).
             auto fetch_l = [&](frag &to, int i, int kk, unsigned slot, unsigned next) __attribute__((always_inline)) {
                 const unsigned at = (l_lds + block_of(kk, slot, next, L_BLK, l_shift)) ^ ((kk & 1) * 64);
-                to = *(lds_frag_t)(uintptr_t)(at + i * 2048);
+                to = ((lds_frag_t)(uintptr_t)at)[i * 128];
             };
             auto fetch_s = [&](frag &to, int j, int kk, unsigned slot, unsigned next) __attribute__((always_inline)) {
                 const unsigned at = (s_lds + block_of(kk, slot, next, S_BLK, s_shift)) ^ ((kk & 1) * 64);
-                to = *(lds_frag_t)(uintptr_t)(at + j * 2048);
+                to = ((lds_frag_t)(uintptr_t)at)[j * 128];
             };
             auto behind_slot = [&](unsigned slot) __attribute__((always_inline)) { return slot + STAGE == S * STAGE ? 0 : slot + STAGE; };
             auto meet = [&]() __attribute__((always_inline)) {
@@ -419,95 +457,76 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                 asm volatile("" ::: "memory");
                 __builtin_amdgcn_sched_barrier(0);
             };
-            // A step's accumulator blocks in their order.
-            constexpr int NB = FL * FS, LEAD_B = FL % 2 * FS;  // blocks, of those in a first strip of one
-            struct block { int i, j; };
-            auto block_at = [](int c) constexpr {
-                if (c < LEAD_B) return block{0, c};
-                const int e = c - LEAD_B, j = e % (2 * FS) / 2;
-                return block{FL % 2 + e / (2 * FS) * 2 + ((e & 1) ^ (j & 1)), j};
-            };
-            auto mul = [&](frag l, frag q, block b) __attribute__((always_inline)) {
+            auto mul = [&](frag l, frag q, typename T::block b) __attribute__((always_inline)) {
                 if constexpr (LONG_B)
                     acc[b.j][b.i] = X::go(l, q, acc[b.j][b.i]);
                 else
                     acc[b.i][b.j] = X::go(q, l, acc[b.i][b.j]);
             };
-            constexpr int NF = (FL + FS) * KK, NM = NB * KK;  // fetches and MFMAs of a step
-            // AHEAD: fetch number t of a stage, in the order in which its blocks want them.
-            auto fetch_nth = [&](int t, int set, unsigned slot, unsigned next) __attribute__((always_inline)) {
-                int n = 0;
-#pragma unroll
-                for (int c = 0; c < NB; c++) {
-                    const block x = block_at(c);
-                    bool new_l = true, new_s = true;
-#pragma unroll
-                    for (int d = 0; d < c; d++) {
-                        const block y = block_at(d);
-                        if (y.i == x.i) new_l = false;
-                        if (y.j == x.j) new_s = false;
-                    }
-#pragma unroll
-                    for (int kk = 0; kk < KK; kk++) {
-                        if (new_s && n++ == t) fetch_s(sf[AHEAD ? set : 0][x.j][kk], x.j, kk, slot, next);
-                        if (new_l && n++ == t) fetch_l(lf[set][AHEAD ? x.i : 0][kk], x.i, kk, slot, next);
-                    }
-                }
+            // AHEAD: fetch number `nth` of a stage into a set.
+            auto fetch_nth = [&](auto nth, auto set_c, unsigned slot, unsigned next) __attribute__((always_inline)) {
+                constexpr typename T::fetch f = T::fetches().nth[decltype(nth)::value];
+                constexpr int set = decltype(set_c)::value;
+                if constexpr (f.is_long)
+                    fetch_l(lf[set][AHEAD ? f.at : 0][f.kk], f.at, f.kk, slot, next);
+                else
+                    fetch_s(sf[AHEAD ? set : 0][f.at][f.kk], f.at, f.kk, slot, next);
             };
             // The step on set SET: the first half of its MFMAs, the meeting, the rest with the next stage's fetches.
             // (Met at the start, a stage that arrives late holds up the MFMAs of two stages.)
             auto step_ahead = [&](auto set_c, unsigned next, unsigned after) __attribute__((always_inline)) {
                 constexpr int SET = decltype(set_c)::value, MEET = NB / 2 * KK, SPAN = NB == 1 ? NM : (NM - MEET) * 3 / 4;
-#pragma unroll
-                for (int m = 0; m < NM; m++) {
-                    const block b = block_at(m / KK);
-                    if (m == MEET) meet();
+                static_for<NM>([&](auto mfma) __attribute__((always_inline)) {
+                    constexpr int m = decltype(mfma)::value;
+                    constexpr typename T::block b = T::block_at(m / KK);
+                    if constexpr (m == MEET) meet();
                     mul(lf[SET][AHEAD ? b.i : 0][m % KK], sf[AHEAD ? SET : 0][b.j][m % KK], b);
                     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int t = 0; t < NF; t++)
-                        if (m >= MEET && t * SPAN >= (m - MEET) * NF && t * SPAN < (m - MEET + 1) * NF) fetch_nth(t, 1 - SET, next, after);
+                    if constexpr (m >= MEET) {
+                        constexpr int first = T::first_at(m - MEET, NF, SPAN), last = T::first_at(m - MEET + 1, NF, SPAN);
+                        static_for<last - first>([&](auto t) __attribute__((always_inline)) {
+                            fetch_nth(std::integral_constant<int, first + decltype(t)::value>{}, std::integral_constant<int, 1 - SET>{}, next, after);
+                        });
+                    }
                     __builtin_amdgcn_sched_barrier(0);
-                }
+                });
             };
             // The step in strips.  The last strip's long fragments are the last ones fetched from the slot; with four k-steps
             // half of that strip is enough to fetch behind, and the later a stage is asked for, the less often it is late.
             auto step_strips = [&](unsigned slot, unsigned next, unsigned after) __attribute__((always_inline)) {
-                constexpr int LEAD = LEAD_B * KK, PER = 2 * FS * KK, MEET = KK > 2 ? PER / 2 : 0, SPAN = KK > 2 ? PER * 3 / 8 : 2 * KK;
-#pragma unroll
-                for (int m = 0; m < NM; m++) {
-                    const block b = block_at(m / KK);
-                    const int strip = m < LEAD ? 0 : (m - LEAD) / PER + FL % 2, w = m < LEAD ? m : (m - LEAD) % PER;
-                    const int len = m < LEAD ? LEAD : PER;
-                    if (strip == NS - 1 && w == MEET) meet();
+                constexpr int LEAD = T::LEAD_B * KK, PER = 2 * FS * KK, MEET = KK > 2 ? PER / 2 : 0, SPAN = KK > 2 ? PER * 3 / 8 : 2 * KK;
+                static_for<NM>([&](auto mfma) __attribute__((always_inline)) {
+                    constexpr int m = decltype(mfma)::value;
+                    constexpr typename T::block b = T::block_at(m / KK);
+                    constexpr int strip = m < LEAD ? 0 : (m - LEAD) / PER + FL % 2, w = m < LEAD ? m : (m - LEAD) % PER;
+                    constexpr int len = m < LEAD ? LEAD : PER;
+                    if constexpr (strip == NS - 1 && w == MEET) meet();
                     mul(lf[strip % LSETS][AHEAD ? 0 : FL % 2 ? (b.i + 1) % 2 * (b.i > 0) : b.i % 2][m % KK], sf[0][b.j][m % KK], b);
                     __builtin_amdgcn_sched_barrier(0);
-                    if (strip < NS - 1) {
+                    if constexpr (strip < NS - 1) {
                         // the next strip's long fragments; in front of them, in the first strip, the last short one
-                        const int ns = strip == 0 ? KK : 0, n = ns + 2 * KK, span = strip == NS - 2 ? len / 2 : len * 3 / 4;
-#pragma unroll
-                        for (int t = 0; t < 3 * KK; t++) {
-                            if (t < n && t * span >= w * n && t * span < (w + 1) * n) {
-                                const int h = (t - ns) / KK, kk = t % KK;
-                                if (t < ns)
-                                    fetch_s(sf[0][FS - 1][kk], FS - 1, kk, slot, next);
-                                else
-                                    fetch_l(lf[(strip + 1) % LSETS][h][kk], 2 * (strip + 1) - FL % 2 + h, kk, slot, next);
-                            }
-                        }
+                        constexpr int ns = strip == 0 ? KK : 0, n = ns + 2 * KK, span = strip == NS - 2 ? len / 2 : len * 3 / 4;
+                        constexpr int first = T::first_at(w, n, span), last = T::first_at(w + 1, n, span);
+                        static_for<last - first>([&](auto nth) __attribute__((always_inline)) {
+                            constexpr int t = first + decltype(nth)::value, h = (t - ns) / KK, kk = t % KK;
+                            if constexpr (t < ns)
+                                fetch_s(sf[0][FS - 1][kk], FS - 1, kk, slot, next);
+                            else
+                                fetch_l(lf[(strip + 1) % LSETS][h][kk], 2 * (strip + 1) - FL % 2 + h, kk, slot, next);
+                        });
                     } else {
                         // the next stage's: long fragments at once, a short one behind its last MFMA
-#pragma unroll
-                        for (int t = 0; t < (2 - FL % 2) * KK; t++)
-                            if (w == MEET + t * SPAN / (2 * KK)) fetch_l(lf[0][t / KK][t % KK], t / KK, t % KK, next, after);
-#pragma unroll
-                        for (int t = 0; t < (FS - 1) * KK; t++) {
-                            const int freed = (t / KK + 1) * 2 * KK - 1;
-                            if (w == (freed > MEET ? freed : MEET) + t % KK * SPAN / (2 * KK)) fetch_s(sf[0][t / KK][t % KK], t / KK, t % KK, next, after);
-                        }
+                        static_for<(2 - FL % 2) * KK>([&](auto nth) __attribute__((always_inline)) {
+                            constexpr int t = decltype(nth)::value;
+                            if constexpr (w == MEET + t * SPAN / (2 * KK)) fetch_l(lf[0][t / KK][t % KK], t / KK, t % KK, next, after);
+                        });
+                        static_for<(FS - 1) * KK>([&](auto nth) __attribute__((always_inline)) {
+                            constexpr int t = decltype(nth)::value, freed = (t / KK + 1) * 2 * KK - 1;
+                            if constexpr (w == (freed > MEET ? freed : MEET) + t % KK * SPAN / (2 * KK)) fetch_s(sf[0][t / KK][t % KK], t / KK, t % KK, next, after);
+                        });
                     }
                     __builtin_amdgcn_sched_barrier(0);
-                }
+                });
             };
             __builtin_amdgcn_s_setprio(2);
             // While the first stage is on its way: row map entries, and the groups to signal.
@@ -542,8 +561,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             asm volatile("" ::: "memory");
             // Behind the last stage, zeros never used are fetched.
             if constexpr (AHEAD) {
-#pragma unroll
-                for (int t = 0; t < NF; t++) fetch_nth(t, 0, 0, STAGE);
+                static_for<NF>([&](auto t) __attribute__((always_inline)) { fetch_nth(t, std::integral_constant<int, 0>{}, 0, STAGE); });
                 for (int kt = 0;;) {
                     unsigned next = behind_slot(slot);
                     step_ahead(std::integral_constant<int, 0>{}, next, behind_slot(next));
