@@ -36,12 +36,7 @@ enum {
 //
 // kRsEpilogueBelowFlop, kFewCopies: see fo_overlap_gemm_reducescatter.  They are no thresholds of a handle.
 //
-// kTogetherUpToK: up to this K the batches beside the GEMM are consumed and normalised by one kernel (whole_rows below).  A
-// wave of a longer GEMM lasts long enough for the consumer and the rows one after the other, and a consumer of one
-// wavefront per CU takes less from the GEMM (8192x8192, four waves, whole call, us, one after the other and together:
-// fp16 K = 2048 281 and 271, 4096 450 and 447, 6656 684 and 682, 8192 818 and 823; bf16 273 and 261, 433 and 429, 657 and 653,
-// 781 and 784).  Behind the GEMM the one kernel is the faster in any case (K = 8192 780.9 -> 776.5; 4096x8192x4096 238.2 ->
-// 233.4).
+// kTogetherUpToK, kTogetherAnyKUpToN: what is consumed and normalised by one kernel (rows_together below).
 //
 // kGemmFlopPerNs: what a GEMM is expected to sustain, for sizing the pause
 // between polls only.
@@ -49,7 +44,8 @@ constexpr int kFusedFromGroups = 16;
 constexpr double kInStreamBelowFlop = 6.4e10;
 constexpr double kRsEpilogueBelowFlop = 5e11;
 constexpr int kFewCopies = 16, kFewCopiesOfShort = 6;
-constexpr int kTogetherUpToK = 6144;
+constexpr int kTogetherUpToK = 3072;
+constexpr int kTogetherAnyKUpToN = 2048;
 constexpr double kGemmFlopPerNs = 1.2e6;
 
 }  // namespace
@@ -417,11 +413,29 @@ int last_slots(const int32_t *RA_host, int TM, int TN, std::vector<long> &last_s
     return FO_OK;
 }
 
-// Whether a batch that fills the storage slots [done, done + tiles) is exactly the tile rows `runs` it completes: then one
-// kernel consumes and normalises them, and reads C once for both.  Its registers fit beside the GEMM as the row kernel's do.
-// 8192x8192, bf16, K = 3584: a quarter's consumer and rows took 61 + 30 to 55 us beside the GEMM, more than the 95 us of a
-// wave of it, so that the consumer stream fell behind; together 71, and 28 instead of 17 + 12 and a launch behind the last
-// wave (whole call 409.9 -> 396.8 us).
+// Whether batches that are whole tile rows are consumed and normalised by one kernel, which reads C once for both.  `last`:
+// the batch behind the GEMM, where the one kernel is the faster in any case (28 us instead of 17 + 12 and a launch on 8192
+// columns; whole call, us, 4096x8192x4096 241.6 -> 236.1, 8192x2048x4096 135.2 -> 129.9).
+// Beside the GEMM it depends on how long a wave of it lasts.  In a short one the consumer and the rows (61 + 30 to 55 us
+// for a quarter of 8192x8192, together 71) fall behind if they follow one another; a long one has time for that, and a
+// consumer of one wavefront per CU takes less from it.  Whole call, us, one after the other and together beside the GEMM, 8192
+// columns: fp16, 8192 rows, K = 1536 236 and 228, 2048 273.5 and 271.9, 2560 321.6 and 314.3, 3072 370.4 and 370.1, 3328
+// 378.6 and 385.0, 3584 401.2 and 409.2, 4096 442.3 and 454.4, 6144 651 and 658, 8192 815 and 830; bf16 239 and 222, 268 and 262,
+// 323 and 302, 363 and 361, 367 and 372, 388 and 395, 425 and 432, 631 and 629, 778 and 789; 16384x4096 bf16 K = 2048 278 and
+// 258, 3072 379.5 and 371.7, 3584 397 and 402, 8192 778 and 781.  Rows of up to 2048 elements are the faster together at
+// every K (16384x2048 fp16 3584 225 and 222, 8192 427 and 422; 65536x1024 3584 462 and 445, 8192 851 and 846).
+// The kernel's registers (at most 128) fit beside the 256x256 kernel that counts, and not beside 128x256 tiles that do, no
+// more than the row kernel's by itself: there it follows the GEMM, and is still the faster (8064x8192 by such tiles with the
+// rows in row-major order, fp16 K = 1600 328 and 302, 4096 563 and 540).
+// Rows in more than one run are in an order that the GEMM does not follow: such a batch is complete late, when little is
+// left of the GEMM, and a launch for each run is the faster than one consumer launch and a launch for each run's rows
+// (8192x8192 fp16 in four batches of two, of four runs: K = 2048 309 and 291, 339 and 323, 3584 438 and 412, 473 and 449, 8192
+// 831 and 829, 880 and 862).
+bool rows_together(int M, int N, int K, int BN, int rLDN, int runs, bool last) {
+    return fo_consumes_norm_rows(M, N, BN, rLDN) && (last || runs > 1 || K <= kTogetherUpToK || N <= kTogetherAnyKUpToN);
+}
+
+// Whether a batch that fills the storage slots [done, done + tiles) is exactly the tile rows `runs` it completes.
 bool whole_rows(const int32_t *RA_host, int TN, const std::vector<int> &runs, long done, long tiles) {
     long rows = 0;
     for (size_t k = 0; k + 1 < runs.size(); k += 2) {
@@ -534,7 +548,7 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
         long done = 0;
         uint16_t *c = static_cast<uint16_t *>(C);
         uint16_t *acc = static_cast<uint16_t *>(h->acc);
-        const bool consumes_rows = np && acc && !same_stream && h->link_bytes_per_s <= 0 && fo_consumes_norm_rows(M, N, info[1], rLDN) &&
+        const bool consumes_rows = np && acc && !same_stream && h->link_bytes_per_s <= 0 &&
                                    apart({acc, mn}, {{C, mn}, {np->Y, mn}, {np->Wt, N}}) &&
                                    apart({np->Y, mn}, {{C, mn}});  // the accumulator takes the product, not rows written over it
         for (int i = 0; i < G;) {
@@ -550,7 +564,8 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
             }
             std::vector<int> runs;
             if (np && !same_stream) ready_tile_rows(last_slot.data(), TM, done + tiles, j == G, runs);
-            const bool with_rows = consumes_rows && (j == G || K <= kTogetherUpToK) && whole_rows(np->RA_host, TN, runs, done, tiles);
+            const bool with_rows = consumes_rows && rows_together(M, N, K, info[1], rLDN, (int)runs.size() / 2, j == G) &&
+                                   whole_rows(np->RA_host, TN, runs, done, tiles);
             if (acc && !consumed && !with_rows) {  // the groups of a batch are one contiguous range
                 rc = fo_consumer_reduce_with(dtype, c + off, acc + off, n, 1, 0, nullptr, 0, stream_acc, cstream,
                                              j < G && !same_stream);  // every batch but the last runs beside the GEMM
@@ -608,6 +623,12 @@ extern "C" int fo_overlap_plan_norm_rows(const int32_t *RA_host, int TM, int TN,
         i = j;
     }
     return n;
+}
+
+// Whether the call consumes and normalises a batch of whole tile rows by one kernel.
+extern "C" int fo_overlap_plan_rows_together(int M, int N, int K, int BN, int rLDN, int runs, int last) {
+    if (M <= 0 || N <= 0 || K <= 0 || BN <= 0 || rLDN <= 0 || runs <= 0) return FO_ERR_ARG;
+    return rows_together(M, N, K, BN, rLDN, runs, last != 0) ? 1 : 0;
 }
 
 extern "C" int fo_overlap_gemm_allreduce(fo_overlap_t *h, int dtype, int M, int N, int K,

@@ -293,6 +293,10 @@ int fo_overlap_plan_batches(const int32_t *cseg_host, int G, int wave_tiles, int
  * runs, FO_ERR_LIMIT if there are more than max_runs, or a negative error. */
 int fo_overlap_plan_norm_rows(const int32_t *RA_host, int TM, int TN, const int32_t *cseg_host, int G,
                               int wave_tiles, int32_t *runs, int max_runs);
+/* 1 if that call consumes and normalises a batch that is exactly the tile rows it completes by one kernel, 0 if by a
+ * consumer launch and one for the rows (accumulator apart from product and output, no link rate).  BN: the Algo's tile
+ * width; runs: the batch's runs of consecutive tile rows; last: nothing of the GEMM is left behind it. */
+int fo_overlap_plan_rows_together(int M, int N, int K, int BN, int rLDN, int runs, int last);
 /* fused < 0 (default): chosen per call.  A GEMM below 6.4e10 flop (about 50 us)
  * keeps the whole call on the GEMM stream (the GEMM with its reordered store,
  * then one consumer launch: nothing that short can hide a fork and a join, and

@@ -400,6 +400,23 @@ def test_normalisation_follows_the_groups_that_complete_its_rows():
         _capi.plan_norm_rows(np.arange(4, dtype=np.int32).reshape(2, 2), [3], 0)  # groups do not cover the tiles
 
 
+@pytest.mark.parametrize("M,N,K,beside,behind", [
+    (8192, 8192, 3072, 1, 1),    # a wave of the GEMM is shorter than a consumer and its rows
+    (8192, 8192, 3328, 0, 1),    # it has time for one after the other
+    (8192, 8192, 6144, 0, 1),
+    (8192, 8192, 3584, 0, 1),
+    (16384, 4096, 3584, 0, 1),
+    (16384, 2048, 8192, 1, 1),   # short rows
+    (8192, 16384, 1024, 0, 0),   # rows too long for the kernel
+])
+def test_what_is_consumed_and_normalised_by_one_kernel(M, N, K, beside, behind):
+    together = _capi.lib().fo_overlap_plan_rows_together
+    assert [together(M, N, K, 128, 1, 1, last) for last in (0, 1)] == [beside, behind]
+    assert together(M, N, K, 128, 1, 2, 0) == behind        # an order the GEMM does not follow
+    assert together(M, N, K, 128, 2, 1, 1) == 0             # tiles side by side
+    assert together(0, N, K, 128, 1, 1, 1) == together(M, N, K, 128, 1, 0, 1) == -1
+
+
 def test_front_ends_refuse_undersized_buffers():
     """MM, RA, RE and D are indexed through raw pointers by kernels that store and count through them;
     both front ends must refuse buffers that are too small before anything is launched.  The case the
