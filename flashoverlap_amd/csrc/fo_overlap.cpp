@@ -425,14 +425,17 @@ int last_slots(const int32_t *RA_host, int TM, int TN, std::vector<long> &last_s
 // 258, 3072 379.5 and 371.7, 3584 397 and 402, 8192 778 and 781.  Rows of up to 2048 elements are the faster together at
 // every K (16384x2048 fp16 3584 225 and 222, 8192 427 and 422; 65536x1024 3584 462 and 445, 8192 851 and 846).
 // The kernel's registers (at most 128) fit beside the 256x256 kernel that counts, and not beside 128x256 tiles that do, no
-// more than the row kernel's by itself: there it follows the GEMM, and is still the faster (8064x8192 by such tiles with the
-// rows in row-major order, fp16 K = 1600 328 and 302, 4096 563 and 540).
+// more than the row kernel's by itself.  Those tiles are taken where 256 does not divide M or N; a batch is whole rows there
+// in an order of the caller's only, much of it follows the GEMM, and the one kernel is the faster at every K (rows in row-major
+// order, fp16: 8064x8192 by 128x256 tiles, K = 1600 328 and 302, 4096 564 and 547, 7168 890 and 869; by 128x128 tiles 4096 699
+// and 657; 8064x4096x8192 497 and 482).
 // Rows in more than one run are in an order that the GEMM does not follow: such a batch is complete late, when little is
 // left of the GEMM, and a launch for each run is the faster than one consumer launch and a launch for each run's rows
 // (8192x8192 fp16 in four batches of two, of four runs: K = 2048 309 and 291, 339 and 323, 3584 438 and 412, 473 and 449, 8192
 // 831 and 829, 880 and 862).
 bool rows_together(int M, int N, int K, int BN, int rLDN, int runs, bool last) {
-    return fo_consumes_norm_rows(M, N, BN, rLDN) && (last || runs > 1 || K <= kTogetherUpToK || N <= kTogetherAnyKUpToN);
+    const bool ragged = M % 256 || N % 256;
+    return fo_consumes_norm_rows(M, N, BN, rLDN) && (last || ragged || runs > 1 || K <= kTogetherUpToK || N <= kTogetherAnyKUpToN);
 }
 
 // Whether a batch that fills the storage slots [done, done + tiles) is exactly the tile rows `runs` it completes.

@@ -407,6 +407,7 @@ def test_normalisation_follows_the_groups_that_complete_its_rows():
     (8192, 8192, 3584, 0, 1),
     (16384, 4096, 3584, 0, 1),
     (16384, 2048, 8192, 1, 1),   # short rows
+    (8064, 8192, 7168, 1, 1),    # tiles of another size
     (8192, 16384, 1024, 0, 0),   # rows too long for the kernel
 ])
 def test_what_is_consumed_and_normalised_by_one_kernel(M, N, K, beside, behind):
