@@ -36,7 +36,7 @@ enum {
 //
 // kRsEpilogueBelowFlop, kFewCopies: see fo_overlap_gemm_reducescatter.  They are no thresholds of a handle.
 //
-// kTogetherUpToK, kTogetherAnyKUpToN: what is consumed and normalised by one kernel (rows_together below).
+// kTogetherFromN, kTogetherUpToK, kTogetherAnyKUpToN: what is consumed and normalised by one kernel (rows_together below).
 //
 // kGemmFlopPerNs: what a GEMM is expected to sustain, for sizing the pause
 // between polls only.
@@ -44,6 +44,7 @@ constexpr int kFusedFromGroups = 16;
 constexpr double kInStreamBelowFlop = 6.4e10;
 constexpr double kRsEpilogueBelowFlop = 5e11;
 constexpr int kFewCopies = 16, kFewCopiesOfShort = 6;
+constexpr int kTogetherFromN = 1024;
 constexpr int kTogetherUpToK = 3072;
 constexpr int kTogetherAnyKUpToN = 2048;
 constexpr double kGemmFlopPerNs = 1.2e6;
@@ -433,9 +434,13 @@ int last_slots(const int32_t *RA_host, int TM, int TN, std::vector<long> &last_s
 // left of the GEMM, and a launch for each run is the faster than one consumer launch and a launch for each run's rows
 // (8192x8192 fp16 in four batches of two, of four runs: K = 2048 309 and 291, 339 and 323, 3584 438 and 412, 473 and 449, 8192
 // 831 and 829, 880 and 862).
+// Shorter rows leave most of the workgroup's lanes idle in what was the consumer's traffic (us, by two kernels and by one, fp16
+// / bf16: 131072x256x4096 480 and 523 / 498 and 544, 65536x512x2048 218 and 227 / 230 and 240.5; 32768x1024x4096 257
+// and 251 / 251 and 242).
 bool rows_together(int M, int N, int K, int BN, int rLDN, int runs, bool last) {
     const bool ragged = M % 256 || N % 256;
-    return fo_consumes_norm_rows(M, N, BN, rLDN) && (last || ragged || runs > 1 || K <= kTogetherUpToK || N <= kTogetherAnyKUpToN);
+    return fo_consumes_norm_rows(M, N, BN, rLDN) && N >= kTogetherFromN &&
+           (last || ragged || runs > 1 || K <= kTogetherUpToK || N <= kTogetherAnyKUpToN);
 }
 
 // Whether a batch that fills the storage slots [done, done + tiles) is exactly the tile rows `runs` it completes.

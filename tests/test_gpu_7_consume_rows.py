@@ -21,6 +21,7 @@ pytestmark = pytest.mark.gpu
     (128, 128, 256, 1920, [10, 20]),                 # one chunk, lanes left over
     (128, 128, 384, 4224, [33, 66]),                 # three chunks, most of the third beyond the row
     (128, 256, 128, 256, [1]),                       # one tile
+    (128, 128, 128, 1024, [8]),                      # the shortest rows, one tile row
 ])
 def test_rows_are_consumed_and_normalised(fo, dtype, bm, bn, M, N, cseg):
     _run_both(fo, dtype, bm, bn, M, N, 72, cseg, 0, seed=700)

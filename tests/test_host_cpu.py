@@ -407,6 +407,9 @@ def test_normalisation_follows_the_groups_that_complete_its_rows():
     (8192, 8192, 3584, 0, 1),
     (16384, 4096, 3584, 0, 1),
     (16384, 2048, 8192, 1, 1),   # short rows
+    (32768, 1024, 4096, 1, 1),
+    (65536, 512, 2048, 0, 0),    # rows too short for the kernel's lanes
+    (131072, 256, 4096, 0, 0),
     (8064, 8192, 7168, 1, 1),    # tiles of another size
     (8192, 16384, 1024, 0, 0),   # rows too long for the kernel
 ])
