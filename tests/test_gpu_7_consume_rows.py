@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from gpu_util import BF16, F16, TORCH_DTYPE
+from gpu_util import BF16, F16, TORCH_DTYPE, seeded
 from test_gpu_3_norm_overlap import _run_both
 
 pytestmark = pytest.mark.gpu
@@ -76,3 +76,35 @@ def test_many_wide_rows(fo, dtype, M, N):
     ulp = 2.0 ** -10 if dtype == F16 else 2.0 ** -7
     torch.cuda.synchronize()
     assert ((Y.double() - want).abs() <= 2 * ulp * want.abs() + 2.0 ** -23).all()
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("rows_behind", [0, 256])
+def test_rows_over_the_product(fo, dtype, rows_behind):
+    """Normalised rows written over the product: the accumulator takes the product and none of them.  One batch, tile rows in
+    reverse order, so that most rows are written where another one's product lies (which rows then come out is nobody's
+    promise: they are not looked at)."""
+    bm, bn, M, N, K = 128, 128, 1024, 2048, 256
+    td, TM, TN = TORCH_DTYPE[dtype], M // bm, N // bn
+    algo = fo._capi.find_algo(bm, bn, swizzle=4)
+    hint = [tm * TN + tn for tm in reversed(range(TM)) for tn in range(TN)]
+    RA = fo.layout.reorder_indices(TM * TN, hint, device="cuda").reshape(TM, TN)
+    A, _ = seeded((M, K), dtype, 1)
+    B, _ = seeded((N, K), dtype, 2, scale=K ** -0.5)
+    before, _ = seeded((M * N,), dtype, 3)
+    gamma = torch.ones(N, device="cuda", dtype=td)
+    cs = torch.tensor([TM * TN], dtype=torch.int32)
+    MM = torch.zeros(fo.layout.counter_size(1, TM, TN), dtype=torch.int32, device="cuda")
+    ov = fo.ops.Overlap()
+    ov.set_fused_consumer(0)
+    product, want = torch.empty(M * N, device="cuda", dtype=td), before.clone()
+    ov.set_accumulator(want)
+    ov.gemm_allreduce_overlap(A, B, product, MM, RA, 1, cs, cs.cuda(), algo)
+    room = torch.empty((M + rows_behind) * N, device="cuda", dtype=td)
+    C, Y, acc = room[:M * N], room[rows_behind * N:].view(M, N), before.clone()
+    ov.set_accumulator(acc)
+    ov.gemm_allreduce_rmsnorm_overlap(A, B, C, MM, RA, RA.cpu(), 1, cs, cs.cuda(), algo, Y, gamma, eps=1e-6)
+    torch.cuda.synchronize()
+    assert torch.equal(acc, want) and torch.equal(want, (before.float() + product.float()).to(td))
+    assert (MM == 0).all() and ov.status() == 0
+    ov.close()
