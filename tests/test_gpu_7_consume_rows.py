@@ -83,8 +83,8 @@ def test_many_wide_rows(fo, dtype, M, N):
 def test_rows_over_the_product(fo, dtype, rows_behind):
     """Normalised rows written over the product: the accumulator takes the product and none of them.  One batch, tile rows in
     reverse order, so that most rows are written where another one's product lies (which rows then come out is nobody's
-    promise: they are not looked at)."""
-    bm, bn, M, N, K = 128, 128, 1024, 2048, 256
+    promise: they are not looked at), and four times as many workgroups of rows as the GPU holds at once."""
+    bm, bn, M, N, K = 128, 128, 8192, 4096, 72
     td, TM, TN = TORCH_DTYPE[dtype], M // bm, N // bn
     algo = fo._capi.find_algo(bm, bn, swizzle=4)
     hint = [tm * TN + tn for tm in reversed(range(TM)) for tn in range(TN)]
