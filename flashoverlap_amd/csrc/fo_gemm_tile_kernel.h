@@ -29,10 +29,10 @@
 // Measured against the kernel this one replaced (loads issued by the computing wavefronts; fp16, GEMM alone,
 // operands of three buffer sets in turn, which the memory-side cache holds): 512x4096x4096 39.1 -> 21 us, 256x8192x3584
 // 35.5 -> 19.5, 128x4096x1024 10.4 -> 4.5, 128x1024x8192 71 -> 12.5, 2048x4096x4096 62 -> 55.
-// None of it is at a unit's limit.  512x4096x4096 on 64x128 tiles: 39 bytes a clock and CU of the 64, matrix pipe busy
-// 40 % of the clocks, LDS reads 32 %; with the MFMAs taken out 18.7 us, so what is left is round trips to the operands.
-// With operands that no cache holds (eight sets in turn) the same misses take longer: 29.6 us, 256x8192x3584 20.1 -> 30.0.
-// One round of 128x256 tiles (1024x8192x2048, 31.3 us) has the matrix pipe busy for 64 % and LDS reads for 27 %.
+// None of it is at a unit's limit.  512x4096x4096 on 64x128 tiles (21.0 us): 39 bytes a clock and CU of the 64, matrix pipe
+// busy 41 % of the clocks, LDS reads 32 %; with the MFMAs taken out 19.7 of 21.8 us, so what is left is round trips to the
+// operands.  With operands that no cache holds (eight sets in turn) the same misses take longer: 28.1 us, 256x8192x3584 19.7
+// -> 28.2.  One round of 128x256 tiles (1024x8192x2048, 29.2 us) has the matrix pipe busy for 64 % and LDS reads for 27 %.
 //
 // SHIFT: operand rows that do not begin on 128-byte lines (K no multiple of 64, or an operand's own address).  A load of
 // eight rows x 128 bytes then touches sixteen lines instead of eight, and these sizes slow down by 30 to 40 %.  Shifted,

@@ -299,9 +299,9 @@ int fo_overlap_plan_norm_rows(const int32_t *RA_host, int TM, int TN, const int3
 int fo_overlap_plan_rows_together(int M, int N, int K, int BN, int rLDN, int runs, int last);
 /* fused < 0 (default): chosen per call.  A GEMM below 6.4e10 flop (about 50 us)
  * keeps the whole call on the GEMM stream (the GEMM with its reordered store,
- * then one consumer launch: nothing that short can hide a fork and a join, and
- * the stream orders the two, so MM is not touched and stays zero; with the
- * monitor on, the signalling GEMM and one wait over all groups as elsewhere),
+ * whose epilogue does the consumer's work too: nothing that short can hide a
+ * fork and a join, and nobody waits, so MM is not touched and stays zero; with
+ * the monitor on, the signalling GEMM and one wait over all groups as elsewhere),
  * and so does, without the monitor, a product of less than about one round of
  * 256x256 tiles, one that 256 does not divide in M or N, an all-reduce with
  * neither accumulator nor normalisation, or a reduce-scatter of more than 16
