@@ -130,6 +130,17 @@ constexpr row_fetches256 fetches_of_row256(int r) {
     return f;
 }
 
+// The accumulator's values that a step requests (MODE_ACC): eight, in rows that carry no operand load, behind this step's
+// last load of the next stage (row 6) and in front of FREE.  takes_before256: those in front of MFMA m of row r.
+constexpr int kTakes256 = 8, kTakeAt256[kTakes256] = {7 * 8 + 1, 7 * 8 + 3, 7 * 8 + 5, 8 * 8 + 2, 8 * 8 + 6, 9 * 8 + 1, 9 * 8 + 3, 9 * 8 + 5};
+constexpr int takes_before256(int r, int m) {
+    int n = 0;
+    while (n < kTakes256 && kTakeAt256[n] < r * 8 + m) n++;
+    return n;
+}
+
+constexpr int kTakeFromSteps256 = 5;  // K steps of a tile from which on they are: four take, and the loop behind them has one at least
+
 constexpr int kSmem256 = 2 * 65536 + 4 * 16 * (128 + 8) * 2;  // two slots + four strips of 16 padded rows
 
 template <typename Tag, int MODE>
@@ -442,17 +453,47 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             for (int j = 0; j < F; j++)
 #pragma unroll
                 for (int v = 0; v < 4; v++) acc[i][j][v] = 0.f;
+        if (MODE == MODE_ACC) {
+            // All of them are written here: with two ways to the first MFMA the compiler would write each block's in front of
+            // its own, inside the wait states that the assembly does not bring.
+#pragma unroll
+            for (int i = 0; i < F; i++)
+#pragma unroll
+                for (int j = 0; j < F; j++) asm volatile("" : "+a"(acc[i][j]));
+        }
         fo_mfma_fence();
 
-        // A tile whose predecessor's signal is still owed leaves the K loop after its first step, sends the signal and
-        // re-enters: that step's PUB meeting has waited for the predecessor's stores in every wavefront (part of the
-        // stage's loads was requested behind them, rows 0-6, and vmcnt retires in issue order), with the meeting's
-        // barrier behind the wait.  The test inside the step (one scalar compare and branch per K step, after the PUB
-        // meeting) cost the large square 4 us.
-        int kt = 0;
-        int kt_stop = (COUNTS && owed > 0) ? 1 : KT;
-        for (;;) {
-        do {
+        // MODE_ACC: the accumulator's values of the wavefront's block, 32 pieces a lane: this wavefront owns the SIMD and has the
+        // registers.  They are requested a quarter at a time in the tile's first four steps (a half that is not stored: with an
+        // empty range), where the memory is idle, and read behind the last.  Loads return in order, so the place matters:
+        // behind this step's last load of the next stage, whose wait then counts them as younger, and one K step in front of
+        // the wait for the stage behind that.  Requested in the epilogue, with every CU at its end at the same time, they cost a
+        // round trip and their bandwidth in front of the first store (whole passes, us, in the epilogue -> in the first steps:
+        // 4096x4096x512 44.0 -> 41.6, 4096x4096x1024 55.9 -> 52.2, 4096x8192x264 85.7 -> 77.1, 3456x4352x3072 100.2 -> 97.3,
+        // 8064x8064x4096 463.8 -> 455.7; 8192x8192x2048 by the serial call 276.5 -> 272.4).
+        fo_u32x4 old[ACC ? NST : 1];
+        const bool early = MODE == MODE_ACC && KT >= kTakeFromSteps256;
+        int take_row = 0, take_step = 0;
+        unsigned take_lane = 0;
+        __amdgpu_buffer_rsrc_t take_from;
+        if (early) {
+            const int ldp = reorder ? p.rLDN * p.BN : p.N;
+            const long trow = !reorder ? (long)(pm + wm) * 128 : (long)(r_mine / p.rLDN) * p.BM + (wm * 128) % p.BM;
+            const long tcol = !reorder ? (long)(pn + wn) * 128 : (long)(r_mine % p.rLDN) * p.BN + (wn * 128) % p.BN;
+            const bool keep = !((repeated & 1) && wm == 0) && !((repeated & 2) && wn == 0);
+            take_from = __builtin_amdgcn_make_buffer_rsrc((void *)(p.ACC + trow * ldp + tcol), 0, keep ? (unsigned)(127 * ldp + 128) * 2 : 0, 0x00027000);
+            take_step = RPP * ldp * 2;
+            take_lane = (unsigned)(lane / CPR * ldp + lane % CPR * 8) * 2;
+        }
+        auto take = [&](auto nth) __attribute__((always_inline)) {
+            constexpr int k = decltype(nth)::value;
+            old[ACC ? k : 0] = __builtin_bit_cast(fo_u32x4, __builtin_amdgcn_raw_buffer_load_b128(take_from, take_lane, take_row, 0));
+            take_row += take_step;
+            asm volatile("" ::: "memory");  // stays here: the step's waits count it
+        };
+        // One K step.  TAKES: the quarter of the accumulator's pieces that it requests (-1: none).
+        auto k_step = [&](auto takes) __attribute__((always_inline)) {
+            constexpr int TAKES = decltype(takes)::value;
             unsigned la_ = la0 ^ slot_b, lb_ = lb0 ^ slot_b;
             asm volatile("" : "+v"(la_), "+v"(lb_));
             // by slot (the step's, the next step's) and k-step, found here: computed at each fetch, they stand between the MFMAs
@@ -483,6 +524,8 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                         else
                             load_a(next_a, a_at[f.next][f.kk], f.block, f.kk);
                     });
+                    if constexpr (TAKES >= 0 && takes_before256(r, m + 1) > takes_before256(r, m))
+                        take(std::integral_constant<int, TAKES * kTakes256 + takes_before256(r, m)>{});
                     __builtin_amdgcn_sched_barrier(0);
                 });
                 if constexpr (r == FREE) {
@@ -495,13 +538,34 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                     // The stage the next step reads has landed; younger and allowed in flight: this step's YOUNG loads.
                     // In a tile's first step the wait also covers the previous tile's stores: part of the stage's
                     // loads was requested behind them (rows 0-6), and vmcnt retires in issue order.
-                    wait_vmcnt<YOUNG>();
+                    // (The accumulator's values this step asked for are younger than that stage as well.)
+                    wait_vmcnt<YOUNG + (TAKES >= 0 ? kTakes256 : 0)>();
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" ::: "memory");
                 }
                 __builtin_amdgcn_sched_barrier(0);
             });
             slot_b ^= SLOT_B;
+        };
+        // A tile whose predecessor's signal is still owed leaves the K loop after its first step, sends the signal and
+        // re-enters: that step's PUB meeting has waited for the predecessor's stores in every wavefront (part of the
+        // stage's loads was requested behind them, rows 0-6, and vmcnt retires in issue order), with the meeting's
+        // barrier behind the wait.  The test inside the step (one scalar compare and branch per K step, after the PUB
+        // meeting) cost the large square 4 us.
+        int kt = 0;
+        int kt_stop = (COUNTS && owed > 0) ? 1 : KT;
+        if constexpr (MODE == MODE_ACC) {
+            if (early) {
+                k_step(std::integral_constant<int, 0>{});
+                k_step(std::integral_constant<int, 1>{});
+                k_step(std::integral_constant<int, 2>{});
+                k_step(std::integral_constant<int, 3>{});
+                kt = 4;
+            }
+        }
+        for (;;) {
+        do {
+            k_step(std::integral_constant<int, -1>{});
         } while (++kt < kt_stop);
             if (!COUNTS || owed == 0) break;
             owed = 0;
@@ -542,11 +606,8 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             const unsigned lane_off = (unsigned)(srow * ldp + scol * 8) * 2;
             const bool stream_out = p.stream_out != 0;  // wave-uniform
             const bool keep = !((repeated & 1) && wm == 0) && !((repeated & 2) && wn == 0);  // wave-uniform
-            // MODE_ACC: the accumulator's values of the whole block, 32 pieces a lane: this wavefront owns the SIMD and
-            // has the registers.  They are awaited together, in front of the first store: a later wait would count the
-            // stores between them as well.  4096x4096x512: 30 us, where the reordering GEMM took 21 and a consumer
-            // launch behind it 16 (whole pass 52 -> 46).
-            fo_u32x4 old[ACC ? NST : 1];
+            // The accumulator's values are awaited together, in front of the first store: a later wait would count the
+            // stores between them as well.
             char *abase = ACC ? reinterpret_cast<char *>(p.ACC) + (trow * ldp + tcol) * 2 : nullptr;
             // MODE_RS: the accumulator rows of the wavefront's rows, held as re_lo and re_hi are.
             int ac_lo = 0, ac_hi = 0;
@@ -561,7 +622,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                 ac_lo = rs_row(p.cseg, p.G, p.BM, p.W, p.seg_rows, re_lo, first * p.BM, count * p.BM);
                 ac_hi = rs_row(p.cseg, p.G, p.BM, p.W, p.seg_rows, re_hi, first * p.BM, count * p.BM);
             }
-            if (sums && keep) {
+            if (sums && keep && !early) {
 #pragma unroll
                 for (int k = 0; k < NST; k++) {
                     if (MODE == MODE_RS) {
@@ -571,7 +632,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                         old[ACC ? k : 0] = *reinterpret_cast<const fo_u32x4 *>(abase + (size_t)(k * RPP) * ldp * 2 + lane_off);
                     }
                 }
-            } else {
+            } else if (!early) {
 #pragma unroll
                 for (int k = 0; k < (ACC ? NST : 1); k++) old[k] = fo_u32x4{0, 0, 0, 0};
             }

@@ -390,3 +390,41 @@ def test_monitor_stamps_of_one_round_are_measured(fo, bm, bn, M, N, K):
     stamps = MM[TN:TN + T].tolist()
     assert MM[0] == T and MM[TN - 1] == T and sorted(stamps) == list(range(T))
     assert stamps != list(range(T))
+
+
+@pytest.mark.parametrize("dtype,bm,bn,M,N,K", [
+    (F16, 128, 128, 4096, 4096, 256),     # 256x256, four K steps: the accumulator is read in the epilogue
+    (F16, 128, 128, 4096, 4096, 320),     # five: requested in the first four, one step left
+    (BF16, 128, 256, 4096, 4096, 328),    # six, the last one partial
+    (BF16, 256, 128, 4224, 7168, 384),    # half a tile left along M, a workgroup's second tile
+    (F16, 128, 128, 4224, 7296, 520),     # half a tile left along both
+])
+def test_accumulator_requested_during_the_product(fo, dtype, bm, bn, M, N, K):
+    """The 256x256 kernel asks for the accumulator's values while it multiplies: sums of every element once rounded, none of
+    another's, over reordered and plain stores."""
+    ops, layout, td = fo.ops, fo.layout, TORCH_DTYPE[dtype]
+    algo = fo._capi.find_algo(bm, bn, swizzle=4)
+    TM, TN = M // bm, N // bn
+    A, _ = seeded((M, K), dtype, M + K)
+    B, _ = seeded((N, K), dtype, N + K, scale=K ** -0.5)
+    before, _ = seeded((M, N), dtype, 11)
+    acc = before.clone()
+    plain, C = (torch.full((M, N), float("nan"), device="cuda", dtype=td) for _ in range(2))
+    ops.gemm(A, B, plain, algo)
+    ov = ops.Overlap()
+    ov.set_schedule(in_stream_below_flop=1e15)
+    ov.set_accumulator(acc)
+    ov.gemm_allreduce(A, B, C, algo)
+    torch.cuda.synchronize()
+    assert torch.equal(C, plain)
+    assert torch.equal(acc, (before.float() + plain.float()).to(td))
+    RA = torch.from_numpy(np.random.default_rng(K).permutation(TM * TN).astype(np.int32)).reshape(TM, TN).cuda()
+    cs = torch.tensor([TM * TN], dtype=torch.int32)
+    MM = torch.zeros(layout.counter_size(1, TM, TN), dtype=torch.int32, device="cuda")
+    C.fill_(float("nan"))
+    acc.copy_(before)
+    ov.gemm_allreduce_overlap(A, B, C, MM, RA, 1, cs, cs.cuda(), algo)
+    torch.cuda.synchronize()
+    assert torch.equal(layout.unpermute(C, M, N, bm, bn, RA), plain)
+    assert torch.equal(acc.reshape(-1), (before.float() + C.float()).to(td).reshape(-1))
+    ov.close()
