@@ -69,16 +69,23 @@ struct launch_plan {
 constexpr int kSignalAfterFromK = 1536;
 
 // What one round of a tile takes, all CUs busy: microseconds at K = 4096, with operand rows on 128-byte lines and off them
-// (the tiles up to 128x160 then load whole lines, the larger ones cannot).  Ratios at K = 1024 are the same.
+// (the tiles up to 128x192 then load whole lines, the larger ones cannot; 128x192 only without a row map, for which its four
+// stages leave no LDS).  Ratios at K = 1024 are the same.  With its line loads (54 -> 46 a round) one round of 128x192 takes the
+// place of two of 96x128 or of one of 128x256; GEMM alone, us: 1152x5120x1720 bf16 23.4 -> 21.0, with an accumulator 26.5 ->
+// 23.7, 1536x3840x2040 26.7 -> 24.8, 1152x5120x4088 48.5 -> 46.4.
 struct tile_cost {
-    int tm, tn, on_lines, off_lines;
+    int tm, tn, on_lines, off_lines, mapped;
 };
-constexpr tile_cost kTileCosts[] = {{96, 128, 26, 27},  {128, 128, 31, 33}, {128, 160, 36, 38}, {128, 192, 42, 54},
-                                    {128, 256, 57, 71}, {256, 128, 57, 71}, {256, 256, 97, 110}};
+constexpr tile_cost kTileCosts[] = {{96, 128, 26, 27, 27},  {128, 128, 31, 33, 33}, {128, 160, 36, 38, 38}, {128, 192, 42, 46, 54},
+                                    {128, 256, 57, 71, 71}, {256, 128, 57, 71, 71}, {256, 256, 97, 110, 110}};
+// Beginning and end of a round of 128x192 with its line loads, beyond the other tiles' (us): with few columns of K two rounds
+// of it are no better than three of 128x128 (with an accumulator, us, 2304x5120x264 20.2 and 18.5, 2048x6144x264 20.7 and 19.8,
+// 2048x6144x776 40.7 and 42.8).
+constexpr double kWide192Ends = 0.5;
 
 // Estimate for `count` tiles: whole rounds, and a last one that costs 60 % of a round plus its share of the CUs (fewer
 // active CUs share the L2s, HBM and the power limit).
-double rounds_cost(long count, long cus, int round) {
+double rounds_cost(long count, long cus, double round) {
     const long full = count / cus, rest = count % cus;
     return round * (full + (rest ? 0.6 + 0.4 * rest / cus : 0.0));
 }
@@ -101,7 +108,8 @@ double rounds_cost(long count, long cus, int round) {
 // was complete in its last round (8064x8192 in four groups: rounds 3, 1, 2, 3 of 0..3).
 // M and N need only be multiples of 128: the last tile of a dimension is moved back or, 256x256, repeats half of its
 // neighbour.
-launch_plan plan_launch(const fo_raster &r, int M, int N, int BM, int BN, bool whole_only, bool counted, bool on_lines) {
+launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN, bool whole_only, bool counted, bool on_lines,
+                        bool mapped) {
     launch_plan p;
     p.tail = p.tail_tm = p.tail_tn = 0;
     auto set = [&](int tm, int tn) {
@@ -148,7 +156,7 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int BM, int BN, bool w
         double least = 0;
         for (const tile_cost &t : kTileCosts) {
             if (M < t.tm || N < t.tn) continue;
-            const int round = on_lines ? t.on_lines : t.off_lines;
+            const double round = on_lines ? t.on_lines : mapped ? t.mapped : t.off_lines + (t.tn == 192 ? kWide192Ends * 4096 / K : 0);
             const bool split = t.tm == 256 && t.tn == 256 && rem;  // the last positions go to a second launch
             const double cost = split ? rounds_cost(nt - rem, cus, round) + (rem * 4 <= cus ? 33 : 60)
                                       : rounds_cost(tiles(t.tm, t.tn), cus, round);
@@ -237,7 +245,8 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     a.rank = rs ? rs->rank : 0;
     a.seg_rows = (int)((int64_t)M * N / a.BN / a.W);
     const bool counts = (mode == MODE_SIGNAL || mode == MODE_SCATTER) && !quiet;
-    const launch_plan plan = plan_launch(r, M, N, a.BM, a.BN, counts && (monitor || K < kSignalAfterFromK), counts, on_lines(a));
+    const launch_plan plan = plan_launch(r, M, N, K, a.BM, a.BN, counts && (monitor || K < kSignalAfterFromK), counts, on_lines(a),
+                                         mode == MODE_SCATTER || mode == MODE_RS);
     a.grid_m = plan.grid_m; a.grid_n = plan.grid_n; a.panel = plan.panel; a.xcd_remap = plan.xcd_remap;
     a.first = 0; a.sub_m = a.sub_n = 1;
     a.count = plan.count;
@@ -247,6 +256,9 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     a.quiet = quiet || signal_after ? 1 : 0;
     a.stream_out = (int64_t)M * N * 2 > kStreamOutAboveBytes ? 1 : 0;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    // The 128x192 tile that loads whole lines takes all of a CU's LDS and is not built for the epilogues that count; the
+    // reordered store without counters is the accumulating epilogue without an accumulator.
+    if (mode == MODE_SIGNAL && !counts && plan.tm == 128 && plan.tn == 192 && !on_lines(a)) mode = MODE_ACC;
     // the tail split was computed for that many workgroups of the main launch
     rc = launch_tile(dtype, mode, a, plan.tm, plan.tn, s, nullptr, plan.tail ? fo_main_tile_resident() : 0);
     if (rc) return rc;
@@ -343,7 +355,7 @@ extern "C" int fo_gemm_wave_tiles(int dtype, int algo, int M, int N, int32_t *ti
     fo_raster r;
     int rc = fo_pick_raster(algo, M, N, &r);
     if (rc) return rc;
-    const launch_plan plan = plan_launch(r, M, N, e->f[0], e->f[1], false, true, true);
+    const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, true, true, false);
     GemmArgs a = {};
     a.count = plan.count;
     int info[5] = {0, 0, 0, 0, 0};
@@ -361,7 +373,8 @@ extern "C" int fo_gemm_kernel_info(int dtype, int algo, int M, int N, int epilog
     int rc = fo_pick_raster(algo, M, N, &r);
     if (rc) return rc;
     const fo_algo_entry *e = fo_algo_lookup(algo);
-    const launch_plan plan = plan_launch(r, M, N, e->f[0], e->f[1], false, epilogue != MODE_PLAIN, true);
+    const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, epilogue != MODE_PLAIN, true,
+                                         epilogue == MODE_SCATTER);
     GemmArgs a = {};
     a.count = plan.count;
     int out[5] = {0, 0, 0, 0, 0};

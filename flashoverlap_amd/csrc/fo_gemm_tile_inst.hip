@@ -38,6 +38,11 @@ int FO_CAT3(fo_gemm_tile_launch_, FO_INST_DTYPE, _, FO_INST_MODE)(const GemmArgs
         FO_TILE_(96, 128, 64, 5, true)
         FO_TILE_(128, 128, 64, 4, true)
         FO_TILE_(128, 160, 64, 4, true)
+        // The whole of a CU's LDS: no consumer that polls could be on the CU beside it, and the row-mapped epilogues' maps do
+        // not fit.  Only for what moves no counters (fo_gemm.hip).
+#if FO_INST_MODE == 0 || FO_INST_MODE == 3
+        FO_TILE_(128, 192, 64, 4, true)
+#endif
     }
     FO_TILE(32, 32, 128, 8)
     FO_TILE(64, 32, 128, 6)

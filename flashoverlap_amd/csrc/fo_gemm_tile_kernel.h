@@ -44,7 +44,8 @@
 // permute a row's chunks by exclusive or: a fetch takes lanes of two chunk columns in one pass, and with the chunks rotated
 // instead half of this form's LDS time was bank conflicts (exclusive or against rotated: 1152x5120x1720 27.8 -> 26.8 us,
 // 512x4096x4088 23.3 -> 22.6, 384x4096x4088 39.0 -> 36.9, 128x4096x4088 12.7 -> 12.3).  Tiles with room for three
-// stages only (128x192 and larger) keep the plain form: with both stages of a step awaited, nothing would be in flight.
+// stages only (128x256, and 128x192 where a row map takes LDS as well: four stages of it are all a CU has) keep the plain form:
+// with both stages of a step awaited, nothing would be in flight.
 //
 // MODE_ACC, the epilogue of calls that stay on one stream: what the consumer kernel would do behind the GEMM (read C and
 // the accumulator, write the accumulator) is done on the tile in LDS.  The loaders, idle by then, request the
@@ -135,6 +136,9 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
     constexpr unsigned A_BLK = TM * 128, B_BLK = TN * 128, STAGE = KB * (A_BLK + B_BLK);
     constexpr bool ACC = MODE == MODE_ACC || MODE == MODE_RS, COUNTS = MODE == MODE_SIGNAL || MODE == MODE_SCATTER;
     constexpr bool MAPPED = MODE == MODE_SCATTER || MODE == MODE_RS;
+    // Where MODE_ACC also stands for the reordered store without counters (fo_gemm.hip).  (Asked where it need not be, the
+    // question waits for an argument in front of the first further load: 1664x4608x904 in 128x128 tiles 27.1 -> 27.6 us.)
+    constexpr bool MAY_LACK = MODE == MODE_RS || (SHIFT && TM == 128 && TN == 192);
     // output staging; with an accumulator the computing wavefronts store the tile and the loaders update the accumulator
     constexpr int STORERS = ACC ? kTileComputers * 64 : kTileThreads;
     constexpr int PITCH = TN + 8, CPR = TN / 8, NCH = (TM * CPR + STORERS - 1) / STORERS;
@@ -341,7 +345,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             unsigned slot = (S - 1) * STAGE;
             // With an accumulator the steps behind the last request ask for its values instead of further stages: they
             // arrive while the last S - 1 stages are multiplied.
-            const bool sums = ACC && (MODE != MODE_RS || p.ACC);
+            const bool sums = ACC && (!MAY_LACK || p.ACC);
             const int stages = SHIFT ? KT + 1 : KT;
             const int fetching = sums ? (stages > S - 1 ? stages - (S - 1) : 0) : KT;
             for (int kt = 0; kt < fetching; kt++) {

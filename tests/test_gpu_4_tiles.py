@@ -428,3 +428,55 @@ def test_accumulator_requested_during_the_product(fo, dtype, bm, bn, M, N, K):
     assert torch.equal(layout.unpermute(C, M, N, bm, bn, RA), plain)
     assert torch.equal(acc.reshape(-1), (before.float() + C.float()).to(td).reshape(-1))
     ov.close()
+
+
+@pytest.mark.parametrize("dtype,bm,bn,M,N,K", [
+    (BF16, 128, 128, 1152, 5120, 8),      # one chunk of K; the last tile moved back along N, tiles across reorder tiles
+    (F16, 128, 128, 1152, 5120, 72),      # fewer K steps than stages
+    (BF16, 128, 128, 1152, 5120, 1720),
+    (F16, 128, 256, 1536, 3840, 1112),    # whole tiles along N, 256-wide reorder tiles
+    (BF16, 256, 128, 1536, 3712, 456),    # 256-high reorder tiles
+    (F16, 128, 128, 1792, 6912, 712),     # more than one round
+])
+def test_whole_lines_in_128x192_tiles(fo, dtype, bm, bn, M, N, K):
+    """The 128x192 tile whose loads are whole lines: plain, reordered without and with an accumulator, and row-mapped (which it
+    is not built for), each the product of the operands padded to whole lines, bit for bit."""
+    ops, layout, td = fo.ops, fo.layout, TORCH_DTYPE[dtype]
+    algo = fo._capi.find_algo(bm, bn, swizzle=4)
+    TM, TN = M // bm, N // bn
+    T = TM * TN
+    A, _ = seeded((M, K), dtype, M + K)
+    B, _ = seeded((N, K), dtype, N + K, scale=K ** -0.5)
+    before, _ = seeded((M, N), dtype, 13)
+    pad = -K % 64
+    want, C = (torch.full((M, N), float("nan"), device="cuda", dtype=td) for _ in range(2))
+    ops.gemm(*(torch.nn.functional.pad(t, (0, pad)) for t in (A, B)), want, algo)
+    assert max_rel_err(want.float(), A.float() @ B.float().T) <= 1e-2
+    ops.gemm(A, B, C, algo)
+    torch.cuda.synchronize()
+    assert torch.equal(C, want)
+    RA = torch.from_numpy(np.random.default_rng(K).permutation(T).astype(np.int32)).reshape(TM, TN).cuda()
+    cs = torch.tensor([T], dtype=torch.int32)
+    RE = layout.generate_row_mapping(M, N, bm, bn, [T], 2)
+    MM = torch.zeros(layout.counter_size(1, TM, TN), dtype=torch.int32, device="cuda")
+    D = torch.empty(M // 2, N, device="cuda", dtype=td)
+    acc = before.clone()
+    ov = ops.Overlap(world=2)
+    ov.set_schedule(in_stream_below_flop=1e15)
+    for rldn in (1, 2 if T % 2 == 0 else 1):
+        C.fill_(float("nan"))
+        ov.gemm_allreduce_overlap(A, B, C, MM, RA, rldn, cs, cs.cuda(), algo)
+        torch.cuda.synchronize()
+        assert torch.equal(layout.unpermute(C, M, N, bm, bn, RA, rLDN=rldn), want)
+    C.fill_(float("nan"))
+    ov.gemm_reducescatter_overlap(A, B, C, D, MM, RA, RE, 1, cs, cs.cuda(), algo)
+    torch.cuda.synchronize()
+    assert torch.equal(layout.unpermute(C, M, N, bm, bn, RA, RE=RE), want)
+    ov.set_accumulator(acc)
+    C.fill_(float("nan"))
+    ov.gemm_allreduce_overlap(A, B, C, MM, RA, 1, cs, cs.cuda(), algo)
+    torch.cuda.synchronize()
+    assert torch.equal(layout.unpermute(C, M, N, bm, bn, RA), want)
+    assert torch.equal(acc.reshape(-1), (before.float() + C.float()).to(td).reshape(-1))
+    assert (MM == 0).all()
+    ov.close()
