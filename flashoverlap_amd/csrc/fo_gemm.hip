@@ -75,9 +75,19 @@ constexpr int kSignalAfterFromK = 1536;
 // 23.7, 1536x3840x2040 26.7 -> 24.8, 1152x5120x4088 48.5 -> 46.4.
 struct tile_cost {
     int tm, tn, on_lines, off_lines, mapped;
+    double sums;
 };
-constexpr tile_cost kTileCosts[] = {{96, 128, 26, 27, 27},  {128, 128, 31, 33, 33}, {128, 160, 36, 38, 38}, {128, 192, 42, 46, 54},
-                                    {128, 256, 57, 71, 71}, {256, 128, 57, 71, 71}, {256, 256, 97, 110, 110}};
+constexpr tile_cost kTileCosts[] = {{96, 128, 26, 27, 27, 2.2},  {128, 128, 31, 33, 33, 2.3}, {128, 160, 36, 38, 38, 4.4},
+                                    {128, 192, 42, 46, 54, 4.4}, {128, 256, 57, 71, 71, 5},   {256, 128, 57, 71, 71, 5},
+                                    {256, 256, 97, 110, 110, 11}};
+// `sums`: what an accumulator adds to a round, microseconds at any K: its values and sums go to and from memory when the round's
+// tiles are done, with little of the next round's product beside them, and a large tile has more of it to wait for.  Over 219
+// products of more than one round with a cold accumulator and 256 to 640 columns of K the chosen tile was 5.0 % slower than the best
+// one without this term and 1.3 % with it (GEMM alone, us: 6784x3712x312 bf16 54.2 -> 42.7, 128x160 -> 128x128, 6400x3200x400 48.7 ->
+// 39.9, 5120x3456x280 39.3 -> 32.9, 7680x2688x424 50.9 -> 43.8); beyond 640 columns it gains in some and loses in others (241
+// products: 1.1 % without, 1.0 % with it).  Not for a row map, whose sums cost otherwise (3456x4352x328 over eight ranks 32.0
+// us for the whole pass, 41.4 in the tile that it would take).
+constexpr int kSumsBelowK = 640;
 // Beginning and end of a round of 128x192 with its line loads, beyond the other tiles' (us): with few columns of K two rounds
 // of it are no better than three of 128x128 (with an accumulator, us, 2304x5120x264 20.2 and 18.5, 2048x6144x264 20.7 and 19.8,
 // 2048x6144x776 40.7 and 42.8).
@@ -109,7 +119,7 @@ double rounds_cost(long count, long cus, double round) {
 // M and N need only be multiples of 128: the last tile of a dimension is moved back or, 256x256, repeats half of its
 // neighbour.
 launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN, bool whole_only, bool counted, bool on_lines,
-                        bool mapped) {
+                        bool mapped, bool acc) {
     launch_plan p;
     p.tail = p.tail_tm = p.tail_tn = 0;
     auto set = [&](int tm, int tn) {
@@ -152,13 +162,19 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN,
     const long nt = tiles(256, 256);
     const int rem = square ? r.tail_tiles : nt > cus && nt % cus * 2 <= cus ? (int)(nt % cus) : 0;
     if (!counted) {
+        const bool sums = acc && !mapped && K < kSumsBelowK;
         const tile_cost *best = nullptr;
         double least = 0;
         for (const tile_cost &t : kTileCosts) {
             if (M < t.tm || N < t.tn) continue;
-            const double round = on_lines ? t.on_lines : mapped ? t.mapped : t.off_lines + (t.tn == 192 ? kWide192Ends * 4096 / K : 0);
+            double round = on_lines ? t.on_lines : mapped ? t.mapped : t.off_lines;
+            if (sums)
+                round += t.sums * 4096 / K;
+            else if (!on_lines && !mapped && t.tn == 192)
+                round += kWide192Ends * 4096 / K;
             const bool split = t.tm == 256 && t.tn == 256 && rem;  // the last positions go to a second launch
-            const double cost = split ? rounds_cost(nt - rem, cus, round) + (rem * 4 <= cus ? 33 : 60)
+            const double second = rem * 4 <= cus ? 33 : 60, second_sums = rem * 4 <= cus ? 2.3 : 5;  // 128x128 or 128x256 tiles
+            const double cost = split ? rounds_cost(nt - rem, cus, round) + second + (sums ? second_sums * 4096 / K : 0)
                                       : rounds_cost(tiles(t.tm, t.tn), cus, round);
             if (best && cost >= least) continue;
             best = &t;
@@ -246,7 +262,7 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     a.seg_rows = (int)((int64_t)M * N / a.BN / a.W);
     const bool counts = (mode == MODE_SIGNAL || mode == MODE_SCATTER) && !quiet;
     const launch_plan plan = plan_launch(r, M, N, K, a.BM, a.BN, counts && (monitor || K < kSignalAfterFromK), counts, on_lines(a),
-                                         mode == MODE_SCATTER || mode == MODE_RS);
+                                         mode == MODE_SCATTER || mode == MODE_RS, acc != nullptr);
     a.grid_m = plan.grid_m; a.grid_n = plan.grid_n; a.panel = plan.panel; a.xcd_remap = plan.xcd_remap;
     a.first = 0; a.sub_m = a.sub_n = 1;
     a.count = plan.count;
@@ -355,7 +371,7 @@ extern "C" int fo_gemm_wave_tiles(int dtype, int algo, int M, int N, int32_t *ti
     fo_raster r;
     int rc = fo_pick_raster(algo, M, N, &r);
     if (rc) return rc;
-    const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, true, true, false);
+    const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, true, true, false, false);
     GemmArgs a = {};
     a.count = plan.count;
     int info[5] = {0, 0, 0, 0, 0};
@@ -374,7 +390,7 @@ extern "C" int fo_gemm_kernel_info(int dtype, int algo, int M, int N, int epilog
     if (rc) return rc;
     const fo_algo_entry *e = fo_algo_lookup(algo);
     const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, epilogue != MODE_PLAIN, true,
-                                         epilogue == MODE_SCATTER);
+                                         epilogue == MODE_SCATTER, false);
     GemmArgs a = {};
     a.count = plan.count;
     int out[5] = {0, 0, 0, 0, 0};
