@@ -9,18 +9,22 @@
 int fo_gemm_dev::fo_gemm256_launch(int dtype, int mode, const GemmArgs &a, hipStream_t stream, int *resident_out,
                                    int expect_resident) {
     if (a.lda != a.ldb) return FO_ERR_ARG;  // the kernel addresses both operands with one leading dimension
-    const int key = (dtype == FO_BF16 ? 5 : 0) + mode;
+    const int key = (dtype == FO_BF16 ? 7 : 0) + mode;
     switch (key) {
         case 0: return fo_gemm256_launch_0_0(a, stream, resident_out, expect_resident);
         case 1: return fo_gemm256_launch_0_1(a, stream, resident_out, expect_resident);
         case 2: return fo_gemm256_launch_0_2(a, stream, resident_out, expect_resident);
         case 3: return fo_gemm256_launch_0_3(a, stream, resident_out, expect_resident);
         case 4: return fo_gemm256_launch_0_4(a, stream, resident_out, expect_resident);
-        case 5: return fo_gemm256_launch_1_0(a, stream, resident_out, expect_resident);
-        case 6: return fo_gemm256_launch_1_1(a, stream, resident_out, expect_resident);
-        case 7: return fo_gemm256_launch_1_2(a, stream, resident_out, expect_resident);
-        case 8: return fo_gemm256_launch_1_3(a, stream, resident_out, expect_resident);
-        case 9: return fo_gemm256_launch_1_4(a, stream, resident_out, expect_resident);
+        case 5: return fo_gemm256_launch_0_5(a, stream, resident_out, expect_resident);
+        case 6: return fo_gemm256_launch_0_6(a, stream, resident_out, expect_resident);
+        case 7: return fo_gemm256_launch_1_0(a, stream, resident_out, expect_resident);
+        case 8: return fo_gemm256_launch_1_1(a, stream, resident_out, expect_resident);
+        case 9: return fo_gemm256_launch_1_2(a, stream, resident_out, expect_resident);
+        case 10: return fo_gemm256_launch_1_3(a, stream, resident_out, expect_resident);
+        case 11: return fo_gemm256_launch_1_4(a, stream, resident_out, expect_resident);
+        case 12: return fo_gemm256_launch_1_5(a, stream, resident_out, expect_resident);
+        case 13: return fo_gemm256_launch_1_6(a, stream, resident_out, expect_resident);
     }
     return FO_ERR_ARG;
 }
@@ -197,6 +201,11 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN,
     return p;
 }
 
+// Whether a launch that counts can do the sums of its last wave itself (MODE_SIGNAL_SUM, MODE_SCATTER_SUM).
+bool last_wave_sums(const launch_plan &p) {
+    return p.tm == 256 && p.tn == 256 && !p.tail && p.count > fo_main_tile_resident();
+}
+
 // Signals of a launch whose workgroup tiles are parts of reorder tiles: behind it on the stream, everything at once
 // (such a launch is a single round of short tiles; its reorder tiles complete together anyway).  MM[g] += cseg[g].
 __global__ __launch_bounds__(256) void fo_signal_all_kernel(const int32_t *cseg, int G, int32_t *MM) {
@@ -238,7 +247,7 @@ int check_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t
 int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *cseg, int G,
              const void *A, const void *B, void *C, int32_t *MM, const int32_t *RA,
              const int32_t *RE, int monitor, int algo, fo_stream_t stream, bool quiet = false, void *acc = nullptr,
-             const rs_args *rs = nullptr) {
+             const rs_args *rs = nullptr, int sum_from = -1) {
     int rc = check_gemm(mode, dtype, M, N, K, rLDN, cseg, G, A, B, C, MM, RA, RE, monitor, algo, quiet, acc);
     if (rc) return rc;
     const fo_algo_entry *e = fo_algo_lookup(algo);
@@ -275,6 +284,11 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     // The 128x192 tile that loads whole lines takes all of a CU's LDS and is not built for the epilogues that count; the
     // reordered store without counters is the accumulating epilogue without an accumulator.
     if (mode == MODE_SIGNAL && !counts && plan.tm == 128 && plan.tn == 192 && !on_lines(a)) mode = MODE_ACC;
+    a.sum_from = sum_from;
+    if (sum_from >= 0) {
+        if (!last_wave_sums(plan) || monitor || !acc) return FO_ERR_STATE;
+        mode = mode == MODE_SCATTER ? MODE_SCATTER_SUM : MODE_SIGNAL_SUM;
+    }
     // the tail split was computed for that many workgroups of the main launch
     rc = launch_tile(dtype, mode, a, plan.tm, plan.tn, s, nullptr, plan.tail ? fo_main_tile_resident() : 0);
     if (rc) return rc;
@@ -362,6 +376,27 @@ int fo_gemm_reduce_scatter(int dtype, int M, int N, int K, const int32_t *cseg_d
     if (W <= 0 || rank < 0 || rank >= W || e->f[0] % W || (((uintptr_t)C | (uintptr_t)acc | (uintptr_t)own) & 15)) return FO_ERR_ARG;
     const rs_args rs = {own, W, rank};
     return run_gemm(MODE_RS, dtype, M, N, K, 1, cseg_dev, G, A, B, C, nullptr, RA, RE, 0, algo, stream, true, acc, &rs);
+}
+
+int fo_gemm_last_wave(int algo, int M, int N, int32_t *first) {
+    const fo_algo_entry *e = fo_algo_lookup(algo);
+    if (!e) return FO_ERR_ALGO;
+    fo_raster r;
+    int rc = fo_pick_raster(algo, M, N, &r);
+    if (rc) return rc;
+    const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, true, true, false, false);
+    const int resident = fo_main_tile_resident();
+    *first = last_wave_sums(plan) ? (plan.count - 1) / resident * resident * (256 / e->f[0]) * (256 / e->f[1])
+                                  : (M / e->f[0]) * (N / e->f[1]);
+    return FO_OK;
+}
+
+int fo_gemm_signal_sums(int dtype, int M, int N, int K, int rLDN, const int32_t *cseg_dev, int G, const void *A, const void *B,
+                        void *C, int32_t *MM, const int32_t *RA, const int32_t *RE, void *acc, int sum_from, void *own, int W,
+                        int rank, int algo, fo_stream_t stream) {
+    const rs_args rs = {own, W, rank};
+    return run_gemm(RE ? MODE_SCATTER : MODE_SIGNAL, dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, MM, RA, RE, 0, algo, stream, false,
+                    acc, &rs, sum_from);
 }
 
 extern "C" int fo_gemm_wave_tiles(int dtype, int algo, int M, int N, int32_t *tiles) {

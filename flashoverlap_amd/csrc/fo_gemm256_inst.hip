@@ -1,12 +1,12 @@
 // One instantiation of the 256x256 GEMM kernel per translation unit (the kernel's
 // K step is a single unrolled body of 128 MFMAs and takes minutes to compile):
-// built ten times with -DFO_INST_DTYPE={0,1} (fp16, bf16) and -DFO_INST_MODE={0,1,2,3,4}
-// (plain, signal, scatter, accumulating, reduce-scatter epilogue).
+// built 14 times with -DFO_INST_DTYPE={0,1} (fp16, bf16) and -DFO_INST_MODE={0,1,2,3,4,5,6}
+// (plain, signal, scatter, accumulating, reduce-scatter epilogue; signal and scatter with the last wave's sums).
 #include "fo_gemm256_kernel.h"
 #include "fo_gemm_launch.h"
 
 #if !defined(FO_INST_DTYPE) || !defined(FO_INST_MODE)
-#error "compile with -DFO_INST_DTYPE=0|1 -DFO_INST_MODE=0|1|2|3|4"
+#error "compile with -DFO_INST_DTYPE=0|1 -DFO_INST_MODE=0|1|2|3|4|5|6"
 #endif
 
 namespace fo_gemm_dev {

@@ -147,8 +147,10 @@ template <typename Tag, int MODE>
 __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     typedef fo_elem<Tag> E;
     typedef fo_mfma256<Tag> X;
-    constexpr bool ACC = MODE == MODE_ACC || MODE == MODE_RS, COUNTS = MODE == MODE_SIGNAL || MODE == MODE_SCATTER;
-    constexpr bool MAPPED = MODE == MODE_SCATTER || MODE == MODE_RS;
+    constexpr bool SUMS = MODE == MODE_SIGNAL_SUM || MODE == MODE_SCATTER_SUM;
+    constexpr bool ACC = MODE == MODE_ACC || MODE == MODE_RS, COUNTS = MODE == MODE_SIGNAL || MODE == MODE_SCATTER || SUMS;
+    constexpr bool MAPPED = MODE == MODE_SCATTER || MODE == MODE_RS || MODE == MODE_SCATTER_SUM;
+    constexpr bool TO_RANKS = MODE == MODE_RS || MODE == MODE_SCATTER_SUM;  // sums go where a reduce-scatter takes them
     constexpr int MT = 256, BK = 64, F = 8, ROWS = 16;
     constexpr int FREE = 9;   // row behind whose MFMAs the step's slot is given up
     constexpr int PUB = 12;   // row behind whose MFMAs the next step's slot is published
@@ -291,7 +293,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     const bool reg_search = p.G <= kPrefixRegs;
     const bool signalling = COUNTS && !p.quiet;
     const bool reorder = MODE == MODE_ACC ? p.RA != nullptr : COUNTS || MODE == MODE_RS;
-    const bool groups = signalling || MODE == MODE_RS;  // group sizes are needed
+    const bool groups = signalling || TO_RANKS;  // group sizes are needed
     // The group sizes are requested in front of the pipeline fill and summed behind it (a round trip to memory and
     // some two dozen dependent cross-lane steps otherwise stand between the kernel's start and its first operand
     // load).  The requests are assembly: their registers are read only behind the fill's wait for loads that were
@@ -608,21 +610,42 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             const bool keep = !((repeated & 1) && wm == 0) && !((repeated & 2) && wn == 0);  // wave-uniform
             // The accumulator's values are awaited together, in front of the first store: a later wait would count the
             // stores between them as well.
-            char *abase = ACC ? reinterpret_cast<char *>(p.ACC) + (trow * ldp + tcol) * 2 : nullptr;
-            // MODE_RS: the accumulator rows of the wavefront's rows, held as re_lo and re_hi are.
+            char *abase = ACC || SUMS ? reinterpret_cast<char *>(p.ACC) + (trow * ldp + tcol) * 2 : nullptr;
+            // TO_RANKS: the accumulator rows of the wavefront's rows, held as re_lo and re_hi are.
             int ac_lo = 0, ac_hi = 0;
-            const bool sums = MODE == MODE_ACC || (MODE == MODE_RS && p.ACC);
-            const int own_first = MODE == MODE_RS ? p.rank * p.seg_rows : 0, own_rows = MODE == MODE_RS && p.OWN ? p.seg_rows : 0;
+            const bool sums = MODE == MODE_ACC || (MODE == MODE_RS && p.ACC) || (SUMS && r >= p.sum_from);  // wave-uniform
+            const int own_first = TO_RANKS ? p.rank * p.seg_rows : 0, own_rows = TO_RANKS && p.OWN && (sums || !SUMS) ? p.seg_rows : 0;
             auto row_of = [&](int k, int lo, int hi) __attribute__((always_inline)) {  // row k * RPP + srow of the block: its entry sits in that lane
                 return __builtin_amdgcn_ds_bpermute((k * RPP % 64 + srow) * 4, k * RPP < 64 ? lo : hi);
             };
-            if (MODE == MODE_RS) {
+            if (MODE == MODE_RS || (MODE == MODE_SCATTER_SUM && sums)) {
                 int first, count;
                 group_range(r, &first, &count);
                 ac_lo = rs_row(p.cseg, p.G, p.BM, p.W, p.seg_rows, re_lo, first * p.BM, count * p.BM);
                 ac_hi = rs_row(p.cseg, p.G, p.BM, p.W, p.seg_rows, re_hi, first * p.BM, count * p.BM);
             }
-            if (sums && keep && !early) {
+            // SUMS, in the workgroup's last tile: the accumulator's values travel into the two slots, which nobody reads any more,
+            // piece by piece in the order in which they are wanted: a wavefront's pieces lie where its operand loads went, each
+            // lane's where it reads them, and no other wavefront has part in it.  (In registers, as with MODE_ACC, they would
+            // leave no room on the SIMD for the consumer that runs beside the earlier waves.)
+            auto piece_lds = [&](int k) __attribute__((always_inline)) { return (wa0 ^ (k / 16 * SLOT_B)) + k % 16 * CHUNK_B; };
+            if (SUMS && sums && !has_next) {
+                if (MAPPED) asm volatile("" : "+v"(re_lo), "+v"(re_hi), "+v"(ac_lo), "+v"(ac_hi));  // nothing else is awaited behind the loads
+                unsigned rows = 0, rows_step = __builtin_amdgcn_readfirstlane(RPP * ldp * 2);
+                const fo_srd_t from = fo_make_srd(TO_RANKS ? reinterpret_cast<char *>(p.ACC) : abase, 0x7fffffffu);
+#pragma unroll
+                for (int k = 0; k < NST; k++) {
+                    if (TO_RANKS) {
+                        const int to = row_of(k, ac_lo, ac_hi);
+                        dma_buf16(from, to < 0 ? 0x80000000u : (unsigned)(to * ldp + (int)tcol + scol * 8) * 2, 0, piece_lds(k));
+                    } else {
+                        dma_buf16(from, lane_off, rows, piece_lds(k));
+                        rows += rows_step;
+                        asm volatile("" : "+s"(rows));  // one scalar, not one for each piece
+                    }
+                }
+            }
+            if (ACC && sums && keep && !early) {
 #pragma unroll
                 for (int k = 0; k < NST; k++) {
                     if (MODE == MODE_RS) {
@@ -639,6 +662,8 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
 #pragma unroll
             for (int i = 0; i < F; i++) {  // 16 output rows = one row of accumulator blocks
                 __builtin_amdgcn_sched_barrier(0);
+                int pitch = ldp;
+                if (SUMS) asm volatile("" : "+s"(pitch));  // a strip's offsets are computed in the strip
 #pragma unroll
                 for (int j = 0; j < F; j++) {
                     fo_float4v a4 = acc[i][j];
@@ -652,10 +677,42 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_s_waitcnt(0xC07F);
                 __builtin_amdgcn_wave_barrier();
-                if (sums && i == 0) {
+                if (ACC && sums && i == 0) {
 #pragma unroll
                     for (int k = 0; k < NST; k++) asm volatile("" : "+v"(old[ACC ? k : 0]));
                 }
+                if (SUMS && sums && !has_next) {
+                    // this strip's values have landed; behind them the later strips' and the stores of the earlier ones
+                    constexpr int PER = MODE == MODE_SIGNAL_SUM ? 2 * (16 / RPP) : 16 / RPP;
+                    switch (i) {  // i is a constant: the loop is unrolled
+                        case 0: wait_vmcnt<28>(); break;
+                        case 1: wait_vmcnt<24 + PER>(); break;
+                        case 2: wait_vmcnt<20 + 2 * PER>(); break;
+                        case 3: wait_vmcnt<16 + 3 * PER>(); break;
+                        case 4: wait_vmcnt<12 + 4 * PER>(); break;
+                        case 5: wait_vmcnt<8 + 5 * PER>(); break;
+                        case 6: wait_vmcnt<4 + 6 * PER>(); break;
+                        default: wait_vmcnt<7 * PER>(); break;
+                    }
+                    asm volatile("" ::: "memory");
+                }
+                // SUMS: the accumulator's piece k; in another than the last tile, which a caller's own order of the slots may
+                // ask for, from memory
+                auto value_of = [&](int k) __attribute__((always_inline)) {
+                    fo_u32x4 x;
+                    if (!has_next) {
+                        x = *reinterpret_cast<lds16_t>(piece_lds(k) + el * 16);
+                    } else {
+                        if (TO_RANKS) {
+                            const int to = row_of(k, ac_lo, ac_hi);
+                            x = *reinterpret_cast<const fo_u32x4 *>(p.ACC + (size_t)(to < 0 ? 0 : to) * pitch + tcol + scol * 8);
+                        } else {
+                            x = *reinterpret_cast<const fo_u32x4 *>(abase + (size_t)(k * RPP) * pitch * 2 + lane_off);
+                        }
+                        asm volatile("" : "+v"(x));  // awaited here: where the two ways meet, the other one would wait for its stores
+                    }
+                    return x;
+                };
                 if (keep)
 #pragma unroll
                 for (int ps = 0; ps < 16 / RPP; ps++) {
@@ -664,13 +721,13 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                     if (MAPPED) {
                         const int k = i * (16 / RPP) + ps;
                         const long prow = row_of(k, re_lo, re_hi);
-                        uint16_t *to = p.C + (size_t)prow * ldp + tcol + scol * 8;
-                        if (MODE == MODE_RS) {
+                        uint16_t *to = p.C + (size_t)prow * pitch + tcol + scol * 8;
+                        if (TO_RANKS && (ACC || sums)) {
                             const int ac = row_of(k, ac_lo, ac_hi);
                             if (sums && ac >= 0)
-                                store16_write_through(p.ACC + (size_t)ac * ldp + tcol + scol * 8, fo_add8<Tag>(old[ACC ? k : 0], v));
+                                store16_write_through(p.ACC + (size_t)ac * pitch + tcol + scol * 8, fo_add8<Tag>(SUMS ? value_of(k) : old[ACC ? k : 0], v));
                             if ((unsigned)(ac - own_first) < (unsigned)own_rows)
-                                store16_write_through(p.OWN + (size_t)(ac - own_first) * ldp + tcol + scol * 8, v);
+                                store16_write_through(p.OWN + (size_t)(ac - own_first) * pitch + tcol + scol * 8, v);
                             store16_write_through(to, v);
                         } else if (stream_out) {
                             store16_write_through_nt(to, v);
@@ -678,20 +735,23 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                             store16_write_through(to, v);
                         }
                     } else {
-                        char *sb = cbase + (size_t)(i * 16 + ps * RPP) * ldp * 2;
-                        if constexpr (MODE == MODE_ACC) {
-                            char *ab = abase + (size_t)(i * 16 + ps * RPP) * ldp * 2;
-                            const fo_u32x4 sum = fo_add8<Tag>(old[i * (16 / RPP) + ps], v);
-                            if (stream_out)
-                                store16_write_through_nt(ab, lane_off, sum);
-                            else
-                                store16_write_through(ab, lane_off, sum);
+                        char *sb = cbase + (size_t)(i * 16 + ps * RPP) * pitch * 2;
+                        if constexpr (MODE == MODE_ACC || MODE == MODE_SIGNAL_SUM) {
+                            if (sums) {
+                                char *ab = abase + (size_t)(i * 16 + ps * RPP) * pitch * 2;
+                                const fo_u32x4 sum = fo_add8<Tag>(SUMS ? value_of(i * (16 / RPP) + ps) : old[ACC ? i * (16 / RPP) + ps : 0], v);
+                                if (stream_out)
+                                    store16_write_through_nt(ab, lane_off, sum);
+                                else
+                                    store16_write_through(ab, lane_off, sum);
+                            }
                         }
                         if (stream_out)
                             store16_write_through_nt(sb, lane_off, v);
                         else
                             store16_write_through(sb, lane_off, v);
                     }
+                    if (SUMS) __builtin_amdgcn_sched_barrier(0);  // a piece at a time: four take more registers than the kernels beside this one leave
                 }
                 __builtin_amdgcn_s_waitcnt(0xC07F);  // strip reads done before the next pass overwrites it
                 __builtin_amdgcn_wave_barrier();
@@ -710,8 +770,8 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
 #pragma unroll
                 for (int s = 0; s < kMaxSub; s++) {
                     if (s < nsub && !((repeated & 1) && s < sub_n) && !((repeated & 2) && s % sub_n == 0)) {
-                        const int g = group_of(__builtin_amdgcn_readlane(v_done, s));
-                        v_g = lane == s ? g : v_g;
+                        const int slot = __builtin_amdgcn_readlane(v_done, s), g = group_of(slot);
+                        v_g = lane == s && !(SUMS && slot >= p.sum_from) ? g : v_g;
                     }
                 }
             }

@@ -40,7 +40,9 @@ __device__ __forceinline__ void static_for(F &&f) {
 // MODE_RS: the same for a reduce-scatter (the scatter epilogue's row map, rLDN == 1): C is cut into ranges of rows, one
 // per group, and each range into W chunks of consecutive rows; row i of chunk q of a range that starts at row f is added
 // to row q * seg_rows + f / W + i of the accumulator (if any) and, for q == rank, stored to row f / W + i of OWN (if any).
-enum { MODE_PLAIN = 0, MODE_SIGNAL = 1, MODE_SCATTER = 2, MODE_ACC = 3, MODE_RS = 4 };
+// MODE_SIGNAL_SUM, MODE_SCATTER_SUM (256x256 kernel only): the signal and scatter epilogues where tiles from storage slot
+// sum_from on are not counted but added to the accumulator as MODE_ACC and MODE_RS do.
+enum { MODE_PLAIN = 0, MODE_SIGNAL = 1, MODE_SCATTER = 2, MODE_ACC = 3, MODE_RS = 4, MODE_SIGNAL_SUM = 5, MODE_SCATTER_SUM = 6 };
 
 // Division by a number that the host knows: n / d for n and d below 32768, exactly (the product exceeds n / d * 2^31 by
 // less than n * d).
@@ -77,6 +79,7 @@ struct GemmArgs {
     uint16_t *OWN;                         // MODE_RS: this rank's rows
     int W, rank, seg_rows;                 // MODE_RS: ranks, this rank, rows of the view per rank
     int stream_out;                        // 256x256 kernel: store the output with the non-temporal hint
+    int sum_from;                          // MODE_SIGNAL_SUM, MODE_SCATTER_SUM: first storage slot that is summed
 };
 
 inline void fo_set_divisors(GemmArgs &a) {

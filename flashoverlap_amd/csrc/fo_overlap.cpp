@@ -143,6 +143,17 @@ int batch_end(const int32_t *cseg_host, int G, int i, long done, int wave) {
     return j;
 }
 
+// Storage slots of the batches in front of the last.
+long slots_before_last_batch(const int32_t *cseg_host, int G, int wave) {
+    long done = 0;
+    for (int i = 0; i < G;) {
+        const int j = batch_end(cseg_host, G, i, done, wave);
+        if (j == G) break;
+        for (; i < j; i++) done += cseg_host[i];
+    }
+    return done;
+}
+
 // Link time of `bytes` on `stream` (nothing without a rate).
 int link_time(const fo_overlap *h, int64_t bytes, fo_stream_t stream) {
     if (h->link_bytes_per_s <= 0 || bytes <= 0) return FO_OK;
@@ -530,8 +541,27 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
     const bool quiet = same_stream && !monitor;
     // With nothing to wait for, the GEMM's epilogue does the consumer's work on the tile it holds in LDS.
     const int64_t mn = (int64_t)M * N;
-    const bool consumed = quiet && h->acc && apart({h->acc, mn}, {{A, (int64_t)M * K}, {B, (int64_t)N * K}, {C, mn}});
-    rc = consumed ? fo_gemm_accumulate(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, h->acc, RA, algo, h->gemm_stream)
+    const bool acc_apart = h->acc && apart({h->acc, mn}, {{A, (int64_t)M * K}, {B, (int64_t)N * K}, {C, mn}});
+    const bool consumed = quiet && acc_apart;
+    // The last wave's sums by the GEMM itself, from storage slot sum_from on: nothing is left to overlap them with, and behind
+    // the GEMM they are a wait, a launch and a second read of the product (17 + 4 us on 4096x8192, of which the GEMM's epilogue
+    // takes 17).  Where the groups' ends are not the waves', the consumer also need not wait for the last wave to begin with the
+    // rest of its first group.  Whole calls, us, consumer -> GEMM: groups across waves, 8192x8192x2048 in one 288 -> 274, 8192x4096x4096
+    // in three 253 -> 242, by the pair of calls 8192x4096x2560 in one 203 -> 184; groups that end with waves, by the pair
+    // 4096x8192x8192 422 -> 419, 8192x8192x8192 828 -> 824.  There the call that also normalises keeps its one kernel for the last
+    // batch's sums and rows (4096x8192x1536 131 against 135 with sums in the GEMM).
+    int32_t sum_from = TM * TN;
+    if (!same_stream && !fused && !monitor && h->link_bytes_per_s <= 0 && acc_apart &&
+        (!np || apart({h->acc, mn}, {{np->Y, mn}, {np->Wt, N}}))) {
+        int32_t first = 0;
+        rc = fo_gemm_last_wave(algo, M, N, &first);
+        if (rc) return rc;
+        if (!np || slots_before_last_batch(cseg_host, G, wave) < first) sum_from = first;
+    }
+    const bool sums_last = sum_from < TM * TN;
+    rc = sums_last  ? fo_gemm_signal_sums(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, MM, RA, nullptr, h->acc, sum_from, nullptr, 1, 0,
+                                          algo, h->gemm_stream)
+         : consumed ? fo_gemm_accumulate(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, h->acc, RA, algo, h->gemm_stream)
          : quiet  ? fo_gemm_reordered_quiet(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, RA, nullptr, algo,
                                             h->gemm_stream)
                   : fo_gemm_signal(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, MM, RA, monitor, algo,
@@ -563,20 +593,27 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
             const int j = batch_end(cseg_host, G, i, done, wave);
             long tiles = 0;
             for (int g = i; g < j; g++) tiles += cseg_host[g];
+            // The batch that the last wave completes: what is left to the consumer is the beginning of its first group, if
+            // that began in an earlier wave.  The GEMM counts no more of it than that.
+            const bool last_wave = done + tiles > sum_from;
+            if (last_wave) tiles = done < sum_from ? sum_from - done : 0;
             const int64_t n = tiles * tile_elems;
+            if (last_wave && !tiles) break;
             if (!quiet) {
                 int32_t *gave_up = h->workspace ? h->workspace + kWsGaveUp : nullptr;
-                rc = j - i == 1 ? fo_wait_with(cseg_host[i], MM + i, h->max_polls, gave_up, cstream)  // resets the counter
+                rc = last_wave  ? fo_wait_with((int)tiles, MM + i, h->max_polls, gave_up, cstream)
+                     : j - i == 1 ? fo_wait_with(cseg_host[i], MM + i, h->max_polls, gave_up, cstream)  // resets the counter
                                 : fo_wait_groups_with(j - i, cseg_dev + i, MM + i, h->max_polls, gave_up, cstream);
                 if (rc) return rc;
             }
             std::vector<int> runs;
-            if (np && !same_stream) ready_tile_rows(last_slot.data(), TM, done + tiles, j == G, runs);
-            const bool with_rows = consumes_rows && rows_together(M, N, K, info[1], rLDN, (int)runs.size() / 2, j == G) &&
+            const bool behind_gemm = j == G && !last_wave;  // every batch but the last runs beside the GEMM
+            if (np && !same_stream) ready_tile_rows(last_slot.data(), TM, done + tiles, behind_gemm, runs);
+            const bool with_rows = consumes_rows && rows_together(M, N, K, info[1], rLDN, (int)runs.size() / 2, behind_gemm) &&
                                    whole_rows(np->RA_host, TN, runs, done, tiles);
             if (acc && !consumed && !with_rows) {  // the groups of a batch are one contiguous range
                 rc = fo_consumer_reduce_with(dtype, c + off, acc + off, n, 1, 0, nullptr, 0, stream_acc, cstream,
-                                             j < G && !same_stream);  // every batch but the last runs beside the GEMM
+                                             !behind_gemm && !same_stream);
                 if (rc) return rc;
             }
             rc = link_time(h, n * 2, cstream);
@@ -589,14 +626,20 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
             } else if (with_rows) {
                 for (size_t k = 0; k + 1 < runs.size(); k += 2) {
                     rc = fo_consume_norm_rows_with(dtype, C, acc, np->Y, np->Wt, runs[k] * info[0], (runs[k + 1] - runs[k]) * info[0], M, N,
-                                                   info[0], info[1], RA, np->eps, fo_streams(mn * 4), j < G, cstream);
+                                                   info[0], info[1], RA, np->eps, fo_streams(mn * 4), !behind_gemm, cstream);
                     if (rc) return rc;
                 }
             } else if (np) {
-                rc = norm_runs(*np, runs, dtype, C, M, N, info[0], info[1], rLDN, RA, j < G, cstream);
+                rc = norm_runs(*np, runs, dtype, C, M, N, info[0], info[1], rLDN, RA, !behind_gemm, cstream);
                 if (rc) return rc;
             }
             i = j;
+        }
+        if (sums_last && np) {  // the rows that the last wave completed: nothing but the GEMM in front of them
+            std::vector<int> runs;
+            ready_tile_rows(last_slot.data(), TM, (long)TM * TN, true, runs);
+            rc = norm_runs(*np, runs, dtype, C, M, N, info[0], info[1], rLDN, RA, false, h->gemm_stream);
+            if (rc) return rc;
         }
     }
     return same_stream ? FO_OK : join(h, captured);
@@ -737,8 +780,22 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
         if (rc) return rc;
         return link_time(h, (int64_t)M * N * 2, h->gemm_stream);
     }
+    // The last batch's sums and rows by the GEMM itself, where that batch is of the last wave only (us: 8192x4096x4096, eight ranks
+    // 235.6 -> 230.4, 8192x8192x3584 bf16 398 -> 389, 4096x8192x2048 bf16 146.7 -> 143.3).
+    int32_t sum_from = TM * TN;
+    if (!same_stream && !fused && !monitor && h->link_bytes_per_s <= 0 && by_epilogue && h->acc && W > 1 &&
+        (int64_t)M * N * 2 <= 0x7FFFFFFFLL) {
+        int32_t first = 0;
+        rc = fo_gemm_last_wave(algo, M, N, &first);
+        if (rc) return rc;
+        const long before = slots_before_last_batch(cseg_host, G, wave);
+        if (before >= first) sum_from = (int32_t)before;
+    }
     rc = quiet ? fo_gemm_reordered_quiet(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, RA, RE, algo,
                                          h->gemm_stream)
+         : sum_from < TM * TN
+             ? fo_gemm_signal_sums(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, MM, RA, RE, h->acc, sum_from, D, W, h->rank, algo,
+                                   h->gemm_stream)
                : fo_gemm_scatter(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, MM, RA, RE, monitor, algo,
                                  h->gemm_stream);
     if (rc) return rc;
@@ -759,6 +816,7 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     int64_t off = 0;
     long done = 0;
     for (int i = 0; i < G;) {
+        if (done >= sum_from) break;
         const int j = fused ? i + 1 : batch_end(cseg_host, G, i, done, wave);
         const int64_t off_batch = off;
         if (!fused && !quiet) {
