@@ -82,11 +82,11 @@ namespace {
 // follows each consumer launch, and it is what the second stream is there to hide.
 //
 // Longer GEMMs stay on one stream too where there is nothing to overlap: `idle`, a call without a consumer and without a
-// normalisation (4224x7168x3584 221 -> 215 us, 3712x8192x3456 216 -> 207), and a product of less than about one round of
-// 256x256 tiles, whose groups all complete at its end, so that the second stream adds its launches and polls and hides
+// normalisation (4224x7168x3584 221 -> 215 us, 3712x8192x3456 216 -> 207), and a product of at most one round of 256x256
+// tiles, whose groups all complete at its end, so that the second stream adds its launches and polls and hides
 // nothing (us, two streams -> one: 2304x4096x3560 96 -> 83, 1792x4608x4520 125 -> 108, 2048x4224x6968 256 -> 167,
-// 2176x5888x3312 133 -> 127, 207 of 256 tiles; with 231 tiles, 5376x2688x3544, 141 -> 147).  in_stream_below_flop = 0
-// still asks for two streams always.
+// 2176x5888x3312 133 -> 127, 4096x4096x4096 133 -> 125, 2048x8192x3000 128 -> 118).  `scatter`, a reduce-scatter: up to five
+// sixths of a round (4096x4096x2560 with four ranks 98 -> 100).  in_stream_below_flop = 0 still asks for two streams always.
 //
 // `ragged`, a call that could do either and whose M or N is an odd multiple of 128: a launch that counts keeps the order of
 // the groups in the Algo's own tile (plan_launch), one that does not takes 256x256 tiles with half tiles at the end, and
@@ -94,12 +94,31 @@ namespace {
 // 3456x4352x3072 127 -> 93, 2432x7040x7056 271 -> 245, 8064x8064x4096 586 -> 465, 6272x8192x7168 661 -> 636; reduce-scatter,
 // eight ranks: 3456x4352x3072 123 -> 95, 4224x7168x3584 205 -> 194, 6272x8192x7168 651 -> 630, 8192x8064x7168 801 -> 751).
 // `fits`: the accumulator is one that every path takes; one that is not aligned is left to the one-launch consumer.
-bool in_stream(const fo_overlap *h, int M, int N, int K, bool idle, bool monitor, bool ragged, bool fits) {
+bool in_stream(const fo_overlap *h, int M, int N, int K, bool idle, bool monitor, bool ragged, bool fits, bool scatter) {
     if (!h->comm_stream) return true;
     if (h->fused >= 0 || h->link_bytes_per_s > 0 || h->in_stream_below_flop <= 0) return false;
     if (2.0 * M * N * K < h->in_stream_below_flop) return true;
     if (monitor || !fits) return false;  // the monitor's GEMM counts and is waited for in any case
-    return idle || ragged || (long)((M + 255) / 256) * ((N + 255) / 256) * 6 <= (long)fo_main_tile_resident() * 5;
+    return idle || ragged || (long)((M + 255) / 256) * ((N + 255) / 256) * 6 <= (long)fo_main_tile_resident() * (scatter ? 5 : 6);
+}
+
+// An all-reduce that could do either, longer than all of those: whether the GEMM's epilogue, which does the sums while the tile
+// is in LDS and asks for the accumulator's values during the product, costs less than the consumer beside the GEMM, which reads
+// the product back and takes bandwidth and power from it, and the last wave's behind it.  Whole calls with an accumulator, us, two
+// streams -> one.  Without the normalisation up to four waves: 8192x8192x1024 205 -> 195, 6144x8192x3072 bf16 308 -> 298,
+// 4096x8192x8192 438 -> 431, 8192x8192x8192 bf16 811 -> 806; eight, 16384x8192x2048, 570 -> 579.  With it the second stream also
+// brings the rows of each wave that is whole rows (xcd_remap 2), which one stream has to leave for the end: 6144x8192x2048 217 ->
+// 227, 16384x8192x1024 366 -> 384, 8192x8192x3584 bf16 396 -> 407; not with few columns of K (8192x8192x512 161 -> 149, 16384x8192x512
+// 301 -> 300, 6144x8192x768 142 -> 146), nor with two waves, of which only the first is beside the GEMM (8192x4096x1024 115 -> 104,
+// 8192x4096x3072 205 -> 199, x4096 245 -> 247).  Where waves are not whole rows there is nothing to bring: 5120x8192x1024 156 -> 142,
+// 6144x6144x4096 301 -> 286, 8192x7168x4096 bf16 439 -> 411, 7168x8192x8192 777 -> 767.
+constexpr int kRowsWaitFromK = 640, kRowsWaitTwoWavesFromK = 3584;
+bool epilogue_sums(int algo, int M, int N, int K, bool norm) {
+    const long tiles = (long)((M + 255) / 256) * ((N + 255) / 256), wave = fo_main_tile_resident();
+    if (!norm) return tiles <= 4 * wave;
+    fo_raster r;
+    if (fo_pick_raster(algo, M, N, &r)) return false;
+    return r.xcd_remap != 2 || K < kRowsWaitFromK || (tiles <= 2 * wave && K < kRowsWaitTwoWavesFromK);
 }
 
 int fused_grid(const fo_overlap *h, int G) {  // 0: per-group launches, otherwise workgroups of the one launch
@@ -504,7 +523,11 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
     }
 
     const bool fits = !h->acc || aligned(C, h->acc);
-    const bool same_stream = in_stream(h, M, N, K, !h->acc && !np, monitor != 0, M % 256 || N % 256, fits);
+    const int64_t mn = (int64_t)M * N;
+    const bool acc_apart = h->acc && apart({h->acc, mn}, {{A, (int64_t)M * K}, {B, (int64_t)N * K}, {C, mn}});
+    const bool automatic = h->fused < 0 && h->link_bytes_per_s <= 0 && h->in_stream_below_flop > 0;
+    const bool same_stream = in_stream(h, M, N, K, !h->acc && !np, monitor != 0, M % 256 || N % 256, fits, false) ||
+                             (automatic && !monitor && fits && acc_apart && epilogue_sums(algo, M, N, K, np != nullptr));
     if (np) {
         // on one stream all rows follow in one launch, whatever their slots
         rc = same_stream ? check_slots(np->RA_host, TM * TN) : last_slots(np->RA_host, TM, TN, last_slot);
@@ -540,8 +563,6 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
     // the counters alone (they stay zero, as the waits would have left them).
     const bool quiet = same_stream && !monitor;
     // With nothing to wait for, the GEMM's epilogue does the consumer's work on the tile it holds in LDS.
-    const int64_t mn = (int64_t)M * N;
-    const bool acc_apart = h->acc && apart({h->acc, mn}, {{A, (int64_t)M * K}, {B, (int64_t)N * K}, {C, mn}});
     const bool consumed = quiet && acc_apart;
     // The last wave's sums by the GEMM itself, from storage slot sum_from on: nothing is left to overlap them with, and behind
     // the GEMM they are a wait, a launch and a second read of the product (17 + 4 us on 4096x8192, of which the GEMM's epilogue
@@ -746,7 +767,7 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     // present, src/overlap_impl.cu:312-313); otherwise a copy per group does.
     const bool own_in_consumer = D && h->acc && W > 1;
     const bool fits = !h->acc || aligned(C, h->acc, own_in_consumer ? D : nullptr);
-    const bool in_any_case = in_stream(h, M, N, K, only_copies, monitor != 0, false, fits);
+    const bool in_any_case = in_stream(h, M, N, K, only_copies, monitor != 0, false, fits, true);
     // A ragged call may leave the rest to launches behind the GEMM, one consumer launch for all groups or a copy for each:
     // the epilogue holds up the next tile's loads.  By the epilogue and by launches, us, eight ranks: with an accumulator
     // 8192x8064x7168 803 and 751, 8064x8064x4096 494 and 470 (two ranks 508 and 509), 4224x7168x3584 194 and 193,
@@ -755,7 +776,7 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     const bool large = 2.0 * M * N * K >= kRsEpilogueBelowFlop;
     const bool by_launches = h->acc ? W > 1 && large : G <= (large ? kFewCopies : kFewCopiesOfShort);
     const bool ragged = (M % 256 || N % 256) && (by_epilogue || by_launches || (h->acc && W > 1));
-    const bool same_stream = in_any_case || in_stream(h, M, N, K, only_copies, monitor != 0, ragged, fits);
+    const bool same_stream = in_any_case || in_stream(h, M, N, K, only_copies, monitor != 0, ragged, fits, true);
     const bool in_epilogue = by_epilogue && (in_any_case || !by_launches);
     const int fused = same_stream ? 0 : fused_grid(h, G);
     fo_stream_t cstream = same_stream ? h->gemm_stream : h->comm_stream;
