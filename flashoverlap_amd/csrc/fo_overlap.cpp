@@ -112,9 +112,13 @@ bool in_stream(const fo_overlap *h, int M, int N, int K, bool idle, bool monitor
 // 301 -> 300, 6144x8192x768 142 -> 146), nor with two waves, of which only the first is beside the GEMM (8192x4096x1024 115 -> 104,
 // 8192x4096x3072 205 -> 199, x4096 245 -> 247).  Where waves are not whole rows there is nothing to bring: 5120x8192x1024 156 -> 142,
 // 6144x6144x4096 301 -> 286, 8192x7168x4096 bf16 439 -> 411, 7168x8192x8192 777 -> 767.
+// `one_launch`, so many groups that one polling launch would consume them and the rows follow at the end: one stream at every
+// size measured (8192x8192x3584 bf16 in 32 groups 430 -> 409, 8192x8192x8192 in 64 847 -> 828, 8192x8192x2048 in 1024 333 -> 281,
+// 4096x8192x4096 in 20 261 -> 241; without the normalisation 16384x8192x1024 in 40 441 -> 375, x4096 bf16 in 100 902 -> 882).
 constexpr int kRowsWaitFromK = 640, kRowsWaitTwoWavesFromK = 3584;
-bool epilogue_sums(int algo, int M, int N, int K, bool norm) {
+bool epilogue_sums(int algo, int M, int N, int K, bool norm, bool one_launch) {
     const long tiles = (long)((M + 255) / 256) * ((N + 255) / 256), wave = fo_main_tile_resident();
+    if (one_launch) return true;
     if (!norm) return tiles <= 4 * wave;
     fo_raster r;
     if (fo_pick_raster(algo, M, N, &r)) return false;
@@ -527,7 +531,7 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
     const bool acc_apart = h->acc && apart({h->acc, mn}, {{A, (int64_t)M * K}, {B, (int64_t)N * K}, {C, mn}});
     const bool automatic = h->fused < 0 && h->link_bytes_per_s <= 0 && h->in_stream_below_flop > 0;
     const bool same_stream = in_stream(h, M, N, K, !h->acc && !np, monitor != 0, M % 256 || N % 256, fits, false) ||
-                             (automatic && !monitor && fits && acc_apart && epilogue_sums(algo, M, N, K, np != nullptr));
+                             (automatic && !monitor && fits && acc_apart && epilogue_sums(algo, M, N, K, np != nullptr, fused_grid(h, G) != 0));
     if (np) {
         // on one stream all rows follow in one launch, whatever their slots
         rc = same_stream ? check_slots(np->RA_host, TM * TN) : last_slots(np->RA_host, TM, TN, last_slot);
