@@ -36,6 +36,8 @@ enum {
 //
 // kRsEpilogueBelowFlop, kFewCopies: see fo_overlap_gemm_reducescatter.  They are no thresholds of a handle.
 //
+// kManySegmentsBelowK: see there as well.
+//
 // kTogetherFromN, kTogetherUpToK, kTogetherAnyKUpToN: what is consumed and normalised by one kernel (rows_together below).
 //
 // kGemmFlopPerNs: what a GEMM is expected to sustain, for sizing the pause
@@ -43,6 +45,7 @@ enum {
 constexpr int kFusedFromGroups = 16;
 constexpr double kInStreamBelowFlop = 6.4e10;
 constexpr double kRsEpilogueBelowFlop = 5e11;
+constexpr int kManySegmentsBelowK = 2048;
 constexpr int kFewCopies = 16, kFewCopiesOfShort = 6;
 constexpr int kTogetherFromN = 1024;
 constexpr int kTogetherUpToK = 3072;
@@ -780,8 +783,13 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     const bool large = 2.0 * M * N * K >= kRsEpilogueBelowFlop;
     const bool by_launches = h->acc ? W > 1 && large : G <= (large ? kFewCopies : kFewCopiesOfShort);
     const bool ragged = (M % 256 || N % 256) && (by_epilogue || by_launches || (h->acc && W > 1));
-    const bool same_stream = in_any_case || in_stream(h, M, N, K, only_copies, monitor != 0, ragged, fits, true);
-    const bool in_epilogue = by_epilogue && (in_any_case || !by_launches);
+    // So many groups that one polling launch would consume them beside the GEMM: the epilogue is the faster while K is short (us,
+    // two streams and one: 8192x8192x1024 in 1024 groups 271 and 232, X
+    // and 305, 4096x8192x4096 bf16 in 20 239 and 251).
+    const bool many = h->acc && by_epilogue && fits && !monitor && h->fused < 0 && h->link_bytes_per_s <= 0 &&
+                      h->in_stream_below_flop > 0 && K < kManySegmentsBelowK && fused_grid(h, G) != 0;
+    const bool same_stream = in_any_case || many || in_stream(h, M, N, K, only_copies, monitor != 0, ragged, fits, true);
+    const bool in_epilogue = by_epilogue && (in_any_case || many || !by_launches);
     const int fused = same_stream ? 0 : fused_grid(h, G);
     fo_stream_t cstream = same_stream ? h->gemm_stream : h->comm_stream;
     int32_t wave = 0;
