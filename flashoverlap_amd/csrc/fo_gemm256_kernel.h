@@ -349,7 +349,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             *first = begin;
             *count = end - begin;
         } else {
-            find_group_range(p.cseg, p.G, r, lane, first, count);
+            find_group_range(p.cseg, p.G, r, lane, lane < p.G ? p.cseg[lane] : 0, first, count);
         }
     };
     // Wavefront 0 announces a macro tile's reorder tiles: lane s < nsub holds the storage slot r and the group g of

@@ -118,6 +118,20 @@ inline bool on_lines(const GemmArgs &a) { return (((uintptr_t)a.A | (uintptr_t)a
 constexpr int kMaxSub = 4;        // reorder tiles per macro tile (256x256 over 128x128)
 constexpr int kPrefixRegs = 256;  // group search on prefix sums held in registers (one per 64 groups) up to this many groups
 
+// Inclusive prefix sum over a wavefront's lanes by the vector unit's own paths (six round trips to the LDS unit otherwise).
+// All lanes take part.
+template <int CTRL, int ROWS> __device__ __forceinline__ int add_shifted(int v) {
+    return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
+__device__ __forceinline__ int wave_prefix_sum(int v) {
+    v = add_shifted<0x111, 0xf>(v);     // row_shr:1, 2, 4, 8: inside rows of sixteen lanes
+    v = add_shifted<0x112, 0xf>(v);
+    v = add_shifted<0x114, 0xf>(v);
+    v = add_shifted<0x118, 0xf>(v);
+    v = add_shifted<0x142, 0xa>(v);     // row_bcast:15: a row's sum to the next, rows 1 and 3
+    return add_shifted<0x143, 0xc>(v);  // row_bcast:31: the first half's to rows 2 and 3
+}
+
 // Group of storage slot r: smallest g with cseg[0]+..+cseg[g] > r
 // (src/overlap/gemm_with_signal.h:343-349), found by one wavefront with a
 // 64-wide prefix sum per step instead of a serial scan.  All 64 lanes call it.
@@ -125,41 +139,29 @@ __device__ __forceinline__ int find_group(const int32_t *cseg, int G, int r, int
     int base = 0;
     for (int it = 0; it < G; it += 64) {
         int idx = it + lane;
-        int s = idx < G ? cseg[idx] : 0;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            int o = __shfl_up(s, d, 64);
-            if (lane >= d) s += o;
-        }
-        s += base;
+        const int s = base + wave_prefix_sum(idx < G ? cseg[idx] : 0);
         unsigned long long hit = __ballot(idx < G && s > r);
         if (hit) return it + (int)__builtin_ctzll(hit);
-        base = __shfl(s, 63, 64);
+        base = __builtin_amdgcn_readlane(s, 63);
     }
     return G - 1;  // unreachable when sum(cseg) covers every slot (validated on the host)
 }
 
-// The same, with the group's first storage slot and its slot count.
-__device__ __forceinline__ void find_group_range(const int32_t *cseg, int G, int r, int lane, int *first, int *count) {
+// The same, with the group's first storage slot and its slot count.  n0: this lane's group size, cseg[lane] (0 beyond G).
+__device__ __forceinline__ void find_group_range(const int32_t *cseg, int G, int r, int lane, int n0, int *first, int *count) {
     int base = 0;
     *first = *count = 0;
     for (int it = 0; it < G; it += 64) {
-        const int idx = it + lane, n = idx < G ? cseg[idx] : 0;
-        int s = n;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            int o = __shfl_up(s, d, 64);
-            if (lane >= d) s += o;
-        }
-        s += base;
+        const int idx = it + lane, n = it == 0 ? n0 : idx < G ? cseg[idx] : 0;
+        const int s = base + wave_prefix_sum(n);
         unsigned long long hit = __ballot(idx < G && s > r);
         if (hit) {
             const int at = (int)__builtin_ctzll(hit);
-            *count = __shfl(n, at, 64);
-            *first = __shfl(s, at, 64) - *count;
+            *count = __builtin_amdgcn_readlane(n, at);
+            *first = __builtin_amdgcn_readlane(s, at) - *count;
             return;
         }
-        base = __shfl(s, 63, 64);
+        base = __builtin_amdgcn_readlane(s, 63);
     }
 }
 

@@ -533,29 +533,40 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                 });
             };
             __builtin_amdgcn_s_setprio(2);
-            // While the first stage is on its way: row map entries, and the groups to signal.
+            // MAPPED: lane e of the computing wavefronts' 256 finds where row e, or (two reorder tiles side by side) row e % TM
+            // of one of them, goes.  The entry of the row map and the group sizes are asked for while the first stage is on its
+            // way, and used behind the first step: they lie two round trips to memory behind the reorder table, and awaited in
+            // front of the first barrier they held up the first step of every tile (whole passes, us: 2048x4096x2048 over eight ranks
+            // 34.7 -> 33.3, 1152x5120x1720 with an accumulator 35.0 -> 33.9, 3456x2176x680 22.9 -> 21.3).  The barrier of the second
+            // step publishes the maps; with too few steps for the loaders to wait for that, they are found in front of the first.
+            const int e = wave * 64 + lane;
+            const bool mapped_later = MAPPED && KT > S;
+            int entry = 0, size0 = 0;
+            const bool second_e = two_n ? e >= TM : e >= split_m;
             if (MAPPED) {
+                const int row = two_n && e >= TM ? e - TM : e, r = second_e ? r1 : r0;
+                if (e < (two_n ? 2 * TM : TM))
+                    entry = p.RE[(r / p.rLDN << bm_shift) + (second_e && two_m ? -split_m : m0 & (p.BM - 1)) + row];
+                if (MODE == MODE_RS && lane < p.G) size0 = p.cseg[lane];
+            }
+            auto write_maps = [&]() __attribute__((always_inline)) {
                 int first0 = 0, count0 = 0, first1 = 0, count1 = 0;  // MODE_RS: the groups' slots
                 if (MODE == MODE_RS) {
-                    find_group_range(p.cseg, p.G, r0, lane, &first0, &count0);
+                    find_group_range(p.cseg, p.G, r0, lane, size0, &first0, &count0);
                     first1 = first0;
                     count1 = count0;
-                    if (r1 != r0) find_group_range(p.cseg, p.G, r1, lane, &first1, &count1);
+                    if (r1 != r0) find_group_range(p.cseg, p.G, r1, lane, size0, &first1, &count1);
                 }
-                const int e = wave * 64 + lane;  // row e, or (two reorder tiles side by side) row e % TM of one of them
                 if (e < (two_n ? 2 * TM : TM)) {
-                    const int row = two_n && e >= TM ? e - TM : e;
-                    const bool second = two_n ? e >= TM : row >= split_m;
-                    const int r = second ? r1 : r0;
-                    const int to = p.RE[(r / p.rLDN << bm_shift) + (second && two_m ? -split_m : m0 & (p.BM - 1)) + row];
-                    row_map[e] = to;
+                    row_map[e] = entry;
                     if (MODE == MODE_RS)
-                        rs_map[e] = rs_row(p.cseg, p.G, p.BM, p.W, p.seg_rows, to, (second ? first1 : first0) << bm_shift,
-                                           (second ? count1 : count0) << bm_shift);
+                        rs_map[e] = rs_row(p.cseg, p.G, p.BM, p.W, p.seg_rows, entry, (second_e ? first1 : first0) << bm_shift,
+                                           (second_e ? count1 : count0) << bm_shift);
                 }
                 asm volatile("" ::: "memory");
-                __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): written when the first barrier is passed
-            }
+                __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): written when the next barrier is passed
+            };
+            if (MAPPED && !mapped_later) write_maps();
             if (signalling && wave == 0) {
                 g0 = find_group(p.cseg, p.G, r0, lane);
                 g1 = r1 != r0 ? find_group(p.cseg, p.G, r1, lane) : g0;
@@ -570,6 +581,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                     unsigned next = behind_slot(slot);
                     step_ahead(std::integral_constant<int, 0>{}, next, behind_slot(next));
                     if (++kt == KT) break;
+                    if (mapped_later && kt == 1) write_maps();
                     slot = behind_slot(next);
                     step_ahead(std::integral_constant<int, 1>{}, slot, behind_slot(slot));
                     if (++kt == KT) break;
@@ -582,6 +594,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                 for (int kt = 0; kt < KT; kt++) {
                     const unsigned next = behind_slot(slot), after = behind_slot(next);
                     step_strips(slot, next, after);
+                    if (mapped_later && kt == 0) write_maps();
                     slot = next;
                 }
             }
