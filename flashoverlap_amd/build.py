@@ -39,9 +39,9 @@ ARCH = "gfx950"
 KERNEL_SOURCES = ["fo_gemm.hip", "fo_aux.hip", "fo_algo.cpp", "fo_overlap.cpp"]
 # fo_gemm256_inst.hip and fo_gemm_tile_inst.hip hold the instantiations of the GEMM kernels for one dtype (fp16 / bf16)
 # and one epilogue (plain / signal / scatter / accumulating / reduce-scatter; of the 256x256 kernel also signal / scatter with the
-# last wave's sums) per compilation; separate jobs, for a build on many cores.
+# last wave's sums and the reordered store without counters) per compilation; separate jobs, for a build on many cores.
 GEMM_INSTANCES = [(src, d, m) for src in ("fo_gemm256_inst.hip", "fo_gemm_tile_inst.hip") for d in (0, 1) for m in (0, 1, 2, 3, 4)]
-GEMM_INSTANCES += [("fo_gemm256_inst.hip", d, m) for d in (0, 1) for m in (5, 6)]
+GEMM_INSTANCES += [("fo_gemm256_inst.hip", d, m) for d in (0, 1) for m in (5, 6, 7)]
 
 # -packed-fp32-ops off: hipcc must not form v_pk_*_f32 from the float code here.
 HIP_FLAGS = [

@@ -9,7 +9,7 @@
 int fo_gemm_dev::fo_gemm256_launch(int dtype, int mode, const GemmArgs &a, hipStream_t stream, int *resident_out,
                                    int expect_resident) {
     if (a.lda != a.ldb) return FO_ERR_ARG;  // the kernel addresses both operands with one leading dimension
-    const int key = (dtype == FO_BF16 ? 7 : 0) + mode;
+    const int key = (dtype == FO_BF16 ? 8 : 0) + mode;
     switch (key) {
         case 0: return fo_gemm256_launch_0_0(a, stream, resident_out, expect_resident);
         case 1: return fo_gemm256_launch_0_1(a, stream, resident_out, expect_resident);
@@ -18,13 +18,15 @@ int fo_gemm_dev::fo_gemm256_launch(int dtype, int mode, const GemmArgs &a, hipSt
         case 4: return fo_gemm256_launch_0_4(a, stream, resident_out, expect_resident);
         case 5: return fo_gemm256_launch_0_5(a, stream, resident_out, expect_resident);
         case 6: return fo_gemm256_launch_0_6(a, stream, resident_out, expect_resident);
-        case 7: return fo_gemm256_launch_1_0(a, stream, resident_out, expect_resident);
-        case 8: return fo_gemm256_launch_1_1(a, stream, resident_out, expect_resident);
-        case 9: return fo_gemm256_launch_1_2(a, stream, resident_out, expect_resident);
-        case 10: return fo_gemm256_launch_1_3(a, stream, resident_out, expect_resident);
-        case 11: return fo_gemm256_launch_1_4(a, stream, resident_out, expect_resident);
-        case 12: return fo_gemm256_launch_1_5(a, stream, resident_out, expect_resident);
-        case 13: return fo_gemm256_launch_1_6(a, stream, resident_out, expect_resident);
+        case 7: return fo_gemm256_launch_0_7(a, stream, resident_out, expect_resident);
+        case 8: return fo_gemm256_launch_1_0(a, stream, resident_out, expect_resident);
+        case 9: return fo_gemm256_launch_1_1(a, stream, resident_out, expect_resident);
+        case 10: return fo_gemm256_launch_1_2(a, stream, resident_out, expect_resident);
+        case 11: return fo_gemm256_launch_1_3(a, stream, resident_out, expect_resident);
+        case 12: return fo_gemm256_launch_1_4(a, stream, resident_out, expect_resident);
+        case 13: return fo_gemm256_launch_1_5(a, stream, resident_out, expect_resident);
+        case 14: return fo_gemm256_launch_1_6(a, stream, resident_out, expect_resident);
+        case 15: return fo_gemm256_launch_1_7(a, stream, resident_out, expect_resident);
     }
     return FO_ERR_ARG;
 }
@@ -284,6 +286,9 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     // The 128x192 tile that loads whole lines takes all of a CU's LDS and is not built for the epilogues that count; the
     // reordered store without counters is the accumulating epilogue without an accumulator.
     if (mode == MODE_SIGNAL && !counts && plan.tm == 128 && plan.tn == 192 && !on_lines(a)) mode = MODE_ACC;
+    const bool only_stores = mode == MODE_SIGNAL && !counts && plan.tm == 256 && plan.tn == 256;
+    const int tail_mode = mode;  // of the second launch, in a smaller tile
+    if (only_stores) mode = MODE_REORDER;
     a.sum_from = sum_from;
     if (sum_from >= 0) {
         if (!last_wave_sums(plan) || monitor || !acc) return FO_ERR_STATE;
@@ -302,7 +307,7 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     t.first = a.count;
     t.sub_m = 256 / plan.tail_tm; t.sub_n = 256 / plan.tail_tn;
     t.count = plan.tail * t.sub_m * t.sub_n;
-    return launch_tile(dtype, mode, t, plan.tail_tm, plan.tail_tn, s);
+    return launch_tile(dtype, tail_mode, t, plan.tail_tm, plan.tail_tn, s);
 }
 
 }  // namespace

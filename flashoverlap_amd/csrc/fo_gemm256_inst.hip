@@ -1,12 +1,13 @@
 // One instantiation of the 256x256 GEMM kernel per translation unit (the kernel's
 // K step is a single unrolled body of 128 MFMAs and takes minutes to compile):
-// built 14 times with -DFO_INST_DTYPE={0,1} (fp16, bf16) and -DFO_INST_MODE={0,1,2,3,4,5,6}
-// (plain, signal, scatter, accumulating, reduce-scatter epilogue; signal and scatter with the last wave's sums).
+// built 16 times with -DFO_INST_DTYPE={0,1} (fp16, bf16) and -DFO_INST_MODE={0,1,2,3,4,5,6,7}
+// (plain, signal, scatter, accumulating, reduce-scatter epilogue; signal and scatter with the last wave's sums,
+// reordered store without counters).
 #include "fo_gemm256_kernel.h"
 #include "fo_gemm_launch.h"
 
 #if !defined(FO_INST_DTYPE) || !defined(FO_INST_MODE)
-#error "compile with -DFO_INST_DTYPE=0|1 -DFO_INST_MODE=0|1|2|3|4|5|6"
+#error "compile with -DFO_INST_DTYPE=0|1 -DFO_INST_MODE=0|1|2|3|4|5|6|7"
 #endif
 
 namespace fo_gemm_dev {

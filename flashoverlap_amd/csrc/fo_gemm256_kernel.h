@@ -292,7 +292,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     for (int q = 0; q < NPRE; q++) pre[q] = 0;
     const bool reg_search = p.G <= kPrefixRegs;
     const bool signalling = COUNTS && !p.quiet;
-    const bool reorder = MODE == MODE_ACC ? p.RA != nullptr : COUNTS || MODE == MODE_RS;
+    const bool reorder = MODE == MODE_ACC ? p.RA != nullptr : COUNTS || MODE == MODE_RS || MODE == MODE_REORDER;
     const bool groups = signalling || TO_RANKS;  // group sizes are needed
     // The group sizes are requested in front of the pipeline fill and summed behind it (a round trip to memory and
     // some two dozen dependent cross-lane steps otherwise stand between the kernel's start and its first operand
@@ -549,6 +549,43 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             });
             slot_b ^= SLOT_B;
         };
+        // A wavefront whose half of the tile another tile computes multiplies nothing: it brings its share of the operands and
+        // meets the others.  (Large products are bound by energy; with M or N an odd multiple of 128 up to a tenth of their MFMAs
+        // were such repeats.  Whole passes without an accumulator, us: 4224x7168x3584 bf16 183.7 -> 179.0, 8064x8064x4096 bf16 418 ->
+        // 409, 6272x5888x2048 152.5 -> 150.2, of which an epilogue without the counters' code brings one percent.  Not in the
+        // accumulating epilogues, which hold the accumulator's values through the K loop: a second way through it there spills
+        // 500 registers.)
+        const bool idle = (MODE == MODE_PLAIN || MODE == MODE_REORDER) && (((repeated & 1) && wm == 0) || ((repeated & 2) && wn == 0));
+        if (idle) {
+            constexpr int BEFORE = loads_before_row256(ROWS - FREE - 1);  // of a stage's loads, those in front of the step's end
+            for (int kt = 0; kt < KT; kt++) {
+#pragma unroll
+                for (int c = BEFORE; c < 16; c++) load_chunk(c, slot_b ^ SLOT_B);
+                __builtin_amdgcn_s_barrier();  // FREE
+                asm volatile("" ::: "memory");
+                advance_loader();
+#pragma unroll
+                for (int c = 0; c < YOUNG; c++) load_chunk(c, slot_b);
+                wait_vmcnt<YOUNG>();
+                __builtin_amdgcn_s_barrier();  // PUB
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int c = YOUNG; c < BEFORE; c++) load_chunk(c, slot_b);
+                slot_b ^= SLOT_B;
+            }
+            // what a step's rows 13-15 fetch
+#pragma unroll
+            for (int q = 0; q < 4; q++) load_a(0, la0 ^ slot_b ^ (q % 2 * KSTEP_X), q / 2, q % 2);
+#pragma unroll
+            for (int q = 0; q < 10; q++) load_b(lb0 ^ slot_b ^ (q % 2 * KSTEP_X), q / 2, q % 2);
+        } else {
+        if (MODE == MODE_PLAIN || MODE == MODE_REORDER) {  // as above: all of them are written on this side of the wait states
+#pragma unroll
+            for (int i = 0; i < F; i++)
+#pragma unroll
+                for (int j = 0; j < F; j++) asm volatile("" : "+a"(acc[i][j]));
+            fo_mfma_fence();
+        }
         // A tile whose predecessor's signal is still owed leaves the K loop after its first step, sends the signal and
         // re-enters: that step's PUB meeting has waited for the predecessor's stores in every wavefront (part of the
         // stage's loads was requested behind them, rows 0-6, and vmcnt retires in issue order), with the meeting's
@@ -577,6 +614,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             __builtin_amdgcn_s_waitcnt(0xC07F);
             if (kt >= KT) break;
             kt_stop = KT;
+        }
         }
 
         fo_mfma_fence();

@@ -41,8 +41,9 @@ __device__ __forceinline__ void static_for(F &&f) {
 // per group, and each range into W chunks of consecutive rows; row i of chunk q of a range that starts at row f is added
 // to row q * seg_rows + f / W + i of the accumulator (if any) and, for q == rank, stored to row f / W + i of OWN (if any).
 // MODE_SIGNAL_SUM, MODE_SCATTER_SUM (256x256 kernel only): the signal and scatter epilogues where tiles from storage slot
-// sum_from on are not counted but added to the accumulator as MODE_ACC and MODE_RS do.
-enum { MODE_PLAIN = 0, MODE_SIGNAL = 1, MODE_SCATTER = 2, MODE_ACC = 3, MODE_RS = 4, MODE_SIGNAL_SUM = 5, MODE_SCATTER_SUM = 6 };
+// sum_from on are not counted but added to the accumulator as MODE_ACC and MODE_RS do.  MODE_REORDER (the same kernel): the signal
+// epilogue's store, nothing counted.
+enum { MODE_PLAIN = 0, MODE_SIGNAL = 1, MODE_SCATTER = 2, MODE_ACC = 3, MODE_RS = 4, MODE_SIGNAL_SUM = 5, MODE_SCATTER_SUM = 6, MODE_REORDER = 7 };
 
 // Division by a number that the host knows: n / d for n and d below 32768, exactly (the product exceeds n / d * 2^31 by
 // less than n * d).

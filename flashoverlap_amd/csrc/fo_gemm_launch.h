@@ -81,15 +81,15 @@ inline int launch_kernel(const GemmArgs &a, hipStream_t stream, int *resident_ou
 }
 
 // The 256x256 kernel (fo_gemm256_kernel.h) for dtype FO_F16 / FO_BF16 and epilogue MODE_PLAIN /
-// MODE_SIGNAL / MODE_SCATTER / MODE_ACC / MODE_RS / MODE_SIGNAL_SUM / MODE_SCATTER_SUM; same arguments as launch_kernel.  One definition per instantiation
+// MODE_SIGNAL / MODE_SCATTER / MODE_ACC / MODE_RS / MODE_SIGNAL_SUM / MODE_SCATTER_SUM / MODE_REORDER; same arguments as launch_kernel.  One definition per instantiation
 // (fo_gemm256_inst.hip compiled with FO_INST_DTYPE and FO_INST_MODE), dispatched in fo_gemm.hip.
 int fo_gemm256_launch(int dtype, int mode, const GemmArgs &a, hipStream_t stream, int *resident_out, int expect_resident);
 #define FO_GEMM256_INST_DECL(D_, M_) \
     int fo_gemm256_launch_##D_##_##M_(const GemmArgs &a, hipStream_t stream, int *resident_out, int expect_resident);
 FO_GEMM256_INST_DECL(0, 0) FO_GEMM256_INST_DECL(0, 1) FO_GEMM256_INST_DECL(0, 2) FO_GEMM256_INST_DECL(0, 3) FO_GEMM256_INST_DECL(0, 4)
-FO_GEMM256_INST_DECL(0, 5) FO_GEMM256_INST_DECL(0, 6)
+FO_GEMM256_INST_DECL(0, 5) FO_GEMM256_INST_DECL(0, 6) FO_GEMM256_INST_DECL(0, 7)
 FO_GEMM256_INST_DECL(1, 0) FO_GEMM256_INST_DECL(1, 1) FO_GEMM256_INST_DECL(1, 2) FO_GEMM256_INST_DECL(1, 3) FO_GEMM256_INST_DECL(1, 4)
-FO_GEMM256_INST_DECL(1, 5) FO_GEMM256_INST_DECL(1, 6)
+FO_GEMM256_INST_DECL(1, 5) FO_GEMM256_INST_DECL(1, 6) FO_GEMM256_INST_DECL(1, 7)
 #undef FO_GEMM256_INST_DECL
 
 // The smaller tiles (fo_gemm_tile_kernel.h), the same way (fo_gemm_tile_inst.hip); FO_ERR_ALGO for a tile that is not built.

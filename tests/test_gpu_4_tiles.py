@@ -480,3 +480,42 @@ def test_whole_lines_in_128x192_tiles(fo, dtype, bm, bn, M, N, K):
     assert torch.equal(acc.reshape(-1), (before.float() + C.float()).to(td).reshape(-1))
     assert (MM == 0).all()
     ov.close()
+
+
+@pytest.mark.parametrize("dtype,bm,bn,M,N,K", [
+    (F16, 128, 128, 8064, 4224, 8),        # half a tile left along both, one K step, a workgroup's tiles half and whole in turn
+    (BF16, 128, 128, 8064, 4224, 200),
+    (F16, 128, 256, 4224, 7168, 648),      # along M
+    (BF16, 256, 128, 4096, 7296, 128),     # along N, rows on the lines
+])
+def test_repeated_halves_are_not_multiplied(fo, dtype, bm, bn, M, N, K):
+    """256x256 tiles with half a tile left: the wavefronts of the half that another tile computes bring operands only.  Plain
+    and reordered without counters, against the launch with counters (other tiles) bit for bit."""
+    ops, layout, td = fo.ops, fo.layout, TORCH_DTYPE[dtype]
+    algo = fo._capi.find_algo(bm, bn, swizzle=4)
+    TM, TN = M // bm, N // bn
+    T = TM * TN
+    A, _ = seeded((M, K), dtype, M + K)
+    B, _ = seeded((N, K), dtype, N + K, scale=K ** -0.5)
+    RA = torch.from_numpy(np.random.default_rng(K).permutation(T).astype(np.int32)).reshape(TM, TN).cuda()
+    cs = torch.tensor([T], dtype=torch.int32)
+    MM = torch.zeros(layout.counter_size(1, TM, TN), dtype=torch.int32, device="cuda")
+    Cp = torch.full((M * N,), float("nan"), device="cuda", dtype=td)
+    ops.gemm_signal(A, B, Cp, MM, RA, cs.cuda(), algo)
+    torch.cuda.synchronize()
+    want = layout.unpermute(Cp, M, N, bm, bn, RA)
+    assert MM[0] == T
+    MM.zero_()
+    plain = torch.full((M, N), float("nan"), device="cuda", dtype=td)
+    ops.gemm(A, B, plain, algo)
+    torch.cuda.synchronize()
+    assert torch.equal(plain, want)
+    assert max_rel_err(plain.float(), A.float() @ B.float().T) <= 1e-2
+    ov = ops.Overlap()
+    for rldn in (1, 2 if T % 2 == 0 else 1):
+        Cp.fill_(float("nan"))
+        ov.gemm_allreduce_overlap(A, B, Cp, MM, RA, rldn, cs, cs.cuda(), algo)
+        torch.cuda.synchronize()
+        assert torch.equal(layout.unpermute(Cp, M, N, bm, bn, RA, rLDN=rldn), want)
+    assert (MM == 0).all()
+    ov.close()
