@@ -347,6 +347,8 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             // arrive while the last S - 1 stages are multiplied.
             const bool sums = ACC && (!MAY_LACK || p.ACC);
             const int stages = SHIFT ? KT + 1 : KT;
+            // (At least two steps in front of it where the maps are written behind the first: KT > S there, and the second step's
+            // barrier publishes rs_map, from which the addresses come.)
             const int fetching = sums ? (stages > S - 1 ? stages - (S - 1) : 0) : KT;
             for (int kt = 0; kt < fetching; kt++) {
                 request(kt + S - 1, slot);  // the slot of stage kt - 1, given up at the last barrier
