@@ -1,5 +1,6 @@
 """Calls on two streams whose last wave is summed by the GEMM itself: product, accumulator, this rank's rows, counters and
-normalised rows against their definitions, at the partitions and storage orders where the rule changes sides."""
+normalised rows against their definitions, at the partitions and storage orders where the rule changes sides; and what
+automatic mode keeps on one stream against what two streams leave."""
 import numpy as np
 import pytest
 import torch
@@ -107,4 +108,45 @@ def test_reduce_scatter(fo, dtype, bm, bn, M, N, K, cseg, order, W, own):
     assert torch.equal(acc, (before.float() + want.reshape(-1).float()).to(td))
     if own:
         assert torch.equal(D.view(-1, bn), torch.cat(mine))
+    ov.close()
+
+
+@pytest.mark.parametrize("dtype,bm,bn,M,N,K,groups,order,rldn", [
+    (F16, 128, 128, 4096, 4096, 2048, 4, "schedule", 1),      # one round
+    (BF16, 128, 256, 4096, 4096, 2104, 20, "any", 2),         # one round, more groups than per-wave launches are made for
+    (F16, 128, 128, 8192, 4096, 1032, 3, "schedule", 1),      # two waves of whole rows, groups across them
+    (BF16, 256, 128, 6144, 6144, 1024, 5, "any", 1),          # two waves and a quarter, not whole rows
+    (F16, 128, 128, 8192, 8192, 520, 700, "schedule", 2),     # four waves, very many groups
+])
+@pytest.mark.parametrize("norm", [False, True])
+def test_automatic_choice_against_two_streams(fo, dtype, bm, bn, M, N, K, groups, order, rldn, norm):
+    """What automatic mode does on one stream and what two streams leave: the same product, accumulator, counters and rows."""
+    T = (M // bm) * (N // bn)
+    cuts = [T * g // groups for g in range(groups + 1)]
+    cseg = [b - a for a, b in zip(cuts, cuts[1:])]
+    algo, A, B, before, plain, RA, cs, cs_gpu, MM, ov = _setup(fo, dtype, bm, bn, M, N, K, cseg, order)
+    ov.set_schedule()
+    td = TORCH_DTYPE[dtype]
+    gamma = (1 + 0.01 * torch.randn(N, generator=torch.Generator().manual_seed(5))).to(td).cuda()
+    RA_cpu = RA.cpu()
+    left = []
+    for fused in (-1, 0):
+        ov.set_fused_consumer(fused)
+        acc = before.clone()
+        C = torch.full((M * N,), float("nan"), device="cuda", dtype=td)
+        Y = torch.full((M, N), float("nan"), device="cuda", dtype=td)
+        ov.set_accumulator(acc)
+        for rep in range(2):
+            if norm:
+                ov.gemm_allreduce_rmsnorm_overlap(A, B, C, MM, RA, RA_cpu, rldn, cs, cs_gpu, algo, Y, gamma, eps=EPS)
+            else:
+                ov.gemm_allreduce_overlap(A, B, C, MM, RA, rldn, cs, cs_gpu, algo)
+        torch.cuda.synchronize()
+        assert ov.status() == 0 and (MM == 0).all()
+        left.append((C, acc, Y))
+    assert torch.equal(fo.layout.unpermute(left[0][0], M, N, bm, bn, RA, rLDN=rldn), plain)
+    assert torch.equal(left[0][0], left[1][0])
+    assert torch.equal(left[0][1], left[1][1])
+    if norm:
+        assert torch.equal(left[0][2], left[1][2])
     ov.close()
