@@ -134,8 +134,8 @@ int fo_gemm_reduce_scatter(int dtype, int M, int N, int K, const int32_t *cseg_d
 int fo_gemm_last_wave(int algo, int M, int N, int32_t *first);
 // fo_gemm_signal / fo_gemm_scatter (RE != nullptr) where tiles from storage slot sum_from on are not counted but summed: added
 // to the accumulator (RE: in its reduce-scatter layout, and this rank's rows copied to `own`, if any, as
-// fo_gemm_reduce_scatter does).  For slots of the last wave (fo_gemm_last_wave) as fo_schedule_order deals them out; others
-// come out right, and late.
+// fo_gemm_reduce_scatter does; of accumulator and rows one may be missing).  For slots of the last wave (fo_gemm_last_wave)
+// as fo_schedule_order deals them out; others come out right, and late.
 int fo_gemm_signal_sums(int dtype, int M, int N, int K, int rLDN, const int32_t *cseg_dev, int G, const void *A, const void *B,
                         void *C, int32_t *MM, const int32_t *RA, const int32_t *RE, void *acc, int sum_from, void *own, int W,
                         int rank, int algo, fo_stream_t stream);

@@ -291,7 +291,7 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     if (only_stores) mode = MODE_REORDER;
     a.sum_from = sum_from;
     if (sum_from >= 0) {
-        if (!last_wave_sums(plan) || monitor || !acc) return FO_ERR_STATE;
+        if (!last_wave_sums(plan) || monitor || (!acc && (mode != MODE_SCATTER || !a.OWN))) return FO_ERR_STATE;
         mode = mode == MODE_SCATTER ? MODE_SCATTER_SUM : MODE_SIGNAL_SUM;
     }
     // the tail split was computed for that many workgroups of the main launch

@@ -652,6 +652,8 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             // TO_RANKS: the accumulator rows of the wavefront's rows, held as re_lo and re_hi are.
             int ac_lo = 0, ac_hi = 0;
             const bool sums = MODE == MODE_ACC || (MODE == MODE_RS && p.ACC) || (SUMS && r >= p.sum_from);  // wave-uniform
+            // SUMS: the sums of such a tile; a reduce-scatter without an accumulator only wants its rows
+            const bool adds = sums && (MODE != MODE_SCATTER_SUM || p.ACC);
             const int own_first = TO_RANKS ? p.rank * p.seg_rows : 0, own_rows = TO_RANKS && p.OWN && (sums || !SUMS) ? p.seg_rows : 0;
             auto row_of = [&](int k, int lo, int hi) __attribute__((always_inline)) {  // row k * RPP + srow of the block: its entry sits in that lane
                 return __builtin_amdgcn_ds_bpermute((k * RPP % 64 + srow) * 4, k * RPP < 64 ? lo : hi);
@@ -667,7 +669,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             // lane's where it reads them, and no other wavefront has part in it.  (In registers, as with MODE_ACC, they would
             // leave no room on the SIMD for the consumer that runs beside the earlier waves.)
             auto piece_lds = [&](int k) __attribute__((always_inline)) { return (wa0 ^ (k / 16 * SLOT_B)) + k % 16 * CHUNK_B; };
-            if (SUMS && sums && !has_next) {
+            if (SUMS && adds && !has_next) {
                 if (MAPPED) asm volatile("" : "+v"(re_lo), "+v"(re_hi), "+v"(ac_lo), "+v"(ac_hi));  // nothing else is awaited behind the loads
                 unsigned rows = 0, rows_step = __builtin_amdgcn_readfirstlane(RPP * ldp * 2);
                 const fo_srd_t from = fo_make_srd(TO_RANKS ? reinterpret_cast<char *>(p.ACC) : abase, 0x7fffffffu);
@@ -719,7 +721,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
 #pragma unroll
                     for (int k = 0; k < NST; k++) asm volatile("" : "+v"(old[ACC ? k : 0]));
                 }
-                if (SUMS && sums && !has_next) {
+                if (SUMS && adds && !has_next) {
                     // this strip's values have landed; behind them the later strips' and the stores of the earlier ones
                     constexpr int PER = MODE == MODE_SIGNAL_SUM ? 2 * (16 / RPP) : 16 / RPP;
                     switch (i) {  // i is a constant: the loop is unrolled
@@ -762,7 +764,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                         uint16_t *to = p.C + (size_t)prow * pitch + tcol + scol * 8;
                         if (TO_RANKS && (ACC || sums)) {
                             const int ac = row_of(k, ac_lo, ac_hi);
-                            if (sums && ac >= 0)
+                            if ((SUMS ? adds : sums) && ac >= 0)
                                 store16_write_through(p.ACC + (size_t)ac * pitch + tcol + scol * 8, fo_add8<Tag>(SUMS ? value_of(k) : old[ACC ? k : 0], v));
                             if ((unsigned)(ac - own_first) < (unsigned)own_rows)
                                 store16_write_through(p.OWN + (size_t)(ac - own_first) * pitch + tcol + scol * 8, v);

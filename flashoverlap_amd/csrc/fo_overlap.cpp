@@ -815,8 +815,10 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     }
     // The last batch's sums and rows by the GEMM itself, where that batch is of the last wave only (us: 8192x4096x4096, eight ranks
     // 235.6 -> 230.4, 8192x8192x3584 bf16 398 -> 389, 4096x8192x2048 bf16 146.7 -> 143.3).
+    // Without an accumulator this rank's rows of those groups, which are else a copy per group behind the GEMM (8192x4096x4096
+    // bf16 in sixteen groups, eight ranks, 211.8 -> 203.5; 8192x4096x2048 in four, four ranks, 124.0 -> 122.5, 4096x4096x4096 the same).
     int32_t sum_from = TM * TN;
-    if (!same_stream && !fused && !monitor && h->link_bytes_per_s <= 0 && by_epilogue && h->acc && W > 1 &&
+    if (!same_stream && !fused && !monitor && h->link_bytes_per_s <= 0 && by_epilogue && (h->acc || D) && W > 1 &&
         (int64_t)M * N * 2 <= 0x7FFFFFFFLL) {
         int32_t first = 0;
         rc = fo_gemm_last_wave(algo, M, N, &first);

@@ -111,6 +111,36 @@ def test_reduce_scatter(fo, dtype, bm, bn, M, N, K, cseg, order, W, own):
     ov.close()
 
 
+@pytest.mark.parametrize("dtype,bm,bn,M,N,K,cseg,order,W", [
+    (F16, 128, 128, 8192, 4096, 72, [512] * 4, "schedule", 8),
+    (BF16, 256, 128, 8192, 4096, 136, [512, 512], "any", 2),
+    (F16, 128, 256, 4096, 7168, 200, [512, 300, 84], "schedule", 4),
+])
+def test_reduce_scatter_rows_without_accumulator(fo, dtype, bm, bn, M, N, K, cseg, order, W):
+    """The same without an accumulator: this rank's rows of the last wave are the GEMM's too."""
+    algo, A, B, before, plain, RA, cs, cs_gpu, MM, ov = _setup(fo, dtype, bm, bn, M, N, K, cseg, order)
+    ov.close()
+    rank = 0
+    ov = fo.ops.Overlap(rank=rank, world=W)
+    ov.set_schedule(in_stream_below_flop=0)
+    ov.set_fused_consumer(0)
+    RE = fo.layout.generate_row_mapping(M, N, bm, bn, cseg, W)
+    td = TORCH_DTYPE[dtype]
+    for rep in range(2):
+        C = torch.full((M * N,), float("nan"), device="cuda", dtype=td)
+        D = torch.full((M // W * N,), float("nan"), device="cuda", dtype=td)
+        ov.gemm_reducescatter_overlap(A, B, C, D, MM, RA, RE, 1, cs, cs_gpu, algo)
+        torch.cuda.synchronize()
+        assert ov.status() == 0 and (MM == 0).all()
+        assert torch.equal(fo.layout.unpermute(C, M, N, bm, bn, RA, RE=RE), plain)
+        rows, mine, first = C.view(-1, bn), [], 0
+        for n in cseg:
+            mine.append(rows[first:first + n * bm].view(W, n * bm // W, bn)[rank])
+            first += n * bm
+        assert torch.equal(D.view(-1, bn), torch.cat(mine))
+    ov.close()
+
+
 @pytest.mark.parametrize("dtype,bm,bn,M,N,K,groups,order,rldn", [
     (F16, 128, 128, 4096, 4096, 2048, 4, "schedule", 1),      # one round
     (BF16, 128, 256, 4096, 4096, 2104, 20, "any", 2),         # one round, more groups than per-wave launches are made for
