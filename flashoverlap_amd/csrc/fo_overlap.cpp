@@ -784,7 +784,7 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     const bool by_launches = h->acc ? W > 1 && large : G <= (large ? kFewCopies : kFewCopiesOfShort);
     const bool ragged = (M % 256 || N % 256) && (by_epilogue || by_launches || (h->acc && W > 1));
     // So many groups that one polling launch would consume them beside the GEMM: the epilogue is the faster while K is short (us,
-    // two streams and one: 8192x8192x1024 in 1024 groups 271 and 232, X
+    // two streams and one: 8192x8192x1024 in 1024 groups 271 and 232, 8192x4096x1536 bf16 in 40 157 and 137, 8192x8192x2048 bf16 in 18 299
     // and 305, 4096x8192x4096 bf16 in 20 239 and 251).
     const bool many = h->acc && by_epilogue && fits && !monitor && h->fused < 0 && h->link_bytes_per_s <= 0 &&
                       h->in_stream_below_flop > 0 && K < kManySegmentsBelowK && fused_grid(h, G) != 0;
