@@ -695,6 +695,14 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                         old[ACC ? k : 0] = *reinterpret_cast<const fo_u32x4 *>(abase + (size_t)(k * RPP) * ldp * 2 + lane_off);
                     }
                 }
+                // MODE_RS: awaited on this way.  Awaited behind the point where it meets the one without an accumulator, they were to
+                // the compiler still to come on the other, and on both every piece waited, counting, for the stores in front of
+                // it.  Whole calls with the normalisation, us: 4096x3328x4096 bf16 122.5 -> 103.5, 3456x4352x3072 108.2 -> 93.5,
+                // 8192x8192x1024 in 32 groups 221.5 -> 207.0; without an accumulator 8192x4096x4096 in 24 240.2 -> 214.6.
+                if (MODE == MODE_RS) {
+#pragma unroll
+                    for (int k = 0; k < NST; k++) asm volatile("" : "+v"(old[ACC ? k : 0]));
+                }
             } else if (!early) {
 #pragma unroll
                 for (int k = 0; k < (ACC ? NST : 1); k++) old[k] = fo_u32x4{0, 0, 0, 0};
@@ -717,7 +725,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_s_waitcnt(0xC07F);
                 __builtin_amdgcn_wave_barrier();
-                if (ACC && sums && i == 0) {
+                if (MODE == MODE_ACC && sums && i == 0) {
 #pragma unroll
                     for (int k = 0; k < NST; k++) asm volatile("" : "+v"(old[ACC ? k : 0]));
                 }
