@@ -34,9 +34,7 @@ enum {
 // GEMM cost more than such a GEMM can hide (4096x4096x512 with 256 groups:
 // 71 us overlapped, 44 us in stream).
 //
-// kRsEpilogueBelowFlop, kFewCopies: see fo_overlap_gemm_reducescatter.  They are no thresholds of a handle.
-//
-// kManySegmentsBelowK: see there as well.
+// kManyCopiesFromFlop, kFewCopies: see fo_overlap_gemm_reducescatter.  They are no thresholds of a handle.
 //
 // kTogetherFromN, kTogetherUpToK, kTogetherAnyKUpToN: what is consumed and normalised by one kernel (rows_together below).
 //
@@ -44,8 +42,7 @@ enum {
 // between polls only.
 constexpr int kFusedFromGroups = 16;
 constexpr double kInStreamBelowFlop = 6.4e10;
-constexpr double kRsEpilogueBelowFlop = 5e11;
-constexpr int kManySegmentsBelowK = 2048;
+constexpr double kManyCopiesFromFlop = 5e11;
 constexpr int kFewCopies = 16, kFewCopiesOfShort = 6;
 constexpr int kTogetherFromN = 1024;
 constexpr int kTogetherUpToK = 3072;
@@ -85,17 +82,17 @@ namespace {
 // follows each consumer launch, and it is what the second stream is there to hide.
 //
 // Longer GEMMs stay on one stream too where there is nothing to overlap: `idle`, a call without a consumer and without a
-// normalisation (4224x7168x3584 221 -> 215 us, 3712x8192x3456 216 -> 207), and a product of at most one round of 256x256
+// normalisation (4224x7168x3584 221 -> 215 us, 3712x8192x3456 216 -> 207) or as the reduce-scatter says, and a product of at most one round of 256x256
 // tiles, whose groups all complete at its end, so that the second stream adds its launches and polls and hides
 // nothing (us, two streams -> one: 2304x4096x3560 96 -> 83, 1792x4608x4520 125 -> 108, 2048x4224x6968 256 -> 167,
 // 2176x5888x3312 133 -> 127, 4096x4096x4096 133 -> 125, 2048x8192x3000 128 -> 118).  `scatter`, a reduce-scatter: up to five
-// sixths of a round (4096x4096x2560 with four ranks 98 -> 100).  in_stream_below_flop = 0 still asks for two streams always.
+// sixths of a round, with launches behind the GEMM (4096x4096x2560 with four ranks 98 -> 100).  in_stream_below_flop = 0 still asks for two streams always.
 //
 // `ragged`, a call that could do either and whose M or N is an odd multiple of 128: a launch that counts keeps the order of
 // the groups in the Algo's own tile (plan_launch), one that does not takes 256x256 tiles with half tiles at the end, and
 // what that saves is more than the second stream hides (us, two streams -> one, with an accumulator and the normalisation:
 // 3456x4352x3072 127 -> 93, 2432x7040x7056 271 -> 245, 8064x8064x4096 586 -> 465, 6272x8192x7168 661 -> 636; reduce-scatter,
-// eight ranks: 3456x4352x3072 123 -> 95, 4224x7168x3584 205 -> 194, 6272x8192x7168 651 -> 630, 8192x8064x7168 801 -> 751).
+// eight ranks: 3456x4352x3072 123 -> 95, 4224x7168x3584 205 -> 194, 6272x8192x7168 651 -> 630, 8192x8064x7168 801 -> 703).
 // `fits`: the accumulator is one that every path takes; one that is not aligned is left to the one-launch consumer.
 bool in_stream(const fo_overlap *h, int M, int N, int K, bool idle, bool monitor, bool ragged, bool fits, bool scatter) {
     if (!h->comm_stream) return true;
@@ -765,31 +762,27 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     const span a = {A, (int64_t)M * K}, b = {B, (int64_t)N * K}, prod = {C, (int64_t)M * N}, sum = {h->acc, (int64_t)M * N};
     const bool by_epilogue = rLDN == 1 && info[0] % W == 0 && !(((uintptr_t)C | (uintptr_t)D | (uintptr_t)h->acc) & 15) &&
                              apart(sum, {a, b, prod}) && apart({D, seg_stride}, {a, b, prod, sum});
-    // Without an accumulator all there is to overlap are those copies, and with many groups they take longer than the GEMM:
-    // 5504x3840x3640 with four ranks, two streams against one, us: 4 groups 192 and 186, 16 214 and 187, 64 320 and 187, 1290
-    // 3404 and 218; 8192x4096x4096 with two: 4 groups 228 and 249, 16 236 and 247, 24 284 and 252, 64 369 and 253.
-    const bool only_copies = !h->acc && by_epilogue && G > kFewCopies;
     // With an accumulator and W > 1 the consumer also writes this rank's chunk of
     // every group to D (ncclReduceScatter(C+acc -> D+acc/W, n/W) with one rank
     // present, src/overlap_impl.cu:312-313); otherwise a copy per group does.
     const bool own_in_consumer = D && h->acc && W > 1;
     const bool fits = !h->acc || aligned(C, h->acc, own_in_consumer ? D : nullptr);
-    const bool in_any_case = in_stream(h, M, N, K, only_copies, monitor != 0, false, fits, true);
-    // A ragged call may leave the rest to launches behind the GEMM, one consumer launch for all groups or a copy for each:
-    // the epilogue holds up the next tile's loads.  By the epilogue and by launches, us, eight ranks: with an accumulator
-    // 8192x8064x7168 803 and 751, 8064x8064x4096 494 and 470 (two ranks 508 and 509), 4224x7168x3584 194 and 193,
-    // 8064x8192x1024 183 and 200; copies, 6400x2176x4648: four 136 and 126, ten 132 and 130, sixteen 133 and 142;
-    // 3456x7424x3328: six 170 and 165, ten 170 and 174; 8192x8064x7168: sixteen 737 and 693.
-    const bool large = 2.0 * M * N * K >= kRsEpilogueBelowFlop;
-    const bool by_launches = h->acc ? W > 1 && large : G <= (large ? kFewCopies : kFewCopiesOfShort);
-    const bool ragged = (M % 256 || N % 256) && (by_epilogue || by_launches || (h->acc && W > 1));
-    // So many groups that one polling launch would consume them beside the GEMM: the epilogue is the faster while K is short (us,
-    // two streams and one: 8192x8192x1024 in 1024 groups 271 and 232, 8192x4096x1536 bf16 in 40 157 and 137, 8192x8192x2048 bf16 in 18 299
-    // and 305, 4096x8192x4096 bf16 in 20 239 and 251).
-    const bool many = h->acc && by_epilogue && fits && !monitor && h->fused < 0 && h->link_bytes_per_s <= 0 &&
-                      h->in_stream_below_flop > 0 && K < kManySegmentsBelowK && fused_grid(h, G) != 0;
-    const bool same_stream = in_any_case || many || in_stream(h, M, N, K, only_copies, monitor != 0, ragged, fits, true);
-    const bool in_epilogue = by_epilogue && (in_any_case || many || !by_launches);
+    // The epilogue leaves nothing to overlap, and what it adds to the GEMM is less than two streams cost (whole calls with the
+    // normalisation, us, two streams and one): with an accumulator where there is one round, which no consumer runs beside,
+    // 4096x4096x4096 130 and 120, 4096x4096x8192 bf16 212 and 203; and where groups are so many that one polling launch would
+    // consume them, 4096x8192x4096 bf16 in twenty 244 and 225, 8192x8192x3584 bf16 in 32 415 and 401, 8192x8192x8192 in 64 835
+    // and 819, 16384x8192x2048 in 64 564 and 558.  Fewer groups and more rounds are left to the consumer: two rounds are the same
+    // either way (8192x4096x4096 in eight 234 and 234, 4096x8192x1536 129 and 128), four are not (8192x8192x3584 bf16 387 and 401).
+    // Without an accumulator all there is to overlap are copies, and many take longer than the GEMM (8192x4096x4096 in 24
+    // groups 284, on one stream 215).  Up to sixteen groups stay on two streams, where their counters are waited for and reset,
+    // which a caller can see, at 1 to 9 % (16384x8192x1024 285 and 273, 8192x4096x4096 in sixteen 201 and 196).
+    const bool one_round = (long)((M + 255) / 256) * ((N + 255) / 256) <= (long)fo_main_tile_resident();
+    const bool idle = by_epilogue && (h->acc ? one_round || fused_grid(h, G) != 0 : G > kFewCopies);
+    // A ragged call's gain on one stream (see in_stream) is there by the epilogue (us, eight ranks, two streams' 8064x8064x7168 in
+    // four groups with launches behind the GEMM 750, so 719) and with one consumer launch for all groups or a few copies behind it.
+    const bool few_copies = !h->acc && G <= (2.0 * M * N * K >= kManyCopiesFromFlop ? kFewCopies : kFewCopiesOfShort);
+    const bool ragged = (M % 256 || N % 256) && (by_epilogue || (h->acc && W > 1) || few_copies);
+    const bool same_stream = in_stream(h, M, N, K, idle, monitor != 0, ragged, fits, true);
     const int fused = same_stream ? 0 : fused_grid(h, G);
     fo_stream_t cstream = same_stream ? h->gemm_stream : h->comm_stream;
     int32_t wave = 0;
@@ -808,15 +801,16 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
         if (rc) return rc;
     }
     const bool quiet = same_stream && !monitor;  // as in fo_overlap_gemm_allreduce
-    if (quiet && in_epilogue) {
+    if (quiet && by_epilogue) {
         rc = fo_gemm_reduce_scatter(dtype, M, N, K, cseg_dev, G, A, B, C, h->acc, D, RA, RE, W, h->rank, algo, h->gemm_stream);
         if (rc) return rc;
         return link_time(h, (int64_t)M * N * 2, h->gemm_stream);
     }
     // The last batch's sums and rows by the GEMM itself, where that batch is of the last wave only (us: 8192x4096x4096, eight ranks
     // 235.6 -> 230.4, 8192x8192x3584 bf16 398 -> 389, 4096x8192x2048 bf16 146.7 -> 143.3).
-    // Without an accumulator this rank's rows of those groups, which are else a copy per group behind the GEMM (8192x4096x4096
-    // bf16 in sixteen groups, eight ranks, 211.8 -> 203.5; 8192x4096x2048 in four, four ranks, 124.0 -> 122.5, 4096x4096x4096 the same).
+    // Without an accumulator this rank's rows of those groups, else a copy per group behind the
+    // GEMM (8192x4096x4096 bf16 in sixteen groups, eight ranks, 211.8 -> 203.5; 8192x4096x2048 in four, four ranks, 124.0 ->
+    // 122.5, 4096x4096x4096 the same).
     int32_t sum_from = TM * TN;
     if (!same_stream && !fused && !monitor && h->link_bytes_per_s <= 0 && by_epilogue && (h->acc || D) && W > 1 &&
         (int64_t)M * N * 2 <= 0x7FFFFFFFLL) {

@@ -303,10 +303,10 @@ int fo_overlap_plan_rows_together(int M, int N, int K, int BN, int rLDN, int run
  * fork and a join, and nobody waits, so MM is not touched and stays zero; with
  * the monitor on, the signalling GEMM and one wait over all groups as elsewhere),
  * and so does, without the monitor, a product of at most one round of
- * 256x256 tiles (reduce-scatter: five sixths), one that 256 does not divide in M
- * or N, an all-reduce with neither accumulator nor normalisation, a
- * reduce-scatter of more than 16 groups without accumulator or with K below
- * 2048, and an all-reduce with an accumulator (apart from operands and product)
+ * 256x256 tiles (reduce-scatter without accumulator, or whose ranks do not own
+ * whole rows: five sixths), one that 256 does not divide in M or N, an
+ * all-reduce with neither accumulator nor normalisation, a reduce-scatter of
+ * more than 16 groups, and an all-reduce with an accumulator (apart from operands and product)
  * of more than 16 groups, or without the normalisation up to four rounds, or
  * with it where rounds are not whole rows, K is below 640, or two rounds have K
  * below 3584;
