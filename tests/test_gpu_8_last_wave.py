@@ -180,3 +180,34 @@ def test_automatic_choice_against_two_streams(fo, dtype, bm, bn, M, N, K, groups
     if norm:
         assert torch.equal(left[0][2], left[1][2])
     ov.close()
+
+
+@pytest.mark.parametrize("dtype,bm,bn,M,N,K,cseg,W", [
+    (F16, 128, 128, 4096, 4096, 2056, [256] * 4, 8),          # one round
+    (BF16, 256, 128, 4096, 8192, 2048, [50] * 20 + [24], 4),  # two waves, more groups than per-wave launches are made for
+    (F16, 128, 128, 4224, 7168, 1032, [500, 700, 648], 2),    # rows that 256 does not divide
+])
+@pytest.mark.parametrize("with_acc", [True, False])
+def test_automatic_choice_of_a_reduce_scatter(fo, dtype, bm, bn, M, N, K, cseg, W, with_acc):
+    """The same for a reduce-scatter: product, accumulator, this rank's rows and counters."""
+    rank = W - 1
+    algo, A, B, before, plain, RA, cs, cs_gpu, MM, ov = _setup(fo, dtype, bm, bn, M, N, K, cseg, "schedule")
+    ov.close()
+    ov = fo.ops.Overlap(rank=rank, world=W)
+    RE = fo.layout.generate_row_mapping(M, N, bm, bn, cseg, W)
+    left = []
+    for fused in (-1, 0):
+        ov.set_fused_consumer(fused)
+        acc = before.clone()
+        ov.set_accumulator(acc if with_acc else None)
+        C = torch.full((M * N,), float("nan"), device="cuda", dtype=TORCH_DTYPE[dtype])
+        D = torch.full((M // W * N,), float("nan"), device="cuda", dtype=TORCH_DTYPE[dtype])
+        for rep in range(2):
+            ov.gemm_reducescatter_overlap(A, B, C, D, MM, RA, RE, 1, cs, cs_gpu, algo)
+        torch.cuda.synchronize()
+        assert ov.status() == 0 and (MM == 0).all()
+        left.append((C, acc, D))
+    assert torch.equal(fo.layout.unpermute(left[0][0], M, N, bm, bn, RA, RE=RE), plain)
+    for one, two in zip(*left):
+        assert torch.equal(one, two)
+    ov.close()
