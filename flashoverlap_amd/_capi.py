@@ -49,6 +49,8 @@ SIGNATURES = {
     "fo_overlap_plan_batches": (c_int, [vp, c_int, c_int, vp]),
     "fo_overlap_plan_norm_rows": (c_int, [vp, c_int, c_int, vp, c_int, c_int, vp, c_int]),
     "fo_overlap_plan_rows_together": (c_int, [c_int] * 7),
+    "fo_overlap_plan_allreduce": (c_int, [vp, c_int, c_int, c_int, vp, vp, vp, vp, vp, c_int, vp, c_int, c_int, c_int, c_int]),
+    "fo_overlap_plan_reducescatter": (c_int, [vp, c_int, c_int, c_int, vp, vp, vp, vp, c_int, vp, c_int, c_int, c_int, c_int]),
     "fo_overlap_create": (c_int, [ctypes.POINTER(vp)]),
     "fo_overlap_destroy": (c_int, [vp]),
     "fo_overlap_set_gemm_stream": (c_int, [vp, vp]),

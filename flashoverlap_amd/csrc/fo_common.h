@@ -129,9 +129,9 @@ int fo_gemm_accumulate(int dtype, int M, int N, int K, int rLDN, const int32_t *
 int fo_gemm_reduce_scatter(int dtype, int M, int N, int K, const int32_t *cseg_dev, int G, const void *A, const void *B, void *C,
                            void *acc, void *own, const int32_t *RA, const int32_t *RE, int W, int rank, int algo,
                            fo_stream_t stream);
-// First storage slot of the last wave of a counting launch that can do that wave's sums itself; M * N / (BM * BN) where
-// there is no such launch.
-int fo_gemm_last_wave(int algo, int M, int N, int32_t *first);
+// First storage slot of the last wave of a counting launch that can do that wave's sums itself, and all slots,
+// M * N / (BM * BN); the same where there is no such launch.
+int fo_gemm_last_wave(int algo, int M, int N, int32_t *first, int32_t *slots);
 // fo_gemm_signal / fo_gemm_scatter (RE != nullptr) where tiles from storage slot sum_from on are not counted but summed: added
 // to the accumulator (RE: in its reduce-scatter layout, and this rank's rows copied to `own`, if any, as
 // fo_gemm_reduce_scatter does; of accumulator and rows one may be missing).  For slots of the last wave (fo_gemm_last_wave)

@@ -383,7 +383,7 @@ int fo_gemm_reduce_scatter(int dtype, int M, int N, int K, const int32_t *cseg_d
     return run_gemm(MODE_RS, dtype, M, N, K, 1, cseg_dev, G, A, B, C, nullptr, RA, RE, 0, algo, stream, true, acc, &rs);
 }
 
-int fo_gemm_last_wave(int algo, int M, int N, int32_t *first) {
+int fo_gemm_last_wave(int algo, int M, int N, int32_t *first, int32_t *slots) {
     const fo_algo_entry *e = fo_algo_lookup(algo);
     if (!e) return FO_ERR_ALGO;
     fo_raster r;
@@ -391,8 +391,8 @@ int fo_gemm_last_wave(int algo, int M, int N, int32_t *first) {
     if (rc) return rc;
     const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, true, true, false, false);
     const int resident = fo_main_tile_resident();
-    *first = last_wave_sums(plan) ? (plan.count - 1) / resident * resident * (256 / e->f[0]) * (256 / e->f[1])
-                                  : (M / e->f[0]) * (N / e->f[1]);
+    *slots = (M / e->f[0]) * (N / e->f[1]);
+    *first = last_wave_sums(plan) ? (plan.count - 1) / resident * resident * (256 / e->f[0]) * (256 / e->f[1]) : *slots;
     return FO_OK;
 }
 

@@ -95,7 +95,7 @@ namespace {
 // eight ranks: 3456x4352x3072 123 -> 95, 4224x7168x3584 205 -> 194, 6272x8192x7168 651 -> 630, 8192x8064x7168 801 -> 703).
 // `fits`: the accumulator is one that every path takes; one that is not aligned is left to the one-launch consumer.
 bool in_stream(const fo_overlap *h, int M, int N, int K, bool idle, bool monitor, bool ragged, bool fits, bool scatter) {
-    if (!h->comm_stream) return true;
+    if (h->overlap_ready && !h->comm_stream) return true;  // (a planner's handle may not have been initialised)
     if (h->fused >= 0 || h->link_bytes_per_s > 0 || h->in_stream_below_flop <= 0) return false;
     if (2.0 * M * N * K < h->in_stream_below_flop) return true;
     if (monitor || !fits) return false;  // the monitor's GEMM counts and is waited for in any case
@@ -503,6 +503,39 @@ int norm_runs(const norm_plan &np, const std::vector<int> &runs, int dtype, cons
     return FO_OK;
 }
 
+// Whether the accumulator shares no memory with operands and product.
+bool accumulator_apart(const fo_overlap *h, int M, int N, int K, const void *A, const void *B, const void *C) {
+    const int64_t mn = (int64_t)M * N;
+    return h->acc && apart({h->acc, mn}, {{A, (int64_t)M * K}, {B, (int64_t)N * K}, {C, mn}});
+}
+
+// Whether an all-reduce stays on the GEMM stream.  fits: the consumer launches take the buffers.
+bool allreduce_in_stream(const fo_overlap *h, int M, int N, int K, int G, int algo, bool norm, bool monitor, bool fits, bool acc_apart) {
+    const bool automatic = h->fused < 0 && h->link_bytes_per_s <= 0 && h->in_stream_below_flop > 0;
+    return in_stream(h, M, N, K, !h->acc && !norm, monitor, M % 256 || N % 256, fits, false) ||
+           (automatic && !monitor && fits && acc_apart && epilogue_sums(algo, M, N, K, norm, fused_grid(h, G) != 0));
+}
+
+// An all-reduce on two streams whose consumer is launched batch by batch: the storage slot from which on the GEMM does the sums
+// itself (M * N / (BM * BN): nowhere).  Those of the last wave: nothing is left to overlap them with, and behind
+// the GEMM they are a wait, a launch and a second read of the product (17 + 4 us on 4096x8192, of which the GEMM's epilogue
+// takes 17).  Where the groups' ends are not the waves', the consumer also need not wait for the last wave to begin with the
+// rest of its first group.  Whole calls, us, consumer -> GEMM: groups across waves, 8192x8192x2048 in one 288 -> 274, 8192x4096x4096
+// in three 253 -> 242, by the pair of calls 8192x4096x2560 in one 203 -> 184; groups that end with waves, by the pair
+// 4096x8192x8192 422 -> 419, 8192x8192x8192 828 -> 824.  There the call that also normalises keeps its one kernel for the last
+// batch's sums and rows (4096x8192x1536 131 against 135 with sums in the GEMM).
+int allreduce_sum_from(const fo_overlap *h, int M, int N, const int32_t *cseg_host, int G, int wave, int algo, const void *C,
+                       const norm_plan *np, bool monitor, bool acc_apart, int32_t *sum_from) {
+    const int64_t mn = (int64_t)M * N;
+    int32_t first = 0;
+    int rc = fo_gemm_last_wave(algo, M, N, &first, sum_from);
+    if (rc) return rc;
+    if (fused_grid(h, G) || monitor || h->link_bytes_per_s > 0 || !acc_apart) return FO_OK;
+    if (np && !apart({h->acc, mn}, {{np->Y, mn}, {np->Wt, N}})) return FO_OK;
+    if (!np || slots_before_last_batch(cseg_host, G, wave) < first) *sum_from = first;
+    return FO_OK;
+}
+
 // GemmAllReduceOverlap on whatever `h` describes: a caller's handle, or the
 // streams and static workspace of a handle-free call.  np: the normalisation to enqueue behind the consumer
 // (null: none).
@@ -528,10 +561,8 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
 
     const bool fits = !h->acc || aligned(C, h->acc);
     const int64_t mn = (int64_t)M * N;
-    const bool acc_apart = h->acc && apart({h->acc, mn}, {{A, (int64_t)M * K}, {B, (int64_t)N * K}, {C, mn}});
-    const bool automatic = h->fused < 0 && h->link_bytes_per_s <= 0 && h->in_stream_below_flop > 0;
-    const bool same_stream = in_stream(h, M, N, K, !h->acc && !np, monitor != 0, M % 256 || N % 256, fits, false) ||
-                             (automatic && !monitor && fits && acc_apart && epilogue_sums(algo, M, N, K, np != nullptr, fused_grid(h, G) != 0));
+    const bool acc_apart = accumulator_apart(h, M, N, K, A, B, C);
+    const bool same_stream = allreduce_in_stream(h, M, N, K, G, algo, np != nullptr, monitor != 0, fits, acc_apart);
     if (np) {
         // on one stream all rows follow in one launch, whatever their slots
         rc = same_stream ? check_slots(np->RA_host, TM * TN) : last_slots(np->RA_host, TM, TN, last_slot);
@@ -551,6 +582,11 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
     rc = fo_gemm_signal_check(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, MM, RA, nullptr, monitor, algo);
     if (rc) return rc;
     if (!fused && !fits) return FO_ERR_SHAPE;
+    int32_t sum_from = TM * TN;
+    if (!same_stream) {
+        rc = allreduce_sum_from(h, M, N, cseg_host, G, wave, algo, C, np, monitor != 0, acc_apart, &sum_from);
+        if (rc) return rc;
+    }
     const bool captured = !same_stream && capturing(h);
     if (h->static_words) {
         // By a kernel, not a memset node, in case the GEMM stream is being captured.  The give-up word is left standing:
@@ -568,22 +604,7 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
     const bool quiet = same_stream && !monitor;
     // With nothing to wait for, the GEMM's epilogue does the consumer's work on the tile it holds in LDS.
     const bool consumed = quiet && acc_apart;
-    // The last wave's sums by the GEMM itself, from storage slot sum_from on: nothing is left to overlap them with, and behind
-    // the GEMM they are a wait, a launch and a second read of the product (17 + 4 us on 4096x8192, of which the GEMM's epilogue
-    // takes 17).  Where the groups' ends are not the waves', the consumer also need not wait for the last wave to begin with the
-    // rest of its first group.  Whole calls, us, consumer -> GEMM: groups across waves, 8192x8192x2048 in one 288 -> 274, 8192x4096x4096
-    // in three 253 -> 242, by the pair of calls 8192x4096x2560 in one 203 -> 184; groups that end with waves, by the pair
-    // 4096x8192x8192 422 -> 419, 8192x8192x8192 828 -> 824.  There the call that also normalises keeps its one kernel for the last
-    // batch's sums and rows (4096x8192x1536 131 against 135 with sums in the GEMM).
-    int32_t sum_from = TM * TN;
-    if (!same_stream && !fused && !monitor && h->link_bytes_per_s <= 0 && acc_apart &&
-        (!np || apart({h->acc, mn}, {{np->Y, mn}, {np->Wt, N}}))) {
-        int32_t first = 0;
-        rc = fo_gemm_last_wave(algo, M, N, &first);
-        if (rc) return rc;
-        if (!np || slots_before_last_batch(cseg_host, G, wave) < first) sum_from = first;
-    }
-    const bool sums_last = sum_from < TM * TN;
+    const bool sums_last = sum_from < TM * TN;  // the last wave's sums by the GEMM itself
     rc = sums_last  ? fo_gemm_signal_sums(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, MM, RA, nullptr, h->acc, sum_from, nullptr, 1, 0,
                                           algo, h->gemm_stream)
          : consumed ? fo_gemm_accumulate(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, h->acc, RA, algo, h->gemm_stream)
@@ -707,6 +728,40 @@ extern "C" int fo_overlap_plan_rows_together(int M, int N, int K, int BN, int rL
     return rows_together(M, N, K, BN, rLDN, runs, last != 0) ? 1 : 0;
 }
 
+namespace {
+
+// What both planners below refuse, and the Algo's tile.
+int check_plan(const fo_overlap *h, int M, int N, int K, int rLDN, const int32_t *cseg_host, int G, int algo, int32_t *info) {
+    if (!h || K <= 0) return FO_ERR_ARG;
+    int rc = fo_algo_info(algo, info);
+    if (rc) return rc;
+    if (M <= 0 || N <= 0 || M % info[0] || N % info[1]) return FO_ERR_SHAPE;
+    const long tiles = (long)(M / info[0]) * (N / info[1]);
+    if (rLDN <= 0 || tiles % rLDN) return FO_ERR_SHAPE;
+    return check_segments(cseg_host, G, tiles);
+}
+
+}  // namespace
+
+// What the calls do with these buffers (whose addresses alone are looked at), for a caller that wants to know and for tests on a
+// machine without a GPU: the functions the calls decide by.
+extern "C" int fo_overlap_plan_allreduce(const fo_overlap_t *h, int M, int N, int K, const void *A, const void *B, const void *C,
+                                         const void *Y, const void *Wt, int rLDN, const int32_t *cseg_host, int G, int wave_tiles,
+                                         int algo, int monitor) {
+    int32_t info[12], sum_from = 0;
+    int rc = check_plan(h, M, N, K, rLDN, cseg_host, G, algo, info);
+    if (rc) return rc;
+    norm_plan np;
+    np.Y = const_cast<void *>(Y);
+    np.Wt = Wt;
+    const bool acc_apart = accumulator_apart(h, M, N, K, A, B, C), fits = !h->acc || aligned(C, h->acc);
+    const bool same_stream = allreduce_in_stream(h, M, N, K, G, algo, Y != nullptr, monitor != 0, fits, acc_apart);
+    if (!fits && (same_stream || !fused_grid(h, G))) return FO_ERR_SHAPE;
+    if (same_stream) return 0;
+    rc = allreduce_sum_from(h, M, N, cseg_host, G, wave_tiles, algo, C, Y ? &np : nullptr, monitor != 0, acc_apart, &sum_from);
+    return rc ? rc : sum_from;
+}
+
 extern "C" int fo_overlap_gemm_allreduce(fo_overlap_t *h, int dtype, int M, int N, int K,
                                          const void *A, const void *B, void *C, int32_t *MM,
                                          const int32_t *RA, int TM, int TN, int rLDN,
@@ -734,6 +789,84 @@ extern "C" int fo_overlap_gemm_allreduce_norm(fo_overlap_t *h, int dtype, int M,
                              &np);
 }
 
+namespace {
+
+// How a reduce-scatter is carried out.
+struct scatter_route {
+    bool by_epilogue;      // whole rows of the output view are each rank's, and every buffer lies apart
+    bool own_in_consumer;  // the consumer also writes this rank's rows
+    bool fits;             // the consumer launches take the buffers
+    bool same_stream;
+};
+
+scatter_route route_scatter(const fo_overlap *h, int M, int N, int K, const void *A, const void *B, const void *C, const void *D,
+                            int rLDN, int G, int BM, bool monitor) {
+    scatter_route r;
+    const int W = h->world;
+    const int64_t seg_stride = (int64_t)M * N / W;
+    // Where whole rows of the output view are this rank's, the GEMM's epilogue can do what follows it on one stream: a copy
+    // per group (4-5 us each on this GPU) and the consumer.  2048x4096x2048, four groups, eight ranks, no accumulator, whole
+    // pass with the normalisation: 42.0 us with copies, 37.5 so.
+    const span a = {A, (int64_t)M * K}, b = {B, (int64_t)N * K}, prod = {C, (int64_t)M * N}, sum = {h->acc, (int64_t)M * N};
+    r.by_epilogue = rLDN == 1 && BM % W == 0 && !(((uintptr_t)C | (uintptr_t)D | (uintptr_t)h->acc) & 15) &&
+                    apart(sum, {a, b, prod}) && apart({D, seg_stride}, {a, b, prod, sum});
+    // With an accumulator and W > 1 the consumer also writes this rank's chunk of
+    // every group to D (ncclReduceScatter(C+acc -> D+acc/W, n/W) with one rank
+    // present, src/overlap_impl.cu:312-313); otherwise a copy per group does.
+    r.own_in_consumer = D && h->acc && W > 1;
+    r.fits = !h->acc || aligned(C, h->acc, r.own_in_consumer ? D : nullptr);
+    // The epilogue leaves nothing to overlap, and what it adds to the GEMM is less than two streams cost (whole calls with the
+    // normalisation, us, two streams and one): with an accumulator where there is one round, which no consumer runs beside,
+    // 4096x4096x4096 130 and 120, 4096x4096x8192 bf16 212 and 203; and where groups are so many that one polling launch would
+    // consume them, 4096x8192x4096 bf16 in twenty 244 and 225, 8192x8192x3584 bf16 in 32 415 and 401, 8192x8192x8192 in 64 835
+    // and 819, 16384x8192x2048 in 64 564 and 558.  Fewer groups and more rounds are left to the consumer: two rounds are the same
+    // either way (8192x4096x4096 in eight 234 and 234, 4096x8192x1536 129 and 128), four are not (8192x8192x3584 bf16 387 and 401).
+    // Without an accumulator all there is to overlap are copies, and many take longer than the GEMM (8192x4096x4096 in 24
+    // groups 284, on one stream 215).  Up to sixteen groups stay on two streams, where their counters are waited for and reset,
+    // which a caller can see, at 1 to 9 % (16384x8192x1024 285 and 273, 8192x4096x4096 in sixteen 201 and 196).
+    const bool one_round = (long)((M + 255) / 256) * ((N + 255) / 256) <= (long)fo_main_tile_resident();
+    const bool idle = r.by_epilogue && (h->acc ? one_round || fused_grid(h, G) != 0 : G > kFewCopies);
+    // A ragged call's gain on one stream (see in_stream) is there by the epilogue (us, eight ranks, two streams' 8064x8064x7168 in
+    // four groups with launches behind the GEMM 750, so 719) and with one consumer launch for all groups or a few copies behind it.
+    const bool few_copies = !h->acc && G <= (2.0 * M * N * K >= kManyCopiesFromFlop ? kFewCopies : kFewCopiesOfShort);
+    const bool ragged = (M % 256 || N % 256) && (r.by_epilogue || (h->acc && W > 1) || few_copies);
+    r.same_stream = in_stream(h, M, N, K, idle, monitor, ragged, r.fits, true);
+    return r;
+}
+
+// A reduce-scatter on two streams whose consumer is launched batch by batch: the storage slot from which on the GEMM does the
+// rest itself (M * N / (BM * BN): nowhere).  The last batch's sums and rows, where that batch is of the last wave only (us: 8192x4096x4096, eight ranks
+// 235.6 -> 230.4, 8192x8192x3584 bf16 398 -> 389, 4096x8192x2048 bf16 146.7 -> 143.3).
+// Without an accumulator this rank's rows of those groups, else a copy per group behind the
+// GEMM (8192x4096x4096 bf16 in sixteen groups, eight ranks, 211.8 -> 203.5; 8192x4096x2048 in four, four ranks, 124.0 ->
+// 122.5, 4096x4096x4096 the same).
+int scatter_sum_from(const fo_overlap *h, const scatter_route &r, int M, int N, const void *D, const int32_t *cseg_host, int G,
+                     int wave, int algo, bool monitor, int32_t *sum_from) {
+    int32_t first = 0;
+    int rc = fo_gemm_last_wave(algo, M, N, &first, sum_from);
+    if (rc) return rc;
+    if (fused_grid(h, G) || monitor || h->link_bytes_per_s > 0 || !r.by_epilogue || !(h->acc || D) || h->world <= 1) return FO_OK;
+    if ((int64_t)M * N * 2 > 0x7FFFFFFFLL) return FO_OK;  // the accumulator is read through one 31-bit buffer range
+    const long before = slots_before_last_batch(cseg_host, G, wave);
+    if (before >= first) *sum_from = (int32_t)before;
+    return FO_OK;
+}
+
+}  // namespace
+
+extern "C" int fo_overlap_plan_reducescatter(const fo_overlap_t *h, int M, int N, int K, const void *A, const void *B,
+                                             const void *C, const void *D, int rLDN, const int32_t *cseg_host, int G,
+                                             int wave_tiles, int algo, int monitor) {
+    int32_t info[12], sum_from = 0;
+    int rc = check_plan(h, M, N, K, rLDN, cseg_host, G, algo, info);
+    if (rc) return rc;
+    const scatter_route r = route_scatter(h, M, N, K, A, B, C, D, rLDN, G, info[0], monitor != 0);
+    if (!r.fits && (r.same_stream || !fused_grid(h, G))) return FO_ERR_SHAPE;
+    if (r.same_stream) return 0;
+    rc = scatter_sum_from(h, r, M, N, D, cseg_host, G, wave_tiles, algo, monitor != 0, &sum_from);
+    return rc ? rc : sum_from;
+}
+
 extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, int N, int K,
                                              const void *A, const void *B, void *C, void *D,
                                              int32_t *MM, const int32_t *RA, const int32_t *RE,
@@ -756,33 +889,8 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     rc = link_fits(h, (int64_t)M * N * 2);
     if (rc) return rc;
 
-    // Where whole rows of the output view are this rank's, the GEMM's epilogue can do what follows it on one stream: a copy
-    // per group (4-5 us each on this GPU) and the consumer.  2048x4096x2048, four groups, eight ranks, no accumulator, whole
-    // pass with the normalisation: 42.0 us with copies, 37.5 so.
-    const span a = {A, (int64_t)M * K}, b = {B, (int64_t)N * K}, prod = {C, (int64_t)M * N}, sum = {h->acc, (int64_t)M * N};
-    const bool by_epilogue = rLDN == 1 && info[0] % W == 0 && !(((uintptr_t)C | (uintptr_t)D | (uintptr_t)h->acc) & 15) &&
-                             apart(sum, {a, b, prod}) && apart({D, seg_stride}, {a, b, prod, sum});
-    // With an accumulator and W > 1 the consumer also writes this rank's chunk of
-    // every group to D (ncclReduceScatter(C+acc -> D+acc/W, n/W) with one rank
-    // present, src/overlap_impl.cu:312-313); otherwise a copy per group does.
-    const bool own_in_consumer = D && h->acc && W > 1;
-    const bool fits = !h->acc || aligned(C, h->acc, own_in_consumer ? D : nullptr);
-    // The epilogue leaves nothing to overlap, and what it adds to the GEMM is less than two streams cost (whole calls with the
-    // normalisation, us, two streams and one): with an accumulator where there is one round, which no consumer runs beside,
-    // 4096x4096x4096 130 and 120, 4096x4096x8192 bf16 212 and 203; and where groups are so many that one polling launch would
-    // consume them, 4096x8192x4096 bf16 in twenty 244 and 225, 8192x8192x3584 bf16 in 32 415 and 401, 8192x8192x8192 in 64 835
-    // and 819, 16384x8192x2048 in 64 564 and 558.  Fewer groups and more rounds are left to the consumer: two rounds are the same
-    // either way (8192x4096x4096 in eight 234 and 234, 4096x8192x1536 129 and 128), four are not (8192x8192x3584 bf16 387 and 401).
-    // Without an accumulator all there is to overlap are copies, and many take longer than the GEMM (8192x4096x4096 in 24
-    // groups 284, on one stream 215).  Up to sixteen groups stay on two streams, where their counters are waited for and reset,
-    // which a caller can see, at 1 to 9 % (16384x8192x1024 285 and 273, 8192x4096x4096 in sixteen 201 and 196).
-    const bool one_round = (long)((M + 255) / 256) * ((N + 255) / 256) <= (long)fo_main_tile_resident();
-    const bool idle = by_epilogue && (h->acc ? one_round || fused_grid(h, G) != 0 : G > kFewCopies);
-    // A ragged call's gain on one stream (see in_stream) is there by the epilogue (us, eight ranks, two streams' 8064x8064x7168 in
-    // four groups with launches behind the GEMM 750, so 719) and with one consumer launch for all groups or a few copies behind it.
-    const bool few_copies = !h->acc && G <= (2.0 * M * N * K >= kManyCopiesFromFlop ? kFewCopies : kFewCopiesOfShort);
-    const bool ragged = (M % 256 || N % 256) && (by_epilogue || (h->acc && W > 1) || few_copies);
-    const bool same_stream = in_stream(h, M, N, K, idle, monitor != 0, ragged, fits, true);
+    const scatter_route route = route_scatter(h, M, N, K, A, B, C, D, rLDN, G, info[0], monitor != 0);
+    const bool same_stream = route.same_stream, own_in_consumer = route.own_in_consumer;
     const int fused = same_stream ? 0 : fused_grid(h, G);
     fo_stream_t cstream = same_stream ? h->gemm_stream : h->comm_stream;
     int32_t wave = 0;
@@ -794,31 +902,22 @@ extern "C" int fo_overlap_gemm_reducescatter(fo_overlap_t *h, int dtype, int M, 
     }
     rc = fo_gemm_signal_check(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, MM, RA, RE, monitor, algo);
     if (rc) return rc;
-    if (!fused && !fits) return FO_ERR_SHAPE;
+    if (!fused && !route.fits) return FO_ERR_SHAPE;
+    int32_t sum_from = TM * TN;
+    if (!same_stream) {
+        rc = scatter_sum_from(h, route, M, N, D, cseg_host, G, wave, algo, monitor != 0, &sum_from);
+        if (rc) return rc;
+    }
     const bool captured = !same_stream && capturing(h);
     if (!same_stream) {
         rc = fork(h, captured, fused != 0);
         if (rc) return rc;
     }
     const bool quiet = same_stream && !monitor;  // as in fo_overlap_gemm_allreduce
-    if (quiet && by_epilogue) {
+    if (quiet && route.by_epilogue) {
         rc = fo_gemm_reduce_scatter(dtype, M, N, K, cseg_dev, G, A, B, C, h->acc, D, RA, RE, W, h->rank, algo, h->gemm_stream);
         if (rc) return rc;
         return link_time(h, (int64_t)M * N * 2, h->gemm_stream);
-    }
-    // The last batch's sums and rows by the GEMM itself, where that batch is of the last wave only (us: 8192x4096x4096, eight ranks
-    // 235.6 -> 230.4, 8192x8192x3584 bf16 398 -> 389, 4096x8192x2048 bf16 146.7 -> 143.3).
-    // Without an accumulator this rank's rows of those groups, else a copy per group behind the
-    // GEMM (8192x4096x4096 bf16 in sixteen groups, eight ranks, 211.8 -> 203.5; 8192x4096x2048 in four, four ranks, 124.0 ->
-    // 122.5, 4096x4096x4096 the same).
-    int32_t sum_from = TM * TN;
-    if (!same_stream && !fused && !monitor && h->link_bytes_per_s <= 0 && by_epilogue && (h->acc || D) && W > 1 &&
-        (int64_t)M * N * 2 <= 0x7FFFFFFFLL) {
-        int32_t first = 0;
-        rc = fo_gemm_last_wave(algo, M, N, &first);
-        if (rc) return rc;
-        const long before = slots_before_last_batch(cseg_host, G, wave);
-        if (before >= first) sum_from = (int32_t)before;
     }
     rc = quiet ? fo_gemm_reordered_quiet(dtype, M, N, K, rLDN, cseg_dev, G, A, B, C, RA, RE, algo,
                                          h->gemm_stream)
@@ -896,7 +995,7 @@ extern "C" int fo_overlap_gemm_allreduce_serial(fo_overlap_t *h, int dtype, int 
     int rc = link_fits(h, mn * 2);
     if (rc) return rc;
     if (h->acc && !aligned(C, h->acc)) return FO_ERR_SHAPE;
-    const bool consumed = h->acc && apart({h->acc, mn}, {{A, (int64_t)M * K}, {B, (int64_t)N * K}, {C, mn}});
+    const bool consumed = accumulator_apart(h, M, N, K, A, B, C);
     rc = consumed ? fo_gemm_accumulate(dtype, M, N, K, 1, nullptr, 0, A, B, C, h->acc, nullptr, algo, h->gemm_stream)
                   : fo_gemm(dtype, M, N, K, A, B, C, algo, h->gemm_stream);
     if (!rc && h->acc && !consumed) rc = fo_consumer_reduce(dtype, C, h->acc, mn, h->gemm_stream);

@@ -297,6 +297,16 @@ int fo_overlap_plan_norm_rows(const int32_t *RA_host, int TM, int TN, const int3
  * consumer launch and one for the rows (accumulator apart from product and output, no link rate).  BN: the Algo's tile
  * width; runs: the batch's runs of consecutive tile rows; last: nothing of the GEMM is left behind it. */
 int fo_overlap_plan_rows_together(int M, int N, int K, int BN, int rLDN, int runs, int last);
+/* The route of a call (host only; of the buffers the addresses alone are looked at): 0 if it stays on the GEMM stream,
+ * otherwise the first storage slot whose sums the GEMM does itself, M*N/(BM*BN) if the consumer stream does all of them.
+ * fo_overlap_plan_allreduce: fo_overlap_gemm_allreduce, with Y and Wt fo_overlap_gemm_allreduce_norm;
+ * fo_overlap_plan_reducescatter: fo_overlap_gemm_reducescatter.  With the handle's settings, as though fo_overlap_init had
+ * been called.  wave_tiles: what fo_gemm_wave_tiles says.  A negative error for shapes and groups that the calls refuse. */
+int fo_overlap_plan_allreduce(const fo_overlap_t *h, int M, int N, int K, const void *A, const void *B, const void *C,
+                              const void *Y, const void *Wt, int rLDN, const int32_t *cseg_host, int G, int wave_tiles, int algo,
+                              int monitor);
+int fo_overlap_plan_reducescatter(const fo_overlap_t *h, int M, int N, int K, const void *A, const void *B, const void *C,
+                                  const void *D, int rLDN, const int32_t *cseg_host, int G, int wave_tiles, int algo, int monitor);
 /* fused < 0 (default): chosen per call.  A GEMM below 6.4e10 flop (about 50 us)
  * keeps the whole call on the GEMM stream (the GEMM with its reordered store,
  * whose epilogue does the consumer's work too: nothing that short can hide a
