@@ -524,6 +524,9 @@ bool allreduce_in_stream(const fo_overlap *h, int M, int N, int K, int G, int al
 // in three 253 -> 242, by the pair of calls 8192x4096x2560 in one 203 -> 184; groups that end with waves, by the pair
 // 4096x8192x8192 422 -> 419, 8192x8192x8192 828 -> 824.  There the call that also normalises keeps its one kernel for the last
 // batch's sums and rows (4096x8192x1536 131 against 135 with sums in the GEMM).
+//
+// The rows that the last wave completes then follow on the GEMM stream, while the consumer may still read the product and update
+// the accumulator: only rows that share memory with neither.
 int allreduce_sum_from(const fo_overlap *h, int M, int N, const int32_t *cseg_host, int G, int wave, int algo, const void *C,
                        const norm_plan *np, bool monitor, bool acc_apart, int32_t *sum_from) {
     const int64_t mn = (int64_t)M * N;
@@ -531,7 +534,7 @@ int allreduce_sum_from(const fo_overlap *h, int M, int N, const int32_t *cseg_ho
     int rc = fo_gemm_last_wave(algo, M, N, &first, sum_from);
     if (rc) return rc;
     if (fused_grid(h, G) || monitor || h->link_bytes_per_s > 0 || !acc_apart) return FO_OK;
-    if (np && !apart({h->acc, mn}, {{np->Y, mn}, {np->Wt, N}})) return FO_OK;
+    if (np && !(apart({np->Y, mn}, {{C, mn}, {h->acc, mn}}) && apart({h->acc, mn}, {{np->Wt, N}}))) return FO_OK;
     if (!np || slots_before_last_batch(cseg_host, G, wave) < first) *sum_from = first;
     return FO_OK;
 }

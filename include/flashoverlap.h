@@ -387,7 +387,9 @@ int fo_overlap_gemm_allreduce(fo_overlap_t *h, int dtype, int M, int N, int K, c
  * goes behind the last batch), so with a reorder table built from fo_schedule_order
  * and whole-row waves (fo_gemm_set_row_waves) only the last wave's consumer and rows
  * remain behind the GEMM.  RA_host: a host copy of RA (the call plans from it; it is
- * not kept).  Y[M,N] row-major, Wt[N]; N <= 16384, M*N*2 bytes below 4 GiB.  The GEMM
+ * not kept).  Y[M,N] row-major, Wt[N]; N <= 16384, M*N*2 bytes below 4 GiB.  Y may share
+ * memory with C: the accumulator takes the product and none of the rows (which rows come
+ * out where another one's product was written over first is unspecified).  The GEMM
  * stream continues when Y is complete.  Results: C, MM and the accumulator exactly as
  * fo_overlap_gemm_allreduce leaves them; Y as fo_reorder_rmsnorm_rows computes it
  * (same arithmetic as fo_reorder_rmsnorm, partial sums in another order). */

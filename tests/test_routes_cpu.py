@@ -82,6 +82,15 @@ def test_route_of_an_allreduce(M, N, K, cseg, kw, want):
         assert h.allreduce(M, N, K, cseg, **kw) == want
 
 
+@pytest.mark.parametrize("offset", [0, 256 * 4096 * 2, 8192 * 4096 * 2 - 16, -8192 * 4096 * 2 + 16])
+@pytest.mark.parametrize("settings", [dict(), dict(fused=0)])
+def test_rows_over_the_product_follow_its_consumer(settings, offset):
+    """Rows that share memory with the product, behind it on one stream: a consumer on the other that had yet to read the first
+    wave's slots would add rows to the accumulator."""
+    with Handle(**settings) as h:
+        assert h.allreduce(8192, 4096, 4096, 1, norm=True, Y=3 * BUFFER + offset) == two(8192, 4096)
+
+
 @pytest.mark.parametrize("settings", [dict(in_stream_below_flop=0, fused_from_groups=1 << 20), dict(link=100.0)])
 @pytest.mark.parametrize("M,N,cseg,tile,first", [
     (8192, 4096, [1024, 1024], (128, 128), 1024),
