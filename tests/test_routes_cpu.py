@@ -91,6 +91,13 @@ def test_rows_over_the_product_follow_its_consumer(settings, offset):
         assert h.allreduce(8192, 4096, 4096, 1, norm=True, Y=3 * BUFFER + offset) == two(8192, 4096)
 
 
+@pytest.mark.parametrize("Y", [BUFFER, 2 * BUFFER, 4 * BUFFER - 16])
+def test_rows_over_the_operands_follow_the_gemm(Y):
+    """One group: its rows follow the whole GEMM, also where its first waves complete some of them."""
+    with Handle() as h:
+        assert h.allreduce(8192, 4096, 4096, 1, norm=True, Y=Y) == two(8192, 4096)
+
+
 @pytest.mark.parametrize("settings", [dict(in_stream_below_flop=0, fused_from_groups=1 << 20), dict(link=100.0)])
 @pytest.mark.parametrize("M,N,cseg,tile,first", [
     (8192, 4096, [1024, 1024], (128, 128), 1024),
