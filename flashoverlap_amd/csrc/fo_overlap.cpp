@@ -516,7 +516,7 @@ bool allreduce_in_stream(const fo_overlap *h, int M, int N, int K, int G, int al
            (automatic && !monitor && fits && acc_apart && epilogue_sums(algo, M, N, K, norm, fused_grid(h, G) != 0));
 }
 
-// An all-reduce on two streams whose consumer is launched batch by batch: the storage slot from which on the GEMM does the sums
+// An all-reduce that chose two streams and launches per batch by itself: the storage slot from which on the GEMM does the sums
 // itself (M * N / (BM * BN): nowhere).  Those of the last wave: nothing is left to overlap them with, and behind
 // the GEMM they are a wait, a launch and a second read of the product (17 + 4 us on 4096x8192, of which the GEMM's epilogue
 // takes 17).  Where the groups' ends are not the waves', the consumer also need not wait for the last wave to begin with the
@@ -534,7 +534,7 @@ int allreduce_sum_from(const fo_overlap *h, int M, int N, int K, const int32_t *
     int32_t first = 0;
     int rc = fo_gemm_last_wave(algo, M, N, &first, sum_from);
     if (rc) return rc;
-    if (fused_grid(h, G) || monitor || h->link_bytes_per_s > 0 || !acc_apart) return FO_OK;
+    if (h->fused >= 0 || fused_grid(h, G) || monitor || h->link_bytes_per_s > 0 || !acc_apart) return FO_OK;
     if (np && !(apart({np->Y, mn}, {{A, (int64_t)M * K}, {B, (int64_t)N * K}, {C, mn}, {h->acc, mn}}) &&
                 apart({h->acc, mn}, {{np->Wt, N}})))
         return FO_OK;
@@ -840,7 +840,7 @@ scatter_route route_scatter(const fo_overlap *h, int M, int N, int K, const void
     return r;
 }
 
-// A reduce-scatter on two streams whose consumer is launched batch by batch: the storage slot from which on the GEMM does the
+// A reduce-scatter that chose two streams and launches per batch by itself: the storage slot from which on the GEMM does the
 // rest itself (M * N / (BM * BN): nowhere).  The last batch's sums and rows, where that batch is of the last wave only (us: 8192x4096x4096, eight ranks
 // 235.6 -> 230.4, 8192x8192x3584 bf16 398 -> 389, 4096x8192x2048 bf16 146.7 -> 143.3).
 // Without an accumulator this rank's rows of those groups, else a copy per group behind the
@@ -851,7 +851,8 @@ int scatter_sum_from(const fo_overlap *h, const scatter_route &r, int M, int N, 
     int32_t first = 0;
     int rc = fo_gemm_last_wave(algo, M, N, &first, sum_from);
     if (rc) return rc;
-    if (fused_grid(h, G) || monitor || h->link_bytes_per_s > 0 || !r.by_epilogue || !(h->acc || D) || h->world <= 1) return FO_OK;
+    if (h->fused >= 0 || fused_grid(h, G) || monitor || h->link_bytes_per_s > 0) return FO_OK;
+    if (!r.by_epilogue || !(h->acc || D) || h->world <= 1) return FO_OK;
     if ((int64_t)M * N * 2 > 0x7FFFFFFFLL) return FO_OK;  // the accumulator is read through one 31-bit buffer range
     const long before = slots_before_last_batch(cseg_host, G, wave);
     if (before >= first) *sum_from = (int32_t)before;

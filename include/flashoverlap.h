@@ -273,7 +273,9 @@ int fo_overlap_init(fo_overlap_t *h);
  * for world == 1). */
 int fo_overlap_set_world(fo_overlap_t *h, int rank, int world);
 /* Accumulation buffer of the stand-in consumer (no counterpart: the reference
- * reduces across ranks in place).  acc == NULL detaches it.  For W > 1 it is
+ * reduces across ranks in place).  A call reads and writes it on the GEMM stream,
+ * on the consumer stream or on both, between what precedes the call on the GEMM
+ * stream and what follows it there.  acc == NULL detaches it.  For W > 1 it is
  * [W, M/W, N] (seg_stride = M/W*N elements). */
 int fo_overlap_set_accumulator(fo_overlap_t *h, void *acc, int64_t nelem);
 /* How the per-group consumer path batches its launches (host-only, no GPU
@@ -321,7 +323,9 @@ int fo_overlap_plan_reducescatter(const fo_overlap_t *h, int M, int N, int K, co
  * with it where rounds are not whole rows, K is below 640, or two rounds have K
  * below 3584;
  * otherwise one launch when there are more than 16 groups, else per-wave
- * launches.  0: always the second stream with wait + consumer launches per
+ * launches, where the GEMM may do the last wave's sums itself: the slots of
+ * that wave are then neither counted nor waited for (fo_overlap_plan_allreduce
+ * and fo_overlap_plan_reducescatter report which).  0: always the second stream with wait + consumer launches per
  * group (per GEMM wave) as the reference's host loop
  * (src/overlap_impl.cu:250-258); 1: always one fo_wait_reduce_groups launch
  * with the default grid; n > 1: the same with n workgroups. */

@@ -9,6 +9,7 @@ from gpu_util import BF16, F16, TORCH_DTYPE, seeded
 
 pytestmark = pytest.mark.gpu
 EPS = 1e-6
+TWO_STREAMS = dict(in_stream_below_flop=0, fused_from_groups=1 << 20)  # however short, and launches per wave however many groups
 
 
 def _setup(fo, dtype, bm, bn, M, N, K, cseg, order):
@@ -28,8 +29,7 @@ def _setup(fo, dtype, bm, bn, M, N, K, cseg, order):
     cs = torch.tensor(cseg, dtype=torch.int32)
     MM = torch.zeros(fo.layout.counter_size(len(cseg), TM, TN), dtype=torch.int32, device="cuda")
     ov = fo.ops.Overlap()
-    ov.set_schedule(in_stream_below_flop=0)  # two streams, however short
-    ov.set_fused_consumer(0)                 # per-wave launches, however many groups
+    ov.set_schedule(**TWO_STREAMS)
     return algo, A, B, before, plain, RA, cs, cs.cuda(), MM, ov
 
 
@@ -86,8 +86,7 @@ def test_reduce_scatter(fo, dtype, bm, bn, M, N, K, cseg, order, W, own):
     rank = W - 1
     ov.close()
     ov = fo.ops.Overlap(rank=rank, world=W)
-    ov.set_schedule(in_stream_below_flop=0)
-    ov.set_fused_consumer(0)
+    ov.set_schedule(**TWO_STREAMS)
     RE = fo.layout.generate_row_mapping(M, N, bm, bn, cseg, W)
     acc = before.clone()
     ov.set_accumulator(acc)
@@ -122,8 +121,7 @@ def test_reduce_scatter_rows_without_accumulator(fo, dtype, bm, bn, M, N, K, cse
     ov.close()
     rank = 0
     ov = fo.ops.Overlap(rank=rank, world=W)
-    ov.set_schedule(in_stream_below_flop=0)
-    ov.set_fused_consumer(0)
+    ov.set_schedule(**TWO_STREAMS)
     RE = fo.layout.generate_row_mapping(M, N, bm, bn, cseg, W)
     td = TORCH_DTYPE[dtype]
     for rep in range(2):

@@ -135,6 +135,15 @@ def test_route_of_a_reduce_scatter(M, N, K, cseg, W, kw, want):
         assert h.reducescatter(M, N, K, cseg, **kw) == want
 
 
+@pytest.mark.parametrize("M,N,cseg", [(8192, 4096, [1024, 1024]), (8192, 8192, 3), (8192, 4096, 700), (128, 1024, 1), (8064, 8192, 4)])
+def test_launches_per_group_asked_for_are_all_there(M, N, cseg):
+    """set_fused_consumer(0): every slot is counted, waited for and summed on the second stream."""
+    with Handle(fused=0) as h:
+        assert h.allreduce(M, N, 4096, cseg) == h.allreduce(M, N, 4096, cseg, norm=True) == two(M, N)
+    with Handle(world=8, fused=0) as h:
+        assert h.reducescatter(M, N, 4096, cseg) == h.reducescatter(M, N, 4096, cseg, acc=None) == two(M, N)
+
+
 def test_a_planner_refuses_what_the_calls_refuse():
     with Handle() as h:
         for call in (h.allreduce, h.reducescatter):
