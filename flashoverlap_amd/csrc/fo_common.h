@@ -129,12 +129,15 @@ int fo_gemm_accumulate(int dtype, int M, int N, int K, int rLDN, const int32_t *
 int fo_gemm_reduce_scatter(int dtype, int M, int N, int K, const int32_t *cseg_dev, int G, const void *A, const void *B, void *C,
                            void *acc, void *own, const int32_t *RA, const int32_t *RE, int W, int rank, int algo,
                            fo_stream_t stream);
+// Whether a 128x128 block of rows that are `pitch` elements apart lies in one 31-bit buffer range (pitch up to 8.4 million).
+inline bool fo_block_in_range(int64_t pitch) { return (127 * pitch + 128) * 2 <= 0x7FFFFFFFLL; }
 // First storage slot of the last wave of a counting launch that can do that wave's sums itself, and all slots,
 // M * N / (BM * BN); the same where there is no such launch.
 int fo_gemm_last_wave(int algo, int M, int N, int32_t *first, int32_t *slots);
 // fo_gemm_signal / fo_gemm_scatter (RE != nullptr) where tiles from storage slot sum_from on are not counted but summed: added
 // to the accumulator (RE: in its reduce-scatter layout, and this rank's rows copied to `own`, if any, as
-// fo_gemm_reduce_scatter does; of accumulator and rows one may be missing).  For slots of the last wave (fo_gemm_last_wave)
+// fo_gemm_reduce_scatter does; of accumulator and rows one may be missing).  The accumulator is read through 31-bit
+// buffer ranges: fo_block_in_range(rLDN * BN), RE: M * N * 2 bytes within one.  For slots of the last wave (fo_gemm_last_wave)
 // as fo_schedule_order deals them out; others come out right, and late.
 int fo_gemm_signal_sums(int dtype, int M, int N, int K, int rLDN, const int32_t *cseg_dev, int G, const void *A, const void *B,
                         void *C, int32_t *MM, const int32_t *RA, const int32_t *RE, void *acc, int sum_from, void *own, int W,

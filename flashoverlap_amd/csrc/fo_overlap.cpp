@@ -528,13 +528,15 @@ bool allreduce_in_stream(const fo_overlap *h, int M, int N, int K, int G, int al
 // The rows that the last wave completes then follow on the GEMM stream, while the consumer's may still read the product and update
 // the accumulator, and rows of earlier waves may be written while the GEMM reads its operands: only rows that share memory with
 // none of these.
-int allreduce_sum_from(const fo_overlap *h, int M, int N, int K, const int32_t *cseg_host, int G, int wave, int algo, const void *A,
-                       const void *B, const void *C, const norm_plan *np, bool monitor, bool acc_apart, int32_t *sum_from) {
+int allreduce_sum_from(const fo_overlap *h, int M, int N, int K, int rLDN, int BN, const int32_t *cseg_host, int G, int wave, int algo,
+                       const void *A, const void *B, const void *C, const norm_plan *np, bool monitor, bool acc_apart,
+                       int32_t *sum_from) {
     const int64_t mn = (int64_t)M * N;
     int32_t first = 0;
     int rc = fo_gemm_last_wave(algo, M, N, &first, sum_from);
     if (rc) return rc;
     if (h->fused >= 0 || fused_grid(h, G) || monitor || h->link_bytes_per_s > 0 || !acc_apart) return FO_OK;
+    if (!fo_block_in_range((int64_t)rLDN * BN)) return FO_OK;
     if (np && !(apart({np->Y, mn}, {{A, (int64_t)M * K}, {B, (int64_t)N * K}, {C, mn}, {h->acc, mn}}) &&
                 apart({h->acc, mn}, {{np->Wt, N}})))
         return FO_OK;
@@ -590,7 +592,7 @@ int allreduce_overlap(fo_overlap *h, int dtype, int M, int N, int K, const void 
     if (!fused && !fits) return FO_ERR_SHAPE;
     int32_t sum_from = TM * TN;
     if (!same_stream) {
-        rc = allreduce_sum_from(h, M, N, K, cseg_host, G, wave, algo, A, B, C, np, monitor != 0, acc_apart, &sum_from);
+        rc = allreduce_sum_from(h, M, N, K, rLDN, info[1], cseg_host, G, wave, algo, A, B, C, np, monitor != 0, acc_apart, &sum_from);
         if (rc) return rc;
     }
     const bool captured = !same_stream && capturing(h);
@@ -764,7 +766,7 @@ extern "C" int fo_overlap_plan_allreduce(const fo_overlap_t *h, int M, int N, in
     const bool same_stream = allreduce_in_stream(h, M, N, K, G, algo, Y != nullptr, monitor != 0, fits, acc_apart);
     if (!fits && (same_stream || !fused_grid(h, G))) return FO_ERR_SHAPE;
     if (same_stream) return 0;
-    rc = allreduce_sum_from(h, M, N, K, cseg_host, G, wave_tiles, algo, A, B, C, Y ? &np : nullptr, monitor != 0, acc_apart, &sum_from);
+    rc = allreduce_sum_from(h, M, N, K, rLDN, info[1], cseg_host, G, wave_tiles, algo, A, B, C, Y ? &np : nullptr, monitor != 0, acc_apart, &sum_from);
     return rc ? rc : sum_from;
 }
 

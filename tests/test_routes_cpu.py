@@ -82,6 +82,18 @@ def test_route_of_an_allreduce(M, N, K, cseg, kw, want):
         assert h.allreduce(M, N, K, cseg, **kw) == want
 
 
+@pytest.mark.parametrize("M,N,rldn,in_range", [
+    (337 * 256, 49 * 256, 66052, True),   # rows of the view of 8454656 elements: the last that fit
+    (272 * 256, 64 * 256, 69632, False),  # 8912896
+    (272 * 256, 64 * 256, 1, True),
+])
+def test_rows_of_the_view_longer_than_a_buffer_range(M, N, rldn, in_range):
+    """The GEMM reads the accumulator of a 128x128 block through one 31-bit buffer range: what does not fit is the consumer's."""
+    assert (((127 * rldn * 128 + 128) * 2) < 1 << 31) == in_range
+    with Handle() as h:
+        assert (h.allreduce(M, N, 264, 1, rldn=rldn) < two(M, N)) == in_range
+
+
 @pytest.mark.parametrize("offset", [0, 256 * 4096 * 2, 8192 * 4096 * 2 - 16, -8192 * 4096 * 2 + 16])
 @pytest.mark.parametrize("settings", [dict(), dict(fused=0)])
 def test_rows_over_the_product_follow_its_consumer(settings, offset):
