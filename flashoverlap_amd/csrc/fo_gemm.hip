@@ -277,7 +277,7 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     a.grid_m = plan.grid_m; a.grid_n = plan.grid_n; a.panel = plan.panel; a.xcd_remap = plan.xcd_remap;
     a.first = 0; a.sub_m = a.sub_n = 1;
     a.count = plan.count;
-    a.half = (M % 256 ? 1 : 0) | (N % 256 ? 2 : 0);
+    a.half = (M % 256 ? 1 : 0) | (N % 256 ? 2 : 0) | (mode == MODE_ACC && !fo_block_in_range(RA ? (int64_t)rLDN * a.BN : N) ? 4 : 0);
     // counters the launch cannot move itself are moved behind it
     const bool signal_after = counts && !plan.whole;
     a.quiet = quiet || signal_after ? 1 : 0;

@@ -474,7 +474,8 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
         // 4096x4096x512 44.0 -> 41.6, 4096x4096x1024 55.9 -> 52.2, 4096x8192x264 85.7 -> 77.1, 3456x4352x3072 100.2 -> 97.3,
         // 8064x8064x4096 463.8 -> 455.7; 8192x8192x2048 by the serial call 276.5 -> 272.4).
         fo_u32x4 old[ACC ? NST : 1];
-        const bool early = MODE == MODE_ACC && KT >= kTakeFromSteps256;
+        // Not where rows are so long that the block's offsets leave a 31-bit range (p.half, bit 2).
+        const bool early = MODE == MODE_ACC && KT >= kTakeFromSteps256 && !(half & 4);
         int take_row = 0, take_step = 0;
         unsigned take_lane = 0;
         __amdgpu_buffer_rsrc_t take_from;

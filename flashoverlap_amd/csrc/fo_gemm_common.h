@@ -76,7 +76,7 @@ struct GemmArgs {
     int32_t *MM;
     int monitor;
     int quiet;                             // signalling epilogues: store the tiles reordered, touch no counter
-    int half;                              // 256x256 kernel: half a tile is left at the end of M (bit 0), N (bit 1)
+    int half;                              // 256x256 kernel: half a tile is left at the end of M (bit 0), N (bit 1); rows too long for early requests (bit 2)
     uint16_t *OWN;                         // MODE_RS: this rank's rows
     int W, rank, seg_rows;                 // MODE_RS: ranks, this rank, rows of the view per rank
     int stream_out;                        // 256x256 kernel: store the output with the non-temporal hint

@@ -519,3 +519,39 @@ def test_repeated_halves_are_not_multiplied(fo, dtype, bm, bn, M, N, K):
         assert torch.equal(layout.unpermute(Cp, M, N, bm, bn, RA, rLDN=rldn), want)
     assert (MM == 0).all()
     ov.close()
+
+
+@pytest.mark.parametrize("N,settings", [
+    (32768, dict(in_stream_below_flop=1e15)),                         # one stream: rows of 17.8 million elements
+    (16384, dict(in_stream_below_flop=0, fused_from_groups=1 << 20)),  # two: 8.9 million
+])
+def test_accumulator_rows_longer_than_a_buffer_range(fo, N, settings):
+    """An output view as wide as all tiles side by side: a 128x128 block of the accumulator then spans more than 31 bits, and its
+    old values are read with whole addresses, or left to the consumer."""
+    ops, td, M, K, bm, bn = fo.ops, TORCH_DTYPE[F16], 69632, 640, 128, 128
+    algo = fo._capi.find_algo(bm, bn, swizzle=4)
+    TM, TN = M // bm, N // bn
+    T = TM * TN
+    g = torch.Generator(device="cuda").manual_seed(5)
+    A = torch.randn(M, K, generator=g, device="cuda", dtype=td)
+    B = torch.randn(N, K, generator=g, device="cuda", dtype=td) * K ** -0.5
+    before = torch.randn(M * N, generator=g, device="cuda", dtype=td)
+    plain, C, acc = torch.empty(M, N, device="cuda", dtype=td), torch.empty(M * N, device="cuda", dtype=td), before.clone()
+    ops.gemm(A, B, plain, algo)
+    RA = torch.arange(T, dtype=torch.int32, device="cuda").reshape(TM, TN)
+    cs = torch.tensor([T], dtype=torch.int32)
+    MM = torch.zeros(fo.layout.counter_size(1, TM, TN), dtype=torch.int32, device="cuda")
+    ov = ops.Overlap()
+    ov.set_schedule(**settings)
+    ov.set_accumulator(acc)
+    ov.gemm_allreduce_overlap(A, B, C, MM, RA, T, cs, cs.cuda(), algo)
+    torch.cuda.synchronize()
+    assert ov.status() == 0 and (MM == 0).all()
+    step = TM // 8
+    for t in range(0, TM, step):  # tile rows, all rows of a tile
+        got = C.view(bm, TM, TN, bn)[:, t:t + step].permute(1, 0, 2, 3)
+        assert torch.equal(got, plain.view(TM, bm, TN, bn)[t:t + step])
+    step = M * N // 16
+    for i in range(0, M * N, step):
+        assert torch.equal(acc[i:i + step], (before[i:i + step].float() + C[i:i + step].float()).to(td))
+    ov.close()
