@@ -1,6 +1,8 @@
 """Helpers shared by the GPU parity tests: seeded inputs that the GPU path and the
 CPU checker see bit-for-bit, and conversions between torch tensors and the
 checker's uint16 bit patterns."""
+import ctypes
+
 import numpy as np
 import torch
 
@@ -23,6 +25,16 @@ def seeded(shape, dtype, seed, scale=1.0, dist="normal"):
     x = torch.randn(*shape, generator=g) if dist == "normal" else torch.rand(*shape, generator=g) * 2 - 1
     x16 = (x * scale).to(TORCH_DTYPE[dtype])
     return x16.cuda(), bits_of(x16)
+
+
+def planned_route(fo, ov, dtype, A, B, C, cseg, algo, rldn=1, Y=None, Wt=None, D=None, scatter=False):
+    """What the planners say of this call: 0 one stream, else the first storage slot that the GEMM sums itself."""
+    ptr = lambda t: None if t is None else t.data_ptr()
+    M, N, K = A.shape[0], B.shape[0], A.shape[1]
+    arr, wave, L = (ctypes.c_int32 * len(cseg))(*cseg), fo._capi.wave_tiles(algo, M, N, dtype), fo._capi.lib()
+    if scatter:
+        return L.fo_overlap_plan_reducescatter(ov._h, M, N, K, ptr(A), ptr(B), ptr(C), ptr(D), rldn, arr, len(cseg), wave, algo, 0)
+    return L.fo_overlap_plan_allreduce(ov._h, M, N, K, ptr(A), ptr(B), ptr(C), ptr(Y), ptr(Wt), rldn, arr, len(cseg), wave, algo, 0)
 
 
 def _f32(bits, dtype):

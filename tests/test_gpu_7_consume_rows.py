@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from gpu_util import BF16, F16, TORCH_DTYPE, seeded
+from gpu_util import BF16, F16, TORCH_DTYPE, planned_route, seeded
 from test_gpu_3_norm_overlap import _run_both
 
 pytestmark = pytest.mark.gpu
@@ -80,7 +80,8 @@ def test_many_wide_rows(fo, dtype, M, N):
 
 @pytest.mark.parametrize("dtype", [F16, BF16])
 @pytest.mark.parametrize("rows_behind", [0, 256])
-def test_rows_over_the_product(fo, dtype, rows_behind):
+@pytest.mark.parametrize("settings", [dict(), dict(in_stream_below_flop=0)])
+def test_rows_over_the_product(fo, dtype, rows_behind, settings):
     """Normalised rows written over the product: the accumulator takes the product and none of them.  One batch, tile rows in
     reverse order, so that most rows are written where another one's product lies (which rows then come out is nobody's
     promise: they are not looked at), and four times as many workgroups of rows as the GPU holds at once."""
@@ -96,13 +97,16 @@ def test_rows_over_the_product(fo, dtype, rows_behind):
     cs = torch.tensor([TM * TN], dtype=torch.int32)
     MM = torch.zeros(fo.layout.counter_size(1, TM, TN), dtype=torch.int32, device="cuda")
     ov = fo.ops.Overlap()
-    ov.set_fused_consumer(0)
+    ov.set_fused_consumer(-1 if settings else 0)  # launches per wave, by choice and always
+    ov.set_schedule(**settings)
     product, want = torch.empty(M * N, device="cuda", dtype=td), before.clone()
     ov.set_accumulator(want)
     ov.gemm_allreduce_overlap(A, B, product, MM, RA, 1, cs, cs.cuda(), algo)
     room = torch.empty((M + rows_behind) * N, device="cuda", dtype=td)
     C, Y, acc = room[:M * N], room[rows_behind * N:].view(M, N), before.clone()
     ov.set_accumulator(acc)
+    # on one stream, consumer and rows one behind the other: the rows of a last wave that the GEMM sums are behind the GEMM only
+    assert planned_route(fo, ov, dtype, A, B, C, [TM * TN], algo, 1, Y, gamma) == TM * TN
     ov.gemm_allreduce_rmsnorm_overlap(A, B, C, MM, RA, RA.cpu(), 1, cs, cs.cuda(), algo, Y, gamma, eps=1e-6)
     torch.cuda.synchronize()
     assert torch.equal(acc, want) and torch.equal(want, (before.float() + product.float()).to(td))

@@ -1,11 +1,12 @@
 """Calls on two streams whose last wave is summed by the GEMM itself: product, accumulator, this rank's rows, counters and
 normalised rows against their definitions, at the partitions and storage orders where the rule changes sides; and what
-automatic mode keeps on one stream against what two streams leave."""
+automatic mode keeps on one stream against what two streams leave.  Every route gives the same bits: which one a call takes
+is asked of the planners that the calls decide with."""
 import numpy as np
 import pytest
 import torch
 
-from gpu_util import BF16, F16, TORCH_DTYPE, seeded
+from gpu_util import BF16, F16, TORCH_DTYPE, planned_route, seeded
 
 pytestmark = pytest.mark.gpu
 EPS = 1e-6
@@ -52,10 +53,16 @@ def test_allreduce(fo, dtype, bm, bn, M, N, K, cseg, order, norm):
     ov.set_accumulator(acc)
     RA_cpu = RA.cpu()
     want_y = torch.empty(M, N, device="cuda", dtype=td)
+    per_wave = 256 * (256 // bm) * (256 // bn)
+    first = (sum(cseg) - 1) // per_wave * per_wave
+    across = first not in np.cumsum(cseg)  # groups across waves: the call that also normalises leaves the GEMM its sums then
+    last_begins = sum(cseg) if norm and not across else first
     for rep in range(2):
         C = torch.full((M * N,), float("nan"), device="cuda", dtype=td)
         Y = torch.full((M, N), float("nan"), device="cuda", dtype=td)
         was = acc.clone()
+        rows = (Y, gamma) if norm else (None, None)
+        assert planned_route(fo, ov, dtype, A, B, C, cseg, algo, 1, *rows) == last_begins
         if norm:
             ov.gemm_allreduce_rmsnorm_overlap(A, B, C, MM, RA, RA_cpu, 1, cs, cs_gpu, algo, Y, gamma, eps=EPS)
         else:
@@ -78,6 +85,8 @@ def test_allreduce(fo, dtype, bm, bn, M, N, K, cseg, order, norm):
     (F16, 128, 128, 8192, 4096, 72, [1000, 1048], "schedule", 4),          # the last begins in the wave before: as ever
     (BF16, 256, 128, 8192, 4096, 64, [512, 512], "any", 8),
     (F16, 128, 256, 4096, 7168, 200, [512, 300, 84], "schedule", 4),       # a partial last wave
+    (BF16, 128, 128, 8192, 4096, 136, [4] * 512, "schedule", 8),           # more groups than their sizes are held in registers
+    (F16, 128, 128, 8192, 4096, 72, [1024] + [1, 3] * 256, "any", 2),
 ])
 @pytest.mark.parametrize("own", [False, True])
 def test_reduce_scatter(fo, dtype, bm, bn, M, N, K, cseg, order, W, own):
@@ -92,6 +101,10 @@ def test_reduce_scatter(fo, dtype, bm, bn, M, N, K, cseg, order, W, own):
     ov.set_accumulator(acc)
     C = torch.full((M * N,), float("nan"), device="cuda", dtype=td)
     D = torch.full((M // W * N,), float("nan"), device="cuda", dtype=td) if own else None
+    per_wave = 256 * (256 // bm) * (256 // bn)
+    first = (sum(cseg) - 1) // per_wave * per_wave
+    route = planned_route(fo, ov, dtype, A, B, C, cseg, algo, D=D, scatter=True)
+    assert route == (first if first in np.cumsum(cseg) else sum(cseg))
     ov.gemm_reducescatter_overlap(A, B, C, D, MM, RA, RE, 1, cs, cs_gpu, algo)
     torch.cuda.synchronize()
     assert ov.status() == 0 and (MM == 0).all()
@@ -114,6 +127,7 @@ def test_reduce_scatter(fo, dtype, bm, bn, M, N, K, cseg, order, W, own):
     (F16, 128, 128, 8192, 4096, 72, [512] * 4, "schedule", 8),
     (BF16, 256, 128, 8192, 4096, 136, [512, 512], "any", 2),
     (F16, 128, 256, 4096, 7168, 200, [512, 300, 84], "schedule", 4),
+    (BF16, 128, 128, 8192, 4096, 64, [4] * 512, "schedule", 8),            # groups beyond the registers again
 ])
 def test_reduce_scatter_rows_without_accumulator(fo, dtype, bm, bn, M, N, K, cseg, order, W):
     """The same without an accumulator: this rank's rows of the last wave are the GEMM's too."""
@@ -127,6 +141,8 @@ def test_reduce_scatter_rows_without_accumulator(fo, dtype, bm, bn, M, N, K, cse
     for rep in range(2):
         C = torch.full((M * N,), float("nan"), device="cuda", dtype=td)
         D = torch.full((M // W * N,), float("nan"), device="cuda", dtype=td)
+        first = 256 * (256 // bm) * (256 // bn)  # two waves
+        assert planned_route(fo, ov, dtype, A, B, C, cseg, algo, D=D, scatter=True) == first
         ov.gemm_reducescatter_overlap(A, B, C, D, MM, RA, RE, 1, cs, cs_gpu, algo)
         torch.cuda.synchronize()
         assert ov.status() == 0 and (MM == 0).all()
@@ -164,6 +180,8 @@ def test_automatic_choice_against_two_streams(fo, dtype, bm, bn, M, N, K, groups
         C = torch.full((M * N,), float("nan"), device="cuda", dtype=td)
         Y = torch.full((M, N), float("nan"), device="cuda", dtype=td)
         ov.set_accumulator(acc)
+        rows = (Y, gamma) if norm else (None, None)
+        assert planned_route(fo, ov, dtype, A, B, C, cseg, algo, rldn, *rows) == (0 if fused < 0 else T)
         for rep in range(2):
             if norm:
                 ov.gemm_allreduce_rmsnorm_overlap(A, B, C, MM, RA, RA_cpu, rldn, cs, cs_gpu, algo, Y, gamma, eps=EPS)
@@ -181,7 +199,8 @@ def test_automatic_choice_against_two_streams(fo, dtype, bm, bn, M, N, K, groups
 
 
 @pytest.mark.parametrize("dtype,bm,bn,M,N,K,cseg,W", [
-    (F16, 128, 128, 4096, 4096, 2056, [256] * 4, 8),          # one round
+    (F16, 128, 128, 4096, 4096, 2056, [256] * 4, 8),          # one round; without an accumulator two streams all the same
+    (F16, 128, 128, 3328, 4096, 2504, [208] * 4, 8),          # five sixths of one
     (BF16, 256, 128, 4096, 8192, 2048, [50] * 20 + [24], 4),  # two waves, more groups than per-wave launches are made for
     (F16, 128, 128, 4224, 7168, 1032, [500, 700, 648], 2),    # rows that 256 does not divide
 ])
@@ -200,6 +219,8 @@ def test_automatic_choice_of_a_reduce_scatter(fo, dtype, bm, bn, M, N, K, cseg, 
         ov.set_accumulator(acc if with_acc else None)
         C = torch.full((M * N,), float("nan"), device="cuda", dtype=TORCH_DTYPE[dtype])
         D = torch.full((M // W * N,), float("nan"), device="cuda", dtype=TORCH_DTYPE[dtype])
+        one_stream = fused < 0 and (with_acc or M != 4096 or N != 4096)
+        assert planned_route(fo, ov, dtype, A, B, C, cseg, algo, D=D, scatter=True) == (0 if one_stream else sum(cseg))
         for rep in range(2):
             ov.gemm_reducescatter_overlap(A, B, C, D, MM, RA, RE, 1, cs, cs_gpu, algo)
         torch.cuda.synchronize()
@@ -208,4 +229,77 @@ def test_automatic_choice_of_a_reduce_scatter(fo, dtype, bm, bn, M, N, K, cseg, 
     assert torch.equal(fo.layout.unpermute(left[0][0], M, N, bm, bn, RA, RE=RE), plain)
     for one, two in zip(*left):
         assert torch.equal(one, two)
+    ov.close()
+
+
+@pytest.mark.parametrize("call,cseg", [
+    ("allreduce", [700, 700, 648]),
+    ("norm", [2048]),
+    ("reducescatter", [512] * 4),
+    ("reducescatter without accumulator", [512] * 4),
+])
+def test_captured_in_a_hip_graph(fo, call, cseg):
+    """A call whose last wave the GEMM sums, captured once and replayed with other operands and eager work between the replays."""
+    dtype, bm, bn, M, N, K, W = F16, 128, 128, 8192, 4096, 200, 8
+    td, scatter, with_acc = TORCH_DTYPE[dtype], call.startswith("reducescatter"), "without" not in call
+    algo, A, B, before, plain, RA, cs, cs_gpu, MM, ov = _setup(fo, dtype, bm, bn, M, N, K, cseg, "schedule")
+    ov.close()
+    gamma = (1 + 0.01 * torch.randn(N, generator=torch.Generator().manual_seed(7))).to(td).cuda()
+    RA_cpu, RE = RA.cpu(), fo.layout.generate_row_mapping(M, N, bm, bn, cseg, W) if scatter else None
+    C, acc = torch.empty(M * N, device="cuda", dtype=td), before.clone()
+    D, Y, want_y = (torch.empty(r, N, device="cuda", dtype=td) for r in (M // W, M, M))
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        ov = fo.ops.Overlap(rank=W - 1, world=W) if scatter else fo.ops.Overlap()
+        ov.set_schedule(**TWO_STREAMS)
+        ov.set_accumulator(acc if with_acc else None)
+
+        def step():
+            if scatter:
+                ov.gemm_reducescatter_overlap(A, B, C, D, MM, RA, RE, 1, cs, cs_gpu, algo)
+            elif call == "norm":
+                ov.gemm_allreduce_rmsnorm_overlap(A, B, C, MM, RA, RA_cpu, 1, cs, cs_gpu, algo, Y, gamma, eps=EPS)
+            else:
+                ov.gemm_allreduce_overlap(A, B, C, MM, RA, 1, cs, cs_gpu, algo)
+
+        step()  # one-time kernel attribute set-up
+    torch.cuda.synchronize()
+    rows = (Y, gamma) if call == "norm" else (None, None)
+    assert planned_route(fo, ov, dtype, A, B, C, cseg, algo, 1, *rows, D=D, scatter=scatter) == 1024
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        step()
+    torch.cuda.synchronize()
+    acc.copy_(before)
+    A0 = A.clone()
+    for rep in range(4):
+        A.copy_((A0 * (0.5 + 0.25 * rep)).roll(rep * 11, dims=1))
+        C.fill_(float("nan"))
+        Y.fill_(float("nan"))
+        D.fill_(float("nan"))
+        was = acc.clone()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        fo.ops.gemm(A, B, plain, algo)
+        torch.cuda.synchronize()
+        assert torch.equal(fo.layout.unpermute(C, M, N, bm, bn, RA, RE=RE), plain), f"replay {rep}"
+        if scatter:
+            view, seg = C.view(-1, bn), M * N // bn // W
+            want, mine, first = torch.empty_like(view), [], 0
+            for n in cseg:
+                chunk = view[first:first + n * bm].view(W, n * bm // W, bn)
+                want.view(W, seg, bn)[:, first // W:(first + n * bm) // W] = chunk
+                mine.append(chunk[W - 1])
+                first += n * bm
+            assert torch.equal(D.view(-1, bn), torch.cat(mine)), f"replay {rep}"
+        else:
+            want = C
+        if with_acc:
+            assert torch.equal(acc, (was.float() + want.reshape(-1).float()).to(td)), f"replay {rep}"
+        if call == "norm":
+            fo.ops.reorder_rmsnorm_rows(C.view(M, N), want_y, gamma, 0, M, bm, bn, 1, RA, eps=EPS)
+            torch.cuda.synchronize()
+            assert torch.equal(Y, want_y), f"replay {rep}"
+        assert (MM == 0).all() and ov.status() == 0
     ov.close()
