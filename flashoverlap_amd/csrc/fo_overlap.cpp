@@ -843,11 +843,10 @@ scatter_route route_scatter(const fo_overlap *h, int M, int N, int K, const void
 }
 
 // A reduce-scatter that chose two streams and launches per batch by itself: the storage slot from which on the GEMM does the
-// rest itself (M * N / (BM * BN): nowhere).  The last batch's sums and rows, where that batch is of the last wave only (us: 8192x4096x4096, eight ranks
-// 235.6 -> 230.4, 8192x8192x3584 bf16 398 -> 389, 4096x8192x2048 bf16 146.7 -> 143.3).
-// Without an accumulator this rank's rows of those groups, else a copy per group behind the
-// GEMM (8192x4096x4096 bf16 in sixteen groups, eight ranks, 211.8 -> 203.5; 8192x4096x2048 in four, four ranks, 124.0 ->
-// 122.5, 4096x4096x4096 the same).
+// rest itself (M * N / (BM * BN): nowhere).  The last batch's sums and rows, where that batch is of the last wave only (us:
+// 8192x4096x4096, eight ranks 235.6 -> 230.4, 8192x8192x3584 bf16 398 -> 389, 4096x8192x2048 bf16 146.7 -> 143.3).
+// Without an accumulator this rank's rows of those groups, else a copy per group behind the GEMM (8192x4096x4096 bf16 in
+// sixteen groups, eight ranks, 211.8 -> 203.5; 8192x4096x2048 in four, four ranks, 124.0 -> 122.5).
 int scatter_sum_from(const fo_overlap *h, const scatter_route &r, int M, int N, const void *D, const int32_t *cseg_host, int G,
                      int wave, int algo, bool monitor, int32_t *sum_from) {
     int32_t first = 0;

@@ -281,7 +281,8 @@ int fo_overlap_set_accumulator(fo_overlap_t *h, void *acc, int64_t nelem);
 /* How the per-group consumer path batches its launches (host-only, no GPU
  * needed): groups whose last tiles fall into the same stretch of wave_tiles
  * consecutive storage slots complete together and share one wait and one
- * consumer launch.  first[0..n] receives the first group of each batch and G
+ * consumer launch (the last batch only as far as the GEMM leaves it to the consumer,
+ * see fo_overlap_plan_allreduce).  first[0..n] receives the first group of each batch and G
  * at the end (room for G + 1 entries); returns n, or a negative error.
  * wave_tiles <= 0: no batching. */
 int fo_overlap_plan_batches(const int32_t *cseg_host, int G, int wave_tiles, int32_t *first);
@@ -291,12 +292,15 @@ int fo_overlap_plan_batches(const int32_t *cseg_host, int G, int wave_tiles, int
  * fo_overlap_plan_batches(cseg_host, G, wave_tiles, ...), i.e. as soon as the groups
  * holding all their tiles have been consumed.  At most four runs follow a batch that
  * is not the last (what a scattered reorder table leaves over goes behind the last
- * one).  RA_host: the reorder table [TM, TN] on the host.  Returns the number of
+ * one).  Where the GEMM does the last wave's sums itself (fo_overlap_plan_allreduce says
+ * from which slot on), the last batch ends at that slot: the rows complete below it
+ * follow its consumer, at most four runs beside the GEMM, and all that are left follow
+ * the GEMM on its own stream.  RA_host: the reorder table [TM, TN] on the host.  Returns the number of
  * runs, FO_ERR_LIMIT if there are more than max_runs, or a negative error. */
 int fo_overlap_plan_norm_rows(const int32_t *RA_host, int TM, int TN, const int32_t *cseg_host, int G,
                               int wave_tiles, int32_t *runs, int max_runs);
 /* 1 if that call consumes and normalises a batch that is exactly the tile rows it completes by one kernel, 0 if by a
- * consumer launch and one for the rows (accumulator apart from product and output, no link rate).  BN: the Algo's tile
+ * consumer launch and one for the rows (accumulator, product and output apart from one another, no link rate).  BN: the Algo's tile
  * width; runs: the batch's runs of consecutive tile rows; last: nothing of the GEMM is left behind it. */
 int fo_overlap_plan_rows_together(int M, int N, int K, int BN, int rLDN, int runs, int last);
 /* The route of a call (host only; of the buffers the addresses alone are looked at): 0 if it stays on the GEMM stream,
@@ -318,7 +322,8 @@ int fo_overlap_plan_reducescatter(const fo_overlap_t *h, int M, int N, int K, co
  * 256x256 tiles (reduce-scatter without accumulator, or whose ranks do not own
  * whole rows: five sixths), one that 256 does not divide in M or N, an
  * all-reduce with neither accumulator nor normalisation, a reduce-scatter of
- * more than 16 groups, and an all-reduce with an accumulator (apart from operands and product)
+ * more than 16 groups whose ranks own whole rows (rLDN 1, W divides the tile's
+ * height, buffers 16-byte aligned and apart), and an all-reduce with an accumulator (apart from operands and product)
  * of more than 16 groups, or without the normalisation up to four rounds, or
  * with it where rounds are not whole rows, K is below 640, or two rounds have K
  * below 3584;
@@ -388,7 +393,7 @@ int fo_overlap_gemm_allreduce(fo_overlap_t *h, int dtype, int M, int N, int K, c
  * holding its last tile has been consumed: behind each wait + consumer batch the
  * consumer stream gets the rows that batch completed (runs of consecutive tile
  * rows, at most four launches per batch; what a scattered reorder table leaves over
- * goes behind the last batch), so with a reorder table built from fo_schedule_order
+ * goes behind the last batch, or behind the GEMM where that does the last wave's sums), so with a reorder table built from fo_schedule_order
  * and whole-row waves (fo_gemm_set_row_waves) only the last wave's consumer and rows
  * remain behind the GEMM.  RA_host: a host copy of RA (the call plans from it; it is
  * not kept).  Y[M,N] row-major, Wt[N]; N <= 16384, M*N*2 bytes below 4 GiB.  Y may share
