@@ -23,7 +23,7 @@ typedef fo_bf16_tag inst_tag;
 
 int FO_CAT3(fo_gemm256_launch_, FO_INST_DTYPE, _, FO_INST_MODE)(const GemmArgs &a, hipStream_t stream, int *resident_out,
                                                              int expect_resident) {
-    return launch_kernel<fo_gemm256_kernel<inst_tag, FO_INST_MODE>, kSmem256, 256>(a, stream, resident_out, expect_resident);
+    return launch_kernel<GemmArgs, FO_INST_MODE, fo_gemm256_kernel<inst_tag, FO_INST_MODE>, kSmem256, 256>(a, stream, resident_out, expect_resident);
 }
 
 }  // namespace fo_gemm_dev

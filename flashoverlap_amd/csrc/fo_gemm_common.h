@@ -56,7 +56,7 @@ __host__ __device__ inline __attribute__((always_inline)) int fo_divide(int n, f
 constexpr long kMaxDivide = 32767;
 inline fo_div fo_divisor(long d) { return {d > 0 ? (uint32_t)(((1ULL << 31) + d - 1) / d) : 0}; }
 
-// The fields that a kernel's first operand load needs stand in front: they come with one load.
+// A launch as the host describes it, and the 256x256 kernel's arguments.
 struct GemmArgs {
     const uint16_t *A;
     const uint16_t *B;
@@ -64,8 +64,6 @@ struct GemmArgs {
     int lda, ldb;          // row strides of A and B in elements (multiples of 8)
     int grid_m, grid_n, panel, xcd_remap;  // the raster of this launch's parent tiles
     int first, sub_m, sub_n, count;        // this launch: positions from `first`, each cut into sub_m x sub_n macro tiles, `count` of them
-    fo_div by_panel, by_rows, by_last_rows;  // divisors of the raster walk (fo_set_divisors): tiles of a panel, its rows, the last panel's
-    int general;                           // another walk, or numbers too large for those
     uint16_t *C;
     uint16_t *ACC;         // MODE_ACC, MODE_RS: the accumulator
     int BM, BN, TN, rLDN;  // reorder/signal tile, tiles along N, reshaped width in tiles
@@ -81,34 +79,109 @@ struct GemmArgs {
     int W, rank, seg_rows;                 // MODE_RS: ranks, this rank, rows of the view per rank
     int stream_out;                        // 256x256 kernel: store the output with the non-temporal hint
     int sum_from;                          // MODE_SIGNAL_SUM, MODE_SCATTER_SUM: first storage slot that is summed
+
+    static GemmArgs of(const GemmArgs &a, int, int) { return a; }
 };
 
-inline void fo_set_divisors(GemmArgs &a) {
-    const long positions = (long)a.grid_m * a.grid_n;
-    a.by_panel = fo_divisor((long)a.panel * a.grid_n);
-    a.by_rows = fo_divisor(a.panel);
-    a.by_last_rows = fo_divisor(a.panel > 0 ? a.grid_m % a.panel : 1);
-    a.general = a.xcd_remap == 2 || a.sub_m * a.sub_n > 1 || positions > kMaxDivide;
+// The smaller tiles' arguments: 112 bytes, because a launch takes the host 2.7 us with up to 112 bytes of arguments and 3.1 to
+// 3.7 with 120 or more, those that the runtime adds for gridDim among them (an empty kernel in a process with torch, which
+// brings its own runtime; the struct above has 208, and 256 were added).  One plain product: 3.9 -> 3.1 us of host time; whole
+// passes that wait for the host: 128x4096x1024 12.3 -> 11.3 us, 128x3328x488 9.5 -> 9.0, 128x2432x320 12.6 -> 12.1.  (The launch's
+// size out of the dispatch packet instead of an argument: the packet lies in host memory, 9 us more on every kernel.)
+// What the kernel can derive is derived there, what only one epilogue needs shares its place, and the fields that the first
+// operand load needs stand in front: they come with one load.
+struct TileArgs {
+    const uint16_t *A;
+    const uint16_t *B;
+    int M, N, K;            // K is also the row stride of both operands
+    int grid_m, grid_n;
+    int stride;             // workgroups of the launch
+    fo_div by_panel, by_rows, by_last_rows;  // divisors of the raster walk: tiles of a panel, its rows, the last panel's (general: panel, first, count)
+    uint32_t bits;
+    uint16_t *C;
+    const int32_t *RA;
+    union {
+        uint16_t *ACC;      // MODE_ACC, MODE_RS
+        int32_t *MM;        // the epilogues that count
+    };
+    const int32_t *cseg;
+    const int32_t *RE;
+    union {
+        uint16_t *OWN;      // MODE_RS, whose rLDN is 1
+        int rLDN;
+    };
+    int G;
+
+    // bits
+    static constexpr uint32_t GENERAL = 1;  // another walk than the divisors', or numbers too large for them or for the bits below
+    static constexpr uint32_t SUB_M = 2, SUB_N = 4;  // general: positions cut in two along M, N
+    static constexpr int REMAP = 3;                  // two bits: xcd_remap
+    static constexpr uint32_t TALL = 32, WIDE = 64;  // reorder tiles of 256 rows, columns (else 128)
+    static constexpr uint32_t MONITOR = 128, QUIET = 256;
+    static constexpr int RANKS = 9, RANK = 13;       // MODE_RS: four bits, log2 of W; eight bits, rank
+    static constexpr int PANEL = 21;                 // eight bits, not general: panel
+
+    static TileArgs of(const GemmArgs &a, int workgroups, int mode) {
+        const long positions = (long)a.grid_m * a.grid_n;
+        const bool general = a.xcd_remap == 2 || a.sub_m * a.sub_n > 1 || a.count != positions || positions > kMaxDivide || a.panel > 255;
+        TileArgs t = {};
+        t.A = a.A; t.B = a.B; t.C = a.C;
+        t.M = a.M; t.N = a.N; t.K = a.K;
+        t.grid_m = a.grid_m; t.grid_n = a.grid_n; t.stride = workgroups;
+        if (general) {
+            t.by_panel.mul = (uint32_t)a.panel;
+            t.by_rows.mul = (uint32_t)a.first;
+            t.by_last_rows.mul = (uint32_t)a.count;
+        } else {
+            t.by_panel = fo_divisor((long)a.panel * a.grid_n);
+            t.by_rows = fo_divisor(a.panel);
+            t.by_last_rows = fo_divisor(a.panel > 0 ? a.grid_m % a.panel : 1);
+        }
+        t.RA = a.RA; t.RE = a.RE; t.cseg = a.cseg; t.G = a.G;
+        if (mode == MODE_ACC || mode == MODE_RS)
+            t.ACC = a.ACC;
+        else
+            t.MM = a.MM;
+        if (mode == MODE_RS)
+            t.OWN = a.OWN;
+        else
+            t.rLDN = a.rLDN;
+        int log_w = 0;
+        while (1 << log_w < a.W) log_w++;
+        t.bits = (general ? GENERAL : 0) | (a.sub_m > 1 ? SUB_M : 0) | (a.sub_n > 1 ? SUB_N : 0) | (uint32_t)a.xcd_remap << REMAP |
+                 (a.BM == 256 ? TALL : 0) | (a.BN == 256 ? WIDE : 0) | (a.monitor ? MONITOR : 0) | (a.quiet ? QUIET : 0) |
+                 (uint32_t)log_w << RANKS | (uint32_t)a.rank << RANK | (general ? 0 : (uint32_t)a.panel << PANEL);
+        return t;
+    }
+};
+static_assert(sizeof(TileArgs) == 112, "a launch costs more from here on");
+
+// Tiles of a launch.
+__host__ __device__ inline __attribute__((always_inline)) int fo_tile_count(const TileArgs &p) {
+    return p.bits & TileArgs::GENERAL ? (int)p.by_last_rows.mul : p.grid_m * p.grid_n;
 }
+
 
 // Tile of unit u of a launch: what fo_unit_to_tile gives, without its divisions where the host could prepare them.  (A
 // division is some thirty instructions, and in front of a kernel's first load those are fetched from memory as well.)
-__host__ __device__ inline __attribute__((always_inline)) void fo_tile_of(const GemmArgs &p, int u, int *pm, int *pn) {
-    if (__builtin_expect(p.general, 0)) {
-        int sub_m = p.sub_m, sub_n = p.sub_n, grid_m = p.grid_m, grid_n = p.grid_n, panel = p.panel;
+__host__ __device__ inline __attribute__((always_inline)) void fo_tile_of(const TileArgs &p, int u, int *pm, int *pn) {
+    const int remap = p.bits >> TileArgs::REMAP & 3;
+    if (__builtin_expect(p.bits & TileArgs::GENERAL, 0)) {
+        int sub_m = p.bits & TileArgs::SUB_M ? 2 : 1, sub_n = p.bits & TileArgs::SUB_N ? 2 : 1;
+        int grid_m = p.grid_m, grid_n = p.grid_n, panel = (int)p.by_panel.mul;
 #ifdef __HIP_DEVICE_COMPILE__
         asm volatile("" : "+s"(sub_m), "+s"(sub_n), "+s"(grid_m), "+s"(grid_n), "+s"(panel));  // its divisions stay in here
 #endif
-        fo_unit_to_tile(u, p.first, sub_m, sub_n, grid_m, grid_n, panel, p.xcd_remap, pm, pn);
+        fo_unit_to_tile(u, (int)p.by_rows.mul, sub_m, sub_n, grid_m, grid_n, panel, remap, pm, pn);
         return;
     }
-    const int t = p.first + u, nt = p.grid_m * p.grid_n, x = t & 7, rem = nt & 7;
-    const int v = p.xcd_remap ? x * (nt >> 3) + (x < rem ? x : rem) + (t >> 3) : t;
-    const int q = fo_divide(v, p.by_panel), first_m = q * p.panel, in = v - first_m * p.grid_n;
-    const bool last = p.grid_m - first_m < p.panel;
+    const int nt = p.grid_m * p.grid_n, x = u & 7, rem = nt & 7, panel = p.bits >> TileArgs::PANEL & 255;
+    const int v = remap ? x * (nt >> 3) + (x < rem ? x : rem) + (u >> 3) : u;
+    const int q = fo_divide(v, p.by_panel), first_m = q * panel, in = v - first_m * p.grid_n;
+    const bool last = p.grid_m - first_m < panel;
     fo_div by;
     by.mul = last ? p.by_last_rows.mul : p.by_rows.mul;
-    const int rows = last ? p.grid_m - first_m : p.panel, col = fo_divide(in, by);
+    const int rows = last ? p.grid_m - first_m : panel, col = fo_divide(in, by);
     *pm = first_m + in - col * rows;
     *pn = col;
 }

@@ -23,11 +23,12 @@ inline std::atomic<int> &gemm_cu_limit() {
 // One compiled shape of the kernel template.  The launch is persistent: as many
 // workgroups as the device keeps resident at once (or fewer, if the problem has
 // fewer macro tiles); each walks the raster with that stride.
+// ARGS, MODE: the kernel's arguments, made from `a` for that epilogue.
 // With `resident_out` set nothing is launched: the call only reports how many workgroups the
 // launch would hold, in resident_out[1..3] the kernel's registers per lane, LDS bytes and
 // threads per workgroup, and in resident_out[4] how many workgroups stay resident at most.
 // expect_resident > 0: refuse (FO_ERR_STATE) unless that many stay resident.
-template <auto KERN, int SMEM, int THREADS>
+template <typename ARGS, int MODE, auto KERN, int SMEM, int THREADS>
 inline int launch_kernel(const GemmArgs &a, hipStream_t stream, int *resident_out, int expect_resident) {
     auto kern = KERN;
     constexpr int smem = SMEM;
@@ -73,9 +74,7 @@ inline int launch_kernel(const GemmArgs &a, hipStream_t stream, int *resident_ou
         return FO_OK;
     }
     dim3 grid(ntiles < resident ? ntiles : resident), block(threads);
-    GemmArgs args = a;
-    fo_set_divisors(args);
-    hipLaunchKernelGGL(kern, grid, block, smem, stream, args);
+    hipLaunchKernelGGL(kern, grid, block, smem, stream, ARGS::of(a, (int)grid.x, MODE));
     FO_LAUNCH_CHECK();
     return FO_OK;
 }

@@ -25,7 +25,7 @@ int FO_CAT3(fo_gemm_tile_launch_, FO_INST_DTYPE, _, FO_INST_MODE)(const GemmArgs
 #define FO_TILE(TM_, TN_, BK_, S_) FO_TILE_(TM_, TN_, BK_, S_, false)
 #define FO_TILE_(TM_, TN_, BK_, S_, SHIFT_)                                                                                       \
     if (tm == TM_ && tn == TN_)                                                                                          \
-        return launch_kernel<fo_gemm_tile_kernel<inst_tag, TM_, TN_, BK_, S_, FO_INST_MODE, SHIFT_>,                     \
+        return launch_kernel<TileArgs, FO_INST_MODE, fo_gemm_tile_kernel<inst_tag, TM_, TN_, BK_, S_, FO_INST_MODE, SHIFT_>,                     \
                              tile_smem_bytes<TM_, TN_, BK_, S_>(), kTileThreads>(a, stream, resident_out, expect_resident);
     // Operand rows that do not begin on 128-byte lines: the form that loads whole lines, for the tiles whose stages leave
     // LDS for one more in flight beside the two a step then reads.

@@ -126,7 +126,7 @@ struct tile_step {
 };
 
 template <typename Tag, int TM, int TN, int BK, int S, int MODE, bool SHIFT>
-__global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs args) {
+__global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(TileArgs args) {
     typedef fo_elem<Tag> E;
     typedef fo_mfma16<Tag> X;
     typedef typename X::frag frag;
@@ -162,15 +162,17 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
     const int wm = wave >> 1, wn = wave & 1;
     const int KT = (args.K + BK - 1) / BK;
 
+    const int count = fo_tile_count(args);
+
     // The first tile from position `tile` on.  (One cut from a 256x256 position may lie beyond the matrix.)
     int tile = blockIdx.x, pm = 0, pn = 0;
     auto settle = [&]() __attribute__((always_inline)) {
-        while (tile < args.count) {
+        while (tile < count) {
             fo_tile_of(args, tile, &pm, &pn);
             pm = __builtin_amdgcn_readfirstlane(pm);
             pn = __builtin_amdgcn_readfirstlane(pn);
-            if (__builtin_expect(!args.general, 1) || (pm * TM < args.M && pn * TN < args.N)) break;
-            tile += gridDim.x;
+            if (__builtin_expect(!(args.bits & TileArgs::GENERAL), 1) || (pm * TM < args.M && pn * TN < args.N)) break;
+            tile += args.stride;
         }
     };
     // A loader's part of the tile: load u of a 64-column block brings rows (u * NL + wave) * 8 + lane / 8 of an operand, 128
@@ -181,7 +183,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
     fo_srd_t ra = {}, rb = {};
     int a_chunk = 0, b_chunk = 0;
     unsigned lane_row = 0, wave_lds = 0;
-    const unsigned row_step = (unsigned)(NL * 8 * args.lda * 2);
+    const unsigned row_step = (unsigned)(NL * 8 * args.K * 2);
     // With twelve loads a stage the row offsets no longer fit the scalar registers.
     auto load = [&](fo_srd_t srd, unsigned voff, unsigned row_off, unsigned col_off, unsigned lds_addr) __attribute__((always_inline)) {
         if constexpr (P >= 12)
@@ -215,38 +217,42 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
         asm volatile("" : "+v"(lane));
         const int m0 = pm * TM + TM > args.M ? args.M - TM : pm * TM, n0 = pn * TN + TN > args.N ? args.N - TN : pn * TN;  // as below
         const int lrow = lane >> 3, lkey = ((wave * 8 + lrow) >> 1) & 7;
-        const uint16_t *a0 = args.A + (size_t)m0 * args.lda, *b0 = args.B + (size_t)n0 * args.ldb;
-        const int a_shift = SHIFT ? row_shift(a0, args.lda, lrow) : 0, b_shift = SHIFT ? row_shift(b0, args.ldb, lrow) : 0;
+        const uint16_t *a0 = args.A + (size_t)m0 * args.K, *b0 = args.B + (size_t)n0 * args.K;
+        const int a_shift = SHIFT ? row_shift(a0, args.K, lrow) : 0, b_shift = SHIFT ? row_shift(b0, args.K, lrow) : 0;
         a_chunk = SHIFT ? ((((lane & 7) ^ lkey) + a_shift) & 7) - a_shift : (lane & 7) ^ lkey;
         b_chunk = SHIFT ? ((((lane & 7) ^ lkey) + b_shift) & 7) - b_shift : (lane & 7) ^ lkey;
         constexpr int LEAD = SHIFT ? 128 : 0;  // the range starts a line early: no lane's offset is negative
-        lane_row = (unsigned)((wave * 8 + lrow) * args.lda * 2 + LEAD);
-        ra = fo_make_srd(a0 - LEAD / 2, (unsigned)TM * args.lda * 2 + LEAD);
-        rb = fo_make_srd(b0 - LEAD / 2, (unsigned)TN * args.ldb * 2 + LEAD);
+        lane_row = (unsigned)((wave * 8 + lrow) * args.K * 2 + LEAD);
+        ra = fo_make_srd(a0 - LEAD / 2, (unsigned)TM * args.K * 2 + LEAD);
+        rb = fo_make_srd(b0 - LEAD / 2, (unsigned)TN * args.K * 2 + LEAD);
         wave_lds = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024);
         asm volatile("" : "+s"(wave_lds));  // the loads' LDS addresses are sums made where they are used
         __builtin_amdgcn_s_setprio(3);
 #pragma unroll
         for (int s = 0; s < S - 1; s++) request(s, s * STAGE);
     };
-    asm volatile("" : : "s"(args.A), "s"(args.B), "s"(args.count), "s"(args.general));  // all of them with the first round trip
+    asm volatile("" : : "s"(args.A), "s"(args.B), "s"(args.bits));  // all of them with the first round trip
     settle();
-    if (loader && tile < args.count) begin();
+    if (loader && tile < count) begin();
 
     // The arguments that are not needed before this point are read from here on, not at the kernel's entry.
-    typedef const __attribute__((address_space(4))) GemmArgs *args_t;
+    typedef const __attribute__((address_space(4))) TileArgs *args_t;
     args_t rest = (args_t)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(rest));
-    const __attribute__((address_space(4))) GemmArgs &p = *rest;
+    const __attribute__((address_space(4))) TileArgs &p = *rest;
 
-    const int bm_shift = p.BM == 256 ? 8 : 7, bn_shift = p.BN == 256 ? 8 : 7;  // reorder tiles: 128 or 256 each way
+    const uint32_t bits = p.bits;
+    const int bm_shift = bits & TileArgs::TALL ? 8 : 7, bn_shift = bits & TileArgs::WIDE ? 8 : 7;  // reorder tiles: 128 or 256 each way
+    const int RTN = p.N >> bn_shift;  // reorder tiles along N
+    const int log_ranks = bits >> TileArgs::RANKS & 15, ranks = 1 << log_ranks;  // MODE_RS
     const bool reorder = MODE == MODE_ACC ? p.RA != nullptr : MODE != MODE_PLAIN;
-    const int ldp = reorder ? p.rLDN * p.BN : p.N;  // leading dimension of the output view
-    const bool signalling = COUNTS && !p.quiet;
+    const int rLDN = MODE == MODE_RS ? 1 : p.rLDN;
+    const int ldp = reorder ? rLDN << bn_shift : p.N;  // leading dimension of the output view
+    const bool signalling = COUNTS && !(bits & TileArgs::QUIET);
     typedef const __attribute__((address_space(4))) int32_t *cptr_t;  // read-only for the whole launch: scalar loads
     const cptr_t RAc = (cptr_t)(uintptr_t)p.RA;
 
-    while (tile < args.count) {
+    while (tile < count) {
         // What is computed from the lane is computed for each tile: kept from one to the next, the group search's and the
         // loaders' part of it alone took twenty registers through the K loop.
         int lane = tid & 63;
@@ -266,25 +272,25 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             two_n = (n0 + TN - 1) >> bn_shift != tn0;
             if (two_m) split_m = ((tm0 + 1) << bm_shift) - m0;
             if (two_n) split_n = ((tn0 + 1) << bn_shift) - n0;
-            r0 = RAc[tm0 * p.TN + tn0];
-            r1 = two_m || two_n ? RAc[(tm0 + two_m) * p.TN + tn0 + two_n] : r0;
+            r0 = RAc[tm0 * RTN + tn0];
+            r1 = two_m || two_n ? RAc[(tm0 + two_m) * RTN + tn0 + two_n] : r0;
         }
         int g0 = 0, g1 = 0;  // groups of r0 and r1 (the wavefront that signals)
         // Row and column of the output view at which the tile's row and column 0 are, or would be, in r0 and in r1.
         int row0 = m0, row1 = m0, col0 = n0, col1 = n0;
         auto find_bases = [&]() __attribute__((always_inline)) {
             if (!reorder) return;
-            int rldn = p.rLDN;
+            int rldn = rLDN;
             asm volatile("" : "+s"(rldn));  // the divisions by it are done here, not in front of the K loop
             int q0 = r0, q1 = r1;
             if (rldn != 1) {
                 q0 /= rldn;
                 q1 /= rldn;
             }
-            row0 = (q0 << bm_shift) + (m0 & (p.BM - 1));
-            row1 = (q1 << bm_shift) + (two_m ? -split_m : m0 & (p.BM - 1));
-            col0 = (r0 - q0 * rldn << bn_shift) + (n0 & (p.BN - 1));
-            col1 = (r1 - q1 * rldn << bn_shift) + (two_n ? -split_n : n0 & (p.BN - 1));
+            row0 = (q0 << bm_shift) + (m0 & ((1 << bm_shift) - 1));
+            row1 = (q1 << bm_shift) + (two_m ? -split_m : m0 & ((1 << bm_shift) - 1));
+            col0 = (r0 - q0 * rldn << bn_shift) + (n0 & ((1 << bn_shift) - 1));
+            col1 = (r1 - q1 * rldn << bn_shift) + (two_n ? -split_n : n0 & ((1 << bn_shift) - 1));
         };
         // The tile in pieces of 16 bytes: act(u, row, column, address in the view `out`) for thread t's piece u, those
         // to be stored or (EVERY) all of them.  A tile that lies in one reorder tile and is stored whole needs one address
@@ -412,7 +418,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                     each_mapped_piece(wave * 64 + lane, rs_map, p.OWN, std::false_type{},
                                       [&](int, int row, int col, uint16_t *at) __attribute__((always_inline)) {
                         store16_write_through(at, piece(row, col));
-                    }, p.rank * p.seg_rows, p.seg_rows);
+                    }, (int)(bits >> TileArgs::RANK & 255) * ((p.M >> log_ranks) * RTN), (p.M >> log_ranks) * RTN);
                 }
             }
         } else {
@@ -443,7 +449,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             // in the following block from 8 on (all rows of a lane have the same shift: they are 16 apart).
             int l_shift = 0, s_shift = 0;
             if (SHIFT) {
-                const int a_shift = row_shift(p.A + (size_t)m0 * p.lda, p.lda, frow), b_shift = row_shift(p.B + (size_t)n0 * p.ldb, p.ldb, frow);
+                const int a_shift = row_shift(p.A + (size_t)m0 * p.K, p.K, frow), b_shift = row_shift(p.B + (size_t)n0 * p.K, p.K, frow);
                 l_shift = fk + (LONG_B ? b_shift : a_shift);
                 s_shift = fk + (LONG_B ? a_shift : b_shift);
             }
@@ -553,7 +559,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             if (MAPPED) {
                 const int row = two_n && e >= TM ? e - TM : e, r = second_e ? r1 : r0;
                 if (e < (two_n ? 2 * TM : TM))
-                    entry = p.RE[(r / p.rLDN << bm_shift) + (second_e && two_m ? -split_m : m0 & (p.BM - 1)) + row];
+                    entry = p.RE[(r / rLDN << bm_shift) + (second_e && two_m ? -split_m : m0 & ((1 << bm_shift) - 1)) + row];
                 if (MODE == MODE_RS && lane < p.G) size0 = p.cseg[lane];
             }
             auto write_maps = [&]() __attribute__((always_inline)) {
@@ -567,7 +573,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                 if (e < (two_n ? 2 * TM : TM)) {
                     row_map[e] = entry;
                     if (MODE == MODE_RS)
-                        rs_map[e] = rs_row(p.cseg, p.G, p.BM, p.W, p.seg_rows, entry, (second_e ? first1 : first0) << bm_shift,
+                        rs_map[e] = rs_row(p.cseg, p.G, 1 << bm_shift, ranks, (p.M >> log_ranks) * RTN, entry, (second_e ? first1 : first0) << bm_shift,
                                            (second_e ? count1 : count0) << bm_shift);
                 }
                 asm volatile("" ::: "memory");
@@ -605,6 +611,10 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
                     slot = next;
                 }
             }
+            // To the compiler these two loads may still be on their way behind the loop (it does not know that one of its steps, or the
+            // call in front of it, has used them), and where it takes their registers for something else in the epilogue it waits, with
+            // every piece, for the stores of the one before: 2048x4096x2048 over eight ranks 32.5 us or 35.4, by the registers it chose.
+            if (MAPPED) asm volatile("" : "+v"(entry), "+v"(size0));
             __builtin_amdgcn_s_waitcnt(0xC07F);
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
@@ -659,15 +669,15 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(GemmArgs 
             if (wave_id == NL && ((lane == 0 && first_counts) || (lane == 1 && (two_m || two_n)))) {
                 const int g = lane ? g1 : g0, r = lane ? r1 : r0;
                 __hip_atomic_fetch_add(p.MM + g, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (p.monitor) {
-                    int o = __hip_atomic_fetch_add(p.MM + (p.TN - 1), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_store(p.MM + p.TN + r, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (bits & TileArgs::MONITOR) {
+                    int o = __hip_atomic_fetch_add(p.MM + (RTN - 1), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(p.MM + RTN + r, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
             }
         }
-        tile += gridDim.x;
+        tile += args.stride;
         settle();
-        if (tile < args.count) {
+        if (tile < count) {
             __syncthreads();  // the staged tile has been read by everyone
             if (loader) begin();
         }
