@@ -74,36 +74,41 @@ struct launch_plan {
 // whatever the monitor watches: its stamps say in which order the launch completed its tiles.
 constexpr int kSignalAfterFromK = 1536;
 
-// What one round of a tile takes, all CUs busy: microseconds at K = 4096, with operand rows on 128-byte lines and off them
-// (the tiles up to 128x192 then load whole lines, the larger ones cannot; 128x192 only without a row map, for which its four
-// stages leave no LDS).  Ratios at K = 1024 are the same.  With its line loads (54 -> 46 a round) one round of 128x192 takes the
-// place of two of 96x128 or of one of 128x256; GEMM alone, us: 1152x5120x1720 bf16 23.4 -> 21.0, with an accumulator 26.5 ->
-// 23.7, 1536x3840x2040 26.7 -> 24.8, 1152x5120x4088 48.5 -> 46.4.
+// What launches without counters of more than one round of 128x160 tiles take, microseconds.  Each round, all CUs busy, has a share
+// that goes with K (given at K = 4096: operand rows on 128-byte lines, off them, and off them with a row map, which leaves
+// 128x192 no LDS for its line loads; 128x256 and 256x256 have none) and an end that does not: a tile's stores, which nothing of the
+// next one runs beside, dearer by a row map, and an accumulator's values and sums.  Fitted to whole passes, GEMM and
+// normalisation, of 2220 products (plain, with an accumulator, over four ranks with and without one; K = 256 to 8192), each in
+// all tiles, three states in turn: the pass in the tile of least estimate is 0.65 % longer than in the best one, in the mean;
+// with estimates in proportion to K, an end for short sums only and the Algo's tile in the second launch it was 1.7 % (one in seven
+// is more than 3 % faster now, one in thirty more than 3 % slower; 5376x3584x1096 bf16 90.1 -> 76.5 us, 2432x7424x664 62.5 -> 57.6).
 struct tile_cost {
-    int tm, tn, on_lines, off_lines, mapped;
-    double sums;
+    int tm, tn;
+    double on_lines, off_lines, mapped;  // at K = 4096
+    double end, end_mapped, sums, sums_mapped;
 };
-constexpr tile_cost kTileCosts[] = {{96, 128, 26, 27, 27, 2.2},  {128, 128, 31, 33, 33, 2.3}, {128, 160, 36, 38, 38, 4.4},
-                                    {128, 192, 42, 46, 54, 4.4}, {128, 256, 57, 71, 71, 5},   {256, 128, 57, 71, 71, 5},
-                                    {256, 256, 97, 110, 110, 11}};
-// `sums`: what an accumulator adds to a round, microseconds at any K: its values and sums go to and from memory when the round's
-// tiles are done, with little of the next round's product beside them, and a large tile has more of it to wait for.  Over 219
-// products of more than one round with a cold accumulator and 256 to 640 columns of K the chosen tile was 5.0 % slower than the best
-// one without this term and 1.3 % with it (GEMM alone, us: 6784x3712x312 bf16 54.2 -> 42.7, 128x160 -> 128x128, 6400x3200x400 48.7 ->
-// 39.9, 5120x3456x280 39.3 -> 32.9, 7680x2688x424 50.9 -> 43.8); beyond 640 columns it gains in some and loses in others (241
-// products: 1.1 % without, 1.0 % with it).  Not for a row map, whose sums cost otherwise (3456x4352x328 over eight ranks 32.0
-// us for the whole pass, 41.4 in the tile that it would take).
-constexpr int kSumsBelowK = 640;
-// Beginning and end of a round of 128x192 with its line loads, beyond the other tiles' (us): with few columns of K two rounds
-// of it are no better than three of 128x128 (with an accumulator, us, 2304x5120x264 20.2 and 18.5, 2048x6144x264 20.7 and 19.8,
-// 2048x6144x776 40.7 and 42.8).
-constexpr double kWide192Ends = 0.5;
+constexpr tile_cost kTileCosts[] = {
+    {96, 128, 25.3, 25.5, 25, 1.7, 3.0, 1.3, 1.9},    {128, 128, 30.5, 31.5, 30.5, 1.7, 3.4, 2.0, 2.4},
+    {128, 160, 35.2, 37, 36.5, 2.2, 4.2, 3.0, 3.4},   {128, 192, 40.5, 41.5, 52, 2.8, 4.1, 3.1, 3.7},
+    {128, 256, 52, 65.5, 64.5, 2.8, 5.1, 3.7, 5.1},   {256, 128, 52, 65.5, 64.5, 2.8, 5.1, 3.7, 5.1},
+    {256, 256, 88.5, 104.5, 101.5, 5.2, 10.5, 8.7, 9.9}};
+constexpr double kLastRound = 0.6;
+// A last round of 256x256 tiles that is at most half full may go to a second launch: its start and end behind the first one's,
+// its share of K and an accumulator's sums, for each tile that it may have; fitted to the same passes.  (With rem * 16 tiles of 64x64 on
+// a chip that is otherwise idle instead of rem * 2 of 128x256: 2944x6144x3848 over four ranks 166 -> 133 us, 7168x4736x7928 616 -> 519,
+// 3072x6400x4936 with an accumulator 251 -> 214.)
+struct tail_cost {
+    int tm, tn;
+    double start, at_4096, sums;
+};
+constexpr tail_cost kTailCosts[] = {{64, 64, 5.3, 18.2, 1.1}, {64, 128, 4.9, 24.5, 2.2}, {128, 128, 4.7, 38.5, 4.6}, {128, 256, 5.5, 66, 7.8}};
+constexpr double kTailLastRound = 0.5;
 
-// Estimate for `count` tiles: whole rounds, and a last one that costs 60 % of a round plus its share of the CUs (fewer
-// active CUs share the L2s, HBM and the power limit).
-double rounds_cost(long count, long cus, double round) {
+// Rounds of `count` tiles: a last one that is not full costs a part of a round and its share of the CUs (fewer active CUs
+// share the L2s, HBM and the power limit).
+double rounds(long count, long cus, double last) {
     const long full = count / cus, rest = count % cus;
-    return round * (full + (rest ? 0.6 + 0.4 * rest / cus : 0.0));
+    return full + (rest ? last + (1 - last) * rest / cus : 0.0);
 }
 
 // What fits the chip in one round, one tile per CU, takes the smallest tile that does: a smaller tile moves
@@ -137,14 +142,6 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN,
         p.count = p.grid_m * p.grid_n;
         p.xcd_remap = p.count >= 16 ? 1 : 0;
     };
-    // The tile of the second launch: 128x128 while one round of them does it, else 128x256 or 256x128.
-    auto set_tail = [&](int positions, long cus) {
-        p.tail = positions;
-        p.count -= positions;
-        p.tail_tm = BM;
-        p.tail_tn = BN;
-        if (BM == 128 && BN == 128 && positions * 4 > cus && N % 256 == 0) p.tail_tn = 256;
-    };
     const bool square = r.mtm == 256 && r.mtn == 256;  // what fo_schedule_order assumes
     const long cus = fo_main_tile_resident();
     auto tiles = [&](int tm, int tn) { return (long)((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
@@ -166,29 +163,37 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN,
         return p;
     }
     const long nt = tiles(256, 256);
-    const int rem = square ? r.tail_tiles : nt > cus && nt % cus * 2 <= cus ? (int)(nt % cus) : 0;
     if (!counted) {
-        const bool sums = acc && !mapped && K < kSumsBelowK;
+        const int rem = nt > cus && nt % cus * 2 <= cus ? (int)(nt % cus) : 0;  // what a second launch may take
+        const double k = K / 4096.0;
         const tile_cost *best = nullptr;
+        const tail_cost *best_tail = nullptr;
         double least = 0;
         for (const tile_cost &t : kTileCosts) {
             if (M < t.tm || N < t.tn) continue;
-            double round = on_lines ? t.on_lines : mapped ? t.mapped : t.off_lines;
-            if (sums)
-                round += t.sums * 4096 / K;
-            else if (!on_lines && !mapped && t.tn == 192)
-                round += kWide192Ends * 4096 / K;
-            const bool split = t.tm == 256 && t.tn == 256 && rem;  // the last positions go to a second launch
-            const double second = rem * 4 <= cus ? 33 : 60, second_sums = rem * 4 <= cus ? 2.3 : 5;  // 128x128 or 128x256 tiles
-            const double cost = split ? rounds_cost(nt - rem, cus, round) + second + (sums ? second_sums * 4096 / K : 0)
-                                      : rounds_cost(tiles(t.tm, t.tn), cus, round);
-            if (best && cost >= least) continue;
-            best = &t;
-            least = cost;
+            const double round = k * (on_lines ? t.on_lines : mapped ? t.mapped : t.off_lines) + (mapped ? t.end_mapped : t.end) +
+                                 (!acc ? 0 : mapped ? t.sums_mapped : t.sums);
+            auto offer = [&](double cost, const tail_cost *tail) {
+                if (best && cost >= least) return;
+                best = &t;
+                best_tail = tail;
+                least = cost;
+            };
+            offer(round * rounds(tiles(t.tm, t.tn), cus, kLastRound), nullptr);
+            if (t.tm != 256 || t.tn != 256 || !rem) continue;
+            for (const tail_cost &u : kTailCosts)
+                offer(round * rounds(nt - rem, cus, kLastRound) + u.start +
+                          (k * u.at_4096 + (acc ? u.sums : 0)) * rounds((long)rem * (256 / u.tm) * (256 / u.tn), cus, kTailLastRound),
+                      &u);
         }
         set_shared(best->tm, best->tn);  // the 96x128 tile at least: M and N are multiples of 128
         if (p.tm == 256 && p.tn == 256) {
-            if (rem) set_tail(rem, cus);
+            if (best_tail) {
+                p.tail = rem;
+                p.count -= rem;
+                p.tail_tm = best_tail->tm;
+                p.tail_tn = best_tail->tn;
+            }
             if (square) {
                 p.panel = r.panel;
                 p.xcd_remap = r.xcd_remap;
@@ -199,7 +204,14 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN,
     set(r.mtm, r.mtn);
     p.panel = r.panel;
     p.xcd_remap = r.xcd_remap;
-    if (r.tail_tiles) set_tail(r.tail_tiles, r.resident);
+    if (r.tail_tiles) {
+        // 128x128 while one round of them does it, else 128x256 or 256x128
+        p.tail = r.tail_tiles;
+        p.count -= r.tail_tiles;
+        p.tail_tm = BM;
+        p.tail_tn = BN;
+        if (BM == 128 && BN == 128 && r.tail_tiles * 4 > r.resident && N % 256 == 0) p.tail_tn = 256;
+    }
     return p;
 }
 

@@ -114,12 +114,12 @@ struct TileArgs {
 
     // bits
     static constexpr uint32_t GENERAL = 1;  // another walk than the divisors', or numbers too large for them or for the bits below
-    static constexpr uint32_t SUB_M = 2, SUB_N = 4;  // general: positions cut in two along M, N
-    static constexpr int REMAP = 3;                  // two bits: xcd_remap
-    static constexpr uint32_t TALL = 32, WIDE = 64;  // reorder tiles of 256 rows, columns (else 128)
-    static constexpr uint32_t MONITOR = 128, QUIET = 256;
-    static constexpr int RANKS = 9, RANK = 13;       // MODE_RS: four bits, log2 of W; eight bits, rank
-    static constexpr int PANEL = 21;                 // eight bits, not general: panel
+    static constexpr uint32_t TALL = 2, WIDE = 4;    // reorder tiles of 256 rows, columns (else 128)
+    static constexpr uint32_t MONITOR = 8, QUIET = 16;
+    static constexpr int REMAP = 5;                  // two bits: xcd_remap
+    static constexpr int SUB_M = 7, SUB_N = 9;       // two bits each, general: log2 of the tiles a position is cut into along M, N
+    static constexpr int RANKS = 11, RANK = 15;      // MODE_RS: four bits, log2 of W; eight bits, rank
+    static constexpr int PANEL = 23;                 // eight bits, not general: panel
 
     static TileArgs of(const GemmArgs &a, int workgroups, int mode) {
         const long positions = (long)a.grid_m * a.grid_n;
@@ -146,11 +146,10 @@ struct TileArgs {
             t.OWN = a.OWN;
         else
             t.rLDN = a.rLDN;
-        int log_w = 0;
-        while (1 << log_w < a.W) log_w++;
-        t.bits = (general ? GENERAL : 0) | (a.sub_m > 1 ? SUB_M : 0) | (a.sub_n > 1 ? SUB_N : 0) | (uint32_t)a.xcd_remap << REMAP |
+        auto log2 = [](int n) { return (uint32_t)__builtin_ctz((unsigned)n); };  // W, sub_m and sub_n are powers of two
+        t.bits = (general ? GENERAL : 0) | log2(a.sub_m) << SUB_M | log2(a.sub_n) << SUB_N | (uint32_t)a.xcd_remap << REMAP |
                  (a.BM == 256 ? TALL : 0) | (a.BN == 256 ? WIDE : 0) | (a.monitor ? MONITOR : 0) | (a.quiet ? QUIET : 0) |
-                 (uint32_t)log_w << RANKS | (uint32_t)a.rank << RANK | (general ? 0 : (uint32_t)a.panel << PANEL);
+                 log2(a.W) << RANKS | (uint32_t)a.rank << RANK | (general ? 0 : (uint32_t)a.panel << PANEL);
         return t;
     }
 };
@@ -167,7 +166,7 @@ __host__ __device__ inline __attribute__((always_inline)) int fo_tile_count(cons
 __host__ __device__ inline __attribute__((always_inline)) void fo_tile_of(const TileArgs &p, int u, int *pm, int *pn) {
     const int remap = p.bits >> TileArgs::REMAP & 3;
     if (__builtin_expect(p.bits & TileArgs::GENERAL, 0)) {
-        int sub_m = p.bits & TileArgs::SUB_M ? 2 : 1, sub_n = p.bits & TileArgs::SUB_N ? 2 : 1;
+        int sub_m = 1 << (p.bits >> TileArgs::SUB_M & 3), sub_n = 1 << (p.bits >> TileArgs::SUB_N & 3);
         int grid_m = p.grid_m, grid_n = p.grid_n, panel = (int)p.by_panel.mul;
 #ifdef __HIP_DEVICE_COMPILE__
         asm volatile("" : "+s"(sub_m), "+s"(sub_n), "+s"(grid_m), "+s"(grid_n), "+s"(panel));  // its divisions stay in here

@@ -51,7 +51,7 @@ int main() {
                         a.grid_m = g[0]; a.grid_n = g[1]; a.panel = panel; a.xcd_remap = remap;
                         const int positions = g[0] * g[1];
                         a.first = part ? positions / 3 : 0;
-                        a.sub_m = part & 1 ? 2 : 1; a.sub_n = part & 2 ? 2 : 1;
+                        a.sub_m = part & 1 ? 2 << (panel & 1) : 1; a.sub_n = part & 2 ? 4 >> remap : 1;
                         a.count = (positions - a.first) * a.sub_m * a.sub_n;
                         a.BM = part & 2 ? 256 : 128; a.BN = part & 1 ? 256 : 128;
                         a.M = a.grid_m * 256; a.N = a.grid_n * 256; a.K = 8 * panel; a.rLDN = 1 + part; a.G = 5 + part;
