@@ -150,6 +150,12 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN,
     auto set_shared = [&](int tm, int tn) {
         set(tm, tn);
         p.panel = p.grid_m < 8 ? p.grid_m : 8;
+        // One or two rows left over would be a panel whose XCDs share one operand hardly at all (a block of 32 tiles reads 12
+        // panels of operand rows as 8 x 4, 18 as 2 x 16, 33 as 1 x 32): panels of about one height instead.  Whole passes, us:
+        // 1152x5120x1720 (9 rows of 128x192) 27.4 -> 26.4, 640x1024x4408 (10 of 64x64) 18.3 -> 17.7, 4224x7168x3584 (17 of 256x256)
+        // 176.6 -> 172.4.  With three and more rows left over eight stay: 1408x3328x1240 (11) 19.6 -> 19.9, 1792x3584x3936 (14) 60 -> 65.
+        const int panels = (p.grid_m + 7) / 8, left = p.grid_m % 8;
+        if (panels > 1 && (left == 1 || left == 2)) p.panel = (p.grid_m + panels - 1) / panels;
     };
     static const int shapes[][2] = {{32, 32},  {64, 32},   {64, 64},   {64, 96},   {64, 128}, {96, 128},
                                     {128, 128}, {128, 160}, {128, 192}, {128, 256}, {256, 128}};
