@@ -369,14 +369,27 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(TileArgs 
             if (ACC && sums) {
                 fo_u32x4 old[ACC ? NCH : 1];  // the accumulator's values
                 // every wavefront loads every piece, needed or not: the waits below count
-                auto take = [&](int u, int, int, uint16_t *at) __attribute__((always_inline)) {
-                    old[ACC ? u : 0] = *reinterpret_cast<const fo_u32x4 *>(at);
-                };
                 find_bases();
-                if constexpr (MODE == MODE_RS)
-                    each_mapped_piece(wave * 64 + lane, rs_map, p.ACC, std::true_type{}, take);
-                else
-                    each_piece(wave * 64 + lane, p.ACC, std::true_type{}, take);
+                if constexpr (MODE == MODE_RS) {
+                    each_mapped_piece(wave * 64 + lane, rs_map, p.ACC, std::true_type{},
+                                      [&](int u, int, int, uint16_t *at) __attribute__((always_inline)) {
+                        old[ACC ? u : 0] = *reinterpret_cast<const fo_u32x4 *>(at);
+                    });
+                } else {
+                    // The addresses first, the loads behind the point where the ways to them meet: with loads on both ways the compiler,
+                    // which takes the second for a way that may follow the first, waited there for the registers of the first,
+                    // and with them for every operand stage in flight (whole passes, us: 896x3968x4088 by the serial call 33.2 -> 32.2,
+                    // 512x4096x1000 13.3 -> 12.8, 7680x2560x368 in 300 groups 52.6 -> 52.1; the others up to 0.7 %).
+                    typedef const __attribute__((address_space(1))) fo_u32x4 *global_t;
+                    global_t from[ACC ? NCH : 1];
+                    each_piece(wave * 64 + lane, p.ACC, std::true_type{}, [&](int u, int, int, uint16_t *at) __attribute__((always_inline)) {
+                        from[ACC ? u : 0] = (global_t)(uintptr_t)at;
+                    });
+#pragma unroll
+                    for (int u = 0; u < (ACC ? NCH : 1); u++) asm volatile("" : "+v"(from[u]));
+#pragma unroll
+                    for (int u = 0; u < (ACC ? NCH : 1); u++) old[u] = *from[u];
+                }
                 asm volatile("" ::: "memory");
 #pragma unroll
                 for (int j = 0; j < S - 1; j++) {
