@@ -399,9 +399,9 @@ __device__ __forceinline__ float wave_sum(float v) {
 enum { NORM_PLAIN = 0, NORM_SLOTS = 1, NORM_GENERAL = 2 };
 
 template <typename Tag, int MAXCH, bool STREAM, int PATH>
-__global__ __launch_bounds__(256, MAXCH <= 16 ? 4 : 2) void fo_rmsnorm_kernel(const fo_u32x4 *X, fo_u32x4 *Y, const fo_u32x4 *Wt,
+__global__ __launch_bounds__(256, MAXCH <= 16 ? 4 : 2) void fo_rmsnorm_kernel(const int32_t *RA, const fo_u32x4 *X, const fo_u32x4 *Wt,
                                                          int bs, int dim, int BM, int BN, int rldn,
-                                                         const int32_t *RA, float eps) {
+                                                         fo_u32x4 *Y, float eps) {
     typedef norm_math<Tag> MATH;
     // The weight goes through LDS, fetched once per workgroup ahead of the rows: a weight
     // load from memory between two stores of the output row would make its wait (vmcnt
@@ -514,13 +514,13 @@ int launch_rmsnorm_on(const void *X, void *Y, const void *Wt, int bs, int dim, i
     fo_u32x4 *y = static_cast<fo_u32x4 *>(Y);
     const fo_u32x4 *w = static_cast<const fo_u32x4 *>(Wt);
     if (nch <= 64 * 4)
-        hipLaunchKernelGGL((fo_rmsnorm_kernel<Tag, 4, STREAM, PATH>), grid, block, 0, stream, x, y, w, bs, dim, BM, BN, rldn, RA, eps);
+        hipLaunchKernelGGL((fo_rmsnorm_kernel<Tag, 4, STREAM, PATH>), grid, block, 0, stream, RA, x, w, bs, dim, BM, BN, rldn, y, eps);
     else if (nch <= 64 * 8)
-        hipLaunchKernelGGL((fo_rmsnorm_kernel<Tag, 8, STREAM, PATH>), grid, block, 0, stream, x, y, w, bs, dim, BM, BN, rldn, RA, eps);
+        hipLaunchKernelGGL((fo_rmsnorm_kernel<Tag, 8, STREAM, PATH>), grid, block, 0, stream, RA, x, w, bs, dim, BM, BN, rldn, y, eps);
     else if (nch <= 64 * 16)
-        hipLaunchKernelGGL((fo_rmsnorm_kernel<Tag, 16, STREAM, PATH>), grid, block, 0, stream, x, y, w, bs, dim, BM, BN, rldn, RA, eps);
+        hipLaunchKernelGGL((fo_rmsnorm_kernel<Tag, 16, STREAM, PATH>), grid, block, 0, stream, RA, x, w, bs, dim, BM, BN, rldn, y, eps);
     else if (nch <= 64 * 32)
-        hipLaunchKernelGGL((fo_rmsnorm_kernel<Tag, 32, STREAM, PATH>), grid, block, 0, stream, x, y, w, bs, dim, BM, BN, rldn, RA, eps);
+        hipLaunchKernelGGL((fo_rmsnorm_kernel<Tag, 32, STREAM, PATH>), grid, block, 0, stream, RA, x, w, bs, dim, BM, BN, rldn, y, eps);
     else
         return FO_ERR_SHAPE;  // rows above 16384 elements (the reference's limit too)
     FO_LAUNCH_CHECK();
@@ -586,10 +586,22 @@ int launch_rmsnorm(const void *X, void *Y, const void *Wt, int bs, int dim, int 
 // is read once for both (ACC is laid out as X).  The accumulator's chunks are requested when the row before is done with and
 // used last; up to 128 registers, which fit beside the signalling GEMM's wavefront (384).
 template <typename Tag, int CH, bool STREAM, int PATH, bool ADD>
-__global__ __launch_bounds__(256, !ADD && CH <= 4 ? 5 : 4) void fo_norm_rows_kernel(const fo_u32x4 *X, fo_u32x4 *Y, const fo_u32x4 *Wt,
-                                                              int row0, int nrows, int rows_per_wg, int dim, int BM,
-                                                              int BN, int rldn, const int32_t *RA, float eps,
-                                                              unsigned x_bytes, fo_u32x4 *ACC) {
+__global__ __launch_bounds__(256, !ADD && CH <= 4 ? 5 : 4) void fo_norm_rows_kernel(uint64_t RA_, uint64_t X_, uint64_t Wt_, uint64_t row0_nrows,
+                                                              uint64_t rows_per_wg_dim, uint64_t BM_BN, uint64_t x_bytes_rldn,
+                                                              uint64_t Y_, uint64_t ACC_, float eps) {
+    // What the first loads need stands in front, fourteen words, which arrive in scalar registers with the wavefront.  (Words instead
+    // of pointers, and two integers in one: a launch takes the host longer by some 20 ns for each argument that is a pointer.)
+    typedef const __attribute__((address_space(1))) int32_t *table_t;
+    typedef const __attribute__((address_space(1))) fo_u32x4 *chunks_t;
+    const table_t RA = (table_t)RA_;
+    const chunks_t Wt = (chunks_t)Wt_;
+    const fo_u32x4 *X = (const fo_u32x4 *)X_;
+    fo_u32x4 *Y = (fo_u32x4 *)Y_, *ACC = (fo_u32x4 *)ACC_;
+    const int row0 = (int)row0_nrows, nrows = (int)(row0_nrows >> 32);
+    const int rows_per_wg = (int)rows_per_wg_dim, dim = (int)(rows_per_wg_dim >> 32);
+    const int BM = (int)BM_BN, BN = (int)(BM_BN >> 32);
+    const unsigned x_bytes = (unsigned)x_bytes_rldn;
+    const int rldn = (int)(x_bytes_rldn >> 32);
     typedef norm_math<Tag> MATH;
     __shared__ float part[2][4];
     // every argument with one wait, in front of the branch below
@@ -788,9 +800,8 @@ int launch_norm_rows_on(const void *X, void *Y, const void *Wt, int row0, int nr
     const int rows_per_wg = (nrows + grid - 1) / grid;
     grid = (nrows + rows_per_wg - 1) / rows_per_wg;
     const int lds = beside_gemm ? kBesideGemmLds : 0;
-    const fo_u32x4 *x = static_cast<const fo_u32x4 *>(X);
-    fo_u32x4 *y = static_cast<fo_u32x4 *>(Y);
-    const fo_u32x4 *w = static_cast<const fo_u32x4 *>(Wt);
+    auto word = [](const void *p) { return (uint64_t)(uintptr_t)p; };
+    auto both = [](uint32_t low, uint32_t high) { return (uint64_t)high << 32 | low; };
     // info != null: nothing is launched; info = {registers per lane, LDS bytes per workgroup} of the kernel that would run
 #define FO_NORM_ROWS(CH_)                                                                                               \
     if (info) {                                                                                                         \
@@ -800,8 +811,8 @@ int launch_norm_rows_on(const void *X, void *Y, const void *Wt, int row0, int nr
         info[1] = (int)attr.sharedSizeBytes + lds;                                                                      \
         return FO_OK;                                                                                                   \
     }                                                                                                                   \
-    hipLaunchKernelGGL((fo_norm_rows_kernel<Tag, CH_, STREAM, PATH, ADD>), dim3(grid), dim3(256), lds, stream, x, y, w, row0, \
-                       nrows, rows_per_wg, dim, BM, BN, rldn, RA, eps, x_bytes, static_cast<fo_u32x4 *>(acc))
+    hipLaunchKernelGGL((fo_norm_rows_kernel<Tag, CH_, STREAM, PATH, ADD>), dim3(grid), dim3(256), lds, stream, word(RA), word(X), word(Wt), both(row0, nrows), \
+                       both(rows_per_wg, dim), both(BM, BN), both(x_bytes, rldn), word(Y), word(acc), eps)
     if (nch <= 256) {
         FO_NORM_ROWS(1);
     } else if (nch <= 512) {

@@ -14,6 +14,8 @@
 // accumulator registers per instruction, half of their traffic per flop), and large products are power-limited.
 #pragma once
 
+#include <cstddef>
+#include <cstring>
 #include <type_traits>
 #include <utility>
 
@@ -154,6 +156,12 @@ struct TileArgs {
     }
 };
 static_assert(sizeof(TileArgs) == 112, "a launch costs more from here on");
+// The kernel takes the fields in front of C as seven words of 64 bits, which arrive in registers with the wavefront, and the rest as
+// they are.  (Words, not pointers: with pointers and integers one by one, thirteen arguments, a launch was as dear as with 208 bytes.)
+struct TileRest {
+    uint64_t words[7];
+};
+static_assert(offsetof(TileArgs, C) == 56 && sizeof(TileRest) == sizeof(TileArgs) - 56, "the fields in front, and the rest");
 
 // Tiles of a launch.
 __host__ __device__ inline __attribute__((always_inline)) int fo_tile_count(const TileArgs &p) {

@@ -20,6 +20,19 @@ inline std::atomic<int> &gemm_cu_limit() {
     return limit;
 }
 
+template <typename KERN>
+inline void launch_with(KERN kern, dim3 grid, dim3 block, int smem, hipStream_t stream, const GemmArgs &a) {
+    hipLaunchKernelGGL(kern, grid, block, smem, stream, a);
+}
+template <typename KERN>
+inline void launch_with(KERN kern, dim3 grid, dim3 block, int smem, hipStream_t stream, const TileArgs &t) {
+    TileRest rest;
+    memcpy(&rest, reinterpret_cast<const char *>(&t) + offsetof(TileArgs, C), sizeof rest);
+    auto both = [](uint32_t low, uint32_t high) { return (uint64_t)high << 32 | low; };
+    hipLaunchKernelGGL(kern, grid, block, smem, stream, (uint64_t)(uintptr_t)t.A, (uint64_t)(uintptr_t)t.B, both(t.M, t.N), both(t.K, t.grid_m), both(t.grid_n, t.stride),
+                       both(t.by_panel.mul, t.by_rows.mul), both(t.by_last_rows.mul, t.bits), rest);
+}
+
 // One compiled shape of the kernel template.  The launch is persistent: as many
 // workgroups as the device keeps resident at once (or fewer, if the problem has
 // fewer macro tiles); each walks the raster with that stride.
@@ -74,7 +87,7 @@ inline int launch_kernel(const GemmArgs &a, hipStream_t stream, int *resident_ou
         return FO_OK;
     }
     dim3 grid(ntiles < resident ? ntiles : resident), block(threads);
-    hipLaunchKernelGGL(kern, grid, block, smem, stream, ARGS::of(a, (int)grid.x, MODE));
+    launch_with(kern, grid, block, smem, stream, ARGS::of(a, (int)grid.x, MODE));
     FO_LAUNCH_CHECK();
     return FO_OK;
 }

@@ -126,7 +126,23 @@ struct tile_step {
 };
 
 template <typename Tag, int TM, int TN, int BK, int S, int MODE, bool SHIFT>
-__global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(TileArgs args) {
+__global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(uint64_t A, uint64_t B, uint64_t M_N,
+                                                                          uint64_t K_grid_m, uint64_t grid_n_stride,
+                                                                          uint64_t by_panel_rows, uint64_t by_last_bits, TileRest) {
+    // The fields of TileArgs that the first operand load needs.
+    TileArgs args;
+    args.A = (const uint16_t *)(uintptr_t)A;
+    args.B = (const uint16_t *)(uintptr_t)B;
+    args.M = (int)M_N;
+    args.N = (int)(M_N >> 32);
+    args.K = (int)K_grid_m;
+    args.grid_m = (int)(K_grid_m >> 32);
+    args.grid_n = (int)grid_n_stride;
+    args.stride = (int)(grid_n_stride >> 32);
+    args.by_panel.mul = (uint32_t)by_panel_rows;
+    args.by_rows.mul = (uint32_t)(by_panel_rows >> 32);
+    args.by_last_rows.mul = (uint32_t)by_last_bits;
+    args.bits = (uint32_t)(by_last_bits >> 32);
     typedef fo_elem<Tag> E;
     typedef fo_mfma16<Tag> X;
     typedef typename X::frag frag;
