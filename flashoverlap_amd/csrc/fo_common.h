@@ -219,9 +219,9 @@ int fo_pace_with(double seconds, fo_stream_t stream);  // a one-lane kernel that
 __host__ __device__ inline int fo_pack_row_waves(int log_bh, int log_bw, int log_xc, int resident) {
     return log_bh | log_bw << 4 | log_xc << 8 | resident << 12;
 }
-__host__ __device__ inline __attribute__((always_inline)) void fo_row_wave_tile(int t, int packed, int *pm, int *pn) {
+__host__ __device__ inline __attribute__((always_inline)) void fo_row_wave_tile(int t, int k, int packed, int *pm, int *pn) {  // k: t / R
     const int log_bh = packed & 15, log_bw = (packed >> 4) & 15, log_xc = (packed >> 8) & 15, R = packed >> 12;
-    const int k = t / R, w = t - k * R;
+    const int w = t - k * R;
     const int x = w & 7, j = w >> 3;
     const int rows_per_wave = (8 >> log_xc) << log_bh;
     *pm = k * rows_per_wave + ((x >> log_xc) << log_bh) + (j & ((1 << log_bh) - 1));
@@ -232,7 +232,7 @@ __host__ __device__ inline __attribute__((always_inline)) void fo_row_wave_tile(
 __host__ __device__ inline __attribute__((always_inline)) void fo_wg_to_tile(int wg, int grid_m, int grid_n, int panel,
                                               int xcd_remap, int *pm, int *pn) {
     if (xcd_remap == 2) {
-        fo_row_wave_tile(wg, panel, pm, pn);
+        fo_row_wave_tile(wg, wg / (panel >> 12), panel, pm, pn);
         return;
     }
     int nt = grid_m * grid_n;

@@ -144,7 +144,20 @@ constexpr int kTakeFromSteps256 = 5;  // K steps of a tile from which on they ar
 constexpr int kSmem256 = 2 * 65536 + 4 * 16 * (128 + 8) * 2;  // two slots + four strips of 16 padded rows
 
 template <typename Tag, int MODE>
-__global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
+__global__ __launch_bounds__(256) void fo_gemm256_kernel(uint64_t A_, uint64_t B_, uint64_t K_count, uint64_t grid_m_n, uint64_t panel_bits,
+                                                         uint64_t by_panel_rows, uint64_t by_last_rows, GemmArgs) {
+    Front256 f;
+    f.A = (const uint16_t *)(uintptr_t)A_;
+    f.B = (const uint16_t *)(uintptr_t)B_;
+    f.K = (int)K_count;
+    f.count = (int)(K_count >> 32);
+    f.grid_m = (int)grid_m_n;
+    f.grid_n = (int)(grid_m_n >> 32);
+    f.panel = (int)panel_bits;
+    f.bits = (uint32_t)(panel_bits >> 32);
+    f.by_panel.mul = (uint32_t)by_panel_rows;
+    f.by_rows.mul = (uint32_t)(by_panel_rows >> 32);
+    f.by_last_rows.mul = (uint32_t)by_last_rows;
     typedef fo_elem<Tag> E;
     typedef fo_mfma256<Tag> X;
     constexpr bool SUMS = MODE == MODE_SIGNAL_SUM || MODE == MODE_SCATTER_SUM;
@@ -182,9 +195,9 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
-    const int ntiles = p.count;
-    const int KT = (p.K + BK - 1) / BK;
-    const bool ktail = (p.K % BK) != 0;
+    const int ntiles = f.count;
+    const int KT = (f.K + BK - 1) / BK;
+    const bool ktail = (f.K % BK) != 0;
 
     // Fragment addressing as in fo_gemm_tile_kernel.h: lane l supplies row l & 15, k-chunk l >> 4 of a 16x32 block.
     const int frow = lane & 15, fk = lane >> 4;
@@ -198,31 +211,31 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     // phys ^ key(row).
     const int lrow = lane >> 3;
     const int lchunk = (lane & 7) ^ (((wave * 8 + lrow) >> 1) & 7);
-    const unsigned a_off = (unsigned)((wave * 8 + lrow) * p.lda * 2 + lchunk * 16);
-    const bool tail_out = (KT - 1) * BK + lchunk * 8 >= p.K;  // this lane's chunk of the last K step lies beyond K
+    const unsigned a_off = (unsigned)((wave * 8 + lrow) * f.K * 2 + lchunk * 16);
+    const bool tail_out = (KT - 1) * BK + lchunk * 8 >= f.K;  // this lane's chunk of the last K step lies beyond K
     const unsigned a_off_t = tail_out ? 0x80000000u : a_off;  // beyond every descriptor's range
     // The descriptors point at the stage's first column of the tile's first row and cover exactly the
     // tile's rows from there (the host checks that this fits 31 bits).
-    const unsigned a_span = (unsigned)((255 * p.lda + p.K) * 2);
+    const unsigned a_span = (unsigned)((255 * f.K + f.K) * 2);
     // A and B have one leading dimension (the launcher checks it), so the lane offsets, the span and the
     // row-block offsets of the eight loads per operand serve both.
     unsigned soff_a[8];
 #pragma unroll
     for (int c = 0; c < 8; c++) {
-        soff_a[c] = __builtin_amdgcn_readfirstlane((unsigned)(c * 32 * p.lda * 2));
+        soff_a[c] = __builtin_amdgcn_readfirstlane((unsigned)(c * 32 * f.K * 2));
     }
 
     // M and N are multiples of 128, not of 256: where half a tile is left at the end of a dimension, the tile is moved
     // back by half its size, so that all of its operand rows exist; its first half there repeats the neighbour's
-    // product and is not stored (p.half: bit 0 along M, bit 1 along N; never in a launch that counts, see plan_launch).
-    int half = p.half;
+    // product and is not stored (half: bit 0 along M, bit 1 along N; never in a launch that counts, see plan_launch).
+    int half = f.bits >> 3;
     asm volatile("" : "+s"(half));  // in a register from here on: loaded again inside the K loop, it would turn every wait for LDS data into a wait for everything
     // Coordinates of raster position t in halves of tiles, bits 0 and 1 of *repeated: which halves another tile
     // computes (the upper rows, the left columns).
     auto locate = [&](int t, int *pm_, int *pn_, int *repeated_) {
         int qm, qn;
-        fo_wg_to_tile(t, p.grid_m, p.grid_n, p.panel, p.xcd_remap, &qm, &qn);
-        const int rep = __builtin_amdgcn_readfirstlane(half & ((qm == p.grid_m - 1 ? 1 : 0) | (qn == p.grid_n - 1 ? 2 : 0)));
+        fo_tile_of(f, t, &qm, &qn);
+        const int rep = __builtin_amdgcn_readfirstlane(half & ((qm == f.grid_m - 1 ? 1 : 0) | (qn == f.grid_n - 1 ? 2 : 0)));
         *pm_ = __builtin_amdgcn_readfirstlane(2 * qm - (rep & 1));
         *pn_ = __builtin_amdgcn_readfirstlane(2 * qn - (rep >> 1));
         *repeated_ = rep;
@@ -235,8 +248,8 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     unsigned a_cur = (ktail && KT == 1) ? a_off_t : a_off;  // this stage's lane offsets, A and B alike
     fo_srd_t ra, rb;
     auto point_loader = [&](int pm_, int pn_) {
-        ra = fo_make_srd(p.A + (size_t)pm_ * 128 * p.lda, a_span);
-        rb = fo_make_srd(p.B + (size_t)pn_ * 128 * p.lda, a_span);
+        ra = fo_make_srd(f.A + (size_t)pm_ * 128 * f.K, a_span);
+        rb = fo_make_srd(f.B + (size_t)pn_ * 128 * f.K, a_span);
     };
     auto set_loader_tile = [&]() {
         if (ld_tile < ntiles) {
@@ -244,8 +257,8 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             locate(ld_tile, &pm_, &pn_, &rep_);
             point_loader(pm_, pn_);
         } else {
-            ra = fo_make_srd(p.A, 0);  // behind the last tile: every load is out of range, nothing is fetched
-            rb = fo_make_srd(p.B, 0);
+            ra = fo_make_srd(f.A, 0);  // behind the last tile: every load is out of range, nothing is fetched
+            rb = fo_make_srd(f.B, 0);
         }
     };
     auto advance_loader = [&]() {
@@ -282,8 +295,22 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
         X::template go_load<c * CHUNK_B>(x, y, cc, lds_base, c < 8 ? ra : rb, a_cur, soff_a[c & 7]);
     };
 
+    // ---- the first stage, in front of all that its addresses do not need.  A workgroup takes one or two tiles of a product that
+    // fits the chip, so what stands in front of its first load counts: the arguments in memory, the slot table and the raster's
+    // divisions were 513 instructions and 21 scalar loads and waits there in the signal epilogue, these are 172 and 4 (Front256
+    // arrives in registers, its divisors come from the host).  Whole passes:
+    // 4096x4096x512 with its normalisation 41.1 -> 40.2 us, 4096x4096x1024 with an accumulator 52.5 -> 51.5, over eight ranks 45.8 -> 44.4.
+    point_loader(pm, pn);
+#pragma unroll
+    for (int c = 0; c < 16; c++) load_chunk(c, 0);
+    typedef const __attribute__((address_space(4))) char *args_t;
+    args_t rest = (args_t)__builtin_amdgcn_kernarg_segment_ptr() + 7 * 8;
+    asm volatile("" : "+s"(rest));  // the other arguments are read from here on
+    const __attribute__((address_space(4))) GemmArgs &p = *(const __attribute__((address_space(4))) GemmArgs *)rest;
+
     // ---- signalling state (signal and scatter epilogues)
-    const int sub_n = MT / p.BN, nsub = (MT / p.BM) * sub_n;  // reorder tiles per macro tile
+    const int bm_shift = p.BM == 256 ? 8 : 7, bn_shift = p.BN == 256 ? 8 : 7;
+    const int log_sub_n = 8 - bn_shift, sub_n = 1 << log_sub_n, nsub = sub_n << (8 - bm_shift);  // reorder tiles per macro tile
     typedef const __attribute__((address_space(4))) int32_t *cptr_t;
     const cptr_t RAc = (cptr_t)(uintptr_t)p.RA;
     constexpr int NPRE = kPrefixRegs / 64;
@@ -294,7 +321,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
     const bool signalling = COUNTS && !p.quiet;
     const bool reorder = MODE == MODE_ACC ? p.RA != nullptr : COUNTS || MODE == MODE_RS || MODE == MODE_REORDER;
     const bool groups = signalling || TO_RANKS;  // group sizes are needed
-    // The group sizes are requested in front of the pipeline fill and summed behind it (a round trip to memory and
+    // The group sizes are requested between the pipeline fill's two stages and summed behind it (a round trip to memory and
     // some two dozen dependent cross-lane steps otherwise stand between the kernel's start and its first operand
     // load).  The requests are assembly: their registers are read only behind the fill's wait for loads that were
     // requested after them, and the compiler, which knows nothing of the fill's loads, would otherwise wait for
@@ -379,8 +406,8 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             }
         }
     };
-    // Storage slots of a macro tile's reorder tiles (scalar loads).  They are requested one tile ahead (in front of
-    // the pipeline fill for the first tile, in front of the previous tile's epilogue otherwise) and awaited at the
+    // Storage slots of a macro tile's reorder tiles (scalar loads).  They are requested one tile ahead (behind
+    // the pipeline fill's loads for the first tile, in front of the previous tile's epilogue otherwise) and awaited at the
     // tile's start: the round trip to memory then costs nothing, and no scalar load is pending at the K loop's head,
     // where it would turn every wait for LDS data into a wait for everything (scalar loads return out of order).
     int rs_next[kMaxSub] = {0, 0, 0, 0};
@@ -389,12 +416,12 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
             const int tm_ = pm_ >> (p.BM >> 8), tn_ = pn_ >> (p.BN >> 8);  // in reorder tiles (BM, BN: 128 or 256)
 #pragma unroll
             for (int s = 0; s < kMaxSub; s++)
-                if (s < nsub) rs_next[s] = RAc[(tm_ + s / sub_n) * p.TN + tn_ + s % sub_n];
+                if (s < nsub) rs_next[s] = RAc[(tm_ + (s >> log_sub_n)) * p.TN + tn_ + (s & (sub_n - 1))];
         }
     };
     // The slots that request_slots brought, as the rest of the kernel uses them: this wavefront's own reorder tile as a
     // scalar, all of them in lanes 0 .. nsub-1 of one register.
-    const int my_sub = __builtin_amdgcn_readfirstlane(((wm * 128) / p.BM) * sub_n + (wn * 128) / p.BN);
+    const int my_sub = __builtin_amdgcn_readfirstlane(((wm * 128 >> bm_shift) << log_sub_n) + (wn * 128 >> bn_shift));
     int r_mine = 0, v_rs = 0;
     auto take_slots = [&]() {
         if (reorder) {
@@ -419,14 +446,11 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
         bf[kk][j] = *reinterpret_cast<lds16_t>(base + j * BLOCK_B);
     };
 
-    // ---- pipeline fill: stage 0 -> slot 0, stage 1 -> slot 1; the loader then stands at stage 1
-    request_slots(pm, pn);
-    point_loader(pm, pn);
-#pragma unroll
-    for (int c = 0; c < 16; c++) load_chunk(c, 0);
+    // ---- pipeline fill: stage 0 -> slot 0 (above), stage 1 -> slot 1; the loader then stands at stage 1
     advance_loader();
 #pragma unroll
     for (int c = 0; c < 16; c++) load_chunk(c, SLOT_B);
+    request_slots(pm, pn);
     wait_vmcnt<16>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -474,7 +498,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(GemmArgs p) {
         // 4096x4096x512 44.0 -> 41.6, 4096x4096x1024 55.9 -> 52.2, 4096x8192x264 85.7 -> 77.1, 3456x4352x3072 100.2 -> 97.3,
         // 8064x8064x4096 463.8 -> 455.7; 8192x8192x2048 by the serial call 276.5 -> 272.4).
         fo_u32x4 old[ACC ? NST : 1];
-        // Not where rows are so long that the block's offsets leave a 31-bit range (p.half, bit 2).
+        // Not where rows are so long that the block's offsets leave a 31-bit range (half, bit 2).
         const bool early = MODE == MODE_ACC && KT >= kTakeFromSteps256 && !(half & 4);
         int take_row = 0, take_step = 0;
         unsigned take_lane = 0;

@@ -58,7 +58,22 @@ __host__ __device__ inline __attribute__((always_inline)) int fo_divide(int n, f
 constexpr long kMaxDivide = 32767;
 inline fo_div fo_divisor(long d) { return {d > 0 ? (uint32_t)(((1ULL << 31) + d - 1) / d) : 0}; }
 
-// A launch as the host describes it, and the 256x256 kernel's arguments.
+// Position t of the raster that fo_wg_to_tile walks (xcd_remap 0 or 1), by divisors that the host prepared.
+__host__ __device__ inline __attribute__((always_inline)) void fo_raster_tile(int t, int remap, int grid_m, int grid_n, int panel,
+                                                                              fo_div by_panel, fo_div by_rows, fo_div by_last_rows,
+                                                                              int *pm, int *pn) {
+    const int nt = grid_m * grid_n, x = t & 7, rem = nt & 7;
+    const int v = remap ? x * (nt >> 3) + (x < rem ? x : rem) + (t >> 3) : t;
+    const int q = fo_divide(v, by_panel), first_m = q * panel, in = v - first_m * grid_n;
+    const bool last = grid_m - first_m < panel;
+    fo_div by;
+    by.mul = last ? by_last_rows.mul : by_rows.mul;
+    const int rows = last ? grid_m - first_m : panel, col = fo_divide(in, by);
+    *pm = first_m + in - col * rows;
+    *pn = col;
+}
+
+// A launch as the host describes it, and, behind those words that its first load needs, the 256x256 kernel's arguments.
 struct GemmArgs {
     const uint16_t *A;
     const uint16_t *B;
@@ -182,15 +197,49 @@ __host__ __device__ inline __attribute__((always_inline)) void fo_tile_of(const 
         fo_unit_to_tile(u, (int)p.by_rows.mul, sub_m, sub_n, grid_m, grid_n, panel, remap, pm, pn);
         return;
     }
-    const int nt = p.grid_m * p.grid_n, x = u & 7, rem = nt & 7, panel = p.bits >> TileArgs::PANEL & 255;
-    const int v = remap ? x * (nt >> 3) + (x < rem ? x : rem) + (u >> 3) : u;
-    const int q = fo_divide(v, p.by_panel), first_m = q * panel, in = v - first_m * p.grid_n;
-    const bool last = p.grid_m - first_m < panel;
-    fo_div by;
-    by.mul = last ? p.by_last_rows.mul : p.by_rows.mul;
-    const int rows = last ? p.grid_m - first_m : panel, col = fo_divide(in, by);
-    *pm = first_m + in - col * rows;
-    *pn = col;
+    fo_raster_tile(u, remap, p.grid_m, p.grid_n, p.bits >> TileArgs::PANEL & 255, p.by_panel, p.by_rows, p.by_last_rows, pm, pn);
+}
+
+// What the first operand load of the 256x256 kernel needs, as words of 64 bits that arrive in registers with the wavefront, low half
+// first: A, B, K and count, grid_m and grid_n, panel and bits, the divisors of the raster walk.
+struct Front256 {
+    const uint16_t *A, *B;
+    int K, count, grid_m, grid_n, panel;
+    fo_div by_panel, by_rows, by_last_rows;  // tiles of a panel (waves of whole tile rows: workgroups of a wave), its rows, the last panel's
+    uint32_t bits;                           // 1: numbers too large for the divisors; from bit 1: xcd_remap, two bits; from bit 3: half
+
+    static Front256 of(const GemmArgs &a) {
+        Front256 f = {};
+        const bool waves = a.xcd_remap == 2;
+        f.A = a.A; f.B = a.B; f.K = a.K; f.count = a.count;
+        f.grid_m = a.grid_m; f.grid_n = a.grid_n; f.panel = a.panel;
+        const bool general = (long)a.grid_m * a.grid_n > kMaxDivide || (!waves && a.panel <= 0);
+        if (!general) {
+            f.by_panel = fo_divisor(waves ? a.panel >> 12 : (long)a.panel * a.grid_n);
+            f.by_rows = fo_divisor(waves ? 1 : a.panel);
+            f.by_last_rows = fo_divisor(waves ? 1 : a.grid_m % a.panel);
+        }
+        f.bits = (general ? 1 : 0) | (uint32_t)a.xcd_remap << 1 | (uint32_t)a.half << 3;
+        return f;
+    }
+};
+
+// Raster position t of such a launch: what fo_wg_to_tile gives.
+__host__ __device__ inline __attribute__((always_inline)) void fo_tile_of(const Front256 &f, int t, int *pm, int *pn) {
+    const int remap = f.bits >> 1 & 3;
+    if (__builtin_expect(f.bits & 1, 0)) {
+        int grid_m = f.grid_m, grid_n = f.grid_n, panel = f.panel;
+#ifdef __HIP_DEVICE_COMPILE__
+        asm volatile("" : "+s"(grid_m), "+s"(grid_n), "+s"(panel));  // its divisions stay in here
+#endif
+        fo_wg_to_tile(t, grid_m, grid_n, panel, remap, pm, pn);
+        return;
+    }
+    if (remap == 2) {
+        fo_row_wave_tile(t, fo_divide(t, f.by_panel), f.panel, pm, pn);
+        return;
+    }
+    fo_raster_tile(t, remap, f.grid_m, f.grid_n, f.panel, f.by_panel, f.by_rows, f.by_last_rows, pm, pn);
 }
 
 // Every operand row begins on a 128-byte line.

@@ -20,16 +20,19 @@ inline std::atomic<int> &gemm_cu_limit() {
     return limit;
 }
 
+inline uint64_t word(const void *p) { return (uint64_t)(uintptr_t)p; }
+inline uint64_t both(uint32_t low, uint32_t high) { return (uint64_t)high << 32 | low; }
 template <typename KERN>
 inline void launch_with(KERN kern, dim3 grid, dim3 block, int smem, hipStream_t stream, const GemmArgs &a) {
-    hipLaunchKernelGGL(kern, grid, block, smem, stream, a);
+    const Front256 f = Front256::of(a);
+    hipLaunchKernelGGL(kern, grid, block, smem, stream, word(f.A), word(f.B), both(f.K, f.count), both(f.grid_m, f.grid_n),
+                       both(f.panel, f.bits), both(f.by_panel.mul, f.by_rows.mul), (uint64_t)f.by_last_rows.mul, a);
 }
 template <typename KERN>
 inline void launch_with(KERN kern, dim3 grid, dim3 block, int smem, hipStream_t stream, const TileArgs &t) {
     TileRest rest;
     memcpy(&rest, reinterpret_cast<const char *>(&t) + offsetof(TileArgs, C), sizeof rest);
-    auto both = [](uint32_t low, uint32_t high) { return (uint64_t)high << 32 | low; };
-    hipLaunchKernelGGL(kern, grid, block, smem, stream, (uint64_t)(uintptr_t)t.A, (uint64_t)(uintptr_t)t.B, both(t.M, t.N), both(t.K, t.grid_m), both(t.grid_n, t.stride),
+    hipLaunchKernelGGL(kern, grid, block, smem, stream, word(t.A), word(t.B), both(t.M, t.N), both(t.K, t.grid_m), both(t.grid_n, t.stride),
                        both(t.by_panel.mul, t.by_rows.mul), both(t.by_last_rows.mul, t.bits), rest);
 }
 

@@ -1,5 +1,5 @@
-"""The smaller tiles' launch arguments: what the host packs into 112 bytes, and the raster walk that reads them, against the
-launch as it is described (host code of the library's own header, built for the CPU)."""
+"""The launch arguments: what the host packs into the smaller tiles' 112 bytes and into the words in front of the 256x256
+tile's, and the raster walks that read them, against the launch as it is described (host code of the library's own header, built for the CPU)."""
 import subprocess
 
 import pytest
@@ -33,6 +33,17 @@ static void compare(const GemmArgs &a, int mode) {
         fo_unit_to_tile(u, a.first, a.sub_m, a.sub_n, a.grid_m, a.grid_n, a.panel, a.xcd_remap, &pm, &pn);
         bad += m != pm || n != pn;
         walked += !general;
+    }
+    GemmArgs h = a;
+    h.half = (mode & 3) | (a.quiet ? 4 : 0);
+    const Front256 f = Front256::of(h);
+    bad += f.A != a.A || f.B != a.B || f.K != a.K || f.count != a.count || (int)(f.bits >> 3) != h.half;
+    const int positions = a.grid_m * a.grid_n;
+    for (int u = 0; u < positions; u += positions > 3000 ? positions / 1500 : 1) {
+        int m, n, pm, pn;
+        fo_tile_of(f, u, &m, &n);
+        fo_wg_to_tile(u, a.grid_m, a.grid_n, a.panel, a.xcd_remap, &pm, &pn);
+        bad += m != pm || n != pn;
     }
     seen++;
 }
