@@ -1,6 +1,6 @@
 // Python extension module _fo_native: the per-call host path of ops.py and layers.py.
 //
-// The small calls of this framework are bound by the host: a kernel launch costs 2.4 us, and the checks, pointer
+// The small calls of this framework are bound by the host: a kernel launch costs 2.7 us or more, and the checks, pointer
 // objects and stream lookup of a call written in Python another 5 to 9.  Host time per call, before and with this module:
 // the two layers of a decode step (128x4096x1024, whose kernels run 8.5 us) 17.3 -> 11.1 us, the all-reduce call
 // 9.6 -> 4.0, the same with the normalisation 13.9 -> 6.8, the normalisation alone 9.3 -> 3.6.  Each function here does what its Python counterpart does
