@@ -145,7 +145,7 @@ constexpr int kSmem256 = 2 * 65536 + 4 * 16 * (128 + 8) * 2;  // two slots + fou
 
 template <typename Tag, int MODE>
 __global__ __launch_bounds__(256) void fo_gemm256_kernel(uint64_t A_, uint64_t B_, uint64_t K_count, uint64_t grid_m_n, uint64_t panel_bits,
-                                                         uint64_t by_panel_rows, uint64_t by_last_rows, GemmArgs) {
+                                                         uint64_t by_panel_rows, uint64_t by_last_stride, GemmArgs) {
     Front256 f;
     f.A = (const uint16_t *)(uintptr_t)A_;
     f.B = (const uint16_t *)(uintptr_t)B_;
@@ -157,7 +157,8 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(uint64_t A_, uint64_t B
     f.bits = (uint32_t)(panel_bits >> 32);
     f.by_panel.mul = (uint32_t)by_panel_rows;
     f.by_rows.mul = (uint32_t)(by_panel_rows >> 32);
-    f.by_last_rows.mul = (uint32_t)by_last_rows;
+    f.by_last_rows.mul = (uint32_t)by_last_stride;
+    const int stride = (int)(by_last_stride >> 32);  // workgroups of the launch
     typedef fo_elem<Tag> E;
     typedef fo_mfma256<Tag> X;
     constexpr bool SUMS = MODE == MODE_SIGNAL_SUM || MODE == MODE_SCATTER_SUM;
@@ -265,7 +266,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(uint64_t A_, uint64_t B
         ld_kt++;
         if (ld_kt == KT) {
             ld_kt = 0;
-            ld_tile += gridDim.x;
+            ld_tile += stride;
             set_loader_tile();
         } else {
             // the next K step of the same tile: 128 bytes further along the rows
@@ -307,6 +308,16 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(uint64_t A_, uint64_t B
     args_t rest = (args_t)__builtin_amdgcn_kernarg_segment_ptr() + 7 * 8;
     asm volatile("" : "+s"(rest));  // the other arguments are read from here on
     const __attribute__((address_space(4))) GemmArgs &p = *(const __attribute__((address_space(4))) GemmArgs *)rest;
+    // Those that the first tile's group sizes and slots need, in one round trip.
+    int first_BM = 0, first_BN = 0, first_TN = 0, first_G = 0;
+    const int32_t *first_RA = nullptr, *first_cseg = nullptr;
+    if (MODE != MODE_PLAIN) {
+        first_BM = p.BM; first_BN = p.BN; first_TN = p.TN; first_RA = p.RA;
+        if (COUNTS || TO_RANKS) {
+            first_G = p.G; first_cseg = p.cseg;
+        }
+        asm volatile("" : "+s"(first_BM), "+s"(first_BN), "+s"(first_TN), "+s"(first_RA), "+s"(first_G), "+s"(first_cseg));
+    }
 
     // ---- signalling state (signal and scatter epilogues)
     const int bm_shift = p.BM == 256 ? 8 : 7, bn_shift = p.BN == 256 ? 8 : 7;
@@ -330,9 +341,20 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(uint64_t A_, uint64_t B
     if (groups && reg_search) {
 #pragma unroll
         for (int q = 0; q < NPRE; q++) {
-            const int32_t *src = p.cseg + (q * 64 + lane < p.G ? q * 64 + lane : 0);
+            const int32_t *src = first_cseg + (q * 64 + lane < first_G ? q * 64 + lane : 0);
             asm volatile("global_load_dword %0, %1, off" : "=v"(cs_raw[q]) : "v"(src) : "memory");
         }
+    }
+    // The first tile's storage slots, lane s the one of its reorder tile s: one load, in the same place and manner.  As scalar loads
+    // they were four round trips, one behind the other (there are no scalar registers to hold them side by side), and the fill took
+    // 3 us, of which the operands need 1.5.  Whole passes, us: layers 4096x4096x1024 39.7 -> 39.2, over eight ranks 44.7 -> 44.0.  Lanes beyond
+    // the tile's last slot ask for that one again, without a table all of them for the first word of A.
+    int slots_raw = 0;
+    if (MODE != MODE_PLAIN) {
+        const int q = lane < nsub ? lane : nsub - 1;
+        const int at = ((pm >> (first_BM >> 8)) + (q >> log_sub_n)) * first_TN + (pn >> (first_BN >> 8)) + (q & (sub_n - 1));
+        const int32_t *src = reorder ? first_RA + at : reinterpret_cast<const int32_t *>(f.A);
+        asm volatile("global_load_dword %0, %1, off" : "=v"(slots_raw) : "v"(src) : "memory");
     }
     auto sum_groups = [&]() {
         if (groups && reg_search) {
@@ -406,9 +428,8 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(uint64_t A_, uint64_t B
             }
         }
     };
-    // Storage slots of a macro tile's reorder tiles (scalar loads).  They are requested one tile ahead (behind
-    // the pipeline fill's loads for the first tile, in front of the previous tile's epilogue otherwise) and awaited at the
-    // tile's start: the round trip to memory then costs nothing, and no scalar load is pending at the K loop's head,
+    // Storage slots of a further tile's reorder tiles (scalar loads).  They are requested one tile ahead, in front of the previous
+    // tile's epilogue, and awaited in it: the round trip to memory then costs nothing, and no scalar load is pending at the K loop's head,
     // where it would turn every wait for LDS data into a wait for everything (scalar loads return out of order).
     int rs_next[kMaxSub] = {0, 0, 0, 0};
     auto request_slots = [&](int pm_, int pn_) {
@@ -427,7 +448,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(uint64_t A_, uint64_t B
         if (reorder) {
 #pragma unroll
             for (int s = 0; s < kMaxSub; s++) {
-                int rr = rs_next[s];
+                int rr = __builtin_amdgcn_readfirstlane(rs_next[s]);
                 asm volatile("" : "+s"(rr));  // the scalar loads complete here
                 if (s == my_sub) r_mine = rr;
                 v_rs = lane == s ? rr : v_rs;
@@ -450,7 +471,6 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(uint64_t A_, uint64_t B
     advance_loader();
 #pragma unroll
     for (int c = 0; c < 16; c++) load_chunk(c, SLOT_B);
-    request_slots(pm, pn);
     wait_vmcnt<16>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -458,12 +478,16 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(uint64_t A_, uint64_t B
     for (int q = 0; q < 4; q++) load_a(0, la0 ^ (q % 2 * KSTEP_X), q / 2, q % 2);
 #pragma unroll
     for (int q = 0; q < 10; q++) load_b(lb0 ^ (q % 2 * KSTEP_X), q / 2, q % 2);
+    if (MODE != MODE_PLAIN) asm volatile("" : "+v"(slots_raw));  // has arrived with them
     sum_groups();  // the group sizes arrived before stage 0 did (requested earlier, vmcnt retires in issue order)
 
     int tile = blockIdx.x;
     unsigned slot_b = 0;  // byte offset of the slot the next K step reads
     for (;;) {
-        if (tile == (int)blockIdx.x) take_slots();  // later tiles: taken inside the previous tile's epilogue
+        if (MODE != MODE_PLAIN && reorder && tile == (int)blockIdx.x) {  // later tiles: taken inside the previous tile's epilogue
+            v_rs = slots_raw;
+            r_mine = __builtin_amdgcn_readlane(slots_raw, my_sub);
+        }
         // Scatter: the row map entries of the wavefront's 128 rows, two per lane (lane l: rows l and 64 + l), are
         // requested here and rest in two registers through the K loop; the epilogue hands them to the lanes that
         // store each row.  Requested in the epilogue they cost every tile a round trip to memory with nothing to hide it.
@@ -643,7 +667,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(uint64_t A_, uint64_t B
         }
 
         fo_mfma_fence();
-        const int next = tile + gridDim.x;
+        const int next = tile + stride;
         const bool has_next = next < ntiles;
         int next_pm = 0, next_pn = 0, next_repeated = 0;
         if (has_next) {

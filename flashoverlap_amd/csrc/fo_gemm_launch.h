@@ -26,7 +26,7 @@ template <typename KERN>
 inline void launch_with(KERN kern, dim3 grid, dim3 block, int smem, hipStream_t stream, const GemmArgs &a) {
     const Front256 f = Front256::of(a);
     hipLaunchKernelGGL(kern, grid, block, smem, stream, word(f.A), word(f.B), both(f.K, f.count), both(f.grid_m, f.grid_n),
-                       both(f.panel, f.bits), both(f.by_panel.mul, f.by_rows.mul), (uint64_t)f.by_last_rows.mul, a);
+                       both(f.panel, f.bits), both(f.by_panel.mul, f.by_rows.mul), both(f.by_last_rows.mul, grid.x), a);
 }
 template <typename KERN>
 inline void launch_with(KERN kern, dim3 grid, dim3 block, int smem, hipStream_t stream, const TileArgs &t) {
