@@ -91,7 +91,7 @@ constexpr tile_cost kTileCosts[] = {
     {96, 128, 25.3, 25.5, 25, 1.7, 3.0, 1.3, 1.9},    {128, 128, 30.5, 31.5, 30.5, 1.7, 3.4, 2.0, 2.4},
     {128, 160, 35.2, 37, 36.5, 2.2, 4.2, 3.0, 3.4},   {128, 192, 40.5, 41.5, 52, 2.8, 4.1, 3.1, 3.7},
     {128, 256, 52, 65.5, 64.5, 2.8, 5.1, 3.7, 5.1},   {256, 128, 52, 65.5, 64.5, 2.8, 5.1, 3.7, 5.1},
-    {256, 256, 88.5, 104.5, 101.5, 5.2, 10.5, 8.7, 9.9}};
+    {256, 256, 88.5, 106, 103, 5.2, 10.5, 8.7, 9.9}};
 constexpr double kLastRound = 0.6;
 // A last round of 256x256 tiles that is at most half full may go to a second launch: its start and end behind the first one's,
 // its share of K and an accumulator's sums, for each tile that it may have; fitted to the same passes.  (With rem * 16 tiles of 64x64 on
@@ -153,9 +153,10 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN,
         // One or two rows left over would be a panel whose XCDs share one operand hardly at all (a block of 32 tiles reads 12
         // panels of operand rows as 8 x 4, 18 as 2 x 16, 33 as 1 x 32): panels of about one height instead.  Whole passes, us:
         // 1152x5120x1720 (9 rows of 128x192) 27.4 -> 26.4, 640x1024x4408 (10 of 64x64) 18.3 -> 17.7, 4224x7168x3584 (17 of 256x256)
-        // 176.6 -> 172.4.  With three and more rows left over eight stay: 1408x3328x1240 (11) 19.6 -> 19.9, 1792x3584x3936 (14) 60 -> 65.
+        // 176.6 -> 172.4.  With three and more rows left over eight stay: 1408x3328x1240 (11) 19.6 -> 19.9, 1792x3584x3936 (14) 60 -> 65; and
+        // where the panel left over is a small part: 6656x6272x5088 (26 of 256x256) 381 -> 386, 6400x6528x5840 (25) 432 -> 437.
         const int panels = (p.grid_m + 7) / 8, left = p.grid_m % 8;
-        if (panels > 1 && (left == 1 || left == 2)) p.panel = (p.grid_m + panels - 1) / panels;
+        if (panels > 1 && panels < 4 && (left == 1 || left == 2)) p.panel = (p.grid_m + panels - 1) / panels;
     };
     static const int shapes[][2] = {{32, 32},  {64, 32},   {64, 64},   {64, 96},   {64, 128}, {96, 128},
                                     {128, 128}, {128, 160}, {128, 192}, {128, 256}, {256, 128}};
@@ -172,15 +173,22 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN,
     if (!counted) {
         const int rem = nt > cus && nt % cus * 2 <= cus ? (int)(nt % cus) : 0;  // what a second launch may take
         const double k = K / 4096.0;
+        // Several rounds of the 256x256 tile.  With an odd multiple of 32 as K only every other row is off the lines, otherwise most
+        // are.  Without an accumulator the halves that repeat a neighbour's multiply nothing.  Whole passes, us, in 128x192 tiles, which
+        // looked the cheaper ones without the two -> in these: 6656x6272x5088 405 -> 373, 6400x6528x5840 bf16 438 -> 424.
+        const double off_share = nt <= cus ? 0.9 : K % 64 == 32 ? 0.57 : 1.0;
+        const double area = acc || mapped ? 1.0 : (double)M * N / (nt * 65536.0);
         const tile_cost *best = nullptr;
         const tail_cost *best_tail = nullptr;
         double least = 0;
         for (const tile_cost &t : kTileCosts) {
             if (M < t.tm || N < t.tn) continue;
+            const bool largest = t.tm * t.tn == 256 * 256;
+            const double off = ((mapped ? t.mapped : t.off_lines) - t.on_lines) * (largest ? off_share : 1.0);
             // near ties of several rounds go to the 256x256 tiles, which take the least energy: 5248x7936x2496 222 us, in 128x256 232
-            const double round = (k * (on_lines ? t.on_lines : mapped ? t.mapped : t.off_lines) + (mapped ? t.end_mapped : t.end) +
+            const double round = (k * (t.on_lines + (on_lines ? 0 : off)) + (mapped ? t.end_mapped : t.end) +
                                   (!acc ? 0 : mapped ? t.sums_mapped : t.sums)) *
-                                 (nt > cus && t.tm * t.tn == 256 * 256 ? 0.985 : 1.0);
+                                 (nt > cus && largest ? 0.98 * area : 1.0);
             auto offer = [&](double cost, const tail_cost *tail) {
                 if (best && cost >= least) return;
                 best = &t;
