@@ -8,7 +8,6 @@
 
 int fo_gemm_dev::fo_gemm256_launch(int dtype, int mode, const GemmArgs &a, hipStream_t stream, int *resident_out,
                                    int expect_resident) {
-    if (a.lda != a.ldb) return FO_ERR_ARG;  // the kernel addresses both operands with one leading dimension
     const int key = (dtype == FO_BF16 ? 8 : 0) + mode;
     switch (key) {
         case 0: return fo_gemm256_launch_0_0(a, stream, resident_out, expect_resident);
@@ -290,7 +289,6 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     a.C = static_cast<uint16_t *>(C);
     a.ACC = static_cast<uint16_t *>(acc);
     a.M = M; a.N = N; a.K = K;
-    a.lda = K; a.ldb = K;
     a.BM = e->f[0]; a.BN = e->f[1];
     a.TN = N / a.BN;
     a.rLDN = rLDN;

@@ -218,7 +218,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(uint64_t A_, uint64_t B
     // The descriptors point at the stage's first column of the tile's first row and cover exactly the
     // tile's rows from there (the host checks that this fits 31 bits).
     const unsigned a_span = (unsigned)((255 * f.K + f.K) * 2);
-    // A and B have one leading dimension (the launcher checks it), so the lane offsets, the span and the
+    // Rows of A and of B are K elements apart (GemmArgs has no other stride), so the lane offsets, the span and the
     // row-block offsets of the eight loads per operand serve both.
     unsigned soff_a[8];
 #pragma unroll

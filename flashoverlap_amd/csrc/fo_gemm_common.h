@@ -77,8 +77,7 @@ __host__ __device__ inline __attribute__((always_inline)) void fo_raster_tile(in
 struct GemmArgs {
     const uint16_t *A;
     const uint16_t *B;
-    int M, N, K;
-    int lda, ldb;          // row strides of A and B in elements (multiples of 8)
+    int M, N, K;           // K is also the row stride of both operands
     int grid_m, grid_n, panel, xcd_remap;  // the raster of this launch's parent tiles
     int first, sub_m, sub_n, count;        // this launch: positions from `first`, each cut into sub_m x sub_n macro tiles, `count` of them
     uint16_t *C;
@@ -243,7 +242,7 @@ __host__ __device__ inline __attribute__((always_inline)) void fo_tile_of(const 
 }
 
 // Every operand row begins on a 128-byte line.
-inline bool on_lines(const GemmArgs &a) { return (((uintptr_t)a.A | (uintptr_t)a.B | (uintptr_t)a.lda * 2) & 127) == 0; }
+inline bool on_lines(const GemmArgs &a) { return (((uintptr_t)a.A | (uintptr_t)a.B | (uintptr_t)a.K * 2) & 127) == 0; }
 
 constexpr int kMaxSub = 4;        // reorder tiles per macro tile (256x256 over 128x128)
 constexpr int kPrefixRegs = 256;  // group search on prefix sums held in registers (one per 64 groups) up to this many groups

@@ -96,3 +96,31 @@ def test_packed_arguments_say_what_the_launch_is(tmp_path):
     out = subprocess.run([str(tmp_path / "args")], check=True, capture_output=True, text=True).stdout.split()
     bad, seen, walked = map(int, out)
     assert bad == 0 and seen > 1000 and walked > 100000
+
+
+NO_STRIDES = r"""
+#include "fo_gemm_common.h"
+#include <cstdio>
+using namespace fo_gemm_dev;
+template <typename T> auto has_a(int) -> decltype((void)T::lda, true) { return true; }
+template <typename T> bool has_a(...) { return false; }
+template <typename T> auto has_b(int) -> decltype((void)T::ldb, true) { return true; }
+template <typename T> bool has_b(...) { return false; }
+int main() {
+    std::printf("%d\n", has_a<GemmArgs>(0) || has_b<GemmArgs>(0) || has_a<TileArgs>(0) || has_b<TileArgs>(0));
+    return 0;
+}
+"""
+
+
+def test_a_launch_cannot_name_a_row_stride_that_the_kernels_ignore(tmp_path):
+    """Both kernels take K as the row stride of A and B: a launch described with another one would read wrong rows."""
+    src = tmp_path / "strides.hip"
+    src.write_text(NO_STRIDES)
+    flags = [f for f in build.HIP_FLAGS if not f.startswith("--offload-arch") and f not in ("-Xclang", "-target-feature", "-packed-fp32-ops")]
+    try:
+        subprocess.run([build.HIPCC, "--cuda-host-only"] + flags + [str(src), "-o", str(tmp_path / "strides")], check=True, capture_output=True, text=True)
+    except FileNotFoundError:
+        pytest.skip("no hipcc")
+    out = subprocess.run([str(tmp_path / "strides")], check=True, capture_output=True, text=True).stdout.split()
+    assert out == ["0"]
