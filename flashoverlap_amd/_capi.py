@@ -25,6 +25,7 @@ SIGNATURES = {
     "fo_workgroup_tiles": (c_int, [c_int, c_int, c_int, vp, vp]),
     "fo_gemm_wave_tiles": (c_int, [c_int, c_int, c_int, c_int, vp]),
     "fo_gemm_kernel_info": (c_int, [c_int, c_int, c_int, c_int, c_int, vp]),
+    "fo_gemm_plan": (c_int, [c_int, c_int, c_int, c_int, vp, vp, c_int, c_int, c_int, vp]),
     "fo_set": (c_int, [vp, c_int, vp]),
     "fo_wait_groups": (c_int, [c_int, vp, vp, vp]),
     "fo_gemm": (c_int, [c_int, c_int, c_int, c_int, vp, vp, vp, c_int, vp]),
@@ -200,6 +201,15 @@ def kernel_info(algo, M, N, epilogue=1, dtype=F16):
     info = (ctypes.c_int32 * 4)()
     check(lib().fo_gemm_kernel_info(int(dtype), int(algo), M, N, int(epilogue), info), "fo_gemm_kernel_info")
     return {"resident": info[0], "vgprs": info[1], "lds_bytes": info[2], "threads": info[3]}
+
+
+def gemm_plan(algo, M, N, K, epilogue=0, counts=False, acc=False, A=0, B=0):
+    """How a GEMM is launched: {tile, tiles of the main launch, panel, positions of 256x256 left to a second launch, its
+    tile}.  A, B: addresses of the operands (their alignment counts); epilogue 0 plain, 1 reordered, 2 row-mapped."""
+    plan = (ctypes.c_int32 * 7)()
+    check(lib().fo_gemm_plan(int(algo), M, N, K, int(A) or None, int(B) or None, int(epilogue), int(bool(counts)), int(bool(acc)),
+                             plan), "fo_gemm_plan")
+    return {"tile": (plan[0], plan[1]), "count": plan[2], "panel": plan[3], "second": plan[4], "second_tile": (plan[5], plan[6])}
 
 
 def norm_rows_kernel_info(dim, reorder=True, BN=128, rldn=1, beside_gemm=True, dtype=F16):

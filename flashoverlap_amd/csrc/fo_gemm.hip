@@ -103,6 +103,13 @@ struct tail_cost {
 constexpr tail_cost kTailCosts[] = {{64, 64, 5.3, 18.2, 1.1}, {64, 128, 4.9, 24.5, 2.2}, {128, 128, 4.7, 38.5, 4.6}, {128, 256, 5.5, 66, 7.8}};
 constexpr double kTailLastRound = 0.5;
 
+// Share of an operand's rows that do not begin on a 128-byte line.  Its row stride is a multiple of `step` bytes, a power of two up
+// to 128: from a base that is one too, every 128 / step-th row lies on a line, from another one none.
+double off_lines_share(const void *base, int K) {
+    const unsigned pitch = (unsigned)K * 2 | 128, step = pitch & (0 - pitch);
+    return (uintptr_t)base % step ? 1.0 : 1.0 - step / 128.0;
+}
+
 // Rounds of `count` tiles: a last one that is not full costs a part of a round and its share of the CUs (fewer active CUs
 // share the L2s, HBM and the power limit).
 double rounds(long count, long cus, double last) {
@@ -128,8 +135,9 @@ double rounds(long count, long cus, double last) {
 // was complete in its last round (8064x8192 in four groups: rounds 3, 1, 2, 3 of 0..3).
 // M and N need only be multiples of 128: the last tile of a dimension is moved back or, 256x256, repeats half of its
 // neighbour.
-launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN, bool whole_only, bool counted, bool on_lines,
+launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN, bool whole_only, bool counted, double off_lines,
                         bool mapped, bool acc) {
+    const bool on_lines = off_lines == 0;
     launch_plan p;
     p.tail = p.tail_tm = p.tail_tn = 0;
     auto set = [&](int tm, int tn) {
@@ -172,10 +180,9 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN,
     if (!counted) {
         const int rem = nt > cus && nt % cus * 2 <= cus ? (int)(nt % cus) : 0;  // what a second launch may take
         const double k = K / 4096.0;
-        // Several rounds of the 256x256 tile.  With an odd multiple of 32 as K only every other row is off the lines, otherwise most
-        // are.  Without an accumulator the halves that repeat a neighbour's multiply nothing.  Whole passes, us, in 128x192 tiles, which
+        // Several rounds of the 256x256 tile.  Where every other row lies on a line its loads cost less.  Without an accumulator the halves that repeat a neighbour's multiply nothing.  Whole passes, us, in 128x192 tiles, which
         // looked the cheaper ones without the two -> in these: 6656x6272x5088 405 -> 373, 6400x6528x5840 bf16 438 -> 424.
-        const double off_share = nt <= cus ? 0.9 : K % 64 == 32 ? 0.57 : 1.0;
+        const double off_share = nt <= cus ? 0.9 : off_lines <= 0.5 ? 0.57 : 1.0;
         const double area = acc || mapped ? 1.0 : (double)M * N / (nt * 65536.0);
         const tile_cost *best = nullptr;
         const tail_cost *best_tail = nullptr;
@@ -228,6 +235,13 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN,
         if (BM == 128 && BN == 128 && r.tail_tiles * 4 > r.resident && N % 256 == 0) p.tail_tn = 256;
     }
     return p;
+}
+
+// The plan of a GEMM whose operands lie at A and B.
+launch_plan plan_gemm(const fo_raster &r, const fo_algo_entry &e, int M, int N, int K, const void *A, const void *B, int mode,
+                      bool counts, bool monitor, bool acc) {
+    return plan_launch(r, M, N, K, e.f[0], e.f[1], counts && (monitor || K < kSignalAfterFromK), counts,
+                       (off_lines_share(A, K) + off_lines_share(B, K)) / 2, mode == MODE_SCATTER || mode == MODE_RS, acc);
 }
 
 // Whether a launch that counts can do the sums of its last wave itself (MODE_SIGNAL_SUM, MODE_SCATTER_SUM).
@@ -298,8 +312,7 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     a.rank = rs ? rs->rank : 0;
     a.seg_rows = (int)((int64_t)M * N / a.BN / a.W);
     const bool counts = (mode == MODE_SIGNAL || mode == MODE_SCATTER) && !quiet;
-    const launch_plan plan = plan_launch(r, M, N, K, a.BM, a.BN, counts && (monitor || K < kSignalAfterFromK), counts, on_lines(a),
-                                         mode == MODE_SCATTER || mode == MODE_RS, acc != nullptr);
+    const launch_plan plan = plan_gemm(r, *e, M, N, K, A, B, mode, counts, monitor, acc != nullptr);
     a.grid_m = plan.grid_m; a.grid_n = plan.grid_n; a.panel = plan.panel; a.xcd_remap = plan.xcd_remap;
     a.first = 0; a.sub_m = a.sub_n = 1;
     a.count = plan.count;
@@ -415,7 +428,7 @@ int fo_gemm_last_wave(int algo, int M, int N, int32_t *first, int32_t *slots) {
     fo_raster r;
     int rc = fo_pick_raster(algo, M, N, &r);
     if (rc) return rc;
-    const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, true, true, false, false);
+    const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, true, 0.0, false, false);
     const int resident = fo_main_tile_resident();
     *slots = (M / e->f[0]) * (N / e->f[1]);
     *first = last_wave_sums(plan) ? (plan.count - 1) / resident * resident * (256 / e->f[0]) * (256 / e->f[1]) : *slots;
@@ -437,7 +450,7 @@ extern "C" int fo_gemm_wave_tiles(int dtype, int algo, int M, int N, int32_t *ti
     fo_raster r;
     int rc = fo_pick_raster(algo, M, N, &r);
     if (rc) return rc;
-    const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, true, true, false, false);
+    const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, true, 0.0, false, false);
     GemmArgs a = {};
     a.count = plan.count;
     int info[5] = {0, 0, 0, 0, 0};
@@ -455,7 +468,7 @@ extern "C" int fo_gemm_kernel_info(int dtype, int algo, int M, int N, int epilog
     int rc = fo_pick_raster(algo, M, N, &r);
     if (rc) return rc;
     const fo_algo_entry *e = fo_algo_lookup(algo);
-    const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, epilogue != MODE_PLAIN, true,
+    const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, epilogue != MODE_PLAIN, 0.0,
                                          epilogue == MODE_SCATTER, false);
     GemmArgs a = {};
     a.count = plan.count;
@@ -464,6 +477,23 @@ extern "C" int fo_gemm_kernel_info(int dtype, int algo, int M, int N, int epilog
     rc = launch_tile(dtype, epilogue, a, plan.tm, plan.tn, nullptr, out);
     if (rc) return rc;
     for (int i = 0; i < 4; i++) info[i] = out[i];
+    return FO_OK;
+}
+
+extern "C" int fo_gemm_plan(int algo, int M, int N, int K, const void *A, const void *B, int epilogue, int counts, int acc,
+                            int32_t plan[7]) {
+    if (!plan || epilogue < MODE_PLAIN || epilogue > MODE_SCATTER || (counts && (acc || epilogue == MODE_PLAIN))) return FO_ERR_ARG;
+    if (K <= 0) return FO_ERR_ARG;
+    if (K % 8) return FO_ERR_SHAPE;
+    const fo_algo_entry *e = fo_algo_lookup(algo);
+    if (!e) return FO_ERR_ALGO;
+    if (e->f[0] % 128 || e->f[1] % 128) return FO_ERR_ALGO;
+    fo_raster r;
+    int rc = fo_pick_raster(algo, M, N, &r);
+    if (rc) return rc;
+    const launch_plan p = plan_gemm(r, *e, M, N, K, A, B, epilogue, counts != 0, false, acc != 0);
+    const int32_t out[7] = {p.tm, p.tn, p.count, p.panel, p.tail, p.tail_tm, p.tail_tn};
+    for (int i = 0; i < 7; i++) plan[i] = out[i];
     return FO_OK;
 }
 

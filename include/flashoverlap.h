@@ -83,6 +83,13 @@ int fo_gemm_wave_tiles(int dtype, int algo, int M, int N, int32_t *tiles);
  * workgroup): that holds while GEMM wavefronts per SIMD x registers stays at or
  * below 448. */
 int fo_gemm_kernel_info(int dtype, int algo, int M, int N, int epilogue, int32_t info[4]);
+/* How a GEMM is launched (host only; of A and B the addresses alone are looked at; no counterpart in the reference): plan =
+ * {rows, columns of the workgroup tile, tiles of the main launch, its raster's panel height (packed where
+ * waves are whole tile rows); raster positions of 256x256 left to a second launch, rows and columns of that one's tile}.
+ * epilogue: 0 plain, 1 reordered, 2 row-mapped (a reduce-scatter's too); counts: it moves counters, without the monitor; acc: it
+ * adds to an accumulator itself (epilogues 0 to 2; not together with counts). */
+int fo_gemm_plan(int algo, int M, int N, int K, const void *A, const void *B, int epilogue, int counts, int acc,
+                 int32_t plan[7]);
 /* The GEMM launches count on n CUs from this call on (n <= 0: on all of the
  * device's; 0 < n < 8 is FO_ERR_ARG): the persistent launches hold
  * n x workgroups-per-CU workgroups (rounded down to a multiple of 8), and
