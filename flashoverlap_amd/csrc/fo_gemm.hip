@@ -76,31 +76,41 @@ constexpr int kSignalAfterFromK = 1536;
 // What launches without counters of more than one round of 128x160 tiles take, microseconds.  Each round, all CUs busy, has a share
 // that goes with K (given at K = 4096: operand rows on 128-byte lines, off them, and off them with a row map, which leaves
 // 128x192 no LDS for its line loads; 128x256 and 256x256 have none) and an end that does not: a tile's stores, which nothing of the
-// next one runs beside, dearer by a row map, and an accumulator's values and sums.  Fitted to whole passes, GEMM and
-// normalisation, of 2220 products (plain, with an accumulator, over four ranks with and without one; K = 256 to 8192), each in
-// all tiles, three states in turn: the pass in the tile of least estimate is 0.65 % longer than in the best one, in the mean;
-// with estimates in proportion to K, an end for short sums only and the Algo's tile in the second launch it was 1.7 % (one in seven
-// is more than 3 % faster now, one in thirty more than 3 % slower; 5376x3584x1096 bf16 90.1 -> 76.5 us, 2432x7424x664 62.5 -> 57.6).
+// next one runs beside, dearer by a row map, and an accumulator's values and sums.
+//
+// The constants of both tables and those beside them are the ones that leave least of (r + 4 r r), r the part by which the pass in the tile of
+// least estimate is longer than in the best one, over whole passes, GEMM and normalisation, of 8400 products: calls that come here, K =
+// 256 to 8192, 500 of them with operands 16 bytes off the lines, each in all tiles, three states in turn, in five runs.
+// The pass in the tile of least estimate is longer than in the best one by 0.49 % in the mean and by more than 3 % in one of 18; over 1500
+// products that were not fitted by 0.60 % and in one of 13.  (Before, a fit to 2220 products of one box with corrections behind it: 0.71 %
+// and one of 11, 0.78 % and one of 10, with operands off the lines 1.1 % and one of 7; estimates in proportion to K: 1.76 % and one of 5.)
+// What the former fit had lost came from too dear sums in the smaller tiles, and from counting a 256x256 tile of which half
+// repeats its neighbour's as half a tile: us, its choice -> now, 6144x2048x5544 bf16 169 -> 138, 5120x3200x1232 with an accumulator 73.7 ->
+// 67.1, 6912x1152x936 30.9 -> 28.7, 3456x7936x376 72.4 -> 70.4; near ties also go the other way, 6400x6528x5840 bf16 424 -> 438.
 struct tile_cost {
     int tm, tn;
     double on_lines, off_lines, mapped;  // at K = 4096
     double end, end_mapped, sums, sums_mapped;
 };
 constexpr tile_cost kTileCosts[] = {
-    {96, 128, 25.3, 25.5, 25, 1.7, 3.0, 1.3, 1.9},    {128, 128, 30.5, 31.5, 30.5, 1.7, 3.4, 2.0, 2.4},
-    {128, 160, 35.2, 37, 36.5, 2.2, 4.2, 3.0, 3.4},   {128, 192, 40.5, 41.5, 52, 2.8, 4.1, 3.1, 3.7},
-    {128, 256, 52, 65.5, 64.5, 2.8, 5.1, 3.7, 5.1},   {256, 128, 52, 65.5, 64.5, 2.8, 5.1, 3.7, 5.1},
-    {256, 256, 88.5, 106, 103, 5.2, 10.5, 8.7, 9.9}};
+    {96, 128, 25.3, 25.5, 25, 1.5, 3.0, 1.4, 2.3},     {128, 128, 30.5, 31.5, 30.5, 1.7, 3.4, 1.6, 2.8},
+    {128, 160, 35.2, 37, 37, 2.3, 4.0, 2.7, 3.7},      {128, 192, 40.5, 40.5, 52, 3.0, 4.2, 3.0, 4.0},
+    {128, 256, 52, 65.5, 64.5, 2.8, 5.1, 3.7, 5.1},    {256, 128, 52, 65.5, 64.5, 2.8, 5.1, 3.7, 5.1},
+    {256, 256, 88.5, 106, 104, 4.7, 10.5, 8.9, 10.5}};
 constexpr double kLastRound = 0.6;
+constexpr double kHalfOffLines = 0.22;  // 256x256, several rounds: of what rows off the lines cost, where every other one lies on one
+// Near ties of several rounds go to the 256x256 tiles, which take the least energy: 5248x7936x2496 222 us, in 128x256 232.
+constexpr double kLargestTile = 0.98;
 // A last round of 256x256 tiles that is at most half full may go to a second launch: its start and end behind the first one's,
-// its share of K and an accumulator's sums, for each tile that it may have; fitted to the same passes.  (With rem * 16 tiles of 64x64 on
-// a chip that is otherwise idle instead of rem * 2 of 128x256: 2944x6144x3848 over four ranks 166 -> 133 us, 7168x4736x7928 616 -> 519,
-// 3072x6400x4936 with an accumulator 251 -> 214.)
+// its share of K and an accumulator's sums, for each tile that it may have; from the same passes, where rows off the lines and a row map
+// are not told apart (two or three rounds of small tiles differ little by them).  (With rem * 16 tiles of 64x64 on a chip that is otherwise idle
+// instead of rem * 2 of 128x256: 2944x6144x3848 over four ranks 166 -> 133 us, 7168x4736x7928 616 -> 519, 3072x6400x4936 with an
+// accumulator 251 -> 214.)
 struct tail_cost {
     int tm, tn;
     double start, at_4096, sums;
 };
-constexpr tail_cost kTailCosts[] = {{64, 64, 5.3, 18.2, 1.1}, {64, 128, 4.9, 24.5, 2.2}, {128, 128, 4.7, 38.5, 4.6}, {128, 256, 5.5, 66, 7.8}};
+constexpr tail_cost kTailCosts[] = {{64, 64, 3.7, 18.5, 1.9}, {64, 128, 4.3, 24.5, 2.0}, {128, 128, 5.1, 33, 4.0}, {128, 256, 5.1, 65, 7.9}};
 constexpr double kTailLastRound = 0.5;
 
 // Share of an operand's rows that do not begin on a 128-byte line.  Its row stride is a multiple of `step` bytes, a power of two up
@@ -158,10 +168,11 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN,
         set(tm, tn);
         p.panel = p.grid_m < 8 ? p.grid_m : 8;
         // One or two rows left over would be a panel whose XCDs share one operand hardly at all (a block of 32 tiles reads 12
-        // panels of operand rows as 8 x 4, 18 as 2 x 16, 33 as 1 x 32): panels of about one height instead.  Whole passes, us:
-        // 1152x5120x1720 (9 rows of 128x192) 27.4 -> 26.4, 640x1024x4408 (10 of 64x64) 18.3 -> 17.7, 4224x7168x3584 (17 of 256x256)
-        // 176.6 -> 172.4.  With three and more rows left over eight stay: 1408x3328x1240 (11) 19.6 -> 19.9, 1792x3584x3936 (14) 60 -> 65; and
-        // where the panel left over is a small part: 6656x6272x5088 (26 of 256x256) 381 -> 386, 6400x6528x5840 (25) 432 -> 437.
+        // panels of operand rows as 8 x 4, 18 as 2 x 16, 33 as 1 x 32): panels of about one height instead, while that panel would be a large part
+        // of the raster.  Whole passes of 1600 problems of more than eight tile rows in both: 0.8 % shorter in the mean for 9, 10, 17
+        // and 18 rows (1.8 % for 9; 43 of 255 by more than 2 %, 9 longer by that), the same within 0.2 % for 25 and 26 and for other remainders.
+        // 1152x5120x1720 (9 rows of 128x192) 27.4 -> 26.4 us, 640x1024x4408 (10 of 64x64) 18.3 -> 17.7, 4224x7168x3584 (17 of 256x256) 176.6 ->
+        // 172.4.  (From 33 rows on, rasters of many rounds, one or two rows left over would gain 0.6 %; they keep eight.)
         const int panels = (p.grid_m + 7) / 8, left = p.grid_m % 8;
         if (panels > 1 && panels < 4 && (left == 1 || left == 2)) p.panel = (p.grid_m + panels - 1) / panels;
     };
@@ -180,21 +191,17 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN,
     if (!counted) {
         const int rem = nt > cus && nt % cus * 2 <= cus ? (int)(nt % cus) : 0;  // what a second launch may take
         const double k = K / 4096.0;
-        // Several rounds of the 256x256 tile.  Where every other row lies on a line its loads cost less.  Without an accumulator the halves that repeat a neighbour's multiply nothing.  Whole passes, us, in 128x192 tiles, which
-        // looked the cheaper ones without the two -> in these: 6656x6272x5088 405 -> 373, 6400x6528x5840 bf16 438 -> 424.
-        const double off_share = nt <= cus ? 0.9 : off_lines <= 0.5 ? 0.57 : 1.0;
-        const double area = acc || mapped ? 1.0 : (double)M * N / (nt * 65536.0);
         const tile_cost *best = nullptr;
         const tail_cost *best_tail = nullptr;
         double least = 0;
         for (const tile_cost &t : kTileCosts) {
             if (M < t.tm || N < t.tn) continue;
             const bool largest = t.tm * t.tn == 256 * 256;
-            const double off = ((mapped ? t.mapped : t.off_lines) - t.on_lines) * (largest ? off_share : 1.0);
-            // near ties of several rounds go to the 256x256 tiles, which take the least energy: 5248x7936x2496 222 us, in 128x256 232
+            const bool rounds_of_largest = nt > cus && largest;
+            const double off = ((mapped ? t.mapped : t.off_lines) - t.on_lines) * (rounds_of_largest && off_lines <= 0.5 ? kHalfOffLines : 1.0);
             const double round = (k * (t.on_lines + (on_lines ? 0 : off)) + (mapped ? t.end_mapped : t.end) +
                                   (!acc ? 0 : mapped ? t.sums_mapped : t.sums)) *
-                                 (nt > cus && largest ? 0.98 * area : 1.0);
+                                 (rounds_of_largest ? kLargestTile : 1.0);
             auto offer = [&](double cost, const tail_cost *tail) {
                 if (best && cost >= least) return;
                 best = &t;
