@@ -3,8 +3,7 @@ addresses only."""
 import pytest
 
 from flashoverlap_amd import _capi
-
-LINE = 1 << 20  # an address on a 128-byte line
+from second_launch_cases import CASES, FORMS, LINE, expected, planned
 
 
 def plan(M, N, K, form="reordered", bm=128, bn=128, counts=False, off=0):
@@ -42,6 +41,20 @@ def test_rows_off_the_lines_by_their_base_address(form, bm, bn, M, N, K):
 ])
 def test_smaller_tiles_where_they_are_faster(form, bm, bn, M, N, K, off, tile):
     assert plan(M, N, K, form, bm, bn, off=off) == (tile,)
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(v) for v in c[:6]))
+def test_second_launches_are_what_their_cases_say(case, form):
+    _, second, edges = planned(case, form)
+    assert (second, edges) == (expected(case, form), case[7] if second else "")
+
+
+def test_each_second_launch_is_in_some_case_with_each_epilogue_and_edge():
+    seen = {(form, *planned(case, form)[1:]) for case in CASES for form in FORMS}
+    for form in FORMS:
+        for tile in ((64, 64), (64, 128), (128, 128), (128, 256)):
+            assert (form, tile, "MN") in seen
 
 
 def test_plan_refuses_what_no_launch_takes():
