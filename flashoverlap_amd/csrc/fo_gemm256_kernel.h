@@ -305,7 +305,7 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(uint64_t A_, uint64_t B
 #pragma unroll
     for (int c = 0; c < 16; c++) load_chunk(c, 0);
     typedef const __attribute__((address_space(4))) char *args_t;
-    args_t rest = (args_t)__builtin_amdgcn_kernarg_segment_ptr() + 7 * 8;
+    args_t rest = (args_t)__builtin_amdgcn_kernarg_segment_ptr() + kGemmArgsAt;
     asm volatile("" : "+s"(rest));  // the other arguments are read from here on
     const __attribute__((address_space(4))) GemmArgs &p = *(const __attribute__((address_space(4))) GemmArgs *)rest;
     // Those that the first tile's group sizes and slots need, in one round trip.

@@ -74,7 +74,7 @@ __host__ __device__ inline __attribute__((always_inline)) void fo_raster_tile(in
 }
 
 // A launch as the host describes it, and, behind those words that its first load needs, the 256x256 kernel's arguments.
-struct GemmArgs {
+struct alignas(64) GemmArgs {
     const uint16_t *A;
     const uint16_t *B;
     int M, N, K;           // K is also the row stride of both operands
@@ -98,6 +98,10 @@ struct GemmArgs {
 
     static GemmArgs of(const GemmArgs &a, int, int) { return a; }
 };
+// What the 256x256 kernel's epilogue reads of it, C and on, are two 64-byte lines of its launch's 256 bytes of arguments (in front stand
+// Front256's seven words, one of padding and the part up to C); eight bytes earlier they are three: 4096x4096x512 with an accumulator 40.65 -> 41.0 us.
+constexpr int kGemmArgsAt = 64;
+static_assert(offsetof(GemmArgs, C) == 64 && sizeof(GemmArgs) == 192, "the kernel's part begins on a line and ends with the second one");
 
 // The smaller tiles' arguments: 112 bytes, because a launch takes the host 2.7 us with up to 112 bytes of arguments and 3.1 to
 // 3.7 with 120 or more, those that the runtime adds for gridDim among them (an empty kernel in a process with torch, which
