@@ -478,13 +478,21 @@ __global__ __launch_bounds__(256) void fo_gemm256_kernel(uint64_t A_, uint64_t B
     for (int q = 0; q < 4; q++) load_a(0, la0 ^ (q % 2 * KSTEP_X), q / 2, q % 2);
 #pragma unroll
     for (int q = 0; q < 10; q++) load_b(lb0 ^ (q % 2 * KSTEP_X), q / 2, q % 2);
-    if (MODE != MODE_PLAIN) asm volatile("" : "+v"(slots_raw));  // has arrived with them
-    sum_groups();  // the group sizes arrived before stage 0 did (requested earlier, vmcnt retires in issue order)
+    // Slots and group sizes, requested between the two stages, have arrived too (vmcnt retires in issue order).  Pinned here: to the
+    // compiler they were in their registers from the request on, and nothing else keeps a use of them behind the wait.
+    if (MODE != MODE_PLAIN) asm volatile("" : "+v"(slots_raw));
+    if (groups && reg_search) {
+#pragma unroll
+        for (int q = 0; q < NPRE; q++) asm volatile("" : "+v"(cs_raw[q]));
+    }
+    sum_groups();
 
     int tile = blockIdx.x;
     unsigned slot_b = 0;  // byte offset of the slot the next K step reads
     for (;;) {
-        if (MODE != MODE_PLAIN && reorder && tile == (int)blockIdx.x) {  // later tiles: taken inside the previous tile's epilogue
+        // Later tiles: taken inside the previous tile's epilogue.  (In front of the loop, without the test, slots_raw would not live through
+        // it, but the accumulating epilogue's K loop is laid out otherwise and slower: 4096x8192x8192 421.7 -> 423.5 us.)
+        if (MODE != MODE_PLAIN && reorder && tile == (int)blockIdx.x) {
             v_rs = slots_raw;
             r_mine = __builtin_amdgcn_readlane(slots_raw, my_sub);
         }
