@@ -81,12 +81,13 @@ constexpr int kSignalAfterFromK = 1536;
 // The constants of both tables and those beside them are the ones that leave least of (r + 4 r r), r the part by which the pass in the tile of
 // least estimate is longer than in the best one, over whole passes, GEMM and normalisation, of 8400 products: calls that come here, K =
 // 256 to 8192, 500 of them with operands 16 bytes off the lines, each in all tiles, three states in turn, in five runs.
-// The pass in the tile of least estimate is longer than in the best one by 0.49 % in the mean and by more than 3 % in one of 18; over 1500
-// products that were not fitted by 0.60 % and in one of 13.  (Before, a fit to 2220 products of one box with corrections behind it: 0.71 %
+// The pass in the tile of least estimate is longer than in the best one by 0.45 % in the mean and by more than 3 % in one of 20; over 1500
+// products that were not fitted by 0.56 % and in one of 15.  (Before, a fit to 2220 products of one box with corrections behind it: 0.71 %
 // and one of 11, 0.78 % and one of 10, with operands off the lines 1.1 % and one of 7; estimates in proportion to K: 1.76 % and one of 5.)
 // What the former fit had lost came from too dear sums in the smaller tiles, and from counting a 256x256 tile of which half
 // repeats its neighbour's as half a tile: us, its choice -> now, 6144x2048x5544 bf16 169 -> 138, 5120x3200x1232 with an accumulator 73.7 ->
-// 67.1, 6912x1152x936 30.9 -> 28.7, 3456x7936x376 72.4 -> 70.4; near ties also go the other way, 6400x6528x5840 bf16 424 -> 438.
+// 67.1, 6912x1152x936 30.9 -> 28.7, 3456x7936x376 72.4 -> 70.4; others go the other way, 6400x6528x5840 bf16 424 -> 438,
+// 8192x4224x264 with an accumulator 84 -> 98.
 struct tile_cost {
     int tm, tn;
     double on_lines, off_lines, mapped;  // at K = 4096
@@ -97,6 +98,9 @@ constexpr tile_cost kTileCosts[] = {
     {128, 160, 35.2, 37, 37, 2.3, 4.0, 2.7, 3.7},      {128, 192, 40.5, 40.5, 52, 3.0, 4.2, 3.0, 4.0},
     {128, 256, 52, 65.5, 64.5, 2.8, 5.1, 3.7, 5.1},    {256, 128, 52, 65.5, 64.5, 2.8, 5.1, 3.7, 5.1},
     {256, 256, 88.5, 106, 104, 4.7, 10.5, 8.9, 10.5}};
+// An accumulator's sums in a tile between 128x160 and 256x256 that lies in one reorder tile, or in a product that is not reordered, cost
+// that much less: its pieces need one address (each_piece in the kernel).  Without this term the passes above are 0.04 % longer.
+constexpr double kOnePiece = 0.4;
 constexpr double kLastRound = 0.6;
 constexpr double kHalfOffLines = 0.22;  // 256x256, several rounds: of what rows off the lines cost, where every other one lies on one
 // Near ties of several rounds go to the 256x256 tiles, which take the least energy: 5248x7936x2496 222 us, in 128x256 232.
@@ -146,7 +150,7 @@ double rounds(long count, long cus, double last) {
 // M and N need only be multiples of 128: the last tile of a dimension is moved back or, 256x256, repeats half of its
 // neighbour.
 launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN, bool whole_only, bool counted, double off_lines,
-                        bool mapped, bool acc) {
+                        bool reordered, bool mapped, bool acc) {
     const bool on_lines = off_lines == 0;
     launch_plan p;
     p.tail = p.tail_tm = p.tail_tn = 0;
@@ -171,8 +175,8 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN,
         // panels of operand rows as 8 x 4, 18 as 2 x 16, 33 as 1 x 32): panels of about one height instead, while that panel would be a large part
         // of the raster.  Whole passes of 1600 problems of more than eight tile rows in both: 0.8 % shorter in the mean for 9, 10, 17
         // and 18 rows (1.8 % for 9; 43 of 255 by more than 2 %, 9 longer by that), the same within 0.2 % for 25 and 26 and for other remainders.
-        // 1152x5120x1720 (9 rows of 128x192) 27.4 -> 26.4 us, 640x1024x4408 (10 of 64x64) 18.3 -> 17.7, 4224x7168x3584 (17 of 256x256) 176.6 ->
-        // 172.4.  (From 33 rows on, rasters of many rounds, one or two rows left over would gain 0.6 %; they keep eight.)
+        // 640x1024x4408 (10 rows of 64x64) 18.8 -> 18.3 us, 4224x7168x3584 (17 of 256x256) 180.5 -> 177.7, 1152x5120x1720 (9 of 128x192) the same.
+        // (From 33 rows on, rasters of many rounds, one or two rows left over would gain 0.6 %; they keep eight.)
         const int panels = (p.grid_m + 7) / 8, left = p.grid_m % 8;
         if (panels > 1 && panels < 4 && (left == 1 || left == 2)) p.panel = (p.grid_m + panels - 1) / panels;
     };
@@ -199,8 +203,9 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN,
             const bool largest = t.tm * t.tn == 256 * 256;
             const bool rounds_of_largest = nt > cus && largest;
             const double off = ((mapped ? t.mapped : t.off_lines) - t.on_lines) * (rounds_of_largest && off_lines <= 0.5 ? kHalfOffLines : 1.0);
+            const bool one_piece = !mapped && !largest && t.tm * t.tn > 128 * 160 && (!reordered || (BM % t.tm == 0 && BN % t.tn == 0));
             const double round = (k * (t.on_lines + (on_lines ? 0 : off)) + (mapped ? t.end_mapped : t.end) +
-                                  (!acc ? 0 : mapped ? t.sums_mapped : t.sums)) *
+                                  (!acc ? 0 : mapped ? t.sums_mapped : t.sums - (one_piece ? kOnePiece : 0))) *
                                  (rounds_of_largest ? kLargestTile : 1.0);
             auto offer = [&](double cost, const tail_cost *tail) {
                 if (best && cost >= least) return;
@@ -246,9 +251,9 @@ launch_plan plan_launch(const fo_raster &r, int M, int N, int K, int BM, int BN,
 
 // The plan of a GEMM whose operands lie at A and B.
 launch_plan plan_gemm(const fo_raster &r, const fo_algo_entry &e, int M, int N, int K, const void *A, const void *B, int mode,
-                      bool counts, bool monitor, bool acc) {
+                      bool reordered, bool counts, bool monitor, bool acc) {
     return plan_launch(r, M, N, K, e.f[0], e.f[1], counts && (monitor || K < kSignalAfterFromK), counts,
-                       (off_lines_share(A, K) + off_lines_share(B, K)) / 2, mode == MODE_SCATTER || mode == MODE_RS, acc);
+                       (off_lines_share(A, K) + off_lines_share(B, K)) / 2, reordered, mode == MODE_SCATTER || mode == MODE_RS, acc);
 }
 
 // Whether a launch that counts can do the sums of its last wave itself (MODE_SIGNAL_SUM, MODE_SCATTER_SUM).
@@ -319,7 +324,7 @@ int run_gemm(int mode, int dtype, int M, int N, int K, int rLDN, const int32_t *
     a.rank = rs ? rs->rank : 0;
     a.seg_rows = (int)((int64_t)M * N / a.BN / a.W);
     const bool counts = (mode == MODE_SIGNAL || mode == MODE_SCATTER) && !quiet;
-    const launch_plan plan = plan_gemm(r, *e, M, N, K, A, B, mode, counts, monitor, acc != nullptr);
+    const launch_plan plan = plan_gemm(r, *e, M, N, K, A, B, mode, RA != nullptr, counts, monitor, acc != nullptr);
     a.grid_m = plan.grid_m; a.grid_n = plan.grid_n; a.panel = plan.panel; a.xcd_remap = plan.xcd_remap;
     a.first = 0; a.sub_m = a.sub_n = 1;
     a.count = plan.count;
@@ -435,7 +440,7 @@ int fo_gemm_last_wave(int algo, int M, int N, int32_t *first, int32_t *slots) {
     fo_raster r;
     int rc = fo_pick_raster(algo, M, N, &r);
     if (rc) return rc;
-    const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, true, 0.0, false, false);
+    const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, true, 0.0, true, false, false);
     const int resident = fo_main_tile_resident();
     *slots = (M / e->f[0]) * (N / e->f[1]);
     *first = last_wave_sums(plan) ? (plan.count - 1) / resident * resident * (256 / e->f[0]) * (256 / e->f[1]) : *slots;
@@ -457,7 +462,7 @@ extern "C" int fo_gemm_wave_tiles(int dtype, int algo, int M, int N, int32_t *ti
     fo_raster r;
     int rc = fo_pick_raster(algo, M, N, &r);
     if (rc) return rc;
-    const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, true, 0.0, false, false);
+    const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, true, 0.0, true, false, false);
     GemmArgs a = {};
     a.count = plan.count;
     int info[5] = {0, 0, 0, 0, 0};
@@ -476,7 +481,7 @@ extern "C" int fo_gemm_kernel_info(int dtype, int algo, int M, int N, int epilog
     if (rc) return rc;
     const fo_algo_entry *e = fo_algo_lookup(algo);
     const launch_plan plan = plan_launch(r, M, N, 4096, e->f[0], e->f[1], false, epilogue != MODE_PLAIN, 0.0,
-                                         epilogue == MODE_SCATTER, false);
+                                         epilogue != MODE_PLAIN, epilogue == MODE_SCATTER, false);
     GemmArgs a = {};
     a.count = plan.count;
     int out[5] = {0, 0, 0, 0, 0};
@@ -498,7 +503,7 @@ extern "C" int fo_gemm_plan(int algo, int M, int N, int K, const void *A, const 
     fo_raster r;
     int rc = fo_pick_raster(algo, M, N, &r);
     if (rc) return rc;
-    const launch_plan p = plan_gemm(r, *e, M, N, K, A, B, epilogue, counts != 0, false, acc != 0);
+    const launch_plan p = plan_gemm(r, *e, M, N, K, A, B, epilogue, epilogue != MODE_PLAIN, counts != 0, false, acc != 0);
     const int32_t out[7] = {p.tm, p.tn, p.count, p.panel, p.tail, p.tail_tm, p.tail_tn};
     for (int i = 0; i < 7; i++) plan[i] = out[i];
     return FO_OK;

@@ -23,7 +23,7 @@ CASES = [
     (BF16, 128, 128, 3200, 5248, 1536, (S64W, S64W, S64W, S64W), "MN"),
     (BF16, 128, 128, 6272, 2944, 1536, (S128, S128, S128, S128), "MN"),
     (F16, 128, 128, 4224, 4992, 520, (S256, None, S256, S256), "MN"),
-    (BF16, 128, 128, 5504, 3712, 4096, (S256, S256, S256, S256), "MN"),
+    (BF16, 128, 128, 5504, 3712, 4608, (S256, S256, S256, S256), "MN"),
 ]
 
 
