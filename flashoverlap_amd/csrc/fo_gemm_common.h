@@ -105,11 +105,11 @@ static_assert(offsetof(GemmArgs, C) == 64 && sizeof(GemmArgs) == 192, "the kerne
 
 // The smaller tiles' arguments: 112 bytes, because a launch takes the host 2.7 us with up to 112 bytes of arguments and 3.1 to
 // 3.7 with 120 or more, those that the runtime adds for gridDim among them (an empty kernel in a process with torch, which
-// brings its own runtime; the struct above has 208, and 256 were added).  One plain product: 3.9 -> 3.1 us of host time; whole
-// passes that wait for the host: 128x4096x1024 12.3 -> 11.3 us, 128x3328x488 9.5 -> 9.0, 128x2432x320 12.6 -> 12.1.  (The launch's
+// brings its own runtime; a launch of the struct above had 208 bytes and 256 that were added).  One plain product: 3.9 -> 3.1 us of host time; whole
+// passes that wait for the host: 128x4096x1024 11.8 -> 11.4 us, 128x3328x488 9.5 -> 9.0, 128x2432x320 12.6 -> 12.1.  (The launch's
 // size out of the dispatch packet instead of an argument: the packet lies in host memory, 9 us more on every kernel.)
 // What the kernel can derive is derived there, what only one epilogue needs shares its place, and the fields that the first
-// operand load needs stand in front: they come with one load.
+// operand load needs stand in front: they arrive in registers with the wavefront (see TileRest).
 struct TileArgs {
     const uint16_t *A;
     const uint16_t *B;

@@ -247,7 +247,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void fo_gemm_tile_kernel(uint64_t 
 #pragma unroll
         for (int s = 0; s < S - 1; s++) request(s, s * STAGE);
     };
-    asm volatile("" : : "s"(args.A), "s"(args.B), "s"(args.bits));  // all of them with the first round trip
+    asm volatile("" : : "s"(args.A), "s"(args.B), "s"(args.bits));  // in registers from here on, not put together again where they are used
     settle();
     if (loader && tile < count) begin();
 
