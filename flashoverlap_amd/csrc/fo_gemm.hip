@@ -106,8 +106,8 @@ constexpr double kHalfOffLines = 0.22;  // 256x256, several rounds: of what rows
 // Near ties of several rounds go to the 256x256 tiles, which take the least energy: 5248x7936x2496 222 us, in 128x256 232.
 constexpr double kLargestTile = 0.98;
 // A last round of 256x256 tiles that is at most half full may go to a second launch: its start and end behind the first one's,
-// its share of K and an accumulator's sums, for each tile that it may have; from the same passes, where rows off the lines and a row map
-// are not told apart (two or three rounds of small tiles differ little by them).  (With rem * 16 tiles of 64x64 on a chip that is otherwise idle
+// its share of K and an accumulator's sums, for each tile that it may have; from the same passes, which a term for rows off
+// the lines or for a row map, or counting only the tiles that lie inside of the matrix, makes no shorter.  (With rem * 16 tiles of 64x64 on a chip that is otherwise idle
 // instead of rem * 2 of 128x256: 2944x6144x3848 over four ranks 166 -> 133 us, 7168x4736x7928 616 -> 519, 3072x6400x4936 with an
 // accumulator 251 -> 214.)
 struct tail_cost {
